@@ -2,7 +2,7 @@
 //
 // Per matrix (work matrix W, lower triangle) a right-looking blocked Cholesky that keeps the inverses of its 128 x 128
 // diagonal blocks, then the triangular inverse by levels, then out = M^T M (cg_right_looking below):
-//   for every diagonal block k:  leaf: W_kk -> M_kk = L_kk^-1 (one work group, in the LDS: chol_leaf.hpp);
+//   for every diagonal block k:  leaf: W_kk -> M_kk = L_kk^-1 (one work group, in registers: chol_leaf.hpp);
 //                                panel: L21 = A21 M_kk^T;  update: A22 -= L21 L21^T
 //   for every level of a balanced tree over the blocks:  T2 = L21 M11;  M21 = -M22 T2
 // d^3 FLOP in total, like POTRF + POTRI.  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
@@ -189,12 +189,11 @@ static __global__ __launch_bounds__(256) void cg_scale_kernel(CgArgs a, int coun
 // One work group (16 waves) per leaf task of the step.  Every table is read with one load that depends on nothing
 // but the work group's index: a chain of dependent loads from cold device memory costs a microsecond per link.
 static __global__ __launch_bounds__(LEAF_THREADS) void cg_leaf_kernel(CgArgs a, const CgLeafTask* __restrict__ tasks) {
-  extern __shared__ __attribute__((aligned(16))) float leaf_smem[];
+  __shared__ __attribute__((aligned(16))) LeafShared sh;
   const CgLeafTask t = tasks[blockIdx.x];
   const int live = a.skip != nullptr ? a.skip[static_cast<int64_t>(t.mat) * a.skip_stride] : 1;   // used at the end
   const int tid = threadIdx.x;
-  leaf_block(a.ws + t.blk_off, t.ld, t.n, leaf_smem, tid);
-  const int bad = leaf_bad_pivot(leaf_smem);
+  const int bad = leaf_block(a.ws + t.blk_off, t.ld, t.n, sh, tid);
   // a bad pivot inside the identity padding cannot happen; one inside the matrix is reported like LAPACK's potrf.
   // A skipped matrix's work area holds whatever the last call left there; its steps still run (they touch nothing
   // but that work area) and report nothing.
@@ -547,13 +546,6 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
   if (ws == nullptr || (reinterpret_cast<uintptr_t>(ws) & 255) != 0 ||
       ws_bytes < static_cast<size_t>(h->ws_floats) * sizeof(float))
     return AK_ERR_WORKSPACE;
-  static bool leaf_attr_set = false;     // idempotent; a benign race sets it twice at worst
-  if (!leaf_attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(cg_leaf_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(LEAF_LDS_BYTES)) != hipSuccess)
-      return AK_ERR_LAUNCH;
-    leaf_attr_set = true;
-  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   CgArgs a;
   a.plan = static_cast<const unsigned char*>(plan_dev);
@@ -570,7 +562,7 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
       hipLaunchKernelGGL(cg_copy_in_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
       hipLaunchKernelGGL(cg_scale_kernel, dim3(h->count), dim3(256), 0, s, a, h->count, CG_HALF_MAX_COND);
     } else if (st.type == CG_LEAF)
-      hipLaunchKernelGGL(cg_leaf_kernel, dim3(st.grid), dim3(LEAF_THREADS), LEAF_LDS_BYTES, s, a,
+      hipLaunchKernelGGL(cg_leaf_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, a,
                          reinterpret_cast<const CgLeafTask*>(a.plan + h->leaves_off) + st.first);
     else
       hipLaunchKernelGGL(cg_prod_kernel, dim3(st.grid), dim3(256), 0, s, a,

@@ -1,7 +1,7 @@
 // out <- (A + lam I)^-1 for a batch of same-size symmetric positive definite fp32 matrices.
 //
 // Recursive blocked Cholesky that carries the triangular inverse along:
-//   F(lo, hi): n <= 128 -> one work group factors the block in LDS and inverts the factor.
+//   F(lo, hi): n <= 128 -> one work group factors the block and inverts the factor.
 //              otherwise, with [lo,mid) / [mid,hi) and M11 = L11^-1 already in place,
 //                T1  = A21 M11^T            (= L21; the triangular solve is a product)
 //                A22 -= T1 T1^T             (lower triangle only)
@@ -47,20 +47,17 @@ static __global__ __launch_bounds__(256) void chol_copy_in_kernel(BatchPtrs bp, 
   }
 }
 
-// One work group (16 waves) per matrix: the n x n (n <= LEAF) diagonal block at `lo`, padded with an identity to
-// a power-of-two multiple of 16, is factored in LDS by the recursion above: 16 x 16 blocks in the registers of one
-// wave, everything else as 16x16x4 fp32 MFMA products over all waves.  On exit the block holds L^-1 in its lower
-// triangle and zeros above the diagonal.
+// One work group (16 waves) per matrix: the n x n (n <= LEAF) diagonal block at `lo` is factored in the registers of the
+// work group (chol_leaf.hpp).  On exit it holds L^-1 in its lower triangle and zeros above the diagonal.
 static __global__ __launch_bounds__(LEAF_THREADS) void chol_leaf_kernel(float* __restrict__ W, int64_t strideW,
                                                                         int64_t d, int lo, int n,
                                                                         int* __restrict__ info, const int* active,
                                                                         int active_stride) {
-  extern __shared__ __attribute__((aligned(16))) float leaf_smem[];
+  __shared__ __attribute__((aligned(16))) LeafShared sh;
   const int z = blockIdx.x;
   if (active != nullptr && active[static_cast<int64_t>(z) * active_stride] == 0) return;
   const int tid = threadIdx.x;
-  leaf_block(W + z * strideW + static_cast<int64_t>(lo) * d + lo, d, n, leaf_smem, tid);
-  const int bad = leaf_bad_pivot(leaf_smem);
+  const int bad = leaf_block(W + z * strideW + static_cast<int64_t>(lo) * d + lo, d, n, sh, tid);
   if (tid == 0 && bad != 0 && bad <= n && info[z] == 0) info[z] = lo + bad;
 }
 
@@ -88,7 +85,7 @@ static void run_gemm(CholCtx& c, GemmParams p) {
 static void factor_range(CholCtx& c, int lo, int hi, int64_t t1_off) {
   const int n = hi - lo;
   if (n <= LEAF) {
-    hipLaunchKernelGGL(chol_leaf_kernel, dim3(c.batch), dim3(LEAF_THREADS), LEAF_LDS_BYTES, c.stream, c.W, c.strideW,
+    hipLaunchKernelGGL(chol_leaf_kernel, dim3(c.batch), dim3(LEAF_THREADS), 0, c.stream, c.W, c.strideW,
                        c.d, lo, n, c.info, c.active, c.active_stride);
     return;
   }
@@ -164,13 +161,6 @@ extern "C" int ak_chol_inv_batched(const float* const* A_list, float* const* out
   c.active = skip_flags; c.active_stride = skip_stride;
   c.stream = static_cast<hipStream_t>(stream);
   c.rc = AK_OK;
-  static bool leaf_attr_set = false;     // idempotent; a benign race sets it twice at worst
-  if (!leaf_attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(chol_leaf_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(LEAF_LDS_BYTES)) != hipSuccess)
-      return AK_ERR_LAUNCH;
-    leaf_attr_set = true;
-  }
   BatchPtrs bp{A_list, skip_flags, skip_stride};
   dim3 grid(static_cast<unsigned>((d + 15) / 16), static_cast<unsigned>((d + 63) / 64), batch);
   hipLaunchKernelGGL(chol_copy_in_kernel, grid, dim3(256), 0, c.stream, bp, c.W, c.strideW, d, lam, lam_stride, info);

@@ -1,74 +1,40 @@
-// LDS-resident Cholesky factorization + triangular inverse of one diagonal block of at most 128 x 128, shared by
-// the batched (one size) and the grouped (many sizes) damped inverse: 16 x 16 blocks are factored and inverted in
-// the registers of one wave (v_readlane broadcasts), everything larger is the same recursion as the global one
-//   T1 = A21 M11^T,  A22 -= T1 T1^T,  factor(A22),  M21 = -M22 (T1 M11)
-// on LDS operands with v_mfma_f32_16x16x4_f32 tiles spread over the 16 waves of the work group.
+// Cholesky factorization + triangular inverse of one diagonal block of at most 128 x 128 by one work group of 16 waves,
+// shared by the batched (one size) and the grouped (many sizes) damped inverse.
+//
+// The block is 8 x 8 tiles of 16 x 16 and lives in the accumulator registers of the waves for the whole factorization.
+// With A = U^T U (U = L^T) the augmented matrix [A | I] is eliminated by block rows; for block row k
+//   factor   one wave turns the diagonal tile into M_kk = L_kk^-1 in registers (leaf_tile_inverse)
+//   panel    row_k <- M_kk row_k: tiles (k, j > k) become U_kj, tiles (k, j < k) row k of the inverse, which is final
+//   update   tile(i, j) -= U_ki^T row_k(j) for the rows i > k: j >= i updates A, j <= k the inverse
+// so both halves of a row obey one formula, every row is 8 tiles wide (position j < i: inverse, j > i: U), 64 tiles in
+// all, and the inverse is complete when the factorization is: there is no second chain for it.  Only the finished row
+// (16 x 128) and M_kk pass through the LDS.  A tile in the accumulator layout is the right operand of the next product as
+// it is (v_mfma_f32_16x16x4_f32: register r of lane 16 g + c is row 4 g + r, column c; step r of a product contracts the
+// rows {4 g + r}), which is why U and not L is kept.
+//
+// What bounds it: the chain of 8 x (factor -> barrier -> panel -> barrier -> update of the next diagonal tile), about 4 k
+// cycles per link; the wave that owns diagonal tile k + 1 updates it first and factors it while the others still
+// update.  The fp32 matrix instructions of all 224 tile products fill 7 k cycles of the four SIMDs beside it.
 #pragma once
 #include "common.hpp"
 
 namespace ak {
 
 constexpr int LEAF = 128;
+constexpr int LT = 16;                       // tile
+constexpr int LEAF_THREADS = 1024;
+constexpr int LEAF_SLOTS = 5;                // tiles a wave holds at most
+constexpr int LEAF_ROW_LD = LEAF + 4;        // 4 rows apart: 16 banks apart, so the rows 4 g + r of one step do not collide
+constexpr int LEAF_INV_LD = LT + 4;
+
+struct LeafShared {
+  float row[LT * LEAF_ROW_LD];
+  float inv[LT * LEAF_INV_LD];
+  int bad;
+};
 
 __device__ __forceinline__ float lane_bcast(float v, int src_lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src_lane));
-}
-
-constexpr int PB = 16;              // base block handled in registers by one wave
-constexpr int LLD = LEAF + 4;       // LDS leading dimension: rows 4 banks apart, so the [row][k] operand reads of the
-                                    // 16x16x4 MFMA (16 rows x 4 k per instruction) touch 64 different banks
-constexpr int LEAF_THREADS = 1024;
-constexpr int LEAF_WAVES = LEAF_THREADS / 64;
-constexpr int T1_LD = 68;
-// work block, T1 pool (64x64 + 32x32 + 16x16 panels of nested levels) and T2, plus the bad-pivot word
-constexpr int LEAF_T1_FLOATS = 64 * T1_LD + 32 * T1_LD + 16 * T1_LD;
-constexpr int LEAF_T2_FLOATS = 64 * T1_LD;
-constexpr size_t LEAF_LDS_BYTES = (LEAF * LLD + LEAF_T1_FLOATS + LEAF_T2_FLOATS + 8) * sizeof(float);
-
-// Cholesky factor and its inverse of a PB x PB block held one row per lane (lanes >= PB carry an identity
-// row).  On exit a[] is row `lane` of L (entries right of the diagonal are meaningless) and m[] is row `lane` of
-// L^-1 (zeros right of the diagonal).  Returns 0 or the 1-based index of the first non-positive pivot.
-//
-// One loop over the pivots does both.  Row i of the inverse is (e_i - sum_{k<i} l_ik m_k) / l_ii; every lane keeps the
-// numerator u_i of its own row, and pivot k, whose row u_k is complete by then, subtracts (l_ik / l_kk) u_k from the
-// rows below it: k + 1 lane reads and as many multiply-adds that do not depend on one another, next to the 15 - k of
-// the factorization's own update, so that every pivot issues the same 16 + 16 and the wait states of the serial
-// pivot chain (lane read, reciprocal square root, scaling, lane read, multiply-add) are filled.  A forward
-// substitution after the factorization costs the same arithmetic as chains of up to 15 dependent multiply-adds,
-// and took as long again as the factorization.
-// Every step is applied to all lanes without masks where that is harmless: entries above the diagonal and the rows
-// that are already final only ever receive values nobody reads (each broadcast below takes a[k] of a lane j >= k);
-// the rows of the inverse are protected by a factor that is zero for the lanes at and above the pivot.
-__device__ __forceinline__ int small_chol_inv(float (&a)[PB], float (&m)[PB], int lane) {
-  int bad = 0;
-  float my_inv = 1.f;
-#pragma unroll
-  for (int j = 0; j < PB; ++j) m[j] = (j == lane) ? 1.f : 0.f;
-#pragma unroll
-  for (int k = 0; k < PB; ++k) {
-    float akk = lane_bcast(a[k], k);
-    if (!(akk > 0.f)) {             // also catches NaN
-      if (bad == 0) bad = k + 1;
-      akk = 1.f;
-    }
-    float inv = __builtin_amdgcn_rsqf(akk);                 // hardware rsqrt, then one Newton step:
-    inv = inv * (1.5f - 0.5f * akk * inv * inv);             // keeps the serial pivot chain short
-    my_inv = (lane == k) ? inv : my_inv;
-    a[k] *= inv;                    // lane k: a_kk / sqrt(a_kk) = l_kk; lanes below: l_ik
-    const float f = (lane > k) ? a[k] * inv : 0.f;          // l_ik / l_kk for the rows below the pivot
-    float l[PB], u[PB];
-#pragma unroll
-    for (int j = k + 1; j < PB; ++j) l[j] = lane_bcast(a[k], j);
-#pragma unroll
-    for (int j = 0; j <= k; ++j) u[j] = lane_bcast(m[j], k);
-#pragma unroll
-    for (int j = k + 1; j < PB; ++j) a[j] -= a[k] * l[j];
-#pragma unroll
-    for (int j = 0; j <= k; ++j) m[j] -= f * u[j];
-  }
-#pragma unroll
-  for (int j = 0; j < PB; ++j) m[j] *= my_inv;
-  return bad;
 }
 
 // v_mfma_f32_16x16x4_f32: lane l feeds A[i = l%16][k = l/16] and B[k = l/16][j = l%16]; accumulator register r of
@@ -77,136 +43,195 @@ __device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Which part of the contraction range a 16x16 output tile (ib, jb) needs when one operand is triangular (the rest
-// multiplies zeros).
-enum LeafK { LK_FULL, LK_LE_J, LK_GE_J, LK_LE_I };
+// Lane 16 g + c receives register g of lane 16 q + c: the four registers of row group q, one to each row group (a
+// column of the 4 x 4 transposition of registers and 16-lane rows: swap the halves, then the odd with the even rows).
+template <int Q>
+__device__ __forceinline__ float spread_row_group(const floatx4& v) {
+  const auto bits = [](float x) { return __builtin_bit_cast(unsigned, x); };
+  const auto s02 = __builtin_amdgcn_permlane32_swap(bits(v[0]), bits(v[2]), false, false);
+  const auto s13 = __builtin_amdgcn_permlane32_swap(bits(v[1]), bits(v[3]), false, false);
+  const auto t = __builtin_amdgcn_permlane16_swap(s02[Q >> 1], s13[Q >> 1], false, false);
+  return __builtin_bit_cast(float, static_cast<unsigned>(t[Q & 1]));
+}
 
-// C[M x N] (=, -=) alpha * A[M x K] * op(B) for small matrices in LDS, all sizes multiples of 16, one 16x16 output
-// tile per wave and turn.  TB: op(B)[k][j] = B[j][k].  LOWER: only tiles on or below the diagonal (M == N).
-// ACC: C -= product, else C = alpha * product.  The caller synchronises before and after.
-template <int M, int N, int K, bool TB, bool LOWER, bool ACC, LeafK KM>
-__device__ __forceinline__ void leaf_gemm(float* __restrict__ C, int ldc, const float* __restrict__ A, int lda,
-                                          const float* __restrict__ B, int ldb, float alpha, int wave, int lane) {
-  constexpr int TM = M / 16, TN = N / 16;
-  const int li = lane & 15, lk = lane >> 4;
-#pragma unroll 1
-  for (int t = wave; t < TM * TN; t += LEAF_WAVES) {
-    const int ib = t / TN, jb = t % TN;
-    if (LOWER && jb > ib) continue;
-    // The whole contraction range, whatever KM says: the triangular operands hold zeros outside their triangle, and
-    // a loop whose bounds depend on the tile waits for the LDS once per step (the recursion is a chain of some thirty
-    // of these products, each as long as its slowest tile).  Here every operand of the tile is requested before
-    // the first matrix instruction is issued.
-    constexpr int KS = K / 4;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    const float* pa = A + (16 * ib + li) * lda + lk;
-    const float* pb = TB ? B + (16 * jb + li) * ldb + lk : B + lk * ldb + 16 * jb + li;
-    float av[KS], bv[KS];
+// Pivots 4 Q ... 4 Q + 3 of leaf_tile_inverse.
+template <int Q>
+__device__ __forceinline__ void leaf_tile_step(floatx4& a, floatx4& inv, floatx4& piv, int& bad, int g, int c) {
+  // the 4 x 4 block on the diagonal, in every lane: column i of its lower triangle sits in lane (Q, 4 Q + i)
+  float d[4][4];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      av[s] = pa[4 * s];
-      bv[s] = TB ? pb[4 * s] : pb[4 * s * ldb];
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r <= i; ++r) d[i][r] = lane_bcast(a[r], 16 * Q + 4 * Q + i);
+  float l[4][4], rec[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (!(d[k][k] > 0.f)) {                  // also catches NaN
+      if (bad == 0) bad = 4 * Q + k + 1;
+      d[k][k] = 1.f;
     }
+    float r = __builtin_amdgcn_rcpf(d[k][k]);             // hardware reciprocal, then one Newton step
+    r = __builtin_fmaf(__builtin_fmaf(-d[k][k], r, 1.f), r, r);
+    rec[k] = r;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) acc = mfma16(av[s], bv[s], acc);
-    float* pc = C + (16 * ib + 4 * lk) * ldc + 16 * jb + li;
+    for (int i = k + 1; i < 4; ++i) l[i][k] = d[i][k] * r;
+#pragma unroll
+    for (int i = k + 1; i < 4; ++i)
+#pragma unroll
+      for (int j = k + 1; j <= i; ++j) d[i][j] -= d[i][k] * l[j][k];
+  }
+  // x: the inverse of the unit lower triangle l
+  const float x10 = -l[1][0], x21 = -l[2][1], x32 = -l[3][2];
+  const float x20 = -l[2][0] - l[2][1] * x10, x31 = -l[3][1] - l[3][2] * x21;
+  const float x30 = -l[3][0] - l[3][1] * x10 - l[3][2] * x20;
+  // rows 4 Q + t of D L^T and of the unit inverse; meaningful in the lanes of row group Q, which hold those rows
+  floatx4 z, w;
+  z[0] = a[0];                                              w[0] = inv[0];
+  z[1] = a[1] + x10 * a[0];                                 w[1] = inv[1] + x10 * inv[0];
+  z[2] = a[2] + x21 * a[1] + x20 * a[0];                    w[2] = inv[2] + x21 * inv[1] + x20 * inv[0];
+  z[3] = a[3] + x32 * a[2] + x31 * a[1] + x30 * a[0];       w[3] = inv[3] + x32 * inv[2] + x31 * inv[1] + x30 * inv[0];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    inv[r] = g == Q ? w[r] : inv[r];
+    piv[r] = g == Q ? d[r][r] : piv[r];
+  }
+  if constexpr (Q < 3) {
+    const float zq = spread_row_group<Q>(z), wq = spread_row_group<Q>(w);     // lane (g, c): row 4 Q + g, column c
+    const float r = g < 2 ? (g == 0 ? rec[0] : rec[1]) : (g == 2 ? rec[2] : rec[3]);
+    const float lq = c >= 4 * Q + 4 ? -zq * r : 0.f;                           // -L[c][4 Q + g]; finished rows are left alone
+    a = mfma16(lq, zq, a);
+    inv = mfma16(lq, wq, inv);
+  }
+}
+
+// a: a symmetric 16 x 16 tile in the accumulator layout (only elements with column >= row are looked at), replaced by
+// L^-1 of its Cholesky factor (zeros above the diagonal).  Returns 0 or the 1-based index of the first non-positive
+// pivot.  L D L^T by blocks of 4 pivots: the 4 x 4 blocks are factored and inverted by every lane for itself (ten
+// lane reads and a chain of four reciprocals; no square root before the end), and the rank-4 updates of the tile and of
+// its inverse are one matrix instruction each.
+__device__ __forceinline__ int leaf_tile_inverse(floatx4& a, int lane) {
+  const int g = lane >> 4, c = lane & 15;
+  int bad = 0;
+  floatx4 inv, piv = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) inv[r] = 4 * g + r == c ? 1.f : 0.f;
+  leaf_tile_step<0>(a, inv, piv, bad, g, c);
+  leaf_tile_step<1>(a, inv, piv, bad, g, c);
+  leaf_tile_step<2>(a, inv, piv, bad, g, c);
+  leaf_tile_step<3>(a, inv, piv, bad, g, c);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float s = __builtin_amdgcn_rsqf(piv[r]);
+    s = __builtin_fmaf(0.5f * s, __builtin_fmaf(-piv[r] * s, s, 1.f), s);      // one Newton step
+    a[r] = inv[r] * s;
+  }
+  return bad;
+}
+
+// Tile of slot s of a wave: waves 0 ... 7 hold the diagonal tile of their own row in slot 0 and two tiles of the row above
+// (finished when they factor), waves 8 ... 15 five tiles each, spread over the rows.  row = 8: none.
+__device__ __forceinline__ void leaf_slot(int wave, int s, int& row, int& col) {
+  int t;
+  if (wave < 8) {
+    if (s == 0) { row = col = wave; return; }
+    row = s < 3 ? (wave + 7) & 7 : 8;
+    t = s - 1;
+  } else {
+    const int u = 8 * s + wave - 8;
+    row = u / 5;
+    t = 2 + u % 5;
+  }
+  col = t < row ? t : t + 1;
+}
+
+// The n x n block at `blk` (row stride ld, lower triangle) is replaced by the inverse of its Cholesky factor (zeros
+// above the diagonal).  Returns the 1-based index of the first non-positive pivot inside the block, or 0, to every
+// thread.  All 1024 threads of the work group call it.  (26 us for n = 128 as a recursion on an LDS-resident block that
+// handled 16 x 16 blocks one row per lane; 16.7 us in this form, launch included.)
+__device__ __forceinline__ int leaf_block(float* __restrict__ blk, int64_t ld, int n, LeafShared& sh, int tid) {
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int nb = (n + LT - 1) / LT;
+  const bool vec = (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(blk) & 15) == 0 && (n & 3) == 0;
+  int row[LEAF_SLOTS], col[LEAF_SLOTS];
+  floatx4 acc[LEAF_SLOTS];
+#pragma unroll
+  for (int s = 0; s < LEAF_SLOTS; ++s) {
+    leaf_slot(wave, s, row[s], col[s]);
+    if (row[s] >= nb || col[s] >= nb) row[s] = 8;
+    acc[s] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (row[s] < 8 && col[s] >= row[s]) {
+      // element (16 row + 4 g + r, 16 col + c) of U's side is element (16 col + c, 16 row + 4 g + r) of the lower triangle
+      const int i = LT * col[s] + c, j = LT * row[s] + 4 * g;
+      const float* src = blk + static_cast<int64_t>(i) * ld + j;
+      if (vec) {
+        if (i < n && j < n && j <= i) acc[s] = *reinterpret_cast<const floatx4*>(src);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (i < n && j + r <= i) acc[s][r] = src[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (i >= n) acc[s][r] = i == j + r ? 1.f : 0.f;      // identity padding
+        if (j + r > i) acc[s][r] = 0.f;
+      }
+    }
+  }
+  if (tid == 0) sh.bad = 0;
+#pragma unroll 1
+  for (int k = 0; k < nb; ++k) {
+    if (wave == k) {
+      __builtin_amdgcn_s_setprio(3);
+      const int bad = leaf_tile_inverse(acc[0], lane);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.inv[(4 * g + r) * LEAF_INV_LD + c] = acc[0][r];
+      if (bad != 0 && lane == 0 && sh.bad == 0) sh.bad = LT * k + bad;
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < LEAF_SLOTS; ++s) {
+      if (row[s] != k) continue;
+      if (col[s] != k) {
+        const floatx4 m = *reinterpret_cast<const floatx4*>(sh.inv + c * LEAF_INV_LD + 4 * g);
+        floatx4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p = mfma16(m[r], acc[s][r], p);
+        acc[s] = p;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.row[(4 * g + r) * LEAF_ROW_LD + LT * col[s] + c] = acc[s][r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < LEAF_SLOTS; ++s) {
+      if (row[s] > k && row[s] < 8 && (col[s] >= row[s] || col[s] <= k)) {
+        const float* pa = sh.row + 4 * g * LEAF_ROW_LD + LT * row[s] + c;
+        const float* pb = sh.row + 4 * g * LEAF_ROW_LD + LT * col[s] + c;
+        float av[4], bv[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          av[r] = -pa[r * LEAF_ROW_LD];
+          bv[r] = pb[r * LEAF_ROW_LD];
+        }
+        __builtin_amdgcn_sched_barrier(0);       // all eight reads before the first product: one wait, not one per step
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[s] = mfma16(av[r], bv[r], acc[s]);
+      }
+    }
+  }
+  // every element of the block was read before the first barrier released the last row of tiles that needed it
+#pragma unroll
+  for (int s = 0; s < LEAF_SLOTS; ++s) {
+    if (row[s] >= 8) continue;
+    const int j = LT * col[s] + c;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      if (ACC) pc[r * ldc] -= acc[r];
-      else pc[r * ldc] = alpha * acc[r];
+      const int i = LT * row[s] + 4 * g + r;
+      if (i < n && j < n) blk[static_cast<int64_t>(i) * ld + j] = col[s] > row[s] ? 0.f : acc[s][r];
     }
   }
-}
-
-// Factors the N x N block of Wm at (lo, lo) and leaves the inverse of its Cholesky factor in the lower triangle;
-// same recursion as the global one, on LDS operands.  t1: this level's slice of the T1 pool.
-template <int N>
-__device__ __forceinline__ void leaf_factor(float* __restrict__ Wm, int lo, float* __restrict__ t1,
-                                            float* __restrict__ t2, int* __restrict__ s_bad, int tid) {
-  const int wave = tid >> 6, lane = tid & 63;
-  if constexpr (N == PB) {
-    if (wave == 0) {
-      float a[PB], m[PB];
-      // every lane reads a whole row (the lanes beyond the block re-read its last one) with four 16-byte loads that
-      // are all in flight together; a load under a per-element condition would be waited for on its own
-      const floatx4* row = reinterpret_cast<const floatx4*>(Wm + (lo + (lane < PB ? lane : PB - 1)) * LLD + lo);
-      floatx4 q[PB / 4];
-#pragma unroll
-      for (int c = 0; c < PB / 4; ++c) q[c] = row[c];
-#pragma unroll
-      for (int j = 0; j < PB; ++j) a[j] = (lane < PB && j <= lane) ? q[j >> 2][j & 3] : ((j == lane) ? 1.f : 0.f);
-      const int bad = small_chol_inv(a, m, lane);
-      if (lane < PB) {
-        floatx4* dst = reinterpret_cast<floatx4*>(Wm + (lo + lane) * LLD + lo);
-#pragma unroll
-        for (int c = 0; c < PB / 4; ++c) {
-          const floatx4 w = {m[4 * c], m[4 * c + 1], m[4 * c + 2], m[4 * c + 3]};     // zeros above the diagonal
-          dst[c] = w;
-        }
-      }
-      if (lane == 0 && bad != 0 && *s_bad == 0) *s_bad = lo + bad;
-    }
-    __syncthreads();
-  } else {
-    constexpr int H = N / 2;
-    leaf_factor<H>(Wm, lo, t1, t2, s_bad, tid);
-    float* W11 = Wm + lo * LLD + lo;
-    float* W21 = Wm + (lo + H) * LLD + lo;
-    float* W22 = Wm + (lo + H) * LLD + lo + H;
-    leaf_gemm<H, H, H, true, false, false, LK_LE_J>(t1, T1_LD, W21, LLD, W11, LLD, 1.f, wave, lane);   // T1 = A21 M11^T
-    __syncthreads();
-    leaf_gemm<H, H, H, true, true, true, LK_FULL>(W22, LLD, t1, T1_LD, t1, T1_LD, 1.f, wave, lane);    // A22 -= T1 T1^T
-    __syncthreads();
-    leaf_factor<H>(Wm, lo + H, t1 + H * T1_LD, t2, s_bad, tid);
-    leaf_gemm<H, H, H, false, false, false, LK_GE_J>(t2, T1_LD, t1, T1_LD, W11, LLD, 1.f, wave, lane); // T2 = T1 M11
-    __syncthreads();
-    leaf_gemm<H, H, H, false, false, false, LK_LE_I>(W21, LLD, W22, LLD, t2, T1_LD, -1.f, wave, lane); // M21 = -M22 T2
-    __syncthreads();
-  }
-}
-
-
-// Loads the n x n block at `blk` (row stride ld), padded with an identity to npad in {16, 32, 64, 128}, factors it
-// in the LDS and writes L^-1 back (lower triangle, zeros above the diagonal).  Returns in *s_bad the 1-based index
-// of the first non-positive pivot inside the block, or 0.  All 1024 threads of the work group call it.
-__device__ __forceinline__ void leaf_block(float* __restrict__ blk, int64_t ld, int n, float* leaf_smem, int tid) {
-  float* Wm = leaf_smem;
-  float* t1 = leaf_smem + LEAF * LLD;
-  float* t2 = t1 + LEAF_T1_FLOATS;
-  int* s_bad = reinterpret_cast<int*>(t2 + LEAF_T2_FLOATS);
-  const int npad = n <= 16 ? 16 : (n <= 32 ? 32 : (n <= 64 ? 64 : 128));
-  {
-    // all of this thread's elements are requested before the first one is stored: a load and its store per turn
-    // would pay the latency of the device memory sixteen times over
-    constexpr int ROWS_PER_TURN = LEAF_THREADS / 128, TURNS = LEAF / ROWS_PER_TURN;
-    const int j = tid & 127;
-    float v[TURNS];
-#pragma unroll
-    for (int t = 0; t < TURNS; ++t) {
-      const int i = (tid >> 7) + ROWS_PER_TURN * t;
-      v[t] = (i == j) ? 1.f : 0.f;                 // identity padding beyond n
-      if (i < n && j < n) v[t] = (j <= i) ? blk[static_cast<int64_t>(i) * ld + j] : 0.f;
-    }
-#pragma unroll
-    for (int t = 0; t < TURNS; ++t) {
-      const int i = (tid >> 7) + ROWS_PER_TURN * t;
-      if (i < npad && j < npad) Wm[i * LLD + j] = v[t];
-    }
-  }
-  if (tid == 0) *s_bad = 0;
-  __syncthreads();
-  if (npad == 16) leaf_factor<16>(Wm, 0, t1, t2, s_bad, tid);
-  else if (npad == 32) leaf_factor<32>(Wm, 0, t1, t2, s_bad, tid);
-  else if (npad == 64) leaf_factor<64>(Wm, 0, t1, t2, s_bad, tid);
-  else leaf_factor<128>(Wm, 0, t1, t2, s_bad, tid);
-  for (int i = tid >> 7; i < n; i += LEAF_THREADS / 128) {
-    const int j = tid & 127;
-    if (j < n) blk[static_cast<int64_t>(i) * ld + j] = (j <= i) ? Wm[i * LLD + j] : 0.f;
-  }
-}
-
-__device__ __forceinline__ int leaf_bad_pivot(const float* leaf_smem) {
-  return *reinterpret_cast<const int*>(leaf_smem + LEAF * LLD + LEAF_T1_FLOATS + LEAF_T2_FLOATS);
+  return sh.bad;
 }
 
 }  // namespace ak

@@ -609,6 +609,23 @@ def test_chol_inv_grouped_mixed_sizes_match_oracle(K):
         assert torch.equal(out, out.T), d
 
 
+@pytest.mark.parametrize('d', [3, 15, 16, 17, 31, 33, 48, 100, 127, 129, 260])
+def test_chol_inv_at_the_edges_of_the_leaf_tiles(K, d):
+    """Diagonal blocks that end inside, at and behind a 16 x 16 tile, both entry points, against fp64; and the first
+    non-positive pivot on either side of every tile boundary of the block."""
+    A, lam = _spd(d, 300 + d), 0.05
+    ref = torch.linalg.inv(A.double() + lam * torch.eye(d, dtype=torch.float64))
+    lam_dev = torch.tensor([lam], device='cuda')
+    for call in (K.chol_inv_batched, K.chol_inv_grouped):
+        out = torch.empty(d, d, device='cuda')
+        assert int(call([A.cuda()], [out], lam_dev).cpu()) == 0
+        assert relerr(out, ref) < 2e-6, (call.__name__, relerr(out, ref))
+        for bad in sorted({1, 4, 5, 16, 17, d} & set(range(1, d + 1))):
+            B = A.clone()
+            B[bad - 1, bad - 1] = -5.0
+            assert int(call([B.cuda()], [out], lam_dev).cpu()) == bad, (call.__name__, bad)
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
