@@ -12,8 +12,8 @@
 // The per-matrix sequences of steps (leaf | products) of ALL matrices are merged into one sequence of "super-steps":
 // super-step s holds, for every matrix whose next step has the type chosen for s, that step.  One launch per
 // super-step: a grouped leaf launch (one work group per diagonal block) or a grouped product launch (one work group
-// per 128 x 128 tile of any product of the step, split-operand MFMA tile of gemm_x3.hpp, descriptor found through a
-// tile -> product map).  The longest chain (the largest matrix) sets the number of launches; the work of all smaller
+// per tile of any product of the step, descriptor found through a tile -> product map; 128 x 128 split-operand MFMA tiles of
+// gemm_x3.hpp, or the smaller fp32 tiles of gemm_deep.hpp where those would leave the device idle: cg_prefer_deep).  The longest chain (the largest matrix) sets the number of launches; the work of all smaller
 // matrices runs in the shadow of its steps.  ResNet-50 (108 factors, 13 sizes): 121 launches.
 //
 // The plan (descriptor tables, launch sequence) depends on the sizes only; every address in it is an offset into the
@@ -32,8 +32,8 @@
 namespace ak {
 
 constexpr int64_t CG_MAGIC = 0x3247524c4f4843ll;     // "CHOLGR2"
-constexpr int CG_COPY = 0, CG_LEAF = 1, CG_PROD = 2;
-constexpr int CG_FLAG_TRANSA = 1, CG_FLAG_TRANSB = 2, CG_FLAG_OUT_USER = 4;
+constexpr int CG_COPY = 0, CG_LEAF = 1, CG_PROD = 2, CG_PROD_DEEP = 3;
+constexpr int CG_FLAG_TRANSA = 1, CG_FLAG_TRANSB = 2, CG_FLAG_OUT_USER = 4, CG_FLAG_PANEL = 8;
 // What an operand of a product holds, for the fp16-piece products (bits 4-5 of CgProd::flags: A, bits 6-7: B).  With
 // a = the largest diagonal element of A + lam I, every element is bounded in magnitude: a block of the (updated)
 // matrix by a, of its Cholesky factor L by sqrt(a), of M = L^-1 by 1 / sqrt(lam), of L21 L11^-1 by sqrt(a / lam).
@@ -267,6 +267,31 @@ static __global__ __launch_bounds__(256) void cg_prod_kernel(CgArgs a, const CgP
   }
 }
 
+// The same for the steps whose 128 x 128 tiles would leave most of the device idle: deep fp32 tiles (gemm_deep.hpp) of
+// 64 x 64, or of 32 x 128 for a panel, which is formed in place and whose work groups have to own whole rows.
+static __global__ __launch_bounds__(256) void cg_prod_deep_kernel(CgArgs a, const CgProd* __restrict__ prods,
+                                                                  const int32_t* __restrict__ tile_map) {
+  constexpr int kSquare = deep_lds_floats<64, 64, 128>(), kPanel = deep_lds_floats<32, 128, 64>();
+  __shared__ __attribute__((aligned(16))) float lds[kSquare > kPanel ? kSquare : kPanel];
+  const int w = blockIdx.x;
+  const CgProd d = prods[tile_map[w]];
+  if ((d.flags & CG_FLAG_OUT_USER) && cg_skipped(a, d.mat)) return;
+  int ti, tj;
+  cg_decode_tile(d, w - d.first_tile, ti, tj);
+  GemmParams p;
+  p.A = a.ws + d.a_off;
+  p.B = a.ws + d.b_off;
+  p.C = (d.flags & CG_FLAG_OUT_USER) ? a.out_list[d.mat] : a.ws + d.c_off;
+  p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
+  p.M = d.M; p.N = d.N; p.K = d.K;
+  p.transA = (d.flags & CG_FLAG_TRANSA) ? 1 : 0;
+  p.transB = (d.flags & CG_FLAG_TRANSB) ? 1 : 0;
+  p.alpha = d.alpha; p.beta = d.beta;
+  p.kmode = d.kmode; p.tile_mode = d.tile_mode;
+  if (d.flags & CG_FLAG_PANEL) gemm_deep_tile<32, 128, 64>(p, ti, tj, 0, lds);
+  else gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
+}
+
 // ---- host: the plan ------------------------------------------------------------------------------------------
 
 struct CgOp {                 // one step of one matrix's own sequence
@@ -290,8 +315,32 @@ static int64_t cg_pool(int64_t n) {
 static inline int64_t cg_align64(int64_t x) { return (x + 63) / 64 * 64; }
 
 static int64_t cg_tiles(const CgProd& p) {
-  const int64_t tm = (p.M + 127) / 128, tn = (p.N + 127) / 128;
-  return p.tile_mode == TILE_ALL ? tm * tn : tm * (tm + 1) / 2;
+  return p.tile_mode == TILE_ALL ? static_cast<int64_t>(p.tiles_m) * p.tiles_n
+                                 : static_cast<int64_t>(p.tiles_m) * (p.tiles_m + 1) / 2;
+}
+
+// Tiles of the deep kernel instead of 128 x 128.
+static void cg_make_deep(CgProd& p) {
+  const int bm = (p.flags & CG_FLAG_PANEL) ? 32 : 64, bn = (p.flags & CG_FLAG_PANEL) ? 128 : 64;
+  p.tiles_m = (p.M + bm - 1) / bm;
+  p.tiles_n = (p.N + bn - 1) / bn;
+}
+
+// Which kernel a super-step's products take.  The split kernel's 128 x 128 tiles have three times the rate once they
+// fill the device (about 1 us per k-tile of 32 and CU), but a tile takes 1.6 us per k-tile however few there are; the
+// deep tiles take 2 us per chunk of 128 k.  The step is as long as its longest tile or as its work spread over the CUs.
+static bool cg_prefer_deep(const std::vector<CgProd>& ps) {
+  double chunk_max = 0, chunks = 0, ktile_max = 0, ktiles = 0;
+  for (const CgProd& p : ps) {
+    CgProd q = p;
+    cg_make_deep(q);
+    const double c = (p.K + 127) / 128, k = (p.K + 31) / 32;
+    chunk_max = std::max(chunk_max, c);
+    ktile_max = std::max(ktile_max, k);
+    chunks += c * static_cast<double>(cg_tiles(q));
+    ktiles += k * static_cast<double>(cg_tiles(p));
+  }
+  return 2.0 * std::max(chunk_max, chunks / 256) < std::max(1.6 * ktile_max, 1.05 * ktiles / 256);
 }
 
 static CgProd cg_prod(int mat, int flags, int kind_a, int kind_b, int M, int N, int K, float alpha, int64_t a, int lda,
@@ -343,7 +392,7 @@ static void cg_right_looking(std::vector<CgOp>& ops, int mat, int64_t w, int d, 
       auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
       CgOp panel, update;
       panel.type = update.type = CG_PROD;
-      panel.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB, CG_KIND_W, CG_KIND_M, below, n, n, 1.f, at(lo + n, lo), dp,
+      panel.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB | CG_FLAG_PANEL, CG_KIND_W, CG_KIND_M, below, n, n, 1.f, at(lo + n, lo), dp,
                                     at(lo, lo), dp, 0.f, at(lo + n, lo), dp, K_LE_J, TILE_ALL));
       ops.push_back(panel);
       const int next = lo + n;
@@ -451,6 +500,10 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
           for (const CgProd& p : seq[m][cur[m]].prods) ps.push_back(p);
           ++cur[m];
         }
+      if (cg_prefer_deep(ps)) {
+        st.type = CG_PROD_DEEP;
+        for (CgProd& p : ps) cg_make_deep(p);
+      }
       // longest contraction first: the long tiles start early, the short ones fill the tail
       std::stable_sort(ps.begin(), ps.end(), [](const CgProd& x, const CgProd& y) { return x.K > y.K; });
       int64_t tiles = 0;
@@ -565,7 +618,7 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
       hipLaunchKernelGGL(cg_leaf_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, a,
                          reinterpret_cast<const CgLeafTask*>(a.plan + h->leaves_off) + st.first);
     else
-      hipLaunchKernelGGL(cg_prod_kernel, dim3(st.grid), dim3(256), 0, s, a,
+      hipLaunchKernelGGL(st.type == CG_PROD ? cg_prod_kernel : cg_prod_deep_kernel, dim3(st.grid), dim3(256), 0, s, a,
                          reinterpret_cast<const CgProd*>(a.plan + h->prods_off) + st.first,
                          reinterpret_cast<const int32_t*>(a.plan + h->map_off) + st.first_tile);
   }

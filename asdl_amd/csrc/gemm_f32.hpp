@@ -272,6 +272,7 @@ static __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
 
 }  // namespace ak
 
+#include "gemm_deep.hpp"
 #include "gemm_x3.hpp"
 
 namespace ak {
@@ -279,10 +280,10 @@ namespace ak {
 // Constants of the product library; variables that a setter can change only in tuning builds (-DAK_TUNING_HOOKS).
 #ifdef AK_TUNING_HOOKS
 inline int g_x3_double_buffer = 1;
-inline int g_x3_min_groups = 100, g_x3_min_k = 256;
+inline int g_x3_min_groups = 192, g_x3_min_k = 256;
 #else
 constexpr int g_x3_double_buffer = 1;
-constexpr int g_x3_min_groups = 100, g_x3_min_k = 256;
+constexpr int g_x3_min_groups = 192, g_x3_min_k = 256;
 #endif
 
 inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
@@ -290,8 +291,8 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
   const int64_t tiles128 = static_cast<int64_t>((p.N + 127) / 128) * ((p.M + 127) / 128) * batch;
   const bool lower = p.tile_mode != TILE_ALL;
   const int64_t work_groups = lower ? tiles128 / 2 : tiles128;
-  // The split kernel (128 x 128 tiles, a pipeline that needs a few k-tiles to fill) pays off once its tiles
-  // fill most of the device; below that the 64 x 64 tiles of the fp32 kernel spread the work better.
+  // The split kernel (128 x 128 tiles) has twice the rate of fp32 tiles once its tiles fill most of the device (2048^3, one
+  // tile per CU: 96 us against 128); below that the deep 64 x 64 tiles spread the work better (1024^3: 20 us against 50).
   if (p.split >= 2 && work_groups >= g_x3_min_groups && p.K >= g_x3_min_k && gemm_x3_ok(p)) {
     dim3 grid((p.N + 127) / 128, (p.M + 127) / 128, batch);
     GemmParams q = p;
@@ -315,15 +316,14 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
     }
     return check_launch();
   }
-  // 128 x 128 tiles when they alone fill the 256 CUs twice over, else 64 x 64 tiles (four times the work groups)
+  // 128 x 128 tiles when they alone fill the 256 CUs twice over, else the deep 64 x 64 tiles (four times the work groups)
   if (work_groups >= 512) {
     dim3 grid((p.N + 127) / 128, (p.M + 127) / 128, batch);
     if (p.chunked) hipLaunchKernelGGL((gemm_f32_kernel<2, true>), grid, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL(gemm_f32_kernel<2>, grid, dim3(256), 0, stream, p);
   } else {
     dim3 grid((p.N + 63) / 64, (p.M + 63) / 64, batch);
-    if (p.chunked) hipLaunchKernelGGL((gemm_f32_kernel<1, true>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(gemm_f32_kernel<1>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(gemm_deep_kernel, grid, dim3(256), 0, stream, p);
   }
   return check_launch();
 }

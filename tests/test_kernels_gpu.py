@@ -739,6 +739,28 @@ def test_gemm_matches_fp64(K, tA, tB, M, N, K_):
     assert relerr(out, ref) < 1e-5
 
 
+@pytest.mark.parametrize('tA', [False, True])
+@pytest.mark.parametrize('tB', [False, True])
+@pytest.mark.parametrize('M,N,K_', [(1, 1, 1), (64, 64, 128), (63, 65, 127), (66, 62, 129), (33, 130, 257)])
+def test_gemm_at_the_edges_of_the_deep_tiles(K, tA, tB, M, N, K_):
+    """Tiles of 64 x 64 and chunks of 128 k that end before, at and behind a boundary; rows of an odd stride (loads of 16
+    bytes at 4-byte alignment)."""
+    g = torch.Generator().manual_seed(7 * M + N + K_)
+
+    def rows(r, c):
+        return torch.randn(r, c + 3, generator=g)[:, 1:1 + c]
+    A = rows(K_, M) if tA else rows(M, K_)
+    B = rows(N, K_) if tB else rows(K_, N)
+    ref = (A.double().T if tA else A.double()) @ (B.double().T if tB else B.double())
+    wide = [torch.zeros(t.shape[0], t.shape[1] + 3, device='cuda') for t in (A, B)]
+    views = []
+    for w, t in zip(wide, (A, B)):
+        v = w[:, 1:1 + t.shape[1]]
+        v.copy_(t)
+        views.append(v)
+    assert relerr(K.gemm(views[0], views[1], transA=tA, transB=tB), ref) < 2e-6
+
+
 @pytest.mark.parametrize('pieces,tol', [(3, 2e-6), (2, 3e-5)])
 @pytest.mark.parametrize('tA', [False, True])
 @pytest.mark.parametrize('tB', [False, True])
