@@ -84,7 +84,8 @@ template <int BM, int BN, int KC>
 constexpr int deep_lds_floats() { return DeepPanel<BM, KC>::FLOATS + DeepPanel<BN, KC>::FLOATS; }
 
 // One BM x BN tile (ti, tj) of batch entry z of the product described by p; lds: deep_lds_floats() floats.  The sum is
-// always a chunked one (GemmParams::chunked).
+// always taken in chunks: a fresh accumulator for every KC of the contraction, added to a running total.  The rounding
+// error of a long sum stays near that of one rounding instead of growing with the number of matrix instructions.
 template <int BM, int BN, int KC>
 __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int tj, int z, float* lds) {
   static_assert((BM / 32) * (BN / 32) == 4, "four waves");
@@ -148,8 +149,9 @@ __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int 
     }
   }
 
-  const bool lower_only = (p.tile_mode == TILE_LOWER);
-  const bool mirror = (p.tile_mode == TILE_LOWER_MIRROR) && i0 != j0;
+  // mirrored results are exactly symmetric: a tile on the diagonal keeps its lower triangle and mirrors it as well
+  const bool lower_only = p.tile_mode != TILE_ALL;
+  const bool mirror = p.tile_mode == TILE_LOWER_MIRROR;
   float* __restrict__ C2 = p.C2 != nullptr ? p.C2 + static_cast<int64_t>(z) * p.sC2 : nullptr;
   float vmax = 0.f;
   const int gj = j0 + 32 * wc + l32;
@@ -183,16 +185,16 @@ __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int 
         const int gi = gi0 + 8 * q;
         const floatx4 v = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
         float* dst = C + static_cast<int64_t>(gj) * p.ldc + gi;
-        if (gi + 4 <= p.M) *reinterpret_cast<floatx4u*>(dst) = v;
+        if (gi > gj && gi + 4 <= p.M) *reinterpret_cast<floatx4u*>(dst) = v;
         else
 #pragma unroll
-          for (int e = 0; e < 3; ++e)
-            if (gi + e < p.M) dst[e] = v[e];
+          for (int e = 0; e < 4; ++e)
+            if (gi + e > gj && gi + e < p.M) dst[e] = v[e];
         if (C2 != nullptr) {
           float* dst2 = C2 + static_cast<int64_t>(gj) * p.ldc2 + gi;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (gi + e < p.M) dst2[e] = p.c2_scale * v[e];
+            if (gi + e > gj && gi + e < p.M) dst2[e] = p.c2_scale * v[e];
         }
       }
     }

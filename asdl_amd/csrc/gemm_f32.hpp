@@ -39,15 +39,12 @@ struct GemmParams {
   const int* active = nullptr;        // optional per-batch flags: batch z runs only if active[z*active_stride] != 0
   int active_stride = 0;
   int split = 0;                      // 0: fp32 MFMA; 2 / 3: bf16 MFMA on operands split into that many bf16 pieces (gemm_x3.hpp)
-  int chunked = 0;                    // non-zero: the contraction is summed in chunks (a fresh accumulator every 128 / 256 k, added
-                                      // to a running total), which keeps the rounding error of a long sum near that of one
-                                      // rounding instead of growing with the number of matrix instructions (fp32 kernel, and the
-                                      // three-piece kernel for untransposed operands; ignored elsewhere)
   float scaleA = 1.f, scaleB = 1.f;   // fp16-piece variant only: powers of two the operands are multiplied by before the split
   float* absmax_out = nullptr;        // optional: the largest |C| of the result (of batch entry z: absmax_out[z * absmax_stride]) is
   int64_t absmax_stride = 0;          // folded into this word with an integer atomic maximum on its bit pattern (the caller
   int absmax_identity = 0;            // zeroes it first).  absmax_identity: the largest |C - I| instead, and a NaN in C ends up
-                                      // in the word (as torch.max would return it) instead of being skipped
+                                      // in the word (as torch.max would return it) instead of being skipped (split and deep tiles
+                                      // only, as C2)
   float* C2 = nullptr;                // optional second result, same shape and batch layout as C with its own strides:
   int64_t ldc2 = 0, sC2 = 0;          // C2 = c2_scale * C + c2_diag * I (the next iterate's polynomial of a Newton iteration,
   float c2_scale = 0.f, c2_diag = 0.f;   // written while C is still in registers)
@@ -131,14 +128,14 @@ __device__ __forceinline__ void gemm_store_absmax(float* out, float vmax, int la
     vmax = (other > vmax || other != other) ? other : vmax;
   }
   vmax = fabsf(vmax);       // (a NaN of either sign: the pattern without the sign bit)
-  if (lane == 0) atomicMax(reinterpret_cast<unsigned int*>(out), __builtin_bit_cast(unsigned int, vmax));
+  // (most waves find a larger value there already and spare the word, which hundreds of them share, an atomic)
+  unsigned int* word = reinterpret_cast<unsigned int*>(out);
+  const unsigned int bits = __builtin_bit_cast(unsigned int, vmax);
+  if (lane == 0 && __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < bits) atomicMax(word, bits);
 }
 
 // One BT x BT tile (ti, tj) of batch entry z of the product described by p; lds: [2][2][PANEL] floats.
-// CHUNKED: every 8 k-tiles (128 k) the accumulators are added to a running total and start again from zero: the
-// matrix instruction rounds its accumulator once per two k, so a contraction over K rounds K/2 times at the full
-// magnitude of the sum; in chunks, 64 roundings happen at the magnitude of one chunk and K/128 at the full one.
-template <int TI, bool CHUNKED = false>
+template <int TI>
 __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int tj, int z,
                                               float (*lds)[2][GemmTile<64 * TI>::PANEL]) {
   constexpr int BT = 64 * TI;
@@ -170,16 +167,6 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int t
     for (int b = 0; b < TI; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-  constexpr int TT = CHUNKED ? TI : 1;
-  floatx16 tot[TT][TT];
-  if constexpr (CHUNKED) {
-#pragma unroll
-    for (int a = 0; a < TI; ++a)
-#pragma unroll
-      for (int b = 0; b < TI; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tot[a][b][r] = 0.f;
-  }
 
   const int nk = kbeg < kend ? (kend - kbeg + GBK - 1) / GBK : 0;
   floatx4 ra[GemmTile<BT>::CHUNKS], rb[GemmTile<BT>::CHUNKS];
@@ -208,16 +195,6 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int t
       for (int a = 0; a < TI; ++a)
 #pragma unroll
         for (int b = 0; b < TI; ++b) acc[a][b] = mfma_f32(fa[a][m], fb[b][m], acc[a][b]);
-    if constexpr (CHUNKED) {
-      if ((kt & 7) == 7) {
-#pragma unroll
-        for (int a = 0; a < TI; ++a)
-#pragma unroll
-          for (int b = 0; b < TI; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) { tot[a][b][r] += acc[a][b][r]; acc[a][b][r] = 0.f; }
-      }
-    }
     if (kt + 1 < nk) {
       gemm_stash<BT>(ra, lds[buf ^ 1][0], a_kc, tid);
       gemm_stash<BT>(rb, lds[buf ^ 1][1], b_kc, tid);
@@ -225,17 +202,8 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int t
     __syncthreads();
   }
 
-  if constexpr (CHUNKED) {
-#pragma unroll
-    for (int a = 0; a < TI; ++a)
-#pragma unroll
-      for (int b = 0; b < TI; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] += tot[a][b][r];
-  }
   const bool lower_only = (p.tile_mode == TILE_LOWER);
   const bool mirror = (p.tile_mode == TILE_LOWER_MIRROR) && (ti != tj);
-  float* __restrict__ C2 = p.C2 != nullptr ? p.C2 + static_cast<int64_t>(z) * p.sC2 : nullptr;
   float vmax = 0.f;
 #pragma unroll
   for (int a = 0; a < TI; ++a)
@@ -253,21 +221,16 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int t
         if (p.beta != 0.f) v += p.beta * *dst;
         *dst = v;
         if (mirror) C[static_cast<int64_t>(gj) * p.ldc + gi] = v;
-        vmax = gemm_fold_absmax(vmax, v, gi == gj, p.absmax_identity);
-        if (C2 != nullptr) {
-          const float w = p.c2_scale * v + (gi == gj ? p.c2_diag : 0.f);
-          C2[static_cast<int64_t>(gi) * p.ldc2 + gj] = w;
-          if (mirror) C2[static_cast<int64_t>(gj) * p.ldc2 + gi] = w;
-        }
+        vmax = fmaxf(vmax, fabsf(v));
       }
     }
   if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out + static_cast<int64_t>(z) * p.absmax_stride, vmax, lane);
 }
 
-template <int TI, bool CHUNKED = false>
+template <int TI>
 static __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float lds[2][2][GemmTile<64 * TI>::PANEL];
-  gemm_f32_tile<TI, CHUNKED>(p, blockIdx.y, blockIdx.x, blockIdx.z, lds);
+  gemm_f32_tile<TI>(p, blockIdx.y, blockIdx.x, blockIdx.z, lds);
 }
 
 }  // namespace ak
@@ -305,7 +268,6 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
     // hand), one instantiation per pair of operand layouts; two pieces: the single-buffered loop
     if (p.split == 3 && g_x3_double_buffer) {
       if (p.transA == 0 && p.transB != 0) hipLaunchKernelGGL((gemm_x3_kernel<3, true, 1, 1>), grid, dim3(256), 0, stream, q);
-      else if (p.transA == 0 && p.chunked) hipLaunchKernelGGL((gemm_x3_kernel<3, true, 1, 0, true>), grid, dim3(256), 0, stream, q);
       else if (p.transA == 0) hipLaunchKernelGGL((gemm_x3_kernel<3, true, 1, 0>), grid, dim3(256), 0, stream, q);
       else if (p.transB != 0) hipLaunchKernelGGL((gemm_x3_kernel<3, true, 0, 1>), grid, dim3(256), 0, stream, q);
       else hipLaunchKernelGGL((gemm_x3_kernel<3, true, 0, 0>), grid, dim3(256), 0, stream, q);
@@ -319,8 +281,7 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
   // 128 x 128 tiles when they alone fill the 256 CUs twice over, else the deep 64 x 64 tiles (four times the work groups)
   if (work_groups >= 512) {
     dim3 grid((p.N + 127) / 128, (p.M + 127) / 128, batch);
-    if (p.chunked) hipLaunchKernelGGL((gemm_f32_kernel<2, true>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(gemm_f32_kernel<2>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(gemm_f32_kernel<2>, grid, dim3(256), 0, stream, p);
   } else {
     dim3 grid((p.N + 63) / 64, (p.M + 63) / 64, batch);
     hipLaunchKernelGGL(gemm_deep_kernel, grid, dim3(256), 0, stream, p);

@@ -31,23 +31,34 @@
 
 namespace ak {
 
-constexpr int kPlaneTile = 192;
+constexpr int kPlaneTile = 192, kPlaneSmallTile = 64;
+constexpr int kErrStride = 16;          // floats between error words: a cache line each, all tiles of all matrices fold into theirs at once
 constexpr int kPlaneLdsBytes = 4 * 6 * 6 * 16 * 64;      // four stages of six plane panels of six [16 rows][64 bytes] blocks
 constexpr int kPlaneMaxDim = 16128;      // 32-bit byte offsets inside a plane set, virtual k-tile numbers below 2^15
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
+// Number of a matrix buffer of an iteration: plain, or one of a pair (k, k + 1) of which an iteration reads one and writes the
+// other; which one is decided on the device by the parity of the matrix's own step count.
+struct PairedBuf {
+  int16_t index, sel;       // sel 0: plain; 1: the one an iteration reads; 2: the one it writes
+};
+__device__ __forceinline__ int paired_buf(PairedBuf b, int parity) {
+  return b.index + (b.sel == 0 ? 0 : (b.sel == 1 ? parity : parity ^ 1));
+}
+
 struct PlaneGemm {
-  const __bf16* A;          // plane set of batch entry z at A + z * set_elems (plane q: + q * plane_elems)
-  const __bf16* B;
-  __bf16* C;
-  __bf16* C2;               // optional
-  float* errword;           // optional, one word per batch entry
-  const int* active;        // optional: entry z runs only if active[z] != 0
-  int* overflow;            // optional, fp16 form: word z is set when a value of C or C2 does not fit the fp16 range
-  int64_t sA, sB, sC, sC2;  // elements between the plane sets of consecutive batch entries
+  __bf16* bufs;             // buffer i, plane set of batch entry z: bufs + i * buf_elems + z * set_elems (plane q: + q * plane_elems)
+  int64_t buf_elems, set_elems;
+  PairedBuf A, B, C, C2;    // C2.index < 0: no second result
+  const int* count;         // steps taken by each batch entry (the parity of its paired buffers)
+  const float* coef;        // C2 = coef[2 (count + 1)] I - coef[2 (count + 1) + 1] C of the entry's own table
+  int64_t coef_stride;
+  int coef_last;            // steps beyond the table take its last entry
+  float* errword;           // optional, one word per batch entry, kErrStride apart
+  const int* active;        // entry z runs only if active[z] != 0
+  int* overflow;            // fp16 form: word z is set when a value of C or C2 does not fit the fp16 range
   int64_t plane_elems;      // n_pad * n_pad
-  int n, n_pad, T;          // T = n_pad / kPlaneTile
-  float c2_scale, c2_diag;
+  int n, n_pad, T;          // T = n_pad / tile
   // fp16 form only (powers of two): 1 / (scale of A's planes * scale of B's), scale of C's planes, scale of C2's
   float in_unscale, c_scale, c2_plane_scale;
 };
@@ -80,20 +91,29 @@ __device__ __forceinline__ void plane_bits(float x, unsigned short (&o)[3]) {
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
 // Epilogue of a tile: planes of C (and of C2 = c2_scale C + c2_diag I), the mirror image of an off-diagonal tile, the
-// error word max |C - I|.  sum(a, b, r): the tile's sums in the accumulator layout of the 2 x 2 waves with 3 x 3 blocks each.
-template <int NP, class Sum>
+// error word max |C - I|.  sum(a, b, r): the tile's sums in the accumulator layout of the 2 x 2 waves with FR x FR blocks each.
+template <int NP, int FR, class Sum>
 __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int tj, int z, Sum sum) {
-  constexpr int FR = 3, FC = 3, WC = 2;
+  constexpr int FC = FR, WC = 2, TILE = 64 * FR;
+  static_assert(FR == 1 || FR == 3, "blocks are named below");
   // (the empty statement keeps the address arithmetic below from being moved above the k-loop of the caller, where
   // every register is taken)
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
+  asm volatile("" : "+s"(z));
   const int lane = tid & 63, wave = tid >> 6;
   const int wr = wave / WC, wc = wave % WC, g = lane >> 5, l32 = lane & 31;
-  const int i0 = ti * kPlaneTile, j0 = tj * kPlaneTile;
-  unsigned short* __restrict__ C = reinterpret_cast<unsigned short*>(p.C) + static_cast<int64_t>(z) * p.sC;
-  unsigned short* __restrict__ C2 =
-      p.C2 != nullptr ? reinterpret_cast<unsigned short*>(p.C2) + static_cast<int64_t>(z) * p.sC2 : nullptr;
+  const int i0 = ti * TILE, j0 = tj * TILE;
+  const int steps = p.count[z], parity = steps & 1;
+  unsigned short* __restrict__ sets = reinterpret_cast<unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
+  unsigned short* __restrict__ C = sets + paired_buf(p.C, parity) * p.buf_elems;
+  unsigned short* __restrict__ C2 = p.C2.index >= 0 ? sets + paired_buf(p.C2, parity) * p.buf_elems : nullptr;
+  float c2_diag = 0.f, c2_scale = 0.f;
+  if (C2 != nullptr) {
+    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
+    c2_diag = next[0];
+    c2_scale = -next[1];
+  }
   const bool off_diag = ti != tj;
   const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
   float vmax = 0.f;
@@ -128,7 +148,7 @@ __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int t
             m1[s][e] = o[s];
           }
           if (C2 != nullptr) {
-            const float w = p.c2_scale * v + ((diagonal && inside) ? p.c2_diag : 0.f);
+            const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
             if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
             plane_bits<NP>(w * c2s, o);
 #pragma unroll
@@ -153,11 +173,14 @@ __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int t
   using J0 = std::integral_constant<int, 0>;
   using J1 = std::integral_constant<int, 1>;
   using J2 = std::integral_constant<int, 2>;
-  block(J0{}, J0{}); block(J0{}, J1{}); block(J0{}, J2{});
-  block(J1{}, J0{}); block(J1{}, J1{}); block(J1{}, J2{});
-  block(J2{}, J0{}); block(J2{}, J1{}); block(J2{}, J2{});
-  if (p.errword != nullptr) gemm_store_absmax(p.errword + z, vmax, lane);
-  if (NP == 2 && p.overflow != nullptr && !fits) atomicOr(p.overflow + z, 1);
+  block(J0{}, J0{});
+  if constexpr (FR == 3) {
+    block(J0{}, J1{}); block(J0{}, J2{});
+    block(J1{}, J0{}); block(J1{}, J1{}); block(J1{}, J2{});
+    block(J2{}, J0{}); block(J2{}, J1{}); block(J2{}, J2{});
+  }
+  if (p.errword != nullptr) gemm_store_absmax(p.errword + static_cast<int64_t>(z) * kErrStride, vmax, lane);
+  if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
 }
 
 // One 192 x 192 tile (ti <= tj) of batch entry z.  4 waves (2 x 2), 3 x 3 blocks of 32 x 32 per wave.
@@ -178,7 +201,8 @@ __device__ __forceinline__ void plane_tile(const PlaneGemm& p, int ti, int tj, i
   extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
   AK_LDS unsigned char* lds = (AK_LDS unsigned char*)dtl_smem;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-  if (p.active != nullptr && p.active[z] == 0) return;
+  const int steps = p.count[z], parity = steps & 1;
+  if (p.active[z] == 0 || (steps == 0 && p.C.index == 0)) return;      // (buffer 0 of the first step is given)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -189,8 +213,8 @@ __device__ __forceinline__ void plane_tile(const PlaneGemm& p, int ti, int tj, i
   u32x4 rsrc[2];
 #pragma unroll
   for (int P = 0; P < 2; ++P) {
-    const uint64_t ba = reinterpret_cast<uint64_t>(P == 0 ? p.A + static_cast<int64_t>(z) * p.sA
-                                                          : p.B + static_cast<int64_t>(z) * p.sB);
+    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : p.B, parity) * p.buf_elems +
+                                                   static_cast<int64_t>(z) * p.set_elems);
     rsrc[P][0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
     rsrc[P][1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
     rsrc[P][2] = kDtlRange;
@@ -321,7 +345,7 @@ __device__ __forceinline__ void plane_tile(const PlaneGemm& p, int ti, int tj, i
   }
   wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
 
-  plane_epilogue<3>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue<3, 3>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
 // The same tile on two fp16 planes per operand.  A k-tile is 16 rows of four plane panels (24 KB per stage, six
@@ -340,7 +364,8 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
   AK_LDS unsigned char* lds = (AK_LDS unsigned char*)dtl_smem;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-  if (p.active != nullptr && p.active[z] == 0) return;
+  const int steps = p.count[z], parity = steps & 1;
+  if (p.active[z] == 0 || (steps == 0 && p.C.index == 0)) return;      // (buffer 0 of the first step is given)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -351,8 +376,8 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   u32x4 rsrc[2];
 #pragma unroll
   for (int P = 0; P < 2; ++P) {
-    const uint64_t ba = reinterpret_cast<uint64_t>(P == 0 ? p.A + static_cast<int64_t>(z) * p.sA
-                                                          : p.B + static_cast<int64_t>(z) * p.sB);
+    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : p.B, parity) * p.buf_elems +
+                                                   static_cast<int64_t>(z) * p.set_elems);
     rsrc[P][0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
     rsrc[P][1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
     rsrc[P][2] = kDtlRange;
@@ -466,7 +491,97 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
         for (int r = 0; r < 16; ++r) tot[a][b][r] += acc[a][b][r];
   }
   wait_vmcnt<0>();
-  plane_epilogue<2>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue<2, 3>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
+}
+
+// A 64 x 64 tile (ti <= tj) for groups with too few 192-wide tiles to fill the device: 4 waves (2 x 2) of one 32 x 32 block.
+// A tile is bound by the latency of its operands, so a stage is 64 rows of all plane panels (32 KB with two planes, 48 with
+// three) and all but one of the stages are requested ahead; one barrier per stage.  Every element is summed in the order of
+// the 192-wide tile (piece products of 16 k, chunks of 256 k): the same bits, whichever tile a group takes.
+template <int NP>
+__device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int tj, int z, AK_LDS unsigned char* lds) {
+  constexpr int BK = 64, BLOCK = BK * 64, LOADS = 4 * NP, STAGE = LOADS * BLOCK, S = NP == 2 ? 4 : 3;
+  constexpr int CHUNK = 256 / BK;
+  static_assert(S * STAGE <= kPlaneLdsBytes, "LDS");
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  const int parity = p.count[z] & 1;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 1, wc = wave & 1;
+  const int nk = p.n_pad / BK;
+  const uint32_t plane_bytes = static_cast<uint32_t>(p.plane_elems) * 2u, colblock_bytes = static_cast<uint32_t>(p.n_pad) * 64u;
+  u32x4 rsrc[2];
+#pragma unroll
+  for (int P = 0; P < 2; ++P) {
+    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : p.B, parity) * p.buf_elems +
+                                                   static_cast<int64_t>(z) * p.set_elems);
+    rsrc[P][0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
+    rsrc[P][1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
+    rsrc[P][2] = kDtlRange;
+    rsrc[P][3] = 0x00020000u;
+  }
+  // block l = (operand P, plane q, column block cb) of a stage is 4 KB of consecutive bytes, one for each wave
+  const uint32_t lane_off = static_cast<uint32_t>(wave * 1024 + lane * 16);
+  auto issue = [&](int kt, int stage) {
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+      const int P = l / (2 * NP), q = (l / 2) % NP, cb = l & 1;
+      const uint32_t col = static_cast<uint32_t>(2 * (P == 0 ? ti : tj) + cb) * colblock_bytes;
+      load_to_lds(rsrc[P], lds0 + stage * STAGE + l * BLOCK + wave * 1024,
+                  kt < nk ? static_cast<uint32_t>(kt * BK) * 64u + lane_off + q * plane_bytes + col : 0u);
+    }
+  };
+  const int g = lane >> 5, hl = (lane >> 4) & 1, j16 = lane & 15;
+  const int frag_lane = (8 * g + (j16 >> 2)) * 64 + hl * 32 + (j16 & 3) * 8;
+  AK_LDS const unsigned char* fragI = lds + frag_lane + wr * BLOCK;
+  AK_LDS const unsigned char* fragJ = lds + frag_lane + (2 * NP + wc) * BLOCK;
+  auto frag = [](AK_LDS const unsigned char* q) {
+    return pack_bf16x8(__builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(q)),
+                       __builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(q + 256)));
+  };
+  floatx16 acc, tot;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) tot[r] = acc[r] = 0.f;
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t) issue(t, t);
+  int stage = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    wait_vmcnt<(S - 2) * LOADS>();               // this wave's part of k-tile kt has landed, then everybody's; and all are
+    __syncthreads();                             // done with k-tile kt - 1, whose stage the next loads fill
+    issue(kt + S - 1, stage == 0 ? S - 1 : stage - 1);
+    const int soff = stage * STAGE;
+#pragma unroll
+    for (int h = 0; h < BK / 16; ++h) {
+      bf16x8 fa[NP], fb[NP];
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        fa[q] = frag(fragI + soff + 2 * q * BLOCK + h * 1024);
+        fb[q] = frag(fragJ + soff + 2 * q * BLOCK + h * 1024);
+      }
+      if constexpr (NP == 2) {
+        acc = x3_mfma<true>(fa[1], fb[0], acc);
+        acc = x3_mfma<true>(fa[0], fb[0], acc);
+        acc = x3_mfma<true>(fa[0], fb[1], acc);
+      } else {
+        acc = mfma_bf16(fa[2], fb[0], acc);
+        acc = mfma_bf16(fa[1], fb[0], acc);
+        acc = mfma_bf16(fa[1], fb[1], acc);
+        acc = mfma_bf16(fa[0], fb[1], acc);
+        acc = mfma_bf16(fa[0], fb[2], acc);
+        acc = mfma_bf16(fa[0], fb[0], acc);
+      }
+    }
+    stage = stage + 1 == S ? 0 : stage + 1;
+    if (kt % CHUNK == CHUNK - 1 || kt + 1 == nk) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        tot[r] += acc[r];
+        acc[r] = 0.f;
+      }
+    }
+  }
+  wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
+  plane_epilogue<NP, 1>(p, ti, tj, z, [&](int, int, int r) { return tot[r]; });
 }
 
 // Tile number -> (ti <= tj), in bands of 8 tile columns, row by row inside a band: the 32 work groups that share an

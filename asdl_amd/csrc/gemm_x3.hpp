@@ -467,7 +467,7 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
   if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out + static_cast<int64_t>(z) * p.absmax_stride, vmax, lane);
 }
 
-template <int NSPLIT, bool DB, int AKC = -1, int BKC = -1, bool CHUNKED = false>
+template <int NSPLIT, bool DB, int AKC = -1, int BKC = -1>
 static __global__ __launch_bounds__(256) void gemm_x3_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[(DB ? 2 : 1) * 2 * NSPLIT * X3_PLANE];
   int ti = blockIdx.y, tj = blockIdx.x;
@@ -475,7 +475,7 @@ static __global__ __launch_bounds__(256) void gemm_x3_kernel(GemmParams p) {
     p.tile_mode &= ~TILE_LINEAR_GRID;
     decode_lower_tile(blockIdx.x, ti, tj);
   }
-  gemm_x3_tile<NSPLIT, DB, AKC, BKC, false, CHUNKED>(p, ti, tj, blockIdx.z, (AK_LDS3 unsigned char*)x3_smem);
+  gemm_x3_tile<NSPLIT, DB, AKC, BKC>(p, ti, tj, blockIdx.z, (AK_LDS3 unsigned char*)x3_smem);
 }
 
 // Grouped products: many independent C_i <- alpha_i * op(A_i) op(B_i) + beta_i * C_i of different sizes in one
@@ -518,7 +518,6 @@ __device__ __forceinline__ bool grouped_lookup(const int64_t* __restrict__ table
   p.tile_mode = (r[9] & 4) ? TILE_LOWER_MIRROR : TILE_ALL;     // symmetric result: lower tiles only, mirrored
   p.active = nullptr; p.active_stride = 0;
   p.split = 0;
-  p.chunked = 0;
   p.scaleA = p.scaleB = 1.f;
   p.absmax_out = reinterpret_cast<float*>(r[14]);
   const int local = w - static_cast<int>(r[11]);

@@ -1,14 +1,35 @@
-// Shampoo's inverse p-th root of a batch of same-size symmetric PSD statistics:
+// Shampoo's inverse p-th roots of symmetric PSD statistics, in groups of one size n and power p each:
 //   out <- (S + r I)^(-1/p),  r = ridge_eps * lambda_max(S),
-// power iteration for lambda_max followed by the coupled Newton iteration, with every convergence
-// test evaluated on the device.  The host enqueues the maximum number of iterations; each kernel
-// first reads its matrix's `active` word and returns at once when that matrix has converged (or
-// stopped because its error grew by more than 1.2x, in which case the previous root is kept).
-// Statistics of 512 columns and more keep every matrix of the iteration as 16-bit planes and multiply them with the
-// plane kernel (gemm_planes.hpp); smaller ones keep fp32 matrices and run on the split-operand tile kernel (gemm_x3.hpp)
-// or the fp32 tile of gemm_f32.hpp.  All sum in chunks; the product that forms the next M also folds max |M - I| into a
-// device word and writes the next step's polynomial, and the iterates alternate between two buffer pairs, so a step is
-// its products and one decision kernel.
+// lambda_max by the power iteration of the reference, then a coupled Newton iteration, every convergence test
+// evaluated on the device: each kernel reads its matrix's `active` word first and returns at once when that matrix has
+// converged (or stopped because its error grew, in which case the previous root is kept).
+//
+// Power iteration.  The estimate after k steps is mu_{2k+1} / mu_{2k} with mu_j = v0^T S^j v0, a functional of the spectral
+// measure of v0.  32 Lanczos steps give the tridiagonal matrix T whose measure matches it (the first 63 moments exactly,
+// and what dominates the higher ones, the top of the spectrum, to rounding); the power iteration itself, with its stopping
+// rule and its limit of 100 steps, then runs on T in the registers of one wave.  Same estimate to 1e-6 (fp32 rounding),
+// a third of the passes over the statistics and a sixth of the launches.
+//
+// Newton iteration.  M_0 = z S, X_0 = z^(1/p) I;  T = a I - b M;  X <- X T;  M <- T^p M.  The classical step a = 1 + 1/p,
+// b = 1/p raises a small eigenvalue of M by (1 + 1/p)^p = 2.44 (p = 4): 12 of its 18 steps on a statistic of condition 1e6.
+// With a lower bound l of the spectrum known (the ridge: l >= ridge_eps lambda_max / ||S||_F for z = 1 / ||S||_F, which
+// puts the spectrum into [l, 1]) the step that raises l most is a larger a with b = a^(p+1) p^p / (p+1)^(p+1), which
+// keeps max m (a - b m)^p = 1: up to 7.4 per step, 12 or 13 steps in all (root_schedule_kernel).
+// The first kRootEarly steps stay classical, in the summation order of one fixed kernel per size.  What an ill-conditioned
+// root ends up with is decided there: the rounding of M' perturbs the smallest eigenvalues by about 5e-8, 1 to 2 % of the
+// root at condition 1e6, and every later step's perturbation counts 2.44 times less.  Another order, though as accurate, gives
+// another root within that percent; with the first three steps alike two computations agree to 0.2 %.
+//
+// The matrices of the iteration, all polynomials of one symmetric matrix, so that only tiles on one side of the diagonal
+// are computed and mirrored, are kept
+//  * as 16-bit planes from 512 columns up (gemm_planes.hpp): 192 x 192 tiles, one launch per product and group, where a group
+//    has enough of them to fill the device, else 64 x 64 tiles;
+//  * in fp32 below: 32 x 32 tiles whose four waves split the contraction, or 64 x 64 tiles (gemm_deep.hpp).
+// The small tiles of all groups of a kind share one launch per step of the product sequence.
+// All sum in chunks; the product that forms the next M also folds max |M - I| into a device word and writes the next
+// step's polynomial T.  X, M and T alternate between two buffers by the parity of the matrix's own step count: nothing is
+// copied per step and a rejected step leaves its matrix where it was.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include "gemm_f32.hpp"
@@ -16,34 +37,24 @@
 
 namespace ak {
 
-// products of the Newton iteration: 3 = split-bf16 kernel (fp32-grade accuracy), 0 = fp32 MFMA
-#ifdef AK_TUNING_HOOKS
-inline int g_root_split = 3;
-#else
-constexpr int g_root_split = 3;
-#endif
-
-constexpr int RCHUNKS = 64;   // partial-reduction chunks per matrix
-constexpr int kRootSymmetricMinDim = 512;   // products of matrices this large compute the lower tiles only
-// Statistics this large iterate on bf16 planes (gemm_planes.hpp): every matrix of the iteration is stored as the three
-// planes of its exact split, written by the product that makes it.  Smaller ones keep fp32 matrices and the tile
-// kernels that split (or multiply in fp32) as they read.
-#ifdef AK_TUNING_HOOKS
-inline int g_root_planes_min = 512;
-#else
-constexpr int g_root_planes_min = 512;
-#endif
-static bool root_uses_planes(int64_t n) { return n >= g_root_planes_min && n <= kPlaneMaxDim; }
+constexpr int RCHUNKS = 64;             // partial-reduction chunks per matrix
+constexpr int kRootMaxGroups = 16;      // groups of one call (they travel in the kernel arguments)
+constexpr int kLanczosSteps = 32;
+constexpr int kLanczosRows = 16;        // rows of the statistic per work group and step: four waves, four rows each
+constexpr int kRootEarly = 3;           // classical steps before the accelerated ones
+constexpr int kRootSteps = 32;          // entries of a matrix's step table; the last one repeats
+constexpr int kRootBuffers = 10;        // R0 R1 M0 M1 T0 T1 and four product buffers
+constexpr int kRootMinPlaneDim = 512;
 
 // Scales of the two-plane fp16 form (gemm_planes.hpp).  M, the polynomials T and their powers are bounded by the
-// normalisation of the iteration: ||M_0||_F = (1 + p) / 2, T <= (1 + 1/p) I and T^k <= e for a positive definite
-// statistic, so 2^12 keeps them (and a fair excess of an indefinite input) below the fp16 maximum.  The root is kept
-// without its factor z^(1/p): it grows from I to (z A)^(-1/p) <= lambda_min(M_0)^(-1/p), and the ridge bounds
-// lambda_min(M_0) >= ridge_eps (1 + p) / (2 sqrt(n)) from below (lambda_max from the power iteration; a value that is
-// low by a factor f moves the bound by f^(1/p), which the four spare bits cover).  The root's scale must not be below
-// one (the identity it starts from needs its 22 bits too), so the bound has to stay below 2^12: p = 4 with a ridge
-// of 1e-6 gives 70, p = 2 at the same ridge 8000 and more.  Beyond that, without a ridge, or with a power above 8 the
-// iteration stays on the bf16 planes, which have the range of fp32.
+// normalisation of the iteration: M <= (1 + p) / 2, T^k <= 12 (root_schedule_kernel), so 2^12 keeps them (and a fair excess of an
+// indefinite input) below the fp16 maximum.  The root is kept without its factor z^(1/p): it grows from I to
+// (z A)^(-1/p) <= lambda_min(M_0)^(-1/p), and the ridge bounds lambda_min(M_0) >= ridge_eps (1 + p) / (2 sqrt(n)) from
+// below (lambda_max from the power iteration; a value that is low by a factor f moves the bound by f^(1/p), which the four
+// spare bits cover).  The root's scale must
+// not be below one (the identity it starts from needs its 22 bits too), so the bound has to stay below 2^12: p = 4 with a
+// ridge of 1e-6 gives 70, p = 2 at the same ridge 8000 and more.  Beyond that, without a ridge, or with a power above 8
+// the iteration stays on the bf16 planes, which have the range of fp32.
 constexpr float kRootScaleM = 4096.f;
 static bool root_fp16_allowed() {
   static const bool on = [] {
@@ -52,9 +63,10 @@ static bool root_fp16_allowed() {
   }();
   return on;
 }
+static bool root_plane_dim(int64_t n) { return n >= kRootMinPlaneDim && n <= kPlaneMaxDim; }
 // 0: not on fp16 planes; else the scale of the root's planes
 static float root_fp16_scale(int64_t n, int p, float ridge_eps) {
-  if (!root_fp16_allowed() || !root_uses_planes(n) || p > 8 || !(ridge_eps > 0.f)) return 0.f;
+  if (!root_fp16_allowed() || !root_plane_dim(n) || p > 8 || !(ridge_eps > 0.f)) return 0.f;
   const double lam = static_cast<double>(ridge_eps) * (1 + p) / (2.0 * std::sqrt(static_cast<double>(n)));
   const double bound = std::pow(lam, -1.0 / p);                 // of the root's largest eigenvalue
   if (!(bound < 1e30)) return 0.f;
@@ -62,30 +74,69 @@ static float root_fp16_scale(int64_t n, int p, float ridge_eps) {
   if (e < 0) return 0.f;
   return static_cast<float>(std::ldexp(1.0, e < 12 ? e : 12));
 }
-static int64_t root_pad(int64_t n) { return (n + kPlaneTile - 1) / kPlaneTile * kPlaneTile; }
-// floats of the matrix buffers of one statistic: ten plane sets (two roots, two M, two T, four products) of
-// 3 n_pad^2 bf16, or nine fp32 matrices (two M, the second root, two T, four products)
-static size_t root_matrix_floats(int64_t n) {
-  if (root_uses_planes(n)) return static_cast<size_t>(15) * root_pad(n) * root_pad(n);
-  return static_cast<size_t>(9) * n * n;
+static int64_t root_pad(int64_t n, int tile) { return (n + tile - 1) / tile * tile; }
+static int64_t root_ld(int64_t n) { return (n + 3) / 4 * 4; }
+
+// Tile of a group on planes.  A 192-wide tile takes 0.75 us per k-tile of 16 and CU however few there are; a 64-wide one
+// 0.55 us per 64 k beside 5 us of latency, one at a time on a CU.
+static int root_plane_tile(int64_t n, int64_t batch) {
+  const double big = static_cast<double>(root_pad(n, kPlaneTile)), small = static_cast<double>(root_pad(n, kPlaneSmallTile));
+  const double T = big / kPlaneTile, t = small / kPlaneSmallTile;
+  const double us_big = std::max(1.0, T * (T + 1) / 2 * batch / 256) * (big / 16) * 0.75;
+  const double us_small = std::ceil(t * (t + 1) / 2 * batch / 256) * (5.0 + small / 64 * 0.55);
+  return us_small < us_big ? kPlaneSmallTile : kPlaneTile;
+}
+
+// floats of the matrix buffers of one statistic: plane sets of 3 n_pad^2 16-bit values, or fp32 matrices
+static size_t root_matrix_floats(int64_t n, int64_t batch) {
+  if (!root_plane_dim(n)) return static_cast<size_t>(kRootBuffers) * n * root_ld(n);
+  const size_t n_pad = static_cast<size_t>(root_pad(n, root_plane_tile(n, batch)));
+  return kRootBuffers * 3 * n_pad * n_pad / 2;
 }
 
 struct RootState {
-  // per matrix, all device memory
-  float* sv;        // current eigenvalue estimate
-  float* nrm2;      // squared norm of the current power-iteration vector
+  // per matrix of the call, all device memory
+  float* sv;        // eigenvalue estimate
   float* err;       // current Newton error max|M - I|
   float* zscale;
-  float* partial;   // [batch, RCHUNKS]
-  int* pi_active;   // power iteration still running
+  float* partial;   // [RCHUNKS]: sums of squares, then max |M_0 - I|
+  float* partial_tr;  // [RCHUNKS]: partial traces
+  float* alpha;     // [kLanczosSteps] the tridiagonal matrix: diagonal,
+  float* beta;      // [kLanczosSteps] and beta[j] next to alpha[j - 1], alpha[j]
+  float* coef;      // [2 kRootSteps]: (a, b) of every step
+  float* errword;   // [kErrStride] max |M' - I| of the step under way, folded in by the epilogue of the product that forms M'
+  int* lz_dim;      // Lanczos steps that counted (0: all)
   int* pi_iters;
   int* active;      // Newton iteration still running
-  int* commit;      // last Newton step accepted
-  int* count;
-  int* par;         // which of the two root / M buffers holds the matrix's latest accepted iterate
-  float* errword;   // max |M' - I| of the step under way, folded in by the epilogue of the product that forms M'
+  int* count;       // accepted steps
+  int* accel;       // steps of the table that are not the classical one
   int* ovf;         // fp16 planes: a product of the step under way left the fp16 range
 };
+
+struct RootGroup {
+  float* S;
+  float* out;
+  const float* v0;
+  float* stats;
+  float* bufs;          // kRootBuffers buffers of `batch` fp32 matrices (n rows of ld) or plane sets
+  float* vec;           // Lanczos vectors: q ring of 3, S q ring of 2, each [batch, n]
+  int64_t strideS, strideOut;
+  int n, ld, batch, p;
+  int z0;               // first matrix of the group in the state arrays
+  int np, n_pad, tile;  // planes per matrix: 0 (fp32), 2, 3; tile of the products on planes
+  float scale_r;
+};
+struct RootGroups {
+  RootState st;
+  int count, total;
+  RootGroup g[kRootMaxGroups];
+};
+
+__device__ __forceinline__ int root_group_of(const RootGroups& G, int z) {
+  int g = 0;
+  while (g + 1 < G.count && G.g[g + 1].z0 <= z) ++g;
+  return g;
+}
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -97,133 +148,394 @@ __device__ __forceinline__ float wave_max(float v) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
   return v;
 }
-
-// grid (batch): v <- v0, norm, flags
-static __global__ __launch_bounds__(256) void root_init_kernel(RootState st, const float* __restrict__ v0,
-                                                               float* __restrict__ v, int64_t n) {
-  __shared__ float red[4];
-  const int z = blockIdx.x;
-  float s = 0.f;
-  for (int64_t i = threadIdx.x; i < n; i += 256) {
-    const float x = v0[z * n + i];
-    v[z * n + i] = x;
-    s += x * x;
-  }
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+// Sum over the 256 threads of a work group, the same value in all of them.  red: 4 floats, free again after the next barrier.
+__device__ __forceinline__ float block_sum(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    st.nrm2[z] = red[0] + red[1] + red[2] + red[3];
-    st.sv[z] = 0.f;
-    st.pi_active[z] = 1;
-    st.pi_iters[z] = 0;
-    st.active[z] = 0;
-    st.commit[z] = 0;
-    st.count[z] = 0;
-    st.par[z] = 0;
-    st.errword[z] = 0.f;
-    st.ovf[z] = 0;
-  }
+  return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// grid (ceil(n/4), batch): mv[row] = S[row,:] . v / ||v||   (one wave per row)
-static __global__ __launch_bounds__(256) void power_matvec_kernel(RootState st, const float* __restrict__ S,
-                                                                  int64_t strideS, const float* __restrict__ v,
-                                                                  float* __restrict__ mv, int64_t n) {
-  const int z = blockIdx.y;
-  if (st.pi_active[z] == 0) return;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= n) return;
-  const int lane = threadIdx.x & 63;
-  const float* __restrict__ Sr = S + z * strideS + row * n;
-  const float* __restrict__ vz = v + z * n;
-  float s = 0.f;
-  for (int64_t k = lane; k < n; k += 64) s += Sr[k] * vz[k];
-  s = wave_sum(s);
-  if (lane == 0) mv[z * n + row] = s / sqrtf(st.nrm2[z]);
-}
+// What a Lanczos step needs of a group; `first`: its first work group.  (The first numbers of all groups lie side by side: a
+// work group finds its own with one load.  Kernel arguments behind a dependent index cost a trip to memory each.)
+struct LanczosGroup {
+  const float* S;
+  const float* v0;
+  float* vec;
+  int64_t strideS;
+  int n, batch, z0, pad;
+};
+struct LanczosGroups {
+  int first[kRootMaxGroups];
+  LanczosGroup g[kRootMaxGroups];
+};
 
-// grid (batch): s_v = (v/||v||) . mv; error = |s_v - sv|; v <- mv
-static __global__ __launch_bounds__(256) void power_update_kernel(RootState st, float* __restrict__ v,
-                                                                  const float* __restrict__ mv, int64_t n, float tol,
-                                                                  int max_iters) {
-  __shared__ float red[8];
-  const int z = blockIdx.x;
-  if (st.pi_active[z] == 0) return;
-  const float inv_norm = 1.f / sqrtf(st.nrm2[z]);
-  float dot = 0.f, nn = 0.f;
-  for (int64_t i = threadIdx.x; i < n; i += 256) {
-    const float m = mv[z * n + i];
-    dot += v[z * n + i] * inv_norm * m;
-    nn += m * m;
-    v[z * n + i] = m;
+// Lanczos step j: q_j from S q_{j-1}, then its work group's rows of S q_j.  Every work group of a matrix forms q_j for
+// itself in the LDS (three vectors from the L2, two reductions): one launch per step, no hand-over inside it.  The
+// rows of S are requested before that, their first 1024 columns kept in registers.
+// Bound by the launch and the chain of loads and reductions for small n, by reading S for a full batch.
+static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, LanczosGroups L, int j) {
+  extern __shared__ __attribute__((aligned(16))) float q[];
+  __shared__ float red[3][4];
+  const int wg = blockIdx.x;
+  int gi = 0;
+#pragma unroll
+  for (int k = 1; k < kRootMaxGroups; ++k) gi += wg >= L.first[k] ? 1 : 0;
+  const LanczosGroup g = L.g[gi];
+  const int n = g.n, per = (n + kLanczosRows - 1) / kLanczosRows;
+  const int local = wg - L.first[gi], zl = local / per, part = local - zl * per;
+  const int z = g.z0 + zl, tid = threadIdx.x, lane = tid & 63, row0 = part * kLanczosRows + 4 * (tid >> 6);
+  const float* __restrict__ S = g.S + zl * g.strideS;
+  const int n4 = n & ~3;
+  floatx4 early[4][4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = 4 * lane + 256 * c, row = row0 + r < n ? row0 + r : n - 1;
+      early[c][r] = k < n4 ? *reinterpret_cast<const floatx4u*>(S + static_cast<int64_t>(row) * n + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  const int64_t vec = static_cast<int64_t>(g.batch) * n;
+  float* __restrict__ qj = g.vec + (j % 3) * vec + static_cast<int64_t>(zl) * n;
+  if (j == 0) {
+    const float* __restrict__ v0 = g.v0 + static_cast<int64_t>(zl) * n;
+    float s = 0.f;
+    for (int i = tid; i < n; i += 256) {
+      const float x = v0[i];
+      q[i] = x;
+      s += x * x;
+    }
+    const float inv = 1.f / sqrtf(block_sum(s, red[0]));
+    for (int i = tid; i < n; i += 256) {
+      q[i] *= inv;
+      if (part == 0) qj[i] = q[i];
+    }
+    if (part == 0 && tid == 0) {
+      st.lz_dim[z] = 0;
+      st.active[z] = st.count[z] = st.ovf[z] = 0;
+      st.errword[z * kErrStride] = 0.f;
+      st.beta[z * kLanczosSteps] = 0.f;
+    }
+  } else {
+    if (j > 1 && st.lz_dim[z] != 0) return;            // an invariant subspace: T is complete
+    const float* __restrict__ q1 = g.vec + ((j + 2) % 3) * vec + static_cast<int64_t>(zl) * n;
+    const float* __restrict__ q2 = g.vec + ((j + 1) % 3) * vec + static_cast<int64_t>(zl) * n;
+    const float* __restrict__ w = g.vec + (3 + ((j + 1) & 1)) * vec + static_cast<int64_t>(zl) * n;
+    const float b = st.beta[z * kLanczosSteps + j - 1];
+    float s = 0.f;
+    for (int i = tid; i < n; i += 256) s += w[i] * q1[i];
+    const float a = block_sum(s, red[0]);
+    s = 0.f;
+    for (int i = tid; i < n; i += 256) {
+      const float x = w[i] - a * q1[i] - (j > 1 ? b * q2[i] : 0.f);
+      q[i] = x;
+      s += x * x;
+    }
+    const float norm = sqrtf(block_sum(s, red[1]));
+    const bool done = !(norm > 1e-7f * fabsf(a));
+    if (part == 0 && tid == 0) {
+      st.alpha[z * kLanczosSteps + j - 1] = a;
+      if (done) st.lz_dim[z] = j;
+      else st.beta[z * kLanczosSteps + j] = norm;
+    }
+    if (done) return;
+    const float inv = 1.f / norm;
+    for (int i = tid; i < n; i += 256) {
+      q[i] *= inv;
+      if (part == 0) qj[i] = q[i];
+    }
   }
-  dot = wave_sum(dot);
-  nn = wave_sum(nn);
-  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = dot; red[4 + (threadIdx.x >> 6)] = nn; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const float s_v = red[0] + red[1] + red[2] + red[3];
-    const float error = fabsf(s_v - st.sv[z]);
-    st.sv[z] = s_v;
-    st.nrm2[z] = red[4] + red[5] + red[6] + red[7];
-    const int it = st.pi_iters[z] + 1;
-    st.pi_iters[z] = it;
-    if (!(error > tol && it < max_iters)) st.pi_active[z] = 0;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int k = 4 * lane + 256 * c;
+    if (k >= n4) break;
+    const floatx4 x = *reinterpret_cast<const floatx4*>(q + k);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      acc[r] += early[c][r][0] * x[0] + early[c][r][1] * x[1] + early[c][r][2] * x[2] + early[c][r][3] * x[3];
+  }
+  for (int k = 4 * lane + 1024; k < n4; k += 256) {
+    const floatx4 x = *reinterpret_cast<const floatx4*>(q + k);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = row0 + r < n ? row0 + r : n - 1;
+      const floatx4 m = *reinterpret_cast<const floatx4u*>(S + static_cast<int64_t>(row) * n + k);
+      acc[r] += m[0] * x[0] + m[1] * x[1] + m[2] * x[2] + m[3] * x[3];
+    }
+  }
+  if (n4 + lane < n) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = row0 + r < n ? row0 + r : n - 1;
+      acc[r] += S[static_cast<int64_t>(row) * n + n4 + lane] * q[n4 + lane];
+    }
+  }
+  float* __restrict__ wj = g.vec + (3 + (j & 1)) * vec + static_cast<int64_t>(zl) * n;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float s = wave_sum(acc[r]);
+    if (lane == 0 && row0 + r < n) wj[row0 + r] = s;
   }
 }
 
-// grid (RCHUNKS, batch): S += ridge I (in place), partial sum of squares of the ridged matrix
-static __global__ __launch_bounds__(256) void root_ridge_kernel(RootState st, float* __restrict__ S, int64_t strideS,
-                                                                int64_t n, float ridge_eps) {
-  __shared__ float red[4];
+template <int CTRL>
+__device__ __forceinline__ float dpp_zero(float v) {       // lanes without a source read zero
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// Sum over lanes 0 ... 31, the same value everywhere.
+__device__ __forceinline__ float sum32(float v) {
+  v += dpp_zero<0x111>(v);       // row_shr:1, 2, 4, 8: lane 15 of a row of 16 holds its sum
+  v += dpp_zero<0x112>(v);
+  v += dpp_zero<0x114>(v);
+  v += dpp_zero<0x118>(v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 15)) +
+         __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 31));
+}
+
+// grid (total), one wave: the reference's power iteration (estimate (v/|v|) . S v/|v|, stop on |change| <= tol) on T.
+static __global__ __launch_bounds__(64) void root_power_kernel(RootGroups G, int steps, float tol, int max_iters) {
+  const int z = blockIdx.x, lane = threadIdx.x;
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  const int zl = z - g.z0;
+  int m = G.st.lz_dim[z];
+  if (m == 0) {
+    // the last diagonal element: q . S q of the last step
+    const int64_t vec = static_cast<int64_t>(g.batch) * g.n, at = static_cast<int64_t>(zl) * g.n;
+    const float* __restrict__ q = g.vec + ((steps - 1) % 3) * vec + at;
+    const float* __restrict__ w = g.vec + (3 + ((steps - 1) & 1)) * vec + at;
+    float s = 0.f;
+    for (int i = lane; i < g.n; i += 64) s += q[i] * w[i];
+    s = wave_sum(s);
+    if (lane == 0) G.st.alpha[z * kLanczosSteps + steps - 1] = s;
+    m = steps;
+    __syncthreads();
+  }
+  float a = 0.f, bl = 0.f, br = 0.f;           // diagonal, couplings to the lanes below and above
+  if (lane < m) {
+    a = G.st.alpha[z * kLanczosSteps + lane];
+    if (lane > 0) bl = G.st.beta[z * kLanczosSteps + lane];
+    if (lane + 1 < m) br = G.st.beta[z * kLanczosSteps + lane + 1];
+  }
+  float v = lane == 0 ? 1.f : 0.f, sv = 0.f;
+  int it = 0;
+  bool go_on = max_iters > 0;
+  while (go_on) {
+    const float x = v / sqrtf(sum32(v * v));
+    const float y = a * x + bl * dpp_zero<0x138>(x) + br * dpp_zero<0x130>(x);      // wave_shr:1, wave_shl:1
+    const float s = sum32(x * y);
+    const float error = fabsf(s - sv);
+    sv = s;
+    v = y;
+    ++it;
+    go_on = error > tol && it < max_iters;
+  }
+  if (lane == 0) {
+    G.st.sv[z] = sv;
+    G.st.pi_iters[z] = it;
+  }
+}
+
+// grid (RCHUNKS, total): S += ridge I (in place), partial sum of squares and trace of the ridged matrix
+static __global__ __launch_bounds__(256) void root_ridge_kernel(RootGroups G, float ridge_eps) {
+  __shared__ float red[2][4];
   const int z = blockIdx.y;
-  float* __restrict__ Sz = S + z * strideS;
-  const float ridge = ridge_eps * st.sv[z];
-  const int64_t total = n * n;
-  float s = 0.f;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
-    float x = Sz[i];
-    if (i % (n + 1) == 0) {
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  float* __restrict__ S = g.S + (z - g.z0) * g.strideS;
+  const float ridge = ridge_eps * G.st.sv[z];
+  const uint32_t total = static_cast<uint32_t>(g.n) * static_cast<uint32_t>(g.n), period = static_cast<uint32_t>(g.n) + 1;
+  float s = 0.f, t = 0.f;
+#pragma unroll 4
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
+    float x = S[i];
+    if (i % period == 0) {
       x += ridge;
-      Sz[i] = x;
+      S[i] = x;
+      t += x;
     }
     s += x * x;
   }
   s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  t = wave_sum(t);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s;
+    red[1][threadIdx.x >> 6] = t;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) st.partial[z * RCHUNKS + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  if (threadIdx.x == 0) {
+    G.st.partial[z * RCHUNKS + blockIdx.x] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    G.st.partial_tr[z * RCHUNKS + blockIdx.x] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+  }
 }
 
-// grid (batch)
-static __global__ void root_zscale_kernel(RootState st, int p) {
-  const int z = blockIdx.x;
-  if (threadIdx.x != 0) return;
-  float s = 0.f;
-  for (int c = 0; c < RCHUNKS; ++c) s += st.partial[z * RCHUNKS + c];
-  st.zscale[z] = (1.f + p) / (2.f * sqrtf(s));
+__device__ __forceinline__ float int_power(float x, int p) {
+  float r = 1.f;
+  for (int i = 0; i < p; ++i) r *= x;
+  return r;
 }
 
-// grid (RCHUNKS, batch): M = z S, T = (1 + 1/p) I - M / p, root = z^(1/p) I, partial max |M - I|
-static __global__ __launch_bounds__(256) void root_start_kernel(RootState st, const float* __restrict__ S,
-                                                                int64_t strideS, float* __restrict__ M,
-                                                                float* __restrict__ T, float* __restrict__ root,
-                                                                int64_t strideR, int64_t n, int p) {
+// grid (total), one wave: the scale z and the (a, b) of every step.
+//
+// Accelerated steps where they pay: with a ridge of 1e-7 and more (below, the bound l is not one that fp32 can keep), a
+// power up to 8, room for the classical iteration's own number of steps (a caller that asks for a few steps gets those
+// of the reference), and a statistic whose spectrum is spread: n ||S||_F^2 / tr(S)^2 = mean(lambda^2) / mean(lambda)^2 is
+// 1.3 for a well-conditioned sample covariance, whose eigenvalues the classical step brings together in 7 to 9 steps, fewer
+// than a schedule that has to assume l; 2 and more for the rank-deficient statistics of gradients.
+// A step may not press the top of the spectrum below kTopMin: its rounding error relative to that value is what the root
+// inherits in the dominant directions (0.17: errors against fp64 at or below the classical iteration's on spectra of
+// condition 14 to 1e6; unlimited, 9 steps but 4e-4 instead of 1e-6 at condition 14).  T^p stays below 12 for the fp16 planes.
+static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, float ridge_eps, int max_iter) {
+  constexpr float kTopMin = 0.17f, kSpread = 1.6f, kEnd = 0.97f;
+  const int z = blockIdx.x, lane = threadIdx.x;
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  const int p = g.p;
+  const float part = G.st.partial[z * RCHUNKS + lane], tr = wave_sum(G.st.partial_tr[z * RCHUNKS + lane]);
+  float nrm2 = 0.f;
+#pragma unroll
+  for (int c = 0; c < RCHUNKS; ++c) nrm2 += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, part), c));
+  const float sv = G.st.sv[z], zscale = (1.f + p) / (2.f * sqrtf(nrm2));
+  float* __restrict__ coef = G.st.coef + z * 2 * kRootSteps;
+  const float a0 = 1.f + 1.f / p, b0 = 1.f / p;
+  int k = 0;
+  float l = 0.5f * ridge_eps * sv * zscale;    // half: the estimate of lambda_max may be low, S indefinite by its rounding
+  const bool fast = ridge_eps >= 1e-7f && p >= 2 && p <= 8 && max_iter >= kRootSteps && sv > 0.f &&
+                    g.n * nrm2 > kSpread * tr * tr && l > 1e-9f && l < kEnd;
+  if (fast) {
+    const float cp = int_power(static_cast<float>(p) / (p + 1), p) / (p + 1);       // b = cp a^(p+1)
+    // the classical steps: the spectrum is in [l, (1 + p) / 2], and in (0, 1] after the first
+    const float first = 0.5f * (1 + p) * int_power(a0 - b0 * 0.5f * (1 + p), p);
+    for (; k < kRootEarly; ++k) {
+      l *= int_power(a0 - b0 * l, p);
+      if (k == 0) l = fminf(l, first);
+      if (lane == 0) {
+        coef[2 * k] = a0;
+        coef[2 * k + 1] = b0;
+      }
+    }
+    for (; k < kRootSteps - 1 && l < kEnd; ++k) {
+      // the a in [1 + 1/p, 2.5] that maximises min(f(l), f(1)), f(m) = m (a - b m)^p: two rounds of 64 candidates
+      float lo = a0, hi = 2.5f, a = a0, v = -1.f;
+#pragma unroll
+      for (int round = 0; round < 2; ++round) {
+        const float c = lo + (hi - lo) * (lane / 63.f);
+        const float ap = int_power(c, p), b = cp * ap * c;
+        const float top = int_power(c - b, p), low = l * int_power(c - b * l, p);
+        const float value = c > b && ap <= 12.f && (top >= kTopMin || c == a0) ? fminf(top, low) : -1.f;
+        const float best = wave_max(value);
+        const int who = __ffsll(__ballot(value == best)) - 1;
+        a = __shfl(c, who);
+        v = best;
+        const float h = (hi - lo) / 63.f;
+        lo = fmaxf(a0, a - h);
+        hi = a + h;
+      }
+      if (lane == 0) {
+        coef[2 * k] = a;
+        coef[2 * k + 1] = cp * int_power(a, p) * a;
+      }
+      if (!(v > l)) break;
+      l = v;
+    }
+  }
+  for (int i = k + lane; i < kRootSteps; i += 64) {
+    coef[2 * i] = a0;
+    coef[2 * i + 1] = b0;
+  }
+  if (lane == 0) {
+    G.st.accel[z] = k;
+    G.st.zscale[z] = zscale;
+  }
+}
+
+// grid (RCHUNKS, total), fp32 groups: M = z S, T = a I - b M and the X of the first step, z^(1/p) T (X_0 is a multiple of the
+// identity and never stored); the padding columns are zero; partial max |M - I|
+static __global__ __launch_bounds__(256) void root_start_kernel(RootGroups G) {
   __shared__ float red[4];
   const int z = blockIdx.y;
-  const float zs = st.zscale[z];
-  const float r0 = powf(zs, 1.0f / p);
-  const float alpha = -1.0f / p;
-  const int64_t total = n * n;
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  if (g.np != 0) return;
+  const int n = g.n, ld = g.ld;
+  const float zs = G.st.zscale[z], r0 = powf(zs, 1.0f / g.p);
+  const float a = G.st.coef[z * 2 * kRootSteps], b = G.st.coef[z * 2 * kRootSteps + 1];
+  const int64_t mat = static_cast<int64_t>(n) * ld, buf = mat * g.batch;
+  const float* __restrict__ S = g.S + (z - g.z0) * g.strideS;
+  float* __restrict__ base = g.bufs + (z - g.z0) * mat;
   float e = 0.f;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
-    const bool diag = (i % (n + 1) == 0);
-    const float m = zs * S[z * strideS + i];
-    M[z * total + i] = m;
-    T[z * total + i] = (diag ? (1.f - alpha) : 0.f) + alpha * m;
-    root[z * strideR + i] = diag ? r0 : 0.f;
-    e = fmaxf(e, fabsf(m - (diag ? 1.f : 0.f)));
+  const int lane = threadIdx.x & 63;
+  for (int i = 4 * blockIdx.x + (threadIdx.x >> 6); i < n; i += 4 * RCHUNKS) {
+#pragma unroll 4
+    for (int j = lane; j < ld; j += 64) {
+      const bool inside = j < n, diag = i == j;
+      const float m = inside ? zs * S[static_cast<int64_t>(i) * n + j] : 0.f;
+      const float t = (diag ? a : 0.f) - b * m;
+      const int64_t at = static_cast<int64_t>(i) * ld + j;
+      base[buf + at] = r0 * t;
+      base[2 * buf + at] = m;
+      base[4 * buf + at] = t;
+      if (!inside)                             // no product writes the padding columns
+        for (int k = 0; k < kRootBuffers; ++k) base[k * buf + at] = 0.f;
+      if (inside) e = fmaxf(e, fabsf(m - (diag ? 1.f : 0.f)));
+    }
+  }
+  e = wave_max(e);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
+  __syncthreads();
+  if (threadIdx.x == 0) G.st.partial[z * RCHUNKS + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// grid (RCHUNKS, batch): the same on planes over the padded index range (zero outside n x n).  NP = 2 (fp16 planes): M and T
+// scaled by kRootScaleM, X without its factor z^(1/p): scale_r T.
+template <int NP>
+static __global__ __launch_bounds__(256) void root_start_planes_kernel(RootState st, RootGroup g) {
+  __shared__ float red[4];
+  const int zl = blockIdx.y, z = g.z0 + zl;
+  const float zs = st.zscale[z];
+  const float r0 = NP == 2 ? g.scale_r : powf(zs, 1.0f / g.p);
+  const float sm = NP == 2 ? kRootScaleM : 1.f;
+  const float a = st.coef[z * 2 * kRootSteps], b = st.coef[z * 2 * kRootSteps + 1];
+  const int n = g.n, n_pad = g.n_pad;
+  const int64_t plane = static_cast<int64_t>(n_pad) * n_pad, set = NP * plane, buf = set * g.batch;
+  const float* __restrict__ S = g.S + zl * g.strideS;
+  unsigned short* __restrict__ base = reinterpret_cast<unsigned short*>(g.bufs) + zl * set;
+  float e = 0.f;
+  const int lane = threadIdx.x & 63;
+  for (int i = 4 * blockIdx.x + (threadIdx.x >> 6); i < n_pad; i += 4 * RCHUNKS) {
+    for (int j = 4 * lane; j < n_pad; j += 256) {
+      floatx4 x = {0.f, 0.f, 0.f, 0.f};
+      const float* src = S + static_cast<int64_t>(i) * n + j;
+      if (i < n && j + 4 <= n) {
+        x = *reinterpret_cast<const floatx4u*>(src);
+      } else if (i < n) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (j + k < n) x[k] = src[k];
+      }
+      u16x4 om[NP], ot[NP], ox[NP];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool inside = i < n && j + k < n, diag = i == j + k;
+        const float m = zs * x[k], t = inside ? (diag ? a : 0.f) - b * m : 0.f;
+        if (inside) e = fmaxf(e, fabsf(m - (diag ? 1.f : 0.f)));
+        unsigned short o[3];
+        plane_bits<NP>(m * sm, o);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) om[q][k] = o[q];
+        plane_bits<NP>(t * sm, o);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) ot[q][k] = o[q];
+        plane_bits<NP>(r0 * t, o);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) ox[q][k] = o[q];
+      }
+      const int64_t dst = plane_index(i, j, n_pad);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        *reinterpret_cast<u16x4*>(base + buf + q * plane + dst) = ox[q];
+        *reinterpret_cast<u16x4*>(base + 2 * buf + q * plane + dst) = om[q];
+        *reinterpret_cast<u16x4*>(base + 4 * buf + q * plane + dst) = ot[q];
+      }
+    }
   }
   e = wave_max(e);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
@@ -231,480 +543,654 @@ static __global__ __launch_bounds__(256) void root_start_kernel(RootState st, co
   if (threadIdx.x == 0) st.partial[z * RCHUNKS + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// grid (batch)
+// grid (total), one wave
 static __global__ void root_begin_kernel(RootState st, float tol, int max_iter) {
   const int z = blockIdx.x;
+  const float e = wave_max(st.partial[z * RCHUNKS + threadIdx.x]);
   if (threadIdx.x != 0) return;
-  float e = 0.f;
-  for (int c = 0; c < RCHUNKS; ++c) e = fmaxf(e, st.partial[z * RCHUNKS + c]);
   st.err[z] = e;
   st.active[z] = (e > tol && max_iter > 0) ? 1 : 0;
 }
 
-// grid (batch): accept / reject the step and decide whether to go on.  The error of the step is the word the product
-// M' = T^p M folded max |M' - I| into; `wrote`: which buffer pair that step wrote (the matrix's latest iterate if
-// the step is accepted).
-static __global__ void newton_decide_kernel(RootState st, float tol, int max_iter, int wrote) {
+// grid (total): accept / reject the step and decide whether to go on.  The error of the step is the word the product
+// M' = T^p M folded max |M' - I| into.
+static __global__ void newton_decide_kernel(RootState st, float tol, int max_iter) {
   const int z = blockIdx.x;
   if (threadIdx.x != 0) return;
-  st.commit[z] = 0;
-  const float e = st.errword[z];
-  st.errword[z] = 0.f;
-  const int overflow = st.ovf[z];
+  const float e = st.errword[z * kErrStride], err = st.err[z];
+  const int overflow = st.ovf[z], active = st.active[z], c = st.count[z], accel = st.accel[z];
+  st.errword[z * kErrStride] = 0.f;
   st.ovf[z] = 0;
-  if (st.active[z] == 0) return;
-  const float err = st.err[z];
-  // diverging: keep the previous root (NaN compares false, like the reference).  A step whose products left the range
-  // of the fp16 planes (a statistic far from positive definite) is dropped the same way.
-  if (overflow != 0 || e > err * 1.2f) {
+  if (active == 0) return;
+  // diverging: keep the previous root (NaN compares false, like the reference).  The error of an accelerated step may grow, but
+  // not beyond that of a spectrum in [0, 1].  A step whose products left the range of the fp16 planes (a statistic far
+  // from positive definite) is dropped the same way.
+  const float limit = c >= kRootEarly && c < accel ? 1.2f : err * 1.2f;
+  if (overflow != 0 || e > limit) {
     st.active[z] = 0;
     return;
   }
-  st.commit[z] = 1;
-  st.par[z] = wrote;
   st.err[z] = e;
-  const int c = st.count[z] + 1;
-  st.count[z] = c;
-  if (!(e > tol && c < max_iter)) st.active[z] = 0;
+  st.count[z] = c + 1;
+  if (!(e > tol && c + 1 < max_iter)) st.active[z] = 0;
 }
 
-// grid (RCHUNKS, batch): brings the matrices whose latest iterate sits in the second buffer pair back to the first
-// one (root, M, and T for a matrix that goes on iterating) and resets their marks.  With an even number of iterations
-// per call only the matrices that stopped after an odd number of steps are concerned.
-static __global__ __launch_bounds__(256) void newton_gather_kernel(RootState st, float* __restrict__ root,
-                                                                   int64_t strideR, const float* __restrict__ root1,
-                                                                   float* __restrict__ M, const float* __restrict__ M1,
-                                                                   float* __restrict__ T, const float* __restrict__ T1,
-                                                                   int64_t n) {
+// grid (RCHUNKS, total): the caller's fp32 result
+static __global__ __launch_bounds__(256) void root_out_kernel(RootGroups G) {
   const int z = blockIdx.y;
-  if (st.par[z] == 0) return;
-  const bool go_on = st.active[z] != 0;
-  const int64_t total = n * n;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
-    root[z * strideR + i] = root1[z * total + i];
-    M[z * total + i] = M1[z * total + i];
-    if (go_on) T[z * total + i] = T1[z * total + i];
-  }
-}
-
-// grid (batch): after newton_gather_kernel
-static __global__ void newton_gathered_kernel(RootState st) {
-  if (threadIdx.x == 0) st.par[blockIdx.x] = 0;
-}
-
-// ---- the same on bf16 planes --------------------------------------------------------------------------------------
-
-// grid (RCHUNKS, batch): planes of M = z S, T = (1 + 1/p) I - M / p and root = z^(1/p) I over the padded index range
-// (zero outside n x n), partial max |M - I|.  NP = 2 (fp16 planes): M and T scaled by scale_m, the root without its
-// factor z^(1/p): scale_r I.
-template <int NP>
-static __global__ __launch_bounds__(256) void root_start_planes_kernel(RootState st, const float* __restrict__ S,
-                                                                       int64_t strideS, __bf16* __restrict__ M,
-                                                                       __bf16* __restrict__ T, __bf16* __restrict__ R,
-                                                                       int64_t set_elems, int64_t n, int64_t n_pad, int p,
-                                                                       float scale_m, float scale_r) {
-  __shared__ float red[4];
-  const int z = blockIdx.y;
-  const float zs = st.zscale[z];
-  const float r0 = NP == 2 ? scale_r : powf(zs, 1.0f / p);
-  const float sm = NP == 2 ? scale_m : 1.f;
-  const float alpha = -1.0f / p;
-  const int64_t total = n_pad * n_pad;
-  unsigned short* Mz = reinterpret_cast<unsigned short*>(M) + z * set_elems;
-  unsigned short* Tz = reinterpret_cast<unsigned short*>(T) + z * set_elems;
-  unsigned short* Rz = reinterpret_cast<unsigned short*>(R) + z * set_elems;
-  float e = 0.f;
-  for (int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; at < total; at += RCHUNKS * 256) {
-    const int64_t i = at / n_pad, j = at - i * n_pad;
-    const bool inside = i < n && j < n, diag = i == j;
-    float m = 0.f, t = 0.f, r = 0.f;
-    if (inside) {
-      m = zs * S[z * strideS + i * n + j];
-      t = (diag ? (1.f - alpha) : 0.f) + alpha * m;
-      r = diag ? r0 : 0.f;
-      e = fmaxf(e, fabsf(m - (diag ? 1.f : 0.f)));
-    }
-    unsigned short o[3];
-    const int64_t dst = plane_index(i, j, n_pad);
-    plane_bits<NP>(m * sm, o);
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  const int zl = z - g.z0, n = g.n, count = G.st.count[z], lane = threadIdx.x & 63;
+  float* __restrict__ out = g.out + zl * g.strideOut;
+  const float r0 = powf(G.st.zscale[z], 1.0f / g.p);
+  const int64_t mat = static_cast<int64_t>(n) * g.ld;
+  const float* __restrict__ R = g.bufs + (count & 1) * mat * g.batch + zl * mat;
+  const int64_t plane = static_cast<int64_t>(g.n_pad) * g.n_pad, set = g.np * plane;
+  const unsigned short* __restrict__ P = reinterpret_cast<const unsigned short*>(g.bufs) + (count & 1) * set * g.batch + zl * set;
+  // fp16 planes hold scale_r times the root without its factor z^(1/p); the sum of the bf16 planes is the root
+  const float mul = r0 / g.scale_r;
+  for (int i = 4 * blockIdx.x + (threadIdx.x >> 6); i < n; i += 4 * RCHUNKS) {
+    for (int j = 4 * lane; j < n; j += 256) {
+      floatx4 v;
+      if (count == 0) {                           // no step was accepted
 #pragma unroll
-    for (int q = 0; q < NP; ++q) Mz[q * total + dst] = o[q];
-    plane_bits<NP>(t * sm, o);
+        for (int k = 0; k < 4; ++k) v[k] = i == j + k ? r0 : 0.f;
+      } else if (g.np == 0) {
+        v = *reinterpret_cast<const floatx4*>(R + static_cast<int64_t>(i) * g.ld + j);
+      } else {
+        const int64_t src = plane_index(i, j, g.n_pad);
+        u16x4 o[3];
 #pragma unroll
-    for (int q = 0; q < NP; ++q) Tz[q * total + dst] = o[q];
-    plane_bits<NP>(r, o);
+        for (int q = 0; q < 3; ++q)
+          if (q < g.np) o[q] = *reinterpret_cast<const u16x4*>(P + q * plane + src);
 #pragma unroll
-    for (int q = 0; q < NP; ++q) Rz[q * total + dst] = o[q];
-  }
-  e = wave_max(e);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
-  __syncthreads();
-  if (threadIdx.x == 0) st.partial[z * RCHUNKS + blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-
-// grid (RCHUNKS, batch): newton_gather_kernel on plane sets (set_words 32-bit words each)
-static __global__ __launch_bounds__(256) void newton_gather_planes_kernel(RootState st, uint32_t* __restrict__ R0,
-                                                                          const uint32_t* __restrict__ R1,
-                                                                          uint32_t* __restrict__ M0,
-                                                                          const uint32_t* __restrict__ M1,
-                                                                          uint32_t* __restrict__ T0,
-                                                                          const uint32_t* __restrict__ T1,
-                                                                          int64_t set_words) {
-  const int z = blockIdx.y;
-  if (st.par[z] == 0) return;
-  const bool go_on = st.active[z] != 0;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < set_words; i += RCHUNKS * 256) {
-    R0[z * set_words + i] = R1[z * set_words + i];
-    M0[z * set_words + i] = M1[z * set_words + i];
-    if (go_on) T0[z * set_words + i] = T1[z * set_words + i];
-  }
-}
-
-// grid (RCHUNKS, batch): the caller's fp32 result from the planes of the root (their sum is exact).  NP = 2: the planes
-// hold scale_r times the root without its factor z^(1/p); zscale == nullptr: no such factor (plain product).
-template <int NP>
-static __global__ __launch_bounds__(256) void root_out_planes_kernel(const __bf16* __restrict__ R, int64_t set_elems,
-                                                                     float* __restrict__ out, int64_t strideOut,
-                                                                     int64_t n, int64_t n_pad, const float* zscale, int p,
-                                                                     float scale_r) {
-  const int z = blockIdx.y;
-  const int64_t total = n_pad * n_pad;
-  if constexpr (NP == 3) {
-    const __bf16* Rz = R + z * set_elems;
-    for (int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; at < n * n; at += RCHUNKS * 256) {
-      const int64_t i = at / n, j = at - i * n;
-      const int64_t src = plane_index(i, j, n_pad);
-      out[z * strideOut + at] = (static_cast<float>(Rz[src]) + static_cast<float>(Rz[total + src])) +
-                                static_cast<float>(Rz[2 * total + src]);
-    }
-  } else {
-    const _Float16* Rz = reinterpret_cast<const _Float16*>(R) + z * set_elems;
-    const float mul = (zscale != nullptr ? powf(zscale[z], 1.0f / p) : 1.f) / scale_r;
-    for (int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; at < n * n; at += RCHUNKS * 256) {
-      const int64_t i = at / n, j = at - i * n;
-      const int64_t src = plane_index(i, j, n_pad);
-      out[z * strideOut + at] = mul * (static_cast<float>(Rz[src]) + static_cast<float>(Rz[total + src]));
+        for (int k = 0; k < 4; ++k)
+          v[k] = g.np == 2 ? mul * (static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(o[0][k]))) +
+                                    static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(o[1][k]))))
+                           : (static_cast<float>(__builtin_bit_cast(__bf16, static_cast<unsigned short>(o[0][k]))) +
+                              static_cast<float>(__builtin_bit_cast(__bf16, static_cast<unsigned short>(o[1][k])))) +
+                                 static_cast<float>(__builtin_bit_cast(__bf16, static_cast<unsigned short>(o[2][k])));
+      }
+      float* dst = out + static_cast<int64_t>(i) * n + j;
+      if (j + 4 <= n) {
+        *reinterpret_cast<floatx4u*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (j + k < n) dst[k] = v[k];
+      }
     }
   }
 }
 
-// grid (batch)
-static __global__ void root_stats_kernel(RootState st, float* __restrict__ stats) {
+// grid (total)
+static __global__ void root_stats_kernel(RootGroups G) {
   const int z = blockIdx.x;
   if (threadIdx.x != 0) return;
-  stats[4 * z] = st.sv[z];
-  stats[4 * z + 1] = static_cast<float>(st.pi_iters[z]);
-  stats[4 * z + 2] = static_cast<float>(st.count[z]);
-  stats[4 * z + 3] = st.err[z];
+  const RootGroup& g = G.g[root_group_of(G, z)];
+  float* __restrict__ stats = g.stats + 4 * (z - g.z0);
+  stats[0] = G.st.sv[z];
+  stats[1] = static_cast<float>(G.st.pi_iters[z]);
+  stats[2] = static_cast<float>(G.st.count[z]);
+  stats[3] = G.st.err[z];
 }
 
-static size_t root_state_floats(int batch) { return static_cast<size_t>(batch) * (4 + RCHUNKS + 8) + 16; }
+// ---- products on small tiles ----------------------------------------------------------------------------------------------
 
-}  // namespace ak
+enum RootKind { kFp32Tile32 = 0, kFp32Tile64 = 1, kPlanes2 = 2, kPlanes3 = 3, kFp32Early = 4 };
+enum RootWhen { kAlways = 0, kEarlySteps = 1, kLateSteps = 2 };     // (of each matrix's own count: a caller in parts does not say)
+struct RootJob {
+  float* bufs;                  // of its group
+  int64_t buf_elems, mat_elems; // floats (planes: 16-bit elements) between buffers, between matrices
+  PairedBuf a, b, c, c2;        // C = A B; c2.index >= 0: the product that forms M', which also writes the next T and the error
+  int n, ld;                    // ld: padded size on planes
+  int z0, tiles;                // first matrix; tiles of one matrix: those on one side of the diagonal, all for the early steps
+  int kind, when;
+  float scale_r;
+};
+constexpr int kRootMaxJobs = 2 * kRootMaxGroups;
+struct RootJobs {
+  int first[kRootMaxJobs];      // first work group of each job, INT32_MAX behind the last
+  RootJob j[kRootMaxJobs];
+};
 
-extern "C" size_t ak_inv_root_ws_bytes(int64_t n, int batch) {
-  if (n <= 0 || batch <= 0) return 0;
-  // the matrix buffers, two vectors, state
-  return (static_cast<size_t>(batch) * (ak::root_matrix_floats(n) + 2 * n) + ak::root_state_floats(batch)) * sizeof(float);
-}
+constexpr int kRootKC = 256;        // columns of a chunk of the 32 x 32 tile, 64 per wave
 
-namespace ak {
-
-// Workspace layout: M (two buffers), the second root buffer (the first is the caller's result), T (two buffers), four
-// product buffers, two vectors, then the per-matrix state; `active` (int32 per matrix, non-zero while its Newton
-// iteration runs) sits at root_active_offset().
-static size_t root_active_offset(int64_t n, int batch) {
-  return (static_cast<size_t>(batch) * (root_matrix_floats(n) + 2 * n) + static_cast<size_t>(batch) * (4 + RCHUNKS + 2)) * sizeof(float);
-}
-
-// phases: 1 = power iteration, ridge and start of the Newton iteration; 2 = `iters` Newton iterations; 4 = statistics
-static int inv_root_run(int phases, int iters, float* S, int64_t n, int batch, int64_t strideS, int p, float ridge_eps,
-                        const float* v0, int max_power_iter, float power_tol, int max_iter, float tol, float* out,
-                        int64_t strideOut, float* stats, void* ws, size_t ws_bytes, ak_stream_t stream) {
-  if (S == nullptr || v0 == nullptr || out == nullptr || stats == nullptr || n < 2 || batch <= 0 || p < 1 ||
-      n > (1 << 20) || strideS < n * n || strideOut < n * n)
-    return AK_ERR_ARG;
-  if (ws == nullptr || ws_bytes < ak_inv_root_ws_bytes(n, batch)) return AK_ERR_WORKSPACE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t nn = n * n;
-  float* w = static_cast<float*>(ws);
-  const bool planes = root_uses_planes(n);
-  // two fp16 planes where the ridge bounds the root, else three bf16 planes; every part of a computation in parts
-  // gets the same ridge_eps and p, hence the same answer
-  const float scale_r = root_fp16_scale(n, p, ridge_eps);
-  const int np = scale_r > 0.f ? 2 : 3;
-  const int64_t n_pad = root_pad(n), set_elems = np * n_pad * n_pad;      // 16-bit elements of one plane set
-  float* Mb[2] = {nullptr, nullptr};
-  float* root1 = nullptr;
-  float* Tb[2] = {nullptr, nullptr};
-  float* buf[4] = {nullptr, nullptr, nullptr, nullptr};
-  __bf16* pR[2] = {nullptr, nullptr};
-  __bf16* pM[2] = {nullptr, nullptr};
-  __bf16* pT[2] = {nullptr, nullptr};
-  __bf16* pbuf[4] = {nullptr, nullptr, nullptr, nullptr};
-  if (planes) {
-    __bf16* q = reinterpret_cast<__bf16*>(w);
-    for (int i = 0; i < 2; ++i) { pR[i] = q; q += batch * set_elems; }
-    for (int i = 0; i < 2; ++i) { pM[i] = q; q += batch * set_elems; }
-    for (int i = 0; i < 2; ++i) { pT[i] = q; q += batch * set_elems; }
-    for (int i = 0; i < 4; ++i) { pbuf[i] = q; q += batch * set_elems; }
-  } else {
-    float* q = w;
-    Mb[0] = q;           q += batch * nn;
-    Mb[1] = q;           q += batch * nn;
-    root1 = q;           q += batch * nn;
-    Tb[0] = q;           q += batch * nn;
-    Tb[1] = q;           q += batch * nn;
-    for (int i = 0; i < 4; ++i) { buf[i] = q; q += batch * nn; }
+// One 64 x 64 tile (ti, tj) of C = A B for the early steps: every tile of the product (nothing is mirrored), k pairs
+// (16 t + m, 16 t + 8 + m) in order on one accumulator, chunks of 128 k.  lds: deep_lds_floats<64, 64, 128>() floats.
+__device__ __forceinline__ void root_tile_early(const GemmParams& p, int ti, int tj, float* lds) {
+  using P = DeepPanel<64, 128>;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
+  const int wr = wave >> 1, wc = wave & 1, i0 = 64 * ti, j0 = 64 * tj, ld = static_cast<int>(p.lda);
+  float* ldsA = lds;
+  float* ldsB = lds + P::FLOATS;
+  const float* pa = ldsA + (32 * wr + l32) * P::KC_LD + 8 * g;
+  const float* pb = ldsB + 8 * g * P::IC_LD + 32 * wc + l32;
+  floatx16 acc, tot;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = tot[r] = 0.f;
+  P::Regs ra, rb;
+  deep_fetch<64, 128>(ra, p.A, ld, true, i0, p.M, 0, ld, tid);
+  deep_fetch<64, 128>(rb, p.B, ld, false, j0, ld, 0, p.M, tid);
+  for (int k0 = 0; k0 < p.M; k0 += 128) {
+    if (k0 != 0) __syncthreads();
+    deep_stash<64, 128>(ra, ldsA, true, tid);
+    deep_stash<64, 128>(rb, ldsB, false, tid);
+    __syncthreads();
+    if (k0 + 128 < p.M) {
+      deep_fetch<64, 128>(ra, p.A, ld, true, i0, p.M, k0 + 128, ld, tid);
+      deep_fetch<64, 128>(rb, p.B, ld, false, j0, ld, k0 + 128, p.M, tid);
+    }
+#pragma unroll 2
+    for (int t = 0; t < 8; ++t) {
+      const floatx4 lo = *reinterpret_cast<const floatx4*>(pa + 16 * t), hi = *reinterpret_cast<const floatx4*>(pa + 16 * t + 4);
+      float b[8];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) b[m] = pb[(16 * t + m) * P::IC_LD];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) acc = mfma_f32(m < 4 ? lo[m] : hi[m - 4], b[m], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      tot[r] += acc[r];
+      acc[r] = 0.f;
+    }
   }
-  w += static_cast<size_t>(batch) * root_matrix_floats(n);
-  float* v = w;        w += batch * n;
-  float* mv = w;       w += batch * n;
-  RootState st;
-  st.sv = w; w += batch;
-  st.nrm2 = w; w += batch;
-  st.err = w; w += batch;
-  st.zscale = w; w += batch;
-  st.partial = w; w += static_cast<size_t>(batch) * RCHUNKS;
-  st.pi_active = reinterpret_cast<int*>(w); w += batch;
-  st.pi_iters = reinterpret_cast<int*>(w); w += batch;
-  st.active = reinterpret_cast<int*>(w); w += batch;
-  st.commit = reinterpret_cast<int*>(w); w += batch;
-  st.count = reinterpret_cast<int*>(w); w += batch;
-  st.par = reinterpret_cast<int*>(w); w += batch;
-  st.errword = w; w += batch;
-  st.ovf = reinterpret_cast<int*>(w); w += batch;
+  float vmax = 0.f;
+  const int gj = j0 + 32 * wc + l32;
+  if (gj < p.M) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int gi = i0 + 32 * wr + 8 * (r >> 2) + 4 * g + (r & 3);
+      if (gi >= p.M) continue;
+      p.C[static_cast<int64_t>(gi) * ld + gj] = tot[r];
+      vmax = gemm_fold_absmax(vmax, tot[r], gi == gj, 1);
+      if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi) * ld + gj] = p.c2_scale * tot[r] + (gi == gj ? p.c2_diag : 0.f);
+    }
+  }
+  if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out, vmax, lane);
+}
 
-  if (reinterpret_cast<unsigned char*>(st.active) != static_cast<unsigned char*>(ws) + root_active_offset(n, batch))
-    return AK_ERR_ARG;     // the layout above and root_active_offset() have to agree
-  const dim3 gb(batch), gc(RCHUNKS, batch), b256(256);
+// One 32 x 32 tile (ti >= tj) of C = A B for symmetric matrices stored as n rows of ld: rows of A times rows of B, the
+// contraction of every chunk split over the four waves, which are added up through the LDS at the end.  Four times the
+// tiles of the 64-wide form and a quarter of its matrix instructions per wave: n = 784 takes 325 work groups of 6 us
+// instead of 91 of 15.
+__device__ __forceinline__ void root_tile32(const GemmParams& p, int ti, int tj, float* lds) {
+  using P = DeepPanel<32, kRootKC>;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
+  const int i0 = 32 * ti, j0 = 32 * tj, ld = static_cast<int>(p.lda);
+  float* ldsA = lds;
+  float* ldsB = lds + 32 * P::KC_LD;
+  const float* pa = ldsA + l32 * P::KC_LD + 64 * wave + 4 * g;
+  const float* pb = ldsB + l32 * P::KC_LD + 64 * wave + 4 * g;
+  floatx16 acc, part[2];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = part[0][r] = part[1][r] = 0.f;
+  typename P::Regs ra, rb;
+  deep_fetch<32, kRootKC>(ra, p.A, ld, true, i0, p.M, 0, ld, tid);         // (the padding columns are zero)
+  deep_fetch<32, kRootKC>(rb, p.B, ld, true, j0, p.M, 0, ld, tid);
+  for (int k0 = 0; k0 < ld; k0 += kRootKC) {
+    if (k0 != 0) __syncthreads();
+    deep_stash<32, kRootKC>(ra, ldsA, true, tid);
+    deep_stash<32, kRootKC>(rb, ldsB, true, tid);
+    __syncthreads();
+    if (k0 + kRootKC < ld) {
+      deep_fetch<32, kRootKC>(ra, p.A, ld, true, i0, p.M, k0 + kRootKC, ld, tid);
+      deep_fetch<32, kRootKC>(rb, p.B, ld, true, j0, p.M, k0 + kRootKC, ld, tid);
+    }
+    if (k0 + 64 * wave < ld) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const floatx4 a = *reinterpret_cast<const floatx4*>(pa + 8 * q), b = *reinterpret_cast<const floatx4*>(pb + 8 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[e & 1] = mfma_f32(a[e], b[e], part[e & 1]);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        acc[r] += part[0][r] + part[1][r];
+        part[0][r] = part[1][r] = 0.f;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) lds[(16 * wave + r) * 64 + lane] = acc[r];
+  __syncthreads();
+  // wave w adds up registers 4 w ... 4 w + 3: rows 8 w + 4 g + e, column l32
+  floatx4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float* q = lds + (4 * wave + e) * 64 + lane;
+    v[e] = (q[0] + q[16 * 64]) + (q[32 * 64] + q[48 * 64]);
+  }
+  // exactly symmetric: a tile on the diagonal keeps its lower triangle and mirrors it element by element (the next product
+  // reads this matrix as its own transpose; what is not symmetric grows from step to step)
+  const int gi = i0 + 8 * wave + 4 * g, gj = j0 + l32;
+  float vmax = 0.f;
+  if (gj < p.M) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (gi + e >= p.M || gi + e < gj) continue;
+      p.C[static_cast<int64_t>(gi + e) * ld + gj] = v[e];
+      vmax = gemm_fold_absmax(vmax, v[e], gi + e == gj, 1);
+      if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi + e) * ld + gj] = p.c2_scale * v[e] + (gi + e == gj ? p.c2_diag : 0.f);
+    }
+    float* dst = p.C + static_cast<int64_t>(gj) * ld + gi;
+    float* dst2 = p.C2 != nullptr ? p.C2 + static_cast<int64_t>(gj) * ld + gi : nullptr;
+    floatx4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (gi + e >= p.M) v[e] = 0.f;              // a mirrored row ends in the padding columns, which stay zero
+      w[e] = p.c2_scale * v[e];
+    }
+    if (ti != tj) {
+      if (gi < p.M) {
+        *reinterpret_cast<floatx4*>(dst) = v;
+        if (dst2 != nullptr) *reinterpret_cast<floatx4*>(dst2) = w;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (gi + e <= gj || gi + e >= p.M) continue;
+        dst[e] = v[e];
+        if (dst2 != nullptr) dst2[e] = w[e];
+      }
+    }
+  }
+  if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out, vmax, lane);
+}
+
+// A product on planes (fp16 planes: the two roots carry scale_r, every other matrix kRootScaleM).
+__host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0, int np, int n, int n_pad, int tile, float scale_r,
+                                                     float* bufs, int64_t buf_elems, PairedBuf a, PairedBuf b, PairedBuf c,
+                                                     PairedBuf c2) {
+  PlaneGemm pg;
+  pg.bufs = reinterpret_cast<__bf16*>(bufs);
+  pg.plane_elems = static_cast<int64_t>(n_pad) * n_pad;
+  pg.set_elems = np * pg.plane_elems;
+  pg.buf_elems = buf_elems;
+  pg.A = a; pg.B = b; pg.C = c; pg.C2 = c2;
+  pg.count = st.count + z0;
+  pg.coef = st.coef + static_cast<int64_t>(z0) * 2 * kRootSteps;
+  pg.coef_stride = 2 * kRootSteps; pg.coef_last = kRootSteps - 1;
+  pg.errword = c2.index >= 0 ? st.errword + z0 * kErrStride : nullptr;
+  pg.active = st.active + z0;
+  pg.overflow = st.ovf + z0;
+  pg.n = n; pg.n_pad = n_pad; pg.T = n_pad / tile;
+  const float sa = a.index == 0 ? scale_r : kRootScaleM, sb = b.index == 0 ? scale_r : kRootScaleM;
+  pg.in_unscale = 1.0f / (sa * sb);
+  pg.c_scale = c.index == 0 ? scale_r : kRootScaleM;
+  pg.c2_plane_scale = kRootScaleM;
+  return pg;
+}
+
+__device__ __forceinline__ bool root_idle(const RootState& st, const RootJob& job, int z, int steps) {
+  return st.active[z] == 0 || (steps == 0 && job.c.index == 0) ||          // (the first X is written by the start)
+         (job.when == kEarlySteps && steps >= kRootEarly) || (job.when == kLateSteps && steps < kRootEarly);
+}
+
+// The product of matrix zl of a group in fp32; c2_*: of the step `steps` is followed by.
+__device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, const RootJob& job, int zl, int z, int steps) {
+  const int parity = steps & 1;
+  float* base = job.bufs + zl * job.mat_elems;
+  GemmParams p;
+  p.A = base + paired_buf(job.a, parity) * job.buf_elems;
+  p.B = base + paired_buf(job.b, parity) * job.buf_elems;
+  p.C = base + paired_buf(job.c, parity) * job.buf_elems;
+  p.lda = p.ldb = p.ldc = job.ld;
+  p.M = p.N = job.n;
+  p.K = job.ld;
+  p.transB = 1;                 // (a symmetric operand is its own transpose)
+  p.tile_mode = TILE_LOWER_MIRROR;
+  if (job.c2.index >= 0) {
+    const float* next = st.coef + z * 2 * kRootSteps + 2 * min(steps + 1, kRootSteps - 1);
+    p.C2 = base + paired_buf(job.c2, parity) * job.buf_elems;
+    p.ldc2 = job.ld;
+    p.c2_diag = next[0];
+    p.c2_scale = -next[1];
+    p.absmax_out = st.errword + z * kErrStride;
+    p.absmax_identity = 1;
+  }
+  return p;
+}
+
+// Early products of a group in fp32 with many wide matrices: 128 x 128 tiles of the three-piece split (gemm_x3.hpp).
+static __global__ __launch_bounds__(256) void root_split_kernel(RootState st, RootJob job) {
+  __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 2 * 3 * X3_PLANE];
+  const int zl = static_cast<int>(blockIdx.x) / job.tiles, z = job.z0 + zl, local = static_cast<int>(blockIdx.x) - zl * job.tiles;
+  const int steps = st.count[z], T = (job.n + X3_BT - 1) / X3_BT;
+  if (root_idle(st, job, z, steps)) return;
+  GemmParams p = root_fp32_product(st, job, zl, z, steps);
+  p.K = job.n;
+  p.transB = 0;
+  p.tile_mode = TILE_ALL;
+  gemm_x3_tile<3, true, 1, 0, false, true>(p, local / T, local % T, 0, (AK_LDS3 unsigned char*)x3_smem);
+}
+
+// One step of the product sequences of all groups on small tiles: a work group per tile of any product.
+static __global__ __launch_bounds__(256, 2) void root_small_kernel(RootState st, RootJobs J) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
+  const int wg = blockIdx.x;
+  int ji = 0;
+#pragma unroll
+  for (int k = 1; k < kRootMaxJobs; ++k) ji += wg >= J.first[k] ? 1 : 0;
+  const RootJob job = J.j[ji];
+  int local = wg - J.first[ji];
+  const int zl = local / job.tiles, z = job.z0 + zl;
+  local -= zl * job.tiles;
+  const int steps = st.count[z];
+  if (root_idle(st, job, z, steps)) return;
+  float* lds = reinterpret_cast<float*>(dtl_smem);
+  if (job.kind == kFp32Early) {
+    const int T = (job.n + 63) / 64;
+    root_tile_early(root_fp32_product(st, job, zl, z, steps), local / T, local % T, lds);
+    return;
+  }
+  int ti, tj;
+  decode_lower_tile(local, ti, tj);
+  if (job.kind == kPlanes2 || job.kind == kPlanes3) {
+    const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
+                                         job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
+    if (job.kind == kPlanes2) plane_tile_small<2>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
+    else plane_tile_small<3>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
+    return;
+  }
+  const GemmParams p = root_fp32_product(st, job, zl, z, steps);
+  if (job.kind == kFp32Tile32) root_tile32(p, ti, tj, lds);
+  else gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
+}
+
+// ---- host ----------------------------------------------------------------------------------------------------------
+
+enum RootBuf { R0 = 0, M0 = 2, T0 = 4, B0 = 6 };
+constexpr PairedBuf kRin{R0, 1}, kRout{R0, 2}, kMin{M0, 1}, kMout{M0, 2}, kTin{T0, 1}, kTout{T0, 2}, kNone{-1, 0};
+
+struct RootOp { PairedBuf a, b, c, c2; };
+
+// The products of one Newton step by slots: the products of a slot are independent of each other.  T^p by repeated
+// squaring, with the multiplication order of the reference's MatPower for other powers.
+static int root_ops(int p, RootOp (*slots)[2], int* counts, int max_slots) {
+  int n = 0;
+  auto put = [&](PairedBuf a, PairedBuf b, PairedBuf c, PairedBuf c2) {
+    if (n < max_slots) { slots[n][0] = RootOp{a, b, c, c2}; counts[n] = 1; }
+    ++n;
+  };
+  auto same = [](PairedBuf x, PairedBuf y) { return x.index == y.index && x.sel == y.sel; };
+  PairedBuf base = kTin, power = kNone;
+  auto free_buf = [&] {
+    for (int i = 0; i < 4; ++i) {
+      const PairedBuf b{static_cast<int16_t>(B0 + i), 0};
+      if (!same(b, base) && !same(b, power)) return b;
+    }
+    return PairedBuf{B0 + 3, 0};
+  };
+  for (int q = p; q > 0; q /= 2) {
+    if (q & 1) {
+      if (power.index < 0) {
+        power = base;
+      } else {
+        const PairedBuf out = free_buf();
+        put(base, power, out, kNone);
+        power = out;
+      }
+    }
+    if (q / 2 > 0) {
+      const PairedBuf out = free_buf();
+      put(base, base, out, kNone);
+      base = out;
+    }
+  }
+  put(power, kMin, kMout, kTout);                                  // M' = T^p M, its error, the next T
+  if (n > max_slots) return -1;
+  slots[0][1] = RootOp{kRin, kTin, kRout, kNone};                  // X' = X T, beside the first of them
+  counts[0] = 2;
+  return n;
+}
+
+static size_t root_state_floats(int total) {
+  return static_cast<size_t>(total) * (3 + 2 * RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 16;
+}
+static size_t root_group_floats(int64_t n, int64_t batch) {
+  const size_t m = (static_cast<size_t>(batch) * root_matrix_floats(n, batch) + 63) / 64 * 64;
+  return m + (static_cast<size_t>(5) * batch * n + 63) / 64 * 64;
+}
+static bool root_args_ok(const int64_t* n, const int* batch, int groups) {
+  if (n == nullptr || batch == nullptr || groups <= 0 || groups > kRootMaxGroups) return false;
+  int64_t total = 0;
+  for (int i = 0; i < groups; ++i) {
+    if (n[i] <= 0 || n[i] > 32768 || batch[i] <= 0) return false;
+    total += batch[i];
+  }
+  return total <= 65535;
+}
+// bytes from the workspace's start to the `active` words
+static size_t root_active_offset(const int64_t* n, const int* batch, int groups) {
+  size_t off = 0;
+  for (int i = 0; i < groups; ++i) off += root_group_floats(n[i], batch[i]);
+  return off * sizeof(float);
+}
+
+// phases: 1 = power iteration, ridge and start of the Newton iteration; 2 = `iters` Newton iterations, the first of which
+// is number `begin` of the computation (-1: not known); 4 = results and statistics
+static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge_eps, int max_power_iter, float power_tol,
+                    int max_iter, float tol, hipStream_t s) {
+  const int total = G.total;
+  const dim3 gz(total), gc(RCHUNKS, total), b256(256), b64(64);
   if (phases & 1) {
-    hipLaunchKernelGGL(root_init_kernel, gb, b256, 0, s, st, v0, v, n);
-    const dim3 gmv(static_cast<unsigned>((n + 3) / 4), batch);
-    for (int it = 0; it < max_power_iter; ++it) {
-      hipLaunchKernelGGL(power_matvec_kernel, gmv, b256, 0, s, st, S, strideS, v, mv, n);
-      hipLaunchKernelGGL(power_update_kernel, gb, b256, 0, s, st, v, mv, n, power_tol, max_power_iter);
+    const int steps = std::min(kLanczosSteps, std::max(1, max_power_iter));
+    LanczosGroups L;
+    int blocks = 0, widest = 0;
+    for (int i = 0; i < kRootMaxGroups; ++i) {
+      L.first[i] = i < G.count ? blocks : INT32_MAX;
+      if (i >= G.count) continue;
+      const RootGroup& g = G.g[i];
+      L.g[i] = LanczosGroup{g.S, g.v0, g.vec, g.strideS, g.n, g.batch, g.z0, 0};
+      blocks += g.batch * ((g.n + kLanczosRows - 1) / kLanczosRows);
+      widest = std::max(widest, g.n);
     }
-    hipLaunchKernelGGL(root_ridge_kernel, gc, b256, 0, s, st, S, strideS, n, ridge_eps);
-    hipLaunchKernelGGL(root_zscale_kernel, gb, dim3(64), 0, s, st, p);
-    if (planes && np == 2)
-      hipLaunchKernelGGL(root_start_planes_kernel<2>, gc, b256, 0, s, st, S, strideS, pM[0], pT[0], pR[0], set_elems, n, n_pad,
-                         p, kRootScaleM, scale_r);
-    else if (planes)
-      hipLaunchKernelGGL(root_start_planes_kernel<3>, gc, b256, 0, s, st, S, strideS, pM[0], pT[0], pR[0], set_elems, n, n_pad,
-                         p, 1.f, 1.f);
-    else
-      hipLaunchKernelGGL(root_start_kernel, gc, b256, 0, s, st, S, strideS, Mb[0], Tb[0], out, strideOut, n, p);
-    hipLaunchKernelGGL(root_begin_kernel, gb, dim3(64), 0, s, st, tol, max_iter);
+    const size_t lds = static_cast<size_t>(widest) * sizeof(float);
+    static bool attr_set = false;     // idempotent; a race sets it twice at worst
+    if (lds > 60 * 1024 && !attr_set) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_lanczos_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              32768 * static_cast<int>(sizeof(float))) != hipSuccess)
+        return AK_ERR_LAUNCH;
+      attr_set = true;
+    }
+    for (int j = 0; j < steps; ++j) hipLaunchKernelGGL(root_lanczos_kernel, dim3(blocks), b256, lds, s, G.st, L, j);
+    hipLaunchKernelGGL(root_power_kernel, gz, b64, 0, s, G, steps, power_tol, max_power_iter);
+    hipLaunchKernelGGL(root_ridge_kernel, gc, b256, 0, s, G, ridge_eps);
+    hipLaunchKernelGGL(root_schedule_kernel, gz, b64, 0, s, G, ridge_eps, max_iter);
+    bool fp32 = false;
+    for (int i = 0; i < G.count; ++i) {
+      const RootGroup& g = G.g[i];
+      const dim3 gp(RCHUNKS, g.batch);
+      if (g.np == 2) hipLaunchKernelGGL(root_start_planes_kernel<2>, gp, b256, 0, s, G.st, g);
+      else if (g.np == 3) hipLaunchKernelGGL(root_start_planes_kernel<3>, gp, b256, 0, s, G.st, g);
+      else fp32 = true;
+    }
+    if (fp32) hipLaunchKernelGGL(root_start_kernel, gc, b256, 0, s, G);
+    hipLaunchKernelGGL(root_begin_kernel, gz, b64, 0, s, G.st, tol, max_iter);
   }
-  if (!(phases & 2)) iters = 0;
-
-  const int N = static_cast<int>(n);
-  // The matrices of the iteration by number: two roots, two M, two T, four product buffers.  fp32 form: the first
-  // root is the caller's `out`; plane form: all ten are plane sets of the workspace.
-  enum { R0 = 0, R1, M0, M1, T0, T1, B0, B1, B2, B3, NBUF };
-  float* fptr[NBUF] = {out, root1, Mb[0], Mb[1], Tb[0], Tb[1], buf[0], buf[1], buf[2], buf[3]};
-  int64_t fstride[NBUF];
-  for (int i = 0; i < NBUF; ++i) fstride[i] = nn;
-  fstride[R0] = strideOut;
-  __bf16* pptr[NBUF] = {pR[0], pR[1], pM[0], pM[1], pT[0], pT[1], pbuf[0], pbuf[1], pbuf[2], pbuf[3]};
-  // C = A B for every matrix that still iterates.  next_T >= 0 (the product that forms M' only): the epilogue also
-  // folds max |C - I| into the matrix's error word and writes the polynomial of the next step, (1 + 1/p) I - C / p.
-  auto mm = [&](int ia, int ib, int ic, int next_T) {
-    if (planes) {
-      PlaneGemm g{};
-      g.A = pptr[ia]; g.B = pptr[ib]; g.C = pptr[ic];
-      g.sA = g.sB = g.sC = g.sC2 = set_elems;
-      g.plane_elems = n_pad * n_pad;
-      g.n = N; g.n_pad = static_cast<int>(n_pad); g.T = static_cast<int>(n_pad / kPlaneTile);
-      g.active = st.active;
-      g.overflow = st.ovf;
-      if (next_T >= 0) {
-        g.errword = st.errword;
-        g.C2 = pptr[next_T];
-        g.c2_scale = -1.0f / p; g.c2_diag = 1.0f + 1.0f / p;
-      }
-      // fp16 planes: the two roots carry scale_r, every other matrix kRootScaleM
-      const float sa = ia <= R1 ? scale_r : kRootScaleM, sb = ib <= R1 ? scale_r : kRootScaleM;
-      g.in_unscale = 1.0f / (sa * sb);
-      g.c_scale = ic <= R1 ? scale_r : kRootScaleM;
-      g.c2_plane_scale = kRootScaleM;
-      return launch_plane_gemm(g, np, batch, s);
+  if (phases & 2) {
+    constexpr int kMaxSlots = 64;
+    RootOp slots[kRootMaxGroups][kMaxSlots][2];
+    int counts[kRootMaxGroups][kMaxSlots], nslots[kRootMaxGroups], most = 0;
+    for (int i = 0; i < G.count; ++i) {
+      nslots[i] = root_ops(G.g[i].p, slots[i], counts[i], kMaxSlots);
+      if (nslots[i] < 0) return AK_ERR_ARG;
+      most = std::max(most, nslots[i]);
     }
-    GemmParams g = make_gemm(0, 0, N, N, N, 1.f, fptr[ia], n, fptr[ib], n, 0.f, fptr[ic], n);
-    g.sA = fstride[ia]; g.sB = fstride[ib]; g.sC = fstride[ic];
-    g.active = st.active; g.active_stride = 1;
-    g.split = g_root_split;
-    // sums in chunks: the error of the root is set by the absolute rounding error of the first iterations' products
-    // against the smallest eigenvalues of M (ridge_eps of the largest); a rank-deficient 1024 x 1024 statistic lost a
-    // factor of six against LAPACK-grade fp32 products with one accumulator rounded at every matrix instruction
-    g.chunked = 1;
-    if (next_T >= 0) {
-      g.absmax_out = st.errword; g.absmax_stride = 1; g.absmax_identity = 1;
-      g.C2 = fptr[next_T]; g.ldc2 = n; g.sC2 = fstride[next_T];
-      g.c2_scale = -1.0f / p; g.c2_diag = 1.0f + 1.0f / p;
-    }
-    // Every matrix of the iteration is a polynomial of the one symmetric statistic, so every product is symmetric up
-    // to rounding: large ones compute the tiles on and below the diagonal only and mirror them (half the work; the
-    // results are then exactly symmetric).  Small ones keep the full product.
-    if (N >= kRootSymmetricMinDim) g.tile_mode = TILE_LOWER_MIRROR;
-    return launch_gemm(g, batch, s);
-  };
-  auto copy = [&](int dst, int src) {
-    const hipError_t e = planes
-        ? hipMemcpyAsync(pptr[dst], pptr[src], sizeof(__bf16) * batch * set_elems, hipMemcpyDeviceToDevice, s)
-        : hipMemcpyAsync(fptr[dst], fptr[src], sizeof(float) * batch * nn, hipMemcpyDeviceToDevice, s);
-    return e == hipSuccess ? AK_OK : AK_ERR_LAUNCH;
-  };
-  // Iteration j of this call reads the buffer pair j % 2 (R, M, T) and writes the other one; an accepted step moves the
-  // matrix's mark (st.par) there, so nothing is copied per step.  Every call starts with all marks on pair 0 and ends
-  // by bringing the marked matrices back to it.
-  for (int it = 0; it < iters; ++it) {
-    const int a = it & 1, b = a ^ 1;
-    const int T = T0 + a;
-    int rc = mm(R0 + a, T, R0 + b, -1);                          // new_root = root T
-    if (rc != AK_OK) return rc;
-    // T^p with the multiplication order of MatPower
-    int tp = -1;
-    if ((p & (p - 1)) == 0) {
-      int cur = T, which = B1;
-      for (int done = 1; done < p; done *= 2) {
-        rc = mm(cur, cur, which, -1);
-        if (rc != AK_OK) return rc;
-        cur = which;
-        which = (which == B1) ? B2 : B1;
+    // 32-wide fp32 tiles while a launch's run side by side: four times the tiles of the 64-wide form, each a third as long
+    int64_t small_tiles = 0;
+    for (int i = 0; i < G.count; ++i)
+      if (G.g[i].np == 0) {
+        const int64_t t = (G.g[i].n + 31) / 32;
+        small_tiles += t * (t + 1) / 2 * G.g[i].batch;
       }
-      tp = cur;
-    } else {
-      int base = T, power = -1;     // squares ping-pong in B0 / B1, the running power in B2 / B3
-      int sq = B0, pw = B2;
-      for (int q = p; q > 0; q /= 2) {
-        if (q & 1) {
-          if (power < 0) {
-            power = base;
-          } else {
-            rc = mm(base, power, pw, -1);
-            if (rc != AK_OK) return rc;
-            power = pw;
-            pw = (pw == B2) ? B3 : B2;
+    const int fp32_tile = small_tiles <= 512 ? 32 : 64;
+    constexpr int kLds[5] = {2 * 32 * DeepPanel<32, kRootKC>::KC_LD * 4, deep_lds_floats<64, 64, 128>() * 4, 4 * 8 * 4096,
+                             3 * 12 * 4096, deep_lds_floats<64, 64, 128>() * 4};    // by kind (planes: their stages)
+    static bool attr_set = false;     // idempotent; a race sets it twice at worst
+    if (!attr_set) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_small_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kLds[3]) != hipSuccess)
+        return AK_ERR_LAUNCH;
+      attr_set = true;
+    }
+    for (int it = 0; it < iters; ++it) {
+      const bool early = begin < 0 || begin + it < kRootEarly, late = begin < 0 || begin + it >= kRootEarly;
+      for (int k = 0; k < most; ++k) {
+        RootJobs J;
+        int jobs = 0, blocks = 0, lds = 0;
+        for (int i = 0; i < G.count; ++i) {
+          const RootGroup& g = G.g[i];
+          if (k >= nslots[i]) continue;
+          const int64_t mat = g.np == 0 ? static_cast<int64_t>(g.n) * g.ld : static_cast<int64_t>(g.np) * g.n_pad * g.n_pad;
+          for (int o = 0; o < counts[i][k]; ++o) {
+            const RootOp& op = slots[i][k][o];
+            if (g.np != 0 && g.tile == kPlaneTile) {
+              const int rc = launch_plane_gemm(root_plane_gemm(G.st, g.z0, g.np, g.n, g.n_pad, g.tile, g.scale_r, g.bufs,
+                                                               mat * g.batch, op.a, op.b, op.c, op.c2), g.np, g.batch, s);
+              if (rc != AK_OK) return rc;
+              continue;
+            }
+            RootJob job;
+            job.bufs = g.bufs; job.buf_elems = mat * g.batch; job.mat_elems = mat;
+            job.a = op.a; job.b = op.b; job.c = op.c; job.c2 = op.c2;
+            job.n = g.n; job.ld = g.np == 0 ? g.ld : g.n_pad;
+            job.z0 = g.z0;
+            job.scale_r = g.scale_r;
+            auto put = [&](int kind, int when, int tiles) {
+              job.kind = kind; job.when = when; job.tiles = tiles;
+              J.first[jobs] = blocks;
+              J.j[jobs++] = job;
+              blocks += tiles * g.batch;
+              lds = std::max(lds, kLds[kind]);
+            };
+            if (g.np != 0) {
+              const int t = g.n_pad / kPlaneSmallTile;
+              put(g.np, kAlways, t * (t + 1) / 2);
+              continue;
+            }
+            if (early) {
+              const int t128 = (g.n + 127) / 128, t64 = (g.n + 63) / 64;
+              if (t128 * t128 * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0) {
+                job.kind = kFp32Early; job.when = kEarlySteps; job.tiles = t128 * t128;
+                hipLaunchKernelGGL(root_split_kernel, dim3(job.tiles * g.batch), b256, 0, s, G.st, job);
+              } else {
+                put(kFp32Early, kEarlySteps, t64 * t64);
+              }
+            }
+            if (late) {
+              const int t = (g.n + fp32_tile - 1) / fp32_tile;
+              put(fp32_tile == 32 ? kFp32Tile32 : kFp32Tile64, kLateSteps, t * (t + 1) / 2);
+            }
           }
         }
-        if (q / 2 > 0) {
-          if (power == base && base != T) {      // a later square would overwrite the value `power` points at
-            rc = copy(pw, base);
-            if (rc != AK_OK) return rc;
-            power = pw;
-            pw = (pw == B2) ? B3 : B2;
-          }
-          rc = mm(base, base, sq, -1);
-          if (rc != AK_OK) return rc;
-          base = sq;
-          sq = (sq == B0) ? B1 : B0;
-        }
+        if (jobs == 0) continue;
+        for (int i = jobs; i < kRootMaxJobs; ++i) J.first[i] = INT32_MAX;
+        hipLaunchKernelGGL(root_small_kernel, dim3(blocks), b256, lds, s, G.st, J);
       }
-      tp = power;
+      hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, tol, max_iter);
     }
-    rc = mm(tp, M0 + a, M0 + b, T0 + b);                         // M' = T^p M, its error, the next T
-    if (rc != AK_OK) return rc;
-    hipLaunchKernelGGL(newton_decide_kernel, gb, dim3(64), 0, s, st, tol, max_iter, b);
   }
-  if (iters > 0) {
-    if (planes) {
-      const int64_t words = set_elems / 2;
-      hipLaunchKernelGGL(newton_gather_planes_kernel, gc, b256, 0, s, st, reinterpret_cast<uint32_t*>(pR[0]),
-                         reinterpret_cast<const uint32_t*>(pR[1]), reinterpret_cast<uint32_t*>(pM[0]),
-                         reinterpret_cast<const uint32_t*>(pM[1]), reinterpret_cast<uint32_t*>(pT[0]),
-                         reinterpret_cast<const uint32_t*>(pT[1]), words);
-    } else {
-      hipLaunchKernelGGL(newton_gather_kernel, gc, b256, 0, s, st, out, strideOut, root1, Mb[0], Mb[1], Tb[0], Tb[1], n);
-    }
-    hipLaunchKernelGGL(newton_gathered_kernel, gb, dim3(64), 0, s, st);
+  if (phases & 4) {
+    hipLaunchKernelGGL(root_out_kernel, gc, b256, 0, s, G);
+    hipLaunchKernelGGL(root_stats_kernel, gz, b64, 0, s, G);
   }
-  // plane form: the caller's fp32 root is written with the statistics (the last part of a computation in parts)
-  if ((phases & 4) && planes) {
-    if (np == 2)
-      hipLaunchKernelGGL(root_out_planes_kernel<2>, gc, b256, 0, s, pR[0], set_elems, out, strideOut, n, n_pad, st.zscale, p,
-                         scale_r);
-    else
-      hipLaunchKernelGGL(root_out_planes_kernel<3>, gc, b256, 0, s, pR[0], set_elems, out, strideOut, n, n_pad, nullptr, p, 1.f);
-  }
-  if (phases & 4) hipLaunchKernelGGL(root_stats_kernel, gb, dim3(64), 0, s, st, stats);
   return check_launch();
 }
 
 }  // namespace ak
+
+extern "C" size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, int groups) {
+  if (!ak::root_args_ok(n, batch, groups)) return 0;
+  int total = 0;
+  for (int i = 0; i < groups; ++i) total += batch[i];
+  return ak::root_active_offset(n, batch, groups) + ak::root_state_floats(total) * sizeof(float);
+}
+
+extern "C" size_t ak_inv_root_group_active_offset(const int64_t* n, const int* batch, int groups) {
+  return ak::root_args_ok(n, batch, groups) ? ak::root_active_offset(n, batch, groups) : 0;
+}
+
+extern "C" int ak_inv_root_group(int phases, int begin, int iters, int groups, float* const* S, const int64_t* n,
+                                 const int* batch, const int64_t* strideS, const int* p, float ridge_eps,
+                                 const float* const* v0, int max_power_iter, float power_tol, int max_iter, float tol,
+                                 float* const* out, const int64_t* strideOut, float* const* stats, void* ws,
+                                 size_t ws_bytes, ak_stream_t stream) {
+  using namespace ak;
+  if (phases < 1 || phases > 7 || (begin < 0 && groups != 1) || iters < 0 || S == nullptr || strideS == nullptr ||
+      p == nullptr || v0 == nullptr || out == nullptr || strideOut == nullptr || stats == nullptr || !root_args_ok(n, batch, groups))
+    return AK_ERR_ARG;
+  if (ws == nullptr || ws_bytes < ak_inv_root_group_ws_bytes(n, batch, groups)) return AK_ERR_WORKSPACE;
+  RootGroups G;
+  G.count = groups;
+  G.total = 0;
+  float* w = static_cast<float*>(ws);
+  for (int i = 0; i < groups; ++i) {
+    if (S[i] == nullptr || v0[i] == nullptr || out[i] == nullptr || stats[i] == nullptr || n[i] < 2 || p[i] < 1 ||
+        strideS[i] < n[i] * n[i] || strideOut[i] < n[i] * n[i])
+      return AK_ERR_ARG;
+    RootGroup& g = G.g[i];
+    g.S = S[i]; g.out = out[i]; g.v0 = v0[i]; g.stats = stats[i];
+    g.strideS = strideS[i]; g.strideOut = strideOut[i];
+    g.n = static_cast<int>(n[i]); g.ld = static_cast<int>(root_ld(n[i])); g.batch = batch[i]; g.p = p[i];
+    g.z0 = G.total;
+    g.tile = root_plane_dim(n[i]) ? root_plane_tile(n[i], batch[i]) : kPlaneSmallTile;
+    g.n_pad = static_cast<int>(root_pad(n[i], g.tile));
+    // two fp16 planes where the ridge bounds the root, else three bf16 planes; every part of a computation in parts gets
+    // the same arguments, hence the same answer
+    g.scale_r = root_fp16_scale(n[i], p[i], ridge_eps);
+    g.np = !root_plane_dim(n[i]) ? 0 : (g.scale_r > 0.f ? 2 : 3);
+    g.bufs = w;
+    g.vec = w + (static_cast<size_t>(batch[i]) * root_matrix_floats(n[i], batch[i]) + 63) / 64 * 64;
+    w += root_group_floats(n[i], batch[i]);
+    G.total += batch[i];
+  }
+  const int total = G.total;
+  RootState& st = G.st;
+  auto ints = [&](int k) { int* r = reinterpret_cast<int*>(w); w += k; return r; };
+  auto floats = [&](int64_t k) { float* r = w; w += k; return r; };
+  st.active = ints(total);
+  st.count = ints(total);
+  st.accel = ints(total);
+  st.ovf = ints(total);
+  st.lz_dim = ints(total);
+  st.pi_iters = ints(total);
+  st.sv = floats(total);
+  st.err = floats(total);
+  st.zscale = floats(total);
+  st.errword = floats(static_cast<int64_t>(total) * kErrStride);
+  st.partial = floats(static_cast<int64_t>(total) * RCHUNKS);
+  st.partial_tr = floats(static_cast<int64_t>(total) * RCHUNKS);
+  st.alpha = floats(static_cast<int64_t>(total) * kLanczosSteps);
+  st.beta = floats(static_cast<int64_t>(total) * kLanczosSteps);
+  st.coef = floats(static_cast<int64_t>(total) * 2 * kRootSteps);
+  return root_run(phases, begin, iters, G, ridge_eps, max_power_iter, power_tol, max_iter, tol,
+                  static_cast<hipStream_t>(stream));
+}
+
+extern "C" int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps) {
+  if (n <= 0 || !ak::root_plane_dim(n)) return 0;
+  return ak::root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3;
+}
+
+extern "C" size_t ak_inv_root_ws_bytes(int64_t n, int batch) { return ak_inv_root_group_ws_bytes(&n, &batch, 1); }
 
 extern "C" int ak_inv_root_newton(float* S, int64_t n, int batch, int64_t strideS, int p, float ridge_eps,
                                   const float* v0, int max_power_iter, float power_tol, int max_iter, float tol,
                                   float* out, int64_t strideOut, float* stats, void* ws, size_t ws_bytes,
                                   ak_stream_t stream) {
-  return ak::inv_root_run(7, max_iter, S, n, batch, strideS, p, ridge_eps, v0, max_power_iter, power_tol, max_iter, tol,
-                          out, strideOut, stats, ws, ws_bytes, stream);
+  return ak_inv_root_group(7, 0, max_iter, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0, max_power_iter, power_tol,
+                           max_iter, tol, &out, &strideOut, &stats, ws, ws_bytes, stream);
 }
 
-extern "C" int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps) {
-  if (n <= 0 || !ak::root_uses_planes(n)) return 0;
-  return ak::root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3;
-}
-
-extern "C" size_t ak_inv_root_active_offset(int64_t n, int batch) {
-  if (n <= 0 || batch <= 0) return 0;
-  return ak::root_active_offset(n, batch);
-}
+extern "C" size_t ak_inv_root_active_offset(int64_t n, int batch) { return ak_inv_root_group_active_offset(&n, &batch, 1); }
 
 extern "C" int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batch, int64_t strideS, int p,
                                        float ridge_eps, const float* v0, int max_power_iter, float power_tol,
                                        int max_iter, float tol, float* out, int64_t strideOut, float* stats, void* ws,
                                        size_t ws_bytes, ak_stream_t stream) {
-  if (phases < 1 || phases > 7 || iters < 0) return AK_ERR_ARG;
-  return ak::inv_root_run(phases, iters, S, n, batch, strideS, p, ridge_eps, v0, max_power_iter, power_tol, max_iter,
-                          tol, out, strideOut, stats, ws, ws_bytes, stream);
+  return ak_inv_root_group(phases, (phases & 1) ? 0 : -1, iters, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0,
+                           max_power_iter, power_tol, max_iter, tol, &out, &strideOut, &stats, ws, ws_bytes, stream);
 }
-
-#ifdef AK_TUNING_HOOKS
-namespace ak {
-static __global__ void dbg_to_planes_kernel(const float* __restrict__ X, __bf16* __restrict__ P, int64_t n, int64_t n_pad) {
-  const int64_t total = n_pad * n_pad;
-  for (int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; at < total; at += static_cast<int64_t>(gridDim.x) * 256) {
-    const int64_t i = at / n_pad, j = at - i * n_pad;
-    const float x = (i < n && j < n) ? X[i * n + j] : 0.f;
-    unsigned short o[3];
-    plane_bits<3>(x, o);
-    unsigned short* Q = reinterpret_cast<unsigned short*>(P);
-    const int64_t dst = plane_index(i, j, n_pad);
-    Q[dst] = o[0]; Q[total + dst] = o[1]; Q[2 * total + dst] = o[2];
-  }
-}
-}  // namespace ak
-
-// Tuning builds only: C = A B for symmetric fp32 n x n matrices through the plane kernel (ws: 9 n_pad^2 bf16 + 1 float).
-extern "C" int ak_debug_plane_product(const float* A, const float* B, float* C, int64_t n, void* ws, float* err) {
-  using namespace ak;
-  const int64_t n_pad = root_pad(n), set = 3 * n_pad * n_pad;
-  __bf16* pa = static_cast<__bf16*>(ws);
-  __bf16* pb = pa + set;
-  __bf16* pc = pb + set;
-  float* word = reinterpret_cast<float*>(pc + set);
-  hipMemsetAsync(word, 0, 4, nullptr);
-  hipLaunchKernelGGL(dbg_to_planes_kernel, dim3(512), dim3(256), 0, nullptr, A, pa, n, n_pad);
-  hipLaunchKernelGGL(dbg_to_planes_kernel, dim3(512), dim3(256), 0, nullptr, B, pb, n, n_pad);
-  PlaneGemm g{};
-  g.A = pa; g.B = pb; g.C = pc;
-  g.sA = g.sB = g.sC = g.sC2 = set;
-  g.plane_elems = n_pad * n_pad;
-  g.n = static_cast<int>(n); g.n_pad = static_cast<int>(n_pad); g.T = static_cast<int>(n_pad / kPlaneTile);
-  g.errword = word;
-  const int rc = launch_plane_gemm(g, 3, 1, nullptr);
-  if (rc != AK_OK) return rc;
-  hipLaunchKernelGGL(root_out_planes_kernel<3>, dim3(RCHUNKS, 1), dim3(256), 0, nullptr, pc, set, C, n * n, n, n_pad, nullptr, 1, 1.f);
-  hipMemcpy(err, word, 4, hipMemcpyDeviceToHost);
-  return check_launch();
-}
-
-// Tuning builds only: the smallest statistic that iterates on bf16 planes.
-extern "C" void ak_debug_set_root_planes_min(int n) { ak::g_root_planes_min = n; }
-
-// Tuning builds only: 0 = the fp32 MFMA kernel, 3 = the three-piece split kernel for the products of the Newton
-// iteration.
-extern "C" void ak_debug_set_root_split(int pieces) { ak::g_root_split = pieces; }
-#endif

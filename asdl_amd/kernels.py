@@ -1399,7 +1399,9 @@ def kron_precond_grouped(items, grad_scale=1.0):
 
 
 # ------------------------------------------------------------------------------ Shampoo inverse root
-ROOT_POLL_EVERY = 8      # Newton iterations enqueued between two reads of the convergence flags (0: never read them)
+ROOT_POLL_AFTER = (13, 4)   # Newton iterations enqueued before the first read of the convergence flags (an accelerated
+                            # computation at the usual ridge takes 12 or 13), and between the later ones
+ROOT_MAX_GROUPS = 16
 
 
 def inv_root_newton(S, p, ridge_eps, v0, out=None, max_power_iter=100, power_tol=1e-6, max_iter=100, tol=1e-6,
@@ -1407,46 +1409,75 @@ def inv_root_newton(S, p, ridge_eps, v0, out=None, max_power_iter=100, power_tol
     """out[b] <- (S[b] + ridge_eps * lambda_max I)^(-1/p) for S = [batch, n, n] (or [n, n]); S keeps the
     ridge.  v0 = [batch, n] start vectors of the power iteration.  Returns (out, stats) with
     stats = [batch, 4] = (lambda_max, power iterations, newton iterations, final error) on the device.
-    ``poll_every`` (default ROOT_POLL_EVERY): the Newton iterations are enqueued that many at a time and the host reads
+    ``poll_every`` (default ROOT_POLL_AFTER): the Newton iterations are enqueued that many at a time and the host reads
     the convergence flags in between (one small device-to-host copy), so that nothing is launched for a batch that has
     converged; 0 enqueues all ``max_iter`` iterations without ever waiting (the kernels of converged matrices exit at
     once).  The results are the same either way."""
-    _require_gpu(S, v0, out)
     single = S.ndim == 2
     S3 = S.unsqueeze(0) if single else S
-    batch, n = S3.shape[0], S3.shape[1]
-    if S3.dtype != torch.float32 or S3.shape[2] != n or S3.stride(2) != 1 or S3.stride(1) != n:
+    if S3.ndim != 3 or S3.shape[1] != S3.shape[2]:
         raise ValueError('S has to be float32 [batch, n, n] with dense matrices')
-    if n < 2:
-        raise ValueError('n has to be >= 2 (the inverse root of a 1 x 1 statistic is defined as the identity)')
-    v0 = v0.reshape(batch, n).to(torch.float32).contiguous()
-    if out is None:
-        out = torch.empty(batch, n, n, dtype=torch.float32, device=S.device)
-    out3 = out.unsqueeze(0) if out.ndim == 2 else out
-    if out3.dtype != torch.float32 or out3.shape != (batch, n, n) or out3.stride(2) != 1 or out3.stride(1) != n:
-        raise ValueError('out has to be float32 [batch, n, n] with dense matrices')
-    stats = torch.empty(batch, 4, dtype=torch.float32, device=S.device)
+    (out3, stats), = inv_root_group([(S3, p, v0, out.unsqueeze(0) if out is not None and out.ndim == 2 else out)], ridge_eps,
+                                    max_power_iter, power_tol, max_iter, tol, poll_every)
+    return (out3[0] if single and (out is None or out.ndim == 2) else out3), stats
+
+
+def inv_root_group(items, ridge_eps, max_power_iter=100, power_tol=1e-6, max_iter=100, tol=1e-6, poll_every=None):
+    """inv_root_newton for several groups of statistics of one size and power each, in one launch sequence: items are
+    (S [batch, n, n], p, v0 [batch, n], out [batch, n, n] or None); at most ROOT_MAX_GROUPS of them.  Returns a list of
+    (out, stats)."""
+    if not 0 < len(items) <= ROOT_MAX_GROUPS:
+        raise ValueError(f'between 1 and {ROOT_MAX_GROUPS} groups, got {len(items)}')
+    results, keep_v0, rows = [], [], []
+    dev = items[0][0].device
+    total = sum(it[0].shape[0] for it in items)
+    all_stats = torch.empty(total, 4, dtype=torch.float32, device=dev)
+    first = 0
+    for S, p, v0, out in items:
+        _require_gpu(S, v0, out)
+        batch, n = S.shape[0], S.shape[1]
+        if S.dtype != torch.float32 or S.shape[2] != n or S.stride(2) != 1 or S.stride(1) != n:
+            raise ValueError('S has to be float32 [batch, n, n] with dense matrices')
+        if n < 2:
+            raise ValueError('n has to be >= 2 (the inverse root of a 1 x 1 statistic is defined as the identity)')
+        v0 = v0.reshape(batch, n).to(torch.float32).contiguous()
+        if out is None:
+            out = torch.empty(batch, n, n, dtype=torch.float32, device=dev)
+        if out.dtype != torch.float32 or out.shape != (batch, n, n) or out.stride(2) != 1 or out.stride(1) != n:
+            raise ValueError('out has to be float32 [batch, n, n] with dense matrices')
+        stats = all_stats[first:first + batch]
+        first += batch
+        keep_v0.append(v0)
+        results.append((out, stats))
+        rows.append((S.data_ptr(), n, batch, S.stride(0) if batch > 1 else n * n, int(p), v0.data_ptr(), out.data_ptr(),
+                     out.stride(0) if batch > 1 else n * n, stats.data_ptr()))
+    count = len(rows)
+    i64, i32 = ctypes.c_int64 * count, ctypes.c_int * count
+    col = list(zip(*rows))
+    S_a, n_a, b_a, sS, p_a, v_a, o_a, sO, st_a = (i64(*col[0]), i64(*col[1]), i32(*col[2]), i64(*col[3]), i32(*col[4]),
+                                                  i64(*col[5]), i64(*col[6]), i64(*col[7]), i64(*col[8]))
     lib = _lib.load()
-    ws, ws_bytes, keep = _ws_args(_ws_need('ak_inv_root_ws_bytes', n, batch), S.device)
-    strideS = S3.stride(0) if batch > 1 else n * n
-    strideO = out3.stride(0) if batch > 1 else n * n
-    poll = ROOT_POLL_EVERY if poll_every is None else int(poll_every)
-    args = (ctypes.c_void_p(S3.data_ptr()), n, batch, strideS, int(p), float(ridge_eps), ctypes.c_void_p(v0.data_ptr()),
-            int(max_power_iter), float(power_tol), int(max_iter), float(tol), ctypes.c_void_p(out3.data_ptr()), strideO,
-            ctypes.c_void_p(stats.data_ptr()), ws, ws_bytes, _stream())
-    if poll <= 0 or poll >= max_iter:
-        _lib.check(lib.ak_inv_root_newton(*args), 'ak_inv_root_newton')
-    else:
-        off = lib.ak_inv_root_active_offset(n, batch)
-        active = keep[off:off + 4 * batch].view(torch.int32)
-        _lib.check(lib.ak_inv_root_newton_part(1, 0, *args), 'ak_inv_root_newton_part')
-        done = 0
-        while done < max_iter:
-            with _on_launch_stream():
-                if not bool(active.any().item()):      # waits for what has been enqueued so far
-                    break
-            chunk = min(poll, max_iter - done)
-            _lib.check(lib.ak_inv_root_newton_part(2, chunk, *args), 'ak_inv_root_newton_part')
-            done += chunk
-        _lib.check(lib.ak_inv_root_newton_part(4, 0, *args), 'ak_inv_root_newton_part')
-    return (out3[0] if single and out.ndim == 3 else out), stats
+    ws, ws_bytes, keep = _ws_args(lib.ak_inv_root_group_ws_bytes(n_a, b_a, count), dev)
+
+    def run(phases, begin, iters):
+        _lib.check(lib.ak_inv_root_group(phases, begin, iters, count, S_a, n_a, b_a, sS, p_a, float(ridge_eps), v_a,
+                                         int(max_power_iter), float(power_tol), int(max_iter), float(tol), o_a, sO, st_a,
+                                         ws, ws_bytes, _stream(dev)), 'ak_inv_root_group')
+
+    chunks = ROOT_POLL_AFTER if poll_every is None else (int(poll_every),) * 2
+    if chunks[0] <= 0 or chunks[0] >= max_iter:
+        run(7, 0, max_iter)
+        return results
+    off = lib.ak_inv_root_group_active_offset(n_a, b_a, count)
+    active = keep[off:off + 4 * total].view(torch.int32)
+    run(3, 0, chunks[0])
+    done = chunks[0]
+    while done < max_iter:
+        with _on_launch_stream():
+            if not any(active.tolist()):      # waits for what has been enqueued so far
+                break
+        chunk = min(chunks[1], max_iter - done)
+        run(2, done, chunk)
+        done += chunk
+    run(4, 0, 0)
+    return results

@@ -332,9 +332,9 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
             preconditioner.update_statistics(skip_axes=done.get(id(preconditioner), ()))
 
     def update_preconditioner(self):
-        """All inverse roots of one size in one batched call (per matrix:
+        """The inverse roots of all sizes in one batched call (per matrix:
         asdl/precondition/shampoo.py:341-349)."""
-        damping = self.config.damping
+        keys, items = [], []
         for (n, exp), (stats, precs) in self._groups.items():
             if n == 1:
                 continue                 # ComputePower returns the identity for 1 x 1 input
@@ -343,8 +343,12 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
                 v0 = self.start_vector_fn(count, n, stats.device)
             else:
                 v0 = torch.rand(count, n, device=stats.device) * 2 - 1
-            _, st = kernels.inv_root_newton(stats, exp, damping, v0, out=precs)
-            self.last_root_stats[(n, exp)] = st
+            keys.append((n, exp))
+            items.append((stats, exp, v0, precs))
+        for at in range(0, len(items), kernels.ROOT_MAX_GROUPS):
+            part = items[at:at + kernels.ROOT_MAX_GROUPS]
+            for key, (_, st) in zip(keys[at:], kernels.inv_root_group(part, self.config.damping)):
+                self.last_root_stats[key] = st
 
     def precondition(self):
         """P_0^T G P_1 for every matrix-shaped parameter in two grouped launches (all G^T P_0, then all (.)^T P_1:

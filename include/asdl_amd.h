@@ -356,15 +356,17 @@ int ak_kron_precond_static(const float* Binv, const float* Ainv, float* G, int64
  * v0 [batch, n] (the reference draws them from U(-1, 1)), then the coupled Newton iteration.  S_b keeps
  * the ridge on exit, as in the reference.  Convergence tests run on the device: once a matrix's error is
  * below tol, or grows by more than 1.2x (then its previous root is kept), the remaining launches return
- * immediately for it.  stats: device float [batch, 4] = {lambda_max, power iterations, newton iterations,
+ * immediately for it.  A statistic whose spectrum is spread (n ||S||_F^2 > 1.6 tr(S)^2; ridge_eps >= 1e-7, 2 <= p <= 8,
+ * max_iter >= 32) takes steps whose coefficients follow from the lower bound of the spectrum that the ridge gives, about
+ * half as many.  stats: device float [batch, 4] = {lambda_max, power iterations, newton iterations,
  * final error}.  n >= 2 (the reference returns the identity for n == 1 without any arithmetic).
  * Statistics of 512 columns and more iterate on 16-bit planes written by the product that makes each matrix
- * (192-wide tiles, n padded to a multiple of 192 in the workspace): two fp16 planes (22 bits of the power-of-two
+ * (192- or 64-wide tiles, n padded to a multiple of that in the workspace): two fp16 planes (22 bits of the power-of-two
  * scaled value, three matrix instructions per fp32-grade product) where ridge_eps, p and n bound the root's largest
  * eigenvalue, (ridge_eps (1 + p) / (2 sqrt(n)))^(-1/p), below 4096 and p <= 8; else three bf16 planes (the exact split
  * of the fp32 value, six matrix instructions).  ak_inv_root_plane_format tells which: 0 = fp32 matrices (n < 512),
  * 2, 3.  The environment variable ASDL_AMD_ROOT_FP16_PLANES=0 (read once) keeps every statistic on bf16 planes.
- * ak_inv_root_ws_bytes is 60 bytes per padded element and statistic on planes, 36 per element below that size.
+ * ak_inv_root_ws_bytes is 60 bytes per padded element and statistic on planes, 40 per element below that size.
  * Replaces ComputePower / PowerIter / MatPower (asdl/precondition/shampoo.py:465-586). */
 size_t ak_inv_root_ws_bytes(int64_t n, int batch);
 int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps);
@@ -386,6 +388,17 @@ int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batc
                             float ridge_eps, const float* v0, int max_power_iter, float power_tol, int max_iter,
                             float tol, float* out, int64_t strideOut, float* stats, void* ws, size_t ws_bytes,
                             ak_stream_t stream);
+
+/* Several groups of statistics in one launch sequence (group i: batch[i] matrices of size n[i], power p[i]; all arrays on
+ * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 32768).  Same phases; `begin`: how many Newton
+ * iterations the earlier parts have enqueued (-1: not known, one group only).  The `active` words of all matrices, group
+ * after group, start at ws + ak_inv_root_group_active_offset(). */
+size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, int groups);
+size_t ak_inv_root_group_active_offset(const int64_t* n, const int* batch, int groups);
+int ak_inv_root_group(int phases, int begin, int iters, int groups, float* const* S, const int64_t* n, const int* batch,
+                      const int64_t* strideS, const int* p, float ridge_eps, const float* const* v0, int max_power_iter,
+                      float power_tol, int max_iter, float tol, float* const* out, const int64_t* strideOut,
+                      float* const* stats, void* ws, size_t ws_bytes, ak_stream_t stream);
 
 /* ---- stream helpers (no counterpart in the reference) ------------------------------------ */
 

@@ -96,6 +96,33 @@ def test_inv_root_closed_form(n, p, batch):
         assert abs(int(stats[b, 2]) - iters) <= 1, (int(stats[b, 2]), iters)
 
 
+@pytest.mark.parametrize('groups', [
+    ((2, 4, 1), (31, 2, 1), (32, 3, 2), (33, 4, 1), (63, 8, 1), (65, 4, 3), (129, 6, 1)),      # 32-wide fp32 tiles
+    ((255, 4, 40), (256, 4, 25), (511, 2, 3)),                                # 64-wide ones, early steps on split products
+    ((512, 4, 1), (577, 4, 2), (640, 2, 1), (300, 4, 1)),                     # small tiles of planes beside fp32 ones
+    ((513, 4, 45), (20, 4, 2)),                                               # 192-wide tiles of planes
+])
+def test_inv_root_group_of_several_sizes(groups):
+    """Groups of different size and power in one call: each root exactly symmetric and against the fp64
+    closed form."""
+    g = torch.Generator().manual_seed(5)
+    items, before = [], []
+    for n, p, batch in groups:
+        X = torch.randn(batch, 2 * n, n, generator=g) * torch.logspace(0, -1, n)
+        S = (X.transpose(1, 2) @ X / (2 * n)).cuda()
+        items.append((S, p, (torch.rand(batch, n, generator=g) * 2 - 1).cuda(), None))
+        before.append(S.clone())
+    print(f'inv_root groups {groups}', flush=True)
+    results = K.inv_root_group(items, 1e-6)
+    for (n, p, batch), (S, _, _, _), old, (root, stats) in zip(groups, items, before, results):
+        assert (stats[:, 2] > 0).all() and (stats[:, 3] <= 1e-6).all(), (n, p, stats)
+        assert torch.equal(root, root.transpose(1, 2))
+        for b in (0, batch - 1):
+            lam = float(stats[b, 0])
+            assert relerr(S[b], old[b].double() + 1e-6 * lam * torch.eye(n, device='cuda')) < 1e-6
+            assert relerr(root[b], _closed_form_root(S[b], p)) < 1e-3, (n, p, b)
+
+
 def test_inv_root_polled_and_unpolled_enqueue_give_the_same_result():
     """The host may stop enqueuing Newton iterations once the convergence flags are all zero (read every few
     iterations) or enqueue all of them blindly: bit-equal roots and the same iteration counts."""
