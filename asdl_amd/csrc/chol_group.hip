@@ -5,6 +5,7 @@
 //   for every diagonal block k:  leaf: W_kk -> M_kk = L_kk^-1 (one work group, in registers: chol_leaf.hpp);
 //                                panel: L21 = A21 M_kk^T;  update: A22 -= L21 L21^T
 //   for every level of a balanced tree over the blocks:  T2 = L21 M11;  M21 = -M22 T2
+// (Groups whose matrices are few and small enough take the block sweep of chol_sweep.hpp instead: one launch per block.)
 // d^3 FLOP in total, like POTRF + POTRI.  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
 // as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: 1.4-1.7
 // times the error of LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half was at 3-8).
@@ -28,11 +29,12 @@
 #include <vector>
 #include "gemm_f32.hpp"
 #include "chol_leaf.hpp"
+#include "chol_sweep.hpp"
 
 namespace ak {
 
-constexpr int64_t CG_MAGIC = 0x3247524c4f4843ll;     // "CHOLGR2"
-constexpr int CG_COPY = 0, CG_LEAF = 1, CG_PROD = 2, CG_PROD_DEEP = 3;
+constexpr int64_t CG_MAGIC = 0x3347524c4f4843ll;     // "CHOLGR3"
+constexpr int CG_COPY = 0, CG_LEAF = 1, CG_PROD = 2, CG_PROD_DEEP = 3, CG_SWEEP = 4;
 constexpr int CG_FLAG_TRANSA = 1, CG_FLAG_TRANSB = 2, CG_FLAG_OUT_USER = 4, CG_FLAG_PANEL = 8;
 // What an operand of a product holds, for the fp16-piece products (bits 4-5 of CgProd::flags: A, bits 6-7: B).  With
 // a = the largest diagonal element of A + lam I, every element is bounded in magnitude: a block of the (updated)
@@ -325,22 +327,23 @@ static void cg_make_deep(CgProd& p) {
   p.tiles_n = (p.N + bn - 1) / bn;
 }
 
+// Microseconds of the products of one super-step (cg_prefer_deep), its launch not counted.
+static double cg_product_us(const std::vector<CgProd>& ps, bool deep) {
+  double longest = 0, sum = 0;
+  for (const CgProd& p : ps) {
+    CgProd q = p;
+    if (deep) cg_make_deep(q);
+    const double c = deep ? (p.K + 127) / 128 : (p.K + 31) / 32;
+    longest = std::max(longest, c);
+    sum += c * static_cast<double>(cg_tiles(q));
+  }
+  return deep ? 2.0 * std::max(longest, sum / 256) : std::max(1.6 * longest, 1.05 * sum / 256);
+}
+
 // Which kernel a super-step's products take.  The split kernel's 128 x 128 tiles have three times the rate once they
 // fill the device (about 1 us per k-tile of 32 and CU), but a tile takes 1.6 us per k-tile however few there are; the
 // deep tiles take 2 us per chunk of 128 k.  The step is as long as its longest tile or as its work spread over the CUs.
-static bool cg_prefer_deep(const std::vector<CgProd>& ps) {
-  double chunk_max = 0, chunks = 0, ktile_max = 0, ktiles = 0;
-  for (const CgProd& p : ps) {
-    CgProd q = p;
-    cg_make_deep(q);
-    const double c = (p.K + 127) / 128, k = (p.K + 31) / 32;
-    chunk_max = std::max(chunk_max, c);
-    ktile_max = std::max(ktile_max, k);
-    chunks += c * static_cast<double>(cg_tiles(q));
-    ktiles += k * static_cast<double>(cg_tiles(p));
-  }
-  return 2.0 * std::max(chunk_max, chunks / 256) < std::max(1.6 * ktile_max, 1.05 * ktiles / 256);
-}
+static bool cg_prefer_deep(const std::vector<CgProd>& ps) { return cg_product_us(ps, true) < cg_product_us(ps, false); }
 
 static CgProd cg_prod(int mat, int flags, int kind_a, int kind_b, int M, int N, int K, float alpha, int64_t a, int lda,
                       int64_t b, int ldb, float beta, int64_t c, int ldc, int kmode, int tile_mode) {
@@ -441,6 +444,7 @@ struct CgPlan {
   std::vector<CgLeafTask> leaves;
   std::vector<CgProd> prods;
   std::vector<int32_t> tile_map;
+  std::vector<SwTask> sweep_leaves, sweep_tiles;
 };
 
 static inline int64_t cg_align(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
@@ -452,7 +456,105 @@ static bool cg_dims_ok(const int64_t* dims, int count) {
   return true;
 }
 
+// The sweep: per step the leaf's work group, or as many waves of tiles as the device needs (one work group per CU).
+static double cg_sweep_us(const int64_t* dims, int count) {
+  int64_t nb_max = 0;
+  for (int m = 0; m < count; ++m) nb_max = std::max<int64_t>(nb_max, (dims[m] + LEAF - 1) / LEAF);
+  double us = 16;
+  for (int64_t k = 0; k < nb_max; ++k) {
+    int64_t groups = 0;
+    for (int m = 0; m < count; ++m) {
+      const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
+      if (nb > k) groups += nb * (nb + 1) / 2 + (nb > k + 1 ? 1 : 0);
+    }
+    us += std::max(25.0, 22.0 * static_cast<double>((groups + 255) / 256));
+  }
+  return us;
+}
+
+// The tables of the sweep: matrices in the order of their number of block columns, so that those still at work in step k
+// are the first ones of both lists.
+static void cg_build_sweep(const int64_t* dims, int count, CgPlan& plan) {
+  std::vector<int> order(count);
+  for (int m = 0; m < count; ++m) order[m] = m;
+  auto blocks = [&](int m) { return static_cast<int>((dims[m] + LEAF - 1) / LEAF); };
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blocks(x) > blocks(y); });
+  int64_t off = 0;
+  for (int m : order) {
+    const int nb = blocks(m);
+    SwTask t;
+    std::memset(&t, 0, sizeof(t));
+    t.mat = m; t.d = static_cast<int>(dims[m]); t.nb = nb;
+    t.x_off = off;
+    t.y_off = off + static_cast<int64_t>(nb) * (nb + 1) / 2 * SW_TILE;
+    t.m_off = t.y_off + static_cast<int64_t>(2) * nb * SW_TILE;
+    off = t.m_off + 2 * SW_TILE;
+    plan.sweep_leaves.push_back(t);
+    const int64_t x0 = t.x_off;
+    for (t.bi = 0; t.bi < nb; ++t.bi)
+      for (t.bj = 0; t.bj <= t.bi; ++t.bj) {
+        t.x_off = x0 + (static_cast<int64_t>(t.bi) * (t.bi + 1) / 2 + t.bj) * SW_TILE;
+        plan.sweep_tiles.push_back(t);
+      }
+  }
+  const int nb_max = blocks(order[0]);
+  for (int k = -1; k < nb_max; ++k) {
+    int leaves = 0, tiles = 0;
+    for (int m : order) {
+      if (blocks(m) > k + 1) ++leaves;
+      if (k >= 0 && blocks(m) > k) tiles += blocks(m) * (blocks(m) + 1) / 2;
+    }
+    plan.steps.push_back(CgStep{CG_SWEEP, k, leaves, leaves + tiles, 0, 0});
+  }
+  CgHeader& h = plan.h;
+  std::memset(&h, 0, sizeof(h));
+  h.magic = CG_MAGIC;
+  h.ws_floats = off;
+  h.count = count;
+  h.nsteps = static_cast<int>(plan.steps.size());
+  int64_t b = cg_align(sizeof(CgHeader), 64);
+  h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
+  h.leaves_off = b; b = cg_align(b + plan.sweep_leaves.size() * sizeof(SwTask), 64);
+  h.prods_off = b; b = cg_align(b + plan.sweep_tiles.size() * sizeof(SwTask), 64);
+  h.mats_off = h.map_off = b;
+  h.total_bytes = b;
+}
+
+static void cg_build_right_looking(const int64_t* dims, int count, CgPlan& plan);
+#ifdef AK_TUNING_HOOKS
+static int CG_FORCE = 0;               // tuning builds: 1 the sweep, 2 the factorization (ak_debug_force_chol_plan)
+#else
+constexpr int CG_FORCE = 0;
+#endif
+
+// The sweep wins while its tiles fit the device once (25 us a step against 41 for leaf, panel and update), and often when
+// they fit it twice (44 us a step: 2 x 2048, 272 tiles, 757 against 908 us); beyond that its K = 128 updates of the whole
+// triangle cost more than the factorization's shorter, deeper and split ones (4 x 2048: 1139 against 980 us).  The bound of
+// 4096 tiles only keeps the tables of hopeless cases from being built.
 static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
+  int64_t tiles = 0;
+  for (int m = 0; m < count; ++m) {
+    const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
+    tiles += nb * (nb + 1) / 2;
+  }
+  if (CG_FORCE == 1) { cg_build_sweep(dims, count, plan); return; }
+  CgPlan right;
+  cg_build_right_looking(dims, count, right);
+  double us = 0;
+  for (const CgStep& st : right.steps) {
+    us += 4;              // the launch's own start and the wait for the one before
+    if (st.type == CG_LEAF) us += 15;
+    else if (st.type == CG_COPY) us += 8;
+    else {
+      const std::vector<CgProd> ps(right.prods.begin() + st.first, right.prods.begin() + st.first + st.count);
+      us += cg_product_us(ps, st.type == CG_PROD_DEEP);
+    }
+  }
+  if (CG_FORCE != 2 && tiles <= 4096 && cg_sweep_us(dims, count) < us) cg_build_sweep(dims, count, plan);
+  else plan = std::move(right);
+}
+
+static void cg_build_right_looking(const int64_t* dims, int count, CgPlan& plan) {
   std::vector<std::vector<CgOp>> seq(count);
   int64_t off = 0;
   int copy_blocks = 0;
@@ -552,13 +654,9 @@ extern "C" size_t ak_chol_group_plan_bytes(const int64_t* dims, int count) {
 
 extern "C" size_t ak_chol_group_ws_bytes(const int64_t* dims, int count) {
   if (!ak::cg_dims_ok(dims, count)) return 0;
-  int64_t off = 0;
-  for (int m = 0; m < count; ++m) {
-    const int64_t dp = (dims[m] + 3) / 4 * 4;
-    off += ak::cg_align(dp * dp, 64) + 2 * ak::cg_align(ak::cg_pool(dp), 64);
-  }
-  off += ak::cg_align(static_cast<int64_t>(count) * ak::CG_SCALE_FLOATS, 64);
-  return static_cast<size_t>(off) * sizeof(float);
+  ak::CgPlan plan;
+  ak::cg_build(dims, count, plan);
+  return static_cast<size_t>(plan.h.ws_floats) * sizeof(float);
 }
 
 extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_host, size_t plan_bytes) {
@@ -570,10 +668,14 @@ extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_hos
   unsigned char* out = static_cast<unsigned char*>(plan_host);
   std::memset(out, 0, static_cast<size_t>(plan.h.total_bytes));
   std::memcpy(out, &plan.h, sizeof(CgHeader));
-  std::memcpy(out + plan.h.mats_off, plan.mats.data(), plan.mats.size() * sizeof(CgMat));
+  if (!plan.mats.empty()) std::memcpy(out + plan.h.mats_off, plan.mats.data(), plan.mats.size() * sizeof(CgMat));
   std::memcpy(out + plan.h.steps_off, plan.steps.data(), plan.steps.size() * sizeof(CgStep));
   if (!plan.leaves.empty()) std::memcpy(out + plan.h.leaves_off, plan.leaves.data(), plan.leaves.size() * sizeof(CgLeafTask));
   if (!plan.prods.empty()) std::memcpy(out + plan.h.prods_off, plan.prods.data(), plan.prods.size() * sizeof(CgProd));
+  if (!plan.sweep_leaves.empty()) {
+    std::memcpy(out + plan.h.leaves_off, plan.sweep_leaves.data(), plan.sweep_leaves.size() * sizeof(SwTask));
+    std::memcpy(out + plan.h.prods_off, plan.sweep_tiles.data(), plan.sweep_tiles.size() * sizeof(SwTask));
+  }
   if (!plan.tile_map.empty())
     std::memcpy(out + plan.h.map_off, plan.tile_map.data(), plan.tile_map.size() * sizeof(int32_t));
   return AK_OK;
@@ -610,7 +712,12 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
   for (int i = 0; i < h->nsteps; ++i) {
     const CgStep& st = steps[i];
     if (st.grid <= 0) continue;
-    if (st.type == CG_COPY) {
+    if (st.type == CG_SWEEP) {
+      const SwArgs w{a.ws, A_list, out_list, lam, skip_flags, info, lam_stride, skip_stride};
+      hipLaunchKernelGGL(cg_sweep_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, w,
+                         reinterpret_cast<const SwTask*>(a.plan + h->leaves_off),
+                         reinterpret_cast<const SwTask*>(a.plan + h->prods_off), st.count, st.first);
+    } else if (st.type == CG_COPY) {
       hipLaunchKernelGGL(cg_copy_in_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
       hipLaunchKernelGGL(cg_scale_kernel, dim3(h->count), dim3(256), 0, s, a, h->count, CG_HALF_MAX_COND);
     } else if (st.type == CG_LEAF)
@@ -627,4 +734,6 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
 #ifdef AK_TUNING_HOOKS
 // Tuning builds only: the bound a / lam up to which a matrix takes the fp16-piece products (0: never).
 extern "C" void ak_debug_set_chol_half_max_cond(float v) { ak::CG_HALF_MAX_COND = v; }
+// Tuning builds only: 1 the sweep, 2 the right-looking factorization, 0 the rule.
+extern "C" void ak_debug_force_chol_plan(int v) { ak::CG_FORCE = v; }
 #endif

@@ -12,9 +12,11 @@
 // it is (v_mfma_f32_16x16x4_f32: register r of lane 16 g + c is row 4 g + r, column c; step r of a product contracts the
 // rows {4 g + r}), which is why U and not L is kept.
 //
-// What bounds it: the chain of 8 x (factor -> barrier -> panel -> barrier -> update of the next diagonal tile), about 4 k
-// cycles per link; the wave that owns diagonal tile k + 1 updates it first and factors it while the others still
-// update.  The fp32 matrix instructions of all 224 tile products fill 7 k cycles of the four SIMDs beside it.
+// What bounds it: the chain factor k -> U_k,k+1 -> update of diagonal tile k + 1 -> factor k + 1.  Wave 0 runs nothing
+// but this chain, at the highest priority; eight waves on the other three SIMDs hold one column of tiles each, form
+// row k and update the rows below beside the next factor, and publish the two tiles that the chain needs next.  The right
+// operand of every product of a column is that column's own tile of row k, in registers.  1.4 us per row of tiles, the
+// factor 0.9 of it; with all waves in step (panel and update of all tiles between two factors) it was 2.2 us.
 #pragma once
 #include "common.hpp"
 
@@ -23,13 +25,14 @@ namespace ak {
 constexpr int LEAF = 128;
 constexpr int LT = 16;                       // tile
 constexpr int LEAF_THREADS = 1024;
-constexpr int LEAF_SLOTS = 5;                // tiles a wave holds at most
+constexpr int LEAF_TILES = LEAF / LT;
 constexpr int LEAF_ROW_LD = LEAF + 4;        // 4 rows apart: 16 banks apart, so the rows 4 g + r of one step do not collide
 constexpr int LEAF_INV_LD = LT + 4;
 
 struct LeafShared {
   float row[LT * LEAF_ROW_LD];
   float inv[LT * LEAF_INV_LD];
+  floatx4 first[64], super[64], diag[64];      // published tiles: (0, 0), (k, k + 1), (k + 1, k + 1)
   int bad;
 };
 
@@ -56,7 +59,7 @@ __device__ __forceinline__ float spread_row_group(const floatx4& v) {
 
 // Pivots 4 Q ... 4 Q + 3 of leaf_tile_inverse.
 template <int Q>
-__device__ __forceinline__ void leaf_tile_step(floatx4& a, floatx4& inv, floatx4& piv, int& bad, int g, int c) {
+__device__ __forceinline__ void leaf_tile_step(floatx4& a, floatx4& inv, floatx4& piv, int g, int c) {
   // the 4 x 4 block on the diagonal, in every lane: column i of its lower triangle sits in lane (Q, 4 Q + i)
   float d[4][4];
 #pragma unroll
@@ -66,15 +69,15 @@ __device__ __forceinline__ void leaf_tile_step(floatx4& a, floatx4& inv, floatx4
   float l[4][4], rec[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    if (!(d[k][k] > 0.f)) {                  // also catches NaN
-      if (bad == 0) bad = 4 * Q + k + 1;
-      d[k][k] = 1.f;
-    }
-    float r = __builtin_amdgcn_rcpf(d[k][k]);             // hardware reciprocal, then one Newton step
-    r = __builtin_fmaf(__builtin_fmaf(-d[k][k], r, 1.f), r, r);
-    rec[k] = r;
+    const float p = fmaxf(d[k][k], 1e-36f);               // a pivot that is not positive (or NaN) is reported by the caller
+    const float r = __builtin_amdgcn_rcpf(p);             // hardware reciprocal; its error e corrects the quotients
+    const float e = __builtin_fmaf(-p, r, 1.f);
+    rec[k] = __builtin_fmaf(e, r, r);
 #pragma unroll
-    for (int i = k + 1; i < 4; ++i) l[i][k] = d[i][k] * r;
+    for (int i = k + 1; i < 4; ++i) {
+      const float q = d[i][k] * r;
+      l[i][k] = __builtin_fmaf(q, e, q);
+    }
 #pragma unroll
     for (int i = k + 1; i < 4; ++i)
 #pragma unroll
@@ -105,133 +108,181 @@ __device__ __forceinline__ void leaf_tile_step(floatx4& a, floatx4& inv, floatx4
 }
 
 // a: a symmetric 16 x 16 tile in the accumulator layout (only elements with column >= row are looked at), replaced by
-// L^-1 of its Cholesky factor (zeros above the diagonal).  Returns 0 or the 1-based index of the first non-positive
-// pivot.  L D L^T by blocks of 4 pivots: the 4 x 4 blocks are factored and inverted by every lane for itself (ten
-// lane reads and a chain of four reciprocals; no square root before the end), and the rank-4 updates of the tile and of
-// its inverse are one matrix instruction each.
-__device__ __forceinline__ int leaf_tile_inverse(floatx4& a, int lane) {
+// L^-1 of its Cholesky factor (zeros above the diagonal).  L D L^T by blocks of 4 pivots: the 4 x 4 blocks are factored and
+// inverted by every lane for itself (ten lane reads and a chain of four reciprocals; no square root before the end), and
+// the rank-4 updates of the tile and of its inverse are one matrix instruction each.  piv: the pivots, register r of the
+// lanes of row group g holds pivot 4 g + r.
+template <class AfterFirst>
+__device__ __forceinline__ void leaf_tile_inverse(floatx4& a, floatx4& piv, int lane, AfterFirst&& after_first_step) {
   const int g = lane >> 4, c = lane & 15;
-  int bad = 0;
-  floatx4 inv, piv = {1.f, 1.f, 1.f, 1.f};
+  floatx4 inv;
+  piv = floatx4{1.f, 1.f, 1.f, 1.f};
 #pragma unroll
   for (int r = 0; r < 4; ++r) inv[r] = 4 * g + r == c ? 1.f : 0.f;
-  leaf_tile_step<0>(a, inv, piv, bad, g, c);
-  leaf_tile_step<1>(a, inv, piv, bad, g, c);
-  leaf_tile_step<2>(a, inv, piv, bad, g, c);
-  leaf_tile_step<3>(a, inv, piv, bad, g, c);
+  leaf_tile_step<0>(a, inv, piv, g, c);
+  after_first_step();
+  leaf_tile_step<1>(a, inv, piv, g, c);
+  leaf_tile_step<2>(a, inv, piv, g, c);
+  leaf_tile_step<3>(a, inv, piv, g, c);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    float s = __builtin_amdgcn_rsqf(piv[r]);
-    s = __builtin_fmaf(0.5f * s, __builtin_fmaf(-piv[r] * s, s, 1.f), s);      // one Newton step
+    const float p = fmaxf(piv[r], 1e-36f);
+    float s = __builtin_amdgcn_rsqf(p);
+    s = __builtin_fmaf(0.5f * s, __builtin_fmaf(-p * s, s, 1.f), s);      // one Newton step
     a[r] = inv[r] * s;
   }
-  return bad;
 }
 
-// Tile of slot s of a wave: waves 0 ... 7 hold the diagonal tile of their own row in slot 0 and two tiles of the row above
-// (finished when they factor), waves 8 ... 15 five tiles each, spread over the rows.  row = 8: none.
-__device__ __forceinline__ void leaf_slot(int wave, int s, int& row, int& col) {
-  int t;
-  if (wave < 8) {
-    if (s == 0) { row = col = wave; return; }
-    row = s < 3 ? (wave + 7) & 7 : 8;
-    t = s - 1;
+// 0 or the 1-based index of the first pivot of leaf_tile_inverse that is not positive.
+__device__ __forceinline__ int leaf_first_bad(const floatx4& piv) {
+  const bool ok = piv[0] > 0.f && piv[1] > 0.f && piv[2] > 0.f && piv[3] > 0.f;
+  const uint64_t bad = __ballot(!ok);
+  if (bad == 0) return 0;
+  const int at = __builtin_ctzll(bad);                 // a lane of the first row group with a bad pivot
+  const int r = !(piv[0] > 0.f) ? 1 : !(piv[1] > 0.f) ? 2 : !(piv[2] > 0.f) ? 3 : 4;
+  return 4 * (at >> 4) + __builtin_amdgcn_readlane(r, at);
+}
+
+// The column of tiles a wave holds (8: none).  None of the waves shares a SIMD with wave 0, beside whose priority it would
+// be the last one at every barrier; the columns are dealt so that the three SIMDs have about the same number of updates.
+__device__ __forceinline__ int leaf_column(int wave) {
+  constexpr uint64_t kColumn = 0x8888821854380678ull;       // wave 0 in the lowest hex digit
+  return static_cast<int>((kColumn >> (4 * wave)) & 15);
+}
+
+// The elimination itself.  load(i, j): tile (i, j), i <= j, of U's side of the block in the accumulator layout; store(i, j,
+// tile): takes tile (i, j) of L^-1, i >= j (both called by the wave that holds column j, with constant i, all loads before the
+// first barrier and all stores after the last product).  nb: rows of tiles of the block.  Returns the 1-based index of the
+// first non-positive pivot inside the block, or 0, to every thread.  All branches meet the same barriers in the same
+// order: one before the loop, B_k after the factor of row k, C_k (k + 1 < nb) once row k is complete, one at the end.
+template <class Load, class Store>
+__device__ __forceinline__ int leaf_eliminate(int nb, LeafShared& sh, int wave, int lane, Load&& load, Store&& store) {
+  const int j = leaf_column(wave);
+  const int g = lane >> 4, c = lane & 15;
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    __syncthreads();
+    floatx4 a = sh.first[lane], piv;
+    int first_bad = 0;
+#pragma unroll 1
+    for (int k = 0; k < nb; ++k) {
+      leaf_tile_inverse(a, piv, lane, [k]() {
+        if (k > 0) __syncthreads();                            // C_(k - 1): here the chain has not got to wait for it
+      });
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.inv[(4 * g + r) * LEAF_INV_LD + c] = a[r];
+      __syncthreads();                                         // B_k
+      if (k + 1 < nb) {
+        const floatx4 m = *reinterpret_cast<const floatx4*>(sh.inv + c * LEAF_INV_LD + 4 * g);
+        const floatx4 t = sh.super[lane], d = sh.diag[lane];
+        // two chains of two products each time: half the latency of one of four
+        const floatx4 u = mfma16(m[1], t[1], mfma16(m[0], t[0], zero)) + mfma16(m[3], t[3], mfma16(m[2], t[2], zero));
+        a = mfma16(-u[1], u[1], mfma16(-u[0], u[0], d)) + mfma16(-u[3], u[3], mfma16(-u[2], u[2], zero));
+      }
+      const int bad = leaf_first_bad(piv);
+      if (bad != 0 && first_bad == 0) first_bad = LT * k + bad;
+    }
+    if (lane == 0) sh.bad = first_bad;
+    __builtin_amdgcn_s_setprio(0);
+  } else if (j < nb) {
+    floatx4 acc[LEAF_TILES];
+#pragma unroll
+    for (int i = 0; i < LEAF_TILES; ++i) {
+      acc[i] = zero;
+      if (i <= j) acc[i] = load(i, j);
+    }
+    if (j == 0) sh.first[lane] = acc[0];
+    if (j == 1) {
+      sh.super[lane] = acc[0];
+      sh.diag[lane] = acc[1];
+    }
+    __syncthreads();
+    float* row = sh.row + 4 * g * LEAF_ROW_LD + c;
+#pragma unroll
+    for (int k = 0; k < LEAF_TILES; ++k) {
+      if (k >= nb) break;
+      __syncthreads();                                         // B_k
+      if (j != k) {
+        const floatx4 m = *reinterpret_cast<const floatx4*>(sh.inv + c * LEAF_INV_LD + 4 * g), t = acc[k];
+        acc[k] = mfma16(m[1], t[1], mfma16(m[0], t[0], zero)) + mfma16(m[3], t[3], mfma16(m[2], t[2], zero));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[k][r] = sh.inv[(4 * g + r) * LEAF_INV_LD + c];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) row[r * LEAF_ROW_LD + LT * j] = acc[k][r];
+      if (k + 1 == nb) break;
+      __syncthreads();                                         // C_k
+#pragma unroll
+      for (int i = k + 1; i < LEAF_TILES; ++i) {
+        if (j >= i || j <= k) {
+          float u[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) u[r] = -row[r * LEAF_ROW_LD + LT * i];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i] = mfma16(u[r], acc[k][r], acc[i]);
+          if (i == k + 2 && j == k + 2) {
+            sh.super[lane] = acc[k + 1];
+            sh.diag[lane] = acc[k + 2];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < LEAF_TILES; ++i)
+      if (i >= j && i < nb) store(i, j, acc[i]);
   } else {
-    const int u = 8 * s + wave - 8;
-    row = u / 5;
-    t = 2 + u % 5;
+    __syncthreads();
+#pragma unroll 1
+    for (int k = 0; k < nb; ++k) {
+      __syncthreads();                                         // B_k
+      if (k + 1 < nb) __syncthreads();                         // C_k
+    }
   }
-  col = t < row ? t : t + 1;
+  __syncthreads();
+  return sh.bad;
 }
 
 // The n x n block at `blk` (row stride ld, lower triangle) is replaced by the inverse of its Cholesky factor (zeros
 // above the diagonal).  Returns the 1-based index of the first non-positive pivot inside the block, or 0, to every
-// thread.  All 1024 threads of the work group call it.  (26 us for n = 128 as a recursion on an LDS-resident block that
-// handled 16 x 16 blocks one row per lane; 16.7 us in this form, launch included.)
+// thread.  All 1024 threads of the work group call it.
 __device__ __forceinline__ int leaf_block(float* __restrict__ blk, int64_t ld, int n, LeafShared& sh, int tid) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int nb = (n + LT - 1) / LT;
   const bool vec = (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(blk) & 15) == 0 && (n & 3) == 0;
-  int row[LEAF_SLOTS], col[LEAF_SLOTS];
-  floatx4 acc[LEAF_SLOTS];
+  return leaf_eliminate(
+      nb, sh, wave, lane,
+      [&](int s, int col) {
+        // element (16 s + 4 g + r, 16 col + c) of U's side is element (16 col + c, 16 s + 4 g + r) of the lower triangle
+        const int i = LT * col + c, j = LT * s + 4 * g;
+        const float* src = blk + static_cast<int64_t>(i) * ld + j;
+        floatx4 v = {0.f, 0.f, 0.f, 0.f};
+        if (vec) {
+          if (i < n && j < n && j <= i) v = *reinterpret_cast<const floatx4*>(src);
+        } else {
 #pragma unroll
-  for (int s = 0; s < LEAF_SLOTS; ++s) {
-    leaf_slot(wave, s, row[s], col[s]);
-    if (row[s] >= nb || col[s] >= nb) row[s] = 8;
-    acc[s] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (row[s] < 8 && col[s] >= row[s]) {
-      // element (16 row + 4 g + r, 16 col + c) of U's side is element (16 col + c, 16 row + 4 g + r) of the lower triangle
-      const int i = LT * col[s] + c, j = LT * row[s] + 4 * g;
-      const float* src = blk + static_cast<int64_t>(i) * ld + j;
-      if (vec) {
-        if (i < n && j < n && j <= i) acc[s] = *reinterpret_cast<const floatx4*>(src);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (i < n && j + r <= i) acc[s][r] = src[r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (i >= n) acc[s][r] = i == j + r ? 1.f : 0.f;      // identity padding
-        if (j + r > i) acc[s][r] = 0.f;
-      }
-    }
-  }
-  if (tid == 0) sh.bad = 0;
-#pragma unroll 1
-  for (int k = 0; k < nb; ++k) {
-    if (wave == k) {
-      __builtin_amdgcn_s_setprio(3);
-      const int bad = leaf_tile_inverse(acc[0], lane);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sh.inv[(4 * g + r) * LEAF_INV_LD + c] = acc[0][r];
-      if (bad != 0 && lane == 0 && sh.bad == 0) sh.bad = LT * k + bad;
-      __builtin_amdgcn_s_setprio(0);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < LEAF_SLOTS; ++s) {
-      if (row[s] != k) continue;
-      if (col[s] != k) {
-        const floatx4 m = *reinterpret_cast<const floatx4*>(sh.inv + c * LEAF_INV_LD + 4 * g);
-        floatx4 p = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) p = mfma16(m[r], acc[s][r], p);
-        acc[s] = p;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sh.row[(4 * g + r) * LEAF_ROW_LD + LT * col[s] + c] = acc[s][r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < LEAF_SLOTS; ++s) {
-      if (row[s] > k && row[s] < 8 && (col[s] >= row[s] || col[s] <= k)) {
-        const float* pa = sh.row + 4 * g * LEAF_ROW_LD + LT * row[s] + c;
-        const float* pb = sh.row + 4 * g * LEAF_ROW_LD + LT * col[s] + c;
-        float av[4], bv[4];
+          for (int r = 0; r < 4; ++r)
+            if (i < n && j + r <= i) v[r] = src[r];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          av[r] = -pa[r * LEAF_ROW_LD];
-          bv[r] = pb[r * LEAF_ROW_LD];
+          if (i >= n) v[r] = i == j + r ? 1.f : 0.f;      // identity padding
+          if (j + r > i) v[r] = 0.f;
         }
-        __builtin_amdgcn_sched_barrier(0);       // all eight reads before the first product: one wait, not one per step
+        return v;
+      },
+      [&](int s, int col, const floatx4& v) {
+        const int j = LT * col + c;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[s] = mfma16(av[r], bv[r], acc[s]);
-      }
-    }
-  }
-  // every element of the block was read before the first barrier released the last row of tiles that needed it
-#pragma unroll
-  for (int s = 0; s < LEAF_SLOTS; ++s) {
-    if (row[s] >= 8) continue;
-    const int j = LT * col[s] + c;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = LT * row[s] + 4 * g + r;
-      if (i < n && j < n) blk[static_cast<int64_t>(i) * ld + j] = col[s] > row[s] ? 0.f : acc[s][r];
-    }
-  }
-  return sh.bad;
+        for (int r = 0; r < 4; ++r) {
+          const int i = LT * s + 4 * g + r;
+          if (i < n && j < n) {
+            blk[static_cast<int64_t>(i) * ld + j] = v[r];
+            if (s != col) blk[static_cast<int64_t>(j) * ld + i] = 0.f;
+          }
+        }
+      });
 }
 
 }  // namespace ak

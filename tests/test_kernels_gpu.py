@@ -626,6 +626,22 @@ def test_chol_inv_at_the_edges_of_the_leaf_tiles(K, d):
             assert int(call([B.cuda()], [out], lam_dev).cpu()) == bad, (call.__name__, bad)
 
 
+@pytest.mark.parametrize('dims', [(127, 255, 2), (129, 257, 1), (383, 384, 385), (1151, 513, 640, 10), (2049, 127), (2700, 2700)])
+def test_chol_inv_grouped_block_sweep_edges(K, dims):
+    """Groups of matrices that end just before, at and behind a block of 128 columns and leave the sweep at different
+    steps; the last two need more tiles than the device has CUs.  Against fp64, full-rank and rank-deficient."""
+    for rank in (2, 1 / 8):
+        mats = [_spd(d, 900 + i, rows=max(1, int(rank * d))) for i, d in enumerate(dims)]
+        lam = [0.05 * float(m.diagonal().max()) for m in mats]
+        outs = [torch.empty(d, d, device='cuda') for d in dims]
+        info = K.chol_inv_grouped([m.cuda() for m in mats], outs, torch.tensor(lam, device='cuda'))
+        assert torch.all(info == 0)
+        for m, l, out in zip(mats, lam, outs):
+            W = m.cuda().double() + l * torch.eye(m.shape[0], device='cuda', dtype=torch.float64)
+            assert relerr(out, torch.linalg.inv(W)) < 2e-5, (m.shape, relerr(out, torch.linalg.inv(W)))
+            assert torch.equal(out, out.T)
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
