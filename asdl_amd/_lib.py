@@ -47,6 +47,7 @@ _SIGNATURES = {
     'ak_unit_wise_inv': (c_int, [c_ptr, c_i64, c_f32, c_ptr, c_ptr, c_ptr]),
     'ak_unit_wise_mvp': (c_int, [c_ptr, c_i64, c_ptr, c_ptr, c_f32, c_ptr]),
     'ak_unit_wise_mvp_grouped': (c_int, [c_ptr, c_int, c_i64, c_f32, c_ptr]),
+    'ak_unit_wise_keep_grouped': (c_int, [c_ptr, c_int, c_i64, c_ptr]),
     'ak_unit_wise_inv_grouped': (c_int, [c_ptr, c_int, c_i64, c_ptr]),
     'ak_identity_where_zero': (c_int, [c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_ptr]),
     'ak_conv_patch_sum': (c_int, [c_ptr, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_int, c_int,
@@ -58,6 +59,7 @@ _SIGNATURES = {
     'ak_event_create': (c_int, [ctypes.POINTER(ctypes.c_void_p), c_int]),
     'ak_event_destroy': (c_int, [c_ptr]),
     'ak_event_record': (c_int, [c_ptr, c_ptr]),
+    'ak_sample_categorical': (c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr]),
     'ak_stream_order': (c_int, [c_ptr, c_ptr, c_ptr]),
     'ak_event_elapsed_ms': (c_int, [c_ptr, c_ptr, ctypes.POINTER(ctypes.c_float)]),
     'ak_copy_bytes': (c_int, [c_ptr, c_ptr, c_i64, c_ptr]),

@@ -1,0 +1,71 @@
+// One draw per row of a categorical distribution given by logits: the largest of p_i / q_i, q_i exponential random numbers,
+// taken as the largest of logits_i - log q_i (the normalisation of p shifts every term of a row alike).
+// Bound by the device memory: logits and random numbers are read once (8192 x 4096: 268 MB) where softmax, normalisation,
+// their checks, the quotient and the argmax made a dozen passes and launches.
+#include "common.hpp"
+
+namespace ak {
+
+struct Best {
+  float v;
+  int i;
+};
+
+__device__ __forceinline__ void best_of(Best& a, float v, int i) {
+  if (v > a.v || (v == a.v && i < a.i)) { a.v = v; a.i = i; }
+}
+
+// One wave per row (few classes) or one work group of four waves per row.
+template <int WAVES>
+static __global__ __launch_bounds__(256) void sample_categorical_kernel(const float* __restrict__ logits,
+                                                                        const float* __restrict__ q, int64_t rows,
+                                                                        int classes, int64_t* __restrict__ targets) {
+  __shared__ Best part[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row = WAVES == 1 ? static_cast<int64_t>(blockIdx.x) * 4 + wave : blockIdx.x;
+  if (row >= rows) return;
+  const float* __restrict__ x = logits + row * classes;
+  const float* __restrict__ e = q + row * classes;
+  const int t = WAVES == 1 ? lane : threadIdx.x;
+  constexpr int N = 64 * WAVES;
+  Best b{-INFINITY, 0x7fffffff};
+  const bool vec = classes % 4 == 0 && ((reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(q)) & 15) == 0;
+  if (vec) {
+#pragma unroll 4
+    for (int c = 4 * t; c < classes; c += 4 * N) {
+      const floatx4 xv = *reinterpret_cast<const floatx4*>(x + c), ev = *reinterpret_cast<const floatx4*>(e + c);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) best_of(b, xv[u] - logf(ev[u]), c + u);
+    }
+  } else {
+#pragma unroll 4
+    for (int c = t; c < classes; c += N) best_of(b, x[c] - logf(e[c]), c);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) best_of(b, __shfl_xor(b.v, o), __shfl_xor(b.i, o));
+  if constexpr (WAVES > 1) {
+    if (lane == 0) part[wave] = b;
+    __syncthreads();
+    b = part[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) best_of(b, part[w].v, part[w].i);
+  }
+  if (t == 0) targets[row] = b.i < classes ? b.i : 0;
+}
+
+}  // namespace ak
+
+extern "C" int ak_sample_categorical(const float* logits, const float* q, int64_t rows, int64_t classes, int64_t* targets,
+                                     ak_stream_t stream) {
+  if (logits == nullptr || q == nullptr || targets == nullptr || rows <= 0 || classes <= 0) return AK_ERR_ARG;
+  if (classes > (1 << 30) || rows > 0x7fffffff) return AK_ERR_TOO_LARGE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // a wave covers 256 classes per step of four: up to 1024 classes one wave per row leaves no lane idle for long
+  if (classes <= 1024)
+    hipLaunchKernelGGL(ak::sample_categorical_kernel<1>, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, s, logits,
+                       q, rows, static_cast<int>(classes), targets);
+  else
+    hipLaunchKernelGGL(ak::sample_categorical_kernel<4>, dim3(static_cast<unsigned>(rows)), dim3(256), 0, s, logits, q, rows,
+                       static_cast<int>(classes), targets);
+  return ak::check_launch();
+}

@@ -263,6 +263,23 @@ static __global__ __launch_bounds__(256) void uw_inv_grouped_kernel(const int64_
   if (__syncthreads_or(any) && threadIdx.x == 0) flags[0] = 1;
 }
 
+// For modules whose blocks were all zero (flags[0] == 0 after uw_inv_grouped_kernel): inv <- the previous inverse, or the
+// identity where there is none.  table as above with the previous inverse's address (0: none) in place of the blocks'.
+static __global__ __launch_bounds__(256) void uw_keep_grouped_kernel(const int64_t* __restrict__ table, int count) {
+  const int w = blockIdx.x;
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (table[static_cast<int64_t>(mid) * 6 + 4] <= w) lo = mid;
+    else hi = mid - 1;
+  }
+  const int64_t* __restrict__ r = table + static_cast<int64_t>(lo) * 6;
+  if (reinterpret_cast<const int*>(r[2])[0] != 0) return;
+  const floatx4* __restrict__ prev = reinterpret_cast<const floatx4*>(r[0]);
+  const int64_t f = static_cast<int64_t>(w - r[4]) * 256 + threadIdx.x;
+  if (f < r[3]) reinterpret_cast<floatx4*>(r[1])[f] = prev != nullptr ? prev[f] : floatx4{1.f, 0.f, 0.f, 1.f};
+}
+
 static __global__ void uw_reset_kernel(int* flag, int* info) {
   flag[0] = 0;
   info[0] = 0x7fffffff;
@@ -413,6 +430,16 @@ extern "C" int ak_unit_wise_inv_grouped(const int64_t* table, int count, int64_t
   if (count == 0 || total_blocks == 0) return AK_OK;
   if (table == nullptr) return AK_ERR_ARG;
   hipLaunchKernelGGL(uw_inv_grouped_kernel, dim3(static_cast<unsigned>(total_blocks)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), table, count);
+  return check_launch();
+}
+
+extern "C" int ak_unit_wise_keep_grouped(const int64_t* table, int count, int64_t total_blocks, ak_stream_t stream) {
+  using namespace ak;
+  if (count < 0 || total_blocks < 0 || total_blocks > (1ll << 30)) return AK_ERR_ARG;
+  if (count == 0 || total_blocks == 0) return AK_OK;
+  if (table == nullptr) return AK_ERR_ARG;
+  hipLaunchKernelGGL(uw_keep_grouped_kernel, dim3(static_cast<unsigned>(total_blocks)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), table, count);
   return check_launch();
 }

@@ -9,13 +9,14 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
+from . import kernels
 from .core import no_centered_cov
 from .grad_maker import GradientMaker, LOSS_CROSS_ENTROPY, LOSS_MSE
 from .profiling import nvtx_range, phase_mark
 from .matrices import *
 from .operations import OperationContext
 from .symmatrix import SymMatrix, batched_unit_update_inv, batched_update_inv
-from .utils import skip_param_grad
+from .utils import manual_seed, skip_param_grad
 
 __all__ = ['FisherConfig', 'get_fisher_maker', 'FisherMaker']
 
@@ -95,6 +96,10 @@ class FisherMaker(GradientMaker):
         pending, self._caller_flags = self._caller_flags, None
         return pending
 
+    def add_caller_flags(self, late):
+        """``late``: objects with check() that the caller is to read with take_caller_flags()."""
+        self._caller_flags = (self._caller_flags or []) + [l for l in late if l is not None]
+
     def zero_fisher(self, fvp=False):
         attr = self.config.fvp_attr if fvp else self.config.fisher_attr
         for module in self.model.modules():
@@ -158,7 +163,7 @@ class FisherMaker(GradientMaker):
         if not accumulate:
             self.zero_fisher()
         if config.seed is not None:
-            torch.random.manual_seed(config.seed)
+            manual_seed(config.seed)
 
         loss_grad_with_fisher = calc_loss_grad and self.is_fisher_emp
         loss_grad_after_fisher = calc_loss_grad and not self.is_fisher_emp
@@ -234,15 +239,18 @@ class FisherMaker(GradientMaker):
             if deferred is not None:
                 self.check_late_flags()         # of the previous update: read long ago by the device's clock
                 to_caller = self.flags_to_caller and not self.late_inverse_flags
-                late = deferred.finish_late(config.fisher_attr, warn=self.late_inverse_flags) if (self.late_inverse_flags or to_caller) else None
+                late = deferred.finish_late(config.fisher_attr, units=to_caller) if (self.late_inverse_flags or to_caller) else None
                 if late is None:
                     deferred.finish(config.fisher_attr)
                 elif to_caller:
-                    self._caller_flags = late
+                    self.add_caller_flags(late)
                 else:
                     self._late_flags = late
             if early is not None:
-                early.finish()
+                if self.flags_to_caller:
+                    self.add_caller_flags([early.finish_late()])
+                else:
+                    early.finish()
         phase_mark('upd_inv')             # what is left of the inverses once the loss backward pass has ended
         return self._model_output, loss
 
@@ -322,20 +330,29 @@ class FisherMCCrossEntropy(FisherMaker):
     def _fisher_loop(self, closure):
         logits = self._logits
         n_mc_samples = self.config.n_mc_samples
-        probs = F.softmax(logits, dim=-1)
         log_probs = F.log_softmax(logits, dim=-1)
-        # validate_args=False: the check of the simplex constraint would synchronise the host with the forward
-        # pass; the draw itself (normalisation + multinomial) is unchanged
-        dist = torch.distributions.Categorical(probs, validate_args=False)
+        dist = None
+        if self._sampling_replaced or not kernels.sampleable(logits):
+            # validate_args=False: the check of the simplex constraint would synchronise the host with the forward
+            # pass; the draw itself (normalisation + multinomial) is unchanged
+            dist = torch.distributions.Categorical(F.softmax(logits, dim=-1), validate_args=False)
         for i in range(n_mc_samples):
             with torch.no_grad():
-                targets = self.sample_targets(dist, i)
-            closure(lambda: F.nll_loss(log_probs.view(-1, log_probs.size(-1)), targets.view(-1), reduction='sum',
-                                       ignore_index=self.config.ignore_index) / n_mc_samples,
-                    retain_graph=i < n_mc_samples - 1)
+                targets = kernels.sample_categorical(logits) if dist is None else self.sample_targets(dist, i)
+
+            def nll_expr():
+                nll = F.nll_loss(log_probs.view(-1, log_probs.size(-1)), targets.view(-1), reduction='sum',
+                                 ignore_index=self.config.ignore_index)
+                return nll if n_mc_samples == 1 else nll / n_mc_samples
+            closure(nll_expr, retain_graph=i < n_mc_samples - 1)
+
+    @property
+    def _sampling_replaced(self):
+        return 'sample_targets' in self.__dict__ or type(self).sample_targets is not FisherMCCrossEntropy.sample_targets
 
     def sample_targets(self, dist, i):
-        """One draw of the model's predictive distribution; override to replay fixed targets."""
+        """One draw of the model's predictive distribution; override to replay fixed targets.  (Without an override,
+        float32 logits on the GPU are sampled by one kernel from the same random numbers, kernels.sample_categorical.)"""
         return dist.sample()
 
 

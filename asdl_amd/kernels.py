@@ -244,6 +244,41 @@ class main_stream_launches:
         return False
 
 
+class launches_on:
+    """Context: kernel launches of this thread (and the framework ops that feed them) go to the torch stream ``stream``."""
+
+    def __init__(self, stream):
+        self._stream = stream
+
+    def __enter__(self):
+        self._saved = (getattr(_override, 'handle', None), getattr(_override, 'stream', None))
+        _override.handle, _override.stream = self._stream.cuda_stream, self._stream
+
+    def __exit__(self, *exc):
+        _override.handle, _override.stream = self._saved
+        return False
+
+
+_order_events = threading.local()
+
+
+def order_streams(before, after, device):
+    """Stream ``after`` waits for everything enqueued on ``before`` so far (raw handles; None: the calling thread's launch
+    stream).  Two runtime calls on an event of this thread and device."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    events = _order_events.__dict__
+    event = events.get(index)
+    if event is None:
+        event = ctypes.c_void_p()
+        with torch.cuda.device(index):
+            _lib.check(_lib.load().ak_event_create(ctypes.byref(event), 0), 'ak_event_create')
+        events[index] = event
+    main = None if before is not None and after is not None else _stream_handle(device)
+    rc = _lib.load().ak_stream_order(ctypes.c_void_p(main if before is None else before),
+                                     ctypes.c_void_p(main if after is None else after), event)
+    _lib.check(rc, 'ak_stream_order')
+
+
 def _on_launch_stream():
     """Context for the few framework ops (copies to a contiguous layout, casts) that feed a kernel: they have to run
     on the stream the kernel is launched on."""
@@ -839,6 +874,21 @@ def unit_wise_inv_grouped(blocks_list, dampings, outs=None):
     return invs, flags
 
 
+def unit_wise_keep_grouped(invs, previous, flags):
+    """invs[i] <- previous[i] (None: the identity) where flags[i, 0] of unit_wise_inv_grouped() says that all blocks of
+    module i were zero.  No host synchronisation."""
+    rows, first = [], 0
+    for i, (inv, prev) in enumerate(zip(invs, previous)):
+        F = inv.shape[0]
+        if prev is not None and (prev.shape != inv.shape or prev.dtype != inv.dtype or not prev.is_contiguous()):
+            raise ValueError('a previous inverse has to be a contiguous float32 tensor of the same shape')
+        rows.append((0 if prev is None else prev.data_ptr(), inv.data_ptr(), flags.data_ptr() + 8 * i, F, first, 0))
+        first += (F + 255) // 256
+    table = device_table(tuple(rows), flags.device)
+    rc = _lib.load().ak_unit_wise_keep_grouped(ctypes.c_void_p(table.data_ptr()), len(rows), first, _stream())
+    _lib.check(rc, 'ak_unit_wise_keep_grouped')
+
+
 def unit_wise_mvp(mat, vec_weight, vec_bias, scale=1.0):
     """[vec_weight, vec_bias][f] <- mat[f] @ (scale * [vec_weight, vec_bias][f]) in place."""
     _require_gpu(mat, vec_weight, vec_bias)
@@ -903,8 +953,8 @@ def identity_where_zero(outs, nonzero, flag_index):
     _lib.check(rc, 'ak_identity_where_zero')
 
 
-def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None):
-    """Returns (lam [batch, 2] float32, nonzero [batch, 2] int32), both on the device.  A factor is a square
+def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None, nonzero=None):
+    """Returns (lam [batch, 2] float32, nonzero [batch, 2] int32: ``nonzero`` itself if given), both on the device.  A factor is a square
     [d, d] matrix or, for the low-rank (swift) factors, an [n, d] matrix with n < d rows; ``eig_scale``: optional
     per-pair (sA, sB) multiplied into the eigenvalue means before the pi split."""
     _require_gpu(*A_list, *B_list)
@@ -918,7 +968,10 @@ def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None):
             raise ValueError('a factor has to be square or have fewer rows than columns')
         swift = swift or t.shape[0] != t.shape[1]
     lam = torch.empty(batch, 2, dtype=torch.float32, device=dev)
-    nonzero = torch.empty(batch, 2, dtype=torch.int32, device=dev)
+    if nonzero is None:
+        nonzero = torch.empty(batch, 2, dtype=torch.int32, device=dev)
+    if nonzero.dtype != torch.int32 or nonzero.shape != (batch, 2) or not nonzero.is_contiguous():
+        raise ValueError('nonzero has to be a contiguous int32 [batch, 2] tensor')
     pa, pb = device_ptr_array(A_list), device_ptr_array(B_list)
     if not swift:
         dims = device_ints(tuple((a.shape[0], b.shape[0]) for a, b in zip(A_list, B_list)), dev)
@@ -941,6 +994,29 @@ def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None):
                                            ctypes.c_void_p(nonzero.data_ptr()), _stream())
     _lib.check(rc, 'ak_kron_damping_swift')
     return lam, nonzero
+
+
+# ------------------------------------------------------------------------------ sampling
+def sampleable(logits):
+    """Whether sample_categorical() takes these logits."""
+    return logits.is_cuda and logits.dtype == torch.float32 and logits.ndim >= 2 and logits.is_contiguous() and \
+        logits.numel() > 0
+
+
+def sample_categorical(logits):
+    """One class per row of float32 ``logits`` [..., classes] from softmax(logits): the draw of
+    torch.distributions.Categorical(softmax(logits)).sample() from the same exponential random numbers (the largest of
+    p_i / q_i, q exponential), without forming the probabilities, their checks and the quotient in device memory."""
+    _require_gpu(logits)
+    if not sampleable(logits):
+        raise ValueError('logits have to be contiguous float32 with at least two dimensions')
+    logits = logits.detach()
+    q = torch.empty_like(logits.view(-1, logits.shape[-1])).exponential_()
+    targets = torch.empty(logits.shape[:-1], dtype=torch.int64, device=logits.device)
+    rc = _lib.load().ak_sample_categorical(ctypes.c_void_p(logits.data_ptr()), ctypes.c_void_p(q.data_ptr()), q.shape[0],
+                                           q.shape[1], ctypes.c_void_p(targets.data_ptr()), _stream())
+    _lib.check(rc, 'ak_sample_categorical')
+    return targets
 
 
 # ------------------------------------------------------------------------------ low-rank (swift) factors

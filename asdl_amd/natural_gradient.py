@@ -237,6 +237,7 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             OVERLAP_INVERSE_UPDATE and self.do_accumulate and self.do_update_curvature(step)
             and self.do_update_preconditioner(step))
         self._kron_inverses_current = False
+        self.fisher_maker.take_caller_flags()
         # precondition() follows in this very call: it may read the flags of the inverses once it has launched
         self.fisher_maker.flags_to_caller = bool(FLAGS_AFTER_PRECONDITION)
         try:
@@ -285,8 +286,13 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
                 and set(kron) == {'A', 'B'} and damping == self.config.damping:
             matrices = []        # already inverted beside the loss backward pass of this call
             self._kron_inverses_current = False
-        batched_update_inv(matrices, damping, calc_A_inv='A' in kron, calc_B_inv='B' in kron)
-        batched_unit_update_inv(units, damping)
+        # inside forward_and_backward() the preconditioning follows: it launches on the inverses and then reads their flags
+        late = self.fisher_maker.flags_to_caller and not zero_curvature and \
+            all(t is None or t.is_cuda for m in matrices for t in (m.A, m.B)) and all(u.data is None or u.data.is_cuda for u in units)
+        pending = batched_update_inv(matrices, damping, calc_A_inv='A' in kron, calc_B_inv='B' in kron, defer=late, beside=False)
+        late_units = batched_unit_update_inv(units, damping, late=late)
+        if late:
+            self.fisher_maker.add_caller_flags([late_units, pending.finish_late() if pending is not None else None])
         if zero_curvature:
             for unit in units:
                 unit.mul_(0)

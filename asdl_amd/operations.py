@@ -21,7 +21,7 @@ import torch.nn as nn
 from . import kernels
 from . import profiling as _profiling
 from .profiling import nvtx_range
-from .symmatrix import Kron, SymMatrix, UnitWise, batched_update_inv
+from .symmatrix import Kron, LateUnitFlags, SymMatrix, UnitWise, batched_update_inv
 from .utils import UnfoldedInput, im2col_2d, original_requires_grad
 
 OP_COV_KRON = 'cov_kron'
@@ -533,14 +533,17 @@ class DeferredInverses:
         self._chunks = chunks            # [(PendingInverses, [(module, kron), ...]), ...]
         self._context = context
 
-    def finish_late(self, attr=None, warn=True):
+    def finish_late(self, attr=None, units=False):
         """finish() without its host synchronisation (PendingInverses.finish_late): returns objects whose check()
         reads the flags later (and, like finish(), removes from ``module.<attr>.kron`` the inverse of an all-zero
-        factor that had none before).  None when the context also has unit-wise flags to read, which only finish()
-        does."""
+        factor that had none before).  With ``units`` the unit-wise flags are among them; without, None when the context
+        has unit-wise flags to read, which then only finish() does."""
+        late_units = []
+        if self._context is not None and self._context._unit_flags and units:
+            late_units = [self._context.late_unit_flags()]
         if self._context is not None and self._context._unit_flags:
             global _warned_late_fallback
-            if warn and not _warned_late_fallback:
+            if not _warned_late_fallback:
                 _warned_late_fallback = True
                 warnings.warn('late_inverse_flags: this model has unit-wise (BatchNorm / LayerNorm) blocks, whose flags '
                               'are read at once; the flags of the Kronecker factors are read with them.')
@@ -549,8 +552,8 @@ class DeferredInverses:
             self._context._unit_flags_deferred = False      # nothing was deferred to this object's finish()
         for pending, _ in self._chunks:
             pending.join()
-        return [LateChunk(late, targets, attr) for late, targets in
-                ((pending.finish_late(), targets) for pending, targets in self._chunks) if late is not None]
+        return late_units + [LateChunk(late, targets, attr) for late, targets in
+                             ((pending.finish_late(), targets) for pending, targets in self._chunks) if late is not None]
 
     def finish(self, attr):
         if self._context is not None:
@@ -709,6 +712,22 @@ class OperationContext:
             store['inv'] = inv
             self._unit_flags.append((op._module, flags[i]))
 
+    def late_unit_flags(self):
+        """check_unit_flags() as an object whose check() does the reading."""
+        pending, self._unit_flags = self._unit_flags, []
+        self._unit_flags_deferred = False
+        modules = [m for m, _ in pending]
+        return LateUnitFlags(self._unit_flag_rows(pending),
+                             lambda i, block: f'unit-wise block {block} of {modules[i]} + damping is singular')
+
+    @staticmethod
+    def _unit_flag_rows(pending):
+        first = pending[0][1]
+        whole = first._base if first._base is not None else first
+        if whole.ndim == 2 and whole.shape[0] == len(pending):       # the rows of one call, in order: no gathering
+            return whole
+        return torch.stack([f for _, f in pending])
+
     def check_unit_flags(self):
         """torch.inverse raises for a singular block (asdl/operations/operation.py:317-320); here the flags of all
         modules are read with one copy."""
@@ -717,7 +736,7 @@ class OperationContext:
         self._unit_flags_deferred = False
         if not pending:
             return
-        host = torch.stack([f for _, f in pending]).cpu().tolist()
+        host = self._unit_flag_rows(pending).cpu().tolist()
         for (module, _), (nonzero, bad) in zip(pending, host):
             if bad != 0x7fffffff:
                 raise torch.linalg.LinAlgError(f'unit-wise block {bad - 1} of {module} + damping is singular')

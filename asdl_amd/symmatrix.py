@@ -79,25 +79,22 @@ def _side_streams(device, n):
     return pool[:n]
 
 
-_enqueue_workers = {}
 _next_side_stream = 0
-
-
-def _worker(stream_index):
-    """One enqueue thread per side stream.  The launches of a batched inverse are a few dozen small kernels
-    issued from C without the interpreter lock, so the caller can go on (with the backward pass) while they are
-    being issued; a single thread per stream keeps the jobs of that stream, which share its workspace, in
-    order."""
-    w = _enqueue_workers.get(stream_index)
-    if w is None:
-        from concurrent.futures import ThreadPoolExecutor
-        w = ThreadPoolExecutor(max_workers=1, thread_name_prefix=f'asdl_amd_inv{stream_index}')
-        _enqueue_workers[stream_index] = w
-    return w
 
 
 def _is_all_none(xs):
     return all(x is None for x in xs)
+
+
+def _flags_to_host(flags):
+    """(host copy under way, event behind it): a copy to pinned memory on the current stream."""
+    if not flags.is_cuda:
+        return flags.clone(), None
+    host = torch.empty(flags.shape, dtype=flags.dtype, pin_memory=True)
+    host.copy_(flags, non_blocking=True)
+    event = torch.cuda.Event()
+    event.record()
+    return host, event
 
 
 class LateFlags:
@@ -135,25 +132,21 @@ class LateFlags:
 class PendingInverses:
     """Inverses that have been enqueued (on side streams) but whose flags have not been read yet.
     finish() joins the streams into the current one, reads all flags with one device-to-host copy,
-    raises for a matrix that is not positive definite and stores the inverses on the Kron objects."""
+    raises for a matrix that is not positive definite and stores the inverses on the Kron objects.
+    ``flags``: int32 tensor, the Cholesky info word of every record followed by the non-zero words of all factors."""
 
-    def __init__(self, records, infos, nz_flat, events, replace, keep_alive=None, futures=(), fresh=None):
-        self._records, self._infos, self._nz_flat = records, infos, nz_flat
+    def __init__(self, records, flags, nz_flat, side_streams, replace, keep_alive=None, fresh=None):
+        self._records, self._flags, self._nz_flat = records, flags, nz_flat
         self._fresh = list(fresh) if fresh is not None else [True] * len(records)   # output buffers that held no inverse
         self._keep_alive = keep_alive      # tensors the side-stream kernels still read
-        self._events, self._replace = events, replace
-        self._futures = list(futures)      # enqueue jobs running on worker threads; each returns an event
+        self._side_streams, self._replace = side_streams, replace
         self._done = False
 
     def join(self):
-        """Makes the current stream wait for the inverses (no host synchronisation beyond the enqueue
-        jobs themselves)."""
-        events = list(self._events) + [f.result() for f in self._futures]
-        self._events, self._futures = [], []
-        if events:
-            main = torch.cuda.current_stream()
-            for ev in events:
-                main.wait_event(ev)
+        """Makes the current stream wait for the inverses (no host synchronisation)."""
+        side, self._side_streams = self._side_streams, ()
+        for st in side:
+            kernels.order_streams(st.cuda_stream, None, st.device)
 
     def finish_late(self):
         """finish() without its host synchronisation: the inverses are stored on the Kron objects as if every factor
@@ -168,15 +161,8 @@ class PendingInverses:
         fresh = [(flat, out) for (flat, k, which, out), was_fresh in zip(self._records, self._fresh) if was_fresh]
         if fresh:
             kernels.identity_where_zero([out for _, out in fresh], self._nz_flat, [flat for flat, _ in fresh])
-        flags = torch.cat(self._infos + [self._nz_flat])
-        event = None
-        if flags.is_cuda:
-            host = torch.empty(flags.shape, dtype=flags.dtype, pin_memory=True)
-            host.copy_(flags, non_blocking=True)
-            event = torch.cuda.Event()
-            event.record()
-        else:
-            host = flags.clone()
+        flags = self._flags
+        host, event = _flags_to_host(flags)
         for (flat, k, which, out) in self._records:
             setattr(k, which + '_inv', out)
             if self._replace:
@@ -192,7 +178,7 @@ class PendingInverses:
             return
         self._done = True
         self.join()
-        host = torch.cat(self._infos + [self._nz_flat]).cpu().tolist()        # the one synchronisation
+        host = self._flags.cpu().tolist()        # the one synchronisation
         n = len(self._records)
         info_host, nz_host = host[:n], host[n:]
         self._keep_alive = None
@@ -209,14 +195,15 @@ class PendingInverses:
 
 
 def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_inv=True, eps=1e-7, replace=False,
-                       defer=False):
+                       defer=False, beside=True):
     """Kron.update_inv for many Kron objects at once (asdl/symmatrix.py:499-534 per object).
 
     One damping launch for all pairs, one batched Cholesky inverse per distinct matrix size, and
     a single device-to-host read at the end for the zero / not-positive-definite flags (the
     reference synchronises three to five times per layer).  With ``defer=True`` the launches are
     enqueued and a PendingInverses is returned: the caller may enqueue unrelated work (the loss
-    backward pass) before calling its finish()."""
+    backward pass) before calling its finish(); ``beside=False``: that work needs the inverses, so they
+    go to the current stream instead of one beside it."""
     krons = [k for k in krons if k is not None]
     if not krons:
         return None
@@ -239,61 +226,64 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
     eig_scale = None
     if any(getattr(k, '_eig_scale', None) is not None for k in krons):
         eig_scale = [getattr(k, '_eig_scale', None) or (1.0, 1.0) for k in krons]
-    lam, nonzero = kernels.kron_damping(A_list, B_list, float(damping), float(eps), eig_scale=eig_scale)
+    # entries: (flat index, matrix, kron, 'A'|'B'); a row matrix ([n, d], n < d) is inverted through its Gram matrix
+    square, low_rank = [], []
+    for i, k in enumerate(krons):
+        for flat, mat, which, wanted in ((2 * i, A_list[i], 'A', calc_A_inv), (2 * i + 1, B_list[i], 'B', calc_B_inv)):
+            if wanted:
+                (square if mat.shape[0] == mat.shape[1] else low_rank).append((flat, mat, k, which))
+    n_records = len(square) + len(low_rank)
+    # all flags in one tensor, so that one copy reads them: info words of the records, then the non-zero words
+    flags = torch.empty(n_records + 2 * len(krons), dtype=torch.int32, device=dev)
+    infos, nz_flat = flags[:n_records], flags[n_records:]
+    where = dict(nonzero=nz_flat.view(-1, 2)) if mats_on_gpu else {}
+    lam, nonzero = kernels.kron_damping(A_list, B_list, float(damping), float(eps), eig_scale=eig_scale, **where)
+    if not where:
+        nz_flat.copy_(nonzero.view(-1))
     single = [i for i, k in enumerate(krons) if not (k.has_A and k.has_B)]
     if single:
         lam[kernels.device_ints(tuple(single), dev)] = float(damping)      # no pi split without both factors
-    lam_flat, nz_flat = lam.view(-1), nonzero.view(-1)
+    lam_flat = lam.view(-1)
 
-    groups = defaultdict(list)   # d -> [(flat index, matrix, kron, 'A'|'B')]
-    low_rank = []                # the same entries for [n, d] row matrices (n < d), inverted through their Gram matrix
-    for i, k in enumerate(krons):
-        if calc_A_inv:
-            entry = (2 * i, A_list[i], k, 'A')
-            (groups[A_list[i].shape[0]] if A_list[i].shape[0] == A_list[i].shape[1] else low_rank).append(entry)
-        if calc_B_inv:
-            entry = (2 * i + 1, B_list[i], k, 'B')
-            (groups[B_list[i].shape[0]] if B_list[i].shape[0] == B_list[i].shape[1] else low_rank).append(entry)
+    def output(mat, k, which, d):
+        old = getattr(k, which + '_inv')
+        reuse = old is not None and tuple(old.shape) == (d, d) and old.is_contiguous() and old.dtype == mat.dtype
+        fresh.append(not reuse)
+        return old if reuse else torch.empty(d, d, dtype=mat.dtype, device=dev)
+
     # GROUPED_INVERSE: every square factor of the call goes into one grouped inverse, whose launches carry the steps
     # of all matrices at once.  Otherwise each size group is an independent chain of small launches, and the groups
     # are spread over a few side streams (default priority) so that their launch latencies overlap.  Either way
     # everything joins the caller's stream again.
-    if GROUPED_INVERSE and groups:
-        merged = [e for d in sorted(groups, reverse=True) for e in groups[d]]
-        groups = {-1: merged}
-    order = sorted(groups, key=lambda d: sum(e[1].shape[0] ** 3 for e in groups[d]), reverse=True)
-    prepared = []
-    fresh_of = {}                # id(output buffer) -> it held no inverse before
-    for d in order:
-        entries = groups[d]
-        idx = kernels.device_ints(tuple(e[0] for e in entries), dev)
-        outs = []
-        for _, mat, k, which in entries:
-            old = getattr(k, which + '_inv')
-            reuse = old is not None and old.shape == mat.shape and old.is_contiguous() and old.dtype == mat.dtype
-            outs.append(old if reuse else torch.empty_like(mat))
-            fresh_of[id(outs[-1])] = not reuse
-        info = torch.empty(len(entries), dtype=torch.int32, device=dev)
-        prepared.append((entries, outs, lam_flat[idx], nz_flat[idx].contiguous(), info))
-    for flat, mat, k, which in low_rank:
-        # (x^T x / n + lam I)^-1 by Sherman-Morrison-Woodbury (smw_inv, asdl/utils.py:107-115): a group of its own
-        d = mat.shape[1]
-        old = getattr(k, which + '_inv')
-        reuse = old is not None and tuple(old.shape) == (d, d) and old.is_contiguous() and old.dtype == mat.dtype
-        out = old if reuse else torch.empty(d, d, dtype=mat.dtype, device=dev)
-        fresh_of[id(out)] = not reuse
-        info = torch.empty(1, dtype=torch.int32, device=dev)
-        prepared.append(([(flat, mat, k, which)], [out], lam_flat[flat:flat + 1], None, info))
+    if GROUPED_INVERSE:
+        groups = [square] if square else []
+    else:
+        by_size = defaultdict(list)
+        for e in square:
+            by_size[e[1].shape[0]].append(e)
+        groups = list(by_size.values())
+    groups += [[e] for e in low_rank]
+    prepared, records, fresh = [], [], []       # fresh: this record's output buffer held no inverse before
+    for entries in groups:
+        outs = [output(mat, k, which, mat.shape[1]) for _, mat, k, which in entries]
+        info = infos[len(records):len(records) + len(entries)]
+        records.extend((flat, k, which, out) for (flat, _, k, which), out in zip(entries, outs))
+        index = tuple(e[0] for e in entries)
+        low = entries[0][1].shape[0] != entries[0][1].shape[1]
+        if index == tuple(range(index[0], index[0] + len(index))):
+            lam_g, act_g = lam_flat[index[0]:index[0] + len(index)], nz_flat[index[0]:index[0] + len(index)]
+        else:
+            idx = kernels.device_ints(index, dev)
+            lam_g, act_g = lam_flat[idx], nz_flat[idx].contiguous()
+        prepared.append((entries, outs, lam_g, None if low else act_g, info))
     prepared.sort(key=lambda g: -sum(e[1].shape[0] * e[1].shape[1] ** 2 for e in g[0]))
-    infos, records, events, futures = [], [], [], []
-    use_streams = mats_on_gpu and (len(prepared) > 1 or defer)
-
     range_name = 'inv_kron' + ('_A' if calc_A_inv else '') + ('_B' if calc_B_inv else '')
 
     def run_group(group):
         entries, outs, lam_g, act_g, info = group
         with nvtx_range(range_name):
             if act_g is None:          # a low-rank factor
+                # (x^T x / n + lam I)^-1 by Sherman-Morrison-Woodbury (smw_inv, asdl/utils.py:107-115)
                 kernels.smw_inv(entries[0][1], lam_g, out=outs[0], info=info)
             elif GROUPED_INVERSE:
                 kernels.chol_inv_grouped([e[1] for e in entries], outs, lam_g, 1, active=act_g, active_stride=1,
@@ -302,60 +292,75 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
                 kernels.chol_inv_batched([e[1] for e in entries], outs, lam_g, 1, active=act_g, active_stride=1,
                                          info=info)
 
-    if use_streams:
-        main = torch.cuda.current_stream()
-        # successive calls start on different side streams (each with its own enqueue thread and workspace), so
-        # that an early batch and the remainder of one step run side by side
+    side = []
+    if mats_on_gpu and (len(prepared) > 1 or (defer and beside)):
+        # Successive calls start on different side streams (each with its own workspace), so that an early batch and
+        # the remainder of one step run side by side.  The launches are issued from here: handing them to another
+        # thread cost more in interpreter-lock changes (0.6 ms of a small step) than the launches themselves.
         global _next_side_stream
         pool = _side_streams(dev, N_SIDE_STREAMS)
-        first = _next_side_stream % len(pool)
         n_used = min(len(pool), len(prepared))
+        side = [pool[(_next_side_stream + i) % len(pool)] for i in range(n_used)]
         _next_side_stream += n_used
-        chosen = [(first + i) % len(pool) for i in range(n_used)]
-        side = [pool[i] for i in chosen]
-        start = torch.cuda.Event()
-        start.record(main)
-        per_stream = [prepared[i::len(side)] for i in range(len(side))]
-
-        def run_stream(st, groups_of_stream):
-            with torch.cuda.device(dev), torch.cuda.stream(st):
-                st.wait_event(start)
-                for group in groups_of_stream:
+        for i, st in enumerate(side):
+            kernels.order_streams(None, st.cuda_stream, dev)
+            with kernels.launches_on(st):
+                for group in prepared[i::n_used]:
                     run_group(group)
-                done = torch.cuda.Event()
-                done.record(st)
-            return done
-
-        for si, st, groups_of_stream in zip(chosen, side, per_stream):
-            if defer:
-                futures.append(_worker(si).submit(run_stream, st, groups_of_stream))
-            else:
-                events.append(run_stream(st, groups_of_stream))
     else:
         for group in prepared:
             run_group(group)
-    for entries, outs, lam_g, act_g, info in prepared:
-        infos.append(info)
-        records.extend((e[0], e[2], e[3], out) for e, out in zip(entries, outs))
-    pending = PendingInverses(records, infos, nz_flat, events, replace,
-                              keep_alive=(prepared, lam, nonzero, A_list, B_list), futures=futures,
-                              fresh=[fresh_of[id(r[3])] for r in records])
+    pending = PendingInverses(records, flags, nz_flat, side, replace,
+                              keep_alive=(prepared, lam, A_list, B_list), fresh=fresh)
     if defer:
         return pending
     pending.finish()
     return None
 
 
-def batched_unit_update_inv(units, damping=_default_damping, replace=False):
+class LateUnitFlags:
+    """The unread flags of a batch of unit-wise inverses, [count, 2] (non-zero, first singular block) on their way to pinned
+    host memory; ``singular(i, block)`` names module i in the error, ``all_zero(i)`` is told of modules that were all zero."""
+
+    def __init__(self, flags, singular, all_zero=None):
+        self._host, self._event = _flags_to_host(flags)
+        self._flags, self._singular, self._all_zero = flags, singular, all_zero
+
+    def check(self, *args, **kwargs):
+        if self._flags is None:
+            return []
+        if self._event is not None:
+            self._event.synchronize()
+        self._flags = None
+        for i, (nonzero, bad) in enumerate(self._host.tolist()):
+            if not nonzero and self._all_zero is not None:
+                self._all_zero(i)
+            elif bad != 0x7fffffff:
+                raise torch.linalg.LinAlgError(self._singular(i, bad - 1))
+        return []
+
+
+def batched_unit_update_inv(units, damping=_default_damping, replace=False, late=False):
     """UnitWise.update_inv (asdl/symmatrix.py:687-699) for many modules: one grouped launch, then a single
-    device-to-host read for all zero / singular flags instead of one per module."""
+    device-to-host read for all zero / singular flags instead of one per module.  ``late`` (GPU only): the flags are left
+    on the device and returned as a LateUnitFlags; until they are read, all-zero modules without an earlier inverse have
+    the identity, those with one keep it."""
     units = [u for u in units if u is not None]
     for u in units:
         if not u.has_data:
             raise ValueError('data do not exist.')
     if not units:
-        return
+        return None
     invs, flags = kernels.unit_wise_inv_grouped([u.data for u in units], [float(damping)] * len(units))
+    if late:
+        previous = [u.inv for u in units]
+        kernels.unit_wise_keep_grouped(invs, previous, flags)
+        for u, inv in zip(units, invs):
+            u.inv = inv
+            if replace:
+                u.data = None
+        return LateUnitFlags(flags, lambda i, block: f'unit-wise block {block} + damping is singular',
+                             lambda i: setattr(units[i], 'inv', previous[i]))
     host = flags.cpu().tolist()
     for u, inv, (nonzero, bad) in zip(units, invs, host):
         if not nonzero:
@@ -365,6 +370,7 @@ def batched_unit_update_inv(units, damping=_default_damping, replace=False):
         u.inv = inv
         if replace:
             u.data = None
+    return None
 
 
 class Kron:

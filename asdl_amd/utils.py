@@ -43,6 +43,29 @@ def skip_param_grad(model, disable=False):
             restore_original_requires_grad(param)
 
 
+def manual_seed(seed):
+    """torch.random.manual_seed() without what it does for accelerators that are not there (its hook for one of them
+    formats a stack trace on every call: 55 us of a training step)."""
+    if not torch.cuda.is_initialized() or _other_accelerators():
+        torch.random.manual_seed(seed)
+        return
+    seed = int(seed)
+    for generator in torch.cuda.default_generators:
+        generator.manual_seed(seed)
+    torch.default_generator.manual_seed(seed)
+
+
+def _other_accelerators():
+    global _others
+    if _others is None:
+        _others = torch._C._get_privateuse1_backend_name() != 'privateuseone' or torch.backends.mps.is_available() or \
+            (hasattr(torch, 'xpu') and torch.xpu.is_available())
+    return _others
+
+
+_others = None
+
+
 def cholesky_inv(X, damping=1e-7):
     """(X + damping I)^-1 on the GPU; X is left unchanged; raises torch.linalg.LinAlgError when
     the damped matrix is not positive definite (asdl/utils.py:91-96)."""

@@ -150,6 +150,12 @@ int ak_conv_patch_sum(const void* x, int dtype, int64_t sn, int64_t sc, int64_t 
 int ak_identity_where_zero(float* const* out_list, const int64_t* dims, const int* nonzero,
                            const int64_t* flag_index, int count, ak_stream_t stream);
 
+/* targets[r] = argmax_i logits[r][i] - log(q[r][i]) for q exponentially distributed: a draw of softmax(logits[r]) per row
+ * (torch.multinomial's choice from the same random numbers).  Row-major [rows, classes] float32; the lowest index wins ties;
+ * NaN logits are never chosen (a row of NaNs gives 0). */
+int ak_sample_categorical(const float* logits, const float* q, int64_t rows, int64_t classes, int64_t* targets,
+                          ak_stream_t stream);
+
 /* ak_kron_damping for pairs whose factors may be n x d row matrices: dims = device int64 [batch,4]
  * (rows_A, d_A, rows_B, d_B; rows = 0: square d x d factor, eigenvalue mean trace/d; rows > 0: sum(x^2)/d),
  * eig_scale = device float [batch,2] multiplied into the eigenvalue means (may be null).
@@ -236,6 +242,9 @@ int ak_unit_wise_inv(const float* blocks, int64_t F, float damping, float* inv, 
  * inv, flags (addresses; the caller presets each flags pair to {0, 0x7fffffff}), F, first_block (running sum of
  * ceil(F/256)), damping (float bit pattern in the low 32 bits).  Same reference lines as ak_unit_wise_inv. */
 int ak_unit_wise_inv_grouped(const int64_t* table, int count, int64_t total_blocks, ak_stream_t stream);
+/* After ak_unit_wise_inv_grouped, for the modules whose blocks were all zero: inv <- the previous inverse or the identity.
+ * Rows of the table as there, with the previous inverse's address (0: none) in place of the blocks' address. */
+int ak_unit_wise_keep_grouped(const int64_t* table, int count, int64_t total_blocks, ak_stream_t stream);
 
 /* [vec_weight[f], vec_bias[f]] <- mat[f] @ (scale * [vec_weight[f], vec_bias[f]]) in place, mat = [F, 2, 2].
  * Replaces UnitWise.mvp for BatchNorm / LayerNorm (asdl/symmatrix.py:701-709, 716-719) and the grad_scale

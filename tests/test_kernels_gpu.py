@@ -740,6 +740,30 @@ def test_chol_inv_large_matches_fp32_oracle_and_fp64(K, d):
         assert torch.equal(out, out.T)
 
 
+# ------------------------------------------------------------------ sampling
+@pytest.mark.parametrize('shape', [(1, 2), (5, 10), (64, 1000), (3, 1023), (9, 1024), (4, 1025), (2, 3, 5001)])
+def test_sample_categorical_draws_what_torch_draws(K, shape):
+    """One wave per row, one work group per row, vector and scalar loads: the classes torch draws from the same seed."""
+    logits = 3 * torch.randn(shape, device='cuda', generator=torch.Generator('cuda').manual_seed(1))
+    torch.manual_seed(5)
+    ours = K.sample_categorical(logits)
+    torch.manual_seed(5)
+    theirs = torch.distributions.Categorical(torch.softmax(logits, -1), validate_args=False).sample()
+    assert ours.shape == theirs.shape and torch.equal(ours, theirs)
+
+
+@pytest.mark.parametrize('f', [1, 256, 300])
+def test_unit_wise_keep_grouped(K, f):
+    """Modules whose blocks are all zero keep their previous inverse or get the identity; the others are left alone."""
+    blocks = [torch.rand(f, 2, 2, device='cuda') + torch.eye(2, device='cuda'), torch.zeros(f, 2, 2, device='cuda'),
+              torch.zeros(f, 2, 2, device='cuda')]
+    previous = [None, torch.rand(f, 2, 2, device='cuda'), None]
+    invs, flags = K.unit_wise_inv_grouped(blocks, [0.1] * 3)
+    expected = [invs[0].clone(), previous[1], torch.eye(2, device='cuda').expand(f, 2, 2)]
+    K.unit_wise_keep_grouped(invs, previous, flags)
+    assert all(torch.equal(a, b) for a, b in zip(invs, expected))
+
+
 # ------------------------------------------------------------------ products
 @pytest.mark.parametrize('tA', [False, True])
 @pytest.mark.parametrize('tB', [False, True])
