@@ -60,6 +60,10 @@ _SIGNATURES = {
     'ak_event_destroy': (c_int, [c_ptr]),
     'ak_event_record': (c_int, [c_ptr, c_ptr]),
     'ak_sample_categorical': (c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr]),
+    'ak_event_synchronize': (c_int, [c_ptr]),
+    'ak_kron_finish': (c_int, [c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_int, c_ptr, c_ptr]),
+    'ak_kron_precond_deep_ws_bytes': (c_size, [c_ptr, c_int]),
+    'ak_kron_precond_deep': (c_int, [c_ptr, c_int, c_ptr, c_int, c_f32, c_ptr, c_ptr, c_int, c_ptr, c_size, c_ptr]),
     'ak_stream_order': (c_int, [c_ptr, c_ptr, c_ptr]),
     'ak_event_elapsed_ms': (c_int, [c_ptr, c_ptr, ctypes.POINTER(ctypes.c_float)]),
     'ak_copy_bytes': (c_int, [c_ptr, c_ptr, c_i64, c_ptr]),

@@ -56,6 +56,11 @@ extern "C" int ak_event_record(void* event, ak_stream_t stream) {
                                                                                                          : AK_ERR_LAUNCH;
 }
 
+extern "C" int ak_event_synchronize(void* event) {
+  if (event == nullptr) return AK_ERR_ARG;
+  return hipEventSynchronize(static_cast<hipEvent_t>(event)) == hipSuccess ? AK_OK : AK_ERR_LAUNCH;
+}
+
 // `after` waits for everything enqueued on `before` so far (event: scratch, re-recordable).
 extern "C" int ak_stream_order(ak_stream_t before, ak_stream_t after, void* event) {
   if (event == nullptr) return AK_ERR_ARG;

@@ -144,7 +144,41 @@ __global__ __launch_bounds__(256) void identity_where_zero_kernel(float* const* 
     out[i] = (i / d == i % d) ? 1.f : 0.f;
 }
 
+// The end of a batch of inverses, one launch: identity into the matrices out_list[m] (null: none) whose factor was all
+// zero; and, by the first work group, the flags (records' info words, then the non-zero words) to host memory that the device
+// can write, and flags[total] <- whether any inverse failed (info != 0 of a factor that is not zero), for kernels that follow.
+static __global__ __launch_bounds__(256) void kron_finish_kernel(float* const* __restrict__ out_list,
+                                                                 const int64_t* __restrict__ dims,
+                                                                 const int64_t* __restrict__ flag_index, int count,
+                                                                 int* __restrict__ flags, int total,
+                                                                 int* __restrict__ host_flags) {
+  const int m = blockIdx.y;
+  const int* __restrict__ nonzero = flags + count;
+  if (m == 0 && blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < total; i += 256) host_flags[i] = flags[i];
+    int fail = 0;
+    for (int i = threadIdx.x; i < count; i += 256) fail |= nonzero[flag_index[i]] != 0 && flags[i] != 0;
+    fail = __syncthreads_or(fail);
+    if (threadIdx.x == 0) flags[total] = fail != 0;
+  }
+  float* __restrict__ out = out_list[m];
+  if (out == nullptr || nonzero[flag_index[m]] != 0) return;
+  const int64_t d = dims[m], elements = d * d;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < elements; i += static_cast<int64_t>(gridDim.x) * 256)
+    out[i] = (i / d == i % d) ? 1.f : 0.f;
+}
+
 }  // namespace ak
+
+extern "C" int ak_kron_finish(float* const* out_list, const int64_t* dims, const int64_t* flag_index, int count, int* flags,
+                              int total, int* host_flags, ak_stream_t stream) {
+  if (out_list == nullptr || dims == nullptr || flag_index == nullptr || flags == nullptr || host_flags == nullptr ||
+      count <= 0 || total < count || count > 65535)
+    return AK_ERR_ARG;
+  hipLaunchKernelGGL(ak::kron_finish_kernel, dim3(32, count), dim3(256), 0, static_cast<hipStream_t>(stream), out_list, dims,
+                     flag_index, count, flags, total, host_flags);
+  return ak::check_launch();
+}
 
 extern "C" int ak_identity_where_zero(float* const* out_list, const int64_t* dims, const int* nonzero,
                                       const int64_t* flag_index, int count, ak_stream_t stream) {

@@ -234,7 +234,7 @@ class FisherMaker(GradientMaker):
             loss.div_(data_size)
         phase_mark('bwd_loss')            # loss backward pass (the inverses run beside it on side streams)
         if deferred is not None or early is not None:
-            if self.before_inverse_wait is not None:
+            if self.before_inverse_wait is not None and not (self.flags_to_caller and not self.late_inverse_flags):
                 self.before_inverse_wait()      # host work of the caller that needs no flags: the device is still busy
             if deferred is not None:
                 self.check_late_flags()         # of the previous update: read long ago by the device's clock

@@ -182,8 +182,10 @@ def _ws_args(nbytes, device):
 
 def device_ptr_array(tensors):
     """int64 device tensor holding the data pointers of ``tensors`` (cached by pointer tuple)."""
-    ptrs = tuple(t.data_ptr() for t in tensors)
-    dev = tensors[0].device
+    return device_addresses(tuple(t.data_ptr() for t in tensors), tensors[0].device)
+
+
+def device_addresses(ptrs, dev):
     key = (dev.index, ptrs)
     arr = _ptr_cache.get(key)
     if arr is None:
@@ -953,6 +955,98 @@ def identity_where_zero(outs, nonzero, flag_index):
     _lib.check(rc, 'ak_identity_where_zero')
 
 
+class HostFlags:
+    """Flags of a batch of inverses on their way to the host: pinned memory that the batch's last kernel writes and the
+    event behind it.  Both come from a pool per device (at most HostFlags.POOL of them, given back by read(); any thread
+    may take or give back) and are sized in steps, since a model has two or three batches of fixed sizes."""
+    POOL = 16
+    _free = {}
+    _lock = threading.Lock()
+
+    def __init__(self, device, words):
+        self._key = device.index if device.index is not None else torch.cuda.current_device()
+        entry = None
+        with HostFlags._lock:
+            free = HostFlags._free.setdefault(self._key, [])
+            for i, (host, _) in enumerate(free):
+                if host.numel() >= words:
+                    entry = free.pop(i)
+                    break
+        if entry is None:
+            event = ctypes.c_void_p()
+            with torch.cuda.device(self._key):
+                _lib.check(_lib.load().ak_event_create(ctypes.byref(event), 0), 'ak_event_create')
+            entry = (torch.empty((words + 255) // 256 * 256, dtype=torch.int32, pin_memory=True), event)
+        self._host, self._event = entry
+        self._words = words
+        self.address = self._host.data_ptr()
+
+    def record(self):
+        _lib.check(_lib.load().ak_event_record(self._event, _stream()), 'ak_event_record')
+
+    def read(self):
+        """The flags as a list; waits for the kernel that writes them."""
+        if self._host is None:
+            raise RuntimeError('the flags have been read')
+        _lib.check(_lib.load().ak_event_synchronize(self._event), 'ak_event_synchronize')
+        values = self._host[:self._words].tolist()
+        self._give_back()
+        return values
+
+    def _give_back(self):
+        entry, self._host = (self._host, self._event), None
+        with HostFlags._lock:
+            free = HostFlags._free.setdefault(self._key, [])
+            if len(free) < HostFlags.POOL:
+                free.append(entry)
+                return
+        _lib.load().ak_event_destroy(entry[1])
+
+    def __del__(self):
+        # dropped unread (an exception in between): the kernel may still be on its way to the memory
+        try:
+            if self._host is not None:
+                _lib.load().ak_event_synchronize(self._event)
+                self._give_back()
+        except Exception:
+            pass
+
+
+def kron_finish(outs, dims, flag_index, flags):
+    """The end of a batch of inverses, one launch: identity into the outputs of all-zero factors (outs[m] None: left alone),
+    the flags to the host and the batch's fail word.  flags: device int32, len(dims) info words, the non-zero words, and one
+    more word, which becomes 1 if an inverse failed.  Returns the HostFlags."""
+    dev = flags.device
+    total = flags.numel() - 1
+    host = HostFlags(dev, total)
+    ptrs = device_addresses(tuple(0 if o is None else o.data_ptr() for o in outs), dev)
+    rc = _lib.load().ak_kron_finish(ctypes.c_void_p(ptrs.data_ptr()), ctypes.c_void_p(device_ints(dims, dev).data_ptr()),
+                                    ctypes.c_void_p(device_ints(flag_index, dev).data_ptr()), len(dims),
+                                    ctypes.c_void_p(flags.data_ptr()), total, ctypes.c_void_p(host.address), _stream())
+    _lib.check(rc, 'ak_kron_finish')
+    host.record()
+    return host
+
+
+def kron_precond_deep(items, units, grad_scale, device, fail=(), only_if_faster=True):
+    """kron_precond for many modules in two launches.  items: flat list of B_inv, A_inv, grad_w, grad_b or 0 (addresses), dB,
+    dA per module; units: inv, grad_w, grad_b, F per unit-wise module; all contiguous float32.  fail: at most two addresses
+    of device words, nothing is written when one of them is not zero.  False, and nothing done, where the split products of
+    KronPrecondPlan are expected to be faster."""
+    lib = _lib.load()
+    count, n_units = len(items) // 6, len(units) // 4
+    table = (ctypes.c_int64 * len(items))(*items)
+    unit_table = (ctypes.c_int64 * len(units))(*units)
+    ws, ws_bytes, keep = _ws_args(lib.ak_kron_precond_deep_ws_bytes(table, count), device)
+    f0, f1 = (tuple(fail) + (0, 0))[:2]
+    rc = lib.ak_kron_precond_deep(table, count, unit_table, n_units, grad_scale, f0, f1, int(only_if_faster), ws, ws_bytes,
+                                  _stream(device))
+    if rc == AK_ERR_UNSUPPORTED:
+        return False
+    _lib.check(rc, 'ak_kron_precond_deep')
+    return True
+
+
 def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None, nonzero=None):
     """Returns (lam [batch, 2] float32, nonzero [batch, 2] int32: ``nonzero`` itself if given), both on the device.  A factor is a square
     [d, d] matrix or, for the low-rank (swift) factors, an [n, d] matrix with n < d rows; ``eig_scale``: optional
@@ -1120,6 +1214,8 @@ class CholGroupPlan:
         _lib.check(lib.ak_chol_group_plan(arr, len(self.dims), ctypes.c_void_p(self.host.data_ptr()), nbytes),
                    'ak_chol_group_plan')
         self.launches = lib.ak_chol_group_plan_launches(ctypes.c_void_p(self.host.data_ptr()))
+        blocks = (max(self.dims) + 127) // 128
+        self.microseconds = 25 * self.launches if self.launches == blocks + 1 else 20 * self.launches    # about
         with _on_launch_stream():
             self.dev = self.host.to(device, non_blocking=True)
 

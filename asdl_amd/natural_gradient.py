@@ -311,6 +311,8 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             grad_scale = self.grad_scale
         work = self._precondition_work()
         unread = self.fisher_maker.take_caller_flags()
+        if use_inv and GROUPED_PRECONDITION and self._precondition_deep(work, grad_scale, unread or ()):
+            return
         if not unread:
             self._precondition_launch(work, grad_scale, use_inv)
             return
@@ -326,6 +328,51 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             if grads:
                 torch._foreach_copy_(grads, saved)      # as the reference leaves them when its Cholesky raises
             raise
+
+    def _precondition_deep(self, work, grad_scale, unread):
+        """Everything in two launches (kernels.kron_precond_deep) where all modules are small, whatever their sizes'
+        alignment.  The second launch leaves the gradients alone if an inverse whose flags are still unread failed, so
+        that nothing has to be saved.  False, and nothing done, where that form does not apply or does not pay."""
+        fail = [getattr(late, 'fail_word', 0) for late in unread]
+        modules = [m for m, _ in work]
+        if not work or len(fail) > 2 or 0 in fail or modules == getattr(self, '_deep_declined', None):
+            return False
+
+        def dense(t, n):
+            return t is not None and t.is_cuda and t.dtype == torch.float32 and t.numel() == n and t.is_contiguous()
+        items, units = [], []
+        attr = self._fisher_attr
+        for module, shape in work:
+            fisher = getattr(module, attr, None)
+            params = module._parameters
+            weight, bias = params.get('weight'), params.get('bias')
+            if fisher is None or weight is None or not weight.requires_grad:
+                return False
+            gw = weight.grad
+            gb = bias.grad if bias is not None and bias.requires_grad else None
+            if bias is not None and bias.requires_grad and gb is None:
+                return False
+            if shape == SHAPE_UNIT_WISE:
+                inv = fisher.unit.inv if fisher.unit is not None else None
+                F = weight.numel()
+                if not (dense(inv, 4 * F) and dense(gw, F) and dense(gb, F)) or inv.data_ptr() % 16:
+                    return False
+                units += (inv.data_ptr(), gw.data_ptr(), gb.data_ptr(), F)
+                continue
+            kron = fisher.kron
+            B_inv, A_inv = (kron.B_inv, kron.A_inv) if kron is not None else (None, None)
+            if B_inv is None or A_inv is None or B_inv.ndim != 2 or A_inv.ndim != 2:
+                return False
+            dB, dA = B_inv.shape[0], A_inv.shape[0]
+            if not (dense(B_inv, dB * dB) and dense(A_inv, dA * dA) and dense(gw, dB * dA) and (gb is None or dense(gb, dB))):
+                return False
+            items += (B_inv.data_ptr(), A_inv.data_ptr(), gw.data_ptr(), 0 if gb is None else gb.data_ptr(), dB, dA)
+        if not kernels.kron_precond_deep(items, units, float(grad_scale), gw.device, fail):
+            self._deep_declined = modules        # the sizes decide: not asked again for these modules
+            return False
+        for late in unread:
+            late.check(when=None)
+        return True
 
     def _save_gradients(self, grads):
         """Copies of ``grads`` in one reusable buffer (one launch per dtype and device).  The views into the buffer

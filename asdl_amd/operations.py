@@ -512,6 +512,10 @@ class LateChunk:
     def __init__(self, late, targets, attr):
         self._late, self._targets, self._attr = late, targets, attr
 
+    @property
+    def fail_word(self):
+        return self._late.fail_word
+
     def check(self, *args, **kwargs):
         zero = self._late.check(*args, **kwargs)
         if zero and self._attr is not None:

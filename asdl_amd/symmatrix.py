@@ -80,6 +80,7 @@ def _side_streams(device, n):
 
 
 _next_side_stream = 0
+INLINE_MICROSECONDS = 300      # a deferred batch shorter than this runs on the caller's stream
 
 
 def _is_all_none(xs):
@@ -102,8 +103,13 @@ class LateFlags:
     for the copy, which has long arrived when it is called a step later, and raises for a factor that was not
     positive definite."""
 
-    def __init__(self, host, event, records, keep_alive):
-        self._host, self._event, self._records, self._keep_alive = host, event, records, keep_alive
+    def __init__(self, host, records, flags, keep_alive):
+        self._host, self._records, self._flags, self._keep_alive = host, records, flags, keep_alive
+
+    @property
+    def fail_word(self):
+        """Address of a device word that is 1 if an inverse of the batch failed (CPU: 0)."""
+        return self._flags.data_ptr() + 4 * (self._flags.numel() - 1) if self._flags.is_cuda else 0
 
     def check(self, when='reported late: the flags of this update were read after the next one'):
         """Raises for a factor that was not positive definite.  Returns the (Kron, 'A' | 'B') whose factor was all
@@ -111,9 +117,8 @@ class LateFlags:
         device has put the identity there, and the caller removes it again."""
         if self._host is None:
             return []
-        if self._event is not None:
-            self._event.synchronize()
-        host, self._host, self._keep_alive = self._host.tolist(), None, None
+        pending, self._host, self._keep_alive = self._host, None, None
+        host = pending.read() if isinstance(pending, kernels.HostFlags) else pending.tolist()
         n = len(self._records)
         info_host, nz_host = host[:n], host[n:]
         zero = []
@@ -133,7 +138,8 @@ class PendingInverses:
     """Inverses that have been enqueued (on side streams) but whose flags have not been read yet.
     finish() joins the streams into the current one, reads all flags with one device-to-host copy,
     raises for a matrix that is not positive definite and stores the inverses on the Kron objects.
-    ``flags``: int32 tensor, the Cholesky info word of every record followed by the non-zero words of all factors."""
+    ``flags``: int32 tensor, the Cholesky info word of every record, the non-zero words of all factors, and one more
+    word, which becomes 1 if an inverse failed."""
 
     def __init__(self, records, flags, nz_flat, side_streams, replace, keep_alive=None, fresh=None):
         self._records, self._flags, self._nz_flat = records, flags, nz_flat
@@ -158,27 +164,35 @@ class PendingInverses:
             return None
         self._done = True
         self.join()
-        fresh = [(flat, out) for (flat, k, which, out), was_fresh in zip(self._records, self._fresh) if was_fresh]
-        if fresh:
-            kernels.identity_where_zero([out for _, out in fresh], self._nz_flat, [flat for flat, _ in fresh])
-        flags = self._flags
-        host, event = _flags_to_host(flags)
+        host = self._flags_to_host(identity=True)
         for (flat, k, which, out) in self._records:
             setattr(k, which + '_inv', out)
             if self._replace:
                 setattr(k, which, None)
         # (flag index, Kron, side, did the buffer hold no inverse before)
-        late = LateFlags(host, event, [(flat, k, which, was_fresh) for (flat, k, which, _), was_fresh
-                                       in zip(self._records, self._fresh)], (flags, self._keep_alive))
+        late = LateFlags(host, [(flat, k, which, was_fresh) for (flat, k, which, _), was_fresh
+                                in zip(self._records, self._fresh)], self._flags, self._keep_alive)
         self._keep_alive = None
         return late
+
+    def _flags_to_host(self, identity):
+        """The flags on their way to the host (identity: and the identity into the fresh outputs of all-zero factors)."""
+        outs = [out if identity and was_fresh else None for (_, _, _, out), was_fresh in zip(self._records, self._fresh)]
+        index = [flat for flat, _, _, _ in self._records]
+        if self._flags.is_cuda:
+            return kernels.kron_finish(outs, tuple([r[3].shape[0] for r in self._records]), tuple(index), self._flags)
+        kept = [(o, i) for o, i in zip(outs, index) if o is not None]
+        if kept:
+            kernels.identity_where_zero([o for o, _ in kept], self._nz_flat, [i for _, i in kept])
+        return self._flags[:-1].clone()
 
     def finish(self):
         if self._done:
             return
         self._done = True
         self.join()
-        host = self._flags.cpu().tolist()        # the one synchronisation
+        host = self._flags_to_host(identity=False)
+        host = host.read() if isinstance(host, kernels.HostFlags) else host.tolist()        # the one synchronisation
         n = len(self._records)
         info_host, nz_host = host[:n], host[n:]
         self._keep_alive = None
@@ -233,9 +247,9 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
             if wanted:
                 (square if mat.shape[0] == mat.shape[1] else low_rank).append((flat, mat, k, which))
     n_records = len(square) + len(low_rank)
-    # all flags in one tensor, so that one copy reads them: info words of the records, then the non-zero words
-    flags = torch.empty(n_records + 2 * len(krons), dtype=torch.int32, device=dev)
-    infos, nz_flat = flags[:n_records], flags[n_records:]
+    # all flags in one tensor, so that one copy reads them: info words of the records, the non-zero words, the fail word
+    flags = torch.empty(n_records + 2 * len(krons) + 1, dtype=torch.int32, device=dev)
+    infos, nz_flat = flags[:n_records], flags[n_records:-1]
     where = dict(nonzero=nz_flat.view(-1, 2)) if mats_on_gpu else {}
     lam, nonzero = kernels.kron_damping(A_list, B_list, float(damping), float(eps), eig_scale=eig_scale, **where)
     if not where:
@@ -293,6 +307,10 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
                                          info=info)
 
     side = []
+    if beside and defer and mats_on_gpu and GROUPED_INVERSE and square and not low_rank:
+        # A few launches that leave most of the device idle: the two changes of stream cost the host more than running
+        # beside them saves the device.
+        beside = kernels.chol_group_plan([e[1].shape[0] for e in square], dev).microseconds > INLINE_MICROSECONDS
     if mats_on_gpu and (len(prepared) > 1 or (defer and beside)):
         # Successive calls start on different side streams (each with its own workspace), so that an early batch and
         # the remainder of one step run side by side.  The launches are issued from here: handing them to another

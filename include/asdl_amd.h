@@ -150,6 +150,25 @@ int ak_conv_patch_sum(const void* x, int dtype, int64_t sn, int64_t sc, int64_t 
 int ak_identity_where_zero(float* const* out_list, const int64_t* dims, const int* nonzero,
                            const int64_t* flag_index, int count, ak_stream_t stream);
 
+/* The end of a batch of inverses.  flags: device int32 [total + 1]: `count` info words, then the non-zero words of the factors
+ * (flag_index[m]: which of them belongs to record m).  out_list[m] (may be null) <- identity where that word is 0; flags[0 ...
+ * total - 1] are copied to host_flags (pinned host memory the device can write); flags[total] <- 1 if an info word of a
+ * non-zero factor is set, else 0.  out_list, dims, flag_index: device arrays of `count` entries. */
+int ak_kron_finish(float* const* out_list, const int64_t* dims, const int64_t* flag_index, int count, int* flags, int total,
+                   int* host_flags, ak_stream_t stream);
+/* Waits for an event of ak_event_create. */
+int ak_event_synchronize(void* event);
+
+/* grad_w <- s B_inv grad_w A_inv, grad_b <- s B_inv grad_b for many modules of any size in two launches (fp32 products).
+ * items (HOST memory): rows of 6 int64: B_inv, A_inv, grad_w [dB][dA], grad_b or 0 (device addresses), dB, dA;
+ * units (HOST memory): rows of 4: inv [F][2][2], grad_w [F], grad_b [F], F.  fail0 / fail1 (may be null): device words; nothing
+ * is written when one of them is not zero.  only_if_faster: AK_ERR_UNSUPPORTED, and nothing done, where ak_gemm_f32_grouped on
+ * split operands is expected to be faster. */
+size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count);
+int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, int unit_count, float grad_scale,
+                         const int* fail0, const int* fail1, int only_if_faster, void* ws, size_t ws_bytes,
+                         ak_stream_t stream);
+
 /* targets[r] = argmax_i logits[r][i] - log(q[r][i]) for q exponentially distributed: a draw of softmax(logits[r]) per row
  * (torch.multinomial's choice from the same random numbers).  Row-major [rows, classes] float32; the lowest index wins ties;
  * NaN logits are never chosen (a row of NaNs gives 0). */

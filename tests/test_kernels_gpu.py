@@ -740,6 +740,45 @@ def test_chol_inv_large_matches_fp32_oracle_and_fp64(K, d):
         assert torch.equal(out, out.T)
 
 
+@pytest.mark.parametrize('count', [1, 24, 25])
+def test_kron_precond_deep_sizes_units_and_fail_word(K, count):
+    """Sizes at, below and behind the 64-wide tiles and the 16 rows of a bias work group, more modules than one launch
+    takes, unaligned gradients; against fp64.  A fail word that is set leaves everything as it was."""
+    g = torch.Generator().manual_seed(3)
+    shapes = [(1, 1), (10, 17), (64, 64), (65, 63), (16, 129), (130, 257)]
+    scale, mods, units = 0.5, [], []
+    for i in range(count):
+        dB, dA = shapes[i % len(shapes)]
+        flat = torch.randn(dB * dA + 1, generator=g).cuda()
+        mods.append((_spd(dB, i).cuda(), _spd(dA, 50 + i).cuda(), flat[1:].view(dB, dA), torch.randn(dB, generator=g).cuda() if i % 2 else None))
+        units.append((torch.randn(5 + 256 * (i % 2), 2, 2, generator=g).cuda(), torch.randn(5 + 256 * (i % 2), generator=g).cuda(),
+                      torch.randn(5 + 256 * (i % 2), generator=g).cuda()))
+    items, unit_items = [], []
+    for B, A, w, b in mods:
+        items += (B.data_ptr(), A.data_ptr(), w.data_ptr(), 0 if b is None else b.data_ptr(), B.shape[0], A.shape[0])
+    for inv, w, b in units:
+        unit_items += (inv.data_ptr(), w.data_ptr(), b.data_ptr(), w.numel())
+    written = [t for m in mods for t in m[2:] if t is not None] + [t for u in units for t in u[1:]]
+    before = [t.clone() for t in written]
+    expected = []
+    for B, A, w, b in mods:
+        expected.append(scale * B.double() @ w.double() @ A.double())
+        if b is not None:
+            expected.append(scale * B.double() @ b.double())
+    for inv, w, b in units:
+        v = scale * torch.stack([w, b], 1).double()
+        expected += list((inv.double() @ v[:, :, None]).squeeze(2).t())
+    words = torch.tensor([0, 1], dtype=torch.int32, device='cuda')
+    dev = written[0].device
+    assert K.kron_precond_deep(items, unit_items, scale, dev, (words.data_ptr(), words.data_ptr() + 4), only_if_faster=False)
+    assert all(torch.equal(a, b) for a, b in zip(written, before))
+    assert K.kron_precond_deep(items, unit_items, scale, dev, (words.data_ptr(),), only_if_faster=False)
+    for got, want in zip(written, expected):
+        assert relerr(got, want) < 2e-6
+    big = torch.empty(1, device='cuda').data_ptr()
+    assert not K.kron_precond_deep([big, big, big, 0, 8192, 8192], [], 1.0, dev)      # the split products are faster: nothing is launched
+
+
 # ------------------------------------------------------------------ sampling
 @pytest.mark.parametrize('shape', [(1, 2), (5, 10), (64, 1000), (3, 1023), (9, 1024), (4, 1025), (2, 3, 5001)])
 def test_sample_categorical_draws_what_torch_draws(K, shape):
