@@ -214,14 +214,16 @@ __device__ __forceinline__ int leaf_eliminate(int nb, LeafShared& sh, int wave, 
       for (int r = 0; r < 4; ++r) row[r * LEAF_ROW_LD + LT * j] = acc[k][r];
       if (k + 1 == nb) break;
       __syncthreads();                                         // C_k
+      float u[LEAF_TILES][4];            // all left operands requested before the first product
+#pragma unroll
+      for (int i = k + 1; i < LEAF_TILES; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[i][r] = row[r * LEAF_ROW_LD + LT * i];
+      const floatx4 b = -acc[k];
 #pragma unroll
       for (int i = k + 1; i < LEAF_TILES; ++i) {
         if (j >= i || j <= k) {
-          float u[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) u[r] = -row[r * LEAF_ROW_LD + LT * i];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i] = mfma16(u[r], acc[k][r], acc[i]);
+          acc[i] = mfma16(u[i][1], b[1], mfma16(u[i][0], b[0], acc[i])) + mfma16(u[i][3], b[3], mfma16(u[i][2], b[2], zero));
           if (i == k + 2 && j == k + 2) {
             sh.super[lane] = acc[k + 1];
             sh.diag[lane] = acc[k + 2];

@@ -89,13 +89,13 @@ __device__ __forceinline__ void plane_bits(float x, unsigned short (&o)[3]) {
   }
 }
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
 // Epilogue of a tile: planes of C (and of C2 = c2_scale C + c2_diag I), the mirror image of an off-diagonal tile, the
-// error word max |C - I|.  sum(a, b, r): the tile's sums in the accumulator layout of the 2 x 2 waves with FR x FR blocks each.
-template <int NP, int FR, class Sum>
+// error word max |C - I|.  sum(r): a wave's sums of the 64 x 64 tile, one 32 x 32 block each.
+template <int NP, class Sum>
 __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int tj, int z, Sum sum) {
-  constexpr int FC = FR, WC = 2, TILE = 64 * FR;
-  static_assert(FR == 1 || FR == 3, "blocks are named below");
+  constexpr int WC = 2, TILE = kPlaneSmallTile;
   // (the empty statement keeps the address arithmetic below from being moved above the k-loop of the caller, where
   // every register is taken)
   int tid = threadIdx.x;
@@ -118,66 +118,243 @@ __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int t
   const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
   float vmax = 0.f;
   bool fits = true;
-  // one 32 x 32 block of the wave; the block numbers are compile-time constants (a loop the compiler does not unroll
-  // would index the accumulators with a variable, i.e. keep them in memory)
-  auto block = [&](auto a_tag, auto b_tag) {
-    constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value;
-    {
-      const int gj = j0 + 32 * FC * wc + 32 * b + l32;
+  const int gj = j0 + 32 * wc + l32;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int gi = i0 + 32 * wr + 8 * q + 4 * g;      // rows gi .. gi + 3
+    u16x4 m1[NP], m2[NP];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float v = sum(4 * q + e) * unscale;
+      const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
+      if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+      unsigned short o[3];
+      if constexpr (NP == 2) fits = fits && fabsf(v * cs) <= 65504.f;      // (false for a NaN too)
+      plane_bits<NP>(v * cs, o);
+      // a diagonal tile keeps its upper triangle and mirrors it element by element: the next product reads
+      // this matrix as its own transpose, which it has to be exactly
+      const bool keep = off_diag || gi + e <= gj;
+      const int64_t at = plane_index(gi + e, gj, p.n_pad);
+      const int64_t mirror = plane_index(gj, gi + e, p.n_pad);
+#pragma unroll
+      for (int s = 0; s < NP; ++s) {
+        if (keep) C[s * p.plane_elems + at] = o[s];
+        if (!off_diag && gi + e < gj) C[s * p.plane_elems + mirror] = o[s];
+        m1[s][e] = o[s];
+      }
+      if (C2 != nullptr) {
+        const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
+        if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
+        plane_bits<NP>(w * c2s, o);
+#pragma unroll
+        for (int s = 0; s < NP; ++s) {
+          if (keep) C2[s * p.plane_elems + at] = o[s];
+          if (!off_diag && gi + e < gj) C2[s * p.plane_elems + mirror] = o[s];
+          m2[s][e] = o[s];
+        }
+      }
+    }
+    if (off_diag) {        // C[gj][gi .. gi + 3]: four consecutive elements of a row (gi is a multiple of 4)
+      const int64_t at = plane_index(gj, gi, p.n_pad);
+#pragma unroll
+      for (int s = 0; s < NP; ++s) {
+        *reinterpret_cast<u16x4*>(C + s * p.plane_elems + at) = m1[s];
+        if (C2 != nullptr) *reinterpret_cast<u16x4*>(C2 + s * p.plane_elems + at) = m2[s];
+      }
+    }
+  }
+  if (p.errword != nullptr) gemm_store_absmax(p.errword + static_cast<int64_t>(z) * kErrStride, vmax, lane);
+  if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
+}
+
+// The same epilogue for the 192-wide tile, through the LDS, which the k-loop has left free: the tile is written there
+// transposed, [row j][4 consecutive i] as the accumulators hold it, and goes out as whole lines, 1 KB of consecutive bytes
+// per wave and store: the mirror image as it lies, the tile itself through transposing reads (ds_read_b64_tr_b16).
+// What bounds it: the burst of stores of all work groups at once.  As two-byte stores from the accumulators it took 59 us
+// of a work group's 188 at 3072 columns (two results), and a third of every product; in this form 21 us (the clock of the
+// device, which the products keep at its power limit, gives part of that back: 24 x 3072 122 -> 116 ms, 61 x 768 12.4 -> 10.5).  LDS rows of 64 bytes; their 8-byte chunks are permuted by the row (xor with row / 4), so that the 32 rows
+// a wave writes at once fall into different banks.
+template <int NP, class Sum>
+__device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, int tj, int z, AK_LDS unsigned char* lds,
+                                                    Sum sum) {
+  constexpr int FR = 3, WC = 2, TILE = kPlaneTile, BLOCK = TILE * 64, SLOT = 6 * BLOCK;      // one plane of the tile
+  static_assert(2 * SLOT <= kPlaneLdsBytes, "two planes at a time");
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));       // (keeps the address arithmetic below the k-loop of the caller)
+  asm volatile("" : "+s"(z));
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wr = wave / WC, wc = wave % WC, g = lane >> 5, l32 = lane & 31;
+  const int i0 = ti * TILE, j0 = tj * TILE;
+  const int steps = p.count[z], parity = steps & 1;
+  unsigned short* __restrict__ sets = reinterpret_cast<unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
+  float c2_diag = 0.f, c2_scale = 0.f;
+  if (p.C2.index >= 0) {
+    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
+    c2_diag = next[0];
+    c2_scale = -next[1];
+  }
+  const bool off_diag = ti != tj, plain = off_diag && j0 + TILE <= p.n;       // (ti < tj: then the rows are inside too)
+  const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
+  float vmax = 0.f;
+  bool fits = true;
+  uint32_t vmax_bits = 0;             // the largest |C| / scale seen by plain tiles, as bits (those of a NaN are the largest)
+  u16x4 upper = {0, 0, 0, 0};         // the largest magnitudes of the upper fp16 planes
+  // address of element (row, col) of a transposed tile
+  auto at = [](int row, int col) { return (col >> 5) * BLOCK + row * 64 + ((((col >> 2) & 7) ^ ((row >> 2) & 7)) << 3) + (col & 3) * 2; };
+
+  // planes s0, s0 + 1 of one result into the LDS and from there to memory
+  auto pass = [&](auto second_tag, auto s0_tag) {
+    constexpr bool SECOND = decltype(second_tag)::value;
+    constexpr int s0 = decltype(s0_tag)::value, COUNT = NP - s0 < 2 ? NP - s0 : 2;
+    __syncthreads();
+    // a tile on the diagonal or at the border of the matrix
+    auto edge_block = [&](auto a_tag, auto b_tag) {
+      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value;
+      const int lj = 32 * FR * wc + 32 * b + l32, gj = j0 + lj;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int gi = i0 + 32 * FR * wr + 32 * a + 8 * q + 4 * g;      // rows gi .. gi + 3
-        u16x4 m1[NP], m2[NP];
+        const int li = 32 * FR * wr + 32 * a + 8 * q + 4 * g, gi = i0 + li;      // rows gi .. gi + 3
+        u16x4 m[COUNT];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float v = sum(a, b, 4 * q + e) * unscale;
           const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
-          if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+          float x = v * cs;
+          if constexpr (SECOND) x = (c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f)) * c2s;
+          else if constexpr (s0 == 0)
+            if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+          if constexpr (NP == 2) fits = fits && fabsf(x) <= 65504.f;      // (false for a NaN too)
           unsigned short o[3];
-          if constexpr (NP == 2) fits = fits && fabsf(v * cs) <= 65504.f;      // (false for a NaN too)
-          plane_bits<NP>(v * cs, o);
-          // a diagonal tile keeps its upper triangle and mirrors it element by element: the next product reads
-          // this matrix as its own transpose, which it has to be exactly
-          const bool keep = off_diag || gi + e <= gj;
-          const int64_t at = plane_index(gi + e, gj, p.n_pad);
-          const int64_t mirror = plane_index(gj, gi + e, p.n_pad);
+          plane_bits<NP>(x, o);
 #pragma unroll
-          for (int s = 0; s < NP; ++s) {
-            if (keep) C[s * p.plane_elems + at] = o[s];
-            if (!off_diag && gi + e < gj) C[s * p.plane_elems + mirror] = o[s];
-            m1[s][e] = o[s];
-          }
-          if (C2 != nullptr) {
-            const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
-            if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
-            plane_bits<NP>(w * c2s, o);
+          for (int s = 0; s < COUNT; ++s) m[s][e] = o[s0 + s];
+        }
+        if (off_diag) {
 #pragma unroll
-            for (int s = 0; s < NP; ++s) {
-              if (keep) C2[s * p.plane_elems + at] = o[s];
-              if (!off_diag && gi + e < gj) C2[s * p.plane_elems + mirror] = o[s];
-              m2[s][e] = o[s];
+          for (int s = 0; s < COUNT; ++s) *reinterpret_cast<AK_LDS u16x4*>(lds + s * SLOT + at(lj, li)) = m[s];
+        } else {
+          // a diagonal tile keeps its upper triangle and mirrors it element by element: the next product reads this
+          // matrix as its own transpose, which it has to be exactly
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (li + e > lj) continue;
+#pragma unroll
+            for (int s = 0; s < COUNT; ++s) {
+              *reinterpret_cast<AK_LDS unsigned short*>(lds + s * SLOT + at(lj, li + e)) = m[s][e];
+              *reinterpret_cast<AK_LDS unsigned short*>(lds + s * SLOT + at(li + e, lj)) = m[s][e];
             }
           }
         }
-        if (off_diag) {        // C[gj][gi .. gi + 3]: four consecutive elements of a row (gi is a multiple of 4)
-          const int64_t at = plane_index(gj, gi, p.n_pad);
+        __builtin_amdgcn_sched_barrier(0);         // (values of other blocks split ahead would not fit the registers)
+      }
+    };
+    // Every other tile needs no test per element.  The scales are powers of two but for c2_scale, whose product with them
+    // is exact: one rounding, as above.  Two fp16 planes overflow where the upper one is infinite or a NaN.
+    const float scale = SECOND ? c2_scale * (unscale * c2s) : unscale * cs;
+    auto block = [&](auto a_tag, auto b_tag) {
+#pragma clang fp contract(off)             // (x rounds before its planes are taken, as in the other tiles: the same bits)
+      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value;
+      const int lj = 32 * FR * wc + 32 * b + l32;
 #pragma unroll
-          for (int s = 0; s < NP; ++s) {
-            *reinterpret_cast<u16x4*>(C + s * p.plane_elems + at) = m1[s];
-            if (C2 != nullptr) *reinterpret_cast<u16x4*>(C2 + s * p.plane_elems + at) = m2[s];
+      for (int q = 0; q < 4; ++q) {
+        const int li = 32 * FR * wr + 32 * a + 8 * q + 4 * g;
+        u16x4 m[COUNT];
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = sum(a, b, 4 * q + e) * scale;
+        if constexpr (!SECOND && s0 == 0) {
+          if (p.errword != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vmax_bits = max(vmax_bits, __builtin_bit_cast(uint32_t, x[e]) & 0x7fffffffu);
           }
         }
+        if constexpr (NP == 2) {
+          typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+          typedef float f32x4 __attribute__((ext_vector_type(4)));
+          const f32x4 xv = {x[0], x[1], x[2], x[3]};
+          const f16x4 hi = __builtin_convertvector(xv, f16x4);
+          const f16x4 lo = __builtin_convertvector(xv - __builtin_convertvector(hi, f32x4), f16x4);
+          m[0] = __builtin_bit_cast(u16x4, hi);
+          m[1] = __builtin_bit_cast(u16x4, lo);
+          upper = __builtin_elementwise_max(upper, m[0] & (unsigned short)0x7fff);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            unsigned short o[3];
+            plane_bits<NP>(x[e], o);
+#pragma unroll
+            for (int s = 0; s < COUNT; ++s) m[s][e] = o[s0 + s];
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < COUNT; ++s) *reinterpret_cast<AK_LDS u16x4*>(lds + s * SLOT + at(lj, li)) = m[s];
+        __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    auto blocks = [](auto&& f) {
+      using J0 = std::integral_constant<int, 0>;
+      using J1 = std::integral_constant<int, 1>;
+      using J2 = std::integral_constant<int, 2>;
+      f(J0{}, J0{}); f(J0{}, J1{}); f(J0{}, J2{});
+      f(J1{}, J0{}); f(J1{}, J1{}); f(J1{}, J2{});
+      f(J2{}, J0{}); f(J2{}, J1{}); f(J2{}, J2{});
+    };
+    if (plain) blocks(block);
+    else blocks(edge_block);
+    __syncthreads();
+    unsigned short* __restrict__ out = sets + paired_buf(SECOND ? p.C2 : p.C, parity) * p.buf_elems + s0 * p.plane_elems;
+    // A wave takes rows 16 (wave + 4 t), t < 3, of every block of 32 columns; all its LDS addresses and all its memory
+    // addresses differ by constants of the wave.
+    {   // rows gj, columns gi: lane = row l / 4 of 16, 16 bytes l % 4
+      const int row = 16 * wave + (lane >> 2), col = 8 * (lane & 3);
+      AK_LDS const unsigned char* lo = lds + at(row, col);
+      AK_LDS const unsigned char* hi = lds + at(row, col + 4);
+      const uint32_t lane_off = (lane >> 2) * 32 + col;
+#pragma unroll
+      for (int s = 0; s < COUNT; ++s)
+#pragma unroll 2
+        for (int blk = 0; blk < 6; ++blk) {
+          unsigned short* dst = out + s * p.plane_elems + plane_index(j0 + 16 * wave, i0 + 32 * blk, p.n_pad);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const u16x4 x = *reinterpret_cast<AK_LDS const u16x4*>(lo + s * SLOT + blk * BLOCK + t * 4096);
+            const u16x4 y = *reinterpret_cast<AK_LDS const u16x4*>(hi + s * SLOT + blk * BLOCK + t * 4096);
+            *reinterpret_cast<u16x8*>(dst + t * 2048 + lane_off) = u16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+          }
+        }
+    }
+    if (off_diag) {
+      // rows gi, columns gj: lane (t4, j16) takes row j16 of 16 and columns 8 t4 .. 8 t4 + 7 of a block, two transposing reads
+      const int t4 = lane >> 4, j16 = lane & 15, c = 16 * wave + 4 * (j16 & 3);
+      AK_LDS const unsigned char* lo = lds + at(8 * t4 + (j16 >> 2), c);
+      AK_LDS const unsigned char* hi = lds + at(8 * t4 + 4 + (j16 >> 2), c);
+      const uint32_t lane_off = j16 * 32 + 8 * t4;
+#pragma unroll
+      for (int s = 0; s < COUNT; ++s)
+#pragma unroll 2
+        for (int blk = 0; blk < 6; ++blk) {
+          unsigned short* dst = out + s * p.plane_elems + plane_index(i0 + 16 * wave, j0 + 32 * blk, p.n_pad);
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const int off = s * SLOT + blk * 2048 + t * 2 * BLOCK;
+            const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(lo + off));
+            const short4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(hi + off));
+            *reinterpret_cast<short8v*>(dst + t * 2048 + lane_off) = short8v{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+          }
+        }
     }
   };
-  using J0 = std::integral_constant<int, 0>;
-  using J1 = std::integral_constant<int, 1>;
-  using J2 = std::integral_constant<int, 2>;
-  block(J0{}, J0{});
-  if constexpr (FR == 3) {
-    block(J0{}, J1{}); block(J0{}, J2{});
-    block(J1{}, J0{}); block(J1{}, J1{}); block(J1{}, J2{});
-    block(J2{}, J0{}); block(J2{}, J1{}); block(J2{}, J2{});
+  using S0 = std::integral_constant<int, 0>;
+  using S2 = std::integral_constant<int, 2>;
+  pass(std::false_type{}, S0{});
+  if constexpr (NP == 3) pass(std::false_type{}, S2{});
+  if (p.C2.index >= 0) {
+    pass(std::true_type{}, S0{});
+    if constexpr (NP == 3) pass(std::true_type{}, S2{});
+  }
+  if (plain) {
+    vmax = __builtin_bit_cast(float, vmax_bits) * (1.f / cs);             // (a power of two)
+    fits = NP != 2 || max(max(upper[0], upper[1]), max(upper[2], upper[3])) < 0x7c00;
   }
   if (p.errword != nullptr) gemm_store_absmax(p.errword + static_cast<int64_t>(z) * kErrStride, vmax, lane);
   if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
@@ -345,7 +522,7 @@ __device__ __forceinline__ void plane_tile(const PlaneGemm& p, int ti, int tj, i
   }
   wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
 
-  plane_epilogue<3, 3>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue_wide<3>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
 // The same tile on two fp16 planes per operand.  A k-tile is 16 rows of four plane panels (24 KB per stage, six
@@ -491,7 +668,7 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
         for (int r = 0; r < 16; ++r) tot[a][b][r] += acc[a][b][r];
   }
   wait_vmcnt<0>();
-  plane_epilogue<2, 3>(p, ti, tj, z, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue_wide<2>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
 // A 64 x 64 tile (ti <= tj) for groups with too few 192-wide tiles to fill the device: 4 waves (2 x 2) of one 32 x 32 block.
@@ -581,7 +758,7 @@ __device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int
     }
   }
   wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
-  plane_epilogue<NP, 1>(p, ti, tj, z, [&](int, int, int r) { return tot[r]; });
+  plane_epilogue<NP>(p, ti, tj, z, [&](int r) { return tot[r]; });
 }
 
 // Tile number -> (ti <= tj), in bands of 8 tile columns, row by row inside a band: the 32 work groups that share an
