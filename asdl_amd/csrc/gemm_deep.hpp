@@ -169,7 +169,10 @@ __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int 
       for (int r = 0; r < 16; ++r) acc[r] = p.alpha * acc[r] + p.beta * old[r];
     } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] *= p.alpha;
+      for (int r = 0; r < 16; ++r) {
+        acc[r] *= p.alpha;
+        if (gi0 + 8 * (r >> 2) + (r & 3) == gj) acc[r] += p.diag;
+      }
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {

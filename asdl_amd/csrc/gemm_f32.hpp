@@ -48,6 +48,7 @@ struct GemmParams {
   float* C2 = nullptr;                // optional second result, same shape and batch layout as C with its own strides:
   int64_t ldc2 = 0, sC2 = 0;          // C2 = c2_scale * C + c2_diag * I (the next iterate's polynomial of a Newton iteration,
   float c2_scale = 0.f, c2_diag = 0.f;   // written while C is still in registers)
+  float diag = 0.f;                   // deep tiles only, beta == 0: C = alpha op(A) op(B) + diag I
 };
 
 constexpr int GBT = 128, GBK = 16;     // GBT: granularity of the triangular contraction ranges (both tile sizes)

@@ -1170,6 +1170,41 @@ def smw_inv(x, lam, out=None, info=None):
     return z, info
 
 
+SMW_GROUP_MAX_ROWS = 512      # more rows: the products fill the device one factor at a time
+
+
+def smw_groupable(x):
+    return x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] <= SMW_GROUP_MAX_ROWS and x.shape[1] <= 65536
+
+
+def smw_inv_grouped(xs, lam_addresses, outs, info):
+    """smw_inv for many row matrices (each smw_groupable): one grouped inverse of all Gram matrices between four grouped
+    launches.  lam_addresses: of one float each; info: int32 device tensor with one word per matrix."""
+    _require_gpu(*xs, *outs, info)
+    lib = _lib.load()
+    dev = xs[0].device
+    sizes = [(x.shape[0], x.shape[1], _ws_need('ak_smw_group_y_floats', x.shape[0], x.shape[1])) for x in xs]
+    grams, invs, items, off = [], [], [], (len(xs) + 63) // 64 * 64
+    total = off + sum(2 * ((n * n + 63) // 64 * 64) + (y + 63) // 64 * 64 for n, _, y in sizes)
+    # (not the stream's workspace: the inverse in the middle uses that)
+    flat = torch.empty(total, dtype=torch.float32, device=dev)
+    base = flat.data_ptr()
+    for i, (x, out, lam, (n, d, y)) in enumerate(zip(xs, outs, lam_addresses, sizes)):
+        if out.dtype != torch.float32 or out.shape != (d, d) or not out.is_contiguous():
+            raise ValueError('every output has to be a contiguous float32 [d, d] tensor')
+        square = (n * n + 63) // 64 * 64
+        grams.append(flat[off:off + n * n].view(n, n))
+        invs.append(flat[off + square:off + square + n * n].view(n, n))
+        items += (x.data_ptr(), base + 4 * off, base + 4 * (off + square), base + 4 * (off + 2 * square), out.data_ptr(), lam,
+                  base + 4 * i, n, d)
+        off += 2 * square + (y + 63) // 64 * 64
+    table = (ctypes.c_int64 * len(items))(*items)
+    _lib.check(lib.ak_smw_group(table, len(xs), 0, _stream(dev)), 'ak_smw_group')
+    chol_inv_grouped(grams, invs, flat[:len(xs)], info=info)
+    _lib.check(lib.ak_smw_group(table, len(xs), 1, _stream(dev)), 'ak_smw_group')
+    return flat         # to be kept until the launches have run, where they are not on the stream that owns it
+
+
 def chol_inv_batched(mats, outs, lam, lam_stride=1, active=None, active_stride=1, info=None):
     """outs[b] <- (mats[b] + lam[b*lam_stride] I)^-1 for same-size matrices; returns the device
     ``info`` tensor (int32 [batch], 0 = ok, k > 0 = leading minor k not positive definite)."""

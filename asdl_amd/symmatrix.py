@@ -276,15 +276,18 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
         for e in square:
             by_size[e[1].shape[0]].append(e)
         groups = list(by_size.values())
-    groups += [[e] for e in low_rank]
-    prepared, records, fresh = [], [], []       # fresh: this record's output buffer held no inverse before
+    together = [e for e in low_rank if mats_on_gpu and kernels.smw_groupable(e[1])]
+    groups += ([together] if together else []) + [[e] for e in low_rank if not any(e is t for t in together)]
+    prepared, records, fresh, scratch = [], [], [], []       # fresh: this record's output buffer held no inverse before
     for entries in groups:
         outs = [output(mat, k, which, mat.shape[1]) for _, mat, k, which in entries]
         info = infos[len(records):len(records) + len(entries)]
         records.extend((flat, k, which, out) for (flat, _, k, which), out in zip(entries, outs))
         index = tuple(e[0] for e in entries)
         low = entries[0][1].shape[0] != entries[0][1].shape[1]
-        if index == tuple(range(index[0], index[0] + len(index))):
+        if low and entries is together:
+            lam_g = act_g = None          # (each factor's value is read where it lies)
+        elif index == tuple(range(index[0], index[0] + len(index))):
             lam_g, act_g = lam_flat[index[0]:index[0] + len(index)], nz_flat[index[0]:index[0] + len(index)]
         else:
             idx = kernels.device_ints(index, dev)
@@ -296,9 +299,13 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
     def run_group(group):
         entries, outs, lam_g, act_g, info = group
         with nvtx_range(range_name):
-            if act_g is None:          # a low-rank factor
+            if act_g is None:          # low-rank factors
                 # (x^T x / n + lam I)^-1 by Sherman-Morrison-Woodbury (smw_inv, asdl/utils.py:107-115)
-                kernels.smw_inv(entries[0][1], lam_g, out=outs[0], info=info)
+                if mats_on_gpu and kernels.smw_groupable(entries[0][1]):
+                    base = lam_flat.data_ptr()
+                    scratch.append(kernels.smw_inv_grouped([e[1] for e in entries], [base + 4 * e[0] for e in entries], outs, info))
+                else:
+                    kernels.smw_inv(entries[0][1], lam_g, out=outs[0], info=info)
             elif GROUPED_INVERSE:
                 kernels.chol_inv_grouped([e[1] for e in entries], outs, lam_g, 1, active=act_g, active_stride=1,
                                          info=info)
@@ -307,11 +314,14 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
                                          info=info)
 
     side = []
-    if beside and defer and mats_on_gpu and GROUPED_INVERSE and square and not low_rank:
-        # A few launches that leave most of the device idle: the two changes of stream cost the host more than running
-        # beside them saves the device.
-        beside = kernels.chol_group_plan([e[1].shape[0] for e in square], dev).microseconds > INLINE_MICROSECONDS
-    if mats_on_gpu and (len(prepared) > 1 or (defer and beside)):
+    inline = not (beside and defer)
+    if mats_on_gpu and GROUPED_INVERSE and len(together) == len(low_rank) and not inline:
+        # A few launches that leave most of the device idle: the changes of stream cost the host more than running beside
+        # them saves the device.  (Low-rank factors: the Gram matrices' chain, then d^2 floats each at 3 TB/s.)
+        us = kernels.chol_group_plan([e[1].shape[0] for e in square], dev).microseconds if square else 0
+        us += 150 + sum(e[1].shape[1] ** 2 for e in together) / 750e3 if together else 0
+        inline = us < INLINE_MICROSECONDS
+    if mats_on_gpu and prepared and not (inline and len(prepared) <= 1 + bool(together)):
         # Successive calls start on different side streams (each with its own workspace), so that an early batch and
         # the remainder of one step run side by side.  The launches are issued from here: handing them to another
         # thread cost more in interpreter-lock changes (0.6 ms of a small step) than the launches themselves.
@@ -329,7 +339,7 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
         for group in prepared:
             run_group(group)
     pending = PendingInverses(records, flags, nz_flat, side, replace,
-                              keep_alive=(prepared, lam, A_list, B_list), fresh=fresh)
+                              keep_alive=(prepared, lam, A_list, B_list, scratch), fresh=fresh)
     if defer:
         return pending
     pending.finish()

@@ -150,6 +150,13 @@ int ak_conv_patch_sum(const void* x, int dtype, int64_t sn, int64_t sc, int64_t 
 int ak_identity_where_zero(float* const* out_list, const int64_t* dims, const int* nonzero,
                            const int64_t* flag_index, int count, ak_stream_t stream);
 
+/* (x^T x / n + lam I)^-1 for many [n, d] row matrices, around a grouped inverse of their Gram matrices by the caller.
+ * items (HOST memory): rows of 9 int64: x, gram [n][n], gram_inv [n][n], y (ak_smw_group_y_floats), out [d][d], lam, lam_n (device
+ * addresses of floats), n, d.  phase 0: gram <- x x^T, lam_n <- n lam; phase 1: out <- (I - x^T gram_inv x) / lam, where gram_inv
+ * is (gram + lam_n I)^-1. */
+size_t ak_smw_group_y_floats(int64_t n, int64_t d);
+int ak_smw_group(const int64_t* items, int count, int phase, ak_stream_t stream);
+
 /* The end of a batch of inverses.  flags: device int32 [total + 1]: `count` info words, then the non-zero words of the factors
  * (flag_index[m]: which of them belongs to record m).  out_list[m] (may be null) <- identity where that word is 0; flags[0 ...
  * total - 1] are copied to host_flags (pinned host memory the device can write); flags[total] <- 1 if an info word of a

@@ -779,6 +779,23 @@ def test_kron_precond_deep_sizes_units_and_fail_word(K, count):
     assert not K.kron_precond_deep([big, big, big, 0, 8192, 8192], [], 1.0, dev)      # the split products are faster: nothing is launched
 
 
+@pytest.mark.parametrize('shapes', [[(1, 2)], [(64, 65), (63, 577), (8, 27)], [(65, 512), (128, 513), (129, 1200)], [(16, 40 + i) for i in range(25)]])
+def test_smw_inv_grouped_matches_fp64(K, shapes):
+    """Tile edges of the Gram matrices and of the results, slices of the long side, more factors than one launch takes."""
+    g = torch.Generator().manual_seed(11)
+    xs = [torch.randn(n, d, generator=g).cuda() for n, d in shapes]
+    lam = torch.rand(len(xs), generator=g).cuda() * 0.2 + 0.05
+    outs = [torch.full((d, d), 7.0, device='cuda') for _, d in shapes]
+    info = torch.full((len(xs),), -1, dtype=torch.int32, device='cuda')
+    K.smw_inv_grouped(xs, [lam.data_ptr() + 4 * i for i in range(len(xs))], outs, info)
+    assert torch.all(info == 0)
+    for x, l, out in zip(xs, lam.double(), outs):
+        n, d = x.shape
+        ref = torch.linalg.inv(x.double().t() @ x.double() / n + l * torch.eye(d, device='cuda', dtype=torch.float64))
+        assert relerr(out, ref) < 1e-5, ((n, d), relerr(out, ref))
+        assert torch.equal(out, out.t())
+
+
 # ------------------------------------------------------------------ sampling
 @pytest.mark.parametrize('shape', [(1, 2), (5, 10), (64, 1000), (3, 1023), (9, 1024), (4, 1025), (2, 3, 5001)])
 def test_sample_categorical_draws_what_torch_draws(K, shape):
