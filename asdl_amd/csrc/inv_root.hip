@@ -18,13 +18,16 @@
 // The first kRootEarly steps stay classical, in the summation order of one fixed kernel per size.  What an ill-conditioned
 // root ends up with is decided there: the rounding of M' perturbs the smallest eigenvalues by about 5e-8, 1 to 2 % of the
 // root at condition 1e6, and every later step's perturbation counts 2.44 times less.  Another order, though as accurate, gives
-// another root within that percent; with the first three steps alike two computations agree to 0.2 %.
+// another root within that percent; rank-deficient statistics of 625 to 1498 columns differ from the root of the wholly
+// classical iteration by 0.6 to 0.9 % after three classical steps, by 0.12 to 0.17 % after five (a fourteenth step; 24 x 3072:
+// 112 -> 121 ms).
 //
-// The matrices of the iteration, all polynomials of one symmetric matrix, so that only tiles on one side of the diagonal
-// are computed and mirrored, are kept
-//  * as 16-bit planes from 512 columns up (gemm_planes.hpp): 192 x 192 tiles, one launch per product and group, where a group
+// The matrices of the iteration, all polynomials of one symmetric matrix, are kept
+//  * as 16-bit planes from 512 columns up (gemm_planes.hpp), of which only tiles on one side of the diagonal are computed,
+//    and mirrored: 192 x 192 tiles, one launch per product and group, where a group
 //    has enough of them to fill the device, else 64 x 64 tiles;
-//  * in fp32 below: 32 x 32 tiles whose four waves split the contraction, or 64 x 64 tiles (gemm_deep.hpp).
+//  * in fp32 below, every tile of a product computed: with mirrored tiles the part of the rounding that is not symmetric
+//    goes elsewhere, and the root of a rank-deficient statistic moves by most of its own error (1 % at 255 columns).
 // The small tiles of all groups of a kind share one launch per step of the product sequence.
 // All sum in chunks; the product that forms the next M also folds max |M - I| into a device word and writes the next
 // step's polynomial T.  X, M and T alternate between two buffers by the parity of the matrix's own step count: nothing is
@@ -41,7 +44,7 @@ constexpr int RCHUNKS = 64;             // partial-reduction chunks per matrix
 constexpr int kRootMaxGroups = 16;      // groups of one call (they travel in the kernel arguments)
 constexpr int kLanczosSteps = 32;
 constexpr int kLanczosRows = 16;        // rows of the statistic per work group and step: four waves, four rows each
-constexpr int kRootEarly = 3;           // classical steps before the accelerated ones
+constexpr int kRootEarly = 5;           // classical steps before the accelerated ones
 constexpr int kRootSteps = 32;          // entries of a matrix's step table; the last one repeats
 constexpr int kRootBuffers = 10;        // R0 R1 M0 M1 T0 T1 and four product buffers
 constexpr int kRootMinPlaneDim = 512;
@@ -636,15 +639,14 @@ static __global__ void root_stats_kernel(RootGroups G) {
 
 // ---- products on small tiles ----------------------------------------------------------------------------------------------
 
-enum RootKind { kFp32Tile32 = 0, kFp32Tile64 = 1, kPlanes2 = 2, kPlanes3 = 3, kFp32Early = 4 };
-enum RootWhen { kAlways = 0, kEarlySteps = 1, kLateSteps = 2 };     // (of each matrix's own count: a caller in parts does not say)
+enum RootKind { kFp32 = 0, kPlanes2 = 2, kPlanes3 = 3 };
 struct RootJob {
   float* bufs;                  // of its group
   int64_t buf_elems, mat_elems; // floats (planes: 16-bit elements) between buffers, between matrices
   PairedBuf a, b, c, c2;        // C = A B; c2.index >= 0: the product that forms M', which also writes the next T and the error
   int n, ld;                    // ld: padded size on planes
-  int z0, tiles;                // first matrix; tiles of one matrix: those on one side of the diagonal, all for the early steps
-  int kind, when;
+  int z0, tiles;                // first matrix; tiles of one matrix: on planes those on one side of the diagonal
+  int kind;
   float scale_r;
 };
 constexpr int kRootMaxJobs = 2 * kRootMaxGroups;
@@ -653,11 +655,9 @@ struct RootJobs {
   RootJob j[kRootMaxJobs];
 };
 
-constexpr int kRootKC = 256;        // columns of a chunk of the 32 x 32 tile, 64 per wave
-
-// One 64 x 64 tile (ti, tj) of C = A B for the early steps: every tile of the product (nothing is mirrored), k pairs
+// One 64 x 64 tile (ti, tj) of C = A B of fp32 matrices: every tile of the product (nothing is mirrored), k pairs
 // (16 t + m, 16 t + 8 + m) in order on one accumulator, chunks of 128 k.  lds: deep_lds_floats<64, 64, 128>() floats.
-__device__ __forceinline__ void root_tile_early(const GemmParams& p, int ti, int tj, float* lds) {
+__device__ __forceinline__ void root_tile_fp32(const GemmParams& p, int ti, int tj, float* lds) {
   using P = DeepPanel<64, 128>;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
   const int wr = wave >> 1, wc = wave & 1, i0 = 64 * ti, j0 = 64 * tj, ld = static_cast<int>(p.lda);
@@ -710,95 +710,6 @@ __device__ __forceinline__ void root_tile_early(const GemmParams& p, int ti, int
   if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out, vmax, lane);
 }
 
-// One 32 x 32 tile (ti >= tj) of C = A B for symmetric matrices stored as n rows of ld: rows of A times rows of B, the
-// contraction of every chunk split over the four waves, which are added up through the LDS at the end.  Four times the
-// tiles of the 64-wide form and a quarter of its matrix instructions per wave: n = 784 takes 325 work groups of 6 us
-// instead of 91 of 15.
-__device__ __forceinline__ void root_tile32(const GemmParams& p, int ti, int tj, float* lds) {
-  using P = DeepPanel<32, kRootKC>;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
-  const int i0 = 32 * ti, j0 = 32 * tj, ld = static_cast<int>(p.lda);
-  float* ldsA = lds;
-  float* ldsB = lds + 32 * P::KC_LD;
-  const float* pa = ldsA + l32 * P::KC_LD + 64 * wave + 4 * g;
-  const float* pb = ldsB + l32 * P::KC_LD + 64 * wave + 4 * g;
-  floatx16 acc, part[2];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = part[0][r] = part[1][r] = 0.f;
-  typename P::Regs ra, rb;
-  deep_fetch<32, kRootKC>(ra, p.A, ld, true, i0, p.M, 0, ld, tid);         // (the padding columns are zero)
-  deep_fetch<32, kRootKC>(rb, p.B, ld, true, j0, p.M, 0, ld, tid);
-  for (int k0 = 0; k0 < ld; k0 += kRootKC) {
-    if (k0 != 0) __syncthreads();
-    deep_stash<32, kRootKC>(ra, ldsA, true, tid);
-    deep_stash<32, kRootKC>(rb, ldsB, true, tid);
-    __syncthreads();
-    if (k0 + kRootKC < ld) {
-      deep_fetch<32, kRootKC>(ra, p.A, ld, true, i0, p.M, k0 + kRootKC, ld, tid);
-      deep_fetch<32, kRootKC>(rb, p.B, ld, true, j0, p.M, k0 + kRootKC, ld, tid);
-    }
-    if (k0 + 64 * wave < ld) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const floatx4 a = *reinterpret_cast<const floatx4*>(pa + 8 * q), b = *reinterpret_cast<const floatx4*>(pb + 8 * q);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) part[e & 1] = mfma_f32(a[e], b[e], part[e & 1]);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        acc[r] += part[0][r] + part[1][r];
-        part[0][r] = part[1][r] = 0.f;
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 16; ++r) lds[(16 * wave + r) * 64 + lane] = acc[r];
-  __syncthreads();
-  // wave w adds up registers 4 w ... 4 w + 3: rows 8 w + 4 g + e, column l32
-  floatx4 v;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float* q = lds + (4 * wave + e) * 64 + lane;
-    v[e] = (q[0] + q[16 * 64]) + (q[32 * 64] + q[48 * 64]);
-  }
-  // exactly symmetric: a tile on the diagonal keeps its lower triangle and mirrors it element by element (the next product
-  // reads this matrix as its own transpose; what is not symmetric grows from step to step)
-  const int gi = i0 + 8 * wave + 4 * g, gj = j0 + l32;
-  float vmax = 0.f;
-  if (gj < p.M) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (gi + e >= p.M || gi + e < gj) continue;
-      p.C[static_cast<int64_t>(gi + e) * ld + gj] = v[e];
-      vmax = gemm_fold_absmax(vmax, v[e], gi + e == gj, 1);
-      if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi + e) * ld + gj] = p.c2_scale * v[e] + (gi + e == gj ? p.c2_diag : 0.f);
-    }
-    float* dst = p.C + static_cast<int64_t>(gj) * ld + gi;
-    float* dst2 = p.C2 != nullptr ? p.C2 + static_cast<int64_t>(gj) * ld + gi : nullptr;
-    floatx4 w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (gi + e >= p.M) v[e] = 0.f;              // a mirrored row ends in the padding columns, which stay zero
-      w[e] = p.c2_scale * v[e];
-    }
-    if (ti != tj) {
-      if (gi < p.M) {
-        *reinterpret_cast<floatx4*>(dst) = v;
-        if (dst2 != nullptr) *reinterpret_cast<floatx4*>(dst2) = w;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (gi + e <= gj || gi + e >= p.M) continue;
-        dst[e] = v[e];
-        if (dst2 != nullptr) dst2[e] = w[e];
-      }
-    }
-  }
-  if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out, vmax, lane);
-}
-
 // A product on planes (fp16 planes: the two roots carry scale_r, every other matrix kRootScaleM).
 __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0, int np, int n, int n_pad, int tile, float scale_r,
                                                      float* bufs, int64_t buf_elems, PairedBuf a, PairedBuf b, PairedBuf c,
@@ -824,8 +735,7 @@ __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0
 }
 
 __device__ __forceinline__ bool root_idle(const RootState& st, const RootJob& job, int z, int steps) {
-  return st.active[z] == 0 || (steps == 0 && job.c.index == 0) ||          // (the first X is written by the start)
-         (job.when == kEarlySteps && steps >= kRootEarly) || (job.when == kLateSteps && steps < kRootEarly);
+  return st.active[z] == 0 || (steps == 0 && job.c.index == 0);            // (the first X is written by the start)
 }
 
 // The product of matrix zl of a group in fp32; c2_*: of the step `steps` is followed by.
@@ -840,7 +750,7 @@ __device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, con
   p.M = p.N = job.n;
   p.K = job.ld;
   p.transB = 1;                 // (a symmetric operand is its own transpose)
-  p.tile_mode = TILE_LOWER_MIRROR;
+  p.tile_mode = TILE_ALL;
   if (job.c2.index >= 0) {
     const float* next = st.coef + z * 2 * kRootSteps + 2 * min(steps + 1, kRootSteps - 1);
     p.C2 = base + paired_buf(job.c2, parity) * job.buf_elems;
@@ -853,7 +763,7 @@ __device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, con
   return p;
 }
 
-// Early products of a group in fp32 with many wide matrices: 128 x 128 tiles of the three-piece split (gemm_x3.hpp).
+// Products of a group in fp32 with many wide matrices: 128 x 128 tiles of the three-piece split (gemm_x3.hpp).
 static __global__ __launch_bounds__(256) void root_split_kernel(RootState st, RootJob job) {
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 2 * 3 * X3_PLANE];
   const int zl = static_cast<int>(blockIdx.x) / job.tiles, z = job.z0 + zl, local = static_cast<int>(blockIdx.x) - zl * job.tiles;
@@ -862,7 +772,6 @@ static __global__ __launch_bounds__(256) void root_split_kernel(RootState st, Ro
   GemmParams p = root_fp32_product(st, job, zl, z, steps);
   p.K = job.n;
   p.transB = 0;
-  p.tile_mode = TILE_ALL;
   gemm_x3_tile<3, true, 1, 0, false, true>(p, local / T, local % T, 0, (AK_LDS3 unsigned char*)x3_smem);
 }
 
@@ -880,23 +789,17 @@ static __global__ __launch_bounds__(256, 2) void root_small_kernel(RootState st,
   const int steps = st.count[z];
   if (root_idle(st, job, z, steps)) return;
   float* lds = reinterpret_cast<float*>(dtl_smem);
-  if (job.kind == kFp32Early) {
+  if (job.kind == kFp32) {
     const int T = (job.n + 63) / 64;
-    root_tile_early(root_fp32_product(st, job, zl, z, steps), local / T, local % T, lds);
+    root_tile_fp32(root_fp32_product(st, job, zl, z, steps), local / T, local % T, lds);
     return;
   }
   int ti, tj;
   decode_lower_tile(local, ti, tj);
-  if (job.kind == kPlanes2 || job.kind == kPlanes3) {
-    const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
-                                         job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
-    if (job.kind == kPlanes2) plane_tile_small<2>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
-    else plane_tile_small<3>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
-    return;
-  }
-  const GemmParams p = root_fp32_product(st, job, zl, z, steps);
-  if (job.kind == kFp32Tile32) root_tile32(p, ti, tj, lds);
-  else gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
+  const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
+                                       job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
+  if (job.kind == kPlanes2) plane_tile_small<2>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
+  else plane_tile_small<3>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------------
@@ -969,10 +872,10 @@ static size_t root_active_offset(const int64_t* n, const int* batch, int groups)
   return off * sizeof(float);
 }
 
-// phases: 1 = power iteration, ridge and start of the Newton iteration; 2 = `iters` Newton iterations, the first of which
-// is number `begin` of the computation (-1: not known); 4 = results and statistics
-static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge_eps, int max_power_iter, float power_tol,
-                    int max_iter, float tol, hipStream_t s) {
+// phases: 1 = power iteration, ridge and start of the Newton iteration; 2 = `iters` Newton iterations; 4 = results and
+// statistics
+static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int max_power_iter, float power_tol, int max_iter,
+                    float tol, hipStream_t s) {
   const int total = G.total;
   const dim3 gz(total), gc(RCHUNKS, total), b256(256), b64(64);
   if (phases & 1) {
@@ -1019,16 +922,7 @@ static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge
       if (nslots[i] < 0) return AK_ERR_ARG;
       most = std::max(most, nslots[i]);
     }
-    // 32-wide fp32 tiles while a launch's run side by side: four times the tiles of the 64-wide form, each a third as long
-    int64_t small_tiles = 0;
-    for (int i = 0; i < G.count; ++i)
-      if (G.g[i].np == 0) {
-        const int64_t t = (G.g[i].n + 31) / 32;
-        small_tiles += t * (t + 1) / 2 * G.g[i].batch;
-      }
-    const int fp32_tile = small_tiles <= 512 ? 32 : 64;
-    constexpr int kLds[5] = {2 * 32 * DeepPanel<32, kRootKC>::KC_LD * 4, deep_lds_floats<64, 64, 128>() * 4, 4 * 8 * 4096,
-                             3 * 12 * 4096, deep_lds_floats<64, 64, 128>() * 4};    // by kind (planes: their stages)
+    constexpr int kLds[4] = {deep_lds_floats<64, 64, 128>() * 4, 0, 4 * 8 * 4096, 3 * 12 * 4096};    // by kind (planes: their stages)
     static bool attr_set = false;     // idempotent; a race sets it twice at worst
     if (!attr_set) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_small_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1037,7 +931,6 @@ static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge
       attr_set = true;
     }
     for (int it = 0; it < iters; ++it) {
-      const bool early = begin < 0 || begin + it < kRootEarly, late = begin < 0 || begin + it >= kRootEarly;
       for (int k = 0; k < most; ++k) {
         RootJobs J;
         int jobs = 0, blocks = 0, lds = 0;
@@ -1059,8 +952,8 @@ static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge
             job.n = g.n; job.ld = g.np == 0 ? g.ld : g.n_pad;
             job.z0 = g.z0;
             job.scale_r = g.scale_r;
-            auto put = [&](int kind, int when, int tiles) {
-              job.kind = kind; job.when = when; job.tiles = tiles;
+            auto put = [&](int kind, int tiles) {
+              job.kind = kind; job.tiles = tiles;
               J.first[jobs] = blocks;
               J.j[jobs++] = job;
               blocks += tiles * g.batch;
@@ -1068,21 +961,15 @@ static int root_run(int phases, int begin, int iters, RootGroups& G, float ridge
             };
             if (g.np != 0) {
               const int t = g.n_pad / kPlaneSmallTile;
-              put(g.np, kAlways, t * (t + 1) / 2);
+              put(g.np, t * (t + 1) / 2);
               continue;
             }
-            if (early) {
-              const int t128 = (g.n + 127) / 128, t64 = (g.n + 63) / 64;
-              if (t128 * t128 * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0) {
-                job.kind = kFp32Early; job.when = kEarlySteps; job.tiles = t128 * t128;
-                hipLaunchKernelGGL(root_split_kernel, dim3(job.tiles * g.batch), b256, 0, s, G.st, job);
-              } else {
-                put(kFp32Early, kEarlySteps, t64 * t64);
-              }
-            }
-            if (late) {
-              const int t = (g.n + fp32_tile - 1) / fp32_tile;
-              put(fp32_tile == 32 ? kFp32Tile32 : kFp32Tile64, kLateSteps, t * (t + 1) / 2);
+            const int t128 = (g.n + 127) / 128, t64 = (g.n + 63) / 64;
+            if (t128 * t128 * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0) {
+              job.kind = kFp32; job.tiles = t128 * t128;
+              hipLaunchKernelGGL(root_split_kernel, dim3(job.tiles * g.batch), b256, 0, s, G.st, job);
+            } else {
+              put(kFp32, t64 * t64);
             }
           }
         }
@@ -1113,13 +1000,13 @@ extern "C" size_t ak_inv_root_group_active_offset(const int64_t* n, const int* b
   return ak::root_args_ok(n, batch, groups) ? ak::root_active_offset(n, batch, groups) : 0;
 }
 
-extern "C" int ak_inv_root_group(int phases, int begin, int iters, int groups, float* const* S, const int64_t* n,
+extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const* S, const int64_t* n,
                                  const int* batch, const int64_t* strideS, const int* p, float ridge_eps,
                                  const float* const* v0, int max_power_iter, float power_tol, int max_iter, float tol,
                                  float* const* out, const int64_t* strideOut, float* const* stats, void* ws,
                                  size_t ws_bytes, ak_stream_t stream) {
   using namespace ak;
-  if (phases < 1 || phases > 7 || (begin < 0 && groups != 1) || iters < 0 || S == nullptr || strideS == nullptr ||
+  if (phases < 1 || phases > 7 || iters < 0 || S == nullptr || strideS == nullptr ||
       p == nullptr || v0 == nullptr || out == nullptr || strideOut == nullptr || stats == nullptr || !root_args_ok(n, batch, groups))
     return AK_ERR_ARG;
   if (ws == nullptr || ws_bytes < ak_inv_root_group_ws_bytes(n, batch, groups)) return AK_ERR_WORKSPACE;
@@ -1166,7 +1053,7 @@ extern "C" int ak_inv_root_group(int phases, int begin, int iters, int groups, f
   st.alpha = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.beta = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.coef = floats(static_cast<int64_t>(total) * 2 * kRootSteps);
-  return root_run(phases, begin, iters, G, ridge_eps, max_power_iter, power_tol, max_iter, tol,
+  return root_run(phases, iters, G, ridge_eps, max_power_iter, power_tol, max_iter, tol,
                   static_cast<hipStream_t>(stream));
 }
 
@@ -1181,7 +1068,7 @@ extern "C" int ak_inv_root_newton(float* S, int64_t n, int batch, int64_t stride
                                   const float* v0, int max_power_iter, float power_tol, int max_iter, float tol,
                                   float* out, int64_t strideOut, float* stats, void* ws, size_t ws_bytes,
                                   ak_stream_t stream) {
-  return ak_inv_root_group(7, 0, max_iter, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0, max_power_iter, power_tol,
+  return ak_inv_root_group(7, max_iter, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0, max_power_iter, power_tol,
                            max_iter, tol, &out, &strideOut, &stats, ws, ws_bytes, stream);
 }
 
@@ -1191,6 +1078,6 @@ extern "C" int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t 
                                        float ridge_eps, const float* v0, int max_power_iter, float power_tol,
                                        int max_iter, float tol, float* out, int64_t strideOut, float* stats, void* ws,
                                        size_t ws_bytes, ak_stream_t stream) {
-  return ak_inv_root_group(phases, (phases & 1) ? 0 : -1, iters, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0,
+  return ak_inv_root_group(phases, iters, 1, &S, &n, &batch, &strideS, &p, ridge_eps, &v0,
                            max_power_iter, power_tol, max_iter, tol, &out, &strideOut, &stats, ws, ws_bytes, stream);
 }

@@ -1666,25 +1666,25 @@ def inv_root_group(items, ridge_eps, max_power_iter=100, power_tol=1e-6, max_ite
     lib = _lib.load()
     ws, ws_bytes, keep = _ws_args(lib.ak_inv_root_group_ws_bytes(n_a, b_a, count), dev)
 
-    def run(phases, begin, iters):
-        _lib.check(lib.ak_inv_root_group(phases, begin, iters, count, S_a, n_a, b_a, sS, p_a, float(ridge_eps), v_a,
+    def run(phases, iters):
+        _lib.check(lib.ak_inv_root_group(phases, iters, count, S_a, n_a, b_a, sS, p_a, float(ridge_eps), v_a,
                                          int(max_power_iter), float(power_tol), int(max_iter), float(tol), o_a, sO, st_a,
                                          ws, ws_bytes, _stream(dev)), 'ak_inv_root_group')
 
     chunks = ROOT_POLL_AFTER if poll_every is None else (int(poll_every),) * 2
     if chunks[0] <= 0 or chunks[0] >= max_iter:
-        run(7, 0, max_iter)
+        run(7, max_iter)
         return results
     off = lib.ak_inv_root_group_active_offset(n_a, b_a, count)
     active = keep[off:off + 4 * total].view(torch.int32)
-    run(3, 0, chunks[0])
+    run(3, chunks[0])
     done = chunks[0]
     while done < max_iter:
         with _on_launch_stream():
             if not any(active.tolist()):      # waits for what has been enqueued so far
                 break
         chunk = min(chunks[1], max_iter - done)
-        run(2, done, chunk)
+        run(2, chunk)
         done += chunk
-    run(4, 0, 0)
+    run(4, 0)
     return results

@@ -425,12 +425,11 @@ int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batc
                             ak_stream_t stream);
 
 /* Several groups of statistics in one launch sequence (group i: batch[i] matrices of size n[i], power p[i]; all arrays on
- * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 32768).  Same phases; `begin`: how many Newton
- * iterations the earlier parts have enqueued (-1: not known, one group only).  The `active` words of all matrices, group
- * after group, start at ws + ak_inv_root_group_active_offset(). */
+ * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 32768).  Same phases.  The
+ * `active` words of all matrices, group after group, start at ws + ak_inv_root_group_active_offset(). */
 size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, int groups);
 size_t ak_inv_root_group_active_offset(const int64_t* n, const int* batch, int groups);
-int ak_inv_root_group(int phases, int begin, int iters, int groups, float* const* S, const int64_t* n, const int* batch,
+int ak_inv_root_group(int phases, int iters, int groups, float* const* S, const int64_t* n, const int* batch,
                       const int64_t* strideS, const int* p, float ridge_eps, const float* const* v0, int max_power_iter,
                       float power_tol, int max_iter, float tol, float* const* out, const int64_t* strideOut,
                       float* const* stats, void* ws, size_t ws_bytes, ak_stream_t stream);
