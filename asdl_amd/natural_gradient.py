@@ -47,6 +47,23 @@ def _bias_requires_grad(module):
     return hasattr(module, 'bias') and module.bias is not None and module.bias.requires_grad
 
 
+def _dense_on_gpu(t, n):
+    return t is not None and t.is_cuda and t.dtype == torch.float32 and t.numel() == n and t.is_contiguous()
+
+
+def _with_shared_gradients(work):
+    """The modules of ``work`` whose weight or bias gradient another of them holds too (tied parameters).  One after the other
+    they give B2 (B1 G A1) A2 on such a gradient (asdl/precondition/natural_gradient.py:478-486, 508-543); launches that take many
+    modules at once, or modules on several streams, would read and write it in no order."""
+    holders = {}
+    for module, _ in work:
+        for name in ('weight', 'bias'):
+            grad = getattr(getattr(module, name, None), 'grad', None)
+            if grad is not None:
+                holders.setdefault(grad.data_ptr(), []).append(module)
+    return {module for modules in holders.values() if len(modules) > 1 for module in modules}
+
+
 class NaturalGradientMaker(PreconditionedGradientMaker):
     _supported_classes = (nn.Linear, nn.Conv2d, nn.BatchNorm1d, nn.BatchNorm2d, nn.LayerNorm, nn.Embedding)
 
@@ -338,9 +355,8 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         if not work or len(fail) > 2 or 0 in fail or modules == getattr(self, '_deep_declined', None):
             return False
 
-        def dense(t, n):
-            return t is not None and t.is_cuda and t.dtype == torch.float32 and t.numel() == n and t.is_contiguous()
-        items, units = [], []
+        dense = _dense_on_gpu
+        items, units, grads = [], [], []
         attr = self._fisher_attr
         for module, shape in work:
             fisher = getattr(module, attr, None)
@@ -350,8 +366,11 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
                 return False
             gw = weight.grad
             gb = bias.grad if bias is not None and bias.requires_grad else None
-            if bias is not None and bias.requires_grad and gb is None:
+            if gw is None or (bias is not None and bias.requires_grad and gb is None):
                 return False
+            grads.append(gw.data_ptr())
+            if gb is not None:
+                grads.append(gb.data_ptr())
             if shape == SHAPE_UNIT_WISE:
                 inv = fisher.unit.inv if fisher.unit is not None else None
                 F = weight.numel()
@@ -367,6 +386,8 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             if not (dense(B_inv, dB * dB) and dense(A_inv, dA * dA) and dense(gw, dB * dA) and (gb is None or dense(gb, dB))):
                 return False
             items += (B_inv.data_ptr(), A_inv.data_ptr(), gw.data_ptr(), 0 if gb is None else gb.data_ptr(), dB, dA)
+        if len(set(grads)) != len(grads):
+            return False                         # a shared gradient (_with_shared_gradients): one module after the other
         if not kernels.kron_precond_deep(items, units, float(grad_scale), gw.device, fail):
             self._deep_declined = modules        # the sizes decide: not asked again for these modules
             return False
@@ -411,8 +432,11 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             for module, shape in work:
                 self._precondition_module(module, shape, grad_scale=grad_scale, use_inv=use_inv)
             return
-        # The layers are independent and most of their GEMMs are too small to fill the device: spread them
-        # over the side streams (largest first) and join.  Everything they touch is waited for before returning.
+        # Layers with gradients of their own are independent and most of their GEMMs are too small to fill the device:
+        # spread them over the side streams (largest first) and join.  Everything they touch is waited for before returning.
+        shared = _with_shared_gradients(work)
+        in_order = [(m, shape) for m, shape in work if m in shared]
+        work = [(m, shape) for m, shape in work if m not in shared]
         from .symmatrix import _side_streams
         dev = grads[0].device
         main = torch.cuda.current_stream(dev)
@@ -429,6 +453,8 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             done = torch.cuda.Event()
             done.record(st)
             main.wait_event(done)
+        for module, shape in in_order:
+            self._precondition_module(module, shape, grad_scale=grad_scale, use_inv=use_inv)
 
     def _precondition_work(self):
         return [(module, shape) for shape in _kernel_shapes for module in self.modules_for(shape)
@@ -441,7 +467,11 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         (plan, rest of ``work`` for the per-module path, signature) or None when no module qualifies;
         the signature lists the objects the plan was built from."""
         items, unit_items, rest, signature = [], [], [], []
+        shared = _with_shared_gradients(work)
         for module, shape in work:
+            if module in shared:
+                rest.append((module, shape))
+                continue
             kron = self._get_module_symmatrix(module, shape) if shape in (SHAPE_KRON, SHAPE_SWIFT_KRON) else None
             weight = getattr(module, 'weight', None)
             item = None

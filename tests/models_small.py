@@ -59,6 +59,19 @@ class SharedNet(nn.Module):
         return self.head(x)
 
 
+def get_tied_mlp(width=10, out=5):
+    """Two pairs of Linear layers with one weight each (the first with one bias too), tied LayerNorms, four layers of their own."""
+    net = nn.Sequential(*(m for _ in range(4) for m in (nn.Linear(width, width), nn.Tanh())), nn.LayerNorm(width),
+                        nn.Linear(width, width), nn.LayerNorm(width), nn.Linear(width, width), nn.Tanh(),
+                        nn.Linear(width, width), nn.Tanh(), nn.Linear(width, out))
+    linear = [m for m in net if isinstance(m, nn.Linear)]
+    norms = [m for m in net if isinstance(m, nn.LayerNorm)]
+    linear[4].weight, linear[4].bias = linear[1].weight, linear[1].bias
+    linear[5].weight = linear[2].weight
+    norms[1].weight, norms[1].bias = norms[0].weight, norms[0].bias
+    return net
+
+
 GOLDEN_KFAC = {
     # tag: (model factory, fisher_type, ema_decay, damping, seed, curvature interval, preconditioner interval)
     'mlp_fisher_emp_ema-1': (get_mlp, 'fisher_emp', -1, 1e-2, None, None, 1),

@@ -2,6 +2,7 @@
 orchestration, with the kernel entry points replaced by oracle-backed stand-ins
 (tests/cpu_backend.py).  Also checks that the C-ABI library loads and exports every declared symbol
 and that the product refuses CPU tensors."""
+import copy
 import os
 
 import numpy as np
@@ -14,7 +15,7 @@ import asdl_amd
 from asdl_amd import (PreconditioningConfig, KfacGradientMaker, GradientMaker, FisherConfig, get_fisher_maker,
                       get_update_schedule, SHAPE_KRON, FISHER_EMP, FISHER_MC, FISHER_EXACT, LOSS_CROSS_ENTROPY, LOSS_MSE)
 from conftest import GOLDEN
-from models_small import GOLDEN_KFAC, get_mlp, get_cnn
+from models_small import GOLDEN_KFAC, get_mlp, get_cnn, get_tied_mlp
 import cpu_backend
 
 
@@ -353,6 +354,53 @@ def test_kfac_host_logic_matches_reference_golden(tag, monkeypatch):
                 assert m.fisher.kron.A is None and m.fisher.kron.B is None    # only inverses are kept
         opt.step()
     assert gm.state_dict()['step'] == n_steps
+
+
+@pytest.mark.parametrize('form', ['deep', 'plan', 'per module'])
+def test_modules_that_share_a_gradient_are_preconditioned_one_after_the_other(form, monkeypatch):
+    """Tied parameters: B2 (B1 G A1) A2 in the order of the modules.  The stand-ins for the launches that take many modules at
+    once accept everything except what those launches cannot do, the same gradient twice."""
+    import asdl_amd.natural_gradient as ng
+    from asdl_amd import kernels
+    from oracle import cpu_ref
+    cpu_backend.install(monkeypatch)
+    taken = []
+
+    def distinct(addresses):
+        assert len(set(addresses)) == len(addresses), 'one launch, the same gradient twice'
+        taken.extend(addresses)
+
+    def deep(items, units, grad_scale, device, fail=()):
+        distinct([p for i in range(0, len(items), 6) for p in items[i + 2:i + 4] if p] + [p for i in range(0, len(units), 4) for p in units[i + 1:i + 3]])
+        return False
+
+    class Plan:
+        def __init__(self, items, grad_scale=1.0, unit_items=()):
+            distinct([g.data_ptr() for it in items for g in it[2:4] if g is not None] + [g.data_ptr() for it in unit_items for g in it[1:3]])
+            self.items, self.grad_scale = items, grad_scale
+
+        def launch(self):
+            for B_inv, A_inv, g, b in self.items:
+                cpu_backend.kron_precond(B_inv, A_inv, g, b, self.grad_scale)
+
+    monkeypatch.setattr(ng, 'GROUPED_PRECONDITION', form != 'per module')
+    monkeypatch.setattr(kernels, 'kron_precond_deep', deep)
+    monkeypatch.setattr(kernels, 'kron_precond_groupable', lambda *a: True)
+    monkeypatch.setattr(kernels, 'KronPrecondPlan', Plan)
+    if form == 'deep':
+        monkeypatch.setattr(ng, '_dense_on_gpu', lambda t, n: t is not None and t.numel() == n)
+    torch.manual_seed(5)
+    model = get_tied_mlp()
+    reference = copy.deepcopy(model)
+    x, t = torch.randn(16, 10), torch.randint(5, (16,))
+    gm = KfacGradientMaker(model, PreconditioningConfig(data_size=16, damping=1e-2), fisher_type=FISHER_EMP, grad_scale=0.5)
+    gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x), t)
+    gm.forward_and_backward()
+    assert bool(taken) == (form != 'per module')
+    orc = cpu_ref.KfacOracle(reference, data_size=16, damping=1e-2, fisher_type='fisher_emp', unit_wise_norm=True, grad_scale=0.5)
+    orc.forward_and_backward(x, t)
+    for (name, p), q in zip(model.named_parameters(), reference.parameters()):
+        assert grad_close(p.grad, q.grad, 2e-4), name
 
 
 def _resume_run(monkeypatch, ema, ci, pi, fisher_type, n_steps=4, stop=2):

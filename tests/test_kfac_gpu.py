@@ -15,7 +15,7 @@ import torch.nn.functional as F
 
 from asdl_amd import PreconditioningConfig, KfacGradientMaker, FISHER_EMP, FISHER_MC, FISHER_EXACT
 from conftest import GOLDEN
-from models_small import GOLDEN_KFAC
+from models_small import GOLDEN_KFAC, get_tied_mlp
 from oracle import cpu_ref as R
 import bench_models
 
@@ -724,6 +724,33 @@ def test_grouped_precondition_and_its_early_preparation_give_the_per_module_resu
     got, _ = run(True, True, False, replace_grad=True)
     for key in ref:
         assert grad_close(got[key], ref[key], 1e-5), key
+
+
+@pytest.mark.parametrize('width', [10, 12])
+@pytest.mark.parametrize('grouped,pi', [(True, 1), (False, 1), (True, 2)])
+def test_tied_parameters_match_the_oracle(width, grouped, pi, monkeypatch):
+    """Modules that share a weight or a bias are preconditioned in their order, B2 (B1 G A1) A2, whatever takes the others:
+    widths that the grouped plan takes (12) and that it does not (10), the per-module path over the side streams, and a step
+    between two renewals."""
+    import asdl_amd.natural_gradient as ng_mod
+    monkeypatch.setattr(ng_mod, 'GROUPED_PRECONDITION', grouped)
+    torch.manual_seed(5)
+    model_cpu = get_tied_mlp(width)
+    model = copy.deepcopy(model_cpu).cuda()
+    assert model[0].weight is not model[2].weight and model[2].weight is model[9].weight
+    gm = KfacGradientMaker(model, PreconditioningConfig(data_size=16, damping=1e-2, preconditioner_upd_interval=pi),
+                           fisher_type=FISHER_EMP, grad_scale=0.5)
+    orc = R.KfacOracle(model_cpu, data_size=16, damping=1e-2, fisher_type='fisher_emp', unit_wise_norm=True, grad_scale=0.5,
+                             preconditioner_upd_interval=pi)
+    for step in range(2):
+        x, t = torch.randn(16, width), torch.randint(5, (16,))
+        for m in (model, model_cpu):
+            m.zero_grad(set_to_none=True)
+        gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x.cuda()), t.cuda())
+        gm.forward_and_backward()
+        orc.forward_and_backward(x, t)
+        for (name, p), q in zip(model.named_parameters(), model_cpu.parameters()):
+            assert grad_close(p.grad, q.grad, 1e-3), (step, name)
 
 
 def test_identity_where_zero_touches_only_the_flagged_matrices():
