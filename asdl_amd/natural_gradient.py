@@ -437,7 +437,7 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         shared = _with_shared_gradients(work)
         in_order = [(m, shape) for m, shape in work if m in shared]
         work = [(m, shape) for m, shape in work if m not in shared]
-        from .symmatrix import _side_streams
+        from .symmatrix import _side_stream_guard, _side_streams
         dev = grads[0].device
         main = torch.cuda.current_stream(dev)
         side = _side_streams(dev, PRECONDITION_STREAMS)
@@ -447,7 +447,8 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         for st in side:
             st.wait_event(start)
         for i, (module, shape) in enumerate(work):
-            with torch.cuda.stream(side[i % len(side)]):
+            st = side[i % len(side)]
+            with _side_stream_guard(st), torch.cuda.stream(st):
                 self._precondition_module(module, shape, grad_scale=grad_scale, use_inv=use_inv)
         for st in side:
             done = torch.cuda.Event()

@@ -6,6 +6,7 @@ save / load :25-87, 226-269, 471-492); the arithmetic runs in the HIP kernels.  
 saved and loaded; KFE and diagonal containers are accepted as opaque attributes but have no kernels here.
 """
 import os
+import threading
 from collections import defaultdict
 
 import numpy as np
@@ -66,6 +67,8 @@ def _load_from_numpy(path, device=None):
 
 
 _side_stream_cache = {}
+_side_stream_locks = {}        # per stream handle: held by the thread that enqueues on it
+_side_stream_lock = threading.Lock()       # of the two dictionaries and of _next_side_stream
 N_SIDE_STREAMS = 8     # groups of a batched inverse that may run side by side
 GROUPED_INVERSE = True  # all square factors of a call in one merged launch sequence (kernels.chol_inv_grouped);
                         # False: one batched inverse per distinct size, spread over the side streams
@@ -73,13 +76,45 @@ GROUPED_INVERSE = True  # all square factors of a call in one merged launch sequ
 
 def _side_streams(device, n):
     key = device.index if device.index is not None else torch.cuda.current_device()
-    pool = _side_stream_cache.setdefault(key, [])
-    while len(pool) < n:
-        pool.append(torch.cuda.Stream(device=device))
-    return pool[:n]
+    with _side_stream_lock:
+        pool = _side_stream_cache.setdefault(key, [])
+        while len(pool) < n:
+            pool.append(torch.cuda.Stream(device=device))
+        return pool[:n]
+
+
+def _side_stream_guard(stream):
+    """The lock that a thread holds while it enqueues a sequence of launches on a side stream.  The pool is the process's: two
+    threads may be given one stream, whose launches share its workspace, and the library's calls drop the interpreter lock,
+    so that the launches of two sequences could otherwise interleave over one scratch buffer."""
+    with _side_stream_lock:
+        return _side_stream_locks.setdefault(stream.cuda_stream, threading.Lock())
 
 
 _next_side_stream = 0
+
+
+def _enqueue_beside(dev, groups, run_group):
+    """Runs run_group(group) for every group with this thread's launches on side streams that wait for the current one, and
+    returns those streams.  Successive calls start on different side streams (each with its own workspace), so that an early
+    batch and the remainder of one step run side by side.  The launches are issued from here: handing them to another
+    thread cost more in interpreter-lock changes (0.6 ms of a small step) than the launches themselves."""
+    global _next_side_stream
+    pool = _side_streams(dev, N_SIDE_STREAMS)
+    n_used = min(len(pool), len(groups))
+    with _side_stream_lock:
+        first = _next_side_stream
+        _next_side_stream += n_used
+    side = [pool[(first + i) % len(pool)] for i in range(n_used)]
+    for i, st in enumerate(side):
+        with _side_stream_guard(st):
+            kernels.order_streams(None, st.cuda_stream, dev)
+            with kernels.launches_on(st):
+                for group in groups[i::n_used]:
+                    run_group(group)
+    return side
+
+
 INLINE_MICROSECONDS = 300      # a deferred batch shorter than this runs on the caller's stream
 
 
@@ -322,19 +357,7 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
         us += 150 + sum(e[1].shape[1] ** 2 for e in together) / 750e3 if together else 0
         inline = us < INLINE_MICROSECONDS
     if mats_on_gpu and prepared and not (inline and len(prepared) <= 1 + bool(together)):
-        # Successive calls start on different side streams (each with its own workspace), so that an early batch and
-        # the remainder of one step run side by side.  The launches are issued from here: handing them to another
-        # thread cost more in interpreter-lock changes (0.6 ms of a small step) than the launches themselves.
-        global _next_side_stream
-        pool = _side_streams(dev, N_SIDE_STREAMS)
-        n_used = min(len(pool), len(prepared))
-        side = [pool[(_next_side_stream + i) % len(pool)] for i in range(n_used)]
-        _next_side_stream += n_used
-        for i, st in enumerate(side):
-            kernels.order_streams(None, st.cuda_stream, dev)
-            with kernels.launches_on(st):
-                for group in prepared[i::n_used]:
-                    run_group(group)
+        side = _enqueue_beside(dev, prepared, run_group)
     else:
         for group in prepared:
             run_group(group)

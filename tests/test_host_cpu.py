@@ -611,3 +611,38 @@ def test_pruned_fisher_backward_equals_full_backward(fisher_type, monkeypatch):
     assert full.keys() == pruned.keys() and any(k.endswith('.unit') for k in full)
     for key in full:
         assert torch.equal(full[key], pruned[key]), key
+
+
+# ------------------------------------------------------------------ side streams of the inverses
+class _FakeStream:
+    def __init__(self, handle):
+        self.cuda_stream = handle
+
+
+def test_threads_do_not_interleave_their_launches_on_one_side_stream(monkeypatch):
+    """The pool of side streams is the process's and a stream's launches share its workspace: while one thread enqueues its
+    groups on a stream, no other one may.  More groups than streams, so that all threads meet on all of them."""
+    import threading
+    import time
+    from asdl_amd import kernels, symmatrix
+    pool = [_FakeStream(h) for h in (11, 12, 13)]
+    monkeypatch.setattr(symmatrix, '_side_streams', lambda dev, n: pool)
+    monkeypatch.setattr(kernels, 'order_streams', lambda *a: None)
+    busy, overlaps, ran = {}, [], []
+
+    def run_group(group):
+        handle = kernels._stream_handle()
+        if busy.setdefault(handle, threading.get_ident()) != threading.get_ident():
+            overlaps.append(handle)
+        time.sleep(0.002)
+        busy.pop(handle, None)
+        ran.append(group)
+
+    threads = [threading.Thread(target=lambda i=i: [symmatrix._enqueue_beside(None, [(i, k, j) for j in range(5)], run_group) for k in range(4)])
+               for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(ran) == len(set(ran)) == 4 * 4 * 5
+    assert not overlaps
