@@ -158,7 +158,9 @@ def _dtype_code(t):
 
 def workspace(nbytes, device):
     """A cached scratch buffer per (device, stream); grows geometrically, never shrinks.
-    Kernels on one stream run in order, so consecutive calls may share it."""
+    Kernels on one stream run in order, so consecutive calls may share it.  The buffer is allocated on the stream whose
+    launches use it (a side stream inside launches_on()): when a larger one takes its place, its memory goes back to that
+    stream, where whatever gets it next runs behind the launches that still use it."""
     if nbytes <= 0:
         return None, 0
     key = (device.index if device.index is not None else torch.cuda.current_device(), _stream_handle(device))
@@ -168,7 +170,8 @@ def workspace(nbytes, device):
             size = max(nbytes, 1 << 20)
             if buf is not None:
                 size = max(size, int(buf.numel() * 1.5))
-            buf = torch.empty(size, dtype=torch.uint8, device=device)
+            with _on_launch_stream():
+                buf = torch.empty(size, dtype=torch.uint8, device=device)
             _workspaces[key] = buf
     return buf, buf.numel()
 

@@ -646,3 +646,27 @@ def test_threads_do_not_interleave_their_launches_on_one_side_stream(monkeypatch
         t.join()
     assert len(ran) == len(set(ran)) == 4 * 4 * 5
     assert not overlaps
+
+
+def test_workspace_belongs_to_the_stream_whose_launches_use_it(monkeypatch):
+    """A workspace that is replaced by a larger one goes back to the stream it was allocated on.  If that was the caller's stream
+    while a side stream's launches used it, the caller's next tensor would take the memory under those launches."""
+    import contextlib
+    from asdl_amd import kernels
+    current, allocated = ['main'], []
+
+    @contextlib.contextmanager
+    def stream(st):
+        current.append(st)
+        yield
+        current.pop()
+
+    empty = torch.empty
+    monkeypatch.setattr(torch.cuda, 'stream', stream)
+    monkeypatch.setattr(torch, 'empty', lambda *a, **k: allocated.append(current[-1]) or empty(*a, **k))
+    monkeypatch.setattr(kernels, '_workspaces', {})
+    side = _FakeStream(77)
+    with kernels.launches_on(side):
+        for nbytes in (1 << 20, 1 << 22):
+            kernels.workspace(nbytes, torch.device('cpu', 0))
+    assert allocated == [side, side]
