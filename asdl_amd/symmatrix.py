@@ -189,6 +189,14 @@ class PendingInverses:
         for st in side:
             kernels.order_streams(st.cuda_stream, None, st.device)
 
+    def __del__(self):
+        # dropped unfinished (the pass beside it raised): its tensors go back to the current stream's memory, which has to
+        # wait for the side streams that still write them
+        try:
+            self.join()
+        except Exception:
+            pass
+
     def finish_late(self):
         """finish() without its host synchronisation: the inverses are stored on the Kron objects as if every factor
         was non-zero and positive definite, the copy of the flags to pinned host memory is enqueued, and the returned

@@ -670,3 +670,16 @@ def test_workspace_belongs_to_the_stream_whose_launches_use_it(monkeypatch):
         for nbytes in (1 << 20, 1 << 22):
             kernels.workspace(nbytes, torch.device('cpu', 0))
     assert allocated == [side, side]
+
+
+def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):
+    """A pass beside the inverses that raises drops them unread: what takes their memory next has to run behind them."""
+    from asdl_amd import kernels, symmatrix
+    ordered = []
+    monkeypatch.setattr(kernels, 'order_streams', lambda before, after, device: ordered.append((before, after)))
+    side = _FakeStream(5)
+    side.device = torch.device('cpu')
+    pending = symmatrix.PendingInverses([], torch.zeros(1, dtype=torch.int32), None, [side], False)
+    assert ordered == []
+    del pending
+    assert ordered == [(5, None)]
