@@ -1,5 +1,7 @@
-// One draw per row of a categorical distribution given by logits: the largest of p_i / q_i, q_i exponential random numbers,
-// taken as the largest of logits_i - log q_i (the normalisation of p shifts every term of a row alike).
+// One draw per row of a categorical distribution given by logits: the largest of p_i / q_i, q_i exponential random numbers.
+// Two classes are compared by (logits_i - logits_j) - (log q_i - log q_j): the normalisation of p drops out, and so does an
+// offset that all logits of a row share, before anything is rounded to its size (logits_i - log q_i at an offset of 1e6 has a
+// spacing of 0.06: another class than softmax's in 1 % of the rows).
 // Bound by the device memory: logits and random numbers are read once (8192 x 4096: 268 MB) where softmax, normalisation,
 // their checks, the quotient and the argmax made a dozen passes and launches.
 #include "common.hpp"
@@ -7,12 +9,14 @@
 namespace ak {
 
 struct Best {
-  float v;
+  float x, l;      // logit and log q of the best class so far
   int i;
 };
 
-__device__ __forceinline__ void best_of(Best& a, float v, int i) {
-  if (v > a.v || (v == a.v && i < a.i)) { a.v = v; a.i = i; }
+// (the difference of two logits of -inf is NaN: the best so far stays)
+__device__ __forceinline__ void best_of(Best& a, float x, float l, int i) {
+  const float d = (x - a.x) - (l - a.l);
+  if (d > 0.f || (d == 0.f && i < a.i)) a = Best{x, l, i};
 }
 
 // One wave per row (few classes) or one work group of four waves per row.
@@ -28,27 +32,27 @@ static __global__ __launch_bounds__(256) void sample_categorical_kernel(const fl
   const float* __restrict__ e = q + row * classes;
   const int t = WAVES == 1 ? lane : threadIdx.x;
   constexpr int N = 64 * WAVES;
-  Best b{-INFINITY, 0x7fffffff};
+  Best b{-INFINITY, 0.f, 0x7fffffff};
   const bool vec = classes % 4 == 0 && ((reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(q)) & 15) == 0;
   if (vec) {
 #pragma unroll 4
     for (int c = 4 * t; c < classes; c += 4 * N) {
       const floatx4 xv = *reinterpret_cast<const floatx4*>(x + c), ev = *reinterpret_cast<const floatx4*>(e + c);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) best_of(b, xv[u] - logf(ev[u]), c + u);
+      for (int u = 0; u < 4; ++u) best_of(b, xv[u], logf(ev[u]), c + u);
     }
   } else {
 #pragma unroll 4
-    for (int c = t; c < classes; c += N) best_of(b, x[c] - logf(e[c]), c);
+    for (int c = t; c < classes; c += N) best_of(b, x[c], logf(e[c]), c);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) best_of(b, __shfl_xor(b.v, o), __shfl_xor(b.i, o));
+  for (int o = 32; o > 0; o >>= 1) best_of(b, __shfl_xor(b.x, o), __shfl_xor(b.l, o), __shfl_xor(b.i, o));
   if constexpr (WAVES > 1) {
     if (lane == 0) part[wave] = b;
     __syncthreads();
     b = part[0];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) best_of(b, part[w].v, part[w].i);
+    for (int w = 1; w < WAVES; ++w) best_of(b, part[w].x, part[w].l, part[w].i);
   }
   if (t == 0) targets[row] = b.i < classes ? b.i : 0;
 }

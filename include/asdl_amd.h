@@ -177,7 +177,7 @@ int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, 
                          ak_stream_t stream);
 
 /* targets[r] = argmax_i logits[r][i] - log(q[r][i]) for q exponentially distributed: a draw of softmax(logits[r]) per row
- * (torch.multinomial's choice from the same random numbers).  Row-major [rows, classes] float32; the lowest index wins ties;
+ * (torch.multinomial's choice from the same random numbers, whatever offset the logits of a row share).  Row-major [rows, classes] float32; the lowest index wins ties;
  * NaN logits are never chosen (a row of NaNs gives 0). */
 int ak_sample_categorical(const float* logits, const float* q, int64_t rows, int64_t classes, int64_t* targets,
                           ak_stream_t stream);

@@ -808,6 +808,32 @@ def test_sample_categorical_draws_what_torch_draws(K, shape):
     assert ours.shape == theirs.shape and torch.equal(ours, theirs)
 
 
+@pytest.mark.parametrize('offset', [0.0, 1e4, -1e5, 1e6])
+@pytest.mark.parametrize('rows,classes', [(20000, 50), (4000, 1027)])
+def test_sample_categorical_with_an_offset_of_the_logits(K, offset, rows, classes):
+    """An offset that all logits of a row share changes no draw of softmax.  Against the same comparison in 64 bits of the same
+    float32 logits and random numbers; only rows whose best two classes are closer than the rounding of the 32-bit terms (log q
+    and the differences stay below 64 in size: 4 roundings of 2^-19) may differ."""
+    g = torch.Generator('cuda').manual_seed(3)
+    logits = 3 * torch.randn(rows, classes, device='cuda', generator=g) + offset
+    torch.manual_seed(7)
+    ours = K.sample_categorical(logits)
+    torch.manual_seed(7)
+    q = torch.empty_like(logits).exponential_()
+    score = logits.double() - q.double().log()
+    best, theirs = score.topk(2, dim=1)
+    clear = best[:, 0] - best[:, 1] > 4 * 2 ** -19
+    assert int(clear.sum()) > 0.99 * rows
+    assert torch.equal(ours[clear], theirs[clear, 0])
+
+
+def test_sample_categorical_leaves_masked_classes_out(K):
+    logits = torch.randn(500, 300, device='cuda', generator=torch.Generator('cuda').manual_seed(1))
+    logits[:, ::2] = float('-inf')
+    logits[:, 1::4] = torch.finfo(torch.float32).min
+    assert torch.all(K.sample_categorical(logits) % 4 == 3)
+
+
 @pytest.mark.parametrize('f', [1, 256, 300])
 def test_unit_wise_keep_grouped(K, f):
     """Modules whose blocks are all zero keep their previous inverse or get the identity; the others are left alone."""
