@@ -59,7 +59,7 @@ _SIGNATURES = {
     'ak_event_create': (c_int, [ctypes.POINTER(ctypes.c_void_p), c_int]),
     'ak_event_destroy': (c_int, [c_ptr]),
     'ak_event_record': (c_int, [c_ptr, c_ptr]),
-    'ak_sample_categorical': (c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr]),
+    'ak_sample_categorical': (c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr, c_ptr]),
     'ak_event_synchronize': (c_int, [c_ptr]),
     'ak_kron_finish': (c_int, [c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_int, c_ptr, c_ptr]),
     'ak_kron_precond_deep_ws_bytes': (c_size, [c_ptr, c_int]),

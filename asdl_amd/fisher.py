@@ -78,17 +78,25 @@ class FisherMaker(GradientMaker):
         self.flags_to_caller = False         # set by a caller that enqueues work between the inverses and their flags
                                              # (the preconditioning) and then reads them itself: take_caller_flags()
         self._caller_flags = None
+        self._sampled = []                   # unread checks of the logits that targets were drawn from,
+        self._late_sampled = []              # and those that late_inverse_flags left unread
         self.before_inverse_wait = None      # optional callable, run right before the host waits for the inverses
         self.after_factors = None            # optional callable, run when the factors are final and before the loss
                                              # backward pass is enqueued; may return an object with finish()
 
     def check_late_flags(self):
         """Reads the flags of the last update whose flags were left unread (late_inverse_flags) and raises
-        torch.linalg.LinAlgError for a factor that was not positive definite.  Called by the next update; call it
-        after the last one."""
-        pending, self._late_flags = self._late_flags, []
+        torch.linalg.LinAlgError for a factor that was not positive definite, RuntimeError for a draw from logits that are
+        no distribution.  Called by the next update; call it after the last one."""
+        pending, self._late_flags, self._late_sampled = self._late_sampled + self._late_flags, [], []
         for late in pending:
             late.check()
+
+    def _check_sampled(self):
+        """Raises torch.multinomial's RuntimeError if this call's targets were drawn from logits that are no distribution."""
+        sampled, self._sampled = self._sampled, []
+        for drawn in sampled:
+            drawn.check()
 
     def take_caller_flags(self):
         """The unread flags of this call's inverses (flags_to_caller), as a list of objects with check(); None when
@@ -164,6 +172,7 @@ class FisherMaker(GradientMaker):
             self.zero_fisher()
         if config.seed is not None:
             manual_seed(config.seed)
+        self._sampled = []
 
         loss_grad_with_fisher = calc_loss_grad and self.is_fisher_emp
         loss_grad_after_fisher = calc_loss_grad and not self.is_fisher_emp
@@ -211,13 +220,17 @@ class FisherMaker(GradientMaker):
             cxt.join_factor_stream()
             phase_mark('bwd_fisher')      # backward pass that feeds the cov_kron_B kernels (early inverses run beside it)
             cxt.finish_registered()
+            defer = loss_grad_after_fisher or self.flags_to_caller
+            if not defer:
+                self._check_sampled()         # (the host waits for the inverses below)
             # The inverses only need the factors: enqueue them now (side streams) and, when a loss backward
             # pass follows, let that pass run on the main stream meanwhile; the flags are read afterwards.
-            deferred = cxt.flush_inverses(defer=loss_grad_after_fisher or self.flags_to_caller)
+            deferred = cxt.flush_inverses(defer=defer)
             self._inverse_cost_prev = cxt.inverse_cost
             self._extract_fisher(cxt)
 
         if inv_after_fisher:
+            self._check_sampled()
             self.replace_fisher_with_inv(damping)
         early = None
         if loss_grad_after_fisher:
@@ -233,6 +246,10 @@ class FisherMaker(GradientMaker):
                 torch._foreach_div_(grads, data_size)     # one launch for all parameters
             loss.div_(data_size)
         phase_mark('bwd_loss')            # loss backward pass (the inverses run beside it on side streams)
+        # Logits that are no distribution raise here, before anything acts on the gradients: the host waits for the draw only, and
+        # the device has both backward passes in its queue meanwhile.
+        if not (self.late_inverse_flags and deferred is not None):
+            self._check_sampled()
         if deferred is not None or early is not None:
             if self.before_inverse_wait is not None and not (self.flags_to_caller and not self.late_inverse_flags):
                 self.before_inverse_wait()      # host work of the caller that needs no flags: the device is still busy
@@ -245,7 +262,7 @@ class FisherMaker(GradientMaker):
                 elif to_caller:
                     self.add_caller_flags(late)
                 else:
-                    self._late_flags = late
+                    self._late_flags, self._late_sampled, self._sampled = late, self._sampled, []
             if early is not None:
                 if self.flags_to_caller:
                     self.add_caller_flags([early.finish_late()])
@@ -338,7 +355,12 @@ class FisherMCCrossEntropy(FisherMaker):
             dist = torch.distributions.Categorical(F.softmax(logits, dim=-1), validate_args=False)
         for i in range(n_mc_samples):
             with torch.no_grad():
-                targets = kernels.sample_categorical(logits) if dist is None else self.sample_targets(dist, i)
+                if dist is None:
+                    targets, drawn = kernels.sample_categorical(logits, late=True)
+                    if i == 0 and drawn is not None:       # (the same logits every time)
+                        self._sampled.append(drawn)
+                else:
+                    targets = self.sample_targets(dist, i)
 
             def nll_expr():
                 nll = F.nll_loss(log_probs.view(-1, log_probs.size(-1)), targets.view(-1), reduction='sum',

@@ -984,6 +984,9 @@ class HostFlags:
         self._words = words
         self.address = self._host.data_ptr()
 
+    def clear(self):
+        self._host[:self._words].zero_()         # (whoever had the memory before has read it)
+
     def record(self):
         _lib.check(_lib.load().ak_event_record(self._event, _stream()), 'ak_event_record')
 
@@ -1100,19 +1103,48 @@ def sampleable(logits):
         logits.numel() > 0
 
 
-def sample_categorical(logits):
+class SampledLogits:
+    """Whether the logits of a draw gave every row a distribution: a word on its way to the host."""
+
+    def __init__(self, device):
+        self._flags = HostFlags(device, 1)
+        self._flags.clear()
+        self.address = self._flags.address
+
+    def record(self):
+        self._flags.record()
+
+    def check(self, *args, **kwargs):
+        """Waits for the draw and raises what torch.multinomial raises."""
+        flags, self._flags = self._flags, None
+        if flags is not None and flags.read()[0]:
+            raise RuntimeError('probability tensor contains either `inf`, `nan` or element < 0')
+        return []
+
+
+def sample_categorical(logits, late=False):
     """One class per row of float32 ``logits`` [..., classes] from softmax(logits): the draw of
     torch.distributions.Categorical(softmax(logits)).sample() from the same exponential random numbers (the largest of
-    p_i / q_i, q exponential), without forming the probabilities, their checks and the quotient in device memory."""
+    p_i / q_i, q exponential), without forming the probabilities, their checks and the quotient in device memory.
+    Logits with NaN or +inf, or a row of -inf, raise torch.multinomial's RuntimeError, which waits for the draw; ``late``:
+    returns (targets, SampledLogits) instead, whose check() raises it.  (A stream capture has no check.)"""
     _require_gpu(logits)
     if not sampleable(logits):
         raise ValueError('logits have to be contiguous float32 with at least two dimensions')
     logits = logits.detach()
     q = torch.empty_like(logits.view(-1, logits.shape[-1])).exponential_()
     targets = torch.empty(logits.shape[:-1], dtype=torch.int64, device=logits.device)
+    valid = None if torch.cuda.is_current_stream_capturing() else SampledLogits(logits.device)
     rc = _lib.load().ak_sample_categorical(ctypes.c_void_p(logits.data_ptr()), ctypes.c_void_p(q.data_ptr()), q.shape[0],
-                                           q.shape[1], ctypes.c_void_p(targets.data_ptr()), _stream())
+                                           q.shape[1], ctypes.c_void_p(targets.data_ptr()),
+                                           ctypes.c_void_p(valid.address if valid is not None else 0), _stream())
     _lib.check(rc, 'ak_sample_categorical')
+    if valid is not None:
+        valid.record()
+    if late:
+        return targets, valid
+    if valid is not None:
+        valid.check()
     return targets
 
 

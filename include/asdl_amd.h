@@ -178,9 +178,10 @@ int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, 
 
 /* targets[r] = argmax_i logits[r][i] - log(q[r][i]) for q exponentially distributed: a draw of softmax(logits[r]) per row
  * (torch.multinomial's choice from the same random numbers, whatever offset the logits of a row share).  Row-major [rows, classes] float32; the lowest index wins ties;
- * NaN logits are never chosen (a row of NaNs gives 0). */
+ * logits of -inf are never chosen.  invalid (may be null; device or pinned host word, cleared by the caller): becomes 1 if a row has
+ * no distribution, i.e. holds a NaN or +inf or nothing but -inf; its target is then a class in range without meaning. */
 int ak_sample_categorical(const float* logits, const float* q, int64_t rows, int64_t classes, int64_t* targets,
-                          ak_stream_t stream);
+                          int* invalid, ak_stream_t stream);
 
 /* ak_kron_damping for pairs whose factors may be n x d row matrices: dims = device int64 [batch,4]
  * (rows_A, d_A, rows_B, d_B; rows = 0: square d x d factor, eigenvalue mean trace/d; rows > 0: sum(x^2)/d),

@@ -834,6 +834,26 @@ def test_sample_categorical_leaves_masked_classes_out(K):
     assert torch.all(K.sample_categorical(logits) % 4 == 3)
 
 
+@pytest.mark.parametrize('classes', [7, 300, 1025, 2052])
+@pytest.mark.parametrize('kind', ['nan', 'inf', 'all -inf'])
+def test_sample_categorical_refuses_rows_without_a_distribution(K, classes, kind):
+    """As torch.multinomial does, wherever in the row and in whichever row the value stands."""
+    for at in (0, classes // 2, classes - 1):
+        logits = torch.randn(70, classes, device='cuda', generator=torch.Generator('cuda').manual_seed(1))
+        if kind == 'all -inf':
+            logits[at % 70] = float('-inf')
+        else:
+            logits[(7 * at) % 70, at] = float(kind)
+        with pytest.raises(RuntimeError, match='probability tensor contains'):
+            K.sample_categorical(logits)
+        targets, drawn = K.sample_categorical(logits, late=True)
+        with pytest.raises(RuntimeError, match='probability tensor contains'):
+            drawn.check()
+        assert int(targets.min()) >= 0 and int(targets.max()) < classes
+        assert drawn.check() == []
+    K.sample_categorical(torch.zeros(70, classes, device='cuda'))       # the word is clear again
+
+
 @pytest.mark.parametrize('f', [1, 256, 300])
 def test_unit_wise_keep_grouped(K, f):
     """Modules whose blocks are all zero keep their previous inverse or get the identity; the others are left alone."""

@@ -753,6 +753,44 @@ def test_tied_parameters_match_the_oracle(width, grouped, pi, monkeypatch):
             assert grad_close(p.grad, q.grad, 1e-3), (step, name)
 
 
+@pytest.mark.parametrize('ema,late', [(-1, False), (-1, True), (0.5, False)])
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+def test_sampled_fisher_of_a_diverged_model_raises(ema, late, value):
+    """Logits that are no distribution raise the error of the draw from forward_and_backward() (with late_inverse_flags from the
+    next reading of the flags), and without accumulated factors the next step is that of a maker that never saw them."""
+    torch.manual_seed(3)
+    model = nn.Sequential(nn.Linear(6, 20), nn.ReLU(), nn.Linear(20, 4)).cuda()
+    x, t = torch.randn(16, 6).cuda(), torch.randint(0, 4, (16,)).cuda()
+
+    def maker():
+        gm = KfacGradientMaker(model, PreconditioningConfig(data_size=16, damping=1e-2, ema_decay=ema), fisher_type=FISHER_MC, seed=1)
+        gm.late_inverse_flags = late
+        return gm
+
+    def step(gm, bias=0.0):
+        model.zero_grad(set_to_none=True)
+        with torch.no_grad():
+            saved = model[2].bias.clone()
+            model[2].bias[1] += bias
+        try:
+            gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x), t)
+            gm.forward_and_backward()
+            return [p.grad.clone() for p in model.parameters()]
+        finally:
+            with torch.no_grad():
+                model[2].bias.copy_(saved)
+    expected = step(maker())
+    gm = maker()
+    step(gm)
+    with pytest.raises(RuntimeError, match='probability tensor contains'):
+        step(gm, value)
+        gm.check_late_flags()
+    if ema == -1:
+        for a, b in zip(step(gm), expected):
+            assert torch.equal(a, b)
+        gm.check_late_flags()
+
+
 def test_identity_where_zero_touches_only_the_flagged_matrices():
     from asdl_amd import kernels as K
     outs = [torch.full((d, d), 7.0, device='cuda') for d in (5, 130, 64)]
