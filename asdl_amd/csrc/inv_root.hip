@@ -12,9 +12,9 @@
 //
 // Newton iteration.  M_0 = z S, X_0 = z^(1/p) I;  T = a I - b M;  X <- X T;  M <- T^p M.  The classical step a = 1 + 1/p,
 // b = 1/p raises a small eigenvalue of M by (1 + 1/p)^p = 2.44 (p = 4): 12 of its 18 steps on a statistic of condition 1e6.
-// With a lower bound l of the spectrum known (the ridge: l >= ridge_eps lambda_max / ||S||_F for z = 1 / ||S||_F, which
-// puts the spectrum into [l, 1]) the step that raises l most is a larger a with b = a^(p+1) p^p / (p+1)^(p+1), which
-// keeps max m (a - b m)^p = 1: up to 7.4 per step, 12 or 13 steps in all (root_schedule_kernel).
+// With a lower bound l of the spectrum known (from the Lanczos steps, at the least the ridge) the step that raises l most is a
+// larger a with b = a^(p+1) p^p / (p+1)^(p+1), which keeps max m (a - b m)^p = 1: up to 7.4 per step.  root_schedule_kernel
+// decides per matrix whether that is the shorter way.
 // The first kRootEarly steps stay classical, in the summation order of one fixed kernel per size.  What an ill-conditioned
 // root ends up with is decided there: the rounding of M' perturbs the smallest eigenvalues by about 5e-8, 1 to 2 % of the
 // root at condition 1e6, and every later step's perturbation counts 2.44 times less.  Another order, though as accurate, gives
@@ -103,7 +103,6 @@ struct RootState {
   float* err;       // current Newton error max|M - I|
   float* zscale;
   float* partial;   // [RCHUNKS]: sums of squares, then max |M_0 - I|
-  float* partial_tr;  // [RCHUNKS]: partial traces
   float* alpha;     // [kLanczosSteps] the tridiagonal matrix: diagonal,
   float* beta;      // [kLanczosSteps] and beta[j] next to alpha[j - 1], alpha[j]
   float* coef;      // [2 kRootSteps]: (a, b) of every step
@@ -340,36 +339,28 @@ static __global__ __launch_bounds__(64) void root_power_kernel(RootGroups G, int
   }
 }
 
-// grid (RCHUNKS, total): S += ridge I (in place), partial sum of squares and trace of the ridged matrix
+// grid (RCHUNKS, total): S += ridge I (in place), partial sum of squares of the ridged matrix
 static __global__ __launch_bounds__(256) void root_ridge_kernel(RootGroups G, float ridge_eps) {
-  __shared__ float red[2][4];
+  __shared__ float red[4];
   const int z = blockIdx.y;
   const RootGroup& g = G.g[root_group_of(G, z)];
   float* __restrict__ S = g.S + (z - g.z0) * g.strideS;
   const float ridge = ridge_eps * G.st.sv[z];
   const uint32_t total = static_cast<uint32_t>(g.n) * static_cast<uint32_t>(g.n), period = static_cast<uint32_t>(g.n) + 1;
-  float s = 0.f, t = 0.f;
+  float s = 0.f;
 #pragma unroll 4
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
     float x = S[i];
     if (i % period == 0) {
       x += ridge;
       S[i] = x;
-      t += x;
     }
     s += x * x;
   }
   s = wave_sum(s);
-  t = wave_sum(t);
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = s;
-    red[1][threadIdx.x >> 6] = t;
-  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    G.st.partial[z * RCHUNKS + blockIdx.x] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-    G.st.partial_tr[z * RCHUNKS + blockIdx.x] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
-  }
+  if (threadIdx.x == 0) G.st.partial[z * RCHUNKS + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 __device__ __forceinline__ float int_power(float x, int p) {
@@ -378,43 +369,81 @@ __device__ __forceinline__ float int_power(float x, int p) {
   return r;
 }
 
+// The smallest eigenvalue of T + ridge I (T: m Lanczos steps) within [lo, hi], from below and to 0.4 %; lo if it lies at or below
+// that.  x lies below the spectrum where every pivot of T + (ridge - x) I is positive (Sturm): two rounds of 64 values of x, one per
+// lane, in geometric progression.
+__device__ __forceinline__ float lowest_ritz(const float* __restrict__ alpha, const float* __restrict__ beta, int m, float ridge,
+                                             float lo, float hi) {
+  const int lane = threadIdx.x;
+#pragma unroll
+  for (int round = 0; round < 2; ++round) {
+    const float x = lo * powf(hi / lo, lane / 63.f);
+    bool below = true;
+    float d = 1.f;
+    for (int i = 0; i < m; ++i) {
+      const float c = i == 0 ? 0.f : beta[i];
+      d = (alpha[i] + ridge - x) - c * c / d;
+      below = below && d > 0.f;
+    }
+    const unsigned long long not_below = ~__ballot(below);
+    if (not_below == 0) return hi;
+    const int f = __ffsll(not_below) - 1;
+    if (f == 0) return lo;
+    hi = __shfl(x, f);
+    lo = __shfl(x, f - 1);
+  }
+  return lo;
+}
+
+// Classical steps after which an eigenvalue m of M lies within tol of one, counted from step `from`.
+__device__ __forceinline__ int classical_steps(float m, int p, float a0, float b0, float tol, int from) {
+  int k = from;
+  for (; k < 2 * kRootSteps && fabsf(m - 1.f) > tol; ++k) m *= int_power(a0 - b0 * m, p);
+  return k;
+}
+
 // grid (total), one wave: the scale z and the (a, b) of every step.
 //
-// Accelerated steps where they pay: with a ridge of 1e-7 and more (below, the bound l is not one that fp32 can keep), a
-// power up to 8, room for the classical iteration's own number of steps (a caller that asks for a few steps gets those
-// of the reference), and a statistic whose spectrum is spread: n ||S||_F^2 / tr(S)^2 = mean(lambda^2) / mean(lambda)^2 is
-// 1.3 for a well-conditioned sample covariance, whose eigenvalues the classical step brings together in 7 to 9 steps, fewer
-// than a schedule that has to assume l; 2 and more for the rank-deficient statistics of gradients.
+// Two schedules are followed on the ends of the spectrum as the Lanczos steps saw it (the Ritz values of T, the ridge added), and the
+// shorter one is used: the classical step throughout, or accelerated steps from a lower bound l of the spectrum.  l is half
+// the smallest Ritz value, at least half the ridge's bound (the estimate of lambda_max may be low, S indefinite by its rounding).
+// Too high a guess costs classical steps at the end, since eigenvalues below l rise faster than by the classical step too; too
+// low a guess (the ridge's bound for a full-rank statistic) costs accelerated steps that nothing needs.  Steps at n = 512, p = 4, a ridge
+// of 1e-6 (classical, from the ridge's bound throughout, by this rule): eigenvalues 1 ... 0.01 10, 14, 9; 1 ... 0.0001 15, 14, 12;
+// summed batches of 128 rows, one (rank 128) 20, 14, 14, four 20, 14, 17, five 12, 14, 10, ten 9, 14, 8, forty 7, 14, 7.
+// Accelerated steps also need a ridge of 1e-7 and more (below, the bound l is not one that fp32 can keep), a power up to 8, and room
+// for the classical iteration's own number of steps (a caller that asks for a few steps gets those of the reference).
+//
 // A step may not press the top of the spectrum below kTopMin: its rounding error relative to that value is what the root
 // inherits in the dominant directions (0.17: errors against fp64 at or below the classical iteration's on spectra of
 // condition 14 to 1e6; unlimited, 9 steps but 4e-4 instead of 1e-6 at condition 14).  T^p stays below 12 for the fp16 planes.
-static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, float ridge_eps, int max_iter) {
-  constexpr float kTopMin = 0.17f, kSpread = 1.6f, kEnd = 0.97f;
+static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, float ridge_eps, int max_iter, float tol, int lanczos_steps) {
+  constexpr float kTopMin = 0.17f, kEnd = 0.97f;
   const int z = blockIdx.x, lane = threadIdx.x;
   const RootGroup& g = G.g[root_group_of(G, z)];
   const int p = g.p;
-  const float part = G.st.partial[z * RCHUNKS + lane], tr = wave_sum(G.st.partial_tr[z * RCHUNKS + lane]);
+  const float part = G.st.partial[z * RCHUNKS + lane];
   float nrm2 = 0.f;
 #pragma unroll
   for (int c = 0; c < RCHUNKS; ++c) nrm2 += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, part), c));
-  const float sv = G.st.sv[z], zscale = (1.f + p) / (2.f * sqrtf(nrm2));
-  float* __restrict__ coef = G.st.coef + z * 2 * kRootSteps;
+  const float sv = G.st.sv[z], zscale = (1.f + p) / (2.f * sqrtf(nrm2)), ridge = ridge_eps * sv;
   const float a0 = 1.f + 1.f / p, b0 = 1.f / p;
+  float ca = a0, cb = b0;                      // of step `lane`
   int k = 0;
-  float l = 0.5f * ridge_eps * sv * zscale;    // half: the estimate of lambda_max may be low, S indefinite by its rounding
-  const bool fast = ridge_eps >= 1e-7f && p >= 2 && p <= 8 && max_iter >= kRootSteps && sv > 0.f &&
-                    g.n * nrm2 > kSpread * tr * tr && l > 1e-9f && l < kEnd;
-  if (fast) {
+  if (ridge_eps >= 1e-7f && p >= 2 && p <= 8 && max_iter >= kRootSteps && sv > 0.f && 0.5f * ridge * zscale > 1e-9f) {
+    const int dim = G.st.lz_dim[z];
+    const float low = lowest_ritz(G.st.alpha + z * kLanczosSteps, G.st.beta + z * kLanczosSteps, dim == 0 ? lanczos_steps : dim,
+                                  ridge, 0.5f * ridge, sv + ridge);
+    const float near = fmaxf(tol, 1e-6f);
+    const int classical = max(classical_steps(low * zscale, p, a0, b0, near, 0),
+                              classical_steps((sv + ridge) * zscale, p, a0, b0, near, 0));
+    float l = fmaxf(0.5f * low, 0.5f * ridge) * zscale;
     const float cp = int_power(static_cast<float>(p) / (p + 1), p) / (p + 1);       // b = cp a^(p+1)
     // the classical steps: the spectrum is in [l, (1 + p) / 2], and in (0, 1] after the first
     const float first = 0.5f * (1 + p) * int_power(a0 - b0 * 0.5f * (1 + p), p);
     for (; k < kRootEarly; ++k) {
       l *= int_power(a0 - b0 * l, p);
       if (k == 0) l = fminf(l, first);
-      if (lane == 0) {
-        coef[2 * k] = a0;
-        coef[2 * k + 1] = b0;
-      }
     }
     for (; k < kRootSteps - 1 && l < kEnd; ++k) {
       // the a in [1 + 1/p, 2.5] that maximises min(f(l), f(1)), f(m) = m (a - b m)^p: two rounds of 64 candidates
@@ -423,8 +452,8 @@ static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, 
       for (int round = 0; round < 2; ++round) {
         const float c = lo + (hi - lo) * (lane / 63.f);
         const float ap = int_power(c, p), b = cp * ap * c;
-        const float top = int_power(c - b, p), low = l * int_power(c - b * l, p);
-        const float value = c > b && ap <= 12.f && (top >= kTopMin || c == a0) ? fminf(top, low) : -1.f;
+        const float top = int_power(c - b, p), low_end = l * int_power(c - b * l, p);
+        const float value = c > b && ap <= 12.f && (top >= kTopMin || c == a0) ? fminf(top, low_end) : -1.f;
         const float best = wave_max(value);
         const int who = __ffsll(__ballot(value == best)) - 1;
         a = __shfl(c, who);
@@ -433,17 +462,23 @@ static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, 
         lo = fmaxf(a0, a - h);
         hi = a + h;
       }
-      if (lane == 0) {
-        coef[2 * k] = a;
-        coef[2 * k + 1] = cp * int_power(a, p) * a;
-      }
       if (!(v > l)) break;
+      if (lane == k) {
+        ca = a;
+        cb = cp * int_power(a, p) * a;
+      }
       l = v;
     }
+    if (classical_steps(l, p, a0, b0, near, k) >= classical) {
+      k = 0;
+      ca = a0;
+      cb = b0;
+    }
   }
-  for (int i = k + lane; i < kRootSteps; i += 64) {
-    coef[2 * i] = a0;
-    coef[2 * i + 1] = b0;
+  float* __restrict__ coef = G.st.coef + z * 2 * kRootSteps;
+  if (lane < kRootSteps) {
+    coef[2 * lane] = ca;
+    coef[2 * lane + 1] = cb;
   }
   if (lane == 0) {
     G.st.accel[z] = k;
@@ -850,7 +885,7 @@ static int root_ops(int p, RootOp (*slots)[2], int* counts, int max_slots) {
 }
 
 static size_t root_state_floats(int total) {
-  return static_cast<size_t>(total) * (3 + 2 * RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 16;
+  return static_cast<size_t>(total) * (3 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 16;
 }
 static size_t root_group_floats(int64_t n, int64_t batch) {
   const size_t m = (static_cast<size_t>(batch) * root_matrix_floats(n, batch) + 63) / 64 * 64;
@@ -901,7 +936,7 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
     for (int j = 0; j < steps; ++j) hipLaunchKernelGGL(root_lanczos_kernel, dim3(blocks), b256, lds, s, G.st, L, j);
     hipLaunchKernelGGL(root_power_kernel, gz, b64, 0, s, G, steps, power_tol, max_power_iter);
     hipLaunchKernelGGL(root_ridge_kernel, gc, b256, 0, s, G, ridge_eps);
-    hipLaunchKernelGGL(root_schedule_kernel, gz, b64, 0, s, G, ridge_eps, max_iter);
+    hipLaunchKernelGGL(root_schedule_kernel, gz, b64, 0, s, G, ridge_eps, max_iter, tol, steps);
     bool fp32 = false;
     for (int i = 0; i < G.count; ++i) {
       const RootGroup& g = G.g[i];
@@ -1049,7 +1084,6 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
   st.zscale = floats(total);
   st.errword = floats(static_cast<int64_t>(total) * kErrStride);
   st.partial = floats(static_cast<int64_t>(total) * RCHUNKS);
-  st.partial_tr = floats(static_cast<int64_t>(total) * RCHUNKS);
   st.alpha = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.beta = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.coef = floats(static_cast<int64_t>(total) * 2 * kRootSteps);

@@ -123,6 +123,59 @@ def test_inv_root_group_of_several_sizes(groups):
             assert relerr(root[b], _closed_form_root(S[b], p)) < 1e-3, (n, p, b)
 
 
+def _classical_root_steps(S, p, ridge, tol=1e-6):
+    """Steps of the reference's iteration (asdl/precondition/shampoo.py:508-521) by its effect on the eigenvalues, in 64 bits."""
+    ev = torch.linalg.eigvalsh(S.double()).clamp_min(0.0)
+    ev = ev + ridge * ev[-1]
+    m = ev * (1 + p) / (2 * ev.norm())
+    steps = 0
+    while float((m - 1).abs().max()) > tol:
+        m = m * (1 + 1 / p - m / p) ** p
+        steps += 1
+    return steps
+
+
+def _with_eigenvalues(ev, g):
+    """A symmetric matrix with these eigenvalues: three random reflections of the diagonal one."""
+    S = torch.diag(ev.double())
+    for _ in range(3):
+        v = torch.randn(len(ev), generator=g, dtype=torch.float64, device=ev.device)
+        v /= v.norm()
+        Sv = S @ v
+        S = S - 2 * torch.outer(v, Sv) - 2 * torch.outer(Sv, v) + 4 * (v @ Sv) * torch.outer(v, v)
+    return ((S + S.T) / 2).float()
+
+
+@pytest.mark.parametrize('p', [2, 4, 8])
+@pytest.mark.parametrize('kind', ['1 to 0.01', '1 to 0.0001', 'few tiny', 'rank 1/4', '3 batches', '10 batches', '40 batches'])
+@pytest.mark.parametrize('n', [130, 512, 3072])
+def test_inv_root_takes_no_more_steps_than_the_classical_iteration(n, kind, p):
+    """Full-rank statistics (summed over several batches of n / 4 rows, or with given eigenvalues) as well as rank-deficient ones:
+    the schedule comes from the spectrum."""
+    if n == 3072 and (p != 4 or kind not in ('1 to 0.01', 'rank 1/4')):
+        pytest.skip('one power and the two ends of the range at the largest size')
+    g = torch.Generator('cuda').manual_seed(n)
+    if 'batches' in kind or 'rank' in kind:
+        rows = n // 4 * (int(kind.split()[0]) if 'batches' in kind else 1)
+        X = torch.randn(rows, n, generator=g, device='cuda')
+        S = X.T @ X
+    else:
+        low = -4 if '0.0001' in kind else -2
+        ev = torch.logspace(0, low, n, device='cuda')
+        if kind == 'few tiny':
+            ev[-3:] = 1e-7
+        S = _with_eigenvalues(ev, g)
+    v0 = torch.rand(1, n, generator=g, device='cuda') * 2 - 1
+    classical = _classical_root_steps(S, p, 1e-6)
+    print(f'inv_root steps n={n} {kind} p={p}: classical {classical}', flush=True)
+    root, stats = K.inv_root_newton(S.unsqueeze(0).clone(), p, 1e-6, v0)
+    steps, error = int(stats[0, 2]), float(stats[0, 3])
+    print(f'  here {steps}', flush=True)
+    assert error <= 1e-6 and steps <= classical, (steps, classical)
+    if kind in ('rank 1/4', 'few tiny'):
+        assert steps < classical - 2, (steps, classical)
+
+
 def test_inv_root_polled_and_unpolled_enqueue_give_the_same_result():
     """The host may stop enqueuing Newton iterations once the convergence flags are all zero (read every few
     iterations) or enqueue all of them blindly: bit-equal roots and the same iteration counts."""
