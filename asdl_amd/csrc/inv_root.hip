@@ -19,8 +19,7 @@
 // root ends up with is decided there: the rounding of M' perturbs the smallest eigenvalues by about 5e-8, 1 to 2 % of the
 // root at condition 1e6, and every later step's perturbation counts 2.44 times less.  Another order, though as accurate, gives
 // another root within that percent; rank-deficient statistics of 625 to 1498 columns differ from the root of the wholly
-// classical iteration by 0.6 to 0.9 % after three classical steps, by 0.12 to 0.17 % after five (a fourteenth step; 24 x 3072:
-// 112 -> 121 ms).
+// classical iteration by 0.6 to 0.9 % after three classical steps, by 0.12 to 0.17 % after five (one step more).
 //
 // The matrices of the iteration, all polynomials of one symmetric matrix, are kept
 //  * as 16-bit planes from 512 columns up (gemm_planes.hpp), of which only tiles on one side of the diagonal are computed,
@@ -409,16 +408,20 @@ __device__ __forceinline__ int classical_steps(float m, int p, float a0, float b
 // the smallest Ritz value, at least half the ridge's bound (the estimate of lambda_max may be low, S indefinite by its rounding).
 // Too high a guess costs classical steps at the end, since eigenvalues below l rise faster than by the classical step too; too
 // low a guess (the ridge's bound for a full-rank statistic) costs accelerated steps that nothing needs.  Steps at n = 512, p = 4, a ridge
-// of 1e-6 (classical, from the ridge's bound throughout, by this rule): eigenvalues 1 ... 0.01 10, 14, 9; 1 ... 0.0001 15, 14, 12;
-// summed batches of 128 rows, one (rank 128) 20, 14, 14, four 20, 14, 17, five 12, 14, 10, ten 9, 14, 8, forty 7, 14, 7.
+// of 1e-6 (classical, from the ridge's bound throughout, by this rule): eigenvalues 1 ... 0.01 10, 15, 9; 1 ... 0.0001 15, 15, 13;
+// summed batches of 128 rows, one (rank 128) 20, 15, 15, four 20, 15, 18, five 12, 15, 10, ten 9, 15, 8, forty 7, 15, 7.
 // Accelerated steps also need a ridge of 1e-7 and more (below, the bound l is not one that fp32 can keep), a power up to 8, and room
 // for the classical iteration's own number of steps (a caller that asks for a few steps gets those of the reference).
 //
-// A step may not press the top of the spectrum below kTopMin: its rounding error relative to that value is what the root
-// inherits in the dominant directions (0.17: errors against fp64 at or below the classical iteration's on spectra of
-// condition 14 to 1e6; unlimited, 9 steps but 4e-4 instead of 1e-6 at condition 14).  T^p stays below 12 for the fp16 planes.
+// A step may not press the top of the spectrum below kTopMin: its rounding error relative to that value is what the root inherits
+// in the dominant directions, the ones that a gradient with this statistic lies in (the error of the whole root does not show
+// it: that is the null space's, 1 to 2 % whatever the steps).  Error against fp64 of L^(-1/4) G R^(-1/4), L = G G^T, R = G^T G, and
+// steps, for the classical iteration and kTopMin = 0.17, 0.5, 0.6, 0.7: G 512 x 784 of rank 128 5.6e-5 (20), 1.9e-4 (14), 8.3e-5 (15),
+// 6.5e-5 (15), 5.1e-5 (15); 256 x 300, rank 64 6.6e-5 (20), 2.0e-4 (14), 7.8e-5 (14), 6.4e-5 (15), 5.8e-5 (15); 300 x 600, rank 16
+// 1.2e-4 (20), 2.8e-4 (13), 1.5e-4 (14), 1.3e-4 (14), 1.3e-4 (15); 768 x 3072, rank 400 4.9e-5 (21), 1.3e-4 (14), 6.1e-5 (15),
+// 5.4e-5 (15), 4.6e-5 (16).  0.7 is the first that loses nothing.  T^p stays below 12 for the fp16 planes.
 static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, float ridge_eps, int max_iter, float tol, int lanczos_steps) {
-  constexpr float kTopMin = 0.17f, kEnd = 0.97f;
+  constexpr float kTopMin = 0.7f, kEnd = 0.97f;
   const int z = blockIdx.x, lane = threadIdx.x;
   const RootGroup& g = G.g[root_group_of(G, z)];
   const int p = g.p;
