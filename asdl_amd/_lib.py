@@ -89,7 +89,7 @@ _SIGNATURES = {
     'ak_inv_root_newton': (c_int, [c_ptr, c_i64, c_int, c_i64, c_int, c_f32, c_ptr, c_int, c_f32, c_int, c_f32,
                                    c_ptr, c_i64, c_ptr, c_ptr, c_size, c_ptr]),
     'ak_inv_root_active_offset': (c_size, [c_i64, c_int]),
-    'ak_inv_root_group_ws_bytes': (c_size, [c_ptr, c_ptr, c_int]),
+    'ak_inv_root_group_ws_bytes': (c_size, [c_ptr, c_ptr, c_ptr, c_f32, c_int]),
     'ak_inv_root_group_active_offset': (c_size, [c_ptr, c_ptr, c_int]),
     'ak_inv_root_group': (c_int, [c_int, c_int, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_f32, c_ptr, c_int, c_f32,
                                   c_int, c_f32, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr]),

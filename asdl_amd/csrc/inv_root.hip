@@ -45,7 +45,7 @@ constexpr int kLanczosSteps = 32;
 constexpr int kLanczosRows = 16;        // rows of the statistic per work group and step: four waves, four rows each
 constexpr int kRootEarly = 5;           // classical steps before the accelerated ones
 constexpr int kRootSteps = 32;          // entries of a matrix's step table; the last one repeats
-constexpr int kRootBuffers = 10;        // R0 R1 M0 M1 T0 T1 and four product buffers
+constexpr int kRootFixedBuffers = 6;    // R0 R1 M0 M1 T0 T1; product buffers behind them (root_buffers)
 constexpr int kRootMinPlaneDim = 512;
 
 // Scales of the two-plane fp16 form (gemm_planes.hpp).  M, the polynomials T and their powers are bounded by the
@@ -89,11 +89,16 @@ static int root_plane_tile(int64_t n, int64_t batch) {
   return us_small < us_big ? kPlaneSmallTile : kPlaneTile;
 }
 
-// floats of the matrix buffers of one statistic: plane sets of 3 n_pad^2 16-bit values, or fp32 matrices
-static size_t root_matrix_floats(int64_t n, int64_t batch) {
-  if (!root_plane_dim(n)) return static_cast<size_t>(kRootBuffers) * n * root_ld(n);
+// Storage of the matrices of a group: 0 (fp32), 2 or 3 planes.
+static int root_planes(int64_t n, int p, float ridge_eps) {
+  return !root_plane_dim(n) ? 0 : (root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3);
+}
+
+// floats of one matrix buffer of a statistic
+static size_t root_buffer_floats(int64_t n, int64_t batch, int np) {
+  if (np == 0) return static_cast<size_t>(n) * root_ld(n);
   const size_t n_pad = static_cast<size_t>(root_pad(n, root_plane_tile(n, batch)));
-  return kRootBuffers * 3 * n_pad * n_pad / 2;
+  return np * n_pad * n_pad / 2;
 }
 
 struct RootState {
@@ -119,10 +124,10 @@ struct RootGroup {
   float* out;
   const float* v0;
   float* stats;
-  float* bufs;          // kRootBuffers buffers of `batch` fp32 matrices (n rows of ld) or plane sets
+  float* bufs;          // `buffers` buffers of `batch` fp32 matrices (n rows of ld) or plane sets
   float* vec;           // Lanczos vectors: q ring of 3, S q ring of 2, each [batch, n]
   int64_t strideS, strideOut;
-  int n, ld, batch, p;
+  int n, ld, batch, p, buffers;
   int z0;               // first matrix of the group in the state arrays
   int np, n_pad, tile;  // planes per matrix: 0 (fp32), 2, 3; tile of the products on planes
   float scale_r;
@@ -515,7 +520,7 @@ static __global__ __launch_bounds__(256) void root_start_kernel(RootGroups G) {
       base[2 * buf + at] = m;
       base[4 * buf + at] = t;
       if (!inside)                             // no product writes the padding columns
-        for (int k = 0; k < kRootBuffers; ++k) base[k * buf + at] = 0.f;
+        for (int k = 0; k < g.buffers; ++k) base[k * buf + at] = 0.f;
       if (inside) e = fmaxf(e, fabsf(m - (diag ? 1.f : 0.f)));
     }
   }
@@ -843,6 +848,7 @@ static __global__ __launch_bounds__(256, 2) void root_small_kernel(RootState st,
 // ---- host ----------------------------------------------------------------------------------------------------------
 
 enum RootBuf { R0 = 0, M0 = 2, T0 = 4, B0 = 6 };
+constexpr int kRootMaxSlots = 64;
 constexpr PairedBuf kRin{R0, 1}, kRout{R0, 2}, kMin{M0, 1}, kMout{M0, 2}, kTin{T0, 1}, kTout{T0, 2}, kNone{-1, 0};
 
 struct RootOp { PairedBuf a, b, c, c2; };
@@ -887,12 +893,27 @@ static int root_ops(int p, RootOp (*slots)[2], int* counts, int max_slots) {
   return n;
 }
 
-static size_t root_state_floats(int total) {
-  return static_cast<size_t>(total) * (3 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 16;
+// Buffers that the products of power p need: the fixed ones and the product buffers that root_ops() names.  0: p has too many steps.
+static int root_buffers(int p) {
+  RootOp slots[kRootMaxSlots][2];
+  int counts[kRootMaxSlots];
+  const int n = root_ops(p, slots, counts, kRootMaxSlots);
+  int most = kRootFixedBuffers;
+  for (int k = 0; k < n; ++k)
+    for (int o = 0; o < counts[k]; ++o)
+      if (slots[k][o].c.sel == 0) most = std::max(most, slots[k][o].c.index + 1);
+  return n < 0 ? 0 : most;
 }
-static size_t root_group_floats(int64_t n, int64_t batch) {
-  const size_t m = (static_cast<size_t>(batch) * root_matrix_floats(n, batch) + 63) / 64 * 64;
-  return m + (static_cast<size_t>(5) * batch * n + 63) / 64 * 64;
+
+static size_t root_state_floats(int total) {
+  return (static_cast<size_t>(total) * (3 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 63) / 64 * 64;
+}
+// matrix buffers and Lanczos vectors of a group
+static size_t root_group_matrix_floats(int64_t n, int64_t batch, int np, int buffers) {
+  return (static_cast<size_t>(batch) * buffers * root_buffer_floats(n, batch, np) + 63) / 64 * 64;
+}
+static size_t root_group_floats(int64_t n, int64_t batch, int np, int buffers) {
+  return root_group_matrix_floats(n, batch, np, buffers) + (static_cast<size_t>(5) * batch * n + 63) / 64 * 64;
 }
 static bool root_args_ok(const int64_t* n, const int* batch, int groups) {
   if (n == nullptr || batch == nullptr || groups <= 0 || groups > kRootMaxGroups) return false;
@@ -903,13 +924,6 @@ static bool root_args_ok(const int64_t* n, const int* batch, int groups) {
   }
   return total <= 65535;
 }
-// bytes from the workspace's start to the `active` words
-static size_t root_active_offset(const int64_t* n, const int* batch, int groups) {
-  size_t off = 0;
-  for (int i = 0; i < groups; ++i) off += root_group_floats(n[i], batch[i]);
-  return off * sizeof(float);
-}
-
 // phases: 1 = power iteration, ridge and start of the Newton iteration; 2 = `iters` Newton iterations; 4 = results and
 // statistics
 static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int max_power_iter, float power_tol, int max_iter,
@@ -952,11 +966,10 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
     hipLaunchKernelGGL(root_begin_kernel, gz, b64, 0, s, G.st, tol, max_iter);
   }
   if (phases & 2) {
-    constexpr int kMaxSlots = 64;
-    RootOp slots[kRootMaxGroups][kMaxSlots][2];
-    int counts[kRootMaxGroups][kMaxSlots], nslots[kRootMaxGroups], most = 0;
+    RootOp slots[kRootMaxGroups][kRootMaxSlots][2];
+    int counts[kRootMaxGroups][kRootMaxSlots], nslots[kRootMaxGroups], most = 0;
     for (int i = 0; i < G.count; ++i) {
-      nslots[i] = root_ops(G.g[i].p, slots[i], counts[i], kMaxSlots);
+      nslots[i] = root_ops(G.g[i].p, slots[i], counts[i], kRootMaxSlots);
       if (nslots[i] < 0) return AK_ERR_ARG;
       most = std::max(most, nslots[i]);
     }
@@ -1027,16 +1040,21 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
 
 }  // namespace ak
 
-extern "C" size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, int groups) {
-  if (!ak::root_args_ok(n, batch, groups)) return 0;
+// Workspace: the state of all matrices (the `active` words first), then the matrices of each group.
+extern "C" size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, const int* p, float ridge_eps, int groups) {
+  if (!ak::root_args_ok(n, batch, groups) || p == nullptr) return 0;
+  size_t floats = 0;
   int total = 0;
-  for (int i = 0; i < groups; ++i) total += batch[i];
-  return ak::root_active_offset(n, batch, groups) + ak::root_state_floats(total) * sizeof(float);
+  for (int i = 0; i < groups; ++i) {
+    const int buffers = p[i] >= 1 ? ak::root_buffers(p[i]) : 0;
+    if (buffers == 0) return 0;
+    floats += ak::root_group_floats(n[i], batch[i], ak::root_planes(n[i], p[i], ridge_eps), buffers);
+    total += batch[i];
+  }
+  return (ak::root_state_floats(total) + floats) * sizeof(float);
 }
 
-extern "C" size_t ak_inv_root_group_active_offset(const int64_t* n, const int* batch, int groups) {
-  return ak::root_args_ok(n, batch, groups) ? ak::root_active_offset(n, batch, groups) : 0;
-}
+extern "C" size_t ak_inv_root_group_active_offset(const int64_t*, const int*, int) { return 0; }
 
 extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const* S, const int64_t* n,
                                  const int* batch, const int64_t* strideS, const int* p, float ridge_eps,
@@ -1047,11 +1065,15 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
   if (phases < 1 || phases > 7 || iters < 0 || S == nullptr || strideS == nullptr ||
       p == nullptr || v0 == nullptr || out == nullptr || strideOut == nullptr || stats == nullptr || !root_args_ok(n, batch, groups))
     return AK_ERR_ARG;
-  if (ws == nullptr || ws_bytes < ak_inv_root_group_ws_bytes(n, batch, groups)) return AK_ERR_WORKSPACE;
+  const size_t need = ak_inv_root_group_ws_bytes(n, batch, p, ridge_eps, groups);
+  if (need == 0) return AK_ERR_ARG;
+  if (ws == nullptr || ws_bytes < need) return AK_ERR_WORKSPACE;
   RootGroups G;
   G.count = groups;
   G.total = 0;
-  float* w = static_cast<float*>(ws);
+  int total = 0;
+  for (int i = 0; i < groups; ++i) total += batch[i];
+  float* w = static_cast<float*>(ws) + root_state_floats(total);
   for (int i = 0; i < groups; ++i) {
     if (S[i] == nullptr || v0[i] == nullptr || out[i] == nullptr || stats[i] == nullptr || n[i] < 2 || p[i] < 1 ||
         strideS[i] < n[i] * n[i] || strideOut[i] < n[i] * n[i])
@@ -1066,13 +1088,14 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
     // two fp16 planes where the ridge bounds the root, else three bf16 planes; every part of a computation in parts gets
     // the same arguments, hence the same answer
     g.scale_r = root_fp16_scale(n[i], p[i], ridge_eps);
-    g.np = !root_plane_dim(n[i]) ? 0 : (g.scale_r > 0.f ? 2 : 3);
+    g.np = root_planes(n[i], p[i], ridge_eps);
+    g.buffers = root_buffers(p[i]);
     g.bufs = w;
-    g.vec = w + (static_cast<size_t>(batch[i]) * root_matrix_floats(n[i], batch[i]) + 63) / 64 * 64;
-    w += root_group_floats(n[i], batch[i]);
+    g.vec = w + root_group_matrix_floats(n[i], batch[i], g.np, g.buffers);
+    w += root_group_floats(n[i], batch[i], g.np, g.buffers);
     G.total += batch[i];
   }
-  const int total = G.total;
+  w = static_cast<float*>(ws);
   RootState& st = G.st;
   auto ints = [&](int k) { int* r = reinterpret_cast<int*>(w); w += k; return r; };
   auto floats = [&](int64_t k) { float* r = w; w += k; return r; };
@@ -1099,7 +1122,12 @@ extern "C" int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps) {
   return ak::root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3;
 }
 
-extern "C" size_t ak_inv_root_ws_bytes(int64_t n, int batch) { return ak_inv_root_group_ws_bytes(&n, &batch, 1); }
+// (for any power and ridge: three planes, four product buffers)
+extern "C" size_t ak_inv_root_ws_bytes(int64_t n, int batch) {
+  if (!ak::root_args_ok(&n, &batch, 1)) return 0;
+  const int np = ak::root_plane_dim(n) ? 3 : 0;
+  return (ak::root_state_floats(batch) + ak::root_group_floats(n, batch, np, ak::kRootFixedBuffers + 4)) * sizeof(float);
+}
 
 extern "C" int ak_inv_root_newton(float* S, int64_t n, int batch, int64_t strideS, int p, float ridge_eps,
                                   const float* v0, int max_power_iter, float power_tol, int max_iter, float tol,
@@ -1109,7 +1137,7 @@ extern "C" int ak_inv_root_newton(float* S, int64_t n, int batch, int64_t stride
                            max_iter, tol, &out, &strideOut, &stats, ws, ws_bytes, stream);
 }
 
-extern "C" size_t ak_inv_root_active_offset(int64_t n, int batch) { return ak_inv_root_group_active_offset(&n, &batch, 1); }
+extern "C" size_t ak_inv_root_active_offset(int64_t, int) { return 0; }
 
 extern "C" int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batch, int64_t strideS, int p,
                                        float ridge_eps, const float* v0, int max_power_iter, float power_tol,

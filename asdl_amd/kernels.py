@@ -176,6 +176,13 @@ def workspace(nbytes, device):
     return buf, buf.numel()
 
 
+def release_workspaces():
+    """Gives the scratch buffers of all streams back to the caching allocator; the next calls allocate them again.  (Launches that
+    still use one are safe: see workspace().  Plans that hold a buffer keep it.)"""
+    with _ws_lock:
+        _workspaces.clear()
+
+
 def _ws_args(nbytes, device):
     buf, size = workspace(nbytes, device)
     if buf is None:
@@ -1699,7 +1706,7 @@ def inv_root_group(items, ridge_eps, max_power_iter=100, power_tol=1e-6, max_ite
     S_a, n_a, b_a, sS, p_a, v_a, o_a, sO, st_a = (i64(*col[0]), i64(*col[1]), i32(*col[2]), i64(*col[3]), i32(*col[4]),
                                                   i64(*col[5]), i64(*col[6]), i64(*col[7]), i64(*col[8]))
     lib = _lib.load()
-    ws, ws_bytes, keep = _ws_args(lib.ak_inv_root_group_ws_bytes(n_a, b_a, count), dev)
+    ws, ws_bytes, keep = _ws_args(lib.ak_inv_root_group_ws_bytes(n_a, b_a, p_a, float(ridge_eps), count), dev)
 
     def run(phases, iters):
         _lib.check(lib.ak_inv_root_group(phases, iters, count, S_a, n_a, b_a, sS, p_a, float(ridge_eps), v_a,

@@ -403,7 +403,8 @@ int ak_kron_precond_static(const float* Binv, const float* Ainv, float* G, int64
  * eigenvalue, (ridge_eps (1 + p) / (2 sqrt(n)))^(-1/p), below 4096 and p <= 8; else three bf16 planes (the exact split
  * of the fp32 value, six matrix instructions).  ak_inv_root_plane_format tells which: 0 = fp32 matrices (n < 512),
  * 2, 3.  The environment variable ASDL_AMD_ROOT_FP16_PLANES=0 (read once) keeps every statistic on bf16 planes.
- * ak_inv_root_ws_bytes is 60 bytes per padded element and statistic on planes, 40 per element below that size.
+ * ak_inv_root_ws_bytes is enough for any power and ridge: 60 bytes per padded element and statistic on planes, 40 per element
+ * below that size (ak_inv_root_group_ws_bytes says what one call needs: 32 and 32 for p = 4 on two planes).
  * Replaces ComputePower / PowerIter / MatPower (asdl/precondition/shampoo.py:465-586). */
 size_t ak_inv_root_ws_bytes(int64_t n, int batch);
 int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps);
@@ -428,8 +429,9 @@ int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batc
 
 /* Several groups of statistics in one launch sequence (group i: batch[i] matrices of size n[i], power p[i]; all arrays on
  * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 32768).  Same phases.  The
- * `active` words of all matrices, group after group, start at ws + ak_inv_root_group_active_offset(). */
-size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, int groups);
+ * `active` words of all matrices, group after group, start at ws + ak_inv_root_group_active_offset().  The workspace is the sum over
+ * the groups of what their sizes, powers and the ridge need (0: the arguments are not accepted). */
+size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, const int* p, float ridge_eps, int groups);
 size_t ak_inv_root_group_active_offset(const int64_t* n, const int* batch, int groups);
 int ak_inv_root_group(int phases, int iters, int groups, float* const* S, const int64_t* n, const int* batch,
                       const int64_t* strideS, const int* p, float ridge_eps, const float* const* v0, int max_power_iter,

@@ -65,6 +65,22 @@ def test_no_hot_kernel_spills_registers():
     assert not spilled, spilled
 
 
+def test_root_workspace_of_a_call_over_all_sizes_is_below_that_of_its_largest_group():
+    """A call takes the roots of all sizes at once, so its workspace is a sum.  For a twelve-layer decoder of 768 columns it has to stay
+    below the bound for the largest group alone, which holds for any power."""
+    import ctypes
+    from asdl_amd import _lib
+    lib = _lib.load()
+    groups = [(768, 61), (2304, 12), (3072, 24), (1024, 1)]
+    count = len(groups)
+    n, batch, p = (ctypes.c_int64 * count)(*(g[0] for g in groups)), (ctypes.c_int * count)(*(g[1] for g in groups)), (ctypes.c_int * count)(*[4] * count)
+    need = lib.ak_inv_root_group_ws_bytes(n, batch, p, 1e-6, count)
+    assert 0 < need < lib.ak_inv_root_ws_bytes(3072, 24), need
+    for n1, b1, p1, eps in ((3072, 24, 4, 1e-6), (3072, 24, 4, 0.0), (600, 3, 7, 1e-6), (130, 2, 11, 1e-6), (2, 1, 1, 1e-6)):
+        one = lib.ak_inv_root_group_ws_bytes(ctypes.byref(ctypes.c_int64(n1)), ctypes.byref(ctypes.c_int(b1)), ctypes.byref(ctypes.c_int(p1)), eps, 1)
+        assert 0 < one <= lib.ak_inv_root_ws_bytes(n1, b1)
+
+
 def test_product_refuses_cpu_tensors():
     from asdl_amd import kernels
     with pytest.raises(RuntimeError, match='ROCm device'):
@@ -669,7 +685,9 @@ def test_workspace_belongs_to_the_stream_whose_launches_use_it(monkeypatch):
     with kernels.launches_on(side):
         for nbytes in (1 << 20, 1 << 22):
             kernels.workspace(nbytes, torch.device('cpu', 0))
-    assert allocated == [side, side]
+    assert allocated == [side, side] and len(kernels._workspaces) == 1
+    kernels.release_workspaces()
+    assert not kernels._workspaces
 
 
 def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):

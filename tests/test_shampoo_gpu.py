@@ -201,6 +201,33 @@ def test_inv_root_is_as_good_as_the_classical_one_where_the_gradient_lies(m, n, 
     assert here <= 1.3 * classical
 
 
+@pytest.mark.parametrize('groups,ridge', [
+    (((2, 1, 1), (65, 3, 2), (130, 4, 1), (33, 5, 3), (40, 7, 1), (64, 11, 1)), 1e-6),
+    (((512, 4, 1), (600, 2, 2), (577, 7, 1), (300, 8, 2), (520, 10, 1)), 1e-6),
+    (((513, 4, 45), (20, 6, 2)), 1e-6),
+    (((520, 4, 1), (600, 3, 2)), 0.0),
+])
+def test_inv_root_stays_within_its_workspace(groups, ridge, monkeypatch):
+    """Storage by size, power and ridge: as many bytes again behind the workspace stay as they were, and the roots are right."""
+    g = torch.Generator().manual_seed(9)
+    items = []
+    for n, p, batch in groups:
+        X = torch.randn(batch, 3 * n, n, generator=g)
+        items.append(((X.transpose(1, 2) @ X / (3 * n)).cuda(), p, (torch.rand(batch, n, generator=g) * 2 - 1).cuda(), None))
+    made = []
+
+    def workspace(nbytes, device):
+        made.append((torch.full((2 * nbytes + 512,), 0xA5, dtype=torch.uint8, device=device), nbytes))
+        return made[-1][0][:nbytes], nbytes
+
+    monkeypatch.setattr(K, 'workspace', workspace)
+    results = K.inv_root_group(items, ridge)
+    (buf, nbytes), = made
+    assert torch.all(buf[nbytes:] == 0xA5)
+    for (S, p, _, _), (root, _) in zip(items, results):
+        assert relerr(root[0], _closed_form_root(S[0], p)) < 1e-3, (S.shape, p)
+
+
 def test_inv_root_polled_and_unpolled_enqueue_give_the_same_result():
     """The host may stop enqueuing Newton iterations once the convergence flags are all zero (read every few
     iterations) or enqueue all of them blindly: bit-equal roots and the same iteration counts."""
