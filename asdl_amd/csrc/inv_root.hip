@@ -42,6 +42,7 @@ namespace ak {
 constexpr int RCHUNKS = 64;             // partial-reduction chunks per matrix
 constexpr int kRootMaxGroups = 16;      // groups of one call (they travel in the kernel arguments)
 constexpr int kLanczosSteps = 32;
+constexpr int kLanczosLdsDim = 32768;  // columns whose vector is kept in the LDS (128 of its 160 KB)
 constexpr int kLanczosRows = 16;        // rows of the statistic per work group and step: four waves, four rows each
 constexpr int kRootEarly = 5;           // classical steps before the accelerated ones
 constexpr int kRootSteps = 32;          // entries of a matrix's step table; the last one repeats
@@ -180,6 +181,8 @@ struct LanczosGroups {
 // itself in the LDS (three vectors from the L2, two reductions): one launch per step, no hand-over inside it.  The
 // rows of S are requested before that, their first 1024 columns kept in registers.
 // Bound by the launch and the chain of loads and reductions for small n, by reading S for a full batch.
+// WIDE: vectors that the LDS does not hold (kLanczosLdsDim) are formed again, element by element, where they are used.
+template <bool WIDE>
 static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, LanczosGroups L, int j) {
   extern __shared__ __attribute__((aligned(16))) float q[];
   __shared__ float red[3][4];
@@ -203,19 +206,33 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     }
   const int64_t vec = static_cast<int64_t>(g.batch) * n;
   float* __restrict__ qj = g.vec + (j % 3) * vec + static_cast<int64_t>(zl) * n;
-  if (j == 0) {
-    const float* __restrict__ v0 = g.v0 + static_cast<int64_t>(zl) * n;
+  const float* __restrict__ v0 = g.v0 + static_cast<int64_t>(zl) * n;
+  const float* __restrict__ q1 = g.vec + ((j + 2) % 3) * vec + static_cast<int64_t>(zl) * n;
+  const float* __restrict__ q2 = g.vec + ((j + 1) % 3) * vec + static_cast<int64_t>(zl) * n;
+  const float* __restrict__ w = g.vec + (3 + ((j + 1) & 1)) * vec + static_cast<int64_t>(zl) * n;
+  float a = 0.f, b = 0.f, inv = 0.f;
+  auto raw = [&](int i) { return j == 0 ? v0[i] : w[i] - a * q1[i] - (j > 1 ? b * q2[i] : 0.f); };     // q_j without its scale
+  auto form = [&](float* sums) {                      // the vector (WIDE: nothing) and its length
     float s = 0.f;
     for (int i = tid; i < n; i += 256) {
-      const float x = v0[i];
-      q[i] = x;
+      const float x = raw(i);
+      if constexpr (!WIDE) q[i] = x;
       s += x * x;
     }
-    const float inv = 1.f / sqrtf(block_sum(s, red[0]));
+    return sqrtf(block_sum(s, sums));
+  };
+  auto scale = [&] {
     for (int i = tid; i < n; i += 256) {
-      q[i] *= inv;
-      if (part == 0) qj[i] = q[i];
+      if constexpr (!WIDE) q[i] *= inv;
+      if (part == 0) {
+        if constexpr (WIDE) qj[i] = raw(i) * inv;
+        else qj[i] = q[i];
+      }
     }
+  };
+  if (j == 0) {
+    inv = 1.f / form(red[0]);
+    scale();
     if (part == 0 && tid == 0) {
       st.lz_dim[z] = 0;
       st.active[z] = st.count[z] = st.ovf[z] = 0;
@@ -224,20 +241,11 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     }
   } else {
     if (j > 1 && st.lz_dim[z] != 0) return;            // an invariant subspace: T is complete
-    const float* __restrict__ q1 = g.vec + ((j + 2) % 3) * vec + static_cast<int64_t>(zl) * n;
-    const float* __restrict__ q2 = g.vec + ((j + 1) % 3) * vec + static_cast<int64_t>(zl) * n;
-    const float* __restrict__ w = g.vec + (3 + ((j + 1) & 1)) * vec + static_cast<int64_t>(zl) * n;
-    const float b = st.beta[z * kLanczosSteps + j - 1];
+    b = st.beta[z * kLanczosSteps + j - 1];
     float s = 0.f;
     for (int i = tid; i < n; i += 256) s += w[i] * q1[i];
-    const float a = block_sum(s, red[0]);
-    s = 0.f;
-    for (int i = tid; i < n; i += 256) {
-      const float x = w[i] - a * q1[i] - (j > 1 ? b * q2[i] : 0.f);
-      q[i] = x;
-      s += x * x;
-    }
-    const float norm = sqrtf(block_sum(s, red[1]));
+    a = block_sum(s, red[0]);
+    const float norm = form(red[1]);
     const bool done = !(norm > 1e-7f * fabsf(a));
     if (part == 0 && tid == 0) {
       st.alpha[z * kLanczosSteps + j - 1] = a;
@@ -245,25 +253,26 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
       else st.beta[z * kLanczosSteps + j] = norm;
     }
     if (done) return;
-    const float inv = 1.f / norm;
-    for (int i = tid; i < n; i += 256) {
-      q[i] *= inv;
-      if (part == 0) qj[i] = q[i];
-    }
+    inv = 1.f / norm;
+    scale();
   }
   __syncthreads();
+  auto four = [&](int k) {
+    if constexpr (!WIDE) return *reinterpret_cast<const floatx4*>(q + k);
+    else return floatx4{raw(k), raw(k + 1), raw(k + 2), raw(k + 3)} * inv;
+  };
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int k = 4 * lane + 256 * c;
     if (k >= n4) break;
-    const floatx4 x = *reinterpret_cast<const floatx4*>(q + k);
+    const floatx4 x = four(k);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       acc[r] += early[c][r][0] * x[0] + early[c][r][1] * x[1] + early[c][r][2] * x[2] + early[c][r][3] * x[3];
   }
   for (int k = 4 * lane + 1024; k < n4; k += 256) {
-    const floatx4 x = *reinterpret_cast<const floatx4*>(q + k);
+    const floatx4 x = four(k);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + r < n ? row0 + r : n - 1;
@@ -272,10 +281,13 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     }
   }
   if (n4 + lane < n) {
+    float x;
+    if constexpr (WIDE) x = raw(n4 + lane) * inv;
+    else x = q[n4 + lane];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + r < n ? row0 + r : n - 1;
-      acc[r] += S[static_cast<int64_t>(row) * n + n4 + lane] * q[n4 + lane];
+      acc[r] += S[static_cast<int64_t>(row) * n + n4 + lane] * x;
     }
   }
   float* __restrict__ wj = g.vec + (3 + (j & 1)) * vec + static_cast<int64_t>(zl) * n;
@@ -352,6 +364,16 @@ static __global__ __launch_bounds__(256) void root_ridge_kernel(RootGroups G, fl
   const float ridge = ridge_eps * G.st.sv[z];
   const uint32_t total = static_cast<uint32_t>(g.n) * static_cast<uint32_t>(g.n), period = static_cast<uint32_t>(g.n) + 1;
   float s = 0.f;
+  if (g.n > kLanczosLdsDim) {                   // row by row: n^2 does not fit 32 bits
+    for (int i = 4 * blockIdx.x + (threadIdx.x >> 6); i < g.n; i += 4 * RCHUNKS) {
+      float* __restrict__ row = S + static_cast<int64_t>(i) * g.n;
+      for (int k = threadIdx.x & 63; k < g.n; k += 64) {
+        float x = row[k];
+        if (k == i) row[k] = x += ridge;
+        s += x * x;
+      }
+    }
+  } else
 #pragma unroll 4
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += RCHUNKS * 256) {
     float x = S[i];
@@ -919,7 +941,7 @@ static bool root_args_ok(const int64_t* n, const int* batch, int groups) {
   if (n == nullptr || batch == nullptr || groups <= 0 || groups > kRootMaxGroups) return false;
   int64_t total = 0;
   for (int i = 0; i < groups; ++i) {
-    if (n[i] <= 0 || n[i] > 32768 || batch[i] <= 0) return false;
+    if (n[i] <= 0 || n[i] > (1 << 20) || batch[i] <= 0) return false;
     total += batch[i];
   }
   return total <= 65535;
@@ -942,15 +964,19 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
       blocks += g.batch * ((g.n + kLanczosRows - 1) / kLanczosRows);
       widest = std::max(widest, g.n);
     }
+    const bool wide = widest > kLanczosLdsDim;
     const size_t lds = static_cast<size_t>(widest) * sizeof(float);
     static bool attr_set = false;     // idempotent; a race sets it twice at worst
-    if (lds > 60 * 1024 && !attr_set) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_lanczos_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              32768 * static_cast<int>(sizeof(float))) != hipSuccess)
+    if (!wide && lds > 60 * 1024 && !attr_set) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_lanczos_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kLanczosLdsDim * static_cast<int>(sizeof(float))) != hipSuccess)
         return AK_ERR_LAUNCH;
       attr_set = true;
     }
-    for (int j = 0; j < steps; ++j) hipLaunchKernelGGL(root_lanczos_kernel, dim3(blocks), b256, lds, s, G.st, L, j);
+    for (int j = 0; j < steps; ++j) {
+      if (wide) hipLaunchKernelGGL(root_lanczos_kernel<true>, dim3(blocks), b256, 0, s, G.st, L, j);
+      else hipLaunchKernelGGL(root_lanczos_kernel<false>, dim3(blocks), b256, lds, s, G.st, L, j);
+    }
     hipLaunchKernelGGL(root_power_kernel, gz, b64, 0, s, G, steps, power_tol, max_power_iter);
     hipLaunchKernelGGL(root_ridge_kernel, gc, b256, 0, s, G, ridge_eps);
     hipLaunchKernelGGL(root_schedule_kernel, gz, b64, 0, s, G, ridge_eps, max_iter, tol, steps);

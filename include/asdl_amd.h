@@ -428,7 +428,7 @@ int ak_inv_root_newton_part(int phases, int iters, float* S, int64_t n, int batc
                             ak_stream_t stream);
 
 /* Several groups of statistics in one launch sequence (group i: batch[i] matrices of size n[i], power p[i]; all arrays on
- * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 32768).  Same phases.  The
+ * the host, S / v0 / out / stats hold device pointers; 1 <= groups <= 16, n <= 2^20).  Same phases.  The
  * `active` words of all matrices, group after group, start at ws + ak_inv_root_group_active_offset().  The workspace is the sum over
  * the groups of what their sizes, powers and the ridge need (0: the arguments are not accepted). */
 size_t ak_inv_root_group_ws_bytes(const int64_t* n, const int* batch, const int* p, float ridge_eps, int groups);

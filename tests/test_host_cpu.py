@@ -79,6 +79,7 @@ def test_root_workspace_of_a_call_over_all_sizes_is_below_that_of_its_largest_gr
     for n1, b1, p1, eps in ((3072, 24, 4, 1e-6), (3072, 24, 4, 0.0), (600, 3, 7, 1e-6), (130, 2, 11, 1e-6), (2, 1, 1, 1e-6)):
         one = lib.ak_inv_root_group_ws_bytes(ctypes.byref(ctypes.c_int64(n1)), ctypes.byref(ctypes.c_int(b1)), ctypes.byref(ctypes.c_int(p1)), eps, 1)
         assert 0 < one <= lib.ak_inv_root_ws_bytes(n1, b1)
+    assert lib.ak_inv_root_ws_bytes(40000, 1) > 4 * 40000 ** 2 and lib.ak_inv_root_ws_bytes((1 << 20) + 1, 1) == 0      # sizes taken
 
 
 def test_product_refuses_cpu_tensors():

@@ -228,6 +228,40 @@ def test_inv_root_stays_within_its_workspace(groups, ridge, monkeypatch):
         assert relerr(root[0], _closed_form_root(S[0], p)) < 1e-3, (S.shape, p)
 
 
+def test_inv_root_of_more_columns_than_the_lds_holds():
+    """A statistic whose Lanczos vectors do not fit the LDS (more than 32768 columns; 64-bit indices throughout): lambda_max against
+    a power iteration here, the ridge, and two steps for p = 1, X_2 = z T_0 T_1 with T_0 = 2 I - z S, T_1 = 2 I - T_0 z S, applied to
+    two vectors in 64 bits.  Three products of 7e13 operations."""
+    n, p, eps = 32772, 1, 1e-3
+    g = torch.Generator('cuda').manual_seed(1)
+    u = torch.randn(n, generator=g, device='cuda')
+    S = torch.outer(u, u) * (10 / float(u @ u))
+    S.diagonal().add_(1 + torch.rand(n, generator=g, device='cuda'))
+    before = S.diagonal().clone()
+    v = torch.randn(n, generator=g, device='cuda')
+    for _ in range(30):
+        v = S @ (v / v.norm())
+    lam = float(v.norm())
+    try:
+        root, stats = K.inv_root_newton(S, p, eps, torch.rand(1, n, generator=g, device='cuda') * 2 - 1, max_iter=2)
+        assert int(stats[0, 2]) == 2
+        assert abs(float(stats[0, 0]) - lam) < 1e-4 * lam
+        assert relerr(S.diagonal() - before, torch.full((n,), eps * lam)) < 1e-3
+        norm = float(sum(float((rows.double() ** 2).sum()) for rows in S.split(4096))) ** 0.5
+        z = (1 + p) / (2 * norm)
+
+        def times(x):
+            return z * torch.cat([rows.double() @ x for rows in S.split(4096)])
+        x = torch.randn(n, 2, generator=g, device='cuda').double()
+        Sx = times(x)
+        t1 = 2 * x - (2 * Sx - times(Sx))                 # T_1 x
+        expected = z * (2 * t1 - times(t1))
+        got = torch.cat([rows.double() @ x for rows in root.split(4096)])
+        assert relerr(got, expected) < 1e-5, relerr(got, expected)
+    finally:
+        K.release_workspaces()
+
+
 def test_inv_root_polled_and_unpolled_enqueue_give_the_same_result():
     """The host may stop enqueuing Newton iterations once the convergence flags are all zero (read every few
     iterations) or enqueue all of them blindly: bit-equal roots and the same iteration counts."""
