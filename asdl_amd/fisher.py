@@ -15,7 +15,7 @@ from .grad_maker import GradientMaker, LOSS_CROSS_ENTROPY, LOSS_MSE
 from .profiling import nvtx_range, phase_mark
 from .matrices import *
 from .operations import OperationContext
-from .symmatrix import SymMatrix, batched_unit_update_inv, batched_update_inv
+from .symmatrix import SymMatrix, batched_unit_update_inv, batched_update_inv, read_flags
 from .utils import manual_seed, skip_param_grad
 
 __all__ = ['FisherConfig', 'get_fisher_maker', 'FisherMaker']
@@ -89,8 +89,7 @@ class FisherMaker(GradientMaker):
         torch.linalg.LinAlgError for a factor that was not positive definite, RuntimeError for a draw from logits that are
         no distribution.  Called by the next update; call it after the last one."""
         pending, self._late_flags, self._late_sampled = self._late_sampled + self._late_flags, [], []
-        for late in pending:
-            late.check()
+        read_flags(pending)
 
     def _check_sampled(self):
         """Raises torch.multinomial's RuntimeError if this call's targets were drawn from logits that are no distribution."""

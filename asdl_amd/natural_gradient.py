@@ -19,7 +19,7 @@ from .fisher import FisherConfig, get_fisher_maker
 from .grad_maker import LOSS_CROSS_ENTROPY
 from .matrices import *
 from .prec_grad_maker import PreconditionedGradientMaker, PreconditioningConfig
-from .symmatrix import Kron, SymMatrix, UnitWise, batched_unit_update_inv, batched_update_inv
+from .symmatrix import Kron, SymMatrix, UnitWise, batched_unit_update_inv, batched_update_inv, read_flags
 
 _invalid_ema_decay = -1
 _module_level_shapes = [SHAPE_LAYER_WISE, SHAPE_KRON, SHAPE_SWIFT_KRON, SHAPE_KFE, SHAPE_UNIT_WISE, SHAPE_DIAG]
@@ -265,8 +265,7 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
             self.fisher_maker.flags_to_caller = False
             unread = self.fisher_maker.take_caller_flags()
             if unread and sys.exc_info()[0] is None:
-                for late in unread:          # no stage read them (precondition() was replaced, say)
-                    late.check(when=None)
+                read_flags(unread, when=None)          # no stage read them (precondition() was replaced, say)
 
     def _curvature_matrices(self, module_name=None):
         matrices, units = [], []
@@ -339,8 +338,7 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         saved = self._save_gradients(grads)
         self._precondition_launch(work, grad_scale, use_inv)
         try:
-            for late in unread:
-                late.check(when=None)
+            read_flags(unread, when=None)
         except torch.linalg.LinAlgError:
             if grads:
                 torch._foreach_copy_(grads, saved)      # as the reference leaves them when its Cholesky raises
@@ -391,8 +389,7 @@ class NaturalGradientMaker(PreconditionedGradientMaker):
         if not kernels.kron_precond_deep(items, units, float(grad_scale), gw.device, fail):
             self._deep_declined = modules        # the sizes decide: not asked again for these modules
             return False
-        for late in unread:
-            late.check(when=None)
+        read_flags(unread, when=None)
         return True
 
     def _save_gradients(self, grads):

@@ -510,21 +510,22 @@ class LateChunk:
     """The unread flags of one chunk of DeferredInverses.finish_late() and the modules its Kron objects belong to."""
 
     def __init__(self, late, targets, attr):
-        self._late, self._targets, self._attr = late, targets, attr
+        self._late = late
+        # the objects that hold this update's inverses (the modules may have those of the next one when the flags are read)
+        self._holders = {id(kron): getattr(module, attr, None) for module, kron in targets} if attr is not None else {}
 
     @property
     def fail_word(self):
         return self._late.fail_word
 
     def check(self, *args, **kwargs):
-        zero = self._late.check(*args, **kwargs)
-        if zero and self._attr is not None:
-            owner = {id(kron): module for module, kron in self._targets}
-            for kron, which in zero:
-                fisher = getattr(owner.get(id(kron)), self._attr, None)
+        try:
+            return self._late.check(*args, **kwargs)
+        finally:
+            for kron, which in self._late.removed:
+                fisher = self._holders.get(id(kron))
                 if fisher is not None and fisher.has_kron:
                     setattr(fisher.kron, which + '_inv', None)
-        return zero
 
 
 class DeferredInverses:
@@ -544,7 +545,7 @@ class DeferredInverses:
         has unit-wise flags to read, which then only finish() does."""
         late_units = []
         if self._context is not None and self._context._unit_flags and units:
-            late_units = [self._context.late_unit_flags()]
+            late_units = [self._context.late_unit_flags(attr)]
         if self._context is not None and self._context._unit_flags:
             global _warned_late_fallback
             if not _warned_late_fallback:
@@ -561,11 +562,19 @@ class DeferredInverses:
 
     def finish(self, attr):
         if self._context is not None:
-            self._context.check_unit_flags()
+            self._context.check_unit_flags(attr)
         for pending, _ in self._chunks:
             pending.join()               # all waits first, then the flag reads
         for pending, targets in self._chunks:
-            pending.finish()
+            try:
+                pending.finish()
+            except torch.linalg.LinAlgError:
+                owner = {id(kron): getattr(module, attr, None) for module, kron in targets}
+                for kron, which in pending.failed:
+                    fisher = owner.get(id(kron))
+                    if fisher is not None and fisher.has_kron:
+                        setattr(fisher.kron, which + '_inv', None)
+                raise
             for module, kron in targets:
                 fisher = getattr(module, attr, None)
                 if fisher is None or not fisher.has_kron:
@@ -716,13 +725,18 @@ class OperationContext:
             store['inv'] = inv
             self._unit_flags.append((op._module, flags[i]))
 
-    def late_unit_flags(self):
+    def late_unit_flags(self, attr=None):
         """check_unit_flags() as an object whose check() does the reading."""
         pending, self._unit_flags = self._unit_flags, []
         self._unit_flags_deferred = False
         modules = [m for m, _ in pending]
+        holders = [getattr(m, attr, None) if attr is not None else None for m in modules]
+
+        def drop(i):
+            if holders[i] is not None and holders[i].has_unit:
+                holders[i].unit.inv = None
         return LateUnitFlags(self._unit_flag_rows(pending),
-                             lambda i, block: f'unit-wise block {block} of {modules[i]} + damping is singular')
+                             lambda i, block: f'unit-wise block {block} of {modules[i]} + damping is singular', failed=drop)
 
     @staticmethod
     def _unit_flag_rows(pending):
@@ -732,21 +746,28 @@ class OperationContext:
             return whole
         return torch.stack([f for _, f in pending])
 
-    def check_unit_flags(self):
+    def check_unit_flags(self, attr=None):
         """torch.inverse raises for a singular block (asdl/operations/operation.py:317-320); here the flags of all
-        modules are read with one copy."""
+        modules are read with one copy.  ``attr``: where the modules hold this update's inverses, so that a failed one is
+        taken away."""
         pending = self._unit_flags
         self._unit_flags = []
         self._unit_flags_deferred = False
         if not pending:
             return
         host = self._unit_flag_rows(pending).cpu().tolist()
+        error = None
         for (module, _), (nonzero, bad) in zip(pending, host):
             if bad != 0x7fffffff:
-                raise torch.linalg.LinAlgError(f'unit-wise block {bad - 1} of {module} + damping is singular')
+                fisher = getattr(module, attr, None) if attr is not None else None
+                if fisher is not None and fisher.has_unit:
+                    fisher.unit.inv = None
+                error = error or torch.linalg.LinAlgError(f'unit-wise block {bad - 1} of {module} + damping is singular')
+        if error is not None:
+            raise error
 
     def _enqueue_pending(self):
-        """Starts the batched inverse of every queued pair (side streams, worker threads) and places the
+        """Starts the batched inverse of every queued pair (on side streams) and places the
         output tensors in the result store; their flags are read by DeferredInverses.finish()."""
         ops = self._pending_inverse
         self._pending_inverse = []

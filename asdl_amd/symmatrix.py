@@ -133,6 +133,19 @@ def _flags_to_host(flags):
     return host, event
 
 
+def read_flags(unread, **kwargs):
+    """check() of every object, also behind one that raises: each removes what failed from where it was stored.  Then the first
+    error is raised."""
+    error = None
+    for late in unread:
+        try:
+            late.check(**kwargs)
+        except RuntimeError as e:           # (torch.linalg.LinAlgError is one)
+            error = error or e
+    if error is not None:
+        raise error
+
+
 class LateFlags:
     """Flags of a batch of inverses on their way to pinned host memory (PendingInverses.finish_late).  check() waits
     for the copy, which has long arrived when it is called a step later, and raises for a factor that was not
@@ -140,6 +153,7 @@ class LateFlags:
 
     def __init__(self, host, records, flags, keep_alive):
         self._host, self._records, self._flags, self._keep_alive = host, records, flags, keep_alive
+        self.removed = []            # (Kron, 'A' | 'B') whose inverse check() has taken away
 
     @property
     def fail_word(self):
@@ -149,23 +163,29 @@ class LateFlags:
     def check(self, when='reported late: the flags of this update were read after the next one'):
         """Raises for a factor that was not positive definite.  Returns the (Kron, 'A' | 'B') whose factor was all
         zero and had no inverse before: the reference computes none for them (asdl/symmatrix.py:517, :527); the
-        device has put the identity there, and the caller removes it again."""
+        device has put the identity there, and the caller removes it again.  An inverse that failed is taken away as well:
+        the next step must not precondition with it."""
         if self._host is None:
             return []
         pending, self._host, self._keep_alive = self._host, None, None
         host = pending.read() if isinstance(pending, kernels.HostFlags) else pending.tolist()
         n = len(self._records)
         info_host, nz_host = host[:n], host[n:]
-        zero = []
+        zero, error = [], None
         for (flat, k, which, was_fresh), inf in zip(self._records, info_host):
             if not nz_host[flat]:
                 if was_fresh:
                     setattr(k, which + '_inv', None)
                     zero.append((k, which))
             elif inf != 0:
-                raise torch.linalg.LinAlgError(
+                setattr(k, which + '_inv', None)
+                self.removed.append((k, which))
+                error = error or torch.linalg.LinAlgError(
                     f'cholesky_inv: the leading minor of order {inf} of kron.{which} + damping was not '
                     f'positive-definite' + (f' ({when})' if when else ''))
+        self.removed += zero
+        if error is not None:
+            raise error
         return zero
 
 
@@ -182,6 +202,7 @@ class PendingInverses:
         self._keep_alive = keep_alive      # tensors the side-stream kernels still read
         self._side_streams, self._replace = side_streams, replace
         self._done = False
+        self.failed = []                   # (Kron, 'A' | 'B') whose inverse finish() found to have failed
 
     def join(self):
         """Makes the current stream wait for the inverses (no host synchronisation)."""
@@ -239,6 +260,11 @@ class PendingInverses:
         n = len(self._records)
         info_host, nz_host = host[:n], host[n:]
         self._keep_alive = None
+        for (flat, k, which, out), inf in zip(self._records, info_host):
+            if nz_host[flat] and inf != 0:
+                self.failed.append((k, which))
+                if getattr(k, which + '_inv') is out:
+                    setattr(k, which + '_inv', None)         # an earlier inverse whose memory the failed one took
         for (flat, k, which, out), inf in zip(self._records, info_host):
             if not nz_host[flat]:
                 continue                                            # all-zero factor: inverse skipped
@@ -379,11 +405,12 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
 
 class LateUnitFlags:
     """The unread flags of a batch of unit-wise inverses, [count, 2] (non-zero, first singular block) on their way to pinned
-    host memory; ``singular(i, block)`` names module i in the error, ``all_zero(i)`` is told of modules that were all zero."""
+    host memory; ``singular(i, block)`` names module i in the error, ``all_zero(i)`` is told of modules that were all zero and
+    ``failed(i)`` of those with a singular block, whose inverse is not to be used."""
 
-    def __init__(self, flags, singular, all_zero=None):
+    def __init__(self, flags, singular, all_zero=None, failed=None):
         self._host, self._event = _flags_to_host(flags)
-        self._flags, self._singular, self._all_zero = flags, singular, all_zero
+        self._flags, self._singular, self._all_zero, self._failed = flags, singular, all_zero, failed
 
     def check(self, *args, **kwargs):
         if self._flags is None:
@@ -391,11 +418,16 @@ class LateUnitFlags:
         if self._event is not None:
             self._event.synchronize()
         self._flags = None
+        error = None
         for i, (nonzero, bad) in enumerate(self._host.tolist()):
             if not nonzero and self._all_zero is not None:
                 self._all_zero(i)
             elif bad != 0x7fffffff:
-                raise torch.linalg.LinAlgError(self._singular(i, bad - 1))
+                if self._failed is not None:
+                    self._failed(i)
+                error = error or torch.linalg.LinAlgError(self._singular(i, bad - 1))
+        if error is not None:
+            raise error
         return []
 
 
@@ -418,8 +450,9 @@ def batched_unit_update_inv(units, damping=_default_damping, replace=False, late
             u.inv = inv
             if replace:
                 u.data = None
-        return LateUnitFlags(flags, lambda i, block: f'unit-wise block {block} + damping is singular',
-                             lambda i: setattr(units[i], 'inv', previous[i]))
+        def put_back(i):
+            units[i].inv = previous[i]
+        return LateUnitFlags(flags, lambda i, block: f'unit-wise block {block} + damping is singular', put_back, put_back)
     host = flags.cpu().tolist()
     for u, inv, (nonzero, bad) in zip(units, invs, host):
         if not nonzero:

@@ -702,3 +702,75 @@ def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):
     assert ordered == []
     del pending
     assert ordered == [(5, None)]
+
+
+# ------------------------------------------------------------------ inverses that fail
+@pytest.mark.parametrize('ema', [-1, 0.5])
+@pytest.mark.parametrize('fisher_type', [FISHER_MC, FISHER_EMP])
+@pytest.mark.parametrize('after', [True, False])
+@pytest.mark.parametrize('earlier', [False, True])
+def test_failed_inverses_are_not_kept(earlier, after, fisher_type, ema, monkeypatch):
+    """A factor that is not positive definite raises from forward_and_backward(); who catches that and goes on must not find the
+    failed inverse where the next step would precondition with it, whether the module had one before or not."""
+    import asdl_amd.natural_gradient as ng_mod
+    from asdl_amd import kernels
+    cpu_backend.install(monkeypatch)
+    monkeypatch.setattr(ng_mod, 'FLAGS_AFTER_PRECONDITION', after)
+    broken, plain = [False], kernels.kron_damping
+
+    def damping(A_list, B_list, *args, **kwargs):
+        lam, nonzero = plain(A_list, B_list, *args, **kwargs)
+        if broken[0]:
+            lam[1] *= -1e6              # the second module's pair
+        return lam, nonzero
+    monkeypatch.setattr(kernels, 'kron_damping', damping)
+    torch.manual_seed(2)
+    model = get_mlp()
+    x, t = torch.randn(8, 5), torch.randint(4, (8,))
+    gm = KfacGradientMaker(model, PreconditioningConfig(data_size=8, damping=1e-2, ema_decay=ema), fisher_type=fisher_type, seed=1)
+
+    def step():
+        model.zero_grad(set_to_none=True)
+        gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x), t)
+        gm.forward_and_backward()
+    if earlier:
+        step()
+    broken[0] = True
+    with pytest.raises(torch.linalg.LinAlgError):
+        step()
+    broken[0] = False
+    fisher = getattr(model[2], 'fisher', None)
+    assert fisher is None or (fisher.kron.A_inv is None and fisher.kron.B_inv is None)
+    step()
+    assert model[2].fisher.kron.has_inv and all(torch.isfinite(p.grad).all() for p in model.parameters())
+
+
+def test_singular_unit_wise_blocks_leave_the_earlier_inverse(monkeypatch):
+    from asdl_amd import kernels, symmatrix
+    flags = torch.tensor([[1, 0x7fffffff], [1, 4], [0, 0x7fffffff]], dtype=torch.int32)
+    new = [torch.full((5, 2, 2), float(i)) for i in range(3)]
+    old = [torch.eye(2).repeat(5, 1, 1) for _ in range(3)]
+    monkeypatch.setattr(kernels, 'unit_wise_inv_grouped', lambda blocks, dampings: (list(new), flags))
+    monkeypatch.setattr(kernels, 'unit_wise_keep_grouped', lambda invs, previous, fl: None)
+    units = [symmatrix.UnitWise(torch.ones(5, 2, 2), inv) for inv in old]
+    late = symmatrix.batched_unit_update_inv(units, 1e-2, late=True)
+    with pytest.raises(torch.linalg.LinAlgError, match='block 3'):
+        late.check(when=None)
+    assert units[0].inv is new[0] and units[1].inv is old[1] and units[2].inv is old[2]
+
+
+def test_all_flags_are_read_before_the_first_error_is_raised():
+    from asdl_amd.symmatrix import read_flags
+    seen = []
+
+    class Late:
+        def __init__(self, name, error=None):
+            self.name, self.error = name, error
+
+        def check(self, when='x'):
+            seen.append((self.name, when))
+            if self.error is not None:
+                raise self.error
+    with pytest.raises(torch.linalg.LinAlgError, match='first'):
+        read_flags([Late('a'), Late('b', torch.linalg.LinAlgError('first')), Late('c', RuntimeError('second'))], when=None)
+    assert seen == [('a', None), ('b', None), ('c', None)]

@@ -953,6 +953,109 @@ def test_flags_read_after_the_preconditioning_leave_raw_gradients_when_they_rais
             assert relerr(g, raw[name]) > 1e-2, name              # preconditioned
 
 
+@pytest.mark.parametrize('fisher_type,norm', [(FISHER_MC, False), (FISHER_EMP, False), (FISHER_EMP, True)])
+@pytest.mark.parametrize('ema', [-1, 0.5])
+@pytest.mark.parametrize('bad_first', [True, False])
+def test_small_modules_are_not_preconditioned_with_inverses_that_failed(bad_first, ema, fisher_type, norm, monkeypatch):
+    """The two-launch preconditioning of small modules runs before the flags of the inverses are read and leaves the gradients alone
+    by the batch's fail word: with a factor that is not positive definite forward_and_backward() raises, .grad holds what the
+    backward pass left, and the failed inverse is gone, as in the strict order (flags first).  Accumulated factors and none, the
+    inverses beside the loss backward pass and behind a single one, with unit-wise blocks (whose flags have no fail word: the
+    gradients are saved and put back)."""
+    import asdl_amd.natural_gradient as ng_mod
+    import asdl_amd.symmatrix as sm_mod
+    from asdl_amd import kernels
+    plain_damping, plain_deep = kernels.kron_damping, kernels.kron_precond_deep
+    broken, deep = [False], []
+
+    def damping(*args, **kwargs):
+        lam, nonzero = plain_damping(*args, **kwargs)
+        return (lam * -1e6 if broken[0] else lam), nonzero
+
+    def spy(*args, **kwargs):
+        deep.append(plain_deep(*args, **kwargs))
+        return deep[-1]
+    monkeypatch.setattr(sm_mod.kernels, 'kron_damping', damping)
+    monkeypatch.setattr(kernels, 'kron_precond_deep', spy)
+    g = torch.Generator().manual_seed(70)
+    x, t = torch.randn(8, 14, generator=g).cuda(), torch.randint(10, (8,), generator=g).cuda()
+    sequence = (True, False) if bad_first else (False, True, False)
+
+    def make():
+        torch.manual_seed(34)
+        return nn.Sequential(nn.Linear(14, 18), nn.ReLU(), *([nn.LayerNorm(18)] if norm else []), nn.Linear(18, 10)).cuda()
+
+    def run(after):
+        monkeypatch.setattr(ng_mod, 'FLAGS_AFTER_PRECONDITION', after)
+        model = make()
+        gm = KfacGradientMaker(model, PreconditioningConfig(data_size=8, damping=1e-2, ema_decay=ema), fisher_type=fisher_type, seed=5)
+        out, held = {}, []
+        for step, bad in enumerate(sequence):
+            broken[0] = bad
+            model.zero_grad(set_to_none=True)
+            gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x), t)
+            if bad:
+                with pytest.raises(torch.linalg.LinAlgError, match='positive-definite'):
+                    gm.forward_and_backward()
+            else:
+                gm.forward_and_backward()
+            for m in model:
+                kron = getattr(getattr(m, 'fisher', None), 'kron', None)
+                held.append(kron is not None and kron.has_inv)
+            for name, p in model.named_parameters():
+                out[(step, name)] = p.grad.clone()
+        return out, held
+
+    strict, held_strict = run(False)
+    del deep[:]
+    after, held = run(True)
+    assert norm or deep == [True] * len(sequence)
+    assert held == held_strict
+    model = make()
+    F.cross_entropy(model(x), t, reduction='sum').div(8).backward()
+    raw = {name: p.grad for name, p in model.named_parameters()}
+    for (step, name), grad in strict.items():
+        if sequence[step]:          # (flags first, behind a single pass: raised before the sum is divided by the data size)
+            assert relerr(after[(step, name)], raw[name]) < 1e-5, (step, name)
+        else:
+            assert relerr(after[(step, name)], grad) < 1e-4, (step, name)
+            assert relerr(grad, raw[name]) > 1e-2, (step, name)
+
+
+@pytest.mark.parametrize('after', [True, False])
+def test_singular_unit_wise_block_with_accumulated_factors(after, monkeypatch):
+    """LateUnitFlags through a maker: a singular 2 x 2 block raises from forward_and_backward(), the gradients stay raw, and the
+    module keeps the inverse it had."""
+    import asdl_amd.natural_gradient as ng_mod
+    from asdl_amd import kernels
+    monkeypatch.setattr(ng_mod, 'FLAGS_AFTER_PRECONDITION', after)
+    plain, broken = kernels.unit_wise_inv_grouped, [False]
+    monkeypatch.setattr(kernels, 'unit_wise_inv_grouped', lambda blocks, dampings, outs=None: plain(
+        [torch.ones_like(b) for b in blocks] if broken[0] else blocks, [0.0] * len(blocks) if broken[0] else dampings, outs))
+    torch.manual_seed(4)
+    model = nn.Sequential(nn.Linear(9, 12), nn.LayerNorm(12), nn.ReLU(), nn.Linear(12, 5)).cuda()
+    x, t = torch.randn(16, 9).cuda(), torch.randint(0, 5, (16,)).cuda()
+    gm = KfacGradientMaker(model, PreconditioningConfig(data_size=16, damping=1e-2, ema_decay=0.5), fisher_type=FISHER_EMP)
+
+    def step():
+        model.zero_grad(set_to_none=True)
+        gm.setup_loss_call(F.cross_entropy, gm.setup_model_call(model, x), t)
+        gm.forward_and_backward()
+    step()
+    earlier = model[1].fisher.unit.inv.clone()
+    broken[0] = True
+    with pytest.raises(torch.linalg.LinAlgError, match='singular'):
+        step()
+    broken[0] = False
+    assert torch.equal(model[1].fisher.unit.inv, earlier)
+    got = [p.grad.clone() for p in model.parameters()]
+    model.zero_grad(set_to_none=True)
+    F.cross_entropy(model(x), t, reduction='sum').div(16).backward()
+    for a, p in zip(got, model.parameters()):
+        assert relerr(a, p.grad) < 1e-5
+    step()
+
+
 @pytest.mark.parametrize('pi', [1, 2])
 def test_overlapped_inverse_update_in_ema_mode_gives_the_same_result(pi, monkeypatch):
     """natural_gradient.OVERLAP_INVERSE_UPDATE: with accumulated factors and a sampled Fisher, the inverses of
