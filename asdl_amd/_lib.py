@@ -40,6 +40,7 @@ _SIGNATURES = {
     'ak_chol_group_ws_bytes': (c_size, [c_ptr, c_int]),
     'ak_chol_group_plan': (c_int, [c_ptr, c_int, c_ptr, c_size]),
     'ak_chol_group_plan_launches': (c_int, [c_ptr]),
+    'ak_chol_group_plan_us': (ctypes.c_double, [c_ptr]),
     'ak_chol_inv_grouped': (c_int, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_int, c_ptr, c_ptr, c_size, c_ptr]),
     'ak_unit_wise_ws_bytes': (c_size, [c_i64, c_i64, c_i64]),
     'ak_unit_wise_stats': (c_int, [c_ptr, c_int, c_i64, c_i64, c_i64, c_ptr, c_int, c_i64, c_i64, c_i64, c_ptr, c_ptr,

@@ -57,6 +57,7 @@ struct CgHeader {
   int64_t mats_off, steps_off, leaves_off, prods_off, map_off;     // byte offsets of the tables inside the plan
   int32_t count, nsteps, nleaves, nprods;
   int32_t copy_blocks, ntiles;
+  double us;                // estimated time of one call (cg_build)
 };
 
 struct CgMat {
@@ -537,7 +538,12 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
     const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
     tiles += nb * (nb + 1) / 2;
   }
-  if (CG_FORCE == 1) { cg_build_sweep(dims, count, plan); return; }
+  const double sweep_us = cg_sweep_us(dims, count);
+  if (CG_FORCE == 1) {
+    cg_build_sweep(dims, count, plan);
+    plan.h.us = sweep_us;
+    return;
+  }
   CgPlan right;
   cg_build_right_looking(dims, count, right);
   double us = 0;
@@ -550,8 +556,10 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
       us += cg_product_us(ps, st.type == CG_PROD_DEEP);
     }
   }
-  if (CG_FORCE != 2 && tiles <= 4096 && cg_sweep_us(dims, count) < us) cg_build_sweep(dims, count, plan);
+  const bool sweep = CG_FORCE != 2 && tiles <= 4096 && sweep_us < us;
+  if (sweep) cg_build_sweep(dims, count, plan);
   else plan = std::move(right);
+  plan.h.us = sweep ? sweep_us : us;
 }
 
 static void cg_build_right_looking(const int64_t* dims, int count, CgPlan& plan) {
@@ -685,6 +693,12 @@ extern "C" int ak_chol_group_plan_launches(const void* plan_host) {
   if (plan_host == nullptr) return AK_ERR_ARG;
   const ak::CgHeader* h = static_cast<const ak::CgHeader*>(plan_host);
   return h->magic == ak::CG_MAGIC ? h->nsteps : AK_ERR_ARG;
+}
+
+extern "C" double ak_chol_group_plan_us(const void* plan_host) {
+  if (plan_host == nullptr) return -1.0;
+  const ak::CgHeader* h = static_cast<const ak::CgHeader*>(plan_host);
+  return h->magic == ak::CG_MAGIC ? h->us : -1.0;
 }
 
 extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, const float* const* A_list,

@@ -1291,8 +1291,7 @@ class CholGroupPlan:
         _lib.check(lib.ak_chol_group_plan(arr, len(self.dims), ctypes.c_void_p(self.host.data_ptr()), nbytes),
                    'ak_chol_group_plan')
         self.launches = lib.ak_chol_group_plan_launches(ctypes.c_void_p(self.host.data_ptr()))
-        blocks = (max(self.dims) + 127) // 128
-        self.microseconds = 25 * self.launches if self.launches == blocks + 1 else 20 * self.launches    # about
+        self.microseconds = lib.ak_chol_group_plan_us(ctypes.c_void_p(self.host.data_ptr()))       # estimated
         with _on_launch_stream():
             self.dev = self.host.to(device, non_blocking=True)
 

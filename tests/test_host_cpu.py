@@ -82,6 +82,24 @@ def test_root_workspace_of_a_call_over_all_sizes_is_below_that_of_its_largest_gr
     assert lib.ak_inv_root_ws_bytes(40000, 1) > 4 * 40000 ** 2 and lib.ak_inv_root_ws_bytes((1 << 20) + 1, 1) == 0      # sizes taken
 
 
+def test_plan_of_the_grouped_inverse_says_how_long_it_takes():
+    """The library's own estimate, by which it chose the sequence: it grows with the sizes on both sides of the choice, and lies near
+    what was measured (206, 284, 757 microseconds for the first three)."""
+    import ctypes
+    from asdl_amd import _lib
+    lib = _lib.load()
+
+    def estimate(dims):
+        arr = (ctypes.c_int64 * len(dims))(*dims)
+        plan = ctypes.create_string_buffer(lib.ak_chol_group_plan_bytes(arr, len(dims)))
+        assert lib.ak_chol_group_plan(arr, len(dims), plan, len(plan)) == 0
+        return lib.ak_chol_group_plan_us(plan)
+    for dims, measured in (((784, 512, 512, 512, 512, 10), 206), ((1153, 512), 284), ((2048, 2048), 757)):
+        assert 0.7 * measured < estimate(dims) < 1.3 * measured, (dims, estimate(dims))
+    assert estimate((4096, 4096)) > estimate((2048,) * 4) > estimate((2048, 2048)) > estimate((128,)) > 0
+    assert lib.ak_chol_group_plan_us(ctypes.create_string_buffer(256)) < 0
+
+
 def test_product_refuses_cpu_tensors():
     from asdl_amd import kernels
     with pytest.raises(RuntimeError, match='ROCm device'):
