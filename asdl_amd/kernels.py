@@ -1647,8 +1647,10 @@ def kron_precond_grouped(items, grad_scale=1.0):
 
 
 # ------------------------------------------------------------------------------ Shampoo inverse root
-ROOT_POLL_AFTER = (13, 4)   # Newton iterations enqueued before the first read of the convergence flags (an accelerated
-                            # computation at the usual ridge takes 12 or 13), and between the later ones
+ROOT_POLL_AFTER = (15, 2)   # Newton iterations enqueued before the first read of the convergence flags, and between the later
+                            # ones: p = 4 takes 8 to 15 at a ridge of 1e-6 (full-rank to rank-deficient statistics), seldom
+                            # 16 to 19 (a few tiny eigenvalues, more than 1000 columns).  An iteration that nothing needs
+                            # costs its launches, a read drains the device.
 ROOT_MAX_GROUPS = 16
 
 
