@@ -55,12 +55,19 @@ def _with_shared_gradients(work):
     """The modules of ``work`` whose weight or bias gradient another of them holds too (tied parameters).  One after the other
     they give B2 (B1 G A1) A2 on such a gradient (asdl/precondition/natural_gradient.py:478-486, 508-543); launches that take many
     modules at once, or modules on several streams, would read and write it in no order."""
+    addresses = []
+    for module, _ in work:
+        for p in module._parameters.values():
+            grad = p.grad if p is not None else None
+            if grad is not None:
+                addresses.append(grad.data_ptr())
+    if len(set(addresses)) == len(addresses):
+        return ()
     holders = {}
     for module, _ in work:
-        for name in ('weight', 'bias'):
-            grad = getattr(getattr(module, name, None), 'grad', None)
-            if grad is not None:
-                holders.setdefault(grad.data_ptr(), []).append(module)
+        for p in module._parameters.values():
+            if p is not None and p.grad is not None:
+                holders.setdefault(p.grad.data_ptr(), []).append(module)
     return {module for modules in holders.values() if len(modules) > 1 for module in modules}
 
 
