@@ -17,7 +17,6 @@ AK_F32, AK_BF16, AK_F32_AS_BF16 = 0, 1, 2
 
 _ws_lock = threading.Lock()
 _workspaces = {}
-_ptr_cache = {}
 _timing_sink = None      # when set to a list, factor launches append (name, flops, start event, end event)
 
 
@@ -190,58 +189,53 @@ def _ws_args(nbytes, device):
     return ctypes.c_void_p(buf.data_ptr()), size, buf
 
 
+def _upload(host, device):
+    """A host tensor on the device, staged through pinned memory and copied asynchronously on the launch stream (a pageable copy would
+    block the caller behind everything that stream has queued)."""
+    if device.type != 'cuda':
+        return host.to(device)
+    with _on_launch_stream():
+        return host.pin_memory().to(device, non_blocking=True)
+
+
+def _stream_key(device):
+    """What a table on the device is kept under: launches of another stream would not wait for its upload, and its memory goes back to
+    the stream it was allocated on when a cache is cleared."""
+    return (device.index, _stream_handle(device)) if device.type == 'cuda' else (device.index, 0)
+
+
+_tables = {}
+MAX_TABLES = 8192
+
+
+def _device_table(kind, values, dtype, device):
+    key = (_stream_key(device), kind, values)
+    t = _tables.get(key)
+    if t is None:
+        if len(_tables) > MAX_TABLES:
+            _tables.clear()
+        t = _tables[key] = _upload(torch.tensor(values, dtype=dtype), device)
+    return t
+
+
 def device_ptr_array(tensors):
     """int64 device tensor holding the data pointers of ``tensors`` (cached by pointer tuple)."""
     return device_addresses(tuple(t.data_ptr() for t in tensors), tensors[0].device)
 
 
 def device_addresses(ptrs, dev):
-    key = (dev.index, ptrs)
-    arr = _ptr_cache.get(key)
-    if arr is None:
-        if len(_ptr_cache) > 4096:
-            _ptr_cache.clear()
-        # staged through pinned memory and copied asynchronously on the launch stream, like device_table(): a
-        # pageable copy would block the caller behind everything that stream has queued
-        host = torch.tensor(ptrs, dtype=torch.int64).pin_memory()
-        with _on_launch_stream():
-            arr = host.to(dev, non_blocking=True)
-        _ptr_cache[key] = arr
-    return arr
-
-
-_int_cache = {}
+    return _device_table('addresses', ptrs, torch.int64, dev)
 
 
 def device_ints(values, device, dtype=torch.int64):
-    """Device tensor holding a small tuple of Python ints (nested tuples give a 2-D tensor).  Cached: the
-    same index sets recur every step, and building them anew costs a synchronous host-to-device copy that
-    stalls the host behind everything already enqueued."""
-    dev = torch.device(device)
-    key = (dev.index, dtype, values)
-    t = _int_cache.get(key)
-    if t is None:
-        if len(_int_cache) > 8192:
-            _int_cache.clear()
-        t = torch.tensor(values, dtype=dtype).to(dev)
-        _int_cache[key] = t
-    return t
+    """Device tensor holding a small tuple of Python ints (nested tuples give a 2-D tensor), for the launch stream.  Cached: the
+    same index sets recur every step."""
+    return _device_table(dtype, values, dtype, torch.device(device))
 
 
 def device_table(rows, device):
-    """device_ints for tables that hold addresses, which may change from call to call: a miss is staged through
-    pinned memory and copied asynchronously on the launch stream, so the host never waits for the device."""
-    dev = torch.device(device)
-    key = (dev.index, 'table', rows)
-    t = _int_cache.get(key)
-    if t is None:
-        if len(_int_cache) > 8192:
-            _int_cache.clear()
-        host = torch.tensor(rows, dtype=torch.int64).pin_memory()
-        with _on_launch_stream():
-            t = host.to(dev, non_blocking=True)
-        _int_cache[key] = t
-    return t
+    """device_ints for tables that hold addresses, which may change from call to call."""
+    return _device_table('table', rows, torch.int64, torch.device(device))
 
 
 class main_stream_launches:
@@ -992,7 +986,7 @@ class HostFlags:
         self.address = self._host.data_ptr()
 
     def clear(self):
-        self._host[:self._words].zero_()         # (whoever had the memory before has read it)
+        ctypes.memset(self.address, 0, 4 * self._words)         # (whoever had the memory before has read it)
 
     def record(self):
         _lib.check(_lib.load().ak_event_record(self._event, _stream()), 'ak_event_record')
@@ -1272,14 +1266,15 @@ def chol_inv_batched(mats, outs, lam, lam_stride=1, active=None, active_stride=1
 
 
 _chol_plans = {}
+_chol_plan_lock = threading.Lock()
 
 
 class CholGroupPlan:
     """Launch plan of ak_chol_inv_grouped for one tuple of matrix sizes: built on the host by the library, kept in
-    pinned memory (the library reads the launch sequence from it on every call) with a copy on the device (the
-    kernels read their descriptors from it)."""
+    pinned memory (the library reads the launch sequence from it on every call) with a copy on the device per launch stream
+    (the kernels read their descriptors from it)."""
 
-    def __init__(self, dims, device):
+    def __init__(self, dims):
         lib = _lib.load()
         self.dims = tuple(int(d) for d in dims)
         arr = (ctypes.c_int64 * len(self.dims))(*self.dims)
@@ -1292,18 +1287,24 @@ class CholGroupPlan:
                    'ak_chol_group_plan')
         self.launches = lib.ak_chol_group_plan_launches(ctypes.c_void_p(self.host.data_ptr()))
         self.microseconds = lib.ak_chol_group_plan_us(ctypes.c_void_p(self.host.data_ptr()))       # estimated
-        with _on_launch_stream():
-            self.dev = self.host.to(device, non_blocking=True)
+        self._dev = {}
+
+    def on_device(self, device):
+        key = _stream_key(device)
+        dev = self._dev.get(key)
+        if dev is None:
+            dev = self._dev[key] = _upload(self.host, device)
+        return dev
 
 
-def chol_group_plan(dims, device):
-    dev = torch.device(device)
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), tuple(int(d) for d in dims))
+def chol_group_plan(dims):
+    key = tuple(int(d) for d in dims)
     plan = _chol_plans.get(key)
     if plan is None:
-        if len(_chol_plans) > 64:
-            _chol_plans.clear()
-        plan = _chol_plans[key] = CholGroupPlan(dims, dev)
+        with _chol_plan_lock:
+            if len(_chol_plans) > 64:
+                _chol_plans.clear()
+            plan = _chol_plans[key] = CholGroupPlan(dims)
     return plan
 
 
@@ -1322,11 +1323,11 @@ def chol_inv_grouped(mats, outs, lam, lam_stride=1, active=None, active_stride=1
         raise ValueError('one output per matrix')
     if info is None:
         info = torch.empty(len(mats), dtype=torch.int32, device=dev)
-    plan = chol_group_plan([m.shape[0] for m in mats], dev)
+    plan = chol_group_plan([m.shape[0] for m in mats])
     ws, ws_bytes, keep = _ws_args(plan.ws_bytes, dev)
     pa, po = device_ptr_array(mats), device_ptr_array(outs)
     rc = _lib.load().ak_chol_inv_grouped(
-        ctypes.c_void_p(plan.host.data_ptr()), ctypes.c_void_p(plan.dev.data_ptr()), ctypes.c_void_p(pa.data_ptr()),
+        ctypes.c_void_p(plan.host.data_ptr()), ctypes.c_void_p(plan.on_device(dev).data_ptr()), ctypes.c_void_p(pa.data_ptr()),
         ctypes.c_void_p(po.data_ptr()), ctypes.c_void_p(lam.data_ptr()), lam_stride,
         ctypes.c_void_p(active.data_ptr()) if active is not None else ctypes.c_void_p(0), active_stride,
         ctypes.c_void_p(info.data_ptr()), ws, ws_bytes, _stream())

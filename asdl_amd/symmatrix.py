@@ -387,7 +387,7 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
     if mats_on_gpu and GROUPED_INVERSE and len(together) == len(low_rank) and not inline:
         # A few launches that leave most of the device idle: the changes of stream cost the host more than running beside
         # them saves the device.  (Low-rank factors: the Gram matrices' chain, then d^2 floats each at 3 TB/s.)
-        us = kernels.chol_group_plan([e[1].shape[0] for e in square], dev).microseconds if square else 0
+        us = kernels.chol_group_plan([e[1].shape[0] for e in square]).microseconds if square else 0
         us += 150 + sum(e[1].shape[1] ** 2 for e in together) / 750e3 if together else 0
         inline = us < INLINE_MICROSECONDS
     if mats_on_gpu and prepared and not (inline and len(prepared) <= 1 + bool(together)):

@@ -709,6 +709,32 @@ def test_workspace_belongs_to_the_stream_whose_launches_use_it(monkeypatch):
     assert not kernels._workspaces
 
 
+def test_tables_on_the_device_belong_to_the_stream_that_reads_them(monkeypatch):
+    """A cached table is uploaded asynchronously: another stream's launches would not wait for it, and when a cache is cleared its
+    memory goes back to the stream it was uploaded on.  So every stream has its own."""
+    from asdl_amd import kernels
+    uploads = []
+
+    def upload(host, device):
+        uploads.append(kernels._stream_handle(device))
+        return host.clone()
+    monkeypatch.setattr(kernels, '_upload', upload)
+    monkeypatch.setattr(kernels, '_tables', {})
+    dev = torch.device('cuda', 0)
+    plan = object.__new__(kernels.CholGroupPlan)
+    plan.host, plan._dev = torch.zeros(8, dtype=torch.uint8), {}
+    made = {}
+    for _ in range(2):
+        for handle in (3, 4):
+            with kernels.launches_on(_FakeStream(handle)):
+                made.setdefault(handle, []).append((kernels.device_ints((1, 2), dev), kernels.device_table(((1, 2),), dev),
+                                                    kernels.device_addresses((1, 2), dev), plan.on_device(dev)))
+    assert sorted(uploads) == [3] * 4 + [4] * 4
+    for first, second in made.values():
+        assert all(a is b for a, b in zip(first, second))
+    assert all(a is not b for a, b in zip(made[3][0], made[4][0]))
+
+
 def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):
     """A pass beside the inverses that raises drops them unread: what takes their memory next has to run behind them."""
     from asdl_amd import kernels, symmatrix
