@@ -11,7 +11,7 @@
 // a third of the passes over the statistics and a sixth of the launches.
 //
 // Newton iteration.  M_0 = z S, X_0 = z^(1/p) I;  T = a I - b M;  X <- X T;  M <- T^p M.  The classical step a = 1 + 1/p,
-// b = 1/p raises a small eigenvalue of M by (1 + 1/p)^p = 2.44 (p = 4): 12 of its 18 steps on a statistic of condition 1e6.
+// b = 1/p raises a small eigenvalue of M by (1 + 1/p)^p = 2.44 (p = 4): most of its 20 steps on a statistic of condition 1e6.
 // With a lower bound l of the spectrum known (from the Lanczos steps, at the least the ridge) the step that raises l most is a
 // larger a with b = a^(p+1) p^p / (p+1)^(p+1), which keeps max m (a - b m)^p = 1: up to 7.4 per step.  root_schedule_kernel
 // decides per matrix whether that is the shorter way.

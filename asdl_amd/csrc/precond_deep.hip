@@ -4,7 +4,8 @@
 // Bound by latency: a few dozen 64 x 64 tiles, K of a few hundred.  The split kernel's 128 x 128 tiles take 44 us for one
 // product of 512 x 784 on a nearly idle device and need the operands' ranges first (two more launches); a deep tile takes
 // 2 us per 128 k.  The addresses travel in the kernel arguments: no table has to be built and uploaded per step.
-// Any size and alignment.  MLP 784-512-512-10 (three modules with bias): 8 launches, 160 us -> 2 launches, 30 us.
+// Any size and alignment; the gradients of a call have to be distinct (nothing orders two items of a launch).  MLP 784-512-512-10
+// (three modules with bias): 8 launches, 160 us -> 2 launches, 25 and 34 us, their matrix pipes 15 and 17 % busy.
 #include <algorithm>
 #include "gemm_f32.hpp"
 

@@ -168,7 +168,8 @@ int ak_event_synchronize(void* event);
 
 /* grad_w <- s B_inv grad_w A_inv, grad_b <- s B_inv grad_b for many modules of any size in two launches (fp32 products).
  * items (HOST memory): rows of 6 int64: B_inv, A_inv, grad_w [dB][dA], grad_b or 0 (device addresses), dB, dA;
- * units (HOST memory): rows of 4: inv [F][2][2], grad_w [F], grad_b [F], F.  fail0 / fail1 (may be null): device words; nothing
+ * units (HOST memory): rows of 4: inv [F][2][2], grad_w [F], grad_b [F], F.  All gradients of a call are distinct (two modules
+ * that share one have to go one after the other).  fail0 / fail1 (may be null): device words; nothing
  * is written when one of them is not zero.  only_if_faster: AK_ERR_UNSUPPORTED, and nothing done, where ak_gemm_f32_grouped on
  * split operands is expected to be faster. */
 size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count);

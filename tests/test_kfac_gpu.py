@@ -463,7 +463,7 @@ def test_resnet50_batch64_channels_last_properties():
 @pytest.mark.parametrize('early_batch,late_flags', [(False, False), (True, False), (False, True)])
 def test_benchmark_path_resnet50_batch64_against_a_sequential_replay(early_batch, late_flags, monkeypatch):
     """The very code path bench.py times, at its size: ResNet-50, batch 64, channels-last, bf16 autocast, sampled
-    (MC) Fisher without EMA, the grouped inverse on a side stream fed by a worker thread beside the loss backward pass
+    (MC) Fisher without EMA, the grouped inverse on a side stream beside the loss backward pass
     (and, with ``early_batch``, a first batch started from inside the hooks of the sampled pass:
     fisher.EAGER_INVERSE_SAMPLED), the grouped preconditioning plan prepared before the flags are read.  On the
     third step (the eager path needs the cost of an earlier step) extra hooks capture, for every Conv2d / Linear,
