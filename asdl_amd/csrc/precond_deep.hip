@@ -12,6 +12,8 @@
 namespace ak {
 
 constexpr int KP_ITEMS = 24;             // modules of one launch
+// Sizes of a module and of a unit (24 of each stay far below 2^31 work groups).  Wider ones are left to the caller's other paths.
+constexpr int64_t KP_MAX_ROWS = 32768, KP_MAX_COLUMNS = 1 << 20, KP_MAX_UNIT = 1 << 24;
 constexpr int KP_GEMV_ROWS = 16;         // rows of a bias product per work group
 
 struct KpItem {
@@ -131,7 +133,8 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
   for (int i = 0; i < count; ++i) {
     const int64_t* r = items + 6 * i;
     const int64_t dB = r[4], dA = r[5];
-    if (r[0] == 0 || r[1] == 0 || r[2] == 0 || dB <= 0 || dA <= 0 || dB > 32768 || dA > (1 << 20)) return AK_ERR_ARG;
+    if (r[0] == 0 || r[1] == 0 || r[2] == 0 || dB <= 0 || dA <= 0) return AK_ERR_ARG;
+    if (dB > KP_MAX_ROWS || dA > KP_MAX_COLUMNS) return AK_ERR_UNSUPPORTED;
     for (const int64_t K : {dB, dA}) {
       const double c = static_cast<double>((K + 127) / 128), t = static_cast<double>((K + 31) / 32);
       longest = std::max(longest, c);
@@ -139,6 +142,11 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
       chunks += c * static_cast<double>(kp_tiles(dB, dA));
       ktiles += t * static_cast<double>(((dB + 127) / 128) * ((dA + 127) / 128));
     }
+  }
+  for (int i = 0; i < unit_count; ++i) {        // (all of them before the first launch)
+    const int64_t* r = units + 4 * i;
+    if (r[0] == 0 || r[1] == 0 || r[2] == 0 || r[3] <= 0) return AK_ERR_ARG;
+    if (r[3] > KP_MAX_UNIT) return AK_ERR_UNSUPPORTED;
   }
   const double deep_us = 2.0 * std::max(2 * longest, chunks / 256);
   const double split_us = std::max(2 * 1.6 * long_tile, ktiles / 256) + 20;
@@ -165,12 +173,10 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
       w += kp_tiles(r[4], r[5]);
       m.bias_first = static_cast<int>(w);
       if (m.b != nullptr) w += (r[4] + KP_GEMV_ROWS - 1) / KP_GEMV_ROWS;
-      if (w > (1 << 30)) return AK_ERR_TOO_LARGE;
     }
     a.end = static_cast<int>(w);
     for (int i = 0; i < a.units; ++i, ++unit_at) {
       const int64_t* r = units + 4 * unit_at;
-      if (r[0] == 0 || r[1] == 0 || r[2] == 0 || r[3] <= 0 || r[3] > (1 << 24)) return AK_ERR_ARG;
       KpUnit& u = a.unit[i];
       u.inv = reinterpret_cast<const float*>(r[0]); u.gw = reinterpret_cast<float*>(r[1]); u.gb = reinterpret_cast<float*>(r[2]);
       u.F = static_cast<int>(r[3]); u.first = static_cast<int>(w);

@@ -170,8 +170,8 @@ int ak_event_synchronize(void* event);
  * items (HOST memory): rows of 6 int64: B_inv, A_inv, grad_w [dB][dA], grad_b or 0 (device addresses), dB, dA;
  * units (HOST memory): rows of 4: inv [F][2][2], grad_w [F], grad_b [F], F.  All gradients of a call are distinct (two modules
  * that share one have to go one after the other).  fail0 / fail1 (may be null): device words; nothing
- * is written when one of them is not zero.  only_if_faster: AK_ERR_UNSUPPORTED, and nothing done, where ak_gemm_f32_grouped on
- * split operands is expected to be faster. */
+ * is written when one of them is not zero.  AK_ERR_UNSUPPORTED, and nothing done: a module or unit beyond the sizes of this form
+ * (dB > 32768, dA > 2^20, F > 2^24), and with only_if_faster where ak_gemm_f32_grouped on split operands is expected to be faster. */
 size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count);
 int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, int unit_count, float grad_scale,
                          const int* fail0, const int* fail1, int only_if_faster, void* ws, size_t ws_bytes,

@@ -100,6 +100,24 @@ def test_plan_of_the_grouped_inverse_says_how_long_it_takes():
     assert lib.ak_chol_group_plan_us(ctypes.create_string_buffer(256)) < 0
 
 
+def test_small_module_preconditioning_leaves_sizes_beyond_its_own_to_the_other_paths():
+    """The row matrices of the swift variant have inverses of more than 32768 columns.  The two-launch form declines them, before it
+    launches anything, instead of refusing the call."""
+    import ctypes
+    from asdl_amd import _lib, kernels
+    lib = _lib.load()
+
+    def ask(items, units, only_if_faster):
+        return lib.ak_kron_precond_deep((ctypes.c_int64 * len(items))(*items), len(items) // 6, (ctypes.c_int64 * len(units))(*units),
+                                        len(units) // 4, 1.0, 0, 0, only_if_faster, 0, 0, 0)
+    small = [16, 16, 16, 0, 8, 8]
+    for only in (0, 1):
+        assert ask(small + [16, 16, 16, 0, 40000, 8], [], only) == kernels.AK_ERR_UNSUPPORTED
+        assert ask([16, 16, 16, 0, 8, (1 << 20) + 1], [], only) == kernels.AK_ERR_UNSUPPORTED
+        assert ask([], [16, 16, 16, (1 << 24) + 1], only) == kernels.AK_ERR_UNSUPPORTED
+    assert ask([16, 16, 0, 0, 8, 8], [], 0) == -1 and ask([], [16, 16, 16, 0], 0) == -1       # (no gradient, no features: errors)
+
+
 def test_product_refuses_cpu_tensors():
     from asdl_amd import kernels
     with pytest.raises(RuntimeError, match='ROCm device'):
