@@ -189,13 +189,23 @@ def _ws_args(nbytes, device):
     return ctypes.c_void_p(buf.data_ptr()), size, buf
 
 
+_kept_for_graphs = []      # what captured launches read: a graph replays the upload of its tables from the same host memory
+
+
+def _capturing(device):
+    return device.type == 'cuda' and torch.cuda.is_current_stream_capturing()
+
+
 def _upload(host, device):
     """A host tensor on the device, staged through pinned memory and copied asynchronously on the launch stream (a pageable copy would
     block the caller behind everything that stream has queued)."""
     if device.type != 'cuda':
         return host.to(device)
     with _on_launch_stream():
-        return host.pin_memory().to(device, non_blocking=True)
+        staged = host.pin_memory()
+        if _capturing(device):
+            _kept_for_graphs.append(staged)
+        return staged.to(device, non_blocking=True)
 
 
 def _stream_key(device):
@@ -204,18 +214,28 @@ def _stream_key(device):
     return (device.index, _stream_handle(device)) if device.type == 'cuda' else (device.index, 0)
 
 
+def _cached_upload(cache, key, host, device):
+    """cache[key], or host() uploaded and kept there.  Under a stream capture the upload happens when the graph is replayed: such a
+    table is not one for eager launches, and one that is found lives as long as the process, as the graph may."""
+    t = cache.get(key)
+    capturing = _capturing(device)
+    if t is None:
+        t = _upload(host(), device)
+        if not capturing:
+            cache[key] = t
+    if capturing:
+        _kept_for_graphs.append(t)
+    return t
+
+
 _tables = {}
 MAX_TABLES = 8192
 
 
 def _device_table(kind, values, dtype, device):
-    key = (_stream_key(device), kind, values)
-    t = _tables.get(key)
-    if t is None:
-        if len(_tables) > MAX_TABLES:
-            _tables.clear()
-        t = _tables[key] = _upload(torch.tensor(values, dtype=dtype), device)
-    return t
+    if len(_tables) > MAX_TABLES:
+        _tables.clear()
+    return _cached_upload(_tables, (_stream_key(device), kind, values), lambda: torch.tensor(values, dtype=dtype), device)
 
 
 def device_ptr_array(tensors):
@@ -1290,11 +1310,7 @@ class CholGroupPlan:
         self._dev = {}
 
     def on_device(self, device):
-        key = _stream_key(device)
-        dev = self._dev.get(key)
-        if dev is None:
-            dev = self._dev[key] = _upload(self.host, device)
-        return dev
+        return _cached_upload(self._dev, _stream_key(device), lambda: self.host, device)
 
 
 def chol_group_plan(dims):

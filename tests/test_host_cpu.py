@@ -737,6 +737,7 @@ def test_tables_on_the_device_belong_to_the_stream_that_reads_them(monkeypatch):
         uploads.append(kernels._stream_handle(device))
         return host.clone()
     monkeypatch.setattr(kernels, '_upload', upload)
+    monkeypatch.setattr(kernels, '_capturing', lambda device: False)
     monkeypatch.setattr(kernels, '_tables', {})
     dev = torch.device('cuda', 0)
     plan = object.__new__(kernels.CholGroupPlan)
@@ -751,6 +752,26 @@ def test_tables_on_the_device_belong_to_the_stream_that_reads_them(monkeypatch):
     for first, second in made.values():
         assert all(a is b for a, b in zip(first, second))
     assert all(a is not b for a, b in zip(made[3][0], made[4][0]))
+
+
+def test_tables_made_under_a_stream_capture(monkeypatch):
+    """The upload of such a table is a node of the graph: it reads the staged host memory at every replay, which therefore stays, and
+    eager launches must not find a table that no replay has filled.  A table that a captured launch finds stays as well."""
+    from asdl_amd import kernels
+    capturing = [False]
+    monkeypatch.setattr(kernels, '_tables', {})
+    monkeypatch.setattr(kernels, '_kept_for_graphs', [])
+    monkeypatch.setattr(kernels, '_capturing', lambda device: capturing[0])
+    monkeypatch.setattr(kernels, '_upload', lambda host, device: host.clone())
+    dev = torch.device('cuda', 0)
+    with kernels.launches_on(_FakeStream(3)):
+        eager = kernels.device_ints((1, 2), dev)
+        capturing[0] = True
+        assert kernels.device_ints((1, 2), dev) is eager
+        inside = kernels.device_ints((3, 4), dev)
+        capturing[0] = False
+        assert kernels.device_ints((3, 4), dev) is not inside
+    assert any(t is eager for t in kernels._kept_for_graphs) and any(t is inside for t in kernels._kept_for_graphs)
 
 
 def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):

@@ -796,6 +796,40 @@ def test_smw_inv_grouped_matches_fp64(K, shapes):
         assert torch.equal(out, out.t())
 
 
+@pytest.mark.parametrize('warm', [True, False])
+def test_grouped_products_in_a_captured_graph(K, warm):
+    """Address tables under a stream capture, found (the call ran before) or made inside it: every replay, with other tables made and
+    memory reused in between, gives the eager result."""
+    g = torch.Generator('cuda').manual_seed(2)
+    problems, expected = [], []
+    for n in (96, 200):
+        A, B = torch.randn(n, 64, device='cuda', generator=g), torch.randn(64, n, device='cuda', generator=g)
+        problems.append((A, B, torch.zeros(n, n, device='cuda'), False, False, 1.0))
+        expected.append((A.double() @ B.double()).float())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        if warm:
+            K.gemm_grouped(problems)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side, capture_error_mode='thread_local'):
+            K.gemm_grouped(problems)
+    torch.cuda.synchronize()
+    K._tables.clear()
+    for _ in range(4):
+        for i in range(20):
+            K.device_ints(tuple(range(i, i + 40)), torch.device('cuda'))
+            torch.full((512,), -1, dtype=torch.int64).pin_memory()
+        for p in problems:
+            p[2].zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for p, want in zip(problems, expected):
+            assert relerr(p[2], want) < 1e-5
+
+
 # ------------------------------------------------------------------ sampling
 @pytest.mark.parametrize('shape', [(1, 2), (5, 10), (64, 1000), (3, 1023), (9, 1024), (4, 1025), (2, 3, 5001)])
 def test_sample_categorical_draws_what_torch_draws(K, shape):
