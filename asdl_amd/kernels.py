@@ -172,12 +172,14 @@ def workspace(nbytes, device):
             with _on_launch_stream():
                 buf = torch.empty(size, dtype=torch.uint8, device=device)
             _workspaces[key] = buf
+        if _capturing(buf.device):
+            _kept_for_graphs.append(buf)
     return buf, buf.numel()
 
 
 def release_workspaces():
     """Gives the scratch buffers of all streams back to the caching allocator; the next calls allocate them again.  (Launches that
-    still use one are safe: see workspace().  Plans that hold a buffer keep it.)"""
+    still use one are safe: see workspace().  Plans that hold a buffer keep it, and so do captured graphs.)"""
     with _ws_lock:
         _workspaces.clear()
 

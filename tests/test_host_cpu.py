@@ -2,6 +2,7 @@
 orchestration, with the kernel entry points replaced by oracle-backed stand-ins
 (tests/cpu_backend.py).  Also checks that the C-ABI library loads and exports every declared symbol
 and that the product refuses CPU tensors."""
+import contextlib
 import copy
 import os
 
@@ -704,7 +705,6 @@ def test_threads_do_not_interleave_their_launches_on_one_side_stream(monkeypatch
 def test_workspace_belongs_to_the_stream_whose_launches_use_it(monkeypatch):
     """A workspace that is replaced by a larger one goes back to the stream it was allocated on.  If that was the caller's stream
     while a side stream's launches used it, the caller's next tensor would take the memory under those launches."""
-    import contextlib
     from asdl_amd import kernels
     current, allocated = ['main'], []
 
@@ -771,7 +771,14 @@ def test_tables_made_under_a_stream_capture(monkeypatch):
         inside = kernels.device_ints((3, 4), dev)
         capturing[0] = False
         assert kernels.device_ints((3, 4), dev) is not inside
-    assert any(t is eager for t in kernels._kept_for_graphs) and any(t is inside for t in kernels._kept_for_graphs)
+        monkeypatch.setattr(kernels, '_workspaces', {})
+        monkeypatch.setattr(kernels, '_on_launch_stream', contextlib.nullcontext)
+        capturing[0] = True
+        scratch, _ = kernels.workspace(1 << 20, torch.device('cpu', 0))
+        capturing[0] = False
+        kernels.release_workspaces()
+    for t in (eager, inside, scratch):
+        assert any(t is k for k in kernels._kept_for_graphs)
 
 
 def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):
