@@ -173,7 +173,7 @@ def workspace(nbytes, device):
                 buf = torch.empty(size, dtype=torch.uint8, device=device)
             _workspaces[key] = buf
         if _capturing(buf.device):
-            _kept_for_graphs.append(buf)
+            _kept_for_graphs[id(buf)] = buf
     return buf, buf.numel()
 
 
@@ -191,7 +191,7 @@ def _ws_args(nbytes, device):
     return ctypes.c_void_p(buf.data_ptr()), size, buf
 
 
-_kept_for_graphs = []      # what captured launches read: a graph replays the upload of its tables from the same host memory
+_kept_for_graphs = {}      # by id: what captured launches read (a graph replays the upload of its tables from the same host memory)
 
 
 def _capturing(device):
@@ -206,7 +206,7 @@ def _upload(host, device):
     with _on_launch_stream():
         staged = host.pin_memory()
         if _capturing(device):
-            _kept_for_graphs.append(staged)
+            _kept_for_graphs[id(staged)] = staged
         return staged.to(device, non_blocking=True)
 
 
@@ -226,7 +226,7 @@ def _cached_upload(cache, key, host, device):
         if not capturing:
             cache[key] = t
     if capturing:
-        _kept_for_graphs.append(t)
+        _kept_for_graphs[id(t)] = t
     return t
 
 

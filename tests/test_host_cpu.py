@@ -760,7 +760,7 @@ def test_tables_made_under_a_stream_capture(monkeypatch):
     from asdl_amd import kernels
     capturing = [False]
     monkeypatch.setattr(kernels, '_tables', {})
-    monkeypatch.setattr(kernels, '_kept_for_graphs', [])
+    monkeypatch.setattr(kernels, '_kept_for_graphs', {})
     monkeypatch.setattr(kernels, '_capturing', lambda device: capturing[0])
     monkeypatch.setattr(kernels, '_upload', lambda host, device: host.clone())
     dev = torch.device('cuda', 0)
@@ -778,7 +778,7 @@ def test_tables_made_under_a_stream_capture(monkeypatch):
         capturing[0] = False
         kernels.release_workspaces()
     for t in (eager, inside, scratch):
-        assert any(t is k for k in kernels._kept_for_graphs)
+        assert kernels._kept_for_graphs[id(t)] is t
 
 
 def test_inverses_dropped_unfinished_are_waited_for(monkeypatch):
