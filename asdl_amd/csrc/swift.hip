@@ -18,6 +18,8 @@ struct PatchSumParams {
   int64_t ldo;
 };
 
+constexpr int kPatchSumEdge = 1024;    // longest plane edge of patch_sum_plane_kernel's tables
+
 template <typename T>
 __device__ __forceinline__ float ps_load(const T* p);
 template <>
@@ -85,8 +87,81 @@ static __global__ __launch_bounds__(256) void patch_sum_chan_kernel(PatchSumPara
   }
 }
 
-// Any other layout (NCHW: columns innermost): one wave per (n, c, tap), lanes along the output columns, rows walked
-// serially, wave reduction at the end.  grid (kh*kw, C, N), 64 threads.
+// Any other layout (NCHW: columns innermost), 1 x 1 and 3 x 3 windows: G lanes hold one (n, c) plane and read each of
+// its elements once; the element goes to the sums of the taps whose window it lies in.  Which taps those are depends
+// on its row and its column alone: two tables of KH / KW bits in the LDS, so that stride, padding and borders cost
+// one LDS read each per element.  Bound by the plane's one reading and, for small planes, by the launch.  The taps of
+// a wave per (n, c, tap) read the plane KH * KW times with Wo of 64 lanes at work: N = 64, 3 x 3, 64 x 32 x 32
+// 76 -> 14 us, 512 x 4 x 4 114 -> 6.4 us (fp32).
+template <typename T, int KH, int KW>
+static __global__ __launch_bounds__(256) void patch_sum_plane_kernel(PatchSumParams p, int G, uint32_t mW) {
+  constexpr int TAPS = KH * KW;
+  __shared__ unsigned char row_taps[kPatchSumEdge], col_taps[kPatchSumEdge];
+  __shared__ float part[4][TAPS];
+  for (int i = threadIdx.x; i < p.H; i += 256) {
+    int bits = 0;
+#pragma unroll
+    for (int k = 0; k < KH; ++k) {
+      const int r = i + p.ph - k;
+      if (r >= 0 && r % p.strh == 0 && r / p.strh < p.Ho) bits |= 1 << k;
+    }
+    row_taps[i] = static_cast<unsigned char>(bits);
+  }
+  for (int i = threadIdx.x; i < p.W; i += 256) {
+    int bits = 0;
+#pragma unroll
+    for (int k = 0; k < KW; ++k) {
+      const int r = i + p.pw - k;
+      if (r >= 0 && r % p.strw == 0 && r / p.strw < p.Wo) bits |= 1 << k;
+    }
+    col_taps[i] = static_cast<unsigned char>(bits);
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & (G - 1);                              // G: a power of two, 8 ... 64, or 256
+  const int64_t plane = static_cast<int64_t>(blockIdx.x) * (256 / G) + threadIdx.x / G;
+  const bool live = plane < static_cast<int64_t>(p.N) * p.C;
+  const int64_t n = live ? plane / p.C : 0, c = live ? plane - n * p.C : 0;
+  const T* __restrict__ base = static_cast<const T*>(p.x) + n * p.sn + c * p.sc;
+  const int total = live ? p.H * p.W : 0;
+  float acc[TAPS];
+#pragma unroll
+  for (int t = 0; t < TAPS; ++t) acc[t] = 0.f;
+#pragma unroll 4
+  for (int e = lane; e < total; e += G) {
+    const int iy = static_cast<int>(fastdiv(e, mW, p.W)), ix = e - iy * p.W;
+    const float v = ps_load<T>(base + static_cast<int64_t>(iy) * p.sh + static_cast<int64_t>(ix) * p.sw);
+    const int rt = row_taps[iy], ct = col_taps[ix];
+#pragma unroll
+    for (int ky = 0; ky < KH; ++ky)
+#pragma unroll
+      for (int kx = 0; kx < KW; ++kx)                                  // selected, not multiplied: an infinity outside a window stays out
+        acc[ky * KW + kx] += ((rt >> ky) & (ct >> kx) & 1) ? v : 0.f;
+  }
+#pragma unroll
+  for (int t = 0; t < TAPS; ++t)
+    for (int o = (G < 64 ? G : 64) >> 1; o > 0; o >>= 1) acc[t] += __shfl_xor(acc[t], o);
+  if (G == 256) {
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+      for (int t = 0; t < TAPS; ++t) part[threadIdx.x >> 6][t] = acc[t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t) acc[t] = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+  }
+  if (!live) return;
+  float* __restrict__ dst = p.out + n * p.ldo + c * TAPS;
+#pragma unroll
+  for (int t = 0; t < TAPS; ++t) {
+    if (lane != (t & (G - 1))) continue;
+    float v = p.alpha * acc[t];
+    if (p.beta != 0.f) v += p.beta * dst[t];
+    dst[t] = v;
+  }
+}
+
+// Other windows of such a layout, and planes longer than the tables: one wave per (n, c, tap), lanes along the output
+// columns, rows walked serially, wave reduction at the end.  grid (kh*kw, C, N), 64 threads.
 template <typename T>
 static __global__ __launch_bounds__(64) void patch_sum_col_kernel(PatchSumParams p) {
   const int tap = blockIdx.x, c = blockIdx.y, n = blockIdx.z, lane = threadIdx.x;
@@ -156,6 +231,23 @@ extern "C" int ak_conv_patch_sum(const void* x, int dtype, int64_t sn, int64_t s
     if (vec8) hipLaunchKernelGGL((ak::patch_sum_chan_kernel<uint16_t, 8>), grid, dim3(256), 0, s, p, cch);
     else if (dtype == AK_BF16) hipLaunchKernelGGL((ak::patch_sum_chan_kernel<uint16_t, 1>), grid, dim3(256), 0, s, p, cch);
     else hipLaunchKernelGGL((ak::patch_sum_chan_kernel<float, 1>), grid, dim3(256), 0, s, p, cch);
+  } else if (((kh == 1 && kw == 1) || (kh == 3 && kw == 3)) && H <= ak::kPatchSumEdge && W <= ak::kPatchSumEdge &&
+             N * C < (1 << 24)) {
+    // N * C * 256 lanes fit the 32-bit grid.  About four elements a lane; from 2048 elements on a whole work group, so that 192 planes of an image still
+    // keep loads in flight (H * W * W < 2^32: the magic division is exact)
+    int G = 8;
+    while (G < 64 && 4 * G < H * W) G *= 2;
+    if (H * W >= 2048) G = 256;
+    const int64_t blocks = (N * C + 256 / G - 1) / (256 / G);
+    const dim3 grid(static_cast<unsigned>(blocks));
+    const uint32_t mW = ak::make_magic(static_cast<uint32_t>(W));
+    if (kh == 1) {
+      if (dtype == AK_BF16) hipLaunchKernelGGL((ak::patch_sum_plane_kernel<uint16_t, 1, 1>), grid, dim3(256), 0, s, p, G, mW);
+      else hipLaunchKernelGGL((ak::patch_sum_plane_kernel<float, 1, 1>), grid, dim3(256), 0, s, p, G, mW);
+    } else {
+      if (dtype == AK_BF16) hipLaunchKernelGGL((ak::patch_sum_plane_kernel<uint16_t, 3, 3>), grid, dim3(256), 0, s, p, G, mW);
+      else hipLaunchKernelGGL((ak::patch_sum_plane_kernel<float, 3, 3>), grid, dim3(256), 0, s, p, G, mW);
+    }
   } else {
     if (C > 65535) return AK_ERR_UNSUPPORTED;
     dim3 grid(kh * kw, static_cast<unsigned>(C), static_cast<unsigned>(N));

@@ -1275,3 +1275,23 @@ def test_kron_damping_with_row_matrices(K):
                                     B * (sb if B.shape[0] == B.shape[1] else sb ** 0.5), 1e-2)
         assert abs(float(lam[i, 0]) - want[0]) < 1e-5 * want[0] and abs(float(lam[i, 1]) - want[1]) < 1e-5 * want[1]
     assert nz.tolist() == [[1, 1], [1, 1], [1, 1], [0, 1]]
+
+
+# Positions are summed per plane: sizes around one lane's share, a wave's and a work group's, both windows, strides with
+# elements that no window takes, planes that are slices of wider ones, and an infinity that only some taps see.
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('case', [(3, 5, 1, 1, 1, 1, 0), (2, 7, 4, 4, 3, 1, 1), (3, 33, 5, 7, 3, 2, 1), (2, 3, 16, 16, 3, 1, 1), (2, 5, 17, 15, 3, 3, 0),
+                                  (1, 3, 45, 46, 3, 1, 2), (2, 2, 64, 33, 3, 2, 1), (5, 4, 9, 9, 1, 2, 0), (1, 2, 1024, 3, 3, 1, 1), (1, 2, 1025, 3, 3, 1, 1)])
+def test_patch_sum_of_planes(K, dtype, case):
+    N, C, H, W, k, s, p = case
+    wide = _inputs((N, C, H, W + 3), dtype, seed=H * W)
+    x = wide[..., 1:W + 1]
+    want = torch.nn.functional.unfold(x.double(), k, padding=p, stride=s).sum(-1)
+    size = torch.nn.functional.unfold(x.double().abs(), k, padding=p, stride=s).sum(-1)
+    print(f'patch_sum dtype={dtype} case={case}', flush=True)
+    out = K.conv_patch_sum(wide.cuda()[..., 1:W + 1], (k, k), (s, s), (p, p))
+    # a chain of additions of a lane and a tree over the lanes: 64 additions at most, 2^-24 of the sum of magnitudes each
+    assert bool(((out.double().cpu() - want).abs() <= 64 * 2.0 ** -24 * size + 1e-30).all())
+    x[0, 0, 0, 0] = float('inf')
+    sees = torch.isinf(torch.nn.functional.unfold(x.double(), k, padding=p, stride=s)).any(-1)
+    assert torch.equal(torch.isinf(K.conv_patch_sum(wide.cuda()[..., 1:W + 1], (k, k), (s, s), (p, p))).cpu(), sees)
