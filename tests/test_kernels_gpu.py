@@ -1295,3 +1295,20 @@ def test_patch_sum_of_planes(K, dtype, case):
     x[0, 0, 0, 0] = float('inf')
     sees = torch.isinf(torch.nn.functional.unfold(x.double(), k, padding=p, stride=s)).any(-1)
     assert torch.equal(torch.isinf(K.conv_patch_sum(wide.cuda()[..., 1:W + 1], (k, k), (s, s), (p, p))).cpu(), sees)
+
+
+@pytest.mark.parametrize('rows,d', [(1, 2), (3, 1365), (64, 512), (64, 513), (5, 8193)])
+def test_kron_damping_of_row_matrices_at_any_alignment(K, rows, d):
+    g = torch.Generator().manual_seed(d)
+    flat = torch.randn(rows * d + 1, generator=g)
+    b = torch.eye(d + rows + 1) * 2
+    for skip in (0, 1):
+        a = flat[skip:skip + rows * d].view(rows, d)
+        lam, nz = K.kron_damping([flat.cuda()[skip:skip + rows * d].view(rows, d)], [b.cuda()], 1e-2)
+        pi = ((a.double() ** 2).sum() / d / 2).sqrt()
+        assert nz.tolist() == [[1, 1]]
+        assert abs(float(lam[0, 0]) - 0.1 * float(pi)) < 1e-5 * 0.1 * float(pi) and abs(float(lam[0, 1]) - 0.1 / float(pi)) < 1e-5 * 0.1 / float(pi)
+    last = torch.zeros(rows, d)
+    last[-1, -1] = 1e-30
+    assert K.kron_damping([last.cuda()], [b.cuda()], 1e-2)[1].tolist() == [[1, 1]]
+    assert K.kron_damping([torch.zeros(rows, d).cuda()], [b.cuda()], 1e-2)[1].tolist() == [[0, 1]]
