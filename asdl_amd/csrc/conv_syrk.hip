@@ -566,9 +566,8 @@ static int launch_conv_syrk_t(ConvPlan& plan, hipStream_t stream) {
   dim3 grid(static_cast<unsigned>(plan.ntiles), static_cast<unsigned>(plan.p.nsplit));
   hipLaunchKernelGGL(kern, grid, dim3(256), plan.lds_bytes, stream, plan.p);
   if (plan.p.nsplit > 1)
-    hipLaunchKernelGGL((syrk_finalize_kernel<TI, TI>), dim3(static_cast<unsigned>(plan.ntiles), 4 * TI * TI), dim3(256), 0,
-                       stream, static_cast<const float*>(plan.p.ws), plan.p.nsplit, plan.p.T, plan.p.A, plan.p.lda,
-                       plan.p.d, plan.p.alpha, plan.p.beta);
+    launch_syrk_finalize<TI>(static_cast<const float*>(plan.p.ws), plan.p.nsplit, plan.ntiles, plan.p.T, plan.p.A, plan.p.lda,
+                             plan.p.d, plan.p.alpha, plan.p.beta, stream);
   return check_launch();
 }
 

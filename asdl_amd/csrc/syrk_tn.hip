@@ -220,8 +220,7 @@ static int launch_syrk_tn(const void* X, int64_t M, int64_t d, int64_t ldx, floa
   }
   hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, stream, p);
   if (nsplit > 1)
-    hipLaunchKernelGGL((syrk_finalize_kernel<TI, TI>), dim3(static_cast<unsigned>(ntiles), 4 * TI * TI), dim3(256), 0, stream,
-                       static_cast<const float*>(ws), nsplit, static_cast<int>(Tn), C, ldc, d, alpha, beta);
+    launch_syrk_finalize<TI>(static_cast<const float*>(ws), nsplit, ntiles, static_cast<int>(Tn), C, ldc, d, alpha, beta, stream);
   return check_launch();
 }
 

@@ -1312,3 +1312,14 @@ def test_kron_damping_of_row_matrices_at_any_alignment(K, rows, d):
     last[-1, -1] = 1e-30
     assert K.kron_damping([last.cuda()], [b.cuda()], 1e-2)[1].tolist() == [[1, 1]]
     assert K.kron_damping([torch.zeros(rows, d).cuda()], [b.cuda()], 1e-2)[1].tolist() == [[0, 1]]
+
+
+# Split counts around the limits of the reduction's slices (4 | 5, 63 | 64), one tile and several, one-tile windows
+@pytest.mark.parametrize('N,C,hw,beta', [(1, 64, 40 * 8, 0.0), (3, 64, 41 * 8, 0.5), (63, 64, 256, 0.0), (64, 60, 256, 0.5), (70, 128, 512, 0.0), (40, 130, 256, 0.5), (9, 500, 64, 0.0)])
+def test_split_reductions_match_fp64(K, N, C, hw, beta):
+    x = _inputs((N, C, hw // 8, 8), torch.float32, N + C)
+    rows = x.double().permute(0, 2, 3, 1).reshape(-1, C)
+    old = torch.ones(C, C)
+    out = old.cuda()
+    K.conv_syrk(x.cuda(), (1, 1), (1, 1), (0, 0), out=out, alpha=0.5, beta=beta)
+    assert relerr(out, 0.5 * rows.T @ rows + beta * old.double()) < TOL_FACTOR_F32 and torch.equal(out, out.T)
