@@ -32,7 +32,9 @@
 namespace ak {
 
 constexpr int kPlaneTile = 192, kPlaneSmallTile = 64;
-constexpr int kErrStride = 16;          // floats between error words: a cache line each, all tiles of all matrices fold into theirs at once
+// Error words: a cache line each, kErrSlots per matrix.  All tiles of a matrix fold into theirs at once, and an atomic on a line
+// that others are on takes 60 ns: with one word for the 91 tiles of 784 columns 5 us of the product.
+constexpr int kErrStride = 16, kErrSlots = 16;
 constexpr int kPlaneLdsBytes = 4 * 6 * 6 * 16 * 64;      // four stages of six plane panels of six [16 rows][64 bytes] blocks
 constexpr int kPlaneMaxDim = 16128;      // 32-bit byte offsets inside a plane set, virtual k-tile numbers below 2^15
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -54,7 +56,7 @@ struct PlaneGemm {
   const float* coef;        // C2 = coef[2 (count + 1)] I - coef[2 (count + 1) + 1] C of the entry's own table
   int64_t coef_stride;
   int coef_last;            // steps beyond the table take its last entry
-  float* errword;           // optional, one word per batch entry, kErrStride apart
+  float* errword;           // optional, kErrSlots words per batch entry, kErrStride apart
   const int* active;        // entry z runs only if active[z] != 0
   int* overflow;            // fp16 form: word z is set when a value of C or C2 does not fit the fp16 range
   int64_t plane_elems;      // n_pad * n_pad
@@ -91,80 +93,83 @@ __device__ __forceinline__ void plane_bits(float x, unsigned short (&o)[3]) {
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
-// Epilogue of a tile: planes of C (and of C2 = c2_scale C + c2_diag I), the mirror image of an off-diagonal tile, the
-// error word max |C - I|.  sum(r): a wave's sums of the 64 x 64 tile, one 32 x 32 block each.
-template <int NP, class Sum>
-__device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int tj, int z, Sum sum) {
-  constexpr int WC = 2, TILE = kPlaneSmallTile;
-  // (the empty statement keeps the address arithmetic below from being moved above the k-loop of the caller, where
-  // every register is taken)
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
-  asm volatile("" : "+s"(z));
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = wave / WC, wc = wave % WC, g = lane >> 5, l32 = lane & 31;
-  const int i0 = ti * TILE, j0 = tj * TILE;
-  const int steps = p.count[z], parity = steps & 1;
+// Wave (group q of GROUPS, block w of BLOCKS) holds chunk first + q of block w: every wave gets its 4 / GROUPS register quads
+// of its block, the chunks first ... first + G - 1 (< chunks) added to `tot` in order.  part: 4 G BLOCKS KB of LDS that
+// nothing else uses once all waves have arrived.
+template <int BLOCKS, int GROUPS>
+__device__ __forceinline__ void add_chunks(const floatx16& acc, floatx4 (&tot)[4 / GROUPS], int first, int chunks, int q, int w, int G,
+                                           AK_LDS floatx4* part) {
+  const int lane = threadIdx.x & 63;
+  __syncthreads();
+  if (q < G && first + q < chunks) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      part[((q * BLOCKS + w) * 4 + k) * 64 + lane] = floatx4{acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]};
+  }
+  __syncthreads();
+  for (int c = 0; c < G && first + c < chunks; ++c) {
+#pragma unroll
+    for (int k = 0; k < 4 / GROUPS; ++k) {
+      const floatx4 v = part[((c * BLOCKS + w) * 4 + q * (4 / GROUPS) + k) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tot[k][e] += v[e];
+    }
+  }
+}
+
+// Epilogue of a quarter of a wave's 32 x 32 block of a 64 x 64 tile, rows 8 q + 4 g + e of it: planes of C (and of
+// C2 = c2_scale C + c2_diag I), the mirror image of an off-diagonal tile, the lanes' largest |C - I| and whether all fits.
+template <int NP>
+__device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int tj, int z, int wr, int wc, int q, floatx4 sum,
+                                               int parity, float c2_diag, float c2_scale, float& vmax, bool& fits) {
+  const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
+  const int i0 = ti * kPlaneSmallTile, j0 = tj * kPlaneSmallTile;
   unsigned short* __restrict__ sets = reinterpret_cast<unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
   unsigned short* __restrict__ C = sets + paired_buf(p.C, parity) * p.buf_elems;
   unsigned short* __restrict__ C2 = p.C2.index >= 0 ? sets + paired_buf(p.C2, parity) * p.buf_elems : nullptr;
-  float c2_diag = 0.f, c2_scale = 0.f;
-  if (C2 != nullptr) {
-    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
-    c2_diag = next[0];
-    c2_scale = -next[1];
-  }
   const bool off_diag = ti != tj;
   const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
-  float vmax = 0.f;
-  bool fits = true;
-  const int gj = j0 + 32 * wc + l32;
+  const int gj = j0 + 32 * wc + l32, gi = i0 + 32 * wr + 8 * q + 4 * g;      // rows gi .. gi + 3
+  u16x4 m1[NP], m2[NP];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int gi = i0 + 32 * wr + 8 * q + 4 * g;      // rows gi .. gi + 3
-    u16x4 m1[NP], m2[NP];
+  for (int e = 0; e < 4; ++e) {
+    const float v = sum[e] * unscale;
+    const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
+    if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+    unsigned short o[3];
+    if constexpr (NP == 2) fits = fits && fabsf(v * cs) <= 65504.f;      // (false for a NaN too)
+    plane_bits<NP>(v * cs, o);
+    // a diagonal tile keeps its upper triangle and mirrors it element by element: the next product reads
+    // this matrix as its own transpose, which it has to be exactly
+    const bool keep = off_diag || gi + e <= gj;
+    const int64_t at = plane_index(gi + e, gj, p.n_pad);
+    const int64_t mirror = plane_index(gj, gi + e, p.n_pad);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float v = sum(4 * q + e) * unscale;
-      const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
-      if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
-      unsigned short o[3];
-      if constexpr (NP == 2) fits = fits && fabsf(v * cs) <= 65504.f;      // (false for a NaN too)
-      plane_bits<NP>(v * cs, o);
-      // a diagonal tile keeps its upper triangle and mirrors it element by element: the next product reads
-      // this matrix as its own transpose, which it has to be exactly
-      const bool keep = off_diag || gi + e <= gj;
-      const int64_t at = plane_index(gi + e, gj, p.n_pad);
-      const int64_t mirror = plane_index(gj, gi + e, p.n_pad);
-#pragma unroll
-      for (int s = 0; s < NP; ++s) {
-        if (keep) C[s * p.plane_elems + at] = o[s];
-        if (!off_diag && gi + e < gj) C[s * p.plane_elems + mirror] = o[s];
-        m1[s][e] = o[s];
-      }
-      if (C2 != nullptr) {
-        const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
-        if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
-        plane_bits<NP>(w * c2s, o);
-#pragma unroll
-        for (int s = 0; s < NP; ++s) {
-          if (keep) C2[s * p.plane_elems + at] = o[s];
-          if (!off_diag && gi + e < gj) C2[s * p.plane_elems + mirror] = o[s];
-          m2[s][e] = o[s];
-        }
-      }
+    for (int s = 0; s < NP; ++s) {
+      if (keep) C[s * p.plane_elems + at] = o[s];
+      if (!off_diag && gi + e < gj) C[s * p.plane_elems + mirror] = o[s];
+      m1[s][e] = o[s];
     }
-    if (off_diag) {        // C[gj][gi .. gi + 3]: four consecutive elements of a row (gi is a multiple of 4)
-      const int64_t at = plane_index(gj, gi, p.n_pad);
+    if (C2 != nullptr) {
+      const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
+      if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
+      plane_bits<NP>(w * c2s, o);
 #pragma unroll
       for (int s = 0; s < NP; ++s) {
-        *reinterpret_cast<u16x4*>(C + s * p.plane_elems + at) = m1[s];
-        if (C2 != nullptr) *reinterpret_cast<u16x4*>(C2 + s * p.plane_elems + at) = m2[s];
+        if (keep) C2[s * p.plane_elems + at] = o[s];
+        if (!off_diag && gi + e < gj) C2[s * p.plane_elems + mirror] = o[s];
+        m2[s][e] = o[s];
       }
     }
   }
-  if (p.errword != nullptr) gemm_store_absmax(p.errword + static_cast<int64_t>(z) * kErrStride, vmax, lane);
-  if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
+  if (off_diag) {        // C[gj][gi .. gi + 3]: four consecutive elements of a row (gi is a multiple of 4)
+    const int64_t at = plane_index(gj, gi, p.n_pad);
+#pragma unroll
+    for (int s = 0; s < NP; ++s) {
+      *reinterpret_cast<u16x4*>(C + s * p.plane_elems + at) = m1[s];
+      if (C2 != nullptr) *reinterpret_cast<u16x4*>(C2 + s * p.plane_elems + at) = m2[s];
+    }
+  }
 }
 
 // The same epilogue for the 192-wide tile, through the LDS, which the k-loop has left free: the tile is written there
@@ -356,7 +361,8 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
     vmax = __builtin_bit_cast(float, vmax_bits) * (1.f / cs);             // (a power of two)
     fits = NP != 2 || max(max(upper[0], upper[1]), max(upper[2], upper[3])) < 0x7c00;
   }
-  if (p.errword != nullptr) gemm_store_absmax(p.errword + static_cast<int64_t>(z) * kErrStride, vmax, lane);
+  if (p.errword != nullptr)
+    gemm_store_absmax(p.errword + (static_cast<int64_t>(z) * kErrSlots + blockIdx.x % kErrSlots) * kErrStride, vmax, lane);
   if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
 }
 
@@ -671,21 +677,39 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   plane_epilogue_wide<2>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
-// A 64 x 64 tile (ti <= tj) for groups with too few 192-wide tiles to fill the device: 4 waves (2 x 2) of one 32 x 32 block.
-// A tile is bound by the latency of its operands, so a stage is 64 rows of all plane panels (32 KB with two planes, 48 with
-// three) and all but one of the stages are requested ahead; one barrier per stage.  Every element is summed in the order of
-// the 192-wide tile (piece products of 16 k, chunks of 256 k): the same bits, whichever tile a group takes.
-template <int NP>
-__device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int tj, int z, AK_LDS unsigned char* lds) {
-  constexpr int BK = 64, BLOCK = BK * 64, LOADS = 4 * NP, STAGE = LOADS * BLOCK, S = NP == 2 ? 4 : 3;
-  constexpr int CHUNK = 256 / BK;
-  static_assert(S * STAGE <= kPlaneLdsBytes, "LDS");
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-  const int parity = p.count[z] & 1;
+// A 64 x 64 tile (ti <= tj) for groups with too few 192-wide tiles to fill the device: 16 waves, of which group q = wave / 4
+// sums the chunk of 256 k number q of every G (G = 4, 2, 1: as many as the matrix has chunks), its four waves one 32 x 32
+// block each.  Every element is summed in the order of the 192-wide tile (piece products of 16 k, chunks of 256 k, the chunks
+// in order through the LDS): the same bits, whichever tile a group takes.
+// Bound by latencies one after the other: the launch with the way to the matrix's step count 4 us, the first operands 1.5, the
+// ring 4 (S stages of 16 k per group keep 100 KB requested on the CU; the matrix instructions hide behind it), the sums 0.5,
+// the two-byte stores and their way out of the L2 3 per result.  One product at 784 columns and four at 512 in one launch, two of them
+// in one launch, one with a second result: 17.2, 28.8, 24.0 us with four waves a tile for all chunks, 14.5, 22.9, 18.7 so.
+// Launches with more tiles than CUs take half as many waves and LDS a tile, two tiles to a CU.
+template <int NP, int GROUPS> constexpr int kSmallTileStages = (NP == 2 ? 4 : 3) * GROUPS;          // of all groups together
+template <int NP, int GROUPS> constexpr int kSmallTileLds = kSmallTileStages<NP, GROUPS> * 4 * NP * 1024;
+
+// Waits until at most `stages` stages of LOADS loads are in flight (a constant once the caller's loop is unrolled).
+template <int LOADS>
+__device__ __forceinline__ void wait_loads(std::integral_constant<int, LOADS>, int stages) {
+#define AK_WAIT(n) case n: wait_vmcnt<(n) * LOADS>(); break;
+  switch (stages) {
+    AK_WAIT(0) AK_WAIT(1) AK_WAIT(2) AK_WAIT(3) AK_WAIT(4) AK_WAIT(5) AK_WAIT(6) AK_WAIT(7) AK_WAIT(8) AK_WAIT(9) AK_WAIT(10)
+    AK_WAIT(11) AK_WAIT(12) AK_WAIT(13) AK_WAIT(14)
+    default: wait_vmcnt<0>();
+  }
+#undef AK_WAIT
+}
+
+template <int NP, int GROUPS, int G>
+__device__ __forceinline__ void plane_tile_chunks(const PlaneGemm& p, int ti, int tj, int z, int parity, AK_LDS unsigned char* lds,
+                                                  floatx4 (&tot)[4 / GROUPS]) {
+  constexpr int BK = 16, BLOCK = BK * 64, STAGE = 4 * NP * BLOCK, S = kSmallTileStages<NP, GROUPS> / G, LOADS = NP, CHUNK = 256 / BK;
+  static_assert((S - 1) * LOADS < 64 && kSmallTileLds<NP, GROUPS> >= G * 16384, "loads in flight; the chunks' sums");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave >> 1, wc = wave & 1;
-  const int nk = p.n_pad / BK;
+  const int group = wave >> 2, w = wave & 3, wr = w >> 1, wc = w & 1;
+  const int nk = p.n_pad / BK, chunks = (nk + CHUNK - 1) / CHUNK;
   const uint32_t plane_bytes = static_cast<uint32_t>(p.plane_elems) * 2u, colblock_bytes = static_cast<uint32_t>(p.n_pad) * 64u;
   u32x4 rsrc[2];
 #pragma unroll
@@ -697,68 +721,93 @@ __device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int
     rsrc[P][2] = kDtlRange;
     rsrc[P][3] = 0x00020000u;
   }
-  // block l = (operand P, plane q, column block cb) of a stage is 4 KB of consecutive bytes, one for each wave
-  const uint32_t lane_off = static_cast<uint32_t>(wave * 1024 + lane * 16);
+  AK_LDS unsigned char* ring = lds + group * S * STAGE;
+  const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
+  // block (operand P, plane q, column block cb) of a stage: 16 rows x 64 bytes, 1 KB of consecutive bytes
   auto issue = [&](int kt, int stage) {
 #pragma unroll
     for (int l = 0; l < LOADS; ++l) {
-      const int P = l / (2 * NP), q = (l / 2) % NP, cb = l & 1;
+      const int blk = w * LOADS + l, P = blk / (2 * NP), q = (blk / 2) % NP, cb = blk & 1;
       const uint32_t col = static_cast<uint32_t>(2 * (P == 0 ? ti : tj) + cb) * colblock_bytes;
-      load_to_lds(rsrc[P], lds0 + stage * STAGE + l * BLOCK + wave * 1024,
-                  kt < nk ? static_cast<uint32_t>(kt * BK) * 64u + lane_off + q * plane_bytes + col : 0u);
+      const u32x4 d = P == 0 ? rsrc[0] : rsrc[1];
+      load_to_lds(d, ring0 + stage * STAGE + blk * BLOCK,
+                  (kt < nk ? static_cast<uint32_t>(kt * BK) * 64u + q * plane_bytes + col : 0u) + lane * 16u);
     }
   };
   const int g = lane >> 5, hl = (lane >> 4) & 1, j16 = lane & 15;
   const int frag_lane = (8 * g + (j16 >> 2)) * 64 + hl * 32 + (j16 & 3) * 8;
-  AK_LDS const unsigned char* fragI = lds + frag_lane + wr * BLOCK;
-  AK_LDS const unsigned char* fragJ = lds + frag_lane + (2 * NP + wc) * BLOCK;
+  AK_LDS const unsigned char* fragI = ring + frag_lane + wr * BLOCK;
+  AK_LDS const unsigned char* fragJ = ring + frag_lane + (2 * NP + wc) * BLOCK;
   auto frag = [](AK_LDS const unsigned char* q) {
     return pack_bf16x8(__builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(q)),
                        __builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(q + 256)));
   };
-  floatx16 acc, tot;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) tot[r] = acc[r] = 0.f;
+  for (int k = 0; k < 4 / GROUPS; ++k) tot[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int first = 0; first < chunks; first += G) {
+    const int kt0 = (first + group) * CHUNK;
+    floatx16 acc;
 #pragma unroll
-  for (int t = 0; t < S - 1; ++t) issue(t, t);
-  int stage = 0;
-  for (int kt = 0; kt < nk; ++kt) {
-    wait_vmcnt<(S - 2) * LOADS>();               // this wave's part of k-tile kt has landed, then everybody's; and all are
-    __syncthreads();                             // done with k-tile kt - 1, whose stage the next loads fill
-    issue(kt + S - 1, stage == 0 ? S - 1 : stage - 1);
-    const int soff = stage * STAGE;
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (group < G) {
 #pragma unroll
-    for (int h = 0; h < BK / 16; ++h) {
-      bf16x8 fa[NP], fb[NP];
+      for (int t = 0; t < S - 1 && t < CHUNK; ++t) issue(kt0 + t, t);
+    }
 #pragma unroll
-      for (int q = 0; q < NP; ++q) {
-        fa[q] = frag(fragI + soff + 2 * q * BLOCK + h * 1024);
-        fb[q] = frag(fragJ + soff + 2 * q * BLOCK + h * 1024);
-      }
-      if constexpr (NP == 2) {
-        acc = x3_mfma<true>(fa[1], fb[0], acc);
-        acc = x3_mfma<true>(fa[0], fb[0], acc);
-        acc = x3_mfma<true>(fa[0], fb[1], acc);
-      } else {
-        acc = mfma_bf16(fa[2], fb[0], acc);
-        acc = mfma_bf16(fa[1], fb[0], acc);
-        acc = mfma_bf16(fa[1], fb[1], acc);
-        acc = mfma_bf16(fa[0], fb[1], acc);
-        acc = mfma_bf16(fa[0], fb[2], acc);
-        acc = mfma_bf16(fa[0], fb[0], acc);
+    for (int t = 0; t < CHUNK; ++t) {
+      // this wave's part of k-tile t has landed, then everybody's; and all are done with k-tile t - 1, whose stage the
+      // next loads fill
+      wait_loads(std::integral_constant<int, LOADS>{}, t + S - 2 < CHUNK ? S - 2 : CHUNK - 1 - t);
+      __syncthreads();
+      if (group < G) {
+        if (t + S - 1 < CHUNK) issue(kt0 + t + S - 1, (t + S - 1) % S);
+        if (kt0 + t < nk) {
+          const int soff = (t % S) * STAGE;
+          bf16x8 fa[NP], fb[NP];
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            fa[q] = frag(fragI + soff + 2 * q * BLOCK);
+            fb[q] = frag(fragJ + soff + 2 * q * BLOCK);
+          }
+          if constexpr (NP == 2) {
+            acc = x3_mfma<true>(fa[1], fb[0], acc);
+            acc = x3_mfma<true>(fa[0], fb[0], acc);
+            acc = x3_mfma<true>(fa[0], fb[1], acc);
+          } else {
+            acc = mfma_bf16(fa[2], fb[0], acc);
+            acc = mfma_bf16(fa[1], fb[0], acc);
+            acc = mfma_bf16(fa[1], fb[1], acc);
+            acc = mfma_bf16(fa[0], fb[1], acc);
+            acc = mfma_bf16(fa[0], fb[2], acc);
+            acc = mfma_bf16(fa[0], fb[0], acc);
+          }
+        }
       }
     }
-    stage = stage + 1 == S ? 0 : stage + 1;
-    if (kt % CHUNK == CHUNK - 1 || kt + 1 == nk) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        tot[r] += acc[r];
-        acc[r] = 0.f;
-      }
-    }
+    add_chunks<4, GROUPS>(acc, tot, first, chunks, group, w, G, reinterpret_cast<AK_LDS floatx4*>(lds));
+    if (first + G < chunks) __syncthreads();               // the next round's loads overwrite the sums
   }
-  wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
-  plane_epilogue<NP>(p, ti, tj, z, [&](int r) { return tot[r]; });
+}
+
+template <int NP, int GROUPS>
+__device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int tj, int z, int steps, AK_LDS unsigned char* lds,
+                                                 float& vmax, bool& fits) {
+  const int chunks = (p.n_pad + 255) / 256, parity = steps & 1;
+  float c2_diag = 0.f, c2_scale = 0.f;                 // (under way while the product is formed)
+  if (p.C2.index >= 0) {
+    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
+    c2_diag = next[0];
+    c2_scale = -next[1];
+  }
+  floatx4 sum[4 / GROUPS];
+  if (GROUPS == 4 && chunks >= 3) plane_tile_chunks<NP, GROUPS, GROUPS>(p, ti, tj, z, parity, lds, sum);
+  else if (chunks >= 2) plane_tile_chunks<NP, GROUPS, 2>(p, ti, tj, z, parity, lds, sum);
+  else plane_tile_chunks<NP, GROUPS, 1>(p, ti, tj, z, parity, lds, sum);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int k = 0; k < 4 / GROUPS; ++k)
+    plane_epilogue<NP>(p, ti, tj, z, (wave >> 1) & 1, wave & 1, (wave >> 2) * (4 / GROUPS) + k, sum[k], parity, c2_diag, c2_scale,
+                       vmax, fits);
 }
 
 // Tile number -> (ti <= tj), in bands of 8 tile columns, row by row inside a band: the 32 work groups that share an

@@ -81,7 +81,7 @@ static int64_t root_pad(int64_t n, int tile) { return (n + tile - 1) / tile * ti
 static int64_t root_ld(int64_t n) { return (n + 3) / 4 * 4; }
 
 // Tile of a group on planes.  A 192-wide tile takes 0.75 us per k-tile of 16 and CU however few there are; a 64-wide one
-// 0.55 us per 64 k beside 5 us of latency, one at a time on a CU.
+// 0.55 us per 64 k beside 5 us of latency for every 256 of them (1024 columns 14.5 us a product, 1536 28, where the wide tile takes 72).
 static int root_plane_tile(int64_t n, int64_t batch) {
   const double big = static_cast<double>(root_pad(n, kPlaneTile)), small = static_cast<double>(root_pad(n, kPlaneSmallTile));
   const double T = big / kPlaneTile, t = small / kPlaneSmallTile;
@@ -105,19 +105,21 @@ static size_t root_buffer_floats(int64_t n, int64_t batch, int np) {
 struct RootState {
   // per matrix of the call, all device memory
   float* sv;        // eigenvalue estimate
-  float* err;       // current Newton error max|M - I|
+  float* err;       // Newton error max|M - I| of the accepted steps
   float* zscale;
   float* partial;   // [RCHUNKS]: sums of squares, then max |M_0 - I|
   float* alpha;     // [kLanczosSteps] the tridiagonal matrix: diagonal,
   float* beta;      // [kLanczosSteps] and beta[j] next to alpha[j - 1], alpha[j]
   float* coef;      // [2 kRootSteps]: (a, b) of every step
-  float* errword;   // [kErrStride] max |M' - I| of the step under way, folded in by the epilogue of the product that forms M'
+  float* errword;   // [kErrSlots kErrStride] max |M' - I| of the step under way, folded in by the epilogue of the product that forms M'
   int* lz_dim;      // Lanczos steps that counted (0: all)
   int* pi_iters;
   int* active;      // Newton iteration still running
   int* count;       // accepted steps
   int* accel;       // steps of the table that are not the classical one
   int* ovf;         // fp16 planes: a product of the step under way left the fp16 range
+  // err, active, count, ovf and errword have a second half, `total` entries further on: root_small_kernel
+  int total;
 };
 
 struct RootGroup {
@@ -138,6 +140,12 @@ struct RootGroups {
   int count, total;
   RootGroup g[kRootMaxGroups];
 };
+
+// Entry z (total + z: of the second half) of what the products of a step fold into.
+__device__ __forceinline__ void root_clear_words(const RootState& st, int z) {
+  for (int s = 0; s < kErrSlots; ++s) st.errword[(z * kErrSlots + s) * kErrStride] = 0.f;
+  st.ovf[z] = 0;
+}
 
 __device__ __forceinline__ int root_group_of(const RootGroups& G, int z) {
   int g = 0;
@@ -235,8 +243,9 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     scale();
     if (part == 0 && tid == 0) {
       st.lz_dim[z] = 0;
-      st.active[z] = st.count[z] = st.ovf[z] = 0;
-      st.errword[z * kErrStride] = 0.f;
+      st.active[z] = st.count[z] = 0;
+      root_clear_words(st, z);
+      root_clear_words(st, st.total + z);
       st.beta[z * kLanczosSteps] = 0.f;
     }
   } else {
@@ -620,27 +629,45 @@ static __global__ void root_begin_kernel(RootState st, float tol, int max_iter) 
   st.active[z] = (e > tol && max_iter > 0) ? 1 : 0;
 }
 
-// grid (total): accept / reject the step and decide whether to go on.  The error of the step is the word the product
-// M' = T^p M folded max |M' - I| into.
-static __global__ void newton_decide_kernel(RootState st, float tol, int max_iter) {
-  const int z = blockIdx.x;
-  if (threadIdx.x != 0) return;
-  const float e = st.errword[z * kErrStride], err = st.err[z];
-  const int overflow = st.ovf[z], active = st.active[z], c = st.count[z], accel = st.accel[z];
-  st.errword[z * kErrStride] = 0.f;
-  st.ovf[z] = 0;
-  if (active == 0) return;
+// A matrix's own state of the iteration.
+struct RootProgress {
+  float err;
+  int count, active;
+};
+// Accepts or rejects the step whose products have run and decides whether to go on.  z: the entry with the state before the
+// step and with the words that the step has folded into.  All lanes of a wave call it.
+__device__ __forceinline__ RootProgress newton_decide(const RootState& st, int z, int accel, float tol, int max_iter) {
+  RootProgress r{st.err[z], st.count[z], st.active[z]};
+  const int overflow = st.ovf[z];
+  uint32_t bits = __builtin_bit_cast(uint32_t, st.errword[(z * kErrSlots + (threadIdx.x & (kErrSlots - 1))) * kErrStride]);
+#pragma unroll
+  for (int o = kErrSlots / 2; o > 0; o >>= 1) bits = max(bits, static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), o)));
+  const float e = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(bits));
+  if (r.active == 0) return r;
   // diverging: keep the previous root (NaN compares false, like the reference).  The error of an accelerated step may grow, but
   // not beyond that of a spectrum in [0, 1].  A step whose products left the range of the fp16 planes (a statistic far
   // from positive definite) is dropped the same way.
-  const float limit = c >= kRootEarly && c < accel ? 1.2f : err * 1.2f;
+  const float limit = r.count >= kRootEarly && r.count < accel ? 1.2f : r.err * 1.2f;
   if (overflow != 0 || e > limit) {
-    st.active[z] = 0;
-    return;
+    r.active = 0;
+    return r;
   }
-  st.err[z] = e;
-  st.count[z] = c + 1;
-  if (!(e > tol && c + 1 < max_iter)) st.active[z] = 0;
+  r.err = e;
+  ++r.count;
+  if (!(e > tol && r.count < max_iter)) r.active = 0;
+  return r;
+}
+
+// grid (total), one wave: the decision about the step in half `half`, into the first half; all words are cleared.
+static __global__ __launch_bounds__(64) void newton_decide_kernel(RootState st, int half, float tol, int max_iter) {
+  const int z = blockIdx.x;
+  const RootProgress r = newton_decide(st, half * st.total + z, st.accel[z], tol, max_iter);
+  if (threadIdx.x != 0) return;
+  st.err[z] = r.err;
+  st.count[z] = r.count;
+  st.active[z] = r.active;
+  root_clear_words(st, z);
+  root_clear_words(st, st.total + z);
 }
 
 // grid (RCHUNKS, total): the caller's fp32 result
@@ -714,65 +741,84 @@ struct RootJob {
   int kind;
   float scale_r;
 };
+// (What leads a work group to its matrix lies side by side: the matrix's step count is then requested beside the job, whose
+// address depends on it, and not a trip to memory after it.)
 constexpr int kRootMaxJobs = 2 * kRootMaxGroups;
 struct RootJobs {
   int first[kRootMaxJobs];      // first work group of each job, INT32_MAX behind the last
+  int tiles[kRootMaxJobs], z0[kRootMaxJobs];
   RootJob j[kRootMaxJobs];
 };
 
-// One 64 x 64 tile (ti, tj) of C = A B of fp32 matrices: every tile of the product (nothing is mirrored), k pairs
-// (16 t + m, 16 t + 8 + m) in order on one accumulator, chunks of 128 k.  lds: deep_lds_floats<64, 64, 128>() floats.
-__device__ __forceinline__ void root_tile_fp32(const GemmParams& p, int ti, int tj, float* lds) {
-  using P = DeepPanel<64, 128>;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
-  const int wr = wave >> 1, wc = wave & 1, i0 = 64 * ti, j0 = 64 * tj, ld = static_cast<int>(p.lda);
-  float* ldsA = lds;
-  float* ldsB = lds + P::FLOATS;
-  const float* pa = ldsA + (32 * wr + l32) * P::KC_LD + 8 * g;
-  const float* pb = ldsB + 8 * g * P::IC_LD + 32 * wc + l32;
-  floatx16 acc, tot;
+// One tile (ti, tj) of C = A B of fp32 matrices: every tile of the product (nothing is mirrored), k pairs (16 t + m, 16 t + 8 + m)
+// in order on one accumulator, chunks of 128 k, the chunks added in order through the LDS.  THREADS = 1024 (512): 64 x 64, wave
+// (q, w) sums chunk q of every four (two) of block w.  THREADS = 256 (launches without planes): 32 x 32, wave q sums chunk q of
+// every four, so that few columns still spread over the device.  Operands go from memory to registers as the matrix instruction wants them.
+// Bound by latency and, in the 64 x 64 form, by the fp32 matrix instruction (1.7 us per chunk and CU).
+template <int THREADS>
+__device__ __forceinline__ float root_tile_fp32(const GemmParams& p, int ti, int tj, AK_LDS floatx4* part) {
+  constexpr int BLOCKS = THREADS == 256 ? 1 : 4, GROUPS = THREADS / 64 / BLOCKS, TILE = BLOCKS == 4 ? 64 : 32;
+  constexpr int U = BLOCKS == 4 ? 2 : 4;                      // steps of 16 k loaded at once
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = wave / BLOCKS, w = wave % BLOCKS;
+  const int i0 = TILE * ti + 32 * (w >> 1), j0 = TILE * tj + 32 * (w & 1), ld = static_cast<int>(p.lda);
+  const bool col_in = j0 + l32 < p.M;
+  const float* __restrict__ A = p.A + static_cast<int64_t>(i0 + l32 < p.M ? i0 + l32 : 0) * ld;
+  const float* __restrict__ B = p.B + (col_in ? j0 + l32 : 0);
+  const int chunks = (p.M + 127) / 128;
+  floatx4 tot[4 / GROUPS];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = tot[r] = 0.f;
-  P::Regs ra, rb;
-  deep_fetch<64, 128>(ra, p.A, ld, true, i0, p.M, 0, ld, tid);
-  deep_fetch<64, 128>(rb, p.B, ld, false, j0, ld, 0, p.M, tid);
-  for (int k0 = 0; k0 < p.M; k0 += 128) {
-    if (k0 != 0) __syncthreads();
-    deep_stash<64, 128>(ra, ldsA, true, tid);
-    deep_stash<64, 128>(rb, ldsB, false, tid);
-    __syncthreads();
-    if (k0 + 128 < p.M) {
-      deep_fetch<64, 128>(ra, p.A, ld, true, i0, p.M, k0 + 128, ld, tid);
-      deep_fetch<64, 128>(rb, p.B, ld, false, j0, ld, k0 + 128, p.M, tid);
+  for (int k = 0; k < 4 / GROUPS; ++k) tot[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int first = 0; first < chunks; first += GROUPS) {
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int k1 = min(p.M, 128 * (first + q + 1));
+    for (int k0 = 128 * (first + q); k0 < k1; k0 += 16 * U) {
+      floatx4 a[U][2];
+      float b[U][8];
+      // (loads without conditions: each of those would be waited for by itself.  Rows and columns beyond the matrix read
+      // others, whose sums are not stored; k beyond it are replaced by zeros.)
+      const bool whole = k0 + 16 * U <= p.M;
+#pragma unroll
+      for (int t = 0; t < U; ++t) {
+        const int k = k0 + 16 * t + 8 * g;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[t][h] = *reinterpret_cast<const floatx4*>(A + (whole ? k + 4 * h : min(k + 4 * h, ld - 4)));
+#pragma unroll
+        for (int m = 0; m < 8; ++m) b[t][m] = B[static_cast<int64_t>(whole ? k + m : min(k + m, p.M - 1)) * ld];
+      }
+      if (!whole) {
+#pragma unroll
+        for (int t = 0; t < U; ++t)
+#pragma unroll
+          for (int m = 0; m < 8; ++m) {
+            const bool in = k0 + 16 * t + 8 * g + m < p.M;
+            a[t][m >> 2][m & 3] = in ? a[t][m >> 2][m & 3] : 0.f;
+            b[t][m] = in ? b[t][m] : 0.f;
+          }
+      }
+#pragma unroll
+      for (int t = 0; t < U; ++t)
+#pragma unroll
+        for (int m = 0; m < 8; ++m) acc = mfma_f32(a[t][m >> 2][m & 3], b[t][m], acc);
     }
-#pragma unroll 2
-    for (int t = 0; t < 8; ++t) {
-      const floatx4 lo = *reinterpret_cast<const floatx4*>(pa + 16 * t), hi = *reinterpret_cast<const floatx4*>(pa + 16 * t + 4);
-      float b[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) b[m] = pb[(16 * t + m) * P::IC_LD];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) acc = mfma_f32(m < 4 ? lo[m] : hi[m - 4], b[m], acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      tot[r] += acc[r];
-      acc[r] = 0.f;
-    }
+    add_chunks<BLOCKS, GROUPS>(acc, tot, first, chunks, q, w, GROUPS, part);
+    if (first + GROUPS < chunks) __syncthreads();
   }
   float vmax = 0.f;
-  const int gj = j0 + 32 * wc + l32;
-  if (gj < p.M) {
+  if (col_in) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int gi = i0 + 32 * wr + 8 * (r >> 2) + 4 * g + (r & 3);
+    for (int r = 0; r < 16 / GROUPS; ++r) {
+      const float v = tot[r >> 2][r & 3];
+      const int gi = i0 + 8 * (q * (4 / GROUPS) + (r >> 2)) + 4 * g + (r & 3), gj = j0 + l32;
       if (gi >= p.M) continue;
-      p.C[static_cast<int64_t>(gi) * ld + gj] = tot[r];
-      vmax = gemm_fold_absmax(vmax, tot[r], gi == gj, 1);
-      if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi) * ld + gj] = p.c2_scale * tot[r] + (gi == gj ? p.c2_diag : 0.f);
+      p.C[static_cast<int64_t>(gi) * ld + gj] = v;
+      vmax = gemm_fold_absmax(vmax, v, gi == gj, 1);
+      if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi) * ld + gj] = p.c2_scale * v + (gi == gj ? p.c2_diag : 0.f);
     }
   }
-  if (p.absmax_out != nullptr) gemm_store_absmax(p.absmax_out, vmax, lane);
+  return vmax;
 }
 
 // A product on planes (fp16 planes: the two roots carry scale_r, every other matrix kRootScaleM).
@@ -788,7 +834,7 @@ __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0
   pg.count = st.count + z0;
   pg.coef = st.coef + static_cast<int64_t>(z0) * 2 * kRootSteps;
   pg.coef_stride = 2 * kRootSteps; pg.coef_last = kRootSteps - 1;
-  pg.errword = c2.index >= 0 ? st.errword + z0 * kErrStride : nullptr;
+  pg.errword = c2.index >= 0 ? st.errword + z0 * kErrSlots * kErrStride : nullptr;
   pg.active = st.active + z0;
   pg.overflow = st.ovf + z0;
   pg.n = n; pg.n_pad = n_pad; pg.T = n_pad / tile;
@@ -799,8 +845,8 @@ __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0
   return pg;
 }
 
-__device__ __forceinline__ bool root_idle(const RootState& st, const RootJob& job, int z, int steps) {
-  return st.active[z] == 0 || (steps == 0 && job.c.index == 0);            // (the first X is written by the start)
+__device__ __forceinline__ bool root_idle(const RootJob& job, int active, int steps) {
+  return active == 0 || (steps == 0 && job.c.index == 0);            // (the first X is written by the start)
 }
 
 // The product of matrix zl of a group in fp32; c2_*: of the step `steps` is followed by.
@@ -822,7 +868,7 @@ __device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, con
     p.ldc2 = job.ld;
     p.c2_diag = next[0];
     p.c2_scale = -next[1];
-    p.absmax_out = st.errword + z * kErrStride;
+    p.absmax_out = st.errword + (z * kErrSlots + blockIdx.x % kErrSlots) * kErrStride;
     p.absmax_identity = 1;
   }
   return p;
@@ -833,38 +879,94 @@ static __global__ __launch_bounds__(256) void root_split_kernel(RootState st, Ro
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 2 * 3 * X3_PLANE];
   const int zl = static_cast<int>(blockIdx.x) / job.tiles, z = job.z0 + zl, local = static_cast<int>(blockIdx.x) - zl * job.tiles;
   const int steps = st.count[z], T = (job.n + X3_BT - 1) / X3_BT;
-  if (root_idle(st, job, z, steps)) return;
+  if (root_idle(job, st.active[z], steps)) return;
   GemmParams p = root_fp32_product(st, job, zl, z, steps);
   p.K = job.n;
   p.transB = 0;
   gemm_x3_tile<3, true, 1, 0, false, true>(p, local / T, local % T, 0, (AK_LDS3 unsigned char*)x3_smem);
 }
 
-// One step of the product sequences of all groups on small tiles: a work group per tile of any product.
-static __global__ __launch_bounds__(256, 2) void root_small_kernel(RootState st, RootJobs J) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
-  const int wg = blockIdx.x;
-  int ji = 0;
+// A tile's largest |M' - I| and whether it fits, folded into entry z, word `slot`.
+__device__ __forceinline__ void root_fold(const RootState& st, int z, int slot, float vmax, bool fits) {
+  __shared__ uint32_t largest[16], lost[16];
+  uint32_t bits = __builtin_bit_cast(uint32_t, fabsf(vmax));            // a NaN is larger than any number
 #pragma unroll
-  for (int k = 1; k < kRootMaxJobs; ++k) ji += wg >= J.first[k] ? 1 : 0;
-  const RootJob job = J.j[ji];
-  int local = wg - J.first[ji];
-  const int zl = local / job.tiles, z = job.z0 + zl;
-  local -= zl * job.tiles;
-  const int steps = st.count[z];
-  if (root_idle(st, job, z, steps)) return;
-  float* lds = reinterpret_cast<float*>(dtl_smem);
-  if (job.kind == kFp32) {
-    const int T = (job.n + 63) / 64;
-    root_tile_fp32(root_fp32_product(st, job, zl, z, steps), local / T, local % T, lds);
-    return;
+  for (int o = 32; o > 0; o >>= 1) bits = max(bits, static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), o)));
+  const bool out = __ballot(!fits) != 0;
+  if ((threadIdx.x & 63) == 0) {
+    largest[threadIdx.x >> 6] = bits;
+    lost[threadIdx.x >> 6] = out ? 1u : 0u;
   }
-  int ti, tj;
-  decode_lower_tile(local, ti, tj);
-  const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
-                                       job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
-  if (job.kind == kPlanes2) plane_tile_small<2>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
-  else plane_tile_small<3>(pg, tj, ti, zl, (AK_LDS unsigned char*)dtl_smem);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  uint32_t any = 0;
+  for (unsigned w = 0; w < blockDim.x / 64; ++w) {
+    bits = max(bits, largest[w]);
+    any |= lost[w];
+  }
+  atomicMax(reinterpret_cast<uint32_t*>(st.errword + (z * kErrSlots + slot) * kErrStride), bits);
+  if (any != 0) atomicOr(st.ovf + z, 1);
+}
+
+// One step of the product sequences of all groups on small tiles: a work group per tile of any product.  THREADS = 256: no
+// product on planes among them; 512: more tiles than CUs (two work groups a CU), 1024 else.
+// Where all products of a call run here the steps need no launch for their decisions (5 us each): the first launch of a step
+// (pending) takes the one about the step before, every work group for itself, from the half of the state that step used; one work
+// group per matrix writes the new state to the other half, `half`, which the step's further launches read.  The words of
+// the half that the next step will fold into are cleared by the last launch of a step: nothing else touches them then.
+template <int THREADS>
+static __global__ __launch_bounds__(THREADS, THREADS == 256 ? 1 : 4) void root_small_kernel(RootState st, RootJobs J, int half,
+                                                                                            int pending, float tol, int max_iter) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
+  const int wg = static_cast<int>(xcd_contiguous_id(blockIdx.x, gridDim.x));      // a matrix's tiles share an L2
+  int ji = 0, start = J.first[0], tiles = J.tiles[0], z0 = J.z0[0];
+#pragma unroll
+  for (int k = 1; k < kRootMaxJobs; ++k) {
+    const bool here = wg >= J.first[k];
+    ji = here ? k : ji;
+    start = here ? J.first[k] : start;
+    tiles = here ? J.tiles[k] : tiles;
+    z0 = here ? J.z0[k] : z0;
+  }
+  const int zl = (wg - start) / tiles, z = z0 + zl, local = wg - start - zl * tiles;
+  const int entry = half * st.total + z;
+  const RootJob job = J.j[ji];
+  int steps, active;
+  if (pending != 0) {
+    const RootProgress r = newton_decide(st, (1 - half) * st.total + z, st.accel[z], tol, max_iter);
+    steps = r.count;
+    active = r.active;
+    if (local == 0 && job.c.index != 0 && threadIdx.x == 0) {
+      st.err[entry] = r.err;
+      st.count[entry] = r.count;
+      st.active[entry] = r.active;
+    }
+  } else {
+    steps = st.count[entry];
+    active = st.active[entry];
+  }
+  steps = __builtin_amdgcn_readfirstlane(steps);
+  if (root_idle(job, __builtin_amdgcn_readfirstlane(active), steps)) return;
+  float vmax = 0.f;
+  bool fits = true;
+  if (THREADS == 256 || job.kind == kFp32) {
+    const int T = (job.n + (THREADS == 256 ? 31 : 63)) / (THREADS == 256 ? 32 : 64);
+    vmax = root_tile_fp32<THREADS>(root_fp32_product(st, job, zl, z, steps), local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+  } else {
+    int ti, tj;
+    decode_lower_tile(local, ti, tj);
+    const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
+                                         job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
+    constexpr int GROUPS = THREADS == 512 ? 2 : 4;
+    if (job.kind == kPlanes2) plane_tile_small<2, GROUPS>(pg, tj, ti, zl, steps, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
+    else plane_tile_small<3, GROUPS>(pg, tj, ti, zl, steps, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
+  }
+  if (job.c2.index >= 0) {
+    if (local == 0 && threadIdx.x == 0) root_clear_words(st, (1 - half) * st.total + z);
+    root_fold(st, entry, local % kErrSlots, vmax, fits);
+  } else if (__ballot(!fits) != 0 && (threadIdx.x & 63) == 0) {
+    atomicOr(st.ovf + entry, 1);
+  }
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------------
@@ -928,7 +1030,7 @@ static int root_buffers(int p) {
 }
 
 static size_t root_state_floats(int total) {
-  return (static_cast<size_t>(total) * (3 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + kErrStride + 6) + 63) / 64 * 64;
+  return (static_cast<size_t>(total) * (4 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + 2 * kErrSlots * kErrStride + 9) + 63) / 64 * 64;
 }
 // matrix buffers and Lanczos vectors of a group
 static size_t root_group_matrix_floats(int64_t n, int64_t batch, int np, int buffers) {
@@ -999,18 +1101,34 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
       if (nslots[i] < 0) return AK_ERR_ARG;
       most = std::max(most, nslots[i]);
     }
-    constexpr int kLds[4] = {deep_lds_floats<64, 64, 128>() * 4, 0, 4 * 8 * 4096, 3 * 12 * 4096};    // by kind (planes: their stages)
+    bool planes = false, small = true;          // products on planes among the small tiles; nothing but small tiles
+    auto split = [&](const RootGroup& g) {      // fp32 groups with many wide matrices
+      const int t = (g.n + 127) / 128;
+      return t * t * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0;
+    };
+    for (int i = 0; i < G.count; ++i) {
+      const RootGroup& g = G.g[i];
+      const bool on_small = g.np != 0 ? g.tile == kPlaneSmallTile : !split(g);
+      planes = planes || (g.np != 0 && on_small);
+      // (with a single slot the first launch of a step is also its last)
+      small = small && on_small && nslots[i] > 1;
+    }
+    const int edge = planes ? 64 : 32;                                               // of an fp32 tile
+    // LDS by kind, with four and with two groups of waves
+    constexpr int kLds[2][4] = {{65536, 0, kSmallTileLds<2, 4>, kSmallTileLds<3, 4>}, {32768, 0, kSmallTileLds<2, 2>, kSmallTileLds<3, 2>}};
     static bool attr_set = false;     // idempotent; a race sets it twice at worst
     if (!attr_set) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_small_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              kLds[3]) != hipSuccess)
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_small_kernel<1024>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kLds[0][3]) != hipSuccess ||
+          hipFuncSetAttribute(reinterpret_cast<const void*>(root_small_kernel<512>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kLds[1][3]) != hipSuccess)
         return AK_ERR_LAUNCH;
       attr_set = true;
     }
     for (int it = 0; it < iters; ++it) {
       for (int k = 0; k < most; ++k) {
         RootJobs J;
-        int jobs = 0, blocks = 0, lds = 0;
+        int jobs = 0, blocks = 0, widest = 0;
         for (int i = 0; i < G.count; ++i) {
           const RootGroup& g = G.g[i];
           if (k >= nslots[i]) continue;
@@ -1031,31 +1149,41 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
             job.scale_r = g.scale_r;
             auto put = [&](int kind, int tiles) {
               job.kind = kind; job.tiles = tiles;
-              J.first[jobs] = blocks;
+              J.first[jobs] = blocks; J.tiles[jobs] = tiles; J.z0[jobs] = g.z0;
               J.j[jobs++] = job;
               blocks += tiles * g.batch;
-              lds = std::max(lds, kLds[kind]);
+              widest = std::max(widest, kind);
             };
             if (g.np != 0) {
               const int t = g.n_pad / kPlaneSmallTile;
               put(g.np, t * (t + 1) / 2);
-              continue;
-            }
-            const int t128 = (g.n + 127) / 128, t64 = (g.n + 63) / 64;
-            if (t128 * t128 * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0) {
-              job.kind = kFp32; job.tiles = t128 * t128;
+            } else if (split(g)) {
+              const int t = (g.n + 127) / 128;
+              job.kind = kFp32; job.tiles = t * t;
               hipLaunchKernelGGL(root_split_kernel, dim3(job.tiles * g.batch), b256, 0, s, G.st, job);
             } else {
-              put(kFp32, t64 * t64);
+              const int t = (g.n + edge - 1) / edge;
+              put(kFp32, t * t);
             }
           }
         }
         if (jobs == 0) continue;
-        for (int i = jobs; i < kRootMaxJobs; ++i) J.first[i] = INT32_MAX;
-        hipLaunchKernelGGL(root_small_kernel, dim3(blocks), b256, lds, s, G.st, J);
+        for (int i = jobs; i < kRootMaxJobs; ++i) {
+          J.first[i] = INT32_MAX;
+          J.tiles[i] = 1;
+          J.z0[i] = 0;
+        }
+        const int half = small ? it & 1 : 0, pending = small && it > 0 && k == 0 ? 1 : 0;
+        if (!planes)
+          hipLaunchKernelGGL(root_small_kernel<256>, dim3(blocks), b256, 16384, s, G.st, J, half, pending, tol, max_iter);
+        else if (blocks > 256)
+          hipLaunchKernelGGL(root_small_kernel<512>, dim3(blocks), dim3(512), kLds[1][widest], s, G.st, J, half, pending, tol, max_iter);
+        else
+          hipLaunchKernelGGL(root_small_kernel<1024>, dim3(blocks), dim3(1024), kLds[0][widest], s, G.st, J, half, pending, tol, max_iter);
       }
-      hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, tol, max_iter);
+      if (!small) hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, 0, tol, max_iter);
     }
+    if (small && iters > 0) hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, (iters - 1) & 1, tol, max_iter);
   }
   if (phases & 4) {
     hipLaunchKernelGGL(root_out_kernel, gc, b256, 0, s, G);
@@ -1125,16 +1253,17 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
   RootState& st = G.st;
   auto ints = [&](int k) { int* r = reinterpret_cast<int*>(w); w += k; return r; };
   auto floats = [&](int64_t k) { float* r = w; w += k; return r; };
-  st.active = ints(total);
-  st.count = ints(total);
+  st.total = total;
+  st.active = ints(2 * total);
+  st.count = ints(2 * total);
   st.accel = ints(total);
-  st.ovf = ints(total);
+  st.ovf = ints(2 * total);
   st.lz_dim = ints(total);
   st.pi_iters = ints(total);
   st.sv = floats(total);
-  st.err = floats(total);
+  st.err = floats(2 * total);
   st.zscale = floats(total);
-  st.errword = floats(static_cast<int64_t>(total) * kErrStride);
+  st.errword = floats(static_cast<int64_t>(2 * total) * kErrSlots * kErrStride);
   st.partial = floats(static_cast<int64_t>(total) * RCHUNKS);
   st.alpha = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.beta = floats(static_cast<int64_t>(total) * kLanczosSteps);

@@ -724,3 +724,30 @@ def test_state_dict_resume_continues_the_run():
     for k, (a, b) in enumerate(zip(straight, resumed)):
         for ga, gb in zip(a, b):
             assert torch.equal(ga, gb), f'step {k}'
+
+
+# A matrix has the same bits whichever launch shape its products take: alone (32 x 32 fp32 tiles; 64 x 64 plane tiles by 16
+# waves), beside planes (64 x 64 fp32 tiles by 16 waves), in a call of more tiles than CUs (8 waves); sizes around the chunks of 128 k
+# (fp32) and 256 k (planes), with and without fp16 planes.
+@pytest.mark.parametrize('p,eps', [(4, 1e-6), (2, 1e-6), (1, 1e-6), (3, 0.0)])
+def test_roots_have_the_same_bits_in_every_launch_shape(p, eps):
+    from asdl_amd import kernels as K
+    sizes = [3, 31, 33, 127, 128, 129, 257, 385, 511, 512, 513, 769, 1025]
+    g = torch.Generator().manual_seed(p)
+    stats, starts = {}, {}
+    for n in sizes:
+        x = torch.randn(2, n + 20, n, generator=g) * torch.logspace(0, -1, n)
+        stats[n], starts[n] = x.transpose(1, 2) @ x / n, torch.rand(2, n, generator=g) * 2 - 1
+
+    def roots(*take):
+        items = [(stats[n][:b].cuda(), p, starts[n][:b].cuda(), None) for n, b in take]
+        return {n: (out[0].cpu(), st[0].cpu()) for (n, _), (out, st) in zip(take, K.inv_root_group(items, eps))}
+    alone = {n: roots((n, 1))[n] for n in sizes}
+    many = roots(*[(n, 2) for n in sizes])
+    few = [roots((n, 1), (512, 1)) for n in sizes if n < 512]
+    for n, (root, st) in alone.items():
+        assert torch.isfinite(root).all() and int(st[2]) > 0
+        assert torch.equal(root, many[n][0]) and torch.equal(st, many[n][1]), n
+    for got in few:
+        for n, (root, _) in got.items():
+            assert torch.equal(root, alone[n][0]), n
