@@ -362,7 +362,7 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
     fits = NP != 2 || max(max(upper[0], upper[1]), max(upper[2], upper[3])) < 0x7c00;
   }
   if (p.errword != nullptr)
-    gemm_store_absmax(p.errword + (static_cast<int64_t>(z) * kErrSlots + blockIdx.x % kErrSlots) * kErrStride, vmax, lane);
+    gemm_store_absmax(p.errword + (static_cast<int64_t>(z) * kErrSlots + (ti + tj) % kErrSlots) * kErrStride, vmax, lane);
   if (NP == 2 && !fits) atomicOr(p.overflow + z, 1);
 }
 
