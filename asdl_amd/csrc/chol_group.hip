@@ -1,21 +1,17 @@
 // out_m <- (A_m + lam_m I)^-1 for many symmetric positive definite fp32 matrices of DIFFERENT sizes in one call.
 //
-// Per matrix (work matrix W, lower triangle) a right-looking blocked Cholesky that keeps the inverses of its 128 x 128
-// diagonal blocks, then the triangular inverse by levels, then out = M^T M (cg_right_looking below):
-//   for every diagonal block k:  leaf: W_kk -> M_kk = L_kk^-1 (one work group, in registers: chol_leaf.hpp);
-//                                panel: L21 = A21 M_kk^T;  update: A22 -= L21 L21^T
-//   for every level of a balanced tree over the blocks:  T2 = L21 M11;  M21 = -M22 T2
-// (Groups whose matrices are few and small enough take the block sweep of chol_sweep.hpp instead: one launch per block.)
-// d^3 FLOP in total, like POTRF + POTRI.  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
-// as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: 1.4-1.7
-// times the error of LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half was at 3-8).
+// A block elimination on Cholesky factors of 128 x 128 diagonal blocks that advances factorization, triangular inverse and
+// L^-T L^-1 together (d^3 FLOP, as POTRF + POTRI), in one of two forms:
+//   chol_sweep.hpp   every step updates the whole triangle: one launch per 128 columns, for groups whose tiles fit the device
+//   chol_chain.hpp   the steps update the block columns that the next steps need, one product per 512 columns the rest
+// The plan takes the one with the shorter estimate.  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
+// as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: below the error of
+// LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half was at 3-8 times that).
 //
-// The per-matrix sequences of steps (leaf | products) of ALL matrices are merged into one sequence of "super-steps":
-// super-step s holds, for every matrix whose next step has the type chosen for s, that step.  One launch per
-// super-step: a grouped leaf launch (one work group per diagonal block) or a grouped product launch (one work group
-// per tile of any product of the step, descriptor found through a tile -> product map; 128 x 128 split-operand MFMA tiles of
-// gemm_x3.hpp, or the smaller fp32 tiles of gemm_deep.hpp where those would leave the device idle: cg_prefer_deep).  The longest chain (the largest matrix) sets the number of launches; the work of all smaller
-// matrices runs in the shadow of its steps.  ResNet-50 (108 factors, 13 sizes): 121 launches.
+// The steps of all matrices are merged: step k of the chain is one launch for all matrices that have a block k, the products
+// at the end of a group are one launch for all matrices (one work group per tile of any product, descriptor found through a
+// tile -> product map; 128 x 128 split-operand MFMA tiles of gemm_x3.hpp, or the smaller fp32 tiles of gemm_deep.hpp where
+// those would leave the device idle: cg_prefer_deep).
 //
 // The plan (descriptor tables, launch sequence) depends on the sizes only; every address in it is an offset into the
 // workspace.  The caller builds it once per size set on the host (ak_chol_group_plan), keeps a device copy, and
@@ -28,25 +24,24 @@
 #include <cstring>
 #include <vector>
 #include "gemm_f32.hpp"
-#include "chol_leaf.hpp"
 #include "chol_sweep.hpp"
+#include "chol_chain.hpp"
 
 namespace ak {
 
-constexpr int64_t CG_MAGIC = 0x3347524c4f4843ll;     // "CHOLGR3"
-constexpr int CG_COPY = 0, CG_LEAF = 1, CG_PROD = 2, CG_PROD_DEEP = 3, CG_SWEEP = 4;
-constexpr int CG_FLAG_TRANSA = 1, CG_FLAG_TRANSB = 2, CG_FLAG_OUT_USER = 4, CG_FLAG_PANEL = 8;
+constexpr int64_t CG_MAGIC = 0x3447524c4f4843ll;     // "CHOLGR4"
+constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_PROD = 2, CG_PROD_DEEP = 3, CG_SWEEP = 4, CG_OUT = 5;
+
 // What an operand of a product holds, for the fp16-piece products (bits 4-5 of CgProd::flags: A, bits 6-7: B).  With
 // a = the largest diagonal element of A + lam I, every element is bounded in magnitude: a block of the (updated)
 // matrix by a, of its Cholesky factor L by sqrt(a), of M = L^-1 by 1 / sqrt(lam), of L21 L11^-1 by sqrt(a / lam).
-constexpr int CG_KIND_W = 0, CG_KIND_L = 1, CG_KIND_M = 2, CG_KIND_T2 = 3;
+constexpr int CG_KIND_L = 1, CG_KIND_M = 2;
 constexpr int CG_SCALE_FLOATS = 8;                    // per matrix: the four scales, the fp16 switch, padding
 #ifdef AK_TUNING_HOOKS
 static float CG_HALF_MAX_COND = 65536.f;              // tuning builds: ak_debug_set_chol_half_max_cond
 #else
 constexpr float CG_HALF_MAX_COND = 65536.f;           // a / lam beyond 2^16: the matrix keeps the bf16 three-piece products
 #endif
-constexpr int CG_GROUP = 4;                           // block columns whose updates of the trailing matrix are merged
 constexpr int CG_COPY_ROWS = 8;                       // rows of W one work group of the copy-in kernel writes
 
 struct CgHeader {
@@ -54,26 +49,20 @@ struct CgHeader {
   int64_t total_bytes;
   int64_t ws_floats;
   int64_t scales_off;       // floats from the workspace base: CG_SCALE_FLOATS per matrix
-  int64_t mats_off, steps_off, leaves_off, prods_off, map_off;     // byte offsets of the tables inside the plan
-  int32_t count, nsteps, nleaves, nprods;
-  int32_t copy_blocks, ntiles;
+  int64_t mats_off, steps_off, tasks_off, prods_off, map_off;      // byte offsets of the tables inside the plan
+  int32_t count, nsteps, copy_blocks, out_blocks;
   double us;                // estimated time of one call (cg_build)
 };
 
 struct CgMat {
   int64_t w_off;            // work matrix [dp, dp], offset in floats from the workspace base
   int32_t d, dp;
-  int32_t first_copy_block, pad0;
+  int32_t first_copy_block, first_out_block;
 };
 
 struct CgStep {
-  int32_t type, first, count, grid;
-  int32_t first_tile, pad0;     // products: where the step's tile -> product map starts
-};
-
-struct CgLeafTask {
-  int64_t blk_off;          // the diagonal block, offset in floats from the workspace base
-  int32_t mat, lo, n, ld, d, pad0;
+  int32_t type, first, count, grid;    // chain: first task, step k, tasks; products: first product, products, tiles
+  int32_t first_tile, pad0;            // products: where the step's tile -> product map starts
 };
 
 struct CgProd {
@@ -189,18 +178,43 @@ static __global__ __launch_bounds__(256) void cg_scale_kernel(CgArgs a, int coun
   sc[4] = half ? 1.f : 0.f;
 }
 
-// One work group (16 waves) per leaf task of the step.  Every table is read with one load that depends on nothing
-// but the work group's index: a chain of dependent loads from cold device memory costs a microsecond per link.
-static __global__ __launch_bounds__(LEAF_THREADS) void cg_leaf_kernel(CgArgs a, const CgLeafTask* __restrict__ tasks) {
-  __shared__ __attribute__((aligned(16))) LeafShared sh;
-  const CgLeafTask t = tasks[blockIdx.x];
-  const int live = a.skip != nullptr ? a.skip[static_cast<int64_t>(t.mat) * a.skip_stride] : 1;   // used at the end
-  const int tid = threadIdx.x;
-  const int bad = leaf_block(a.ws + t.blk_off, t.ld, t.n, sh, tid);
-  // a bad pivot inside the identity padding cannot happen; one inside the matrix is reported like LAPACK's potrf.
-  // A skipped matrix's work area holds whatever the last call left there; its steps still run (they touch nothing
-  // but that work area) and report nothing.
-  if (tid == 0 && live != 0 && bad != 0 && t.lo + bad <= t.d && a.info[t.mat] == 0) a.info[t.mat] = t.lo + bad;
+// out_m <- both triangles of W_m, one work group per 64 x 64 tile of its lower triangle (bisection on first_out_block).
+static __global__ __launch_bounds__(256) void cg_out_kernel(CgArgs a, int count) {
+  __shared__ float tile[64][65];
+  const CgHeader* __restrict__ h = reinterpret_cast<const CgHeader*>(a.plan);
+  const CgMat* __restrict__ mats = reinterpret_cast<const CgMat*>(a.plan + h->mats_off);
+  const int w = blockIdx.x;
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (mats[mid].first_out_block <= w) lo = mid;
+    else hi = mid - 1;
+  }
+  const CgMat m = mats[lo];
+  if (cg_skipped(a, lo)) return;
+  int ti, tj;
+  decode_lower_tile(w - m.first_out_block, ti, tj);
+  const float* __restrict__ W = a.ws + m.w_off;
+  float* __restrict__ out = a.out_list[lo];
+  const int c = 4 * (threadIdx.x & 15), r0 = threadIdx.x >> 4;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = r0 + 16 * u, i = 64 * ti + r, j = 64 * tj + c;
+    const floatx4 v = *reinterpret_cast<const floatx4*>(W + static_cast<int64_t>(min(i, m.dp - 1)) * m.dp + min(j, m.dp - 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[r][c + e] = v[e];
+  }
+  __syncthreads();
+  const int x = threadIdx.x & 63, y0 = threadIdx.x >> 6;
+#pragma unroll 4
+  for (int u = 0; u < 16; ++u) {
+    const int y = y0 + 4 * u;
+    const bool upper = ti == tj && x > y;              // of a diagonal tile: the mirror image
+    const int i = 64 * ti + y, j = 64 * tj + x;
+    if (i < m.d && j < m.d) out[static_cast<int64_t>(i) * m.d + j] = upper ? tile[x][y] : tile[y][x];
+    const int mi = 64 * tj + y, mj = 64 * ti + x;
+    if (ti != tj && mj < m.d) out[static_cast<int64_t>(mi) * m.d + mj] = tile[x][y];
+  }
 }
 
 // Tile (ti, tj) number `local` of a product, longest contraction first where the range depends on the tile.
@@ -238,20 +252,18 @@ static __global__ __launch_bounds__(256) void cg_prod_kernel(CgArgs a, const CgP
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 3 * X3_PLANE];
   const int w = blockIdx.x;
   const CgProd d = prods[tile_map[w]];
-  // only the product that writes the caller's matrix has to respect the skip flag (see cg_leaf_kernel)
-  if ((d.flags & CG_FLAG_OUT_USER) && cg_skipped(a, d.mat)) return;
+  // (a skipped matrix's work area holds whatever the last call left there; its steps still run and touch nothing else)
   int ti, tj;
   cg_decode_tile(d, w - d.first_tile, ti, tj);
   GemmParams p;
   p.A = a.ws + d.a_off;
   p.B = a.ws + d.b_off;
-  p.C = (d.flags & CG_FLAG_OUT_USER) ? a.out_list[d.mat] : a.ws + d.c_off;
+  p.C = a.ws + d.c_off;
   p.C_list = nullptr;
   p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
   p.sA = p.sB = p.sC = 0;
   p.M = d.M; p.N = d.N; p.K = d.K;
-  p.transA = (d.flags & CG_FLAG_TRANSA) ? 1 : 0;
-  p.transB = (d.flags & CG_FLAG_TRANSB) ? 1 : 0;
+  p.transA = 0; p.transB = 1;
   p.alpha = d.alpha; p.beta = d.beta;
   p.kmode = d.kmode; p.tile_mode = d.tile_mode;
   p.active = nullptr; p.active_stride = 0;
@@ -263,56 +275,33 @@ static __global__ __launch_bounds__(256) void cg_prod_kernel(CgArgs a, const CgP
     p.scaleA = sc[(d.flags >> 4) & 3];
     p.scaleB = sc[(d.flags >> 6) & 3];
     p.alpha = d.alpha / (p.scaleA * p.scaleB);      // powers of two: exact
-    gemm_x3_tile<2, false, -1, -1, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
+    gemm_x3_tile<2, false, 1, 1, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
   } else {
-    gemm_x3_tile<3, false>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
+    gemm_x3_tile<3, false, 1, 1>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
   }
 }
 
-// The same for the steps whose 128 x 128 tiles would leave most of the device idle: deep fp32 tiles (gemm_deep.hpp) of
-// 64 x 64, or of 32 x 128 for a panel, which is formed in place and whose work groups have to own whole rows.
-static __global__ __launch_bounds__(256) void cg_prod_deep_kernel(CgArgs a, const CgProd* __restrict__ prods,
+// The same for the steps whose 128 x 128 tiles would leave most of the device idle: deep fp32 tiles of 64 x 64 (gemm_deep.hpp).
+static __global__ __launch_bounds__(256, 2) void cg_prod_deep_kernel(CgArgs a, const CgProd* __restrict__ prods,
                                                                   const int32_t* __restrict__ tile_map) {
-  constexpr int kSquare = deep_lds_floats<64, 64, 128>(), kPanel = deep_lds_floats<32, 128, 64>();
-  __shared__ __attribute__((aligned(16))) float lds[kSquare > kPanel ? kSquare : kPanel];
+  __shared__ __attribute__((aligned(16))) float lds[deep_lds_floats<64, 64, 128>()];
   const int w = blockIdx.x;
   const CgProd d = prods[tile_map[w]];
-  if ((d.flags & CG_FLAG_OUT_USER) && cg_skipped(a, d.mat)) return;
   int ti, tj;
   cg_decode_tile(d, w - d.first_tile, ti, tj);
   GemmParams p;
   p.A = a.ws + d.a_off;
   p.B = a.ws + d.b_off;
-  p.C = (d.flags & CG_FLAG_OUT_USER) ? a.out_list[d.mat] : a.ws + d.c_off;
+  p.C = a.ws + d.c_off;
   p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
   p.M = d.M; p.N = d.N; p.K = d.K;
-  p.transA = (d.flags & CG_FLAG_TRANSA) ? 1 : 0;
-  p.transB = (d.flags & CG_FLAG_TRANSB) ? 1 : 0;
+  p.transA = 0; p.transB = 1;
   p.alpha = d.alpha; p.beta = d.beta;
   p.kmode = d.kmode; p.tile_mode = d.tile_mode;
-  if (d.flags & CG_FLAG_PANEL) gemm_deep_tile<32, 128, 64>(p, ti, tj, 0, lds);
-  else gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
+  gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
 }
 
 // ---- host: the plan ------------------------------------------------------------------------------------------
-
-struct CgOp {                 // one step of one matrix's own sequence
-  int type;
-  CgLeafTask leaf;
-  std::vector<CgProd> prods;
-};
-
-static int64_t cg_half(int64_t n) {
-  const int64_t nb = (n + LEAF - 1) / LEAF;
-  return LEAF * ((nb + 1) / 2);
-}
-
-// Floats of the T1 (and of the T2) pool of an n x n range: a node's panels live while its right half is factored.
-static int64_t cg_pool(int64_t n) {
-  if (n <= LEAF) return 0;
-  const int64_t s1 = cg_half(n), s2 = n - s1;
-  return std::max(cg_pool(s1), s1 * s2 + cg_pool(s2));
-}
 
 static inline int64_t cg_align64(int64_t x) { return (x + 63) / 64 * 64; }
 
@@ -323,9 +312,8 @@ static int64_t cg_tiles(const CgProd& p) {
 
 // Tiles of the deep kernel instead of 128 x 128.
 static void cg_make_deep(CgProd& p) {
-  const int bm = (p.flags & CG_FLAG_PANEL) ? 32 : 64, bn = (p.flags & CG_FLAG_PANEL) ? 128 : 64;
-  p.tiles_m = (p.M + bm - 1) / bm;
-  p.tiles_n = (p.N + bn - 1) / bn;
+  p.tiles_m = (p.M + 63) / 64;
+  p.tiles_n = (p.N + 63) / 64;
 }
 
 // Microseconds of the products of one super-step (cg_prefer_deep), its launch not counted.
@@ -346,15 +334,15 @@ static double cg_product_us(const std::vector<CgProd>& ps, bool deep) {
 // deep tiles take 2 us per chunk of 128 k.  The step is as long as its longest tile or as its work spread over the CUs.
 static bool cg_prefer_deep(const std::vector<CgProd>& ps) { return cg_product_us(ps, true) < cg_product_us(ps, false); }
 
-static CgProd cg_prod(int mat, int flags, int kind_a, int kind_b, int M, int N, int K, float alpha, int64_t a, int lda,
+// C = beta C + alpha A B^T
+static CgProd cg_prod(int mat, int kind_a, int kind_b, int M, int N, int K, float alpha, int64_t a, int lda,
                       int64_t b, int ldb, float beta, int64_t c, int ldc, int kmode, int tile_mode) {
   CgProd p;
   std::memset(&p, 0, sizeof(p));
-  flags |= (kind_a << 4) | (kind_b << 6);
   p.a_off = a; p.b_off = b; p.c_off = c;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.M = M; p.N = N; p.K = K;
-  p.flags = flags; p.kmode = kmode; p.tile_mode = tile_mode;
+  p.flags = (kind_a << 4) | (kind_b << 6); p.kmode = kmode; p.tile_mode = tile_mode;
   p.alpha = alpha; p.beta = beta;
   p.mat = mat;
   p.tiles_m = (M + 127) / 128;
@@ -362,87 +350,48 @@ static CgProd cg_prod(int mat, int flags, int kind_a, int kind_b, int M, int N, 
   return p;
 }
 
-// The right-looking sequence of one matrix: for every diagonal block k of 128 columns
-//   leaf: W_kk -> M_kk = L_kk^-1;   panel: W[below, k] <- W[below, k] M_kk^T = L[below, k] (in place: every work group
-//   reads the 128 x 128 tile it writes, whole, before its epilogue);   update: W22 -= L21 L21^T (lower tiles, K = 128)
-// then the triangular inverse by levels of a balanced tree over the blocks (all nodes of one height are independent
-// and share two launches):   T2 = L21 M11;  W21 <- M21 = -M22 T2.
-// Every product of the factorization phase has as many tiles as the trailing matrix (hundreds for the wide factors).
-struct CgNode { int lo, mid, hi, height; };
-
-static int cg_nodes(std::vector<CgNode>& nodes, int lo, int hi) {
-  const int n = hi - lo;
-  if (n <= LEAF) return 0;
-  const int mid = lo + static_cast<int>(cg_half(n));
-  const int h = 1 + std::max(cg_nodes(nodes, lo, mid), cg_nodes(nodes, mid, hi));
-  nodes.push_back(CgNode{lo, mid, hi, h});
-  return h;
+// The products at the end of the group of columns [c0, c1) of one matrix: X -+ V V^T.  Rows and columns of the group, whose
+// old values have become V, are formed anew.
+static void cg_group_products(std::vector<CgProd>& ps, int mat, int64_t w, int64_t v, int dp, int c0, int c1) {
+  const int width = c1 - c0, below = dp - c1;
+  auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
+  auto put = [&](int kind_a, int kind_b, int r, int M, int c, int N, float alpha, float beta, int kmode, int tile_mode) {
+    if (M <= 0 || N <= 0) return;
+    ps.push_back(cg_prod(mat, kind_a, kind_b, M, N, width, alpha, v + static_cast<int64_t>(r) * CC_VLD, CC_VLD,
+                         v + static_cast<int64_t>(c) * CC_VLD, CC_VLD, beta, at(r, c), dp, kmode, tile_mode));
+  };
+  put(CG_KIND_L, CG_KIND_L, c1, below, c1, below, -1.f, 1.f, K_FULL, TILE_LOWER);
+  put(CG_KIND_L, CG_KIND_M, c1, below, c0, width, -1.f, 0.f, K_GE_J, TILE_ALL);
+  put(CG_KIND_L, CG_KIND_M, c1, below, 0, c0, -1.f, 1.f, K_FULL, TILE_ALL);
+  put(CG_KIND_M, CG_KIND_M, c0, width, 0, c0, 1.f, 0.f, K_GE_I, TILE_ALL);
+  put(CG_KIND_M, CG_KIND_M, c0, width, c0, width, 1.f, 0.f, K_GE_MAXIJ, TILE_LOWER);
+  put(CG_KIND_M, CG_KIND_M, 0, c0, 0, c0, 1.f, 1.f, K_FULL, TILE_LOWER);
 }
 
-static void cg_right_looking(std::vector<CgOp>& ops, int mat, int64_t w, int d, int dp, int64_t t2) {
-  // Block columns are taken in groups of CG_GROUP: inside a group a block's rank-128 update goes to the remaining
-  // columns of the group only; the trailing matrix behind the group gets ONE update with the whole group as its
-  // contraction (K up to 128 CG_GROUP), i.e. it is read and written once per group instead of once per block.
-  for (int gs = 0; gs < dp; gs += CG_GROUP * LEAF) {
-    const int ge = std::min(gs + CG_GROUP * LEAF, dp);
-    for (int lo = gs; lo < ge; lo += LEAF) {
-      const int n = std::min(LEAF, dp - lo), below = dp - lo - n;
-      CgOp leaf;
-      leaf.type = CG_LEAF;
-      leaf.leaf = CgLeafTask{w + static_cast<int64_t>(lo) * dp + lo, mat, lo, n, dp, d, 0};
-      ops.push_back(leaf);
-      if (below == 0) break;
-      auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
-      CgOp panel, update;
-      panel.type = update.type = CG_PROD;
-      panel.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB | CG_FLAG_PANEL, CG_KIND_W, CG_KIND_M, below, n, n, 1.f, at(lo + n, lo), dp,
-                                    at(lo, lo), dp, 0.f, at(lo + n, lo), dp, K_LE_J, TILE_ALL));
-      ops.push_back(panel);
-      const int next = lo + n;
-      if (next < ge) {
-        // the group's remaining columns: the square on the diagonal (lower tiles) and the rows below the group
-        const int sq = ge - next, under = dp - ge;
-        update.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB, CG_KIND_L, CG_KIND_L, sq, sq, n, -1.f, at(next, lo), dp,
-                                       at(next, lo), dp, 1.f, at(next, next), dp, K_FULL, TILE_LOWER));
-        if (under > 0)
-          update.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB, CG_KIND_L, CG_KIND_L, under, sq, n, -1.f, at(ge, lo), dp,
-                                         at(next, lo), dp, 1.f, at(ge, next), dp, K_FULL, TILE_ALL));
-      } else {
-        // end of the group: the trailing matrix, with the group's ge - gs columns as the contraction
-        const int under = dp - ge;
-        update.prods.push_back(cg_prod(mat, CG_FLAG_TRANSB, CG_KIND_L, CG_KIND_L, under, under, ge - gs, -1.f, at(ge, gs), dp,
-                                       at(ge, gs), dp, 1.f, at(ge, ge), dp, K_FULL, TILE_LOWER));
-      }
-      ops.push_back(update);
-    }
-  }
-  std::vector<CgNode> nodes;
-  const int top = cg_nodes(nodes, 0, dp);
-  for (int h = 1; h <= top; ++h) {
-    CgOp first, second;
-    first.type = second.type = CG_PROD;
-    int64_t pool = t2;
-    for (const CgNode& nd : nodes) {
-      if (nd.height != h) continue;
-      const int s1 = nd.mid - nd.lo, s2 = nd.hi - nd.mid;
-      const int64_t W11 = w + static_cast<int64_t>(nd.lo) * dp + nd.lo, W21 = w + static_cast<int64_t>(nd.mid) * dp + nd.lo,
-                    W22 = w + static_cast<int64_t>(nd.mid) * dp + nd.mid;
-      first.prods.push_back(cg_prod(mat, 0, CG_KIND_L, CG_KIND_M, s2, s1, s1, 1.f, W21, dp, W11, dp, 0.f, pool, s1, K_GE_J,
-                                    TILE_ALL));
-      second.prods.push_back(cg_prod(mat, 0, CG_KIND_M, CG_KIND_T2, s2, s1, s2, -1.f, W22, dp, pool, s1, 0.f, W21, dp,
-                                     K_LE_I, TILE_ALL));
-      pool += cg_align64(static_cast<int64_t>(s1) * s2);
-    }
-    ops.push_back(first);
-    ops.push_back(second);
-  }
+// The tiles of step k of one matrix (chol_chain.hpp) as products of 128 columns of V, for launches of their own.
+static void cg_step_products(std::vector<CgProd>& ps, int mat, int64_t w, int64_t v, int64_t e, int dp, int k, int g0, int ge) {
+  const int c0 = g0 * LEAF, c1 = (k + 1) * LEAF, c2 = std::min(ge * LEAF, dp);
+  auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
+  auto row = [&](int r) { return v + static_cast<int64_t>(r) * CC_VLD + (k - g0) * LEAF; };
+  auto put = [&](int kind_b, int r, int M, int c, int N, float beta, int64_t to, int ld, int tile_mode) {
+    if (M > 0 && N > 0)
+      ps.push_back(cg_prod(mat, CG_KIND_L, kind_b, M, N, LEAF, -1.f, row(r), CC_VLD, row(c), CC_VLD, beta, to, ld, K_FULL, tile_mode));
+  };
+  put(CG_KIND_L, c1, c2 - c1, c1, c2 - c1, 1.f, at(c1, c1), dp, TILE_LOWER);
+  put(CG_KIND_L, c2, dp - c2, c1, c2 - c1, 1.f, at(c2, c1), dp, TILE_ALL);
+  put(CG_KIND_L, c2, std::min(LEAF, dp - c2), c2, std::min(LEAF, dp - c2), 1.f, at(c2, c2), dp, TILE_LOWER);
+  put(CG_KIND_M, c1, c2 - c1, 0, c0, 1.f, at(c1, 0), dp, TILE_ALL);
+  for (int r = k + 1; r < ge; ++r)
+    for (int i = g0; i <= k; ++i)
+      put(CG_KIND_M, r * LEAF, std::min(LEAF, dp - r * LEAF), i * LEAF, LEAF, i < k ? 1.f : 0.f,
+          e + static_cast<int64_t>((r - g0) * (r - g0 - 1) / 2 + i - g0) * ST_TILE, LEAF, TILE_ALL);
 }
 
 struct CgPlan {
   CgHeader h;
   std::vector<CgMat> mats;
   std::vector<CgStep> steps;
-  std::vector<CgLeafTask> leaves;
+  std::vector<CcTask> tasks;
   std::vector<CgProd> prods;
   std::vector<int32_t> tile_map;
   std::vector<SwTask> sweep_leaves, sweep_tiles;
@@ -461,14 +410,14 @@ static bool cg_dims_ok(const int64_t* dims, int count) {
 static double cg_sweep_us(const int64_t* dims, int count) {
   int64_t nb_max = 0;
   for (int m = 0; m < count; ++m) nb_max = std::max<int64_t>(nb_max, (dims[m] + LEAF - 1) / LEAF);
-  double us = 16;
+  double us = 14;
   for (int64_t k = 0; k < nb_max; ++k) {
     int64_t groups = 0;
     for (int m = 0; m < count; ++m) {
       const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
       if (nb > k) groups += nb * (nb + 1) / 2 + (nb > k + 1 ? 1 : 0);
     }
-    us += std::max(25.0, 22.0 * static_cast<double>((groups + 255) / 256));
+    us += std::max(22.0, 18.0 * static_cast<double>((groups + 255) / 256));
   }
   return us;
 }
@@ -515,23 +464,156 @@ static void cg_build_sweep(const int64_t* dims, int count, CgPlan& plan) {
   h.nsteps = static_cast<int>(plan.steps.size());
   int64_t b = cg_align(sizeof(CgHeader), 64);
   h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
-  h.leaves_off = b; b = cg_align(b + plan.sweep_leaves.size() * sizeof(SwTask), 64);
+  h.tasks_off = b; b = cg_align(b + plan.sweep_leaves.size() * sizeof(SwTask), 64);
   h.prods_off = b; b = cg_align(b + plan.sweep_tiles.size() * sizeof(SwTask), 64);
   h.mats_off = h.map_off = b;
   h.total_bytes = b;
 }
 
-static void cg_build_right_looking(const int64_t* dims, int count, CgPlan& plan);
 #ifdef AK_TUNING_HOOKS
-static int CG_FORCE = 0;               // tuning builds: 1 the sweep, 2 the factorization (ak_debug_force_chol_plan)
+static int CG_FORCE = 0;               // tuning builds: 1 the sweep, 2 the chain, 3 (4) with (without) launches of their own for its tiles
 #else
 constexpr int CG_FORCE = 0;
 #endif
 
-// The sweep wins while its tiles fit the device once (25 us a step against 41 for leaf, panel and update), and often when
-// they fit it twice (44 us a step: 2 x 2048, 272 tiles, 757 against 908 us); beyond that its K = 128 updates of the whole
-// triangle cost more than the factorization's shorter, deeper and split ones (4 x 2048: 1139 against 980 us).  The bound of
-// 4096 tiles only keeps the tables of hopeless cases from being built.
+// The chain's tables.  Returns its estimated time: 22 us a step or 18 per round of tiles (a panel alone: 9), the products by
+// cg_product_us, the copies by their bytes.
+static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
+  struct Mat { int64_t w, v, e, m; int d, dp, nb; };
+  std::vector<Mat> mats(count);
+  int64_t off = 0;
+  int copy_blocks = 0, out_blocks = 0, nb_max = 0;
+  double bytes = 0;
+  plan.mats.resize(count);
+  for (int i = 0; i < count; ++i) {
+    Mat& x = mats[i];
+    x.d = static_cast<int>(dims[i]);
+    x.dp = (x.d + 3) / 4 * 4;
+    x.nb = (x.dp + LEAF - 1) / LEAF;
+    nb_max = std::max(nb_max, x.nb);
+    auto take = [&](int64_t floats) { const int64_t at = off; off += cg_align64(floats); return at; };
+    x.w = take(static_cast<int64_t>(x.dp) * x.dp);
+    x.v = take(static_cast<int64_t>(2) * x.dp * CC_VLD);
+    x.e = take(static_cast<int64_t>(CG_GROUP * (CG_GROUP - 1) / 2) * ST_TILE);
+    x.m = take(static_cast<int64_t>(2) * ST_TILE);
+    plan.mats[i] = CgMat{x.w, x.d, x.dp, copy_blocks, out_blocks};
+    copy_blocks += (x.dp + CG_COPY_ROWS - 1) / CG_COPY_ROWS;
+    const int t = (x.d + 63) / 64;
+    out_blocks += t * (t + 1) / 2;
+    bytes += 2.5 * 4 * x.d * x.d;
+  }
+  double us = 24 + bytes / 3.5e6;
+  // one launch of products, if any: its estimated time; written to the plan or not
+  auto products = [&](std::vector<CgProd> ps, bool write) {
+    if (ps.empty()) return 0.0;
+    CgStep pr{CG_PROD, static_cast<int>(plan.prods.size()), static_cast<int>(ps.size()), 0, static_cast<int>(plan.tile_map.size()), 0};
+    const bool deep = cg_prefer_deep(ps);
+    if (deep) {
+      pr.type = CG_PROD_DEEP;
+      for (CgProd& p : ps) cg_make_deep(p);
+    }
+    const double time = 4 + cg_product_us(ps, deep);
+    if (!write) return time;
+    // longest contraction first: the long tiles start early, the short ones (those that start in the middle of it) fill the tail
+    auto depth = [](const CgProd& p) { return p.kmode == K_FULL ? 2 * p.K : p.K; };
+    std::stable_sort(ps.begin(), ps.end(), [&](const CgProd& x, const CgProd& y) { return depth(x) > depth(y); });
+    int64_t n = 0;
+    for (size_t i = 0; i < ps.size(); ++i) {
+      ps[i].first_tile = static_cast<int>(n);
+      const int64_t mine = cg_tiles(ps[i]);
+      n += mine;
+      plan.tile_map.insert(plan.tile_map.end(), static_cast<size_t>(mine), static_cast<int32_t>(i));
+    }
+    pr.grid = static_cast<int>(n);
+    plan.prods.insert(plan.prods.end(), ps.begin(), ps.end());
+    plan.steps.push_back(pr);
+    return time;
+  };
+  plan.steps.push_back(CgStep{CG_COPY, 0, count, copy_blocks, 0, 0});
+  for (int k = -1; k < nb_max; ++k) {
+    CgStep st{CG_CHAIN, static_cast<int>(plan.tasks.size()), k, 0, 0, 0};
+    auto each = [&](auto&& f) {
+      for (int i = 0; i < count; ++i)
+        if (mats[i].nb > std::max(k, 0)) f(i, mats[i]);
+    };
+    auto put = [&](int i, int kind, int bi, int bj) {
+      const Mat& x = mats[i];
+      const int g0 = std::max(k, 0) / CG_GROUP * CG_GROUP;
+      plan.tasks.push_back(CcTask{x.w, x.v, x.e, x.m, i, x.d, x.dp, x.nb, kind, bi, bj, g0});
+    };
+    each([&](int i, const Mat& x) {
+      if (k + 1 < x.nb) put(i, CC_LEAF, k + 1, k + 1);
+    });
+    const int g0 = std::max(k, 0) / CG_GROUP * CG_GROUP;
+    std::vector<CgProd> ps;
+    bool split = false;
+    if (k >= 0) {
+      int tiles = 0, rows = 0;
+      each([&](int i, const Mat& x) {
+        const int ge = std::min(g0 + CG_GROUP, x.nb), left = ge - k - 1;
+        rows += x.nb;
+        tiles += left * (x.nb - k - 1) - left * (left - 1) / 2 + left * (k + 1);
+        if (left > 0) cg_step_products(ps, i, x.w, x.v + static_cast<int64_t>(g0 / CG_GROUP & 1) * x.dp * CC_VLD, x.e, x.dp, k, g0, ge);
+      });
+      const double fused = std::max(26.0, 9.0 + 18.0 * tiles / 256), apart = std::max(26.0, 9.0 + 9.0 * rows / 256) + products(ps, false);
+      split = !ps.empty() && (apart < fused || CG_FORCE == 3) && CG_FORCE != 4;
+      us += split || ps.empty() ? std::max(26.0, 9.0 + 9.0 * rows / 256) : fused;
+      each([&](int i, const Mat& x) {
+        const int ge = std::min(g0 + CG_GROUP, x.nb);
+        if (k + 1 == ge || split) {                      // V only
+          for (int b = 0; b < x.nb; ++b)
+            if (b != k && b != k + 1) put(i, CC_PANEL, b, b);
+          return;
+        }
+        for (int j = k + 1; j < ge; ++j)
+          for (int b = j; b < x.nb; ++b)
+            if (b != k + 1 || j != k + 1) put(i, CC_TILE, b, j);
+        for (int r = k + 1; r < ge; ++r)
+          for (int b = 0; b <= k; ++b) put(i, CC_TILE, r, b);
+        if (ge < x.nb) put(i, CC_TILE, ge, ge);
+      });
+    } else {
+      us += 18;
+    }
+    st.grid = static_cast<int>(plan.tasks.size()) - st.first;
+    if (st.grid > 0) plan.steps.push_back(st);
+    if (split) us += products(ps, true);
+    ps.clear();
+    // the group's products, by the matrices whose group ends here
+    if (k >= 0) {
+      each([&](int i, const Mat& x) {
+        if (k + 1 != std::min(g0 + CG_GROUP, x.nb)) return;
+        const int64_t v = x.v + static_cast<int64_t>(g0 / CG_GROUP & 1) * x.dp * CC_VLD;
+        cg_group_products(ps, i, x.w, v, x.dp, g0 * LEAF, std::min((k + 1) * LEAF, x.dp));
+      });
+    }
+    us += products(ps, true);
+  }
+  plan.steps.push_back(CgStep{CG_OUT, 0, count, out_blocks, 0, 0});
+  CgHeader& h = plan.h;
+  std::memset(&h, 0, sizeof(h));
+  h.magic = CG_MAGIC;
+  h.scales_off = off;
+  off += cg_align64(static_cast<int64_t>(count) * CG_SCALE_FLOATS);
+  h.ws_floats = off;
+  h.count = count;
+  h.nsteps = static_cast<int>(plan.steps.size());
+  h.copy_blocks = copy_blocks;
+  h.out_blocks = out_blocks;
+  h.us = us;
+  int64_t b = cg_align(sizeof(CgHeader), 64);
+  h.mats_off = b; b = cg_align(b + plan.mats.size() * sizeof(CgMat), 64);
+  h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
+  h.tasks_off = b; b = cg_align(b + plan.tasks.size() * sizeof(CcTask), 64);
+  h.prods_off = b; b = cg_align(b + plan.prods.size() * sizeof(CgProd), 64);
+  h.map_off = b; b = cg_align(b + plan.tile_map.size() * sizeof(int32_t), 64);
+  h.total_bytes = b;
+  return us;
+}
+
+// The sweep where its estimate is shorter: while its tiles fit the device once or twice (22 us a step, 18 for each further round:
+// 2304 456 us, 3 x 2048 598), beyond that its updates of the whole triangle cost more than the chain's steps and products (3073: 900 us by
+// the chain; the sweep's two rounds 950).  The bound of 4096 tiles keeps the tables of hopeless cases from being built.
 static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
   int64_t tiles = 0;
   for (int m = 0; m < count; ++m) {
@@ -539,116 +621,15 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
     tiles += nb * (nb + 1) / 2;
   }
   const double sweep_us = cg_sweep_us(dims, count);
-  if (CG_FORCE == 1) {
-    cg_build_sweep(dims, count, plan);
-    plan.h.us = sweep_us;
-    return;
+  bool sweep = CG_FORCE == 1;
+  if (!sweep) {
+    const double us = cg_build_chain(dims, count, plan);
+    sweep = CG_FORCE < 2 && tiles <= 4096 && sweep_us < us;
   }
-  CgPlan right;
-  cg_build_right_looking(dims, count, right);
-  double us = 0;
-  for (const CgStep& st : right.steps) {
-    us += 4;              // the launch's own start and the wait for the one before
-    if (st.type == CG_LEAF) us += 15;
-    else if (st.type == CG_COPY) us += 8;
-    else {
-      const std::vector<CgProd> ps(right.prods.begin() + st.first, right.prods.begin() + st.first + st.count);
-      us += cg_product_us(ps, st.type == CG_PROD_DEEP);
-    }
-  }
-  const bool sweep = CG_FORCE != 2 && tiles <= 4096 && sweep_us < us;
-  if (sweep) cg_build_sweep(dims, count, plan);
-  else plan = std::move(right);
-  plan.h.us = sweep ? sweep_us : us;
-}
-
-static void cg_build_right_looking(const int64_t* dims, int count, CgPlan& plan) {
-  std::vector<std::vector<CgOp>> seq(count);
-  int64_t off = 0;
-  int copy_blocks = 0;
-  plan.mats.resize(count);
-  for (int m = 0; m < count; ++m) {
-    const int d = static_cast<int>(dims[m]), dp = (d + 3) / 4 * 4;
-    const int64_t pool = cg_align(cg_pool(dp), 64);
-    CgMat& cm = plan.mats[m];
-    cm.w_off = off; cm.d = d; cm.dp = dp; cm.first_copy_block = copy_blocks; cm.pad0 = 0;
-    copy_blocks += (dp + CG_COPY_ROWS - 1) / CG_COPY_ROWS;
-    const int64_t t1 = off + cg_align(static_cast<int64_t>(dp) * dp, 64), t2 = t1 + pool;
-    off = t2 + pool;
-    cg_right_looking(seq[m], m, cm.w_off, d, dp, t1);     // the T2 panels of one level: at most dp^2 / 4 + 64 per node
-    CgOp fin;
-    fin.type = CG_PROD;     // out = M^T M, both triangles
-    fin.prods.push_back(cg_prod(m, CG_FLAG_TRANSA | CG_FLAG_OUT_USER, CG_KIND_M, CG_KIND_M, d, d, dp, 1.f, cm.w_off, dp,
-                                cm.w_off, dp, 0.f, 0, d, K_GE_MAXIJ, TILE_LOWER_MIRROR));
-    seq[m].push_back(fin);
-  }
-  plan.steps.push_back(CgStep{CG_COPY, 0, count, copy_blocks, 0, 0});
-  // Merge: the matrix with the most steps left decides the type of the next super-step; every matrix whose next
-  // step has that type takes part.
-  std::vector<size_t> cur(count, 0);
-  for (;;) {
-    int lead = -1;
-    size_t most = 0;
-    for (int m = 0; m < count; ++m) {
-      const size_t left = seq[m].size() - cur[m];
-      if (left > most) { most = left; lead = m; }
-    }
-    if (lead < 0) break;
-    const int type = seq[lead][cur[lead]].type;
-    CgStep st{type, 0, 0, 0, 0, 0};
-    if (type == CG_LEAF) {
-      st.first = static_cast<int>(plan.leaves.size());
-      for (int m = 0; m < count; ++m)
-        if (cur[m] < seq[m].size() && seq[m][cur[m]].type == CG_LEAF) plan.leaves.push_back(seq[m][cur[m]++].leaf);
-      st.count = static_cast<int>(plan.leaves.size()) - st.first;
-      st.grid = st.count;
-    } else {
-      std::vector<CgProd> ps;
-      for (int m = 0; m < count; ++m)
-        if (cur[m] < seq[m].size() && seq[m][cur[m]].type == CG_PROD) {
-          for (const CgProd& p : seq[m][cur[m]].prods) ps.push_back(p);
-          ++cur[m];
-        }
-      if (cg_prefer_deep(ps)) {
-        st.type = CG_PROD_DEEP;
-        for (CgProd& p : ps) cg_make_deep(p);
-      }
-      // longest contraction first: the long tiles start early, the short ones fill the tail
-      std::stable_sort(ps.begin(), ps.end(), [](const CgProd& x, const CgProd& y) { return x.K > y.K; });
-      int64_t tiles = 0;
-      st.first_tile = static_cast<int>(plan.tile_map.size());
-      for (size_t i = 0; i < ps.size(); ++i) {
-        ps[i].first_tile = static_cast<int>(tiles);
-        const int64_t n = cg_tiles(ps[i]);
-        tiles += n;
-        plan.tile_map.insert(plan.tile_map.end(), static_cast<size_t>(n), static_cast<int32_t>(i));
-      }
-      st.first = static_cast<int>(plan.prods.size());
-      st.count = static_cast<int>(ps.size());
-      st.grid = static_cast<int>(tiles);
-      plan.prods.insert(plan.prods.end(), ps.begin(), ps.end());
-    }
-    plan.steps.push_back(st);
-  }
-  CgHeader& h = plan.h;
-  std::memset(&h, 0, sizeof(h));
-  h.magic = CG_MAGIC;
-  h.scales_off = off;
-  off += cg_align(static_cast<int64_t>(count) * CG_SCALE_FLOATS, 64);
-  h.ws_floats = off;
-  h.count = count;
-  h.nsteps = static_cast<int>(plan.steps.size());
-  h.nleaves = static_cast<int>(plan.leaves.size());
-  h.nprods = static_cast<int>(plan.prods.size());
-  h.copy_blocks = copy_blocks;
-  h.ntiles = static_cast<int>(plan.tile_map.size());
-  int64_t b = cg_align(sizeof(CgHeader), 64);
-  h.mats_off = b; b = cg_align(b + plan.mats.size() * sizeof(CgMat), 64);
-  h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
-  h.leaves_off = b; b = cg_align(b + plan.leaves.size() * sizeof(CgLeafTask), 64);
-  h.prods_off = b; b = cg_align(b + plan.prods.size() * sizeof(CgProd), 64);
-  h.map_off = b; b = cg_align(b + plan.tile_map.size() * sizeof(int32_t), 64);
-  h.total_bytes = b;
+  if (!sweep) return;
+  plan = CgPlan();
+  cg_build_sweep(dims, count, plan);
+  plan.h.us = sweep_us;
 }
 
 }  // namespace ak
@@ -678,10 +659,10 @@ extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_hos
   std::memcpy(out, &plan.h, sizeof(CgHeader));
   if (!plan.mats.empty()) std::memcpy(out + plan.h.mats_off, plan.mats.data(), plan.mats.size() * sizeof(CgMat));
   std::memcpy(out + plan.h.steps_off, plan.steps.data(), plan.steps.size() * sizeof(CgStep));
-  if (!plan.leaves.empty()) std::memcpy(out + plan.h.leaves_off, plan.leaves.data(), plan.leaves.size() * sizeof(CgLeafTask));
+  if (!plan.tasks.empty()) std::memcpy(out + plan.h.tasks_off, plan.tasks.data(), plan.tasks.size() * sizeof(CcTask));
   if (!plan.prods.empty()) std::memcpy(out + plan.h.prods_off, plan.prods.data(), plan.prods.size() * sizeof(CgProd));
   if (!plan.sweep_leaves.empty()) {
-    std::memcpy(out + plan.h.leaves_off, plan.sweep_leaves.data(), plan.sweep_leaves.size() * sizeof(SwTask));
+    std::memcpy(out + plan.h.tasks_off, plan.sweep_leaves.data(), plan.sweep_leaves.size() * sizeof(SwTask));
     std::memcpy(out + plan.h.prods_off, plan.sweep_tiles.data(), plan.sweep_tiles.size() * sizeof(SwTask));
   }
   if (!plan.tile_map.empty())
@@ -729,15 +710,17 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
     if (st.type == CG_SWEEP) {
       const SwArgs w{a.ws, A_list, out_list, lam, skip_flags, info, lam_stride, skip_stride};
       hipLaunchKernelGGL(cg_sweep_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, w,
-                         reinterpret_cast<const SwTask*>(a.plan + h->leaves_off),
+                         reinterpret_cast<const SwTask*>(a.plan + h->tasks_off),
                          reinterpret_cast<const SwTask*>(a.plan + h->prods_off), st.count, st.first);
     } else if (st.type == CG_COPY) {
       hipLaunchKernelGGL(cg_copy_in_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
       hipLaunchKernelGGL(cg_scale_kernel, dim3(h->count), dim3(256), 0, s, a, h->count, CG_HALF_MAX_COND);
-    } else if (st.type == CG_LEAF)
-      hipLaunchKernelGGL(cg_leaf_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, a,
-                         reinterpret_cast<const CgLeafTask*>(a.plan + h->leaves_off) + st.first);
-    else
+    } else if (st.type == CG_OUT) {
+      hipLaunchKernelGGL(cg_out_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
+    } else if (st.type == CG_CHAIN) {
+      hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, CcArgs{a.ws, skip_flags, info, skip_stride},
+                         reinterpret_cast<const CcTask*>(a.plan + h->tasks_off) + st.first, st.count);
+    } else
       hipLaunchKernelGGL(st.type == CG_PROD ? cg_prod_kernel : cg_prod_deep_kernel, dim3(st.grid), dim3(256), 0, s, a,
                          reinterpret_cast<const CgProd*>(a.plan + h->prods_off) + st.first,
                          reinterpret_cast<const int32_t*>(a.plan + h->map_off) + st.first_tile);
@@ -748,6 +731,6 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
 #ifdef AK_TUNING_HOOKS
 // Tuning builds only: the bound a / lam up to which a matrix takes the fp16-piece products (0: never).
 extern "C" void ak_debug_set_chol_half_max_cond(float v) { ak::CG_HALF_MAX_COND = v; }
-// Tuning builds only: 1 the sweep, 2 the right-looking factorization, 0 the rule.
+// Tuning builds only: the plan (CG_FORCE), 0: the rule.
 extern "C" void ak_debug_force_chol_plan(int v) { ak::CG_FORCE = v; }
 #endif

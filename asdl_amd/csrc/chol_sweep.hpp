@@ -1,5 +1,5 @@
 // Damped inverses of many small and medium matrices by a block sweep: one launch per 128 columns.  Included by
-// chol_group.hip, whose plan picks between this and the right-looking factorization by their estimated times.
+// chol_group.hip, whose plan picks between this and the chain of chol_chain.hpp by their estimated times.
 //
 // In-place block Gauss-Jordan elimination on the Cholesky factors.  With M_k = L_kk^-1 of the updated diagonal block,
 // step k is ONE symmetric rank-128 update of the whole lower triangle,
@@ -10,24 +10,23 @@
 // (i, j <= k): factorization, triangular inverse and L^-T L^-1 advance together, d^3 FLOP in all as POTRF + POTRI, in
 // ceil(d / 128) dependent steps instead of 3 ceil(d / 128) + 2 log2 + 1 launches.
 //
-// What bounds it: the chain leaf -> update of the next diagonal block -> leaf, 25 us per step: 3 for the operands, 5.5 for
-// v_k+1, 4.5 for the block's update, 12 for the leaf.  Every other work group needs less (two v and a 128 x 128 tile: 20 us)
-// and runs beside it as long as the tiles of all matrices fit the device once.  That is why each work group forms the
-// v_i and v_j that it needs for itself (the same value in every work group) instead of waiting for a launch that forms them
-// once, and why the work group of the next diagonal block goes on to factor it in registers (chol_leaf.hpp).  True fp32
-// products, sums in chunks.  Against the right-looking factorization: (784, 4 x 512, 10) 361 -> 206 us, (1153, 512)
-// 526 -> 284 us, (577, 1000) 427 -> 229 us, 512 alone 180 -> 123 us.
+// What bounds it: the chain leaf -> update of the next diagonal block -> leaf, 22 us per step: 2 for the operands, 4.2 for
+// v_k+1, 4.6 for the block's update, 12 for the leaf (54k cycles).  Every other work group needs less (two v and a 128 x 128
+// tile: 14 to 18 us) and runs beside it as long as the tiles of all matrices fit the device once.  That is why each work group
+// forms the v_i and v_j that it needs for itself (the same value in every work group) instead of waiting for a launch that forms
+// them once, and why the work group of the next diagonal block goes on to factor it in registers (chol_leaf.hpp).
+// Three bf16 pieces per operand (chol_step.hpp) instead of true fp32 products: (784, 4 x 512, 10) 206 -> 180 us, (1153, 512)
+// 284 -> 249, 512 alone 123 -> 110, 2 x 2048 768 -> 566; error against 64 bits of the inverses 2.0e-7 to 3.7e-7 (fp32: 2.0e-7 to
+// 3.7e-7), of rank-deficient ones (16 of 512, 64 of 1153) 7.8e-4 and 4.6e-4 (1.2e-3 and 8.1e-4).
 //
 // No work group reads what another one of the same launch writes: the row and column of the next step are written to
 // the other half of the Y buffer, M alternates likewise, an X tile is read and written by its own work group only.
 #pragma once
-#include "gemm_f32.hpp"
-#include "chol_leaf.hpp"
+#include "chol_step.hpp"
 
 namespace ak {
 
-constexpr int SW_LD = LEAF + 4;              // LDS row: 4 banks further per row, 16-byte reads of 8 rows do not collide
-constexpr int SW_TILE = LEAF * LEAF;
+constexpr int SW_TILE = ST_TILE;
 
 struct SwTask {               // one 128 x 128 tile of a lower triangle; of a leaf list: one matrix (x_off: its first tile)
   int64_t x_off, y_off, m_off;     // floats from the workspace base: X tile, Y (2 x [nb][128][128]), M (2 x [128][128])
@@ -44,69 +43,13 @@ struct SwArgs {
   int lam_stride, skip_stride;
 };
 
-// 128 x 128 floats at P (row stride ld, rows x cols inside), 16 values per thread, zeros outside.
-__device__ __forceinline__ void sw_fetch(floatx4 (&reg)[4], const float* __restrict__ P, int ld, int rows, int cols, int tid) {
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = (tid >> 5) + 32 * u, c = 4 * (tid & 31);
-    floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    const float* src = P + (r * ld + c);       // (at most 128 rows of at most 32768)
-    if (r < rows && c + 4 <= cols) {
-      v = *reinterpret_cast<const floatx4u*>(src);
-    } else if (r < rows) {
-#pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (c + e < cols) v[e] = src[e];
-    }
-    reg[u] = v;
-  }
-}
-
-__device__ __forceinline__ void sw_stash(const floatx4 (&reg)[4], float* __restrict__ lds, bool transposed, int tid) {
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = (tid >> 5) + 32 * u, c = 4 * (tid & 31);
-    if (!transposed) {
-      *reinterpret_cast<floatx4*>(lds + r * SW_LD + c) = reg[u];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) lds[(c + e) * SW_LD + r] = reg[u][e];
-    }
-  }
-}
-
-// 32 x 32 block of a product of two [row][k] panels over k < kmax, in four accumulators: the matrix instruction rounds
-// its accumulator once per two k, and long runs of roundings show in the inverses of ill-conditioned factors.
-__device__ __forceinline__ floatx16 sw_dot(const float* __restrict__ pa, const float* __restrict__ pb, int kmax) {
-  floatx16 part[4];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = part[2][r] = part[3][r] = 0.f;
-#pragma unroll 1
-  for (int q = 0; q < kmax; q += 16) {
-    const floatx4 a = *reinterpret_cast<const floatx4*>(pa + q), b = *reinterpret_cast<const floatx4*>(pb + q);
-    const floatx4 c = *reinterpret_cast<const floatx4*>(pa + q + 8), d = *reinterpret_cast<const floatx4*>(pb + q + 8);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) part[e] = mfma_f32(a[e], b[e], part[e]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) part[e] = mfma_f32(c[e], d[e], part[e]);
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) part[0][r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
-  return part[0];
-}
-
-__device__ __forceinline__ void sw_put(const floatx16& v, float* __restrict__ lds, int wr, int wc, int g, int l32) {
-#pragma unroll
-  for (int r = 0; r < 16; ++r) lds[(32 * wr + 8 * (r >> 2) + 4 * g + (r & 3)) * SW_LD + 32 * wc + l32] = v[r];
-}
-
 // Step k (-1: only the first diagonal block of every matrix is factored).  Work groups 0 ... nleaf - 1: the next
 // diagonal block of a matrix, updated and factored; the others: one tile each.
 static __global__ __launch_bounds__(LEAF_THREADS) void cg_sweep_kernel(SwArgs a, const SwTask* __restrict__ leaves,
                                                                        const SwTask* __restrict__ tiles, int nleaf, int k) {
-  __shared__ __attribute__((aligned(16))) float L0[LEAF * SW_LD];
-  __shared__ __attribute__((aligned(16))) float L1[LEAF * SW_LD];
+  __shared__ __attribute__((aligned(16))) unsigned char st_smem[ST_LDS];
   __shared__ __attribute__((aligned(16))) LeafShared sh;
+  AK_LDS3 unsigned char* lds = (AK_LDS3 unsigned char*)st_smem;
   const bool leaf = static_cast<int>(blockIdx.x) < nleaf;
   const SwTask& t = leaf ? leaves[blockIdx.x] : tiles[blockIdx.x - nleaf];
   const int bi = leaf ? k + 1 : t.bi, bj = leaf ? k + 1 : t.bj;
@@ -120,95 +63,41 @@ static __global__ __launch_bounds__(LEAF_THREADS) void cg_sweep_kernel(SwArgs a,
   const float* __restrict__ Y = a.ws + t.y_off + static_cast<int64_t>(k & 1) * t.nb * SW_TILE;
   const float* __restrict__ M = a.ws + t.m_off + (k & 1) * SW_TILE;
   const int kcols = min(LEAF, t.d);
-  const float* pa = L0 + (32 * wr + l32) * SW_LD + 4 * g;
-  const float* pm = L1 + (32 * wc + l32) * SW_LD + 4 * g;
   const int rows_i = t.d - LEAF * bi, rows_j = t.d - LEAF * bj;
   float* __restrict__ X = a.ws + t.x_off + (leaf ? static_cast<int64_t>(bi) * (bi + 3) / 2 * SW_TILE : 0);
+  auto fetch_y = [&](StPart& y, int b, int rows) {
+    if (k == 0) st_fetch(y, A + static_cast<int64_t>(LEAF) * b * t.d, t.d, rows, kcols, tid);
+    else st_fetch(y, Y + static_cast<int64_t>(b) * SW_TILE, LEAF, LEAF, LEAF, tid);
+  };
+  auto stage_m = [&](const StPart& m) {
+    st_stash(m.v[0], lds, false, tid);
+    st_stash(m.v[1], lds + ST_HALF, false, tid);
+  };
 
   if (leaf) {
-    const int n = min(LEAF, rows_i), nb = (n + LT - 1) / LT, g4 = lane >> 4, c = lane & 15;
+    const int n = min(LEAF, rows_i);
     const float l = a.lam[static_cast<int64_t>(t.mat) * a.lam_stride];
+    StPart m, y;
     if (k >= 0) {
-      floatx4 rm[4], ry[4];
-      sw_fetch(rm, M, LEAF, LEAF, LEAF, tid);
-      if (k == 0) sw_fetch(ry, A + static_cast<int64_t>(LEAF) * bi * t.d, t.d, rows_i, kcols, tid);
-      else sw_fetch(ry, Y + static_cast<int64_t>(bi) * SW_TILE, LEAF, LEAF, LEAF, tid);
-      sw_stash(rm, L1, false, tid);
-      sw_stash(ry, L0, false, tid);
+      st_fetch(m, M, LEAF, LEAF, LEAF, tid);
+      fetch_y(y, bi, rows_i);
     }
-    // Tiles (s, col) of 16 x 16, s <= col: element (16 s + 4 g + r, 16 col + c) is element (16 col + c, 16 s + 4 g + r) of the
-    // lower triangle.  They are dealt to all waves for the update and handed to the waves of the columns through the LDS.
-    constexpr int kMine = 3;
-    int ts[kMine], tc[kMine];
-    floatx4 upd[kMine];          // the block's old values: under way while the product runs
+    floatx16 upd;
+    st_leaf_fetch(upd, [&](int i, int j) {
+      if (k > 0) return *reinterpret_cast<const floatx4*>(X + i * LEAF + j);
+      const float* src = A + static_cast<int64_t>(LEAF * bi + i) * t.d + LEAF * bi + j;
+      floatx4 v;
 #pragma unroll
-    for (int u = 0; u < kMine; ++u) {
-      const int id = wave + 16 * u;           // (integers only: the waves' branches below have to be scalar)
-      tc[u] = (id >= 1) + (id >= 3) + (id >= 6) + (id >= 10) + (id >= 15) + (id >= 21) + (id >= 28) + (id >= 36);
-      ts[u] = id - tc[u] * (tc[u] + 1) / 2;
-      upd[u] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (tc[u] >= nb) continue;
-      const int i = LT * tc[u] + c, j = LT * ts[u] + 4 * g4;
-      if (k > 0) {
-        upd[u] = *reinterpret_cast<const floatx4*>(X + i * LEAF + j);
-      } else {
-        const float* src = A + static_cast<int64_t>(LEAF * bi + i) * t.d + LEAF * bi + j;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (i < n && j + r <= i) upd[u][r] = src[r] + (j + r == i ? l : 0.f);
-      }
-    }
+      for (int r = 0; r < 4; ++r) v[r] = src[min(r, i - min(i, j))] + (j + r == i ? l : 0.f);      // (what lies above the diagonal is dropped)
+      return v;
+    }, n, tid);
+    floatx16 v;
     if (k >= 0) {
-      __syncthreads();
-      const floatx16 v = sw_dot(pa, pm, 32 * (wc + 1));
-      __syncthreads();
-      sw_put(v, L0, wr, wc, g, l32);
-      __syncthreads();
+      stage_m(m);
+      v = st_panel(y, false, lds, wr, wc, tid);
     }
-    floatx4* handed = reinterpret_cast<floatx4*>(L1);
-#pragma unroll
-    for (int u = 0; u < kMine; ++u) {
-      if (tc[u] >= nb) continue;
-      const int i = LT * tc[u] + c, j = LT * ts[u] + 4 * g4;
-      if (k >= 0) {
-        const float* pr = L0 + (LT * ts[u] + c) * SW_LD + 4 * g4;
-        const float* pc = L0 + (LT * tc[u] + c) * SW_LD + 4 * g4;
-        floatx4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
-#pragma unroll 2
-        for (int q = 0; q < LEAF; q += 32) {
-          const floatx4 u0 = *reinterpret_cast<const floatx4*>(pr + q), w0 = *reinterpret_cast<const floatx4*>(pc + q);
-          const floatx4 u1 = *reinterpret_cast<const floatx4*>(pr + q + 16), w1 = *reinterpret_cast<const floatx4*>(pc + q + 16);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            p0 = mfma16(u0[e], w0[e], p0);
-            p1 = mfma16(u1[e], w1[e], p1);
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) upd[u][r] -= p0[r] + p1[r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (i >= n) upd[u][r] = i == j + r ? 1.f : 0.f;      // identity padding
-        if (j + r > i) upd[u][r] = 0.f;
-      }
-      handed[(tc[u] * (tc[u] + 1) / 2 + ts[u]) * 64 + lane] = upd[u];
-    }
-    __syncthreads();
     float* __restrict__ Mn = a.ws + t.m_off + ((k + 1) & 1) * SW_TILE;
-    const int bad = leaf_eliminate(
-        nb, sh, wave, lane, [&](int s, int col) { return handed[(col * (col + 1) / 2 + s) * 64 + lane]; },
-        [&](int s, int col, const floatx4& v) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) Mn[(LT * s + 4 * g4 + r) * LEAF + LT * col + c] = v[r];
-          if (s != col) *reinterpret_cast<floatx4*>(Mn + (LT * col + c) * LEAF + LT * s + 4 * g4) = floatx4{0.f, 0.f, 0.f, 0.f};
-        });
-    if (nb < LEAF_TILES) {         // the identity beyond the matrix
-      for (int e = tid; e < SW_TILE; e += LEAF_THREADS) {
-        const int i = e / LEAF, j = e % LEAF;
-        if (i >= LT * nb || j >= LT * nb) Mn[e] = i == j ? 1.f : 0.f;
-      }
-    }
+    const int bad = st_leaf(upd, [](int, int, const floatx4&) {}, v, k >= 0, n, Mn, lds, sh, wr, wc, tid);
     if (tid == 0 && (a.skip == nullptr || a.skip[static_cast<int64_t>(t.mat) * a.skip_stride] != 0)) {
       const int where = bad != 0 && LEAF * bi + bad <= t.d ? LEAF * bi + bad : 0;
       if (k < 0) a.info[t.mat] = where;
@@ -217,36 +106,19 @@ static __global__ __launch_bounds__(LEAF_THREADS) void cg_sweep_kernel(SwArgs a,
     return;
   }
 
-  floatx4 rm[4], ry[4];
-  sw_fetch(rm, M, LEAF, LEAF, LEAF, tid);
-  if (!ik) {
-    if (k == 0) sw_fetch(ry, A + static_cast<int64_t>(LEAF) * bi * t.d, t.d, rows_i, kcols, tid);
-    else sw_fetch(ry, Y + static_cast<int64_t>(bi) * SW_TILE, LEAF, LEAF, LEAF, tid);
-    sw_stash(ry, L0, false, tid);
-  }
-  sw_stash(rm, L1, false, tid);
-  const bool second = !diag && !jk;
-  if (second) {
-    if (k == 0) sw_fetch(ry, A + static_cast<int64_t>(LEAF) * bj * t.d, t.d, rows_j, kcols, tid);
-    else sw_fetch(ry, Y + static_cast<int64_t>(bj) * SW_TILE, LEAF, LEAF, LEAF, tid);
-  }
-  __syncthreads();
+  StPart m, y;
+  st_fetch(m, M, LEAF, LEAF, LEAF, tid);
+  if (!ik) fetch_y(y, bi, rows_i);
+  stage_m(m);
   floatx16 vi, vj;
-  if (!ik) vi = sw_dot(pa, pm, 32 * (wc + 1));       // M_k is lower triangular
-  if (second) {
+  if (!ik) vi = st_panel(y, false, lds, wr, wc, tid);
+  if (!diag && !jk) {
+    fetch_y(y, bj, rows_j);
     __syncthreads();
-    sw_stash(ry, L0, false, tid);
-    __syncthreads();
-    vj = sw_dot(pa, pm, 32 * (wc + 1));
+    vj = st_panel(y, false, lds, wr, wc, tid);
   }
-  if (ik || jk) sw_fetch(rm, M, LEAF, LEAF, LEAF, tid);      // v_k = M_k^T
-  __syncthreads();
-  if (ik) sw_stash(rm, L0, true, tid);
-  else sw_put(vi, L0, wr, wc, g, l32);
-  if (!diag) {
-    if (jk) sw_stash(rm, L1, true, tid);
-    else sw_put(vj, L1, wr, wc, g, l32);
-  }
+  if (ik) vi = st_own(M, tid);             // v_k = M_k^T
+  if (jk && !diag) vj = st_own(M, tid);
 
   const bool last = k + 1 == t.nb, upper = diag && wr < wc;      // the blocks above the diagonal are not needed
   const int i0 = 32 * wr + 4 * g, j = 32 * wc + l32;             // element r of a wave's block: (i0 + 8 (r / 4) + r % 4, j)
@@ -274,9 +146,8 @@ static __global__ __launch_bounds__(LEAF_THREADS) void cg_sweep_kernel(SwArgs a,
       }
     }
   }
-  __syncthreads();
+  floatx16 sum = st_outer(vi, ik, vj, jk, diag, lds, wr, wc, tid);
   if (upper) return;
-  floatx16 sum = sw_dot(L0 + (32 * wr + l32) * SW_LD + 4 * g, (diag ? L0 : L1) + (32 * wc + l32) * SW_LD + 4 * g, LEAF);
 #pragma unroll
   for (int r = 0; r < 16; ++r) sum[r] = bi <= k ? old[r] + sum[r] : old[r] - sum[r];
 

@@ -189,6 +189,7 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
     case K_GE_J: kbeg = tj * BT; break;
     case K_LE_I: kend = min(p.K, (ti + 1) * BT); break;
     case K_GE_MAXIJ: kbeg = max(ti, tj) * BT; break;
+    case K_GE_I: kbeg = ti * BT; break;
     default: break;
   }
   const float* __restrict__ A = p.A + static_cast<int64_t>(z) * p.sA;

@@ -642,6 +642,46 @@ def test_chol_inv_grouped_block_sweep_edges(K, dims):
             assert torch.equal(out, out.T)
 
 
+# The chain: groups that end after one, two, three and four blocks and inside one, tiles in the step's launch and (many rows) in
+# launches of their own, one matrix and many of other sizes beside it; a skipped matrix and one that is not positive definite.
+@pytest.mark.parametrize('dims', [(3073,), (4097, 130, 5), (3500, 2900, 2561), (1100,) * 24 + (3,), (1537,) * 12 + (300,), (641,) * 40, (513,) * 60])
+def test_chol_inv_grouped_chain(K, dims):
+    plan = K.chol_group_plan(list(dims))
+    assert plan.launches != max((d + 127) // 128 for d in dims) + 1, 'the block sweep: one launch per block column'
+    print(f'chain {len(dims)} x {dims[0]}', flush=True)
+    g = torch.Generator('cuda').manual_seed(len(dims))
+    mats = []
+    for d in dims:
+        x = torch.randn(d + 40, d, device='cuda', generator=g)
+        mats.append(x.T @ x / (d + 40))
+    lam = torch.full((len(dims),), 1e-2, device='cuda')
+    bad, skip = (len(dims) - 2, len(dims) - 1) if len(dims) > 1 else (None, None)
+    active = torch.ones(len(dims), dtype=torch.int32, device='cuda')
+    if bad is not None:
+        mats[bad][100, 100] = -1.0
+        mats[bad][0, 1:].fill_(float('nan'))             # above the diagonal: not read
+        active[skip] = 0
+    outs = [torch.full_like(m, 7.0) for m in mats]
+    info = K.chol_inv_grouped(mats, outs, lam, active=active).cpu()
+    for i, (a, o) in enumerate(zip(mats, outs)):
+        if i == skip:
+            assert bool((o == 7.0).all())
+        elif i == bad:
+            assert int(info[i]) == 101
+        else:
+            assert int(info[i]) == 0 and torch.equal(o, o.T)
+            if i in (0, len(dims) - 3):
+                d = a.shape[0]
+                full = torch.tril(a.double()) + torch.tril(a.double(), -1).T + 1e-2 * torch.eye(d, device='cuda', dtype=torch.float64)
+                inv = o.double()
+                for _ in range(2):                       # two Newton steps in 64 bits: the residual to its fourth power
+                    residual = 2 * torch.eye(d, device='cuda', dtype=torch.float64) - full @ inv
+                    assert float((residual - torch.eye(d, device='cuda', dtype=torch.float64)).norm()) < 0.05
+                    inv = inv @ residual
+                # rounding 2^-22 of the operands, condition up to 4.2 / 1e-2 (Marchenko-Pastur edge over the damping)
+                assert relerr(o, inv) < 420 * 2.0 ** -22, (i, d)
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
