@@ -49,6 +49,14 @@ __device__ __forceinline__ void decode_lower_tile(int id, int& ti, int& tj) {
   tj = id - row * (row + 1) / 2;
 }
 
+// Work groups go to the 8 XCDs round-robin by their linear index, and each XCD has its own L2.  Renumbering them so
+// that one XCD gets a contiguous range of work items lets the tiles of one split share the rows they read through
+// one L2 instead of fetching them once per XCD.
+__device__ __forceinline__ uint32_t xcd_contiguous_id(uint32_t wgid, uint32_t nwg) {
+  const uint32_t xcd = wgid & 7, local = wgid >> 3, q = nwg >> 3, rem = nwg & 7;
+  return xcd * q + (xcd < rem ? xcd : rem) + local;
+}
+
 // Upper-triangular tile enumeration: linear id -> (ti, tj), ti <= tj < T, row-major.
 __device__ __forceinline__ void decode_upper_tile(int id, int T, int& ti, int& tj) {
   int row = 0, len = T;

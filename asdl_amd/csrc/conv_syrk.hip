@@ -17,7 +17,8 @@
 // registers before the MFMAs of stage s; LDS fragments of k-step t+1 are read before the MFMAs of
 // k-step t.  kh = kw = 1 with H = 1 is the plain "X X^T, contraction contiguous" case used for
 // Conv2d.cov_kron_B and for Shampoo's G G^T.
-#include "common.hpp"
+#include "syrk_wave.hpp"
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -585,6 +586,7 @@ extern "C" size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t
   if (patch > 0) return patch;
   ak::ConvPlan a, b;
   size_t need = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
+  if (kh == 1 && kw == 1) need = std::max(need, ak::syrk_wave_ws_bytes(C, N * H * W));
   if (ak::make_plan(a, 2, N, C, H, W, kh, kw, sh, sw, ph, pw) && a.ws_need > need) need = a.ws_need;
   if (ak::make_plan(b, 4, N, C, H, W, kh, kw, sh, sw, ph, pw) && b.ws_need > need) need = b.ws_need;
   return need;
@@ -609,6 +611,14 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
     const int rc = ak::conv_corr_syrk_f32(static_cast<const float*>(x), N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, A,
                                           lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
     if (rc != AK_ERR_UNSUPPORTED) return rc;
+  }
+  // 1 x 1 windows: the staged kernel fills its 128 x 128 tiles from 16-byte loads as well, but has too few of them at every size
+  // that a user has (64 channels 128 x 32 x 32: 32 us, 17 here; 4096 channels 128 x 4 x 4: 874 and 401); never slower
+  if (dtype == AK_F32 && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && N > 0 && H * W > 0 && (H * W) % 8 == 0 &&
+      H * W < (1 << 30) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && C * H * W < (1ll << 30) && lda >= C) {
+    const int rc = ak::launch_syrk_wave(static_cast<const float*>(x), C, N * H * W, H * W, C * H * W, static_cast<int>(H * W), alpha,
+                                        beta, A, lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
+    if (rc != AK_ERR_WORKSPACE) return rc;
   }
   ak::ConvPlan plan;
   if (!ak::make_plan(plan, dtype == AK_BF16 ? 2 : 4, N, C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;

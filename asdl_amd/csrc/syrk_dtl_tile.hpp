@@ -170,14 +170,6 @@ struct DtlCfg {
   static_assert(NCB * (kDtlBK / 16) % NW == 0 && IPW >= 1, "loads must split evenly over the waves");
 };
 
-// Work groups go to the 8 XCDs round-robin by their linear index, and each XCD has its own L2.  Renumbering them so
-// that one XCD gets a contiguous range of work items lets the tiles of one split share the rows they read through
-// one L2 instead of fetching them once per XCD.
-__device__ __forceinline__ uint32_t xcd_contiguous_id(uint32_t wgid, uint32_t nwg) {
-  const uint32_t xcd = wgid & 7, local = wgid >> 3, q = nwg >> 3, rem = nwg & 7;
-  return xcd * q + (xcd < rem ? xcd : rem) + local;
-}
-
 // Rows [k_begin, k_begin + rows) of the operand into tile (ti, tj) of one factor.  partial == nullptr: the result is
 // the factor's tile (alpha, beta, mirror image); otherwise the accumulators go to `partial` in accumulator order,
 // [(a, b, q)][thread] float4, for a reduction pass.  raw != nullptr: the bare tile goes to a row-major matrix.

@@ -8,7 +8,8 @@
 //   fp32: MFMA 32x32x2 takes one k per lane; plain ds_read_b32 along i is conflict free.
 // Both operands of the rank-k update come from the same matrix, so diagonal tiles load a
 // single panel.
-#include "common.hpp"
+#include "syrk_wave.hpp"
+#include <algorithm>
 
 namespace ak {
 
@@ -234,7 +235,8 @@ extern "C" size_t ak_syrk_tn_ws_bytes(int64_t M, int64_t d) {
   const int ns = ak::pick_nsplit(ntiles, (M + 15) / 16);
   const size_t staged = ns > 1 ? static_cast<size_t>(ns) * ntiles * 128 * 128 * sizeof(float) : 0;
   const size_t direct = d % 8 == 0 ? ak::syrk_dtl_plain_ws_bytes(M, d, d) : 0;
-  return staged > direct ? staged : direct;
+  const size_t wave = ak::syrk_wave_ws_bytes(d, M);
+  return std::max(std::max(staged, direct), wave);
 }
 
 extern "C" int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_t ldx, float alpha, float beta,
@@ -247,6 +249,10 @@ extern "C" int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_
     if (rc != AK_ERR_UNSUPPORTED && rc != AK_ERR_WORKSPACE) return rc;
   }
   if (dtype == AK_BF16) return ak::launch_syrk_tn<uint16_t>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
+  if (dtype == AK_F32 && ldx <= (1 << 24) && ak::syrk_wave_rows(d, M)) {
+    const int rc = ak::launch_syrk_wave(static_cast<const float*>(X), d, M, ldx, 0, 0, alpha, beta, C, ldc, ws, ws_bytes, s);
+    if (rc != AK_ERR_WORKSPACE) return rc;
+  }
   if (dtype == AK_F32) return ak::launch_syrk_tn<float>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
   return AK_ERR_ARG;
 }

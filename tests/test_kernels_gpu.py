@@ -1363,3 +1363,28 @@ def test_split_reductions_match_fp64(K, N, C, hw, beta):
     out = old.cuda()
     K.conv_syrk(x.cuda(), (1, 1), (1, 1), (0, 0), out=out, alpha=0.5, beta=beta)
     assert relerr(out, 0.5 * rows.T @ rows + beta * old.double()) < TOL_FACTOR_F32 and torch.equal(out, out.T)
+
+
+@pytest.mark.parametrize("M,d,pad", [(1, 1, 0), (1, 63, 1), (15, 64, 0), (16, 65, 3), (17, 127, 0), (63, 128, 5), (64, 129, 0), (129, 300, 1),
+                                     (1023, 40, 0), (2100, 500, 4), (5003, 129, 0)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_fp32_rows_straight_to_the_matrix_instruction(K, M, d, pad, beta):
+    x = _inputs((M, d + pad), torch.float32, M + d)
+    x[:, d:] = float("nan")                 # columns between the rows are not read
+    rows = x[:, :d].double()
+    out = torch.ones(d, d).cuda()
+    K.syrk_tn(x.cuda()[:, :d], out=out, alpha=0.5, beta=beta)
+    assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
+
+
+@pytest.mark.parametrize("N,C,h,w,offset", [(1, 1, 1, 8, 0), (1, 63, 2, 4, 0), (3, 64, 1, 8, 0), (5, 65, 1, 24, 0), (2, 129, 8, 8, 0), (7, 300, 2, 20, 0),
+                                            (1, 200, 1, 1000, 0), (130, 33, 4, 4, 0), (3, 65, 1, 8, 1), (3, 65, 3, 3, 0)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_fp32_runs_straight_to_the_matrix_instruction(K, N, C, h, w, offset, beta):
+    # the last two go the staged way: a base that is no multiple of 16 bytes, runs that are no multiple of 8
+    flat = _inputs((N * C * h * w + offset,), torch.float32, N + C + w)
+    x = flat[offset:].reshape(N, C, h, w)
+    rows = x.double().permute(0, 2, 3, 1).reshape(-1, C)
+    out = torch.ones(C, C).cuda()
+    K.conv_syrk(flat.cuda()[offset:].reshape(N, C, h, w), (1, 1), (1, 1), (0, 0), out=out, alpha=0.5, beta=beta)
+    assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
