@@ -598,6 +598,8 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   if (x == nullptr || A == nullptr || N <= 0 || C <= 0 || H <= 0 || W <= 0 || kh <= 0 || kw <= 0 || sh <= 0 ||
       sw <= 0 || ph < 0 || pw < 0)
     return AK_ERR_ARG;
+  const bool in_order = dtype == AK_F32_IN_ORDER;
+  if (in_order) dtype = AK_F32;
   if (dtype != AK_BF16 && dtype != AK_F32 && dtype != AK_F32_AS_BF16) return AK_ERR_ARG;
   if (!ak::syrk_beta_ok(beta, C * kh * kw, lda)) return AK_ERR_UNSUPPORTED;
   {  // few input channels: the window kernel
@@ -614,7 +616,7 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   }
   // 1 x 1 windows: the staged kernel fills its 128 x 128 tiles from 16-byte loads as well, but has too few of them at every size
   // that a user has (64 channels 128 x 32 x 32: 32 us, 17 here; 4096 channels 128 x 4 x 4: 874 and 401); never slower
-  if (dtype == AK_F32 && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && N > 0 && H * W > 0 && (H * W) % 8 == 0 &&
+  if (dtype == AK_F32 && !in_order && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && N > 0 && H * W > 0 && (H * W) % 8 == 0 &&
       H * W < (1 << 30) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && C * H * W < (1ll << 30) && lda >= C) {
     const int rc = ak::launch_syrk_wave(static_cast<const float*>(x), C, N * H * W, H * W, C * H * W, static_cast<int>(H * W), alpha,
                                         beta, A, lda, ws, ws_bytes, static_cast<hipStream_t>(stream));

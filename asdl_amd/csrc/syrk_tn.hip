@@ -253,6 +253,6 @@ extern "C" int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_
     const int rc = ak::launch_syrk_wave(static_cast<const float*>(X), d, M, ldx, 0, 0, alpha, beta, C, ldc, ws, ws_bytes, s);
     if (rc != AK_ERR_WORKSPACE) return rc;
   }
-  if (dtype == AK_F32) return ak::launch_syrk_tn<float>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
+  if (dtype == AK_F32 || dtype == AK_F32_IN_ORDER) return ak::launch_syrk_tn<float>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
   return AK_ERR_ARG;
 }

@@ -107,11 +107,19 @@ __device__ __forceinline__ void syrk_wave_sum(floatx16 (&tot)[2][2], const SyrkW
     const int b1 = min(b0 + CHUNK, batches);
     int b = b0;
     for (; b + 2 <= b1; b += 2) {
+      const float* __restrict__ src1 = src;
+      const int pos1 = pos;
       fetch(f1);
       __builtin_amdgcn_sched_barrier(0);         // (all loads of a batch leave before the products of the one before)
       multiply(f0, U);
       __builtin_amdgcn_sched_barrier(0);
-      if (b + 2 < batches) fetch(f0);
+      // (always a fetch, at the end of f1's batch again: one under a condition would make every use wait for all loads)
+      const float* __restrict__ src2 = src;
+      const int pos2 = pos;
+      const bool last = b + 2 == batches;
+      if (last) { src = src1; pos = pos1; }
+      fetch(f0);
+      if (last) { src = src2; pos = pos2; }
       __builtin_amdgcn_sched_barrier(0);
       multiply(f1, U);
       __builtin_amdgcn_sched_barrier(0);

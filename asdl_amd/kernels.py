@@ -13,7 +13,7 @@ import torch
 
 from . import _lib
 
-AK_F32, AK_BF16, AK_F32_AS_BF16 = 0, 1, 2
+AK_F32, AK_BF16, AK_F32_AS_BF16, AK_F32_IN_ORDER = 0, 1, 2, 3
 
 _ws_lock = threading.Lock()
 _workspaces = {}
@@ -683,9 +683,10 @@ def _as_bf16(x):
         return x.to(torch.bfloat16)
 
 
-def syrk_tn(x, out=None, alpha=1.0, beta=0.0, round_bf16=False):
+def syrk_tn(x, out=None, alpha=1.0, beta=0.0, round_bf16=False, in_order=False):
     """out <- beta*out + alpha * x^T x for x = [M, d] (rows may be strided, columns contiguous).  round_bf16: an
-    fp32 x is rounded to bf16 first (what a matmul does to it inside a bf16 autocast region)."""
+    fp32 x is rounded to bf16 first (what a matmul does to it inside a bf16 autocast region).  in_order: an fp32 x is
+    summed in the same order whatever its size (include/asdl_amd.h, AK_F32_IN_ORDER)."""
     _require_gpu(x, out)
     if x.ndim != 2:
         raise ValueError(f'x.ndim has to be 2. Got {x.ndim}.')
@@ -714,7 +715,8 @@ def syrk_tn(x, out=None, alpha=1.0, beta=0.0, round_bf16=False):
     need = _ws_need('ak_syrk_tn_ws_bytes', M, d)
     ws, ws_bytes, keep = _ws_args(need, x.device)
     with _Timed('syrk_tn', flops, floor=floor):
-        rc = lib.ak_syrk_tn(ctypes.c_void_p(x.data_ptr()), _dtype_code(x), M, d, ldx, alpha, beta,
+        code = _dtype_code(x)
+        rc = lib.ak_syrk_tn(ctypes.c_void_p(x.data_ptr()), AK_F32_IN_ORDER if in_order and code == AK_F32 else code, M, d, ldx, alpha, beta,
                             ctypes.c_void_p(out.data_ptr()), out.stride(0), ws, ws_bytes, _stream())
     _lib.check(rc, 'ak_syrk_tn')
     return out
@@ -729,12 +731,12 @@ def _is_channels_last(x):
             and not x.is_contiguous())
 
 
-def conv_syrk(x, kernel_size, stride, padding, out=None, alpha=1.0, beta=0.0, round_bf16=False):
+def conv_syrk(x, kernel_size, stride, padding, out=None, alpha=1.0, beta=0.0, round_bf16=False, in_order=False):
     """out <- beta*out + alpha * sum_{n,pos} patch patch^T for x = [N, C, H, W], patches ordered (c, ky, kx);
     no division by the output size (fold it into alpha).  A channels-last bf16 x is read in place
     (rows gathered from the NHWC memory); anything else goes through the NCHW kernel.  round_bf16: an fp32 x is
     rounded to bf16 (what a matmul does to it inside a bf16 autocast region): while it is read, by the window
-    kernel of the few-channel layers, else by a cast beforehand."""
+    kernel of the few-channel layers, else by a cast beforehand.  in_order: as syrk_tn."""
     _require_gpu(x, out)
     if x.ndim != 4:
         raise ValueError(f'x.ndim has to be 4. Got {x.ndim}.')
@@ -793,21 +795,22 @@ def conv_syrk(x, kernel_size, stride, padding, out=None, alpha=1.0, beta=0.0, ro
     need = _ws_need('ak_conv_syrk_ws_bytes', N, C, H, W, kh, kw, sh, sw, ph, pw)
     ws, ws_bytes, keep = _ws_args(need, x.device)
     with _Timed('conv_syrk', flops, floor=floor):
-        rc = lib.ak_conv_syrk(ctypes.c_void_p(x.data_ptr()), code, N, C, H, W, kh, kw, sh, sw, ph, pw,
-                              alpha, beta, ctypes.c_void_p(out.data_ptr()), out.stride(0), ws, ws_bytes, _stream())
+        rc = lib.ak_conv_syrk(ctypes.c_void_p(x.data_ptr()), AK_F32_IN_ORDER if in_order and code == AK_F32 else code,
+                              N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, ctypes.c_void_p(out.data_ptr()), out.stride(0),
+                              ws, ws_bytes, _stream())
     if rc == AK_ERR_UNSUPPORTED and code == AK_F32_AS_BF16:     # a window too large for the LDS: cast, then the bf16 kernels
         return conv_syrk(_as_bf16(x), kernel_size, stride, padding, out=out, alpha=alpha, beta=beta)
     _lib.check(rc, 'ak_conv_syrk')
     return out
 
 
-def syrk_nt(x, out=None, alpha=1.0, beta=0.0):
-    """out <- beta*out + alpha * sum_n x_n x_n^T for x = [d, K] or [N, d, K] (K contiguous)."""
+def syrk_nt(x, out=None, alpha=1.0, beta=0.0, in_order=False):
+    """out <- beta*out + alpha * sum_n x_n x_n^T for x = [d, K] or [N, d, K] (K contiguous).  in_order: as syrk_tn."""
     if x.ndim == 2:
         x = x.unsqueeze(0)
     if x.ndim != 3:
         raise ValueError(f'x.ndim has to be 2 or 3. Got {x.ndim}.')
-    return conv_syrk(x.unsqueeze(2), (1, 1), (1, 1), (0, 0), out=out, alpha=alpha, beta=beta)
+    return conv_syrk(x.unsqueeze(2), (1, 1), (1, 1), (0, 0), out=out, alpha=alpha, beta=beta, in_order=in_order)
 
 
 # ------------------------------------------------------------------------------ unit-wise blocks

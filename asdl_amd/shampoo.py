@@ -91,13 +91,14 @@ class BlockPartitioner:
 
 def _axis_statistic(grad, axis, out, alpha, beta):
     """out <- beta*out + alpha * (grad contracted with itself over every axis but ``axis``)."""
+    # (in_order: the roots of rank-deficient statistics show the order of the sums)
     ndim = grad.ndim
     if axis == ndim - 1:
-        kernels.syrk_tn(grad.reshape(-1, grad.shape[-1]), out=out, alpha=alpha, beta=beta)
+        kernels.syrk_tn(grad.reshape(-1, grad.shape[-1]), out=out, alpha=alpha, beta=beta, in_order=True)
     elif axis == 0:
-        kernels.syrk_nt(grad.reshape(grad.shape[0], -1), out=out, alpha=alpha, beta=beta)
+        kernels.syrk_nt(grad.reshape(grad.shape[0], -1), out=out, alpha=alpha, beta=beta, in_order=True)
     else:
-        kernels.syrk_nt(grad.movedim(axis, 0).reshape(grad.shape[axis], -1).contiguous(), out=out, alpha=alpha, beta=beta)
+        kernels.syrk_nt(grad.movedim(axis, 0).reshape(grad.shape[axis], -1).contiguous(), out=out, alpha=alpha, beta=beta, in_order=True)
 
 
 HALF_PIECE_STATISTICS = True      # the grouped statistics on two fp16 pieces per element instead of true fp32 products,

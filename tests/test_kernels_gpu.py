@@ -1388,3 +1388,13 @@ def test_fp32_runs_straight_to_the_matrix_instruction(K, N, C, h, w, offset, bet
     out = torch.ones(C, C).cuda()
     K.conv_syrk(flat.cuda()[offset:].reshape(N, C, h, w), (1, 1), (1, 1), (0, 0), out=out, alpha=0.5, beta=beta)
     assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
+
+
+@pytest.mark.parametrize("d,k", [(512, 784), (10, 512), (300, 2000), (64, 8)])
+def test_fp32_statistics_in_a_fixed_order(K, d, k):
+    # a base that is no multiple of 16 bytes takes the staged kernel by itself: the same bits
+    flat = _inputs((d * k + 1,), torch.float32, d + k).cuda()
+    x = flat[1:].reshape(d, k)
+    assert torch.equal(K.syrk_nt(x.clone(), in_order=True), K.syrk_nt(x))
+    rows = x.double().cpu()
+    assert relerr(K.syrk_tn(x.T.contiguous(), in_order=True), rows @ rows.T) < TOL_FACTOR_F32
