@@ -26,25 +26,47 @@ template <int R, int KC> struct DeepPanel {
   typedef floatx4 Regs[CHUNKS];
 };
 
+// No branch around a load (a load under a lane's own condition is waited for before the next one leaves): a panel inside the
+// operand is read as it lies, from a uniform address per load and one lane offset; a chunk beyond an edge reads the last one
+// inside, shifts it and counts as zeros from the edge on.  1000^3: 57 -> 40 us; 300 x 75 x 300: 20 -> 17.
 template <int R, int KC>
 __device__ __forceinline__ void deep_fetch(typename DeepPanel<R, KC>::Regs& reg, const float* __restrict__ P,
                                            int64_t ld, bool kcontig, int r0, int r_end, int k0, int k_end, int tid) {
+  const int o0 = kcontig ? r0 : k0, i0 = kcontig ? k0 : r0, o_end = kcontig ? r_end : k_end, i_end = kcontig ? k_end : r_end;
+  const int row_chunks = kcontig ? KC / 4 : R / 4, step = 256 / row_chunks;       // chunks of a memory row; rows per 256 chunks
+  const int outer = tid / row_chunks, inner = 4 * (tid % row_chunks);
+  const float* __restrict__ base = P + static_cast<int64_t>(o0) * ld + i0;
+  if (o0 + (kcontig ? R : KC) <= o_end && i0 + (kcontig ? KC : R) <= i_end) {
+    const int64_t at = static_cast<int64_t>(outer) * ld + inner;
 #pragma unroll
-  for (int u = 0; u < DeepPanel<R, KC>::CHUNKS; ++u) {
-    const int c = tid + 256 * u;
-    int outer, inner, o_end, i_end;
-    if (kcontig) { outer = r0 + c / (KC / 4); inner = k0 + 4 * (c % (KC / 4)); o_end = r_end; i_end = k_end; }
-    else { outer = k0 + c / (R / 4); inner = r0 + 4 * (c % (R / 4)); o_end = k_end; i_end = r_end; }
-    floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    const float* src = P + static_cast<int64_t>(outer) * ld + inner;
-    if (outer < o_end && inner + 4 <= i_end) {
-      v = *reinterpret_cast<const floatx4u*>(src);
-    } else if (outer < o_end) {
+    for (int u = 0; u < DeepPanel<R, KC>::CHUNKS; ++u) reg[u] = *reinterpret_cast<const floatx4u*>(base + u * step * ld + at);
+  } else if (i_end >= 4) {
+    const int first = i_end - 4 < i0 + inner ? i_end - 4 : i0 + inner, shift = i0 + inner - first;
 #pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (inner + e < i_end) v[e] = src[e];
+    for (int u = 0; u < DeepPanel<R, KC>::CHUNKS; ++u) {
+      const int row = o0 + outer + u * step;
+      reg[u] = *reinterpret_cast<const floatx4u*>(P + static_cast<int64_t>(row < o_end ? row : o_end - 1) * ld + first);
     }
-    reg[u] = v;
+#pragma unroll
+    for (int u = 0; u < DeepPanel<R, KC>::CHUNKS; ++u) {
+      const floatx4 w = reg[u];
+      const bool in = o0 + outer + u * step < o_end;
+      floatx4 v;
+      v[0] = shift == 0 ? w[0] : shift == 1 ? w[1] : shift == 2 ? w[2] : w[3];
+      v[1] = shift == 0 ? w[1] : shift == 1 ? w[2] : w[3];
+      v[2] = shift == 0 ? w[2] : w[3];
+      v[3] = w[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) reg[u][e] = in && shift + e < 4 ? v[e] : 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < DeepPanel<R, KC>::CHUNKS; ++u) {
+      const int row = o0 + outer + u * step;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        reg[u][e] = row < o_end && i0 + inner + e < i_end ? P[static_cast<int64_t>(row) * ld + i0 + inner + e] : 0.f;
+    }
   }
 }
 
@@ -208,7 +230,10 @@ __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int 
 
 static __global__ __launch_bounds__(256) void gemm_deep_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float deep_lds[deep_lds_floats<64, 64, 128>()];
-  gemm_deep_tile<64, 64, 128>(p, blockIdx.y, blockIdx.x, blockIdx.z, deep_lds);
+  // rows of tiles, which read the same rows of A, side by side on one XCD
+  const uint32_t id = xcd_contiguous_id((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, gridDim.x * gridDim.y * gridDim.z);
+  const uint32_t row = id / gridDim.x;
+  gemm_deep_tile<64, 64, 128>(p, row % gridDim.y, id % gridDim.x, row / gridDim.y, deep_lds);
 }
 
 }  // namespace ak

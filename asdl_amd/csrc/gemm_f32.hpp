@@ -239,6 +239,7 @@ static __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
 }  // namespace ak
 
 #include "gemm_deep.hpp"
+#include "gemm_wave.hpp"
 #include "gemm_x3.hpp"
 
 namespace ak {
@@ -258,7 +259,7 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
   const bool lower = p.tile_mode != TILE_ALL;
   const int64_t work_groups = lower ? tiles128 / 2 : tiles128;
   // The split kernel (128 x 128 tiles) has twice the rate of fp32 tiles once its tiles fill most of the device (2048^3, one
-  // tile per CU: 96 us against 128); below that the deep 64 x 64 tiles spread the work better (1024^3: 20 us against 50).
+  // tile per CU: 96 us against 128); below that fp32 tiles of 64 x 64 spread the work better (1024^3: 25 us against 50).
   if (p.split >= 2 && work_groups >= g_x3_min_groups && p.K >= g_x3_min_k && gemm_x3_ok(p)) {
     dim3 grid((p.N + 127) / 128, (p.M + 127) / 128, batch);
     GemmParams q = p;
@@ -281,13 +282,19 @@ inline int launch_gemm(const GemmParams& p, int batch, hipStream_t stream) {
     }
     return check_launch();
   }
-  // 128 x 128 tiles when they alone fill the 256 CUs twice over, else the deep 64 x 64 tiles (four times the work groups)
+  // 128 x 128 tiles when they alone fill the 256 CUs twice over, else 64 x 64 tiles (four times the work groups): operands
+  // straight to the matrix instruction (gemm_wave.hpp), or through the LDS (gemm_deep.hpp) where the CUs hold several tiles and
+  // the contraction is short, or contiguous in both operands (us, LDS and straight: 2048 x 2048 x 256 32 and 37, 2000^3 with
+  // A B^T 198 and 207, with A B 203 and 166, 1000^3 40 and 27), and for rows that 32-bit offsets do not reach.
   if (work_groups >= 512) {
     dim3 grid((p.N + 127) / 128, (p.M + 127) / 128, batch);
     hipLaunchKernelGGL(gemm_f32_kernel<2>, grid, dim3(256), 0, stream, p);
   } else {
     dim3 grid((p.N + 63) / 64, (p.M + 63) / 64, batch);
-    hipLaunchKernelGGL(gemm_deep_kernel, grid, dim3(256), 0, stream, p);
+    const int64_t tiles = static_cast<int64_t>(grid.x) * grid.y * batch / (lower ? 2 : 1);
+    const bool staged = tiles > 256 && (p.K <= 512 || (p.transA == 0 && p.transB != 0));
+    if (staged || !gemm_wave_ok(p)) hipLaunchKernelGGL(gemm_deep_kernel, grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(gemm_wave_kernel, grid, dim3(64 * GEMM_WAVES), 0, stream, p);
   }
   return check_launch();
 }

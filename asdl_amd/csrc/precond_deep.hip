@@ -1,11 +1,12 @@
-// Kronecker preconditioning G <- s B_inv G A_inv, b <- s B_inv b of many small modules in two launches: deep fp32 tiles
-// (gemm_deep.hpp) for all products, the bias products and the 2 x 2 blocks of normalisation layers in work groups beside them.
+// Kronecker preconditioning G <- s B_inv G A_inv, b <- s B_inv b of many small modules in two launches: 64 x 64 fp32 tiles
+// (gemm_wave.hpp) for all products, the bias products and the 2 x 2 blocks of normalisation layers in work groups beside them.
 //
 // Bound by latency: a few dozen 64 x 64 tiles, K of a few hundred.  The split kernel's 128 x 128 tiles take 44 us for one
-// product of 512 x 784 on a nearly idle device and need the operands' ranges first (two more launches); a deep tile takes
-// 2 us per 128 k.  The addresses travel in the kernel arguments: no table has to be built and uploaded per step.
+// product of 512 x 784 on a nearly idle device and need the operands' ranges first (two more launches); a tile of
+// gemm_wave.hpp takes 2.3 us per 128 k.  The addresses travel in the kernel arguments: no table has to be built and uploaded per step.
 // Any size and alignment; the gradients of a call have to be distinct (nothing orders two items of a launch).  MLP 784-512-512-10
-// (three modules with bias): 8 launches, 160 us -> 2 launches, 25 and 34 us, their matrix pipes 15 and 17 % busy.
+// (three modules with bias): 8 launches, 160 us -> 2 launches, 17 and 22 us
+// (25 and 34 with tiles staged through the LDS).
 #include <algorithm>
 #include "gemm_f32.hpp"
 
@@ -41,13 +42,13 @@ struct KpArgs {
   KpUnit unit[KP_ITEMS];
 };
 
-__device__ __forceinline__ GemmParams kp_product(const float* A, const float* B, float* C, int M, int N, int K, int transB,
+__device__ __forceinline__ GemmParams kp_product(const float* A, const float* B, float* C, int M, int N, int K,
                                                  float alpha) {
   GemmParams p;
   p.A = A; p.B = B; p.C = C;
-  p.lda = K; p.ldb = transB ? K : N; p.ldc = N;
+  p.lda = K; p.ldb = N; p.ldc = N;
   p.M = M; p.N = N; p.K = K;
-  p.transA = 0; p.transB = transB;
+  p.transA = 0; p.transB = 0;
   p.alpha = alpha; p.beta = 0.f;
   p.kmode = K_FULL; p.tile_mode = TILE_ALL;
   return p;
@@ -60,33 +61,34 @@ __device__ __forceinline__ int kp_item_of(const KpArgs& a, int w) {
 }
 
 // T <- B_inv G, tb <- B_inv b
-static __global__ __launch_bounds__(256) void kp_first_kernel(KpArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds[deep_lds_floats<64, 64, 128>()];
+static __global__ __launch_bounds__(64 * GEMM_WAVES, 2) void kp_first_kernel(KpArgs a) {
+  __shared__ __attribute__((aligned(16))) float lds[wave_lds_floats<GEMM_WAVES>()];
   const int w = blockIdx.x;
   const KpItem& m = a.item[kp_item_of(a, w)];
   if (w < m.bias_first) {
     const int tn = (m.dA + 63) / 64, local = w - m.first;
-    gemm_deep_tile<64, 64, 128>(kp_product(m.B, m.G, m.T, m.dB, m.dA, m.dB, 0, 1.f), local / tn, local % tn, 0, lds);
+    gemm_wave_tile<GEMM_WAVES>(kp_product(m.B, m.G, m.T, m.dB, m.dA, m.dB, 1.f), local / tn, local % tn, 0, lds);
     return;
   }
-  const int lane = threadIdx.x & 63, row0 = (w - m.bias_first) * KP_GEMV_ROWS + (threadIdx.x >> 6) * 4;
-  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr int ROWS = KP_GEMV_ROWS / GEMM_WAVES;
+  const int lane = threadIdx.x & 63, row0 = (w - m.bias_first) * KP_GEMV_ROWS + (threadIdx.x >> 6) * ROWS;
+  float s[ROWS] = {};
   for (int k = lane; k < m.dB; k += 64) {
     const float x = m.b[k];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s[r] += m.B[static_cast<int64_t>(min(row0 + r, m.dB - 1)) * m.dB + k] * x;
+    for (int r = 0; r < ROWS; ++r) s[r] += m.B[static_cast<int64_t>(min(row0 + r, m.dB - 1)) * m.dB + k] * x;
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
+  for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s[r] += __shfl_xor(s[r], o);
     if (lane == 0 && row0 + r < m.dB) m.tb[row0 + r] = s[r];
   }
 }
 
-// G <- s T A_inv (A_inv is symmetric: read as its transpose, so that both operands are contiguous along k), b <- s tb
-static __global__ __launch_bounds__(256) void kp_second_kernel(KpArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds[deep_lds_floats<64, 64, 128>()];
+// G <- s T A_inv, b <- s tb
+static __global__ __launch_bounds__(64 * GEMM_WAVES, 2) void kp_second_kernel(KpArgs a) {
+  __shared__ __attribute__((aligned(16))) float lds[wave_lds_floats<GEMM_WAVES>()];
   if ((a.fail0 != nullptr && *a.fail0 != 0) || (a.fail1 != nullptr && *a.fail1 != 0)) return;
   const int w = blockIdx.x;
   if (w >= a.end) {
@@ -94,7 +96,7 @@ static __global__ __launch_bounds__(256) void kp_second_kernel(KpArgs a) {
     while (i + 1 < a.units && a.unit[i + 1].first <= w) ++i;
     const KpUnit& u = a.unit[i];
     const int f = (w - u.first) * 256 + threadIdx.x;
-    if (f >= u.F) return;
+    if (threadIdx.x >= 256 || f >= u.F) return;
     const floatx4 v = *reinterpret_cast<const floatx4*>(u.inv + 4 * static_cast<int64_t>(f));
     const float x = u.gw[f] * a.scale, y = u.gb[f] * a.scale;
     u.gw[f] = v[0] * x + v[1] * y;
@@ -104,7 +106,7 @@ static __global__ __launch_bounds__(256) void kp_second_kernel(KpArgs a) {
   const KpItem& m = a.item[kp_item_of(a, w)];
   if (w < m.bias_first) {
     const int tn = (m.dA + 63) / 64, local = w - m.first;
-    gemm_deep_tile<64, 64, 128>(kp_product(m.T, m.A, m.G, m.dB, m.dA, m.dA, 1, a.scale), local / tn, local % tn, 0, lds);
+    gemm_wave_tile<GEMM_WAVES>(kp_product(m.T, m.A, m.G, m.dB, m.dA, m.dA, a.scale), local / tn, local % tn, 0, lds);
     return;
   }
   const int row = (w - m.bias_first) * KP_GEMV_ROWS + threadIdx.x;
@@ -126,8 +128,8 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
                                     ak_stream_t stream) {
   using namespace ak;
   if (count < 0 || unit_count < 0 || (count > 0 && items == nullptr) || (unit_count > 0 && units == nullptr)) return AK_ERR_ARG;
-  // The rule: microseconds of both products on deep tiles against those on the split kernel, whose rates gemm_f32.hpp and
-  // chol_group.hip use too (deep: 2 us per chunk of 128 k; split: 1.6 us per k-tile of 32, 1 us once the device is full, and
+  // The rule: microseconds of both products on 64 x 64 tiles against those on the split kernel, whose rates gemm_f32.hpp and
+  // chol_group.hip use too (64 x 64: 2 us per chunk of 128 k; split: 1.6 us per k-tile of 32, 1 us once the device is full, and
   // 20 us for the ranges of its operands).
   double longest = 0, chunks = 0, long_tile = 0, ktiles = 0;
   for (int i = 0; i < count; ++i) {
@@ -182,8 +184,8 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
       u.F = static_cast<int>(r[3]); u.first = static_cast<int>(w);
       w += (r[3] + 255) / 256;
     }
-    if (a.end > 0) hipLaunchKernelGGL(kp_first_kernel, dim3(a.end), dim3(256), 0, s, a);
-    if (w > 0) hipLaunchKernelGGL(kp_second_kernel, dim3(static_cast<unsigned>(w)), dim3(256), 0, s, a);
+    if (a.end > 0) hipLaunchKernelGGL(kp_first_kernel, dim3(a.end), dim3(64 * GEMM_WAVES), 0, s, a);
+    if (w > 0) hipLaunchKernelGGL(kp_second_kernel, dim3(static_cast<unsigned>(w)), dim3(64 * GEMM_WAVES), 0, s, a);
   }
   return check_launch();
 }

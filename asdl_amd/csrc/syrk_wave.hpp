@@ -228,8 +228,8 @@ inline int syrk_wave_split(int64_t d, int64_t K) {
 
 // Rows: while the busiest CU has no more than 1536 of K, or the matrix is at most two tiles wide.  Beyond that the work groups'
 // loads of the same rows (each 32 columns of one row at a time) count, and the staged kernel with its 128 x 128 tiles is the
-// faster one: staged and here, us: 4096 x 700 (1408 a CU) 45 and 33, 333 x 1999 (999) 47 and 35; 2000 x 1000 (2000) 41 and 57,
-// 1000 x 1500 (2000) 50 and 76, 100000 x 256 (4096) 113 and 144; two tiles wide 200000 x 128 87 and 56, 300000 x 64 130 and 29.
+// faster one: staged and here, us: 4096 x 700 (1408 a CU) 45 and 33, 333 x 1999 (999) 47 and 35; 2000 x 1000 (2000) 41 and 50,
+// 1000 x 1500 (2000) 50 and 76, 100000 x 256 (4096) 113 and 107; two tiles wide 200000 x 128 87 and 56, 300000 x 64 130 and 29.
 inline bool syrk_wave_rows(int64_t d, int64_t K) {
   if (d < 1 || K < 1) return false;
   const int64_t T = (d + 63) / 64, tiles = T * (T + 1) / 2, s = syrk_wave_split(d, K);

@@ -1398,3 +1398,23 @@ def test_fp32_statistics_in_a_fixed_order(K, d, k):
     assert torch.equal(K.syrk_nt(x.clone(), in_order=True), K.syrk_nt(x))
     rows = x.double().cpu()
     assert relerr(K.syrk_tn(x.T.contiguous(), in_order=True), rows @ rows.T) < TOL_FACTOR_F32
+
+
+@pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (1, 65, 17), (65, 1, 200), (64, 64, 16), (63, 66, 15), (129, 33, 127), (2, 130, 128), (200, 129, 143),
+                                    (577, 75, 300), (65, 64, 1153), (31, 700, 2049), (1100, 1100, 300)])
+@pytest.mark.parametrize("transA", [False, True])
+@pytest.mark.parametrize("transB", [False, True])
+def test_fp32_products_straight_to_the_matrix_instruction(K, M, N, Kd, transA, transB):
+    # rows of the operands end where the memory of others begins (NaN): nothing beyond an edge may reach a result
+    a = torch.full((Kd if transA else M, (M if transA else Kd) + 3), float("nan"))
+    b = torch.full((N if transB else Kd, (Kd if transB else N) + 1), float("nan"))
+    A, B = a[:, :-3], b[:, :-1]
+    A.copy_(_inputs(tuple(A.shape), torch.float32, M + Kd))
+    B.copy_(_inputs(tuple(B.shape), torch.float32, N + Kd))
+    old = _inputs((M, N), torch.float32, M + N)
+    ref = 0.5 * (A.double().T if transA else A.double()) @ (B.double().T if transB else B.double())
+    Ag, Bg = a.cuda()[:, :-3], b.cuda()[:, :-1]
+    for beta in (0.0, 1.5):
+        out = old.cuda()
+        K.gemm(Ag, Bg, out=out, transA=transA, transB=transB, alpha=0.5, beta=beta)
+        assert relerr(out, ref + beta * old.double()) < TOL_FACTOR_F32
