@@ -267,31 +267,47 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
         return True
 
     @staticmethod
-    def _groupable(pc):
+    def _groupable(pc, align=4):
         """A matrix-shaped, unpartitioned parameter whose gradient, statistics and preconditioners the grouped
-        split-bf16 GEMM takes (float32, dense, 16-byte aligned, sizes multiples of 4)."""
+        split-bf16 GEMM takes (float32, dense, 16-byte aligned, sizes multiples of 4), or with align = 1 the fp32 tiles
+        of kernels.kron_precond_deep (float32, dense)."""
         grad = pc.param.grad
         shape = pc._transformed_shape
         if grad is None or len(shape) != 2 or tuple(grad.shape) != shape or grad.dtype != torch.float32 \
-                or not grad.is_contiguous() or shape[0] % 4 or shape[1] % 4 or grad.data_ptr() % 16:
+                or not grad.is_contiguous() or shape[0] % align or shape[1] % align or grad.data_ptr() % (4 * align):
             return False
         for mats in (pc.statistics, pc.preconditioners):
             if len(mats) != 2:
                 return False
             for q, n in zip(mats, shape):
                 if not isinstance(q, torch.Tensor) or tuple(q.shape) != (n, n) or not q.is_contiguous() \
-                        or q.dtype != torch.float32 or q.data_ptr() % 16:
+                        or q.dtype != torch.float32 or q.data_ptr() % (4 * align):
                     return False
         return True
 
-    def _split_groupable(self):
-        if not GROUPED_PRECONDITION:
-            return [], list(self.preconditioners)
-        grouped = [pc for pc in self.preconditioners if self._groupable(pc)]
+    def _split_groupable(self, among=None):
+        among = list(self.preconditioners) if among is None else among
+        grouped = [pc for pc in among if self._groupable(pc)] if GROUPED_PRECONDITION else []
         if len(grouped) < 2:
-            return [], list(self.preconditioners)
+            return [], among
         taken = set(map(id, grouped))
-        return grouped, [pc for pc in self.preconditioners if id(pc) not in taken]
+        return grouped, [pc for pc in among if id(pc) not in taken]
+
+    def _precondition_deep(self):
+        """All matrix-shaped parameters of a small model in two launches of fp32 tiles, whatever their sizes' alignment
+        (784-512-512-10: seven launches, 132 us, before; two, 39 us, now; the rule of ak_kron_precond_deep, which takes these
+        products for Kronecker factors too).  The roots are symmetric.  Returns the parameters that are left."""
+        small = [pc for pc in self.preconditioners if self._groupable(pc, align=1)] if GROUPED_PRECONDITION else []
+        if not small:
+            return list(self.preconditioners)
+        items = []
+        for pc in small:
+            p0, p1 = pc.preconditioners
+            items += [p0.data_ptr(), p1.data_ptr(), pc.param.grad.data_ptr(), 0, *pc._transformed_shape]
+        if not kernels.kron_precond_deep(items, [], 1.0, small[0].param.device):
+            return list(self.preconditioners)
+        taken = set(map(id, small))
+        return [pc for pc in self.preconditioners if id(pc) not in taken]
 
     def update_curvature(self):
         """Statistics of every axis (asdl/precondition/shampoo.py:331-339).  The large ones of matrix-shaped
@@ -354,9 +370,9 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
     def precondition(self):
         """P_0^T G P_1 for every matrix-shaped parameter in two grouped launches (all G^T P_0, then all (.)^T P_1:
         the per-axis tensordot chain of asdl/precondition/shampoo.py:351-367, on the split-bf16 kernel with all 24
-        mantissa bits); parameters with more axes, blocks or unaligned sizes go one at a time."""
+        mantissa bits), or in fp32 where all are small; parameters with more axes, blocks or unaligned sizes go one at a time."""
         specs_first, specs_second, off = [], [], 0
-        grouped, rest = self._split_groupable()
+        grouped, rest = self._split_groupable(self._precondition_deep())
         if grouped:
             dev = grouped[0].param.device
             buf, _ = kernels.workspace(4 * sum(pc.param.numel() for pc in grouped), dev)

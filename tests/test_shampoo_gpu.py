@@ -751,3 +751,25 @@ def test_roots_have_the_same_bits_in_every_launch_shape(p, eps):
     for got in few:
         for n, (root, _) in got.items():
             assert torch.equal(root, alone[n][0]), n
+
+
+@pytest.mark.parametrize("widths", [(5, 3), (64, 65, 1), (784, 512, 512, 10), (33, 1000, 7)])
+def test_small_matrices_precondition_in_two_launches(widths):
+    torch.manual_seed(0)
+    model = nn.Sequential(*(nn.Linear(a, b) for a, b in zip(widths, widths[1:])), nn.Unflatten(1, (1, widths[-1], 1)),
+                          nn.Conv2d(1, 2, 1)).cuda()
+    maker = ShampooGradientMaker(model, PreconditioningConfig(damping=1e-6))
+    expected = []
+    for pc in maker.preconditioners:
+        for q in pc.preconditioners:
+            x = torch.randn_like(q)
+            q.copy_(x @ x.T / len(x) + torch.eye(len(x), device="cuda"))
+            q.copy_(0.5 * (q + q.T))
+        pc.param.grad = torch.randn_like(pc.param)
+        g = pc.param.grad.double()
+        for q in pc.preconditioners:
+            g = torch.tensordot(g, q.double(), dims=([0], [0]))
+        expected.append(g)
+    maker.precondition()
+    for pc, g in zip(maker.preconditioners, expected):
+        assert relerr(pc.param.grad, g) < 1e-5
