@@ -2,6 +2,7 @@
 // preconditioning G <- grad_scale * Binv G Ainv (+ bias <- grad_scale * Binv bias).
 #include <mutex>
 #include "gemm_f32.hpp"
+#include "gemm_half.hpp"
 
 namespace ak {
 
@@ -241,6 +242,10 @@ extern "C" int ak_gemm_f32_grouped(int pieces, const int64_t* table, int count, 
   const dim3 grid(static_cast<unsigned>(total_tiles));
   if (pieces == 0) hipLaunchKernelGGL(ak::gemm_f32_grouped_kernel, grid, dim3(256), 0, s, table, count);
   else if (pieces == 2) hipLaunchKernelGGL(ak::gemm_x3_grouped_kernel<2>, grid, dim3(256), 0, s, table, count);
+  // 256 x 128 tiles where they fill the device twice over (gemm_half.hpp); with fewer the last wave of them counts: 864 tiles
+  // of 128 x 128 of mixed lengths 212 us, 225 as 432 tall ones; 432 of 768^3 54 and 70
+  else if (pieces == 22 && total_tiles >= 1024)
+    hipLaunchKernelGGL(ak::gemm_half_grouped_kernel, grid, dim3(256), 0, s, table, count);
   else if (pieces == 22) hipLaunchKernelGGL((ak::gemm_x3_grouped_kernel<2, true>), grid, dim3(256), 0, s, table, count);
   else if (pieces == 23) hipLaunchKernelGGL((ak::gemm_x3_grouped_kernel<2, true, true>), grid, dim3(256), 0, s, table, count);
   else hipLaunchKernelGGL(ak::gemm_x3_grouped_kernel<3>, grid, dim3(256), 0, s, table, count);

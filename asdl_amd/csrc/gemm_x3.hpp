@@ -536,19 +536,21 @@ __device__ __forceinline__ float x3_half_scale(float absmax) {
   return ldexpf(1.f, 14 - e);
 }
 
+// fp16 pieces: the operands' largest magnitudes (device words named by the table row) give the scales.
+__device__ __forceinline__ void grouped_half_scales(const int64_t* __restrict__ table, int count, int w, GemmParams& p) {
+  const int64_t* __restrict__ r = table + static_cast<int64_t>(grouped_row_of(table, count, w)) * GROUPED_ROW;
+  p.scaleA = x3_half_scale(*reinterpret_cast<const float*>(r[12]));
+  p.scaleB = x3_half_scale(*reinterpret_cast<const float*>(r[13]));
+  p.alpha = p.alpha / (p.scaleA * p.scaleB);       // powers of two: exact
+}
+
 template <int NSPLIT, bool HALF = false, bool CHUNKED = false>
 static __global__ __launch_bounds__(256, 2) void gemm_x3_grouped_kernel(const int64_t* __restrict__ table, int count) {
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * NSPLIT * X3_PLANE];
   GemmParams p;
   int ti, tj;
   if (!grouped_lookup(table, count, blockIdx.x, p, ti, tj)) return;
-  if constexpr (HALF) {
-    // fp16 pieces: the operands' largest magnitudes (device words named by the table row) give the scales
-    const int64_t* __restrict__ r = table + static_cast<int64_t>(grouped_row_of(table, count, blockIdx.x)) * GROUPED_ROW;
-    p.scaleA = x3_half_scale(*reinterpret_cast<const float*>(r[12]));
-    p.scaleB = x3_half_scale(*reinterpret_cast<const float*>(r[13]));
-    p.alpha = p.alpha / (p.scaleA * p.scaleB);       // powers of two: exact
-  }
+  if constexpr (HALF) grouped_half_scales(table, count, blockIdx.x, p);
   // two work groups per CU with the single-buffered loop serve the mix of long and short contractions of a
   // grouped launch better than one work group with the double-buffered loop (measured: 0.99 against 1.25 ms)
   // one instantiation per pair of operand layouts: with the layout a runtime value every fragment's read stood behind a branch

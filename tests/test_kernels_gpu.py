@@ -1418,3 +1418,41 @@ def test_fp32_products_straight_to_the_matrix_instruction(K, M, N, Kd, transA, t
         out = old.cuda()
         K.gemm(Ag, Bg, out=out, transA=transA, transB=transB, alpha=0.5, beta=beta)
         assert relerr(out, ref + beta * old.double()) < TOL_FACTOR_F32
+
+
+@pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_grouped_half_pieces_in_tall_tiles_have_the_same_bits(K, transA, transB):
+    # alone, every product stays below the number of tiles from which a launch takes two tile rows per work group
+    sizes = [(4100, 3972, 100), (128, 128, 32), (260, 132, 4), (388, 516, 64), (64, 1000, 36), (2052, 260, 96)]
+    A = [_inputs((k, m) if transA else (m, k), torch.float32, m + k).cuda() for m, n, k in sizes]
+    B = [_inputs((n, k) if transB else (k, n), torch.float32, n + k).cuda() for m, n, k in sizes]
+
+    def run(which):
+        mx = torch.zeros(len(sizes), 3, device="cuda")
+        out = [torch.full((m, n), 0.25, device="cuda") for m, n, k in sizes]
+        specs = []
+        for i in which:
+            m, n, k = sizes[i]
+            mx[i, 0], mx[i, 1] = A[i].abs().max(), B[i].abs().max()
+            w = mx.data_ptr() + 12 * i
+            specs.append((A[i].data_ptr(), A[i].stride(0), B[i].data_ptr(), B[i].stride(0), out[i].data_ptr(), n, m, n, k,
+                          transA, transB, 0.5, 2.0 if i == 3 else 0.0, False, w, w + 4, w + 8))
+        K.gemm_grouped_raw(specs, torch.device("cuda"), pieces=22)
+        return out, mx[:, 2]
+    together, largest = run(range(len(sizes)))
+    for i, (m, n, k) in enumerate(sizes):
+        if i == 0:
+            pieces = []
+            for half in (0, 1):                     # 33 x 32 tiles in two launches of fewer than 1024
+                sl = slice(0, 2048) if half == 0 else slice(2048, m)
+                a = A[0][:, sl] if transA else A[0][sl]
+                o, mx = torch.empty(sl.stop - sl.start, n, device="cuda"), torch.zeros(3, device="cuda")
+                mx[0], mx[1] = A[0].abs().max(), B[0].abs().max()
+                K.gemm_grouped_raw([(a.data_ptr(), a.stride(0), B[0].data_ptr(), B[0].stride(0), o.data_ptr(), n, o.shape[0], n, k,
+                                     transA, transB, 0.5, 0.0, False, mx.data_ptr(), mx.data_ptr() + 4, 0)], o.device, pieces=22)
+                pieces.append(o)
+            alone = torch.cat(pieces)
+        else:
+            alone = run([i])[0][i]
+        assert torch.equal(together[i], alone)
+        assert float(largest[i]) == float(alone.abs().max())
