@@ -626,6 +626,11 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   if (!ak::make_plan(plan, dtype == AK_BF16 ? 2 : 4, N, C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;
   if (lda < plan.p.d) return AK_ERR_ARG;
   if (plan.ws_need > 0 && (ws == nullptr || ws_bytes < plan.ws_need)) return AK_ERR_WORKSPACE;
+  // one matrix in the staged kernel's order of sums: the chain, whose groups of 16 k its stages are whole numbers of
+  if (in_order && N == 1 && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && (H * W) % 8 == 0 && plan.p.R == 1 &&
+      plan.p.WC % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && C * H * W < (1ll << 30))
+    return ak::launch_syrk_chain(static_cast<const float*>(x), C, H * W, H * W, true, plan.p.nsplit, plan.p.stages_per_split * plan.p.WC,
+                                 alpha, beta, A, lda, ws, static_cast<hipStream_t>(stream));
   plan.p.x = x; plan.p.alpha = alpha; plan.p.beta = beta; plan.p.A = A; plan.p.lda = lda;
   plan.p.ws = static_cast<float*>(ws);
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -203,6 +203,8 @@ static int launch_syrk_tn(const void* X, int64_t M, int64_t d, int64_t ldx, floa
     const size_t need = static_cast<size_t>(nsplit) * ntiles * BT * BT * sizeof(float);
     if (ws == nullptr || ws_bytes < need) return AK_ERR_WORKSPACE;
   }
+  if (sizeof(T) == 4 && M > 0 && ldx <= (1 << 24) && syrk_chain_rows(d, M))
+    return launch_syrk_chain(static_cast<const float*>(X), d, M, ldx, false, nsplit, steps_per_split * BK, alpha, beta, C, ldc, ws, stream);
   SyrkTnParams p;
   p.X = X; p.M = M; p.d = d; p.ldx = ldx; p.alpha = alpha; p.beta = beta; p.C = C; p.ldc = ldc;
   p.ws = static_cast<float*>(ws); p.T = static_cast<int>(Tn); p.nsplit = nsplit;

@@ -210,6 +210,115 @@ static __global__ __launch_bounds__(256, 2) void syrk_wave_kernel(SyrkWaveParams
   else store_partial<1, 1>(sum, p.ws + static_cast<size_t>(id) * 4096, tid);
 }
 
+// The same result with the staged kernels' order of sums (AK_F32_IN_ORDER): their splits of K, one accumulator over each of
+// them, the k of an instruction paired as there (rows: 2 u and 2 u + 1; runs: 16 t + m and 16 t + 8 + m).  A work group owns a
+// 64 x 64 tile of one split, a wave a 32 x 32 block of it.  Bound by the chain of matrix instructions (64 cycles per two k) behind
+// one way to memory, 64 k of both operands in flight.  us, staged and here:
+// one 512 x 784 matrix 55 and 14.5, 767 x 3072 54 and 48, rows of 512 x 512 18.7 and 11.6.
+template <bool RUNS, bool MASK>
+__device__ __forceinline__ void syrk_chain_fetch(float (&x)[32], const float* __restrict__ X, int64_t ld, uint32_t at, int64_t k, int64_t k1,
+                                                 int g) {
+  if constexpr (RUNS) {                       // X: the matrix, at: the lane's row and 8 g; k1 - k a multiple of 8
+    const float* __restrict__ src = X + k;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int over = MASK ? 16 * t + 8 * g - static_cast<int>(k1 - k - 8) : 0;       // beyond the range: its last eight
+      const int back = over > 0 ? over : 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const floatx4 v = *reinterpret_cast<const floatx4*>(src + 16 * t + 4 * h + (static_cast<int64_t>(at) - back));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[8 * t + 4 * h + e] = back > 0 ? 0.f : v[e];
+      }
+    }
+  } else {                                    // at: the lane's column and g rows
+    const float* __restrict__ src = X + k * ld;
+#pragma unroll
+    for (int u = 0; u < 32; ++u) {
+      const int over = MASK ? 2 * u + g - static_cast<int>(k1 - k - 1) : 0;
+      const int back = over > 0 ? over : 0;
+      const float v = (src + 2 * u * ld)[static_cast<int64_t>(at) - back * ld];
+      x[u] = back > 0 ? 0.f : v;
+    }
+  }
+}
+
+template <bool RUNS>
+static __global__ __launch_bounds__(256, 2) void syrk_chain_kernel(SyrkWaveParams p) {
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 1, wc = wave & 1;
+  const uint32_t ntiles = static_cast<uint32_t>(p.T * (p.T + 1) / 2), split = blockIdx.x / ntiles, tile = blockIdx.x - split * ntiles;
+  int ti, tj;
+  decode_upper_tile(static_cast<int>(tile), p.T, ti, tj);
+  const int i0 = 64 * ti + 32 * wr, j0 = 64 * tj + 32 * wc;
+  const int64_t k0 = static_cast<int64_t>(split) * p.per_split, k1 = k0 + p.per_split < p.K ? k0 + p.per_split : p.K;
+  auto lane_offset = [&](int c0) {            // columns beyond the matrix read the last one: their sums are not stored
+    const int col = min(c0 + l32, p.d - 1);
+    return RUNS ? static_cast<uint32_t>(col) * static_cast<uint32_t>(p.ld) + 8 * g : g * static_cast<uint32_t>(p.ld) + col;
+  };
+  const uint32_t ai = lane_offset(i0), aj = lane_offset(j0);
+  floatx16 acc[1][1];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[0][0][r] = 0.f;
+  struct Batch { float a[32], b[32]; };
+  auto fetch = [&](Batch& f, int64_t k) {
+    syrk_chain_fetch<RUNS, false>(f.a, p.X, p.ld, ai, k, k1, g);
+    syrk_chain_fetch<RUNS, false>(f.b, p.X, p.ld, aj, k, k1, g);
+  };
+  auto multiply = [&](const Batch& f) {
+#pragma unroll
+    for (int u = 0; u < 32; ++u) acc[0][0] = mfma_f32(f.a[u], f.b[u], acc[0][0]);
+  };
+  const int batches = static_cast<int>((k1 - k0) / 64);
+  Batch f0, f1;
+  if (batches > 0) {
+    // (always a fetch, of the last batch again at the end: one under a condition would make every use wait for all loads)
+    fetch(f0, k0);
+    int b = 0;
+    for (; b + 2 <= batches; b += 2) {
+      fetch(f1, k0 + 64 * (b + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(f0);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(f0, k0 + 64 * static_cast<int64_t>(min(b + 2, batches - 1)));
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(f1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (b < batches) multiply(f0);
+  }
+  if (k0 + 64 * batches < k1) {
+    const int64_t k = k0 + 64 * batches;
+    syrk_chain_fetch<RUNS, true>(f0.a, p.X, p.ld, ai, k, k1, g);
+    syrk_chain_fetch<RUNS, true>(f0.b, p.X, p.ld, aj, k, k1, g);
+    multiply(f0);
+  }
+  if (p.nsplit == 1) syrk_epilogue<1, 1>(acc, p.C, p.ldc, p.d, i0, j0, ti == tj, p.alpha, p.beta, lane);
+  else store_partial<1, 1>(acc, p.ws + static_cast<size_t>(blockIdx.x) * 4096, tid);
+}
+
+// Rows: up to 176 k of tiles a CU; beyond that the loads of 32 columns of a row count (staged and here, us: 512 x 767 28 and 21,
+// 700 x 600 24 and 22, 1000 x 700 27.5 and 28, 2000 x 512 24 and 27, 2000 x 700 38 and 47).
+inline bool syrk_chain_rows(int64_t d, int64_t K) {
+  const int64_t T = (d + 63) / 64;
+  return T * (T + 1) / 2 * K <= 176 * 256;
+}
+
+// The staged kernels' plan: nsplit ranges of per_split k.  runs: rows of K contiguous elements (K and per_split multiples of 8, the
+// base 16-byte aligned), else K rows; the caller has checked that d ld and 4 ld fit 32 bits and that ws holds the partial tiles.
+inline int launch_syrk_chain(const float* X, int64_t d, int64_t K, int64_t ld, bool runs, int nsplit, int64_t per_split, float alpha,
+                             float beta, float* C, int64_t ldc, void* ws, hipStream_t stream) {
+  SyrkWaveParams p;
+  const int64_t T = (d + 63) / 64, tiles = T * (T + 1) / 2;
+  p.X = X; p.ld = ld; p.sn = 0; p.K = K; p.per_split = per_split; p.d = static_cast<int>(d); p.run = 0;
+  p.T = static_cast<int>(T); p.nsplit = nsplit; p.alpha = alpha; p.beta = beta; p.C = C; p.ldc = ldc; p.ws = static_cast<float*>(ws);
+  const dim3 grid(static_cast<unsigned>(tiles * nsplit));
+  if (runs) hipLaunchKernelGGL(syrk_chain_kernel<true>, grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(syrk_chain_kernel<false>, grid, dim3(256), 0, stream, p);
+  if (nsplit > 1) launch_syrk_finalize<1>(p.ws, nsplit, tiles, p.T, C, ldc, d, alpha, beta, stream);
+  return check_launch();
+}
+
 // The split of K whose estimated time is shortest: matrix instructions, and for more than one part their way through memory
 // and the second launch.
 inline int syrk_wave_split(int64_t d, int64_t K) {

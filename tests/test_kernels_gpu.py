@@ -1390,14 +1390,27 @@ def test_fp32_runs_straight_to_the_matrix_instruction(K, N, C, h, w, offset, bet
     assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
 
 
-@pytest.mark.parametrize("d,k", [(512, 784), (10, 512), (300, 2000), (64, 8)])
-def test_fp32_statistics_in_a_fixed_order(K, d, k):
-    # a base that is no multiple of 16 bytes takes the staged kernel by itself: the same bits
+@pytest.mark.parametrize("d,k", [(512, 784), (10, 512), (300, 2000), (64, 8), (65, 72), (33, 24), (767, 3072), (1, 136)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_fp32_statistics_in_a_fixed_order(K, d, k, beta):
+    # a base that is no multiple of 16 bytes, and rows 2^24 elements and more apart, take the staged kernels: the same bits
     flat = _inputs((d * k + 1,), torch.float32, d + k).cuda()
     x = flat[1:].reshape(d, k)
-    assert torch.equal(K.syrk_nt(x.clone(), in_order=True), K.syrk_nt(x))
+    old = torch.ones(d, d, device="cuda")
+    a, b = old.clone(), old.clone()
+    K.syrk_nt(x.clone(), out=a, alpha=0.5, beta=beta, in_order=True)
+    K.conv_syrk(x[None, :, None], (1, 1), (1, 1), (0, 0), out=b, alpha=0.5, beta=beta, in_order=True)
+    assert torch.equal(a, b) and torch.equal(a, a.T)
     rows = x.double().cpu()
-    assert relerr(K.syrk_tn(x.T.contiguous(), in_order=True), rows @ rows.T) < TOL_FACTOR_F32
+    assert relerr(a, 0.5 * rows @ rows.T + beta) < TOL_FACTOR_F32
+    if k <= 136:
+        wide = torch.empty((k - 1) * ((1 << 24) + 4) + d, device="cuda").as_strided((k, d), ((1 << 24) + 4, 1))
+        wide.copy_(x.T)
+        c = old.clone()
+        a = old.clone()
+        K.syrk_tn(wide, out=c, alpha=0.5, beta=beta, in_order=True)
+        K.syrk_tn(x.T.contiguous(), out=a, alpha=0.5, beta=beta, in_order=True)
+        assert torch.equal(a, c) and relerr(a, 0.5 * rows @ rows.T + beta) < TOL_FACTOR_F32
 
 
 @pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (1, 65, 17), (65, 1, 200), (64, 64, 16), (63, 66, 15), (129, 33, 127), (2, 130, 128), (200, 129, 143),
