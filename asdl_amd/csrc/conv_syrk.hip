@@ -17,7 +17,7 @@
 // registers before the MFMAs of stage s; LDS fragments of k-step t+1 are read before the MFMAs of
 // k-step t.  kh = kw = 1 with H = 1 is the plain "X X^T, contraction contiguous" case used for
 // Conv2d.cov_kron_B and for Shampoo's G G^T.
-#include "syrk_wave.hpp"
+#include "syrk_window.hpp"
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -587,6 +587,11 @@ extern "C" size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t
   ak::ConvPlan a, b;
   size_t need = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
   if (kh == 1 && kw == 1) need = std::max(need, ak::syrk_wave_ws_bytes(C, N * H * W));
+  {
+    const int64_t Ho = (H + 2 * ph - kh) / sh + 1, Wo = (W + 2 * pw - kw) / sw + 1;
+    if (H + 2 * ph >= kh && W + 2 * pw >= kw && ak::syrk_window_faster(N, C, H, W, kh, kw, sh, sw, Ho, Wo))
+      need = std::max(need, ak::syrk_window_ws_bytes(C * kh * kw, N * Ho * Wo));
+  }
   if (ak::make_plan(a, 2, N, C, H, W, kh, kw, sh, sw, ph, pw) && a.ws_need > need) need = a.ws_need;
   if (ak::make_plan(b, 4, N, C, H, W, kh, kw, sh, sw, ph, pw) && b.ws_need > need) need = b.ws_need;
   return need;
@@ -626,6 +631,12 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   if (!ak::make_plan(plan, dtype == AK_BF16 ? 2 : 4, N, C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;
   if (lda < plan.p.d) return AK_ERR_ARG;
   if (plan.ws_need > 0 && (ws == nullptr || ws_bytes < plan.ws_need)) return AK_ERR_WORKSPACE;
+  const int64_t Ho = (H + 2 * ph - kh) / sh + 1, Wo = (W + 2 * pw - kw) / sw + 1;
+  if (dtype == AK_F32 && !in_order && ak::syrk_window_faster(N, C, H, W, kh, kw, sh, sw, Ho, Wo)) {
+    const int rc = ak::launch_syrk_window(static_cast<const float*>(x), N, C, H, W, kh, kw, sh, sw, ph, pw, Ho, Wo, alpha, beta, A, lda,
+                                          ws, ws_bytes, static_cast<hipStream_t>(stream));
+    if (rc != AK_ERR_WORKSPACE) return rc;
+  }
   // one matrix in the staged kernel's order of sums: the chain, whose groups of 16 k its stages are whole numbers of
   if (in_order && N == 1 && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && (H * W) % 8 == 0 && plan.p.R == 1 &&
       plan.p.WC % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && C * H * W < (1ll << 30))

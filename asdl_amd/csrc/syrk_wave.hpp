@@ -149,6 +149,41 @@ __device__ __forceinline__ void syrk_wave_sum(floatx16 (&tot)[2][2], const SyrkW
   }
 }
 
+// Adds the four waves' sums of a tile and stores them: wave w block w.  part: 64 KB of LDS; id: the tile's place in the partial sums.
+__device__ __forceinline__ void syrk_wave_finish(const floatx16 (&acc)[2][2], floatx4 (*part)[4][4][64], const SyrkWaveParams& p, uint32_t id,
+                                                 int i0, int j0, bool diag) {
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        part[wave][2 * a + b][q][lane] = floatx4{acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+  __syncthreads();
+  const int wr = wave >> 1, wc = wave & 1;
+  floatx16 sum[1][1];
+  if (diag && wave == 2) {           // block (1, 0) of a diagonal tile is block (0, 1) transposed: element (r, c) is its (c, r)
+    const float* flat = reinterpret_cast<const float*>(&part[0][1][0][0]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      // element (row l32, column 8 (r / 4) + 4 g + r % 4) of block (0, 1): quad l32 / 8, lane 32 (l32 / 4 % 2) + column, entry l32 % 4
+      const int at01 = ((l32 >> 3) * 64 + 32 * ((l32 >> 2) & 1) + 8 * (r >> 2) + 4 * g + (r & 3)) * 4 + (l32 & 3);
+      sum[0][0][r] = (flat[at01] + flat[at01 + 4096]) + (flat[at01 + 8192] + flat[at01 + 12288]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 v = (part[0][wave][q][lane] + part[1][wave][q][lane]) + (part[2][wave][q][lane] + part[3][wave][q][lane]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[0][0][4 * q + e] = v[e];
+    }
+  }
+  if (p.nsplit == 1) syrk_epilogue<1, 1>(sum, p.C, p.ldc, p.d, i0 + 32 * wr, j0 + 32 * wc, diag, p.alpha, p.beta, lane);
+  else store_partial<1, 1>(sum, p.ws + static_cast<size_t>(id) * 4096, tid);
+}
+
 template <bool RUNS>
 static __global__ __launch_bounds__(256, 2) void syrk_wave_kernel(SyrkWaveParams p) {
   __shared__ __attribute__((aligned(16))) floatx4 part[4][4][4][64];
@@ -180,34 +215,7 @@ static __global__ __launch_bounds__(256, 2) void syrk_wave_kernel(SyrkWaveParams
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
   if (diag) syrk_wave_sum<RUNS, true>(acc, p, k, k1, at, g);
   else syrk_wave_sum<RUNS, false>(acc, p, k, k1, at, g);
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        part[wave][2 * a + b][q][lane] = floatx4{acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
-  __syncthreads();
-  const int wr = wave >> 1, wc = wave & 1;
-  floatx16 sum[1][1];
-  if (diag && wave == 2) {           // block (1, 0) of a diagonal tile is block (0, 1) transposed: element (r, c) is its (c, r)
-    const float* flat = reinterpret_cast<const float*>(&part[0][1][0][0]);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      // element (row l32, column 8 (r / 4) + 4 g + r % 4) of block (0, 1): quad l32 / 8, lane 32 (l32 / 4 % 2) + column, entry l32 % 4
-      const int at01 = ((l32 >> 3) * 64 + 32 * ((l32 >> 2) & 1) + 8 * (r >> 2) + 4 * g + (r & 3)) * 4 + (l32 & 3);
-      sum[0][0][r] = (flat[at01] + flat[at01 + 4096]) + (flat[at01 + 8192] + flat[at01 + 12288]);
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const floatx4 v = (part[0][wave][q][lane] + part[1][wave][q][lane]) + (part[2][wave][q][lane] + part[3][wave][q][lane]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum[0][0][4 * q + e] = v[e];
-    }
-  }
-  if (p.nsplit == 1) syrk_epilogue<1, 1>(sum, p.C, p.ldc, p.d, i0 + 32 * wr, j0 + 32 * wc, diag, p.alpha, p.beta, lane);
-  else store_partial<1, 1>(sum, p.ws + static_cast<size_t>(id) * 4096, tid);
+  syrk_wave_finish(acc, part, p, id, i0, j0, diag);
 }
 
 // The same result with the staged kernels' order of sums (AK_F32_IN_ORDER): their splits of K, one accumulator over each of

@@ -1469,3 +1469,20 @@ def test_grouped_half_pieces_in_tall_tiles_have_the_same_bits(K, transA, transB)
             alone = run([i])[0][i]
         assert torch.equal(together[i], alone)
         assert float(largest[i]) == float(alone.abs().max())
+
+
+@pytest.mark.parametrize("N,C,H,W,kernel,stride,padding", [
+    (1, 20, 3, 3, (3, 3), (1, 1), (1, 1)), (3, 64, 9, 7, (3, 3), (2, 2), (1, 1)), (2, 33, 5, 12, (3, 2), (1, 2), (0, 1)), (5, 12, 16, 16, (5, 5), (1, 1), (2, 2)),
+    (70, 40, 9, 9, (3, 3), (2, 1), (1, 1)), (4, 65, 7, 7, (1, 1), (2, 2), (0, 0)), (9, 129, 5, 5, (1, 1), (1, 1), (0, 0)), (2, 30, 4, 4, (4, 8), (3, 1), (2, 4)),
+    (300, 24, 6, 6, (3, 3), (2, 2), (1, 1)), (2, 18, 70, 65, (3, 3), (1, 1), (1, 1)), (2, 10, 6, 6, (6, 6), (1, 1), (0, 0))])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_fp32_windows_straight_to_the_matrix_instruction(K, N, C, H, W, kernel, stride, padding, beta):
+    # (the last window has more than the 32 taps of a mask: the staged kernel)
+    memory = torch.full((N * C * H * W + 256,), float("nan"))
+    memory[128:-128] = _inputs((N * C * H * W,), torch.float32, N + C + H)
+    x = memory[128:-128].view(N, C, H, W)
+    rows = nn.functional.unfold(x.double(), kernel, 1, padding, stride).permute(0, 2, 1).reshape(-1, C * kernel[0] * kernel[1])
+    d = rows.shape[1]
+    out = torch.ones(d, d).cuda()
+    K.conv_syrk(memory.cuda()[128:-128].view(N, C, H, W), kernel, stride, padding, out=out, alpha=0.5, beta=beta)
+    assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
