@@ -1486,3 +1486,28 @@ def test_fp32_windows_straight_to_the_matrix_instruction(K, N, C, H, W, kernel, 
     out = torch.ones(d, d).cuda()
     K.conv_syrk(memory.cuda()[128:-128].view(N, C, H, W), kernel, stride, padding, out=out, alpha=0.5, beta=beta)
     assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
+
+
+@pytest.mark.parametrize("N,C,H,W", [(82, 64, 5, 5), (64, 128, 6, 6), (3, 256, 27, 29), (100, 192, 5, 5), (9, 512, 15, 17), (2050, 64, 1, 1)])
+def test_fp32_correlations_on_two_fp16_planes(K, N, C, H, W):
+    """2048 pixels and more: channels scaled by powers of two of their own, from 1e-17 to 1e17, one of them zero."""
+    g = torch.Generator().manual_seed(N + C)
+    x = torch.randn(N, C, H, W, generator=g).relu() * torch.exp(torch.linspace(-39, 39, C)[torch.randperm(C, generator=g)])[None, :, None, None]
+    x[:, 5] = 0
+    x[:, 7, 0, 0] *= 1e-3
+    rows = nn.functional.unfold(x.double(), 3, 1, 1, 1).permute(0, 2, 1).reshape(-1, 9 * C)
+    ref = rows.T @ rows
+    xg = x.cuda()
+    out = K.conv_syrk(xg, (3, 3), (1, 1), (1, 1))
+    # every entry against the norms of its two channels (sums over all pixels, from which the border's are taken away): 22 bits of
+    # each factor, and the accumulation
+    scale = x.double().pow(2).sum(dim=(0, 2, 3)).sqrt().clamp_min(1e-30).repeat_interleave(9)
+    assert float(((out.double().cpu() - ref) / scale / scale[:, None]).abs().max()) < 4e-6
+    assert torch.equal(out, out.T)
+    # a channel that is not finite spoils its own entries only
+    bad = xg.clone()
+    bad[0, 3, 0, 0], bad[1, 9, 0, 0] = float("inf"), float("nan")
+    spoiled = K.conv_syrk(bad, (3, 3), (1, 1), (1, 1)).view(C, 9, C, 9)
+    keep = [c for c in range(C) if c not in (3, 9)]
+    assert torch.equal(spoiled[keep][:, :, keep], out.view(C, 9, C, 9)[keep][:, :, keep])
+    assert not bool(torch.isfinite(spoiled[3, 4, 3, 4])) and bool(torch.isnan(spoiled[9, 4, 9, 4]))
