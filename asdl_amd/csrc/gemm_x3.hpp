@@ -419,19 +419,21 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
   const bool lower_only = (p.tile_mode == TILE_LOWER) || (mirror && ti == tj);
   if (p.beta != 0.f) {
     // all loads of C first: interleaved with the stores they would wait for one another (the compiler cannot tell
-    // that the rows differ), one memory latency per element
+    // that the rows differ), one memory latency per element; and none under a lane's own condition, which is waited for by
+    // itself.  Elements beyond the matrix, or above the diagonal where only the lower ones are written, are not stored.
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const int gj = j0 + 64 * wc + 32 * b + l32;
+        const int gj = min(j0 + 64 * wc + 32 * b + l32, p.N - 1);
+        float c[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int gi = i0 + 64 * wr + 32 * a + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          float c = 0.f;
-          if (gj < p.N && gi < p.M && !(lower_only && gi < gj)) c = C[static_cast<int64_t>(gi) * p.ldc + gj];
-          acc[a][b][r] = p.alpha * acc[a][b][r] + p.beta * c;
+          const int gi = min(i0 + 64 * wr + 32 * a + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), p.M - 1);
+          c[r] = C[static_cast<int64_t>(gi) * p.ldc + gj];
         }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][b][r] = p.alpha * acc[a][b][r] + p.beta * c[r];
       }
   } else {
 #pragma unroll
