@@ -1,5 +1,7 @@
 // fp32 product tile for products that leave most of the device idle: true fp32 products (v_mfma_f32_32x32x2_f32), small
 // tiles, deep k-chunks.  Included by gemm_f32.hpp; same interface (GemmParams).
+// (Most products take gemm_wave.hpp, without the LDS; this form stays for short contractions over more tiles than CUs, A B^T
+// over many tiles, the inverses' small products and those of the low-rank inverses.)
 //
 // A product of a few hundred rows is bound by memory latency, not by the matrix pipes: with k-tiles of 16 or 32 and one
 // of them in flight, every k-tile waits for the L2 or the device memory once (about a microsecond when the operands were
