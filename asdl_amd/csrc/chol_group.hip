@@ -247,7 +247,7 @@ __device__ __forceinline__ void cg_decode_tile(const CgProd& d, int local, int& 
 }
 
 // One work group per 128 x 128 tile of any product of the step; tile_map[w] = the product of work group w.
-static __global__ __launch_bounds__(256) void cg_prod_kernel(CgArgs a, const CgProd* __restrict__ prods,
+static __global__ __launch_bounds__(256, 2) void cg_prod_kernel(CgArgs a, const CgProd* __restrict__ prods,
                                                              const int32_t* __restrict__ tile_map) {
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 3 * X3_PLANE];
   const int w = blockIdx.x;
@@ -275,7 +275,8 @@ static __global__ __launch_bounds__(256) void cg_prod_kernel(CgArgs a, const CgP
     p.scaleA = sc[(d.flags >> 4) & 3];
     p.scaleB = sc[(d.flags >> 6) & 3];
     p.alpha = d.alpha / (p.scaleA * p.scaleB);      // powers of two: exact
-    gemm_x3_tile<2, false, 1, 1, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
+    if (d.beta != 0.f) gemm_x3_tile<2, false, 1, 1, true, false, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
+    else gemm_x3_tile<2, false, 1, 1, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
   } else {
     gemm_x3_tile<3, false, 1, 1>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
   }
