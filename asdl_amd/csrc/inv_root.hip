@@ -190,7 +190,10 @@ struct LanczosGroups {
 // rows of S are requested before that, their first 1024 columns kept in registers.
 // Bound by the launch and the chain of loads and reductions for small n, by reading S for a full batch.
 // WIDE: vectors that the LDS does not hold (kLanczosLdsDim) are formed again, element by element, where they are used.
-template <bool WIDE>
+// HELD: at most 1024 columns, and work groups that wait rather than fill the memory: the three vectors come into registers and are
+// requested first (loads return in order), then the rows of S, none under a lane's own condition, which would be waited for by
+// itself.  784 and 512 columns: 7.4 -> 6.0 us a step; 98 matrices of up to 3072 columns, bound by reading S, lose 7 % by it.
+template <bool WIDE, bool HELD>
 static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, LanczosGroups L, int j) {
   extern __shared__ __attribute__((aligned(16))) float q[];
   __shared__ float red[3][4];
@@ -204,28 +207,60 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
   const int z = g.z0 + zl, tid = threadIdx.x, lane = tid & 63, row0 = part * kLanczosRows + 4 * (tid >> 6);
   const float* __restrict__ S = g.S + zl * g.strideS;
   const int n4 = n & ~3;
-  floatx4 early[4][4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = 4 * lane + 256 * c, row = row0 + r < n ? row0 + r : n - 1;
-      early[c][r] = k < n4 ? *reinterpret_cast<const floatx4u*>(S + static_cast<int64_t>(row) * n + k) : floatx4{0.f, 0.f, 0.f, 0.f};
-    }
   const int64_t vec = static_cast<int64_t>(g.batch) * n;
   float* __restrict__ qj = g.vec + (j % 3) * vec + static_cast<int64_t>(zl) * n;
   const float* __restrict__ v0 = g.v0 + static_cast<int64_t>(zl) * n;
   const float* __restrict__ q1 = g.vec + ((j + 2) % 3) * vec + static_cast<int64_t>(zl) * n;
   const float* __restrict__ q2 = g.vec + ((j + 1) % 3) * vec + static_cast<int64_t>(zl) * n;
   const float* __restrict__ w = g.vec + (3 + ((j + 1) & 1)) * vec + static_cast<int64_t>(zl) * n;
+  float hw[4], h1[4], h2[4];
+  floatx4 early[4][4];
+  if constexpr (HELD) {
+    const float* __restrict__ first = j == 0 ? v0 : w;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {      // (elements beyond the end read the last one and are not used)
+      const int i = min(tid + 256 * u, n - 1);
+      hw[u] = first[i];
+      h1[u] = q1[i];
+      h2[u] = q2[i];
+    }
+    if (n4 > 0) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = min(4 * lane + 256 * c, n4 - 4), row = row0 + r < n ? row0 + r : n - 1;
+          early[c][r] = *reinterpret_cast<const floatx4u*>(S + static_cast<int64_t>(row) * n + k);
+        }
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = 4 * lane + 256 * c, row = row0 + r < n ? row0 + r : n - 1;
+        early[c][r] = k < n4 ? *reinterpret_cast<const floatx4u*>(S + static_cast<int64_t>(row) * n + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
   float a = 0.f, b = 0.f, inv = 0.f;
   auto raw = [&](int i) { return j == 0 ? v0[i] : w[i] - a * q1[i] - (j > 1 ? b * q2[i] : 0.f); };     // q_j without its scale
   auto form = [&](float* sums) {                      // the vector (WIDE: nothing) and its length
     float s = 0.f;
-    for (int i = tid; i < n; i += 256) {
-      const float x = raw(i);
-      if constexpr (!WIDE) q[i] = x;
-      s += x * x;
+    if constexpr (HELD) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = tid + 256 * u;
+        if (i >= n) break;
+        const float x = j == 0 ? hw[u] : hw[u] - a * h1[u] - (j > 1 ? b * h2[u] : 0.f);
+        q[i] = x;
+        s += x * x;
+      }
+    } else {
+      for (int i = tid; i < n; i += 256) {
+        const float x = raw(i);
+        if constexpr (!WIDE) q[i] = x;
+        s += x * x;
+      }
     }
     return sqrtf(block_sum(s, sums));
   };
@@ -252,7 +287,13 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     if (j > 1 && st.lz_dim[z] != 0) return;            // an invariant subspace: T is complete
     b = st.beta[z * kLanczosSteps + j - 1];
     float s = 0.f;
-    for (int i = tid; i < n; i += 256) s += w[i] * q1[i];
+    if constexpr (HELD) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (tid + 256 * u < n) s += hw[u] * h1[u];
+    } else {
+      for (int i = tid; i < n; i += 256) s += w[i] * q1[i];
+    }
     a = block_sum(s, red[0]);
     const float norm = form(red[1]);
     const bool done = !(norm > 1e-7f * fabsf(a));
@@ -1066,18 +1107,19 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
       blocks += g.batch * ((g.n + kLanczosRows - 1) / kLanczosRows);
       widest = std::max(widest, g.n);
     }
-    const bool wide = widest > kLanczosLdsDim;
+    const bool wide = widest > kLanczosLdsDim, held = widest <= 1024 && blocks <= 512;       // (two work groups a CU)
     const size_t lds = static_cast<size_t>(widest) * sizeof(float);
     static bool attr_set = false;     // idempotent; a race sets it twice at worst
     if (!wide && lds > 60 * 1024 && !attr_set) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_lanczos_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(root_lanczos_kernel<false, false>), hipFuncAttributeMaxDynamicSharedMemorySize,
                               kLanczosLdsDim * static_cast<int>(sizeof(float))) != hipSuccess)
         return AK_ERR_LAUNCH;
       attr_set = true;
     }
     for (int j = 0; j < steps; ++j) {
-      if (wide) hipLaunchKernelGGL(root_lanczos_kernel<true>, dim3(blocks), b256, 0, s, G.st, L, j);
-      else hipLaunchKernelGGL(root_lanczos_kernel<false>, dim3(blocks), b256, lds, s, G.st, L, j);
+      if (wide) hipLaunchKernelGGL((root_lanczos_kernel<true, false>), dim3(blocks), b256, 0, s, G.st, L, j);
+      else if (held) hipLaunchKernelGGL((root_lanczos_kernel<false, true>), dim3(blocks), b256, lds, s, G.st, L, j);
+      else hipLaunchKernelGGL((root_lanczos_kernel<false, false>), dim3(blocks), b256, lds, s, G.st, L, j);
     }
     hipLaunchKernelGGL(root_power_kernel, gz, b64, 0, s, G, steps, power_tol, max_power_iter);
     hipLaunchKernelGGL(root_ridge_kernel, gc, b256, 0, s, G, ridge_eps);
