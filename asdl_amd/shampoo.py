@@ -109,6 +109,8 @@ HALF_PIECE_STATISTICS = True      # the grouped statistics on two fp16 pieces pe
                                   # 0.3-1 %; one accumulator for the whole sum: 2-3 % at 2304 columns and up, 10 % at 768)
 HALF_PIECE_PRECONDITION = True     # grouped preconditioning on two fp16 pieces per element (kernels.KronPrecondPlan does the same)
 GROUPED_PRECONDITION = True      # matrix-shaped parameters: all their preconditioning products in two launches
+SMALL_PRECONDITION_ELEMENTS = 1 << 22     # of all matrices; beyond it the split products win (2000^3 172 us a product on fp32 tiles, 2048^3
+                                  # 85 split) and no workspace is taken to find that out
 GROUPED_STATISTIC_MIN_DIM = 768   # statistics of this size and up go into one grouped launch (with GROUPED_PRECONDITION)
 
 
@@ -298,7 +300,7 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
         (784-512-512-10: seven launches, 132 us, before; two, 39 us, now; the rule of ak_kron_precond_deep, which takes these
         products for Kronecker factors too).  The roots are symmetric.  Returns the parameters that are left."""
         small = [pc for pc in self.preconditioners if self._groupable(pc, align=1)] if GROUPED_PRECONDITION else []
-        if not small:
+        if not small or sum(pc.param.numel() for pc in small) > SMALL_PRECONDITION_ELEMENTS:
             return list(self.preconditioners)
         items = []
         for pc in small:
