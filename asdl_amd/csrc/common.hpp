@@ -21,11 +21,6 @@ constexpr int kWave = 64;
 __device__ __forceinline__ floatx16 mfma_bf16(bf16x8 a, bf16x8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
-// The same on fp16 values (passed as the 16-bit patterns they are).
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ floatx16 mfma_f16(bf16x8 a, bf16x8 b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 // v_mfma_f32_32x32x2_f32: lane l feeds A[i = l%32][k = l/32] and B[k = l/32][j = l%32];
 // same accumulator layout.
 __device__ __forceinline__ floatx16 mfma_f32(float a, float b, floatx16 c) {
@@ -300,7 +295,7 @@ size_t conv_corr_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, in
 int conv_corr_syrk(const void* x, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph,
                    int pw, float alpha, float beta, float* A, int64_t lda, void* ws, size_t ws_bytes, hipStream_t stream);
 
-// The same for an fp32 NCHW input: split into fp16 or bf16 planes first (products at the accuracy of fp32).
+// The same for an fp32 NCHW input: split into three bf16 planes first (products at the accuracy of fp32).
 size_t conv_corr_f32_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw);
 int conv_corr_syrk_f32(const float* x, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph,
                        int pw, float alpha, float beta, float* A, int64_t lda, void* ws, size_t ws_bytes,

@@ -34,7 +34,6 @@
 
 namespace ak {
 
-
 constexpr int kCorrProds = 9;          // main, 2 image rows, 2 image columns, 4 corners
 constexpr int kCorrShifts = 13;
 constexpr int kCorrPieces = 29;        // [C, C] pieces of the reduced matrix: 13 shifts, 2 x 3 rows, 2 x 3 columns, 4 corners
@@ -46,8 +45,8 @@ struct CorrProd {
   int32_t Ho, Wo, kw, KK, pw;          // virtual convolution (stride 1, no padding above)
   uint32_t mWo, mHo, mKw, mBlk;
   // Tiles: the row tap's C columns from tile ti0 on, `ntaps` column taps of C columns each from tile tj0 on.  With
-  // an input of two fp16 planes (C = 2 c channels, [hi | lo]) or three bf16 planes (C = 3 c) that are whole tiles, only
-  // the three or six plane pairs that matter are computed: npairs, ppt = c / BT tiles per plane; else npairs = 1, ppt = C / BT.
+  // an input of three bf16 planes (C = 3 c channels, [hi | mid | lo]) whose planes are whole tiles, only the six plane
+  // pairs that matter are computed: npairs = 6, ppt = c / BT tiles per plane; else npairs = 1, ppt = C / BT.
   int32_t ti0, tj0, ntaps, ppt, npairs, tpt;    // tpt: tiles per tap in the column direction (C / BT)
   int32_t kt_split, nsplit;            // k-tiles per row split, splits
   int32_t first_item, first_tile;      // running counts over the products
@@ -78,8 +77,8 @@ __device__ __forceinline__ void corr_tile_of(const CorrProd& cp, int t, int& ti,
   const int pair = t / per_pair, rem = t - pair * per_pair;
   const int tap = rem / (cp.ppt * cp.ppt), r2 = rem - tap * cp.ppt * cp.ppt;
   const int ii = r2 / cp.ppt, jj = r2 - ii * cp.ppt;
-  // plane pairs in the order (0,0) (0,1) (1,0) of two planes, (0,0) (0,1) (1,0) (0,2) (2,0) (1,1) of three
-  const int pi = pair == 2 || pair == 5 ? 1 : (pair == 4 ? 2 : 0), pj = pair == 1 || pair == 5 ? 1 : (pair == 3 ? 2 : 0);
+  // plane pairs in the order (0,0) (0,1) (0,2) (1,0) (1,1) (2,0): hi = 0, mid = 1, lo = 2, sum of the two <= 2
+  const int pi = pair < 3 ? 0 : (pair < 5 ? 1 : 2), pj = pair < 3 ? pair : (pair < 5 ? pair - 3 : 0);
   row = pi * cp.ppt + ii;
   col = tap * cp.tpt + pj * cp.ppt + jj;
   ti = cp.ti0 + row;
@@ -89,7 +88,7 @@ __device__ __forceinline__ void corr_tile_of(const CorrProd& cp, int t, int& ti,
 __device__ __forceinline__ int corr_ntiles(const CorrProd& cp) { return cp.npairs * cp.ntaps * cp.ppt * cp.ppt; }
 
 // One work group per (product, row split, tile).
-template <int WR, int WC, int FR, int FC, bool F16>
+template <int WR, int WC, int FR, int FC>
 __device__ __forceinline__ void corr_products_tile(const CorrArgs& a, uint32_t wg, uint32_t nwg) {
   constexpr int BT = DtlCfg<WR, WC, FR, FC, true>::BT;
   const int w = static_cast<int>(xcd_contiguous_id(wg, nwg));
@@ -115,12 +114,12 @@ __device__ __forceinline__ void corr_products_tile(const CorrArgs& a, uint32_t w
   if (cp.nsplit == 1) {
     // the only split: the tile goes straight into the reduced matrix
     const int64_t ld = static_cast<int64_t>(kCorrPieces) * a.Cin;
-    dtl_tile<WR, WC, FR, FC, true, F16>(p, ti, tj, k_begin, rows, nullptr,
-                                        a.red + cp.out_off + static_cast<int64_t>(row) * BT * ld + static_cast<int64_t>(col) * BT, ld);
+    dtl_tile<WR, WC, FR, FC, true>(p, ti, tj, k_begin, rows, nullptr,
+                                   a.red + cp.out_off + static_cast<int64_t>(row) * BT * ld + static_cast<int64_t>(col) * BT, ld);
     return;
   }
   floatx4* partial = a.part + cp.part_off + static_cast<int64_t>(local) * (BT * BT / 4);
-  dtl_tile<WR, WC, FR, FC, true, F16>(p, ti, tj, k_begin, rows, partial);
+  dtl_tile<WR, WC, FR, FC, true>(p, ti, tj, k_begin, rows, partial);
 }
 
 // Sums the partial tiles of the row splits (fixed order) into the product's columns of ONE row-major matrix
@@ -142,11 +141,12 @@ __device__ __forceinline__ void corr_reduce_tile(const CorrArgs& a, int tile, in
   const int64_t stride = ntiles * tile_f4;
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   int s = 0;
-  for (; s + 8 <= cp.nsplit; s += 8) {                 // eight loads in flight, summed in pairs: 39 roundings in a row show
+  for (; s + 8 <= cp.nsplit; s += 8) {                 // eight loads in flight, summed in order
     floatx4 w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = src[(s + k) * stride];
-    acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc += w[k];
   }
   for (; s < cp.nsplit; ++s) acc += src[s * stride];
   const int ld = kCorrPieces * a.Cin;
@@ -158,9 +158,9 @@ __device__ __forceinline__ void corr_reduce_tile(const CorrArgs& a, int tile, in
 }
 
 // All products of one layer in one launch: one work group per (product, row split, tile).
-template <int WR, int WC, int FR, int FC, bool F16>
+template <int WR, int WC, int FR, int FC>
 __global__ __launch_bounds__(WR * WC * 64) void corr_products_kernel(CorrArgs a) {
-  corr_products_tile<WR, WC, FR, FC, F16>(a, blockIdx.x, gridDim.x);
+  corr_products_tile<WR, WC, FR, FC>(a, blockIdx.x, gridDim.x);
 }
 
 // grid (tiles of all products, 4 * FR * FC): one work group per float4 slot of every thread's accumulators.
@@ -264,65 +264,25 @@ __global__ __launch_bounds__(kAsmThreads) void corr_assemble_kernel(CorrAsm a) {
   }
 }
 
-// ---- fp32 inputs: two fp16 or three bf16 planes -----------------------------------------------------------------
-// An fp32 NCHW input takes the same path on the fp16 matrix cores at the accuracy of fp32 products: channel c, times
-// the power of two that brings its largest magnitude into (2^13, 2^14], is split into two fp16 pieces, hi = the value
-// rounded to the nearest, lo = the remainder rounded (22 significant bits together; fp16 denormals are taken as they
-// are), written as a channels-last tensor with 2 C channels, [hi | lo] per pixel.  The products above then run on that
-// tensor as they are (2 C channels), and before the assembly the 2 x 2 blocks of every [2 C, 2 C] piece are folded
-// into [C, C] and scaled back, exactly:  x^T y ~= hi^T hi' + (hi^T lo' + lo^T hi'); lo^T lo' is below 2^-22 of the
-// product.  Against three bf16 planes (six products of the nine blocks) half the matrix work, two thirds of the bytes
-// and planes of 64 channels that fit one 128-wide tile with both: ResNet-18 on 128 x 3 x 32 x 32, factors of the
-// 3 x 3 / 1 layers of 64,
-// 128, 256 and 512 channels 254, 179, 188 and 251 -> 144, 114, 118 and 157 us each, errors against 64 bits 1.2, 1.5, 1.5
-// and 2.1e-7 -> 1.0, 1.0, 0.9 and 1.4e-7 (ReLU outputs): fewer roundings of the accumulators.
-//
-// Below kCorrMinPixels the 22 bits show (8 x 128 x 4 x 4: 1.2e-7 against 0.8e-7; from 2048 pixels on the accumulation's own
-// error is the larger one), and the element is split exactly into three bf16 pieces, x = hi + mid + lo (each the remainder
-// rounded; the third needs no rounding): 3 C channels, the blocks hi hi' + (hi mid' + mid hi') + (hi lo' + lo hi') + mid mid',
-// the three dropped ones below 2^-24 of the product.  The pairs are added in an order that keeps a symmetric piece
-// symmetric to the last bit.
+// ---- fp32 inputs: three bf16 planes ------------------------------------------------------------------------------
+// An fp32 NCHW input takes the same path on the bf16 matrix cores at the accuracy of fp32 products: every element
+// is split exactly into three bf16 pieces, x = hi + mid + lo (each the remainder rounded to the nearest bf16; the
+// third needs no rounding), written as a channels-last tensor with 3 C channels, [hi | mid | lo] per pixel.  The
+// products above then run on that tensor as they are (3 C channels), and before the assembly the 3 x 3 blocks of
+// every [3 C, 3 C] piece are folded into [C, C]:  x^T y ~= hi^T hi' + (hi^T mid' + mid^T hi') + (hi^T lo' + lo^T hi')
+// + mid^T mid'; the three dropped blocks are below 2^-24 of the product.  The pairs are added in this order so that
+// the fold of a symmetric piece is symmetric to the last bit.
+// Two fp16 planes of channels scaled by powers of two would need half the matrix work (128 x 64 x 32 x 32, 128 x 16 x 16,
+// 256 x 8 x 8, 512 x 4 x 4 channels and pixels: 142, 114, 118, 158 us instead of 254, 179, 188, 251), but hold 22 of the 24 bits:
+// single products are off by up to 4e-7 instead of 1.2e-7, the factor of zero-mean 100 x 64 x 14 x 14 by 1.4e-7 instead of 1.2e-7.
 
-constexpr int kCorrSlices = 8;       // of the samples, for the ranges of the channels
-
-// range[slice][C]: the largest finite magnitude of a channel in a slice of the samples.  2^log_run threads take one sample's
-// channel, 256 of them several samples at once where an image is small.
-__global__ __launch_bounds__(256) void corr_range_kernel(const float* __restrict__ x, float* __restrict__ range, int N, int C, int HW,
-                                                         int log_run) {
-  const int c = blockIdx.x, slice = blockIdx.y;
-  const int n0 = static_cast<int>(static_cast<int64_t>(N) * slice / kCorrSlices),
-            n1 = static_cast<int>(static_cast<int64_t>(N) * (slice + 1) / kCorrSlices);
-  const int run = 1 << log_run, p0 = threadIdx.x & (run - 1), step = 256 >> log_run;
-  float m = 0.f;
-  for (int n = n0 + (threadIdx.x >> log_run); n < n1; n += step) {
-    const float* __restrict__ src = x + (static_cast<int64_t>(n) * C + c) * HW;
-#pragma unroll 4
-    for (int p = p0; p < HW; p += run) {
-      const float v = fabsf(src[p]);
-      m = v > m && v < 3.4e38f ? v : m;
-    }
-  }
-  __shared__ float part[4];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) range[slice * C + c] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-}
-
-// x: [N, C, HW] fp32 (HW contiguous) -> planes: [N, HW, 2 C] fp16 and the exponents e[c] that undo the scaling, or
-// [N, HW, 3 C] bf16.  One
-// work group per (sample, 32 pixels, 32 channels): coalesced 128-byte reads along the pixels, 64-byte runs of channels
-// per pixel and plane on the way out.
-template <int PLANES>
-__global__ __launch_bounds__(256) void corr_split_nchw_kernel(const float* __restrict__ x, const float* __restrict__ range,
-                                                              uint16_t* __restrict__ planes, int* __restrict__ exponent, int C, int HW) {
+// x: [N, C, HW] fp32 (HW contiguous) -> planes: [N, HW, 3 C] bf16.  One work group per (sample, 32 pixels, 32
+// channels): coalesced 128-byte reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
+__global__ __launch_bounds__(256) void corr_split_nchw_kernel(const float* __restrict__ x, uint16_t* __restrict__ planes,
+                                                              int C, int HW) {
   __shared__ float tile[32][33];
-  __shared__ float largest[kCorrSlices][32];
   const int n = blockIdx.z, p0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;          // 32 x 8
-  static_assert(kCorrSlices == 8, "one slice per eighth of a work group");
-  if constexpr (PLANES == 2) largest[ty][tx] = range[ty * C + c0 + tx];
   const float* src = x + (static_cast<int64_t>(n) * C + c0) * HW + p0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -330,57 +290,32 @@ __global__ __launch_bounds__(256) void corr_split_nchw_kernel(const float* __res
     tile[c][tx] = p0 + tx < HW ? src[static_cast<int64_t>(c) * HW + tx] : 0.f;
   }
   __syncthreads();
-  float scale = 1.f;
-  if constexpr (PLANES == 2) {
-    float m = 0.f;
-#pragma unroll
-    for (int q = 0; q < kCorrSlices; ++q) m = fmaxf(m, largest[q][tx]);
-    int e = 0;
-    if (m > 0.f) frexpf(m, &e);                        // m <= 2^e
-    e = max(e - 14, -120);                             // (2^120 is the largest scale: what it leaves below 2^13 squares to nothing)
-    if (blockIdx.x == 0 && n == 0 && ty == 0) exponent[c0 + tx] = e;
-    scale = ldexpf(1.f, -e);
-  }
-  uint16_t* dst = planes + (static_cast<int64_t>(n) * HW + p0) * (PLANES * C) + c0;
+  uint16_t* dst = planes + (static_cast<int64_t>(n) * HW + p0) * (3 * C) + c0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int px = ty + 8 * r;
     if (p0 + px >= HW) continue;
-    const float v = tile[tx][px] * scale;
-    uint16_t* q = dst + static_cast<int64_t>(px) * (PLANES * C) + tx;
-    if constexpr (PLANES == 2) {
-      const _Float16 hi = static_cast<_Float16>(v), lo = static_cast<_Float16>(v - static_cast<float>(hi));
-      q[0] = __builtin_bit_cast(uint16_t, hi);
-      q[C] = __builtin_bit_cast(uint16_t, lo);
-    } else {
-      const __bf16 hi = static_cast<__bf16>(v);
-      const float r1 = v - static_cast<float>(hi);
-      const __bf16 mid = static_cast<__bf16>(r1), lo = static_cast<__bf16>(r1 - static_cast<float>(mid));
-      q[0] = __builtin_bit_cast(uint16_t, hi);
-      q[C] = __builtin_bit_cast(uint16_t, mid);
-      q[2 * C] = __builtin_bit_cast(uint16_t, lo);
-    }
+    const float v = tile[tx][px];
+    const __bf16 hi = static_cast<__bf16>(v);
+    const float r1 = v - static_cast<float>(hi);
+    const __bf16 mid = static_cast<__bf16>(r1);
+    const __bf16 lo = static_cast<__bf16>(r1 - static_cast<float>(mid));
+    uint16_t* q = dst + static_cast<int64_t>(px) * (3 * C) + tx;
+    q[0] = __builtin_bit_cast(uint16_t, hi);
+    q[C] = __builtin_bit_cast(uint16_t, mid);
+    q[2 * C] = __builtin_bit_cast(uint16_t, lo);
   }
 }
 
-// wide: [PLANES C][29 * PLANES C] (pieces of PLANES C columns) -> red: [C][29 * C].  four: the block lo lo' of two planes is
-// there as well (planes that share a tile).  grid (29 C / 256, C).
-template <int PLANES>
-__global__ __launch_bounds__(256) void corr_fold_kernel(const float* __restrict__ wide, const int* __restrict__ exponent,
-                                                        float* __restrict__ red, int C, int four) {
+// red3: [3 C][29 * 3 C] (pieces of 3 C columns) -> red: [C][29 * C].  grid (29 C / 256, C).
+__global__ __launch_bounds__(256) void corr_fold_kernel(const float* __restrict__ red3, float* __restrict__ red, int C) {
   const int col = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
   if (col >= kCorrPieces * C) return;
   const int pc = col / C, c2 = col - pc * C;
-  const int64_t ld = static_cast<int64_t>(kCorrPieces) * PLANES * C;
-  auto at = [&](int p, int q) { return wide[static_cast<int64_t>(p * C + c) * ld + pc * PLANES * C + q * C + c2]; };
-  float v;
-  if constexpr (PLANES == 2) {
-    v = ldexpf((at(0, 0) + (at(0, 1) + at(1, 0))) + (four ? at(1, 1) : 0.f), exponent[c] + exponent[c2]);
-  } else {
-    const float hh = at(0, 0), hm = at(0, 1) + at(1, 0), hl = at(0, 2) + at(2, 0), mm = at(1, 1);
-    v = ((hh + hm) + hl) + mm;
-  }
-  red[static_cast<int64_t>(c) * (kCorrPieces * C) + col] = v;
+  const int64_t ld3 = static_cast<int64_t>(kCorrPieces) * 3 * C;
+  auto at = [&](int p, int q) { return red3[static_cast<int64_t>(p * C + c) * ld3 + pc * 3 * C + q * C + c2]; };
+  const float hh = at(0, 0), hm = at(0, 1) + at(1, 0), hl = at(0, 2) + at(2, 0), mm = at(1, 1);
+  red[static_cast<int64_t>(c) * (kCorrPieces * C) + col] = ((hh + hm) + hl) + mm;
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------
@@ -419,14 +354,14 @@ static bool corr_eligible(int64_t N, int64_t C, int64_t H, int64_t W, int kh, in
   return true;
 }
 
-// planes: 1, or 2 / 3 when the C channels are the two fp16 / three bf16 planes of C / planes channels
+// planes: 1, or 3 when the C channels are the three bf16 planes of C / 3 channels
 static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int planes) {
   CorrPlan pl{};
   const int bt = corr_tile_width(C);
   pl.bt = bt;
   const int cb = static_cast<int>(C / bt);
   // the unneeded plane pairs can be left out when every plane is a whole number of tiles
-  const bool pairs = planes > 1 && (C / planes) % bt == 0;
+  const bool pairs = planes == 3 && (C / 3) % bt == 0;
   const int occ = bt == 64 ? 4 : (bt == 128 ? 2 : 1);      // work groups per CU
   const int64_t slots = 256 * occ;
   CorrArgs& a = pl.args;
@@ -444,8 +379,8 @@ static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int 
     p.mBlk = make_magic(static_cast<uint32_t>(C) * p.KK);
     p.ti0 = ti0; p.tj0 = tj0; p.ntaps = ntaps;
     p.tpt = cb;
-    p.npairs = !pairs ? 1 : (planes == 2 ? 3 : 6);
-    p.ppt = pairs ? cb / planes : cb;
+    p.npairs = pairs ? 6 : 1;
+    p.ppt = pairs ? cb / 3 : cb;
   };
   const int64_t px = C * 2;                      // bytes per pixel
   fill(0, 0, N * H * W, H, W, 3, 5, 2, 2 * cb, 2 * cb, kCorrShifts);
@@ -497,9 +432,7 @@ static CorrPlan corr_plan(int64_t N, int64_t C, int64_t H, int64_t W, int planes
     int64_t N, C, H, W;
     bool operator==(const Key& o) const { return N == o.N && C == o.C && H == o.H && W == o.W; }
   };
-  // the kinds of plan for one shape are several cache entries
-  H = planes == 2 ? -H : H;
-  W = planes == 3 ? -W : W;
+  H = planes == 3 ? -H : H;      // the two kinds of plan for one shape are two cache entries
   struct Hash {
     size_t operator()(const Key& k) const {
       uint64_t h = 0x9e3779b97f4a7c15ull;
@@ -516,7 +449,7 @@ static CorrPlan corr_plan(int64_t N, int64_t C, int64_t H, int64_t W, int planes
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   if (cache.size() > 1024) cache.clear();
-  const CorrPlan plan = corr_plan_build(N, C, H < 0 ? -H : H, W < 0 ? -W : W, planes);
+  const CorrPlan plan = corr_plan_build(N, C, H < 0 ? -H : H, W, planes);
   cache.emplace(key, plan);
   return plan;
 }
@@ -527,10 +460,10 @@ static size_t corr_ws_layout(const CorrPlan& pl, size_t& red_at) {
   return red_at + pl.red_floats * sizeof(float);
 }
 
-template <bool F16, int WR, int WC, int FR, int FC>
+template <int WR, int WC, int FR, int FC>
 static int corr_launch_cfg(const CorrPlan& pl, const CorrArgs& args, hipStream_t stream) {
   using Cfg = DtlCfg<WR, WC, FR, FC, true>;
-  auto kern = corr_products_kernel<WR, WC, FR, FC, F16>;
+  auto kern = corr_products_kernel<WR, WC, FR, FC>;
   if (Cfg::LDS_BYTES > 64 * 1024) {
     static bool attr_set = false;     // idempotent; a race sets it twice at worst
     if (!attr_set) {
@@ -552,18 +485,17 @@ size_t conv_corr_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, in
   return corr_ws_layout(corr_plan(N, C, H, W), red_at);
 }
 
-// All products of the layer on the channels-last bf16 (F16: fp16) tensor x (C channels), reduced into red [C][29 C].
-template <bool F16>
+// All products of the layer on the channels-last bf16 tensor x (C channels), reduced into red [C][29 C].
 static int corr_products(const CorrPlan& plan, const void* x, floatx4* part, float* red, hipStream_t stream) {
   CorrPlan pl = plan;
   CorrArgs& args = pl.args;
   for (int i = 0; i < kCorrProds; ++i) args.prod[i].X = static_cast<const unsigned char*>(x) + pl.x_off[i];
   args.part = part;
   args.red = red;
-  if (pl.bt == 64) return corr_launch_cfg<F16, 2, 2, 1, 1>(pl, args, stream);
-  if (pl.bt == 128) return corr_launch_cfg<F16, 2, 2, 2, 2>(pl, args, stream);
-  if (pl.bt == 192) return corr_launch_cfg<F16, 2, 2, 3, 3>(pl, args, stream);
-  return corr_launch_cfg<F16, 2, 4, 4, 2>(pl, args, stream);
+  if (pl.bt == 64) return corr_launch_cfg<2, 2, 1, 1>(pl, args, stream);
+  if (pl.bt == 128) return corr_launch_cfg<2, 2, 2, 2>(pl, args, stream);
+  if (pl.bt == 192) return corr_launch_cfg<2, 2, 3, 3>(pl, args, stream);
+  return corr_launch_cfg<2, 4, 4, 2>(pl, args, stream);
 }
 
 static int corr_assemble(const float* red, int64_t C, float alpha, float beta, float* A, int64_t lda, hipStream_t stream) {
@@ -596,73 +528,46 @@ int conv_corr_syrk(const void* x, int64_t N, int64_t C, int64_t H, int64_t W, in
   const size_t need = corr_ws_layout(pl, red_at);
   if (ws == nullptr || ws_bytes < need) return AK_ERR_WORKSPACE;
   float* red = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + red_at);
-  const int rc = corr_products<false>(pl, x, static_cast<floatx4*>(ws), red, stream);
+  const int rc = corr_products(pl, x, static_cast<floatx4*>(ws), red, stream);
   if (rc != AK_OK) return rc;
   return corr_assemble(red, C, alpha, beta, A, lda, stream);
 }
 
-// fp32 NCHW input: [planes: N H W P C of 16 bits][workspace of the P C-channel products, its reduced matrix last]
-// [red: C x 29 C][ranges: slices x C][exponents: C]
-static size_t corr_f32_layout(int64_t N, int64_t C, int64_t H, int64_t W, int P, const CorrPlan& plP, size_t& wsP_at,
-                              size_t& redP_in_wsP, size_t& red_at) {
-  const size_t planes = static_cast<size_t>(N) * H * W * P * C * 2;
-  wsP_at = (planes + 255) & ~static_cast<size_t>(255);
-  const size_t wsP = corr_ws_layout(plP, redP_in_wsP);
-  red_at = (wsP_at + wsP + 255) & ~static_cast<size_t>(255);
-  return red_at + (static_cast<size_t>(C) * kCorrPieces * C + (kCorrSlices + 1) * static_cast<size_t>(C)) * sizeof(float);
-}
-
-constexpr int64_t kCorrMinPixels = 2048;       // (above: fp32 inputs)
-
-// Planes of an fp32 input, 0: not for this form.
-static int corr_f32_planes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
-  if (C % 64 != 0) return 0;
-  const int P = N * H * W >= kCorrMinPixels ? 2 : 3;
-  return corr_eligible(N, P * C, H, W, kh, kw, sh, sw, ph, pw) ? P : 0;
+// fp32 NCHW input: [planes: N H W 3C bf16][workspace of the 3 C-channel products, its reduced matrix last][red: C x 29 C]
+static size_t corr_f32_layout(int64_t N, int64_t C, int64_t H, int64_t W, const CorrPlan& pl3, size_t& ws3_at,
+                              size_t& red3_in_ws3, size_t& red_at) {
+  const size_t planes = static_cast<size_t>(N) * H * W * 3 * C * 2;
+  ws3_at = (planes + 255) & ~static_cast<size_t>(255);
+  const size_t ws3 = corr_ws_layout(pl3, red3_in_ws3);
+  red_at = (ws3_at + ws3 + 255) & ~static_cast<size_t>(255);
+  return red_at + static_cast<size_t>(C) * kCorrPieces * C * sizeof(float);
 }
 
 size_t conv_corr_f32_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
-  const int P = corr_f32_planes(N, C, H, W, kh, kw, sh, sw, ph, pw);
-  if (P == 0) return 0;
+  if (C % 64 != 0 || !corr_eligible(N, 3 * C, H, W, kh, kw, sh, sw, ph, pw)) return 0;
   size_t a, b, c;
-  return corr_f32_layout(N, C, H, W, P, corr_plan(N, P * C, H, W, P), a, b, c);
+  return corr_f32_layout(N, C, H, W, corr_plan(N, 3 * C, H, W, 3), a, b, c);
 }
 
 int conv_corr_syrk_f32(const float* x, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph,
                        int pw, float alpha, float beta, float* A, int64_t lda, void* ws, size_t ws_bytes,
                        hipStream_t stream) {
-  const int P = corr_f32_planes(N, C, H, W, kh, kw, sh, sw, ph, pw);
-  if (P == 0) return AK_ERR_UNSUPPORTED;
-  const CorrPlan plP = corr_plan(N, P * C, H, W, P);
-  size_t wsP_at, redP_in_wsP, red_at;
-  const size_t need = corr_f32_layout(N, C, H, W, P, plP, wsP_at, redP_in_wsP, red_at);
+  if (C % 64 != 0 || !corr_eligible(N, 3 * C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;
+  const CorrPlan pl3 = corr_plan(N, 3 * C, H, W, 3);
+  size_t ws3_at, red3_in_ws3, red_at;
+  const size_t need = corr_f32_layout(N, C, H, W, pl3, ws3_at, red3_in_ws3, red_at);
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255) != 0) return AK_ERR_WORKSPACE;
   unsigned char* base = static_cast<unsigned char*>(ws);
   uint16_t* planes = reinterpret_cast<uint16_t*>(base);
+  const int HW = static_cast<int>(H * W);
+  hipLaunchKernelGGL(corr_split_nchw_kernel, dim3((HW + 31) / 32, static_cast<unsigned>(C / 32), static_cast<unsigned>(N)),
+                     dim3(256), 0, stream, x, planes, static_cast<int>(C), HW);
+  float* red3 = reinterpret_cast<float*>(base + ws3_at + red3_in_ws3);
+  const int rc = corr_products(pl3, planes, reinterpret_cast<floatx4*>(base + ws3_at), red3, stream);
+  if (rc != AK_OK) return rc;
   float* red = reinterpret_cast<float*>(base + red_at);
-  float* range = red + static_cast<size_t>(C) * kCorrPieces * C;
-  int* exponent = reinterpret_cast<int*>(range + kCorrSlices * C);
-  float* wide = reinterpret_cast<float*>(base + wsP_at + redP_in_wsP);
-  floatx4* part = reinterpret_cast<floatx4*>(base + wsP_at);
-  const int HW = static_cast<int>(H * W), c32 = static_cast<int>(C);
-  const dim3 split_grid((HW + 31) / 32, static_cast<unsigned>(C / 32), static_cast<unsigned>(N));
-  const dim3 fold_grid(static_cast<unsigned>((kCorrPieces * C + 255) / 256), static_cast<unsigned>(C));
-  if (P == 2) {
-    int log_run = 4;
-    while (log_run < 8 && (1 << log_run) < HW) ++log_run;
-    hipLaunchKernelGGL(corr_range_kernel, dim3(static_cast<unsigned>(C), kCorrSlices), dim3(256), 0, stream, x, range,
-                       static_cast<int>(N), c32, HW, log_run);
-    hipLaunchKernelGGL(corr_split_nchw_kernel<2>, split_grid, dim3(256), 0, stream, x, range, planes, exponent, c32, HW);
-    const int rc = corr_products<true>(plP, planes, part, wide, stream);
-    if (rc != AK_OK) return rc;
-    hipLaunchKernelGGL(corr_fold_kernel<2>, fold_grid, dim3(256), 0, stream, wide, exponent, red, c32,
-                       plP.args.prod[0].npairs == 1 ? 1 : 0);
-  } else {
-    hipLaunchKernelGGL(corr_split_nchw_kernel<3>, split_grid, dim3(256), 0, stream, x, range, planes, exponent, c32, HW);
-    const int rc = corr_products<false>(plP, planes, part, wide, stream);
-    if (rc != AK_OK) return rc;
-    hipLaunchKernelGGL(corr_fold_kernel<3>, fold_grid, dim3(256), 0, stream, wide, exponent, red, c32, 0);
-  }
+  hipLaunchKernelGGL(corr_fold_kernel, dim3(static_cast<unsigned>((kCorrPieces * C + 255) / 256), static_cast<unsigned>(C)),
+                     dim3(256), 0, stream, red3, red, static_cast<int>(C));
   return corr_assemble(red, C, alpha, beta, A, lda, stream);
 }
 

@@ -614,7 +614,7 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   }
   if (dtype == AK_F32_AS_BF16) return AK_ERR_UNSUPPORTED;      // rounding on the fly is the window kernel's
   if (dtype == AK_F32) {
-    // 3 x 3, stride 1, padding 1: shifted correlations of two fp16 (few pixels: three bf16) planes of the input
+    // 3 x 3, stride 1, padding 1: shifted correlations of three bf16 planes of the input
     const int rc = ak::conv_corr_syrk_f32(static_cast<const float*>(x), N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, A,
                                           lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
     if (rc != AK_ERR_UNSUPPORTED) return rc;

@@ -173,8 +173,7 @@ struct DtlCfg {
 // Rows [k_begin, k_begin + rows) of the operand into tile (ti, tj) of one factor.  partial == nullptr: the result is
 // the factor's tile (alpha, beta, mirror image); otherwise the accumulators go to `partial` in accumulator order,
 // [(a, b, q)][thread] float4, for a reduction pass.  raw != nullptr: the bare tile goes to a row-major matrix.
-// F16: the operand holds fp16 values.
-template <int WR, int WC, int FR, int FC, bool GATHER, bool F16 = false>
+template <int WR, int WC, int FR, int FC, bool GATHER>
 __device__ __forceinline__ void dtl_tile(const DtlParams& p, int ti, int tj, int64_t k_begin, int rows,
                                          floatx4* __restrict__ partial, float* __restrict__ raw = nullptr,
                                          int64_t raw_ld = 0) {
@@ -302,8 +301,7 @@ __device__ __forceinline__ void dtl_tile(const DtlParams& p, int ti, int tj, int
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
       const int a = m / FC, b = m % FC;
-      if constexpr (F16) acc[a][b] = mfma_f16(ca[a], cb[b], acc[a][b]);
-      else acc[a][b] = mfma_bf16(ca[a], cb[b], acc[a][b]);
+      acc[a][b] = mfma_bf16(ca[a], cb[b], acc[a][b]);
 #pragma unroll
       for (int sidx = (m * NS) / NM; sidx < ((m + 1) * NS) / NM; ++sidx) {
         __builtin_amdgcn_sched_barrier(0);

@@ -1489,7 +1489,7 @@ def test_fp32_windows_straight_to_the_matrix_instruction(K, N, C, H, W, kernel, 
 
 
 @pytest.mark.parametrize("N,C,H,W", [(82, 64, 5, 5), (64, 128, 6, 6), (3, 256, 27, 29), (100, 192, 5, 5), (9, 512, 15, 17), (2050, 64, 1, 1)])
-def test_fp32_correlations_on_two_fp16_planes(K, N, C, H, W):
+def test_fp32_correlations_of_channels_of_any_scale(K, N, C, H, W):
     """2048 pixels and more: channels scaled by powers of two of their own, from 1e-17 to 1e17, one of them zero."""
     g = torch.Generator().manual_seed(N + C)
     x = torch.randn(N, C, H, W, generator=g).relu() * torch.exp(torch.linspace(-39, 39, C)[torch.randperm(C, generator=g)])[None, :, None, None]
@@ -1499,8 +1499,8 @@ def test_fp32_correlations_on_two_fp16_planes(K, N, C, H, W):
     ref = rows.T @ rows
     xg = x.cuda()
     out = K.conv_syrk(xg, (3, 3), (1, 1), (1, 1))
-    # every entry against the norms of its two channels (sums over all pixels, from which the border's are taken away): 22 bits of
-    # each factor, and the accumulation
+    # every entry against the norms of its two channels (sums over all pixels, from which the border's are taken away): the
+    # accumulation of up to 2050 terms in chunks
     scale = x.double().pow(2).sum(dim=(0, 2, 3)).sqrt().clamp_min(1e-30).repeat_interleave(9)
     assert float(((out.double().cpu() - ref) / scale / scale[:, None]).abs().max()) < 4e-6
     assert torch.equal(out, out.T)
@@ -1511,3 +1511,16 @@ def test_fp32_correlations_on_two_fp16_planes(K, N, C, H, W):
     keep = [c for c in range(C) if c not in (3, 9)]
     assert torch.equal(spoiled[keep][:, :, keep], out.view(C, 9, C, 9)[keep][:, :, keep])
     assert not bool(torch.isfinite(spoiled[3, 4, 3, 4])) and bool(torch.isnan(spoiled[9, 4, 9, 4]))
+
+
+@pytest.mark.parametrize("N,C,H,W", [(82, 64, 5, 5), (64, 128, 6, 6), (40, 256, 8, 8), (128, 64, 32, 32)])
+def test_fp32_correlations_hold_all_24_bits(K, N, C, H, W):
+    """One pixel that is not zero: every entry is one product of two operands with all 24 bits of their significands in
+    use, so that nothing but the product's own roundings (the sum of its pieces, two at 2^-24) may show."""
+    g = torch.Generator().manual_seed(C)
+    x = torch.zeros(N, C, H, W)
+    units = 2 * torch.randint(1024, 2048, (C,), generator=g) + 1        # odd, beyond what 11 + 11 bits hold
+    x[N // 2, :, H // 2, W // 2] = (1 + units * 2.0 ** -23) * (2 * torch.randint(0, 2, (C,), generator=g) - 1)
+    rows = nn.functional.unfold(x.double(), 3, 1, 1, 1).permute(0, 2, 1).reshape(-1, 9 * C)
+    out = K.conv_syrk(x.cuda(), (3, 3), (1, 1), (1, 1))
+    assert float((out.double().cpu() - rows.T @ rows).abs().max()) <= 2.0 ** -23
