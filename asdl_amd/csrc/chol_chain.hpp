@@ -1,4 +1,4 @@
-// Damped inverses of groups that are too large for the block sweep (chol_sweep.hpp): the same elimination, with all but the
+// Damped inverses of groups that are too large for the block sweep (chol_sweep.hpp; cg_build): the same elimination, with all but the
 // columns of the current group of CG_GROUP blocks left to one product of that depth.  Included by chol_group.hip.
 //
 // The sweep's step k updates the whole triangle by v v^T of 128 columns (v_i = Y_i M_k^T): beyond one round of tiles on the

@@ -4,7 +4,7 @@
 // L^-T L^-1 together (d^3 FLOP, as POTRF + POTRI), in one of two forms:
 //   chol_sweep.hpp   every step updates the whole triangle: one launch per 128 columns, for groups whose tiles fit the device
 //   chol_chain.hpp   the steps update the block columns that the next steps need, one product per 512 columns the rest
-// The plan takes the one with the shorter estimate.  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
+// The plan takes the chain where it saves enough (cg_build).  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
 // as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: below the error of
 // LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half was at 3-8 times that).
 //
@@ -407,19 +407,26 @@ static bool cg_dims_ok(const int64_t* dims, int count) {
   return true;
 }
 
-// The sweep: per step the leaf's work group, or as many waves of tiles as the device needs (one work group per CU).
-static double cg_sweep_us(const int64_t* dims, int count) {
-  int64_t nb_max = 0;
+// The sweep: per step the leaf's work group, or the rounds of tiles that the device needs (one work group per CU); rounds: of all
+// steps, of which so many are filled.  Estimated and measured, us: 3072 864 and 868, 6 x 1700 811 and 800, 20 x 1142 712 and 710, 64 x 630 412 and 438,
+// 4 x 2400 with 8 x 512 1216 and 1230.
+static double cg_sweep_us(const int64_t* dims, int count, int64_t& rounds, double& filled) {
+  int64_t nb_max = 0, all = 0;
   for (int m = 0; m < count; ++m) nb_max = std::max<int64_t>(nb_max, (dims[m] + LEAF - 1) / LEAF);
   double us = 14;
+  rounds = 0;
   for (int64_t k = 0; k < nb_max; ++k) {
     int64_t groups = 0;
     for (int m = 0; m < count; ++m) {
       const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
       if (nb > k) groups += nb * (nb + 1) / 2 + (nb > k + 1 ? 1 : 0);
     }
-    us += std::max(22.0, 18.0 * static_cast<double>((groups + 255) / 256));
+    const int64_t r = (groups + 255) / 256;
+    us += std::max(22.0, 14.0 * static_cast<double>(r) + 6.0 * static_cast<double>(groups) / 256);
+    rounds += r;
+    all += groups;
   }
+  filled = static_cast<double>(all) / 256;
   return us;
 }
 
@@ -612,20 +619,29 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
   return us;
 }
 
-// The sweep where its estimate is shorter: while its tiles fit the device once or twice (22 us a step, 18 for each further round:
-// 2304 456 us, 3 x 2048 598), beyond that its updates of the whole triangle cost more than the chain's steps and products (3073: 900 us by
-// the chain; the sweep's two rounds 950).  The bound of 4096 tiles keeps the tables of hopeless cases from being built.
+// The sweep holds more: its sums are 128 long and its operands have all their bits, the chain's products sum 512 and take two
+// fp16 pieces (22 bits).  Error against 64 bits of the inverses, sweep and chain: ReLU rows of rank d / 8, a / lam = 2^12, 3072 4.8e-3 and
+// 1.4e-2, 6 x 1700 2.7e-3 and 6.1e-3; full rank 3072 2.8e-7 and 3.8e-7.  (Three bf16 pieces in the chain's products: 1.7e-2, more
+// roundings.)  It takes half the memory, too (3072: 23 and 51 MB).  So the chain is for groups whose steps take three rounds of tiles
+// and more, and of matrices of 15 block columns and more whose third round is used (the 2.3) it has to save a quarter: up to there
+// the sweep served when it was as slow as fp32 products make it, so that no size has lost accuracy since.  Measured, sweep and
+// chain, us: two rounds 3072 868 and 846, 2600 with 2304, 2048, 1500, 700, 600 1030 and 930; three and more 4 x 2048 855 and 652,
+// 3 x 2304 886 and 704, 4 x 2400 with 8 x 512 1230 and 880, 60 x 513 373 and 346.  The bound of 4096 tiles keeps the tables of
+// hopeless cases from being built.
 static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
-  int64_t tiles = 0;
+  int64_t tiles = 0, nb_max = 0, rounds;
   for (int m = 0; m < count; ++m) {
     const int64_t nb = (dims[m] + LEAF - 1) / LEAF;
+    nb_max = std::max(nb_max, nb);
     tiles += nb * (nb + 1) / 2;
   }
-  const double sweep_us = cg_sweep_us(dims, count);
-  bool sweep = CG_FORCE == 1;
+  double filled;
+  const double sweep_us = cg_sweep_us(dims, count, rounds, filled);
+  bool sweep = CG_FORCE == 1 || (CG_FORCE == 0 && tiles <= 4096 && rounds < 3 * nb_max);
   if (!sweep) {
     const double us = cg_build_chain(dims, count, plan);
-    sweep = CG_FORCE < 2 && tiles <= 4096 && sweep_us < us;
+    const double worth = nb_max >= 15 && filled >= 2.3 * static_cast<double>(nb_max) ? 0.73 : 0.92;
+    sweep = CG_FORCE == 0 && tiles <= 4096 && us >= worth * sweep_us;
   }
   if (!sweep) return;
   plan = CgPlan();

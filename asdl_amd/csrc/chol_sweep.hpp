@@ -1,5 +1,5 @@
 // Damped inverses of many small and medium matrices by a block sweep: one launch per 128 columns.  Included by
-// chol_group.hip, whose plan picks between this and the chain of chol_chain.hpp by their estimated times.
+// chol_group.hip, whose plan leaves groups of three rounds of tiles a step and more to the chain of chol_chain.hpp where that saves enough (cg_build).
 //
 // In-place block Gauss-Jordan elimination on the Cholesky factors.  With M_k = L_kk^-1 of the updated diagonal block,
 // step k is ONE symmetric rank-128 update of the whole lower triangle,

@@ -101,6 +101,22 @@ def test_plan_of_the_grouped_inverse_says_how_long_it_takes():
     assert lib.ak_chol_group_plan_us(ctypes.create_string_buffer(256)) < 0
 
 
+@pytest.mark.parametrize('dims', [(2817,), (2944,), (3072,), (3073,), (3500,), (2600, 2304, 2048, 1500, 700, 600), (2892, 2892, 1400, 700, 300, 200),
+                                  (1601, 2836, 542, 176, 670, 81, 44, 19)])
+def test_inverses_that_the_sweep_can_take_stay_with_its_accuracy(dims):
+    """One launch per block of 128 columns: the block sweep, whose sums round least (the chain's errors on rank-deficient factors are
+    two to three times larger), and whose workspace is the tiles of the triangles and two columns of them."""
+    import ctypes
+    from asdl_amd import _lib
+    lib = _lib.load()
+    arr = (ctypes.c_int64 * len(dims))(*dims)
+    plan = ctypes.create_string_buffer(lib.ak_chol_group_plan_bytes(arr, len(dims)))
+    assert lib.ak_chol_group_plan(arr, len(dims), plan, len(plan)) == 0
+    blocks = [(d + 127) // 128 for d in dims]
+    assert lib.ak_chol_group_plan_launches(plan) == max(blocks) + 1
+    assert lib.ak_chol_group_ws_bytes(arr, len(dims)) == 4 * 128 * 128 * sum(n * (n + 1) // 2 + 2 * n + 2 for n in blocks)
+
+
 def test_small_module_preconditioning_leaves_sizes_beyond_its_own_to_the_other_paths():
     """The row matrices of the swift variant have inverses of more than 32768 columns.  The two-launch form declines them, before it
     launches anything, instead of refusing the call."""

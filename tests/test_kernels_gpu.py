@@ -626,10 +626,10 @@ def test_chol_inv_at_the_edges_of_the_leaf_tiles(K, d):
             assert int(call([B.cuda()], [out], lam_dev).cpu()) == bad, (call.__name__, bad)
 
 
-@pytest.mark.parametrize('dims', [(127, 255, 2), (129, 257, 1), (383, 384, 385), (1151, 513, 640, 10), (2049, 127), (2700, 2700)])
+@pytest.mark.parametrize('dims', [(127, 255, 2), (129, 257, 1), (383, 384, 385), (1151, 513, 640, 10), (2049, 127), (2700, 2700), (3073,)])
 def test_chol_inv_grouped_block_sweep_edges(K, dims):
     """Groups of matrices that end just before, at and behind a block of 128 columns and leave the sweep at different
-    steps; the last two need more tiles than the device has CUs.  Against fp64, full-rank and rank-deficient."""
+    steps; the last three need more tiles than the device has CUs.  Against fp64, full-rank and rank-deficient."""
     for rank in (2, 1 / 8):
         mats = [_spd(d, 900 + i, rows=max(1, int(rank * d))) for i, d in enumerate(dims)]
         lam = [0.05 * float(m.diagonal().max()) for m in mats]
@@ -644,7 +644,7 @@ def test_chol_inv_grouped_block_sweep_edges(K, dims):
 
 # The chain: groups that end after one, two, three and four blocks and inside one, tiles in the step's launch and (many rows) in
 # launches of their own, one matrix and many of other sizes beside it; a skipped matrix and one that is not positive definite.
-@pytest.mark.parametrize('dims', [(3073,), (4097, 130, 5), (3500, 2900, 2561), (1100,) * 24 + (3,), (1537,) * 12 + (300,), (641,) * 40, (513,) * 60])
+@pytest.mark.parametrize('dims', [(4225,), (4097, 130, 5), (3500, 2900, 2561), (1100,) * 24 + (3,), (1537,) * 12 + (300,), (641,) * 40, (513,) * 60])
 def test_chol_inv_grouped_chain(K, dims):
     plan = K.chol_group_plan(list(dims))
     assert plan.launches != max((d + 127) // 128 for d in dims) + 1, 'the block sweep: one launch per block column'
