@@ -195,7 +195,8 @@ __device__ __forceinline__ void add_partial(floatx16 (&acc)[TI][TJ], const float
 //   SL > 1: grid (upper tiles, TI*TJ*16), a work group takes one wave's share of a slot in SL slices of the splits, each
 //           with its loads in flight, and adds the slices through the LDS.  A result of one tile has as many splits as
 //           the device has places, and few work groups to add them: 64 x 64, 256 splits 64 -> 4.5 us, 128 x 128 32 -> 4 us.
-template <int TI, int TJ, int SL>
+//   ORDERED: the slices only load, eight splits each at a time, and the first one adds them one after the other: the bits of SL = 1.
+template <int TI, int TJ, int SL, bool ORDERED = false>
 __global__ __launch_bounds__(SL == 1 ? 256 : 64 * SL) void syrk_finalize_kernel(const float* __restrict__ ws, int nsplit, int T,
                                                                                 float* __restrict__ C, int64_t ldc, int64_t d,
                                                                                 float alpha, float beta) {
@@ -214,12 +215,30 @@ __global__ __launch_bounds__(SL == 1 ? 256 : 64 * SL) void syrk_finalize_kernel(
   const floatx4* src = reinterpret_cast<const floatx4*>(ws) + (static_cast<size_t>(blockIdx.x) * (BT * BT / 4)) +
                        slot * 256 + tid;
   const size_t split_stride = static_cast<size_t>(ntiles) * (BT * BT / 4);
+  if constexpr (ORDERED) {
+    __shared__ floatx4 batch[8 * SL][64];
+    for (int s0 = 0; s0 < nsplit; s0 += 8 * SL) {
+      floatx4 w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = src[min(s0 + 8 * slice + j, nsplit - 1) * split_stride];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) batch[8 * slice + j][lane] = w[j];
+      __syncthreads();
+      if (slice == 0) {
+        const int n = min(8 * SL, nsplit - s0);
+        for (int j = 0; j < n; ++j) acc += batch[j][lane];
+      }
+      __syncthreads();
+    }
+    if (slice != 0) return;
+  } else {
 #pragma unroll 8
-  for (int s = slice; s < nsplit; s += SL) {
-    const floatx4 w = src[s * split_stride];
-    acc[0] += w[0]; acc[1] += w[1]; acc[2] += w[2]; acc[3] += w[3];
+    for (int s = slice; s < nsplit; s += SL) {
+      const floatx4 w = src[s * split_stride];
+      acc[0] += w[0]; acc[1] += w[1]; acc[2] += w[2]; acc[3] += w[3];
+    }
   }
-  if constexpr (SL > 1) {
+  if constexpr (SL > 1 && !ORDERED) {
     __shared__ floatx4 part[SL][64];
     part[slice][lane] = acc;
     __syncthreads();
@@ -251,13 +270,17 @@ __global__ __launch_bounds__(SL == 1 ? 256 : 64 * SL) void syrk_finalize_kernel(
 }
 
 // Up to 4 splits the slices would be idle (36 tiles in 15 splits: 32 -> 7 us with 4 slices); from 64 on 16 slices have loads to overlap.
+// in_order: the splits one after the other, whatever their number (AK_F32_IN_ORDER).
 template <int TI>
 inline void launch_syrk_finalize(const float* ws, int nsplit, int64_t ntiles, int T, float* C, int64_t ldc, int64_t d,
-                                 float alpha, float beta, hipStream_t stream) {
+                                 float alpha, float beta, hipStream_t stream, bool in_order = false) {
   const unsigned tiles = static_cast<unsigned>(ntiles);
   if (nsplit <= 4)
     hipLaunchKernelGGL((syrk_finalize_kernel<TI, TI, 1>), dim3(tiles, 4 * TI * TI), dim3(256), 0, stream, ws, nsplit, T, C, ldc, d,
                        alpha, beta);
+  else if (in_order)
+    hipLaunchKernelGGL((syrk_finalize_kernel<TI, TI, 4, true>), dim3(tiles, 16 * TI * TI), dim3(256), 0, stream, ws, nsplit, T, C, ldc,
+                       d, alpha, beta);
   else if (nsplit < 64)
     hipLaunchKernelGGL((syrk_finalize_kernel<TI, TI, 4>), dim3(tiles, 16 * TI * TI), dim3(256), 0, stream, ws, nsplit, T, C, ldc, d,
                        alpha, beta);

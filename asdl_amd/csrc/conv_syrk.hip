@@ -557,7 +557,7 @@ static bool make_plan(ConvPlan& plan, int esize, int64_t N, int64_t C, int64_t H
 }
 
 template <typename T, int TI>
-static int launch_conv_syrk_t(ConvPlan& plan, hipStream_t stream) {
+static int launch_conv_syrk_t(ConvPlan& plan, bool in_order, hipStream_t stream) {
   auto kern = conv_syrk_kernel<T, TI>;
   if (plan.lds_bytes > 64 * 1024) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -568,13 +568,13 @@ static int launch_conv_syrk_t(ConvPlan& plan, hipStream_t stream) {
   hipLaunchKernelGGL(kern, grid, dim3(256), plan.lds_bytes, stream, plan.p);
   if (plan.p.nsplit > 1)
     launch_syrk_finalize<TI>(static_cast<const float*>(plan.p.ws), plan.p.nsplit, plan.ntiles, plan.p.T, plan.p.A, plan.p.lda,
-                             plan.p.d, plan.p.alpha, plan.p.beta, stream);
+                             plan.p.d, plan.p.alpha, plan.p.beta, stream, in_order);
   return check_launch();
 }
 
 template <typename T>
-static int launch_conv_syrk(ConvPlan& plan, hipStream_t stream) {
-  return plan.BT == 64 ? launch_conv_syrk_t<T, 1>(plan, stream) : launch_conv_syrk_t<T, 2>(plan, stream);
+static int launch_conv_syrk(ConvPlan& plan, bool in_order, hipStream_t stream) {
+  return plan.BT == 64 ? launch_conv_syrk_t<T, 1>(plan, in_order, stream) : launch_conv_syrk_t<T, 2>(plan, in_order, stream);
 }
 
 }  // namespace ak
@@ -645,5 +645,5 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
   plan.p.x = x; plan.p.alpha = alpha; plan.p.beta = beta; plan.p.A = A; plan.p.lda = lda;
   plan.p.ws = static_cast<float*>(ws);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == AK_BF16 ? ak::launch_conv_syrk<uint16_t>(plan, s) : ak::launch_conv_syrk<float>(plan, s);
+  return dtype == AK_BF16 ? ak::launch_conv_syrk<uint16_t>(plan, false, s) : ak::launch_conv_syrk<float>(plan, in_order, s);
 }

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void syrk_tn_kernel(SyrkTnParams p) {
 
 template <typename T>
 static int launch_syrk_tn(const void* X, int64_t M, int64_t d, int64_t ldx, float alpha, float beta, float* C,
-                          int64_t ldc, void* ws, size_t ws_bytes, hipStream_t stream) {
+                          int64_t ldc, void* ws, size_t ws_bytes, bool in_order, hipStream_t stream) {
   constexpr int TI = 2, BT = 64 * TI, BK = TnCfg<T>::BK;
   const int64_t Tn = (d + BT - 1) / BT;
   const int64_t ntiles = Tn * (Tn + 1) / 2;
@@ -223,7 +223,8 @@ static int launch_syrk_tn(const void* X, int64_t M, int64_t d, int64_t ldx, floa
   }
   hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, stream, p);
   if (nsplit > 1)
-    launch_syrk_finalize<TI>(static_cast<const float*>(ws), nsplit, ntiles, static_cast<int>(Tn), C, ldc, d, alpha, beta, stream);
+    launch_syrk_finalize<TI>(static_cast<const float*>(ws), nsplit, ntiles, static_cast<int>(Tn), C, ldc, d, alpha, beta, stream,
+                             in_order);
   return check_launch();
 }
 
@@ -250,11 +251,12 @@ extern "C" int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_
     const int rc = ak::syrk_dtl_plain(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
     if (rc != AK_ERR_UNSUPPORTED && rc != AK_ERR_WORKSPACE) return rc;
   }
-  if (dtype == AK_BF16) return ak::launch_syrk_tn<uint16_t>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
+  if (dtype == AK_BF16) return ak::launch_syrk_tn<uint16_t>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, false, s);
   if (dtype == AK_F32 && ldx <= (1 << 24) && ak::syrk_wave_rows(d, M)) {
     const int rc = ak::launch_syrk_wave(static_cast<const float*>(X), d, M, ldx, 0, 0, alpha, beta, C, ldc, ws, ws_bytes, s);
     if (rc != AK_ERR_WORKSPACE) return rc;
   }
-  if (dtype == AK_F32 || dtype == AK_F32_IN_ORDER) return ak::launch_syrk_tn<float>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, s);
+  if (dtype == AK_F32 || dtype == AK_F32_IN_ORDER)
+    return ak::launch_syrk_tn<float>(X, M, d, ldx, alpha, beta, C, ldc, ws, ws_bytes, dtype == AK_F32_IN_ORDER, s);
   return AK_ERR_ARG;
 }

@@ -323,7 +323,7 @@ inline int launch_syrk_chain(const float* X, int64_t d, int64_t K, int64_t ld, b
   const dim3 grid(static_cast<unsigned>(tiles * nsplit));
   if (runs) hipLaunchKernelGGL(syrk_chain_kernel<true>, grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(syrk_chain_kernel<false>, grid, dim3(256), 0, stream, p);
-  if (nsplit > 1) launch_syrk_finalize<1>(p.ws, nsplit, tiles, p.T, C, ldc, d, alpha, beta, stream);
+  if (nsplit > 1) launch_syrk_finalize<1>(p.ws, nsplit, tiles, p.T, C, ldc, d, alpha, beta, stream, true);
   return check_launch();
 }
 

@@ -1413,6 +1413,21 @@ def test_fp32_statistics_in_a_fixed_order(K, d, k, beta):
         assert torch.equal(a, c) and relerr(a, 0.5 * rows @ rows.T + beta) < TOL_FACTOR_F32
 
 
+@pytest.mark.parametrize("d,k", [(64, 8192), (65, 2560), (300, 4096), (512, 3072), (30, 60000)])
+def test_fp32_statistics_in_a_fixed_order_add_their_splits_one_by_one(K, d, k):
+    """Nonzero columns 320 apart, farther than a split is long, with products that fp32 holds exactly: the result has the bits of their
+    sum from first to last, however many splits there are."""
+    g = torch.Generator().manual_seed(d)
+    x = torch.zeros(d, k)
+    cols = torch.arange(7, k, 320)
+    x[:, cols] = torch.randint(-2047, 2048, (d, len(cols)), generator=g) * torch.exp2(torch.randint(-6, 7, (1, len(cols)), generator=g).float())
+    ref = torch.zeros(d, d)
+    for c in cols:
+        ref += x[:, c, None] * x[None, :, c]
+    assert torch.equal(K.syrk_nt(x.cuda(), in_order=True).cpu(), ref)
+    assert torch.equal(K.syrk_tn(x.T.contiguous().cuda(), in_order=True).cpu(), ref)
+
+
 @pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (1, 65, 17), (65, 1, 200), (64, 64, 16), (63, 66, 15), (129, 33, 127), (2, 130, 128), (200, 129, 143),
                                     (577, 75, 300), (65, 64, 1153), (31, 700, 2049), (1100, 1100, 300)])
 @pytest.mark.parametrize("transA", [False, True])
