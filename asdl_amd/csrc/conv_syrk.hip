@@ -579,22 +579,35 @@ static int launch_conv_syrk(ConvPlan& plan, bool in_order, hipStream_t stream) {
 
 }  // namespace ak
 
-extern "C" size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw,
-                                        int ph, int pw) {
+// 1 x 1 windows of fp32 (not in order): the staged kernel fills its 128 x 128 tiles from 16-byte loads as well, but has too few of
+// them at every size that a user has (64 channels 128 x 32 x 32: 32 us, 17 here; 4096 channels 128 x 4 x 4: 874 and 401); never slower.
+static bool conv_wave_window(int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
+  return kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && (H * W) % 8 == 0 && H * W < (1 << 30) && C * H * W < (1ll << 30);
+}
+
+// A workspace that a kernel may use for its type (AK_F32_IN_ORDER: neither syrk_wave.hpp's nor syrk_window.hpp's).
+extern "C" size_t ak_conv_syrk_ws_bytes_of(int dtype, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw,
+                                           int ph, int pw) {
   if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || kh <= 0 || kw <= 0 || sh <= 0 || sw <= 0 || ph < 0 || pw < 0) return 0;
   const size_t patch = ak::conv_patch_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
   if (patch > 0) return patch;
-  ak::ConvPlan a, b;
-  size_t need = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
-  if (kh == 1 && kw == 1) need = std::max(need, ak::syrk_wave_ws_bytes(C, N * H * W));
-  {
+  size_t need = 0;
+  if (dtype != AK_BF16) need = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
+  if (dtype == AK_F32) {
+    if (conv_wave_window(C, H, W, kh, kw, sh, sw, ph, pw)) need = std::max(need, ak::syrk_wave_ws_bytes(C, N * H * W));
     const int64_t Ho = (H + 2 * ph - kh) / sh + 1, Wo = (W + 2 * pw - kw) / sw + 1;
     if (H + 2 * ph >= kh && W + 2 * pw >= kw && ak::syrk_window_faster(N, C, H, W, kh, kw, sh, sw, Ho, Wo))
       need = std::max(need, ak::syrk_window_ws_bytes(C * kh * kw, N * Ho * Wo));
   }
-  if (ak::make_plan(a, 2, N, C, H, W, kh, kw, sh, sw, ph, pw) && a.ws_need > need) need = a.ws_need;
-  if (ak::make_plan(b, 4, N, C, H, W, kh, kw, sh, sw, ph, pw) && b.ws_need > need) need = b.ws_need;
+  ak::ConvPlan staged;
+  if (ak::make_plan(staged, dtype == AK_BF16 ? 2 : 4, N, C, H, W, kh, kw, sh, sw, ph, pw)) need = std::max(need, staged.ws_need);
   return need;
+}
+
+extern "C" size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw,
+                                        int ph, int pw) {
+  return std::max(ak_conv_syrk_ws_bytes_of(AK_F32, N, C, H, W, kh, kw, sh, sw, ph, pw),
+                  ak_conv_syrk_ws_bytes_of(AK_BF16, N, C, H, W, kh, kw, sh, sw, ph, pw));
 }
 
 extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh,
@@ -619,10 +632,7 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
                                           lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
     if (rc != AK_ERR_UNSUPPORTED) return rc;
   }
-  // 1 x 1 windows: the staged kernel fills its 128 x 128 tiles from 16-byte loads as well, but has too few of them at every size
-  // that a user has (64 channels 128 x 32 x 32: 32 us, 17 here; 4096 channels 128 x 4 x 4: 874 and 401); never slower
-  if (dtype == AK_F32 && !in_order && kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && N > 0 && H * W > 0 && (H * W) % 8 == 0 &&
-      H * W < (1 << 30) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && C * H * W < (1ll << 30) && lda >= C) {
+  if (dtype == AK_F32 && !in_order && conv_wave_window(C, H, W, kh, kw, sh, sw, ph, pw) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && lda >= C) {
     const int rc = ak::launch_syrk_wave(static_cast<const float*>(x), C, N * H * W, H * W, C * H * W, static_cast<int>(H * W), alpha,
                                         beta, A, lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
     if (rc != AK_ERR_WORKSPACE) return rc;

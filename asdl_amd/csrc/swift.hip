@@ -282,7 +282,7 @@ static SmwLayout smw_layout(int64_t n, int64_t d) {
   l.y = off; off += align256(static_cast<size_t>(n) * d * sizeof(float));
   l.misc = off; off += 256;                                   // lam_n, two pointers
   l.chol = off; off += align256(ak_chol_inv_ws_bytes(n, 1));
-  l.syrk = off; off += align256(ak_conv_syrk_ws_bytes(1, n, 1, d, 1, 1, 1, 1, 0, 0));
+  l.syrk = off; off += align256(ak_conv_syrk_ws_bytes_of(AK_F32, 1, n, 1, d, 1, 1, 1, 1, 0, 0));
   l.total = off;
   return l;
 }

@@ -230,16 +230,20 @@ static int launch_syrk_tn(const void* X, int64_t M, int64_t d, int64_t ldx, floa
 
 }  // namespace ak
 
-extern "C" size_t ak_syrk_tn_ws_bytes(int64_t M, int64_t d) {
+// A workspace that a kernel may use for its type: fp32 rows on syrk_wave.hpp's only where its rule takes them.
+extern "C" size_t ak_syrk_tn_ws_bytes_of(int dtype, int64_t M, int64_t d) {
   if (M <= 0 || d <= 0) return 0;
   const int64_t Tn = (d + 127) / 128;
   const int64_t ntiles = Tn * (Tn + 1) / 2;
-  // upper bound over both dtypes (bf16 has the fewer k-steps, fp32 the more)
-  const int ns = ak::pick_nsplit(ntiles, (M + 15) / 16);
-  const size_t staged = ns > 1 ? static_cast<size_t>(ns) * ntiles * 128 * 128 * sizeof(float) : 0;
-  const size_t direct = d % 8 == 0 ? ak::syrk_dtl_plain_ws_bytes(M, d, d) : 0;
-  const size_t wave = ak::syrk_wave_ws_bytes(d, M);
-  return std::max(std::max(staged, direct), wave);
+  const int ns = ak::pick_nsplit(ntiles, (M + 15) / 16);      // (upper bound: bf16 has fewer k-steps)
+  size_t need = ns > 1 ? static_cast<size_t>(ns) * ntiles * 128 * 128 * sizeof(float) : 0;
+  if (dtype == AK_BF16 && d % 8 == 0) need = std::max(need, ak::syrk_dtl_plain_ws_bytes(M, d, d));
+  if (dtype == AK_F32 && ak::syrk_wave_rows(d, M)) need = std::max(need, ak::syrk_wave_ws_bytes(d, M));
+  return need;
+}
+
+extern "C" size_t ak_syrk_tn_ws_bytes(int64_t M, int64_t d) {
+  return std::max(ak_syrk_tn_ws_bytes_of(AK_F32, M, d), ak_syrk_tn_ws_bytes_of(AK_BF16, M, d));
 }
 
 extern "C" int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_t ldx, float alpha, float beta,

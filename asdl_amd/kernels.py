@@ -712,11 +712,13 @@ def syrk_tn(x, out=None, alpha=1.0, beta=0.0, round_bf16=False, in_order=False):
         if _group_take(row, flops, floor, x.data_ptr() & 15, x, out):
             return out
     lib = _lib.load()
-    need = _ws_need('ak_syrk_tn_ws_bytes', M, d)
+    code = _dtype_code(x)
+    if in_order and code == AK_F32:
+        code = AK_F32_IN_ORDER
+    need = _ws_need('ak_syrk_tn_ws_bytes_of', code, M, d)
     ws, ws_bytes, keep = _ws_args(need, x.device)
     with _Timed('syrk_tn', flops, floor=floor):
-        code = _dtype_code(x)
-        rc = lib.ak_syrk_tn(ctypes.c_void_p(x.data_ptr()), AK_F32_IN_ORDER if in_order and code == AK_F32 else code, M, d, ldx, alpha, beta,
+        rc = lib.ak_syrk_tn(ctypes.c_void_p(x.data_ptr()), code, M, d, ldx, alpha, beta,
                             ctypes.c_void_p(out.data_ptr()), out.stride(0), ws, ws_bytes, _stream())
     _lib.check(rc, 'ak_syrk_tn')
     return out
@@ -792,11 +794,12 @@ def conv_syrk(x, kernel_size, stride, padding, out=None, alpha=1.0, beta=0.0, ro
             DirectCall.note('conv_syrk', lib.ak_conv_syrk_nhwc, args, need, x, out, flops, floor)
             return out
     x = _contiguous(x)
-    need = _ws_need('ak_conv_syrk_ws_bytes', N, C, H, W, kh, kw, sh, sw, ph, pw)
+    if in_order and code == AK_F32:
+        code = AK_F32_IN_ORDER
+    need = _ws_need('ak_conv_syrk_ws_bytes_of', code, N, C, H, W, kh, kw, sh, sw, ph, pw)
     ws, ws_bytes, keep = _ws_args(need, x.device)
     with _Timed('conv_syrk', flops, floor=floor):
-        rc = lib.ak_conv_syrk(ctypes.c_void_p(x.data_ptr()), AK_F32_IN_ORDER if in_order and code == AK_F32 else code,
-                              N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, ctypes.c_void_p(out.data_ptr()), out.stride(0),
+        rc = lib.ak_conv_syrk(ctypes.c_void_p(x.data_ptr()), code, N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, ctypes.c_void_p(out.data_ptr()), out.stride(0),
                               ws, ws_bytes, _stream())
     if rc == AK_ERR_UNSUPPORTED and code == AK_F32_AS_BF16:     # a window too large for the LDS: cast, then the bf16 kernels
         return conv_syrk(_as_bf16(x), kernel_size, stride, padding, out=out, alpha=alpha, beta=beta)

@@ -64,7 +64,8 @@ const char* ak_error_string(int code);
  * `.mul_(cov_scale)` and `results[key] += value` passes (asdl/operations/operation.py:133-137,
  * 199-201, 264-266) and the EMA pre-scale Kron.mul_ (asdl/symmatrix.py:448-453), and the 2-D
  * statistic G^T G of Shampoo (asdl/precondition/shampoo.py:331-339). */
-size_t ak_syrk_tn_ws_bytes(int64_t M, int64_t d);
+size_t ak_syrk_tn_ws_bytes(int64_t M, int64_t d);                    /* enough for every dtype */
+size_t ak_syrk_tn_ws_bytes_of(int dtype, int64_t M, int64_t d);      /* for one */
 int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_t ldx,
                float alpha, float beta, float* C, int64_t ldc,
                void* ws, size_t ws_bytes, ak_stream_t stream);
@@ -79,6 +80,8 @@ int ak_syrk_tn(const void* X, int dtype, int64_t M, int64_t d, int64_t ldx,
  * [d, M] matrix (Shampoo's G G^T, asdl/precondition/shampoo.py:331-339). */
 size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W,
                              int kh, int kw, int sh, int sw, int ph, int pw);
+size_t ak_conv_syrk_ws_bytes_of(int dtype, int64_t N, int64_t C, int64_t H, int64_t W,
+                                int kh, int kw, int sh, int sw, int ph, int pw);
 int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int64_t H, int64_t W,
                  int kh, int kw, int sh, int sw, int ph, int pw,
                  float alpha, float beta, float* A, int64_t lda,

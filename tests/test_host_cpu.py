@@ -117,6 +117,23 @@ def test_inverses_that_the_sweep_can_take_stay_with_its_accuracy(dims):
     assert lib.ak_chol_group_ws_bytes(arr, len(dims)) == 4 * 128 * 128 * sum(n * (n + 1) // 2 + 2 * n + 2 for n in blocks)
 
 
+def test_factor_workspaces_are_for_kernels_that_may_run():
+    """fp32 rows beyond the wave kernel's rule, bf16 rows and statistics in a fixed order do not ask for its partial sums."""
+    from asdl_amd import _lib, kernels
+    lib = _lib.load()
+    f32, bf16, ordered = 0, 1, kernels.AK_F32_IN_ORDER
+    assert lib.ak_syrk_tn_ws_bytes_of(f32, 8192, 4096) == lib.ak_syrk_tn_ws_bytes_of(bf16, 8192, 4096) == lib.ak_syrk_tn_ws_bytes(8192, 4096) == 0
+    assert lib.ak_conv_syrk_ws_bytes_of(ordered, 1, 4096, 1, 16384, 1, 1, 1, 1, 0, 0) == 0
+    assert lib.ak_conv_syrk_ws_bytes_of(bf16, 1, 4096, 1, 16384, 1, 1, 1, 1, 0, 0) == 0
+    for M, d in ((128, 784), (1000, 1021), (70000, 40), (4096, 700), (3136, 2048)):       # the query for all types holds each
+        assert lib.ak_syrk_tn_ws_bytes(M, d) >= max(lib.ak_syrk_tn_ws_bytes_of(t, M, d) for t in (f32, bf16, ordered))
+        assert lib.ak_syrk_tn_ws_bytes_of(ordered, M, d) <= lib.ak_syrk_tn_ws_bytes_of(f32, M, d)
+    for conv in ((128, 64, 32, 32, 3, 3, 1, 1, 1, 1), (128, 64, 32, 32, 1, 1, 1, 1, 0, 0), (128, 256, 8, 8, 1, 1, 2, 2, 0, 0), (64, 48, 20, 20, 3, 3, 1, 1, 1, 1),
+                 (64, 3, 32, 32, 3, 3, 1, 1, 1, 1)):
+        each = [lib.ak_conv_syrk_ws_bytes_of(t, *conv) for t in (f32, bf16, ordered)]
+        assert lib.ak_conv_syrk_ws_bytes(*conv) >= max(each) > 0
+
+
 def test_small_module_preconditioning_leaves_sizes_beyond_its_own_to_the_other_paths():
     """The row matrices of the swift variant have inverses of more than 32768 columns.  The two-launch form declines them, before it
     launches anything, instead of refusing the call."""
