@@ -66,6 +66,7 @@ _SIGNATURES = {
     'ak_event_synchronize': (c_int, [c_ptr]),
     'ak_kron_finish': (c_int, [c_ptr, c_ptr, c_ptr, c_int, c_ptr, c_int, c_ptr, c_ptr]),
     'ak_kron_precond_deep_ws_bytes': (c_size, [c_ptr, c_int]),
+    'ak_kron_precond_deep_faster': (c_int, [c_ptr, c_int]),
     'ak_kron_precond_deep': (c_int, [c_ptr, c_int, c_ptr, c_int, c_f32, c_ptr, c_ptr, c_int, c_ptr, c_size, c_ptr]),
     'ak_smw_group_y_floats': (c_size, [c_i64, c_i64]),
     'ak_smw_group': (c_int, [c_ptr, c_int, c_int, c_ptr]),

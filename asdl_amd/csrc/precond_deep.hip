@@ -115,28 +115,13 @@ static __global__ __launch_bounds__(64 * GEMM_WAVES, 2) void kp_second_kernel(Kp
 
 static int64_t kp_tiles(int64_t dB, int64_t dA) { return ((dB + 63) / 64) * ((dA + 63) / 64); }
 
-}  // namespace ak
-
-extern "C" size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count) {
-  size_t floats = 0;
-  for (int i = 0; i < count; ++i) floats += static_cast<size_t>(items[6 * i + 4]) * items[6 * i + 5] + items[6 * i + 4];
-  return floats * sizeof(float);
-}
-
-extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, int unit_count, float grad_scale,
-                                    const int* fail0, const int* fail1, int only_if_faster, void* ws, size_t ws_bytes,
-                                    ak_stream_t stream) {
-  using namespace ak;
-  if (count < 0 || unit_count < 0 || (count > 0 && items == nullptr) || (unit_count > 0 && units == nullptr)) return AK_ERR_ARG;
-  // The rule: microseconds of both products on 64 x 64 tiles against those on the split kernel, whose rates gemm_f32.hpp and
-  // chol_group.hip use too (64 x 64: 2 us per chunk of 128 k; split: 1.6 us per k-tile of 32, 1 us once the device is full, and
-  // 20 us for the ranges of its operands).
+// The rule: microseconds of both products on 64 x 64 tiles against those on the split kernel, whose rates gemm_f32.hpp and
+// chol_group.hip use too (64 x 64: 2 us per chunk of 128 k; split: 1.6 us per k-tile of 32, 1 us once the device is full, and
+// 20 us for the ranges of its operands).  784-512-512-10 39 us here and 132 split, 2000^3 172 us a product here and 85 split.
+static bool kp_faster(const int64_t* items, int count) {
   double longest = 0, chunks = 0, long_tile = 0, ktiles = 0;
   for (int i = 0; i < count; ++i) {
-    const int64_t* r = items + 6 * i;
-    const int64_t dB = r[4], dA = r[5];
-    if (r[0] == 0 || r[1] == 0 || r[2] == 0 || dB <= 0 || dA <= 0) return AK_ERR_ARG;
-    if (dB > KP_MAX_ROWS || dA > KP_MAX_COLUMNS) return AK_ERR_UNSUPPORTED;
+    const int64_t dB = items[6 * i + 4], dA = items[6 * i + 5];
     for (const int64_t K : {dB, dA}) {
       const double c = static_cast<double>((K + 127) / 128), t = static_cast<double>((K + 31) / 32);
       longest = std::max(longest, c);
@@ -145,14 +130,40 @@ extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64
       ktiles += t * static_cast<double>(((dB + 127) / 128) * ((dA + 127) / 128));
     }
   }
+  return 2.0 * std::max(2 * longest, chunks / 256) <= std::max(2 * 1.6 * long_tile, ktiles / 256) + 20;
+}
+
+}  // namespace ak
+
+extern "C" size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count) {
+  size_t floats = 0;
+  for (int i = 0; i < count; ++i) floats += static_cast<size_t>(items[6 * i + 4]) * items[6 * i + 5] + items[6 * i + 4];
+  return floats * sizeof(float);
+}
+
+extern "C" int ak_kron_precond_deep_faster(const int64_t* items, int count) {
+  if (count < 0 || (count > 0 && items == nullptr)) return AK_ERR_ARG;
+  for (int i = 0; i < count; ++i)
+    if (items[6 * i + 4] <= 0 || items[6 * i + 5] <= 0) return AK_ERR_ARG;
+  return ak::kp_faster(items, count) ? 1 : 0;
+}
+
+extern "C" int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, int unit_count, float grad_scale,
+                                    const int* fail0, const int* fail1, int only_if_faster, void* ws, size_t ws_bytes,
+                                    ak_stream_t stream) {
+  using namespace ak;
+  if (count < 0 || unit_count < 0 || (count > 0 && items == nullptr) || (unit_count > 0 && units == nullptr)) return AK_ERR_ARG;
+  for (int i = 0; i < count; ++i) {
+    const int64_t* r = items + 6 * i;
+    if (r[0] == 0 || r[1] == 0 || r[2] == 0 || r[4] <= 0 || r[5] <= 0) return AK_ERR_ARG;
+    if (r[4] > KP_MAX_ROWS || r[5] > KP_MAX_COLUMNS) return AK_ERR_UNSUPPORTED;
+  }
   for (int i = 0; i < unit_count; ++i) {        // (all of them before the first launch)
     const int64_t* r = units + 4 * i;
     if (r[0] == 0 || r[1] == 0 || r[2] == 0 || r[3] <= 0) return AK_ERR_ARG;
     if (r[3] > KP_MAX_UNIT) return AK_ERR_UNSUPPORTED;
   }
-  const double deep_us = 2.0 * std::max(2 * longest, chunks / 256);
-  const double split_us = std::max(2 * 1.6 * long_tile, ktiles / 256) + 20;
-  if (only_if_faster && deep_us > split_us) return AK_ERR_UNSUPPORTED;
+  if (only_if_faster && !kp_faster(items, count)) return AK_ERR_UNSUPPORTED;
   if (count > 0 && (ws == nullptr || ws_bytes < ak_kron_precond_deep_ws_bytes(items, count))) return AK_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* t = static_cast<float*>(ws);

@@ -1082,6 +1082,14 @@ def kron_precond_deep(items, units, grad_scale, device, fail=(), only_if_faster=
     return True
 
 
+def kron_precond_deep_pays(shapes):
+    """Whether kron_precond_deep() takes modules of these (dB, dA) with only_if_faster."""
+    items = [v for dB, dA in shapes for v in (0, 0, 0, 0, dB, dA)]
+    answer = _lib.load().ak_kron_precond_deep_faster((ctypes.c_int64 * len(items))(*items), len(shapes))
+    _lib.check(min(answer, 0), 'ak_kron_precond_deep_faster')
+    return answer == 1
+
+
 def kron_damping(A_list, B_list, damping, eps=1e-7, eig_scale=None, nonzero=None):
     """Returns (lam [batch, 2] float32, nonzero [batch, 2] int32: ``nonzero`` itself if given), both on the device.  A factor is a square
     [d, d] matrix or, for the low-rank (swift) factors, an [n, d] matrix with n < d rows; ``eig_scale``: optional

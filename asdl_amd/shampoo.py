@@ -109,8 +109,6 @@ HALF_PIECE_STATISTICS = True      # the grouped statistics on two fp16 pieces pe
                                   # 0.3-1 %; one accumulator for the whole sum: 2-3 % at 2304 columns and up, 10 % at 768)
 HALF_PIECE_PRECONDITION = True     # grouped preconditioning on two fp16 pieces per element (kernels.KronPrecondPlan does the same)
 GROUPED_PRECONDITION = True      # matrix-shaped parameters: all their preconditioning products in two launches
-SMALL_PRECONDITION_ELEMENTS = 1 << 22     # of all matrices; beyond it the split products win (2000^3 172 us a product on fp32 tiles, 2048^3
-                                  # 85 split) and no workspace is taken to find that out
 GROUPED_STATISTIC_MIN_DIM = 768   # statistics of this size and up go into one grouped launch (with GROUPED_PRECONDITION)
 
 
@@ -234,6 +232,7 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
                                                        preconditioners=[views[(pi, a)][1] for a in range(p.ndim)]))
         self.start_vector_fn = None     # optional: (count, n, device) -> [count, n] start vectors
         self.last_root_stats = {}
+        self._deep_pays = None
 
     def state_dict(self) -> dict:
         """``step`` as in the reference (asdl/precondition/prec_grad_maker.py:129-133) plus, under ``shampoo``, the
@@ -299,8 +298,13 @@ class ShampooGradientMaker(PreconditionedGradientMaker):
         """All matrix-shaped parameters of a small model in two launches of fp32 tiles, whatever their sizes' alignment
         (784-512-512-10: seven launches, 132 us, before; two, 39 us, now; the rule of ak_kron_precond_deep, which takes these
         products for Kronecker factors too).  The roots are symmetric.  Returns the parameters that are left."""
-        small = [pc for pc in self.preconditioners if self._groupable(pc, align=1)] if GROUPED_PRECONDITION else []
-        if not small or sum(pc.param.numel() for pc in small) > SMALL_PRECONDITION_ELEMENTS:
+        if self._deep_pays is None:              # the sizes decide, and stay
+            shapes = [pc._transformed_shape for pc in self.preconditioners if len(pc._transformed_shape) == 2]
+            self._deep_pays = kernels.kron_precond_deep_pays(shapes)
+        if not GROUPED_PRECONDITION or not self._deep_pays:
+            return list(self.preconditioners)
+        small = [pc for pc in self.preconditioners if self._groupable(pc, align=1)]
+        if not small:
             return list(self.preconditioners)
         items = []
         for pc in small:

@@ -180,6 +180,7 @@ int ak_event_synchronize(void* event);
  * is written when one of them is not zero.  AK_ERR_UNSUPPORTED, and nothing done: a module or unit beyond the sizes of this form
  * (dB > 32768, dA > 2^20, F > 2^24), and with only_if_faster where ak_gemm_f32_grouped on split operands is expected to be faster. */
 size_t ak_kron_precond_deep_ws_bytes(const int64_t* items, int count);
+int ak_kron_precond_deep_faster(const int64_t* items, int count);      /* the rule of only_if_faster: 1 or 0; reads dB and dA only */
 int ak_kron_precond_deep(const int64_t* items, int count, const int64_t* units, int unit_count, float grad_scale,
                          const int* fail0, const int* fail1, int only_if_faster, void* ws, size_t ws_bytes,
                          ak_stream_t stream);

@@ -773,3 +773,20 @@ def test_small_matrices_precondition_in_two_launches(widths):
     maker.precondition()
     for pc, g in zip(maker.preconditioners, expected):
         assert relerr(pc.param.grad, g) < 1e-5
+
+
+def test_models_whose_products_go_to_the_grouped_path_are_not_asked_at_every_step(monkeypatch):
+    """The sizes decide between the two-launch form and the split products (one rule, the library's): a declined model pays for the
+    question once, without a call that walks its gradients or takes a workspace."""
+    model = nn.Sequential(nn.Linear(1440, 1440), nn.Linear(1440, 1440)).cuda()
+    assert not K.kron_precond_deep_pays([(1440, 1440)] * 2) and K.kron_precond_deep_pays([(512, 784), (512, 512), (10, 512)])
+    maker = ShampooGradientMaker(model, PreconditioningConfig(damping=1e-6))
+    calls = []
+    monkeypatch.setattr(K, 'kron_precond_deep', lambda *a, **k: calls.append(a))
+    for _ in range(2):
+        for pc in maker.preconditioners:
+            pc.param.grad = torch.randn_like(pc.param)
+        expected = [pc.param.grad.clone() for pc in maker.preconditioners]
+        maker.precondition()                     # (the preconditioners are identities)
+        assert not calls
+        assert all(relerr(pc.param.grad, g) < 1e-5 for pc, g in zip(maker.preconditioners, expected))
