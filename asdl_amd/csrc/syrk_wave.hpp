@@ -327,18 +327,18 @@ inline int launch_syrk_chain(const float* X, int64_t d, int64_t K, int64_t ld, b
   return check_launch();
 }
 
-// The split of K whose estimated time is shortest: matrix instructions, and for more than one part their way through memory
-// and the second launch.
-inline int syrk_wave_split(int64_t d, int64_t K) {
+// The split of K, into `fewest` parts at least, whose estimated time is shortest: matrix instructions, and for more than one part
+// their way through memory and the second launch.
+inline int64_t syrk_wave_split(int64_t d, int64_t K, int64_t fewest = 1) {
   const int64_t T = (d + 63) / 64, tiles = T * (T + 1) / 2;
-  int best = 1;
+  int64_t best = fewest;
   double least = 1e30;
-  for (int64_t s = 1; s <= 512; s = s < 8 ? s + 1 : s + s / 8) {
-    if (s > 1 && K / s < 64) break;
+  for (int64_t s = fewest; s <= std::max<int64_t>(512, fewest); s = s < 8 ? s + 1 : s + s / 8) {
+    if (s > fewest && K / s < 64) break;
     const double rounds = static_cast<double>((tiles * s + 255) / 256);
     double t = 5.0 + 0.0133 * static_cast<double>((K + s - 1) / s + 32) * rounds;
     if (s > 1) t += 4.0 + static_cast<double>(tiles * s) * 16384.0 * 2 / 4e6;
-    if (t < least) { least = t; best = static_cast<int>(s); }
+    if (t < least) { least = t; best = s; }
   }
   return best;
 }
@@ -353,8 +353,7 @@ inline bool syrk_wave_rows(int64_t d, int64_t K) {
   return d <= 128 || (tiles * s + 255) / 256 * ((K + s - 1) / s) <= 1536;
 }
 inline size_t syrk_wave_ws_bytes(int64_t d, int64_t K) {
-  const int64_t T = (d + 63) / 64;
-  const int s = syrk_wave_split(d, K);
+  const int64_t T = (d + 63) / 64, s = syrk_wave_split(d, K);
   return s > 1 ? static_cast<size_t>(s) * (T * (T + 1) / 2) * 4096 * sizeof(float) : 0;
 }
 
@@ -363,16 +362,16 @@ inline int launch_syrk_wave(const float* X, int64_t d, int64_t K, int64_t ld, in
                             int64_t ldc, void* ws, size_t ws_bytes, hipStream_t stream) {
   SyrkWaveParams p;
   const int64_t T = (d + 63) / 64, tiles = T * (T + 1) / 2;
-  int s = syrk_wave_split(d, K);
+  int64_t s = syrk_wave_split(d, K);
   p.per_split = ((K + s - 1) / s + 63) / 64 * 64;
-  s = static_cast<int>((K + p.per_split - 1) / p.per_split);
+  s = (K + p.per_split - 1) / p.per_split;
   if (s > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(s) * tiles * 4096 * sizeof(float))) return AK_ERR_WORKSPACE;
-  p.X = X; p.ld = ld; p.sn = sn; p.K = K; p.d = static_cast<int>(d); p.run = run; p.T = static_cast<int>(T); p.nsplit = s;
-  p.alpha = alpha; p.beta = beta; p.C = C; p.ldc = ldc; p.ws = static_cast<float*>(ws);
+  p.X = X; p.ld = ld; p.sn = sn; p.K = K; p.d = static_cast<int>(d); p.run = run; p.T = static_cast<int>(T);
+  p.nsplit = static_cast<int>(s); p.alpha = alpha; p.beta = beta; p.C = C; p.ldc = ldc; p.ws = static_cast<float*>(ws);
   const dim3 grid(static_cast<unsigned>(tiles * s));        // (d > 2^20 would pass 2^31 - 1: no such matrix fits)
   if (run > 0) hipLaunchKernelGGL(syrk_wave_kernel<true>, grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(syrk_wave_kernel<false>, grid, dim3(256), 0, stream, p);
-  if (s > 1) launch_syrk_finalize<1>(p.ws, s, tiles, p.T, C, ldc, d, alpha, beta, stream);
+  if (s > 1) launch_syrk_finalize<1>(p.ws, p.nsplit, tiles, p.T, C, ldc, d, alpha, beta, stream);
   return check_launch();
 }
 

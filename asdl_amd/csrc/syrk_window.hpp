@@ -161,12 +161,17 @@ static __global__ __launch_bounds__(256, 2) void syrk_window_kernel(SyrkWindowPa
   syrk_wave_finish(acc, reinterpret_cast<floatx4(*)[4][4][64]>(smem), p, id, i0, j0, diag);
 }
 
-// Positions of a work group: as many as the model of syrk_wave_split gives, at most what the table holds.
-inline int64_t syrk_window_per_split(int64_t d, int64_t K, int* nsplit) {
-  const int s = syrk_wave_split(d, K);
-  int64_t per = ((K + s - 1) / s + 63) / 64 * 64;
-  if (per > SWIN_MAX_K) per = SWIN_MAX_K;
-  *nsplit = static_cast<int>((K + per - 1) / per);
+// Positions of a work group, at most what the table holds, and at most 1024 where the partial sums stay below 64 MB: two work groups
+// of a CU hide each other's gathers, and a matrix of a round or less would have one.  Even parts: the model of syrk_wave_split
+// chooses among the splits that fit (a split of its own choice, cut to 4096, left a short one as a round of its own).
+// us, staged, cut to 4096 and here: 3 x 3 of 64 x 100 x 14 x 14 without padding 168, 220 and 138; 128 x 256 x 8 x 8 550, 586 and 335;
+// with padding 128 x 96 x 8 x 8 110, 112 and 103; 5 x 5 of 16 x 24 x 56 x 56 332, 379 and 295.
+inline int64_t syrk_window_per_split(int64_t d, int64_t K, int64_t* nsplit) {
+  const int64_t T = (d + 63) / 64, tiles = T * (T + 1) / 2;
+  const int64_t most = tiles * ((K + 1023) / 1024) <= 4096 ? 1024 : SWIN_MAX_K;
+  const int64_t s = syrk_wave_split(d, K, (K + most - 1) / most);
+  const int64_t per = ((K + s - 1) / s + 63) / 64 * 64;
+  *nsplit = (K + per - 1) / per;
   return per;
 }
 inline bool syrk_window_ok(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int64_t Ho, int64_t Wo) {
@@ -176,15 +181,16 @@ inline bool syrk_window_ok(int64_t N, int64_t C, int64_t H, int64_t W, int kh, i
          N * Ho * Wo < (1ll << 40);
 }
 // The staged kernel stays for strided 1 x 1 windows of many products: a lane's every load is a line of its own there (staged and
-// here, us: 32 x 300 x 14 x 14 86 and 18 (15 tiles), 32 x 1024 x 14 x 14 132 and 143, 64 x 256 x 56 x 56 124 and 147).  Other
-// windows are 0-60 % faster here but for a few with rows of whole stages (128 x 96 x 8 x 8 3 x 3: 109 and 117).
+// here, us: 32 x 300 x 14 x 14 86 and 18 (15 tiles), 32 x 1024 x 14 x 14 132 and 143, 64 x 256 x 56 x 56 124 and 147).  Of 241 other
+// windows (3 x 3 and 5 x 5, strides 1 and 2, 24 to 256 channels) none is more than 1 % slower here (3 x 3 of 32 x 96 x 16 x 16 117.3
+// and 117.5).
 inline bool syrk_window_faster(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int64_t Ho, int64_t Wo) {
   if (!syrk_window_ok(N, C, H, W, kh, kw, Ho, Wo)) return false;
   const int64_t T = (C * kh * kw + 63) / 64, work = T * (T + 1) / 2 * N * Ho * Wo;
   return kh * kw > 1 || (sh == 1 && sw == 1) || work <= 700 * 256;
 }
 inline size_t syrk_window_ws_bytes(int64_t d, int64_t K) {
-  int s;
+  int64_t s;
   syrk_window_per_split(d, K, &s);
   const int64_t T = (d + 63) / 64;
   return s > 1 ? static_cast<size_t>(s) * (T * (T + 1) / 2) * 4096 * sizeof(float) : 0;
@@ -196,18 +202,18 @@ inline int launch_syrk_window(const float* X, int64_t N, int64_t C, int64_t H, i
   SyrkWindowParams q;
   SyrkWaveParams& p = q.w;
   const int64_t d = C * kh * kw, K = N * Ho * Wo, T = (d + 63) / 64, tiles = T * (T + 1) / 2;
-  int s;
+  int64_t s;
   p.per_split = syrk_window_per_split(d, K, &s);
   if (s > 1 && (ws == nullptr || ws_bytes < static_cast<size_t>(s) * tiles * 4096 * sizeof(float))) return AK_ERR_WORKSPACE;
   if (tiles * s >= (1ll << 31)) return AK_ERR_UNSUPPORTED;
-  p.X = X; p.ld = 0; p.sn = 0; p.K = K; p.d = static_cast<int>(d); p.run = 0; p.T = static_cast<int>(T); p.nsplit = s;
+  p.X = X; p.ld = 0; p.sn = 0; p.K = K; p.d = static_cast<int>(d); p.run = 0; p.T = static_cast<int>(T); p.nsplit = static_cast<int>(s);
   p.alpha = alpha; p.beta = beta; p.C = A; p.ldc = lda; p.ws = static_cast<float*>(ws);
   q.image = C * H * W; q.images_bytes = N * q.image * 4;
   q.H = static_cast<int>(H); q.W = static_cast<int>(W); q.Ho = static_cast<int>(Ho); q.Wo = static_cast<int>(Wo);
   q.kh = kh; q.kw = kw; q.sh = sh; q.sw = sw; q.ph = ph; q.pw = pw;
   q.mWo = make_magic(q.Wo); q.mHo = make_magic(q.Ho);
   hipLaunchKernelGGL(syrk_window_kernel, dim3(static_cast<unsigned>(tiles * s)), dim3(256), 0, stream, q);
-  if (s > 1) launch_syrk_finalize<1>(p.ws, s, tiles, p.T, A, lda, d, alpha, beta, stream);
+  if (s > 1) launch_syrk_finalize<1>(p.ws, p.nsplit, tiles, p.T, A, lda, d, alpha, beta, stream);
   return check_launch();
 }
 
