@@ -222,7 +222,7 @@ static __global__ __launch_bounds__(256, 2) void syrk_wave_kernel(SyrkWaveParams
 // them, the k of an instruction paired as there (rows: 2 u and 2 u + 1; runs: 16 t + m and 16 t + 8 + m).  A work group owns a
 // 64 x 64 tile of one split, a wave a 32 x 32 block of it.  Bound by the chain of matrix instructions (64 cycles per two k) behind
 // one way to memory, 64 k of both operands in flight.  us, staged and here:
-// one 512 x 784 matrix 55 and 14.5, 767 x 3072 54 and 48, rows of 512 x 512 18.7 and 11.6.
+// one 512 x 784 matrix 55 and 14, 767 x 3072 53 and 46, rows of 512 x 512 18.7 and 11.6.
 template <bool RUNS, bool MASK>
 __device__ __forceinline__ void syrk_chain_fetch(float (&x)[32], const float* __restrict__ X, int64_t ld, uint32_t at, int64_t k, int64_t k1,
                                                  int g) {
@@ -306,7 +306,10 @@ static __global__ __launch_bounds__(256, 2) void syrk_chain_kernel(SyrkWaveParam
 }
 
 // Rows: up to 176 k of tiles a CU; beyond that the loads of 32 columns of a row count (staged and here, us: 512 x 767 28 and 21,
-// 700 x 600 24 and 22, 1000 x 700 27.5 and 28, 2000 x 512 24 and 27, 2000 x 700 38 and 47).
+// 700 x 600 24 and 22, 1000 x 700 27.5 and 28, 2000 x 512 24 and 27, 2000 x 700 38 and 47).  Runs, read in 16-byte loads, go to the
+// chain at every size: of 55 matrices of 30 to 4096 x 784 to 16384 one of 1536 x 1536 and one of 1536 x 2304 lose 5 % (81 and 86 us,
+// 110 and 115), 767 and 1024 x 16384 4 and 3 %, the others gain (512 x 784 55 and 14, 1024 x 3072 77 and 74, 3072 x 3072 591 and
+// 510, 4096 x 16384 6006 and 4350).
 inline bool syrk_chain_rows(int64_t d, int64_t K) {
   const int64_t T = (d + 63) / 64;
   return T * (T + 1) / 2 * K <= 176 * 256;
