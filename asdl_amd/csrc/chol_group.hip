@@ -33,10 +33,10 @@ constexpr int64_t CG_MAGIC = 0x3447524c4f4843ll;     // "CHOLGR4"
 constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_PROD = 2, CG_PROD_DEEP = 3, CG_SWEEP = 4, CG_OUT = 5;
 
 // What an operand of a product holds, for the fp16-piece products (bits 4-5 of CgProd::flags: A, bits 6-7: B).  With
-// a = the largest diagonal element of A + lam I, every element is bounded in magnitude: a block of the (updated)
-// matrix by a, of its Cholesky factor L by sqrt(a), of M = L^-1 by 1 / sqrt(lam), of L21 L11^-1 by sqrt(a / lam).
+// a = the largest diagonal element of A + lam I, every element is bounded in magnitude: of the Cholesky factor L by sqrt(a),
+// of M = L^-1 by 1 / sqrt(lam).
 constexpr int CG_KIND_L = 1, CG_KIND_M = 2;
-constexpr int CG_SCALE_FLOATS = 8;                    // per matrix: the four scales, the fp16 switch, padding
+constexpr int CG_SCALE_FLOATS = 4;                    // per matrix: the fp16 switch, the scales of both kinds, padding
 #ifdef AK_TUNING_HOOKS
 static float CG_HALF_MAX_COND = 65536.f;              // tuning builds: ak_debug_set_chol_half_max_cond
 #else
@@ -163,19 +163,14 @@ static __global__ __launch_bounds__(256) void cg_scale_kernel(CgArgs a, int coun
   const float lam = live ? a.lam[static_cast<int64_t>(m) * a.lam_stride] : 0.f;
   amax += lam;
   const bool half = live && lam > 0.f && amax > 0.f && amax < 3.0e38f && amax <= max_cond * lam;
-  float s[4] = {1.f, 1.f, 1.f, 1.f};
-  if (half) {
-    const float bound[4] = {amax, sqrtf(amax), 1.f / sqrtf(lam), sqrtf(amax / lam)};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      int e;
-      frexpf(bound[k], &e);              // bound <= 2^e
-      s[k] = ldexpf(1.f, 14 - e);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) sc[k] = s[k];
-  sc[4] = half ? 1.f : 0.f;
+  auto scale = [&](float bound) {
+    int e;
+    frexpf(bound, &e);                   // bound <= 2^e
+    return half ? ldexpf(1.f, 14 - e) : 1.f;
+  };
+  sc[0] = half ? 1.f : 0.f;
+  sc[CG_KIND_L] = scale(sqrtf(amax));
+  sc[CG_KIND_M] = scale(1.f / sqrtf(lam));
 }
 
 // out_m <- both triangles of W_m, one work group per 64 x 64 tile of its lower triangle (bisection on first_out_block).
@@ -226,23 +221,12 @@ __device__ __forceinline__ void cg_decode_tile(const CgProd& d, int local, int& 
     tj = local - ti * (ti + 1) / 2;
     return;
   }
-  switch (d.kmode) {
-    case K_LE_J:                     // k <= column tile: last column first
-      tj = d.tiles_n - 1 - local / d.tiles_m;
-      ti = local % d.tiles_m;
-      break;
-    case K_GE_J:                     // k >= column tile: first column first
-      tj = local / d.tiles_m;
-      ti = local % d.tiles_m;
-      break;
-    case K_LE_I:                     // k <= row tile: last row first
-      ti = d.tiles_m - 1 - local / d.tiles_n;
-      tj = local % d.tiles_n;
-      break;
-    default:
-      ti = local / d.tiles_n;
-      tj = local % d.tiles_n;
-      break;
+  if (d.kmode == K_GE_J) {           // k >= column tile: first column first
+    tj = local / d.tiles_m;
+    ti = local % d.tiles_m;
+  } else {
+    ti = local / d.tiles_n;
+    tj = local % d.tiles_n;
   }
 }
 
@@ -270,7 +254,7 @@ static __global__ __launch_bounds__(256, 2) void cg_prod_kernel(CgArgs a, const 
   p.split = 3;
   p.scaleA = p.scaleB = 1.f;
   const float* __restrict__ sc = a.scales + static_cast<int64_t>(d.mat) * CG_SCALE_FLOATS;
-  if (sc[4] != 0.f) {
+  if (sc[0] != 0.f) {
     // fp16 pieces: two per operand element, three matrix instructions per product instead of six
     p.scaleA = sc[(d.flags >> 4) & 3];
     p.scaleB = sc[(d.flags >> 6) & 3];
@@ -649,27 +633,37 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
   plan.h.us = sweep_us;
 }
 
+// The plan of the sizes that this thread asked for last: a caller asks for the bytes, the workspace and the plan one after the other.
+static const CgPlan& cg_plan(const int64_t* dims, int count) {
+  thread_local std::vector<int64_t> key;
+  thread_local CgPlan plan;
+  std::vector<int64_t> asked(dims, dims + count);
+  asked.push_back(CG_FORCE);
+  if (key != asked) {
+    key.clear();                       // (nothing is kept if the tables do not fit the memory)
+    plan = CgPlan();
+    cg_build(dims, count, plan);
+    key.swap(asked);
+  }
+  return plan;
+}
+
 }  // namespace ak
 
 extern "C" size_t ak_chol_group_plan_bytes(const int64_t* dims, int count) {
   if (!ak::cg_dims_ok(dims, count)) return 0;
-  ak::CgPlan plan;
-  ak::cg_build(dims, count, plan);
-  return static_cast<size_t>(plan.h.total_bytes);
+  return static_cast<size_t>(ak::cg_plan(dims, count).h.total_bytes);
 }
 
 extern "C" size_t ak_chol_group_ws_bytes(const int64_t* dims, int count) {
   if (!ak::cg_dims_ok(dims, count)) return 0;
-  ak::CgPlan plan;
-  ak::cg_build(dims, count, plan);
-  return static_cast<size_t>(plan.h.ws_floats) * sizeof(float);
+  return static_cast<size_t>(ak::cg_plan(dims, count).h.ws_floats) * sizeof(float);
 }
 
 extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_host, size_t plan_bytes) {
   using namespace ak;
   if (!cg_dims_ok(dims, count) || plan_host == nullptr) return AK_ERR_ARG;
-  CgPlan plan;
-  cg_build(dims, count, plan);
+  const CgPlan& plan = cg_plan(dims, count);
   if (plan_bytes < static_cast<size_t>(plan.h.total_bytes)) return AK_ERR_WORKSPACE;
   unsigned char* out = static_cast<unsigned char*>(plan_host);
   std::memset(out, 0, static_cast<size_t>(plan.h.total_bytes));
