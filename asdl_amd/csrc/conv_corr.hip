@@ -141,12 +141,11 @@ __device__ __forceinline__ void corr_reduce_tile(const CorrArgs& a, int tile, in
   const int64_t stride = ntiles * tile_f4;
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   int s = 0;
-  for (; s + 8 <= cp.nsplit; s += 8) {                 // eight loads in flight, summed in order
+  for (; s + 8 <= cp.nsplit; s += 8) {                 // eight loads in flight, summed in pairs: 39 roundings in a row show
     floatx4 w[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) w[k] = src[(s + k) * stride];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) acc += w[k];
+    acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
   }
   for (; s < cp.nsplit; ++s) acc += src[s * stride];
   const int ld = kCorrPieces * a.Cin;
@@ -273,8 +272,8 @@ __global__ __launch_bounds__(kAsmThreads) void corr_assemble_kernel(CorrAsm a) {
 // + mid^T mid'; the three dropped blocks are below 2^-24 of the product.  The pairs are added in this order so that
 // the fold of a symmetric piece is symmetric to the last bit.
 // Two fp16 planes of channels scaled by powers of two would need half the matrix work (128 x 64 x 32 x 32, 128 x 16 x 16,
-// 256 x 8 x 8, 512 x 4 x 4 channels and pixels: 142, 114, 118, 158 us instead of 254, 179, 188, 251), but hold 22 of the 24 bits:
-// single products are off by up to 4e-7 instead of 1.2e-7, the factor of zero-mean 100 x 64 x 14 x 14 by 1.4e-7 instead of 1.2e-7.
+// 256 x 8 x 8, 512 x 4 x 4 channels and pixels: 142, 114, 118, 158 us instead of 203, 146, 164, 258), but hold 22 of the 24 bits:
+// single products are off by up to 3.6e-7 instead of 1.2e-7.
 
 // x: [N, C, HW] fp32 (HW contiguous) -> planes: [N, HW, 3 C] bf16.  One work group per (sample, 32 pixels, 32
 // channels): coalesced 128-byte reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
@@ -401,8 +400,12 @@ static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int 
                   ntiles = static_cast<int64_t>(p.npairs) * p.ntaps * p.ppt * p.ppt;
     int64_t ns = 1;
     if (i == 0 && ntiles > 0) {
-      // the main product fills the device once (the corrections ride in its tail); at least 8 k-tiles per split
-      ns = (slots + ntiles / 2) / ntiles;
+      // the main product fills the device once (the corrections ride in its tail); at least 8 k-tiles per split.  Planes of an
+      // fp32 input: three times (256-wide tiles: twice), because a sum rounds at the magnitude of its split (error against 64 bits
+      // of 128 x 64 x 32 x 32, 128 x 16 x 16, 256 x 8 x 8, 512 x 4 x 4 channels and pixels after a ReLU, once and now: 1.2, 1.5, 1.5,
+      // 2.1e-7 and 0.9, 0.9, 0.9, 1.1e-7; 246, 167, 179, 241 and 203, 146, 164, 258 us).
+      const int64_t rounds = planes == 1 ? 1 : bt < 256 ? 3 : 2;
+      ns = (rounds * slots + ntiles / 2) / ntiles;
       const int64_t cap = ktiles / 8 < 1 ? 1 : ktiles / 8;
       if (ns > cap) ns = cap;
       if (ns < 1) ns = 1;

@@ -1539,3 +1539,14 @@ def test_fp32_correlations_hold_all_24_bits(K, N, C, H, W):
     rows = nn.functional.unfold(x.double(), 3, 1, 1, 1).permute(0, 2, 1).reshape(-1, 9 * C)
     out = K.conv_syrk(x.cuda(), (3, 3), (1, 1), (1, 1))
     assert float((out.double().cpu() - rows.T @ rows).abs().max()) <= 2.0 ** -23
+
+
+@pytest.mark.parametrize("N,C,H", [(128, 64, 32), (128, 128, 16), (128, 256, 8)])
+def test_fp32_correlations_are_as_close_as_one_rounding_of_the_result(K, N, C, H):
+    """Sums over 8192 to 131072 pixels of ReLU outputs: their accumulators round at the magnitude of a split, and the factor ends
+    within 2^-23 of the product in 64 bits (one split per place of the device: 1.3 to 1.5e-7)."""
+    x = torch.randn(N, C, H, H, generator=torch.Generator().manual_seed(C)).relu().cuda()
+    u = nn.functional.unfold(x.double(), 3, padding=1).transpose(1, 2).reshape(-1, 9 * C)
+    out = K.conv_syrk(x, (3, 3), (1, 1), (1, 1)).double()
+    ref = u.T @ u
+    assert float((out - ref).norm() / ref.norm()) < 2.0 ** -23
