@@ -10,7 +10,7 @@
 // instead of one, but no second launch); where they are more than the device takes at once, the launch forms the v only and
 // the tiles are products of a launch of their own.  At the end of the group all tiles get their update from V at once (the
 // products of CgOp: X -+ V V^T, 512 deep, on the split-operand tiles of the grouped products).  Work: d^3 in all, as in the sweep;
-// chain: 22 us per 128 columns for any number of tiles up to one per CU, and one product per 512.
+// chain: 26 to 30 us per 128 columns while a step has up to a tile per CU, and one product per 512.
 //
 // W: the work matrix (lower triangle, row-major, dp columns), lam added by cg_copy_in_kernel.  Tiles (r, i) inside a group live in
 // E from the step that makes them (i = k), because their place in W is column k, which the same launch reads.  M alternates

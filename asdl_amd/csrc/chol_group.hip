@@ -5,8 +5,9 @@
 //   chol_sweep.hpp   every step updates the whole triangle: one launch per 128 columns, for groups whose tiles fit the device
 //   chol_chain.hpp   the steps update the block columns that the next steps need, one product per 512 columns the rest
 // The plan takes the chain where it saves enough (cg_build).  Explicit inverses are taken of 128 x 128 diagonal blocks only, so a panel is
-// as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: below the error of
-// LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half was at 3-8 times that).
+// as accurate as a triangular solve with a block of that size (measured against fp64 on rank-deficient factors: the sweep at 0.8 to 0.9,
+// the chain at 1.4 to 1.7 times the error of LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half
+// was at 3 to 8 times that).
 //
 // The steps of all matrices are merged: step k of the chain is one launch for all matrices that have a block k, the products
 // at the end of a group are one launch for all matrices (one work group per tile of any product, descriptor found through a
@@ -468,8 +469,8 @@ static int CG_FORCE = 0;               // tuning builds: 1 the sweep, 2 the chai
 constexpr int CG_FORCE = 0;
 #endif
 
-// The chain's tables.  Returns its estimated time: 22 us a step or 18 per round of tiles (a panel alone: 9), the products by
-// cg_product_us, the copies by their bytes.
+// The chain's tables.  Returns its estimated time: 26 us a step, or 9 and 18 per round of tiles (of panels alone: 9) where that is
+// more, the products by cg_product_us, the copies by their bytes.
 static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
   struct Mat { int64_t w, v, e, m; int d, dp, nb; };
   std::vector<Mat> mats(count);

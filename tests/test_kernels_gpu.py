@@ -759,6 +759,37 @@ def test_chol_inv_grouped_operand_scaling(K, scale, lam_rel):
         assert e < max(1e-4, 2 * e_ref), (i, cond, e, e_ref)
 
 
+@pytest.mark.parametrize('scale,lam_rel', [(1e-8, 1e-2), (1e6, 1e-2), (1.0, 1e-4), (1e-3, 3e-5), (1.0, 1.4e-5), (1.0, 1e-6), (3e-5, 1e-8), (1.0, 1e-12), (1e4, 0.0)])
+def test_chol_inv_grouped_operand_scaling_on_the_chain(K, scale, lam_rel):
+    """The same for a group of the chain (csrc/chol_chain.hpp), whose products at the end of four blocks are those on fp16 pieces, or
+    on three bf16 pieces where a / lam exceeds 2^16 or lam = 0; 640 columns above are on the block sweep, which has none."""
+    d, count = 1100, 24                                          # three groups of blocks: every kind of product, the last ones ragged
+    assert K.chol_group_plan([d] * count).launches != (d + 127) // 128 + 1, 'the block sweep: one launch per block column'
+    distinct = [_spd(d, 400 + seed, rows=rows) * scale for rows, seed in ((2 * d, 1), (d // 4, 2), (d - 100, 3))]      # full rank; ranks 275, 1000
+    lams = [lam_rel * float(A.diagonal().max()) for A in distinct]
+    mats = [distinct[i % 3].cuda() for i in range(count)]
+    lam = torch.tensor([lams[i % 3] for i in range(count)], device='cuda')
+    outs = [torch.empty_like(m) for m in mats]
+    print(f'chol_inv_grouped chain scale={scale} lam_rel={lam_rel}', flush=True)
+    info = K.chol_inv_grouped(mats, outs, lam).cpu()
+    for i, A in enumerate(distinct):
+        assert all(int(v) == int(info[i]) for v in info[i::3])
+        try:
+            ref = torch.linalg.inv(A.cuda().double() + lams[i] * torch.eye(d, dtype=torch.float64, device='cuda'))
+            e_ref = relerr(R.cholesky_inv(A, lams[i]), ref)
+        except torch.linalg.LinAlgError:
+            e_ref = None
+        if e_ref is None or not np.isfinite(e_ref) or e_ref > 1e-2:      # beyond what fp32 can factor, as above
+            print(f'  matrix {i}: out of reach of fp32 (oracle: {e_ref}; info here {int(info[i])})', flush=True)
+            continue
+        assert int(info[i]) == 0 and torch.isfinite(outs[i]).all()
+        for o in outs[i + 3::3]:
+            assert torch.equal(o, outs[i])
+        e = relerr(outs[i], ref)
+        print(f'  matrix {i}: relative error {e:.1e} (fp32 oracle {e_ref:.1e})', flush=True)
+        assert e < max(1e-4, 2 * e_ref), (i, e, e_ref)
+
+
 @pytest.mark.parametrize('d', [2048, 2304, 4096, 4608])
 def test_chol_inv_large_matches_fp32_oracle_and_fp64(K, d):
     # the sizes of the largest ResNet factors: deepest recursion, every level on the split-bf16 tile kernel
