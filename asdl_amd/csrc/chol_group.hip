@@ -634,19 +634,26 @@ static void cg_build(const int64_t* dims, int count, CgPlan& plan) {
   plan.h.us = sweep_us;
 }
 
-// The plan of the sizes that this thread asked for last: a caller asks for the bytes, the workspace and the plan one after the other.
+// The plan of the sizes that this thread asked for last: a caller asks for the bytes, the workspace and the plan one after the other,
+// and the tables are given back with the plan.
+struct CgKept {
+  std::vector<int64_t> key;
+  CgPlan plan;
+};
+static CgKept& cg_kept() {
+  thread_local CgKept kept;
+  return kept;
+}
 static const CgPlan& cg_plan(const int64_t* dims, int count) {
-  thread_local std::vector<int64_t> key;
-  thread_local CgPlan plan;
+  CgKept& kept = cg_kept();
   std::vector<int64_t> asked(dims, dims + count);
   asked.push_back(CG_FORCE);
-  if (key != asked) {
-    key.clear();                       // (nothing is kept if the tables do not fit the memory)
-    plan = CgPlan();
-    cg_build(dims, count, plan);
-    key.swap(asked);
+  if (kept.key != asked) {
+    kept = CgKept();                   // (nothing is kept if the tables do not fit the memory)
+    cg_build(dims, count, kept.plan);
+    kept.key.swap(asked);
   }
-  return plan;
+  return kept.plan;
 }
 
 }  // namespace ak
@@ -679,6 +686,7 @@ extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_hos
   }
   if (!plan.tile_map.empty())
     std::memcpy(out + plan.h.map_off, plan.tile_map.data(), plan.tile_map.size() * sizeof(int32_t));
+  cg_kept() = CgKept();
   return AK_OK;
 }
 

@@ -39,7 +39,7 @@ extern "C" {
                                 reference's hooks run.  ak_conv_syrk / ak_conv_syrk_nhwc only, and only for layers of
                                 the window kernel (C*kh*kw <= 160, kh*kw > 1); AK_ERR_UNSUPPORTED elsewhere */
 #define AK_F32_IN_ORDER 3    /* fp32, summed in the order of the staged kernels whatever the size, the splits of the sum one after
-                              * the other (ak_syrk_tn, 1 x 1 windows of ak_conv_syrk):
+                              * the other (ak_syrk_tn, 1 x 1 windows of ak_conv_syrk; other windows: as AK_F32):
                               * for statistics whose inverse roots are taken with a ridge of 1e-6 of the largest eigenvalue,
                               * where another order moves the root of a rank-deficient statistic by 0.5-1 % */
 

@@ -101,6 +101,22 @@ def test_plan_of_the_grouped_inverse_says_how_long_it_takes():
     assert lib.ak_chol_group_plan_us(ctypes.create_string_buffer(256)) < 0
 
 
+def test_grouped_inverse_plans_do_not_depend_on_the_queries_before():
+    import ctypes
+    from asdl_amd import _lib
+    lib = _lib.load()
+
+    def plan_of(dims, others=()):
+        arr = (ctypes.c_int64 * len(dims))(*dims)
+        plan = ctypes.create_string_buffer(lib.ak_chol_group_plan_bytes(arr, len(dims)))
+        for other in others:
+            lib.ak_chol_group_ws_bytes((ctypes.c_int64 * len(other))(*other), len(other))
+        assert lib.ak_chol_group_plan(arr, len(dims), plan, len(plan)) == 0
+        return plan.raw, lib.ak_chol_group_ws_bytes(arr, len(dims))
+    for dims in ((784, 512, 10), (1100,) * 24, (4225,)):
+        assert plan_of(dims) == plan_of(dims) == plan_of(dims, others=((300,), dims[:-1] + (9,)))
+
+
 @pytest.mark.parametrize('dims', [(2817,), (2944,), (3072,), (3073,), (3500,), (2600, 2304, 2048, 1500, 700, 600), (2892, 2892, 1400, 700, 300, 200),
                                   (1601, 2836, 542, 176, 670, 81, 44, 19)])
 def test_inverses_that_the_sweep_can_take_stay_with_its_accuracy(dims):
