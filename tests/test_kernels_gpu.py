@@ -1534,6 +1534,14 @@ def test_fp32_windows_straight_to_the_matrix_instruction(K, N, C, H, W, kernel, 
     assert relerr(out, 0.5 * rows.T @ rows + beta) < TOL_FACTOR_F32 and torch.equal(out, out.T)
 
 
+def test_fp32_few_channels_add_their_partial_sums_in_pairs(K):
+    """89 images, one partial sum each.  Every rounding of a sum of positive terms is 2.8e-8 (rms) of its own magnitude: 16 slices of
+    5 or 6 partials added in pairs have 2.0 squares of the result's magnitude, one after the other 6.0, four running sums 3.4."""
+    x = torch.randn(89, 16, 6, 6, generator=torch.Generator().manual_seed(3)).relu()
+    rows = nn.functional.unfold(x.double(), 3, 1, 1, 1).permute(0, 2, 1).reshape(-1, 144)
+    assert relerr(K.conv_syrk(x.cuda(), (3, 3), (1, 1), (1, 1)), rows.T @ rows) < 2.8e-8 * 3.4 ** 0.5
+
+
 @pytest.mark.parametrize("N,C,H,W", [(82, 64, 5, 5), (64, 128, 6, 6), (3, 256, 27, 29), (100, 192, 5, 5), (9, 512, 15, 17), (2050, 64, 1, 1)])
 def test_fp32_correlations_of_channels_of_any_scale(K, N, C, H, W):
     """2048 pixels and more: channels scaled by powers of two of their own, from 1e-17 to 1e17, one of them zero."""
