@@ -1459,6 +1459,18 @@ def test_fp32_statistics_in_a_fixed_order_add_their_splits_one_by_one(K, d, k):
     assert torch.equal(K.syrk_tn(x.T.contiguous().cuda(), in_order=True).cpu(), ref)
 
 
+@pytest.mark.parametrize("transA", [False, True])
+@pytest.mark.parametrize("transB", [False, True])
+@pytest.mark.parametrize("Kd", [16, 24])
+def test_short_contractions_sum_on_two_accumulators(K, Kd, transA, transB):
+    """A matrix instruction adds two products, rounding twice.  Emulated in float32 for zero-mean operands: 7.4e-8 (16 k) and 7.3e-8 (24) on
+    one accumulator per 16 k, 6.1e-8 and 6.2e-8 on two."""
+    g = torch.Generator().manual_seed(Kd)
+    a, b = torch.randn(512, Kd, generator=g), torch.randn(Kd, 512, generator=g)
+    out = K.gemm((a.T if transA else a).contiguous().cuda(), (b.T if transB else b).contiguous().cuda(), transA=transA, transB=transB)
+    assert relerr(out, a.double() @ b.double()) < 6.7e-8
+
+
 @pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (1, 65, 17), (65, 1, 200), (64, 64, 16), (63, 66, 15), (129, 33, 127), (2, 130, 128), (200, 129, 143),
                                     (577, 75, 300), (65, 64, 1153), (31, 700, 2049), (1100, 1100, 300)])
 @pytest.mark.parametrize("transA", [False, True])
