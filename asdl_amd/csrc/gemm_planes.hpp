@@ -42,18 +42,49 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 // Number of a matrix buffer of an iteration: plain, or one of a pair (k, k + 1) of which an iteration reads one and writes the
 // other; which one is decided on the device by the parity of the matrix's own step count.
 struct PairedBuf {
-  int16_t index, sel;       // sel 0: plain; 1: the one an iteration reads; 2: the one it writes
+  int16_t index, sel;       // sel 0: plain; 1: the one an iteration reads; 2: the one it writes; 3: 2 in a quartic step, else 1
 };
-__device__ __forceinline__ int paired_buf(PairedBuf b, int parity) {
-  return b.index + (b.sel == 0 ? 0 : (b.sel == 1 ? parity : parity ^ 1));
+// Kinds of a step (the caller's iteration; products that are the same in all of them name no kind).
+enum StepKind { kStepPlain = 0, kStepLate = 1, kStepQuartic = 2 };
+__device__ __forceinline__ int paired_buf(PairedBuf b, int parity, int kind = kStepPlain) {
+  return b.index + (b.sel == 0 ? 0 : ((b.sel == 1 || (b.sel == 3 && kind != kStepQuartic)) ? parity : parity ^ 1));
+}
+// What the epilogue of a product makes of W = A B, element by element; U, P: elements of two further matrices.
+//   kEpiPlain:   C = W, C2 = a I - b W (the next step's polynomial)
+//   kEpiSquare:  C = 2 W - I, C2 = y_w W - y_w / 2 I + y_u U          (U = A = B)
+//   kEpiQuartic: C = W + t_i I + t_u U + t_p P
+//   kEpiShifted: C = W in plain steps, else W + t_i I + t_u U          (t_i, t_u of the call)
+// Step table of a matrix, kCoefs floats a step: a, b, and of a quartic step y_u, y_w, t_i, t_u, t_p.
+enum EpilogueKind { kEpiPlain = 0, kEpiSquare = 1, kEpiQuartic = 2, kEpiShifted = 3 };
+constexpr int kEpiMatrices[4] = {0, 1, 2, 1};       // further matrices of an epilogue
+constexpr int kCoefs = 8;
+struct QuarticCoefs { float y_u, y_w, t_i, t_u, t_p; };
+__device__ __forceinline__ QuarticCoefs quartic_coefs(const float* __restrict__ entry) {
+  return QuarticCoefs{entry[2], entry[3], entry[4], entry[5], entry[6]};
+}
+// (every tile form rounds the same way: W enters last)
+template <int EPI>
+__device__ __forceinline__ float quartic_first(const QuarticCoefs& q, float w, float u, float pm, bool diagonal) {
+  if constexpr (EPI == kEpiSquare) return __builtin_fmaf(2.f, w, diagonal ? -1.f : 0.f);
+  const float shift = diagonal ? q.t_i : 0.f;
+  return __builtin_fmaf(q.t_u, u, EPI == kEpiQuartic ? __builtin_fmaf(q.t_p, pm, shift) : shift) + w;
+}
+__device__ __forceinline__ float quartic_second(const QuarticCoefs& q, float w, float u, bool diagonal) {
+  return __builtin_fmaf(q.y_w, w, __builtin_fmaf(q.y_u, u, diagonal ? -0.5f * q.y_w : 0.f));
 }
 
 struct PlaneGemm {
   __bf16* bufs;             // buffer i, plane set of batch entry z: bufs + i * buf_elems + z * set_elems (plane q: + q * plane_elems)
   int64_t buf_elems, set_elems;
   PairedBuf A, B, C, C2;    // C2.index < 0: no second result
+  PairedBuf B_late;         // index >= 0: replaces B in steps other than plain ones
+  PairedBuf U, P;           // of the epilogue, in the scale u_scale
+  int epi;                  // EpilogueKind; kEpiSquare and kEpiQuartic run in quartic steps only
+  float u_scale, shift_u, shift_i;
   const int* count;         // steps taken by each batch entry (the parity of its paired buffers)
-  const float* coef;        // C2 = coef[2 (count + 1)] I - coef[2 (count + 1) + 1] C of the entry's own table
+  const int* accel;         // steps of each batch entry's table in front of the classical ones, where that decides the kind
+  int early;                // of a step: plain before this one, quartic before accel, late behind it; 0: every step is plain
+  const float* coef;        // entry's own table: C2 = a I - b C of step count + 1, the quartic's coefficients of step count
   int64_t coef_stride;
   int coef_last;            // steps beyond the table take its last entry
   float* errword;           // optional, kErrSlots words per batch entry, kErrStride apart
@@ -63,6 +94,12 @@ struct PlaneGemm {
   int n, n_pad, T;          // T = n_pad / tile
   // fp16 form only (powers of two): 1 / (scale of A's planes * scale of B's), scale of C's planes, scale of C2's
   float in_unscale, c_scale, c2_plane_scale;
+
+  __device__ __forceinline__ int kind_of(int steps, int z) const {
+    if (early == 0) return kStepPlain;
+    const int quartic = accel[z];
+    return quartic == 0 || steps < early ? kStepPlain : (steps < quartic ? kStepQuartic : kStepLate);
+  }
 };
 
 // Element (i, j) of a plane stored by blocks of 32 columns.
@@ -117,25 +154,42 @@ __device__ __forceinline__ void add_chunks(const floatx16& acc, floatx4 (&tot)[4
   }
 }
 
+// Two fp16 planes of four elements, times the inverse of their scale.
+__device__ __forceinline__ floatx4 plane_values(u16x4 hi, u16x4 lo, float unscale) {
+  floatx4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = unscale * (static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(hi[e]))) +
+                      static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(lo[e]))));
+  return v;
+}
+
 // Epilogue of a quarter of a wave's 32 x 32 block of a 64 x 64 tile, rows 8 q + 4 g + e of it: planes of C (and of
 // C2 = c2_scale C + c2_diag I), the mirror image of an off-diagonal tile, the lanes' largest |C - I| and whether all fits.
-template <int NP>
+// EPI: see EpilogueKind; u, pm: the quarter's elements of the further matrices.
+template <int NP, int EPI>
 __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int tj, int z, int wr, int wc, int q, floatx4 sum,
-                                               int parity, float c2_diag, float c2_scale, float& vmax, bool& fits) {
+                                               int parity, int kind, float c2_diag, float c2_scale, const QuarticCoefs& qc,
+                                               floatx4 u, floatx4 pm, float& vmax, bool& fits) {
   const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
   const int i0 = ti * kPlaneSmallTile, j0 = tj * kPlaneSmallTile;
   unsigned short* __restrict__ sets = reinterpret_cast<unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
-  unsigned short* __restrict__ C = sets + paired_buf(p.C, parity) * p.buf_elems;
-  unsigned short* __restrict__ C2 = p.C2.index >= 0 ? sets + paired_buf(p.C2, parity) * p.buf_elems : nullptr;
+  unsigned short* __restrict__ C = sets + paired_buf(p.C, parity, kind) * p.buf_elems;
+  unsigned short* __restrict__ C2 = p.C2.index >= 0 ? sets + paired_buf(p.C2, parity, kind) * p.buf_elems : nullptr;
   const bool off_diag = ti != tj;
   const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
   const int gj = j0 + 32 * wc + l32, gi = i0 + 32 * wr + 8 * q + 4 * g;      // rows gi .. gi + 3
   u16x4 m1[NP], m2[NP];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float v = sum[e] * unscale;
+    const float w = sum[e] * unscale;
     const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
-    if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+    float v = w;
+    if constexpr (EPI == kEpiPlain) {
+      if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
+    } else {
+      v = quartic_first<EPI>(qc, w, u[e], pm[e], diagonal && inside);
+    }
     unsigned short o[3];
     if constexpr (NP == 2) fits = fits && fabsf(v * cs) <= 65504.f;      // (false for a NaN too)
     plane_bits<NP>(v * cs, o);
@@ -151,9 +205,11 @@ __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int t
       m1[s][e] = o[s];
     }
     if (C2 != nullptr) {
-      const float w = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
-      if constexpr (NP == 2) fits = fits && fabsf(w * c2s) <= 65504.f;
-      plane_bits<NP>(w * c2s, o);
+      float x;
+      if constexpr (EPI == kEpiPlain) x = c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f);
+      else x = quartic_second(qc, w, u[e], diagonal && inside);
+      if constexpr (NP == 2) fits = fits && fabsf(x * c2s) <= 65504.f;
+      plane_bits<NP>(x * c2s, o);
 #pragma unroll
       for (int s = 0; s < NP; ++s) {
         if (keep) C2[s * p.plane_elems + at] = o[s];
@@ -179,9 +235,12 @@ __device__ __forceinline__ void plane_epilogue(const PlaneGemm& p, int ti, int t
 // of a work group's 188 at 3072 columns (two results), and a third of every product; in this form 21 us (the clock of the
 // device, which the products keep at its power limit, gives part of that back: 24 x 3072 122 -> 116 ms, 61 x 768 12.4 -> 10.5).  LDS rows of 64 bytes; their 8-byte chunks are permuted by the row (xor with row / 4), so that the 32 rows
 // a wave writes at once fall into different banks.
-template <int NP, class Sum>
+// EPI other than plain (two planes): what a block of 32 x 32 needs of the further matrices is requested while the block before it
+// is formed, transposed as the accumulators are: four elements of a row (the matrices are symmetric).
+template <int NP, int EPI, class Sum>
 __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, int tj, int z, AK_LDS unsigned char* lds,
                                                     Sum sum) {
+  static_assert(EPI == kEpiPlain || NP == 2, "further matrices in two planes");
   constexpr int FR = 3, WC = 2, TILE = kPlaneTile, BLOCK = TILE * 64, SLOT = 6 * BLOCK;      // one plane of the tile
   static_assert(2 * SLOT <= kPlaneLdsBytes, "two planes at a time");
   int tid = threadIdx.x;
@@ -190,14 +249,42 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
   const int lane = tid & 63, wave = tid >> 6;
   const int wr = wave / WC, wc = wave % WC, g = lane >> 5, l32 = lane & 31;
   const int i0 = ti * TILE, j0 = tj * TILE;
-  const int steps = p.count[z], parity = steps & 1;
+  const int steps = p.count[z], parity = steps & 1, kind = NP == 2 ? p.kind_of(steps, z) : static_cast<int>(kStepPlain);
   unsigned short* __restrict__ sets = reinterpret_cast<unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
+  const float* __restrict__ table = p.coef + static_cast<int64_t>(z) * p.coef_stride;
   float c2_diag = 0.f, c2_scale = 0.f;
-  if (p.C2.index >= 0) {
-    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
+  QuarticCoefs qc = {};
+  if constexpr (EPI != kEpiPlain) {
+    if constexpr (EPI == kEpiShifted) {
+      if (kind != kStepPlain) qc = QuarticCoefs{0.f, 0.f, p.shift_i, p.shift_u, 0.f};
+    } else {
+      qc = quartic_coefs(table + kCoefs * min(steps, p.coef_last));
+    }
+  } else if (p.C2.index >= 0) {
+    const float* __restrict__ next = table + kCoefs * min(steps + 1, p.coef_last);
     c2_diag = next[0];
     c2_scale = -next[1];
   }
+  // elements of the further matrices: [parity of the block][matrix][quarter][plane]
+  constexpr int AUX = kEpiMatrices[EPI];
+  u16x4 aux[2][AUX > 0 ? AUX : 1][4][2] = {};
+  auto load_aux = [&](int number) {
+    if constexpr (AUX > 0) {
+      if (number >= 9 || (EPI == kEpiShifted && kind == kStepPlain)) return;
+      const int a = number / 3, b = number % 3;
+      const int gj = j0 + 32 * FR * wc + 32 * b + l32, gi = i0 + 32 * FR * wr + 32 * a + 4 * g;
+#pragma unroll
+      for (int x = 0; x < AUX; ++x) {
+        const unsigned short* from = sets + paired_buf(x == 0 ? p.U : p.P, parity, kind) * p.buf_elems + plane_index(gj, gi, p.n_pad);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          aux[number & 1][x][q][0] = *reinterpret_cast<const u16x4*>(from + 8 * q);
+          aux[number & 1][x][q][1] = *reinterpret_cast<const u16x4*>(from + 8 * q + p.plane_elems);
+        }
+      }
+    }
+  };
+  const float aux_unscale = 1.f / p.u_scale;
   const bool off_diag = ti != tj, plain = off_diag && j0 + TILE <= p.n;       // (ti < tj: then the rows are inside too)
   const float unscale = NP == 2 ? p.in_unscale : 1.f, cs = NP == 2 ? p.c_scale : 1.f, c2s = NP == 2 ? p.c2_plane_scale : 1.f;
   float vmax = 0.f;
@@ -211,21 +298,29 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
   auto pass = [&](auto second_tag, auto s0_tag) {
     constexpr bool SECOND = decltype(second_tag)::value;
     constexpr int s0 = decltype(s0_tag)::value, COUNT = NP - s0 < 2 ? NP - s0 : 2;
+    constexpr bool NEEDS = EPI == kEpiQuartic || EPI == kEpiShifted || (EPI == kEpiSquare && SECOND);      // of the further matrices
+    if constexpr (NEEDS) load_aux(0);
     __syncthreads();
     // a tile on the diagonal or at the border of the matrix
     auto edge_block = [&](auto a_tag, auto b_tag) {
-      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value;
+      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value, number = 3 * a + b;
       const int lj = 32 * FR * wc + 32 * b + l32, gj = j0 + lj;
+      if constexpr (NEEDS) load_aux(number + 1);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int li = 32 * FR * wr + 32 * a + 8 * q + 4 * g, gi = i0 + li;      // rows gi .. gi + 3
         u16x4 m[COUNT];
+        floatx4 u = {}, pm = {};
+        if constexpr (NEEDS) u = plane_values(aux[number & 1][0][q][0], aux[number & 1][0][q][1], aux_unscale);
+        if constexpr (AUX > 1) pm = plane_values(aux[number & 1][AUX - 1][q][0], aux[number & 1][AUX - 1][q][1], aux_unscale);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float v = sum(a, b, 4 * q + e) * unscale;
           const bool inside = gi + e < p.n && gj < p.n, diagonal = gi + e == gj;
           float x = v * cs;
-          if constexpr (SECOND) x = (c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f)) * c2s;
+          if constexpr (EPI != kEpiPlain) x = SECOND ? quartic_second(qc, v, u[e], diagonal && inside) * c2s
+                                                     : quartic_first<EPI>(qc, v, u[e], pm[e], diagonal && inside) * cs;
+          else if constexpr (SECOND) x = (c2_scale * v + ((diagonal && inside) ? c2_diag : 0.f)) * c2s;
           else if constexpr (s0 == 0)
             if (inside && (off_diag || gi + e <= gj)) vmax = gemm_fold_absmax(vmax, v, diagonal, 1);
           if constexpr (NP == 2) fits = fits && fabsf(x) <= 65504.f;      // (false for a NaN too)
@@ -258,8 +353,9 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
     const float scale = SECOND ? c2_scale * (unscale * c2s) : unscale * cs;
     auto block = [&](auto a_tag, auto b_tag) {
 #pragma clang fp contract(off)             // (x rounds before its planes are taken, as in the other tiles: the same bits)
-      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value;
+      constexpr int a = decltype(a_tag)::value, b = decltype(b_tag)::value, number = 3 * a + b;
       const int lj = 32 * FR * wc + 32 * b + l32;
+      if constexpr (NEEDS) load_aux(number + 1);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int li = 32 * FR * wr + 32 * a + 8 * q + 4 * g;
@@ -267,7 +363,17 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
         float x[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = sum(a, b, 4 * q + e) * scale;
-        if constexpr (!SECOND && s0 == 0) {
+        if constexpr (EPI != kEpiPlain) {
+          floatx4 u = {}, pm = {};
+          if constexpr (NEEDS) u = plane_values(aux[number & 1][0][q][0], aux[number & 1][0][q][1], aux_unscale);
+          if constexpr (AUX > 1) pm = plane_values(aux[number & 1][AUX - 1][q][0], aux[number & 1][AUX - 1][q][1], aux_unscale);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = sum(a, b, 4 * q + e) * unscale;
+            x[e] = SECOND ? quartic_second(qc, v, u[e], false) * c2s : quartic_first<EPI>(qc, v, u[e], pm[e], false) * cs;
+          }
+        }
+        if constexpr (EPI == kEpiPlain && !SECOND && s0 == 0) {
           if (p.errword != nullptr) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) vmax_bits = max(vmax_bits, __builtin_bit_cast(uint32_t, x[e]) & 0x7fffffffu);
@@ -307,7 +413,7 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
     if (plain) blocks(block);
     else blocks(edge_block);
     __syncthreads();
-    unsigned short* __restrict__ out = sets + paired_buf(SECOND ? p.C2 : p.C, parity) * p.buf_elems + s0 * p.plane_elems;
+    unsigned short* __restrict__ out = sets + paired_buf(SECOND ? p.C2 : p.C, parity, kind) * p.buf_elems + s0 * p.plane_elems;
     // A wave takes rows 16 (wave + 4 t), t < 3, of every block of 32 columns; all its LDS addresses and all its memory
     // addresses differ by constants of the wave.
     {   // rows gj, columns gi: lane = row l / 4 of 16, 16 bytes l % 4
@@ -353,7 +459,7 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
   using S2 = std::integral_constant<int, 2>;
   pass(std::false_type{}, S0{});
   if constexpr (NP == 3) pass(std::false_type{}, S2{});
-  if (p.C2.index >= 0) {
+  if ((EPI == kEpiPlain || EPI == kEpiSquare) && p.C2.index >= 0) {
     pass(std::true_type{}, S0{});
     if constexpr (NP == 3) pass(std::true_type{}, S2{});
   }
@@ -528,13 +634,14 @@ __device__ __forceinline__ void plane_tile(const PlaneGemm& p, int ti, int tj, i
   }
   wait_vmcnt<0>();                                             // the loads past the last k-tile, before the LDS is released
 
-  plane_epilogue_wide<3>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue_wide<3, kEpiPlain>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
 // The same tile on two fp16 planes per operand.  A k-tile is 16 rows of four plane panels (24 KB per stage, six
 // stages: the loads run four and a half k-tiles ahead), three pairs of planes x 9 matrix instructions per wave:
 // (lo, hi), (hi, hi), (hi, lo).  On entry fa[1] and fb[0] hold the k-tile's first two groups; the first two steps read
 // the other two, the last one the first two groups of the next k-tile.
+template <int EPI>
 __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj, int z) {
   constexpr int WR = 2, WC = 2, FR = 3, FC = 3, NCB = 6, BK = 16, S = 6;
   constexpr int BT = 32 * FR * WR;
@@ -547,8 +654,10 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
   AK_LDS unsigned char* lds = (AK_LDS unsigned char*)dtl_smem;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-  const int steps = p.count[z], parity = steps & 1;
+  const int steps = p.count[z], parity = steps & 1, kind = p.kind_of(steps, z);
   if (p.active[z] == 0 || (steps == 0 && p.C.index == 0)) return;      // (buffer 0 of the first step is given)
+  if ((EPI == kEpiSquare || EPI == kEpiQuartic) && kind != kStepQuartic) return;
+  const PairedBuf B = p.B_late.index >= 0 && kind != kStepPlain ? p.B_late : p.B;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -559,7 +668,7 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   u32x4 rsrc[2];
 #pragma unroll
   for (int P = 0; P < 2; ++P) {
-    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : p.B, parity) * p.buf_elems +
+    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : B, parity, kind) * p.buf_elems +
                                                    static_cast<int64_t>(z) * p.set_elems);
     rsrc[P][0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
     rsrc[P][1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
@@ -674,7 +783,7 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
         for (int r = 0; r < 16; ++r) tot[a][b][r] += acc[a][b][r];
   }
   wait_vmcnt<0>();
-  plane_epilogue_wide<2>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
+  plane_epilogue_wide<2, EPI>(p, ti, tj, z, lds, [&](int a, int b, int r) { return tot[a][b][r]; });
 }
 
 // A 64 x 64 tile (ti <= tj) for groups with too few 192-wide tiles to fill the device: 16 waves, of which group q = wave / 4
@@ -702,8 +811,8 @@ __device__ __forceinline__ void wait_loads(std::integral_constant<int, LOADS>, i
 }
 
 template <int NP, int GROUPS, int G>
-__device__ __forceinline__ void plane_tile_chunks(const PlaneGemm& p, int ti, int tj, int z, int parity, AK_LDS unsigned char* lds,
-                                                  floatx4 (&tot)[4 / GROUPS]) {
+__device__ __forceinline__ void plane_tile_chunks(const PlaneGemm& p, int ti, int tj, int z, int parity, int kind,
+                                                  AK_LDS unsigned char* lds, floatx4 (&tot)[4 / GROUPS]) {
   constexpr int BK = 16, BLOCK = BK * 64, STAGE = 4 * NP * BLOCK, S = kSmallTileStages<NP, GROUPS> / G, LOADS = NP, CHUNK = 256 / BK;
   static_assert((S - 1) * LOADS < 64 && kSmallTileLds<NP, GROUPS> >= G * 16384, "loads in flight; the chunks' sums");
   const int tid = threadIdx.x, lane = tid & 63;
@@ -711,10 +820,11 @@ __device__ __forceinline__ void plane_tile_chunks(const PlaneGemm& p, int ti, in
   const int group = wave >> 2, w = wave & 3, wr = w >> 1, wc = w & 1;
   const int nk = p.n_pad / BK, chunks = (nk + CHUNK - 1) / CHUNK;
   const uint32_t plane_bytes = static_cast<uint32_t>(p.plane_elems) * 2u, colblock_bytes = static_cast<uint32_t>(p.n_pad) * 64u;
+  const PairedBuf B = p.B_late.index >= 0 && kind != kStepPlain ? p.B_late : p.B;
   u32x4 rsrc[2];
 #pragma unroll
   for (int P = 0; P < 2; ++P) {
-    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : p.B, parity) * p.buf_elems +
+    const uint64_t ba = reinterpret_cast<uint64_t>(p.bufs + paired_buf(P == 0 ? p.A : B, parity, kind) * p.buf_elems +
                                                    static_cast<int64_t>(z) * p.set_elems);
     rsrc[P][0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
     rsrc[P][1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
@@ -789,25 +899,61 @@ __device__ __forceinline__ void plane_tile_chunks(const PlaneGemm& p, int ti, in
   }
 }
 
-template <int NP, int GROUPS>
-__device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int tj, int z, int steps, AK_LDS unsigned char* lds,
-                                                 float& vmax, bool& fits) {
+template <int NP, int GROUPS, int EPI>
+__device__ __forceinline__ void plane_tile_small_epi(const PlaneGemm& p, int ti, int tj, int z, int steps, int kind, AK_LDS unsigned char* lds,
+                                                     float& vmax, bool& fits) {
   const int chunks = (p.n_pad + 255) / 256, parity = steps & 1;
-  float c2_diag = 0.f, c2_scale = 0.f;                 // (under way while the product is formed)
-  if (p.C2.index >= 0) {
-    const float* __restrict__ next = p.coef + static_cast<int64_t>(z) * p.coef_stride + 2 * min(steps + 1, p.coef_last);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const float* __restrict__ table = p.coef + static_cast<int64_t>(z) * p.coef_stride;
+  float c2_diag = 0.f, c2_scale = 0.f;                 // (under way while the product is formed, like the further matrices' elements)
+  QuarticCoefs qc = {};
+  constexpr int AUX = kEpiMatrices[EPI], QUADS = 4 / GROUPS;
+  u16x4 aux[AUX > 0 ? AUX : 1][QUADS][2];
+  if constexpr (EPI != kEpiPlain) {
+    if constexpr (EPI == kEpiShifted) qc = QuarticCoefs{0.f, 0.f, p.shift_i, p.shift_u, 0.f};
+    else qc = quartic_coefs(table + kCoefs * min(steps, p.coef_last));
+    const unsigned short* sets = reinterpret_cast<const unsigned short*>(p.bufs) + static_cast<int64_t>(z) * p.set_elems;
+    const int gj = tj * kPlaneSmallTile + 32 * (wave & 1) + (lane & 31);
+    const int gi = ti * kPlaneSmallTile + 32 * ((wave >> 1) & 1) + 8 * (wave >> 2) * QUADS + 4 * (lane >> 5);
+#pragma unroll
+    for (int x = 0; x < AUX; ++x) {
+      const unsigned short* from = sets + paired_buf(x == 0 ? p.U : p.P, parity, kind) * p.buf_elems + plane_index(gj, gi, p.n_pad);
+#pragma unroll
+      for (int k = 0; k < QUADS; ++k) {
+        aux[x][k][0] = *reinterpret_cast<const u16x4*>(from + 8 * k);
+        aux[x][k][1] = *reinterpret_cast<const u16x4*>(from + 8 * k + p.plane_elems);
+      }
+    }
+  } else if (p.C2.index >= 0) {
+    const float* __restrict__ next = table + kCoefs * min(steps + 1, p.coef_last);
     c2_diag = next[0];
     c2_scale = -next[1];
   }
-  floatx4 sum[4 / GROUPS];
-  if (GROUPS == 4 && chunks >= 3) plane_tile_chunks<NP, GROUPS, GROUPS>(p, ti, tj, z, parity, lds, sum);
-  else if (chunks >= 2) plane_tile_chunks<NP, GROUPS, 2>(p, ti, tj, z, parity, lds, sum);
-  else plane_tile_chunks<NP, GROUPS, 1>(p, ti, tj, z, parity, lds, sum);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  floatx4 sum[QUADS];
+  if (GROUPS == 4 && chunks >= 3) plane_tile_chunks<NP, GROUPS, GROUPS>(p, ti, tj, z, parity, kind, lds, sum);
+  else if (chunks >= 2) plane_tile_chunks<NP, GROUPS, 2>(p, ti, tj, z, parity, kind, lds, sum);
+  else plane_tile_chunks<NP, GROUPS, 1>(p, ti, tj, z, parity, kind, lds, sum);
+  const float aux_unscale = 1.f / p.u_scale;
 #pragma unroll
-  for (int k = 0; k < 4 / GROUPS; ++k)
-    plane_epilogue<NP>(p, ti, tj, z, (wave >> 1) & 1, wave & 1, (wave >> 2) * (4 / GROUPS) + k, sum[k], parity, c2_diag, c2_scale,
-                       vmax, fits);
+  for (int k = 0; k < QUADS; ++k) {
+    floatx4 u = {}, pm = {};
+    if constexpr (AUX > 0) u = plane_values(aux[0][k][0], aux[0][k][1], aux_unscale);
+    if constexpr (AUX > 1) pm = plane_values(aux[AUX - 1][k][0], aux[AUX - 1][k][1], aux_unscale);
+    plane_epilogue<NP, EPI>(p, ti, tj, z, (wave >> 1) & 1, wave & 1, (wave >> 2) * QUADS + k, sum[k], parity, kind, c2_diag, c2_scale,
+                            qc, u, pm, vmax, fits);
+  }
+}
+
+template <int NP, int GROUPS>
+__device__ __forceinline__ void plane_tile_small(const PlaneGemm& p, int ti, int tj, int z, int steps, int kind, AK_LDS unsigned char* lds,
+                                                 float& vmax, bool& fits) {
+  if constexpr (NP == 2) {
+    if (p.epi == kEpiSquare) return plane_tile_small_epi<NP, GROUPS, kEpiSquare>(p, ti, tj, z, steps, kind, lds, vmax, fits);
+    if (p.epi == kEpiQuartic) return plane_tile_small_epi<NP, GROUPS, kEpiQuartic>(p, ti, tj, z, steps, kind, lds, vmax, fits);
+    if (p.epi == kEpiShifted && kind != kStepPlain)
+      return plane_tile_small_epi<NP, GROUPS, kEpiShifted>(p, ti, tj, z, steps, kind, lds, vmax, fits);
+  }
+  plane_tile_small_epi<NP, GROUPS, kEpiPlain>(p, ti, tj, z, steps, kind, lds, vmax, fits);
 }
 
 // Tile number -> (ti <= tj), in bands of 8 tile columns, row by row inside a band: the 32 work groups that share an
@@ -833,36 +979,33 @@ __device__ __forceinline__ void decode_banded_tile(int id, int T, int& ti, int& 
 }
 
 // grid: tiles on and above the diagonal x batch, XCD-contiguous
-template <int NP>
+template <int NP, int EPI>
 static __global__ __launch_bounds__(256) void plane_gemm_kernel(PlaneGemm p, int ntiles) {
   const uint32_t id = xcd_contiguous_id(blockIdx.x, gridDim.x);
   const int z = static_cast<int>(id / static_cast<uint32_t>(ntiles));
   int ti, tj;
   decode_banded_tile(static_cast<int>(id - static_cast<uint32_t>(z) * ntiles), p.T, ti, tj);
   if constexpr (NP == 3) plane_tile(p, ti, tj, z);
-  else plane_tile_h2(p, ti, tj, z);
+  else plane_tile_h2<EPI>(p, ti, tj, z);
 }
 
 // planes: 3 (bf16) or 2 (fp16, with the scales of PlaneGemm)
 inline int launch_plane_gemm(const PlaneGemm& p, int planes, int batch, hipStream_t stream) {
   constexpr int kLds = kPlaneLdsBytes;
   if (p.n_pad % kPlaneTile != 0 || p.n_pad > kPlaneMaxDim || p.T * kPlaneTile != p.n_pad || batch <= 0 ||
-      (planes != 2 && planes != 3))
+      (planes != 2 && planes != 3) || (planes == 3 && p.epi != kEpiPlain))
     return AK_ERR_ARG;
+  void (*const kernels[5])(PlaneGemm, int) = {plane_gemm_kernel<2, kEpiPlain>, plane_gemm_kernel<2, kEpiSquare>, plane_gemm_kernel<2, kEpiQuartic>,
+                                              plane_gemm_kernel<2, kEpiShifted>, plane_gemm_kernel<3, kEpiPlain>};
   static bool attr_set = false;     // idempotent; a race sets it twice at worst
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(plane_gemm_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLds) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(plane_gemm_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLds) != hipSuccess)
-      return AK_ERR_LAUNCH;
+    for (auto* k : kernels)
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+        return AK_ERR_LAUNCH;
     attr_set = true;
   }
   const int ntiles = p.T * (p.T + 1) / 2;
-  if (planes == 3)
-    hipLaunchKernelGGL(plane_gemm_kernel<3>, dim3(static_cast<unsigned>(ntiles) * batch), dim3(256), kLds, stream, p, ntiles);
-  else
-    hipLaunchKernelGGL(plane_gemm_kernel<2>, dim3(static_cast<unsigned>(ntiles) * batch), dim3(256), kLds, stream, p, ntiles);
+  hipLaunchKernelGGL(kernels[planes == 3 ? 4 : p.epi], dim3(static_cast<unsigned>(ntiles) * batch), dim3(256), kLds, stream, p, ntiles);
   return check_launch();
 }
 

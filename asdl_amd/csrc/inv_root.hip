@@ -15,6 +15,13 @@
 // With a lower bound l of the spectrum known (from the Lanczos steps, at the least the ridge) the step that raises l most is a
 // larger a with b = a^(p+1) p^p / (p+1)^(p+1), which keeps max m (a - b m)^p = 1: up to 7.4 per step.  root_schedule_kernel
 // decides per matrix whether that is the shorter way.
+// For p = 4 T is a polynomial of the fourth degree there: two products more than a classical step's four, P = 2 U^2 - I with
+// U = 2 M - I and T = t(U, P) + P y(U, P), for a factor of 29 per step where the first degree, held to the same top of the
+// spectrum, has 4.6: 10 or 11 steps and 45 to 51 products where 15 or 16 steps of the first degree took 59 to 63 (98 statistics of
+// 768 to 3072 columns 140 -> 122 ms; the device's power limit holds the products of either near 1.15 PFLOP/s of fp16).
+// Its rounding: T^4 reaches 29, and T^4 M inherits what rounding T^4 does, that much larger than the top of the spectrum it is
+// added to.  Behind the early steps M' is therefore (T^2 M) T^2, and T^2 and X T are formed from D = T - I as D^2 + 2 D + I
+// and X D + X: without either the root lost a factor of 3.5 where the gradient lies, with both it gains (root_schedule_kernel).
 // The first kRootEarly steps stay classical, in the summation order of one fixed kernel per size.  What an ill-conditioned
 // root ends up with is decided there: the rounding of M' perturbs the smallest eigenvalues by about 5e-8, 1 to 2 % of the
 // root at condition 1e6, and every later step's perturbation counts 2.44 times less.  Another order, though as accurate, gives
@@ -95,6 +102,12 @@ static int root_planes(int64_t n, int p, float ridge_eps) {
   return !root_plane_dim(n) ? 0 : (root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3);
 }
 
+// fp32 groups with many wide matrices take 128 x 128 tiles.
+static bool root_split(int64_t n, int64_t batch) {
+  const int64_t t = (n + 127) / 128;
+  return t * t * batch >= 100 && n >= 256 && n % 4 == 0;
+}
+
 // floats of one matrix buffer of a statistic
 static size_t root_buffer_floats(int64_t n, int64_t batch, int np) {
   if (np == 0) return static_cast<size_t>(n) * root_ld(n);
@@ -110,7 +123,7 @@ struct RootState {
   float* partial;   // [RCHUNKS]: sums of squares, then max |M_0 - I|
   float* alpha;     // [kLanczosSteps] the tridiagonal matrix: diagonal,
   float* beta;      // [kLanczosSteps] and beta[j] next to alpha[j - 1], alpha[j]
-  float* coef;      // [2 kRootSteps]: (a, b) of every step
+  float* coef;      // [kRootSteps kCoefs]: a, b and the quartic's coefficients of every step (gemm_planes.hpp)
   float* errword;   // [kErrSlots kErrStride] max |M' - I| of the step under way, folded in by the epilogue of the product that forms M'
   int* lz_dim;      // Lanczos steps that counted (0: all)
   int* pi_iters;
@@ -133,6 +146,7 @@ struct RootGroup {
   int n, ld, batch, p, buffers;
   int z0;               // first matrix of the group in the state arrays
   int np, n_pad, tile;  // planes per matrix: 0 (fp32), 2, 3; tile of the products on planes
+  int quartic;          // steps of the fourth degree are among its products
   float scale_r;
 };
 struct RootGroups {
@@ -445,6 +459,28 @@ __device__ __forceinline__ float int_power(float x, int p) {
   return r;
 }
 
+// Steps of the fourth degree (p = 4): T(m) = sum c_k T_k(2 m - 1), T_k the Chebyshev polynomials.  A row is for spectra in [l, 1],
+// l its first entry, and raises their lower end most: max m T(m)^4 = 1, and where m T(m)^4 has left the rising edge at the
+// lower end it stays at or above what it is at l (rows behind the first) or kRootQuarticTop (the first).  Solved as linear
+// programmes on 3000 points: maximise v with v <= m^(1/4) T(m) on [l, 1] and m^(1/4) T(m) <= 1 on [0, 1].
+constexpr float kRootQuarticTop = 0.85f;
+constexpr int kRootQuarticRows = 13;
+static __constant__ float kRootQuartics[kRootQuarticRows][6] = {
+    {0.f, 1.36251366f, -0.54698689f, 0.24514824f, -0.11936991f, 0.05869484f},
+    {0.075f, 1.35824512f, -0.52173189f, 0.22080282f, -0.09888875f, 0.04157265f},
+    {0.1f, 1.35174999f, -0.49965946f, 0.20083153f, -0.08334540f, 0.03042332f},
+    {0.13f, 1.34376311f, -0.47852429f, 0.18268849f, -0.07021425f, 0.02228694f},
+    {0.17f, 1.33389297f, -0.45611605f, 0.16439933f, -0.05795065f, 0.01577439f},
+    {0.22f, 1.32310502f, -0.43399607f, 0.14724395f, -0.04736485f, 0.01101190f},
+    {0.28f, 1.31212364f, -0.41293058f, 0.13171368f, -0.03858015f, 0.00767336f},
+    {0.36f, 1.29999203f, -0.39071790f, 0.11619157f, -0.03059383f, 0.00512813f},
+    {0.45f, 1.28877730f, -0.37086123f, 0.10307336f, -0.02449238f, 0.00350292f},
+    {0.55f, 1.27841119f, -0.35295083f, 0.09187384f, -0.01977349f, 0.00243930f},
+    {0.65f, 1.26961606f, -0.33804700f, 0.08302710f, -0.01637640f, 0.00178024f},
+    {0.75f, 1.26190359f, -0.32518863f, 0.07574798f, -0.01380495f, 0.00134192f},
+    {0.85f, 1.25508714f, -0.31399054f, 0.06968431f, -0.01182153f, 0.00104061f},
+};
+
 // The smallest eigenvalue of T + ridge I (T: m Lanczos steps) within [lo, hi], from below and to 0.4 %; lo if it lies at or below
 // that.  x lies below the spectrum where every pivot of T + (ridge - x) I is positive (Sturm): two rounds of 64 values of x, one per
 // lane, in geometric progression.
@@ -497,6 +533,10 @@ __device__ __forceinline__ int classical_steps(float m, int p, float a0, float b
 // 6.5e-5 (15), 5.1e-5 (15); 256 x 300, rank 64 6.6e-5 (20), 2.0e-4 (14), 7.8e-5 (14), 6.4e-5 (15), 5.8e-5 (15); 300 x 600, rank 16
 // 1.2e-4 (20), 2.8e-4 (13), 1.5e-4 (14), 1.3e-4 (14), 1.3e-4 (15); 768 x 3072, rank 400 4.9e-5 (21), 1.3e-4 (14), 6.1e-5 (15),
 // 5.4e-5 (15), 4.6e-5 (16).  0.7 is the first that loses nothing.  T^p stays below 12 for the fp16 planes.
+// Steps of the fourth degree with the top at 0.7, 0.8, 0.85, 0.9 and, last, the first degree, on matrices of the first, second and fourth
+// shape and 300 x 600 of rank 16: 5.7e-5 (10), 5.2e-5 (10), 4.9e-5 (10), 4.4e-5 (11), 5.2e-5 (15); 4.1e-5, 3.9e-5, 3.9e-5, 3.7e-5 (10 each), 5.9e-5 (15);
+// 5.2e-5 (10), 4.8e-5 (10), 4.5e-5 (11), 4.2e-5 (11), 4.6e-5 (16); 6.5e-5, 6.2e-5, 6.0e-5, 6.0e-5 (10 each), 1.3e-4 (15).  0.85 is the lowest that
+// loses nothing to speak of at any of 17 shapes from 64 x 50 to 2048 x 2048 (at the worst 3 %; on average it gains 15 %).
 static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, float ridge_eps, int max_iter, float tol, int lanczos_steps) {
   constexpr float kTopMin = 0.7f, kEnd = 0.97f;
   const int z = blockIdx.x, lane = threadIdx.x;
@@ -509,6 +549,7 @@ static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, 
   const float sv = G.st.sv[z], zscale = (1.f + p) / (2.f * sqrtf(nrm2)), ridge = ridge_eps * sv;
   const float a0 = 1.f + 1.f / p, b0 = 1.f / p;
   float ca = a0, cb = b0;                      // of step `lane`
+  int quartic = -1;                            // its row of kRootQuartics
   int k = 0;
   if (ridge_eps >= 1e-7f && p >= 2 && p <= 8 && max_iter >= kRootSteps && sv > 0.f && 0.5f * ridge * zscale > 1e-9f) {
     const int dim = G.st.lz_dim[z];
@@ -525,7 +566,32 @@ static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, 
       l *= int_power(a0 - b0 * l, p);
       if (k == 0) l = fminf(l, first);
     }
-    for (; k < kRootSteps - 1 && l < kEnd; ++k) {
+    int cost = 4 * kRootEarly;                 // products of the schedule (a classical step takes four, one of the fourth degree six)
+    if (g.quartic != 0) {
+      // a row of the table per lane
+      float row[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) row[i] = kRootQuartics[min(lane, kRootQuarticRows - 1)][i];
+      auto raised = [&](float m) {
+        const float u = 2.f * m - 1.f, t2 = 2.f * u * u - 1.f, t3 = 2.f * u * t2 - u, t4 = 2.f * t2 * t2 - 1.f;
+        return m * int_power(row[1] + row[2] * u + row[3] * t2 + row[4] * t3 + row[5] * t4, 4);
+      };
+      const float floor = lane == 0 ? kRootQuarticTop : raised(row[0]);
+      int then = classical_steps(l, p, a0, b0, near, 0);
+      while (k < kRootSteps - 1) {
+        const unsigned long long fits = __ballot(lane < kRootQuarticRows && (lane == 0 || row[0] <= l));
+        const int which = 63 - __clzll(fits);
+        const float next = __shfl(fminf(raised(l), floor), which);
+        const int after = classical_steps(next, p, a0, b0, near, 0);
+        if (6 + 4 * max(after, 1) >= 4 * then) break;
+        if (lane == k) quartic = which;
+        ++k;
+        cost += 6;
+        l = next;
+        then = after;
+      }
+      cost += 4 * max(then, 1);
+    } else for (; k < kRootSteps - 1 && l < kEnd; ++k) {
       // the a in [1 + 1/p, 2.5] that maximises min(f(l), f(1)), f(m) = m (a - b m)^p: two rounds of 64 candidates
       float lo = a0, hi = 2.5f, a = a0, v = -1.f;
 #pragma unroll
@@ -549,16 +615,28 @@ static __global__ __launch_bounds__(64) void root_schedule_kernel(RootGroups G, 
       }
       l = v;
     }
-    if (classical_steps(l, p, a0, b0, near, k) >= classical) {
+    if (g.quartic != 0 ? cost >= 4 * classical : classical_steps(l, p, a0, b0, near, k) >= classical) {
       k = 0;
       ca = a0;
       cb = b0;
+      quartic = -1;
     }
   }
-  float* __restrict__ coef = G.st.coef + z * 2 * kRootSteps;
   if (lane < kRootSteps) {
-    coef[2 * lane] = ca;
-    coef[2 * lane + 1] = cb;
+    float* __restrict__ coef = G.st.coef + (z * kRootSteps + lane) * kCoefs;
+    if (quartic >= 0) {
+      const float* __restrict__ c = kRootQuartics[quartic] + 1;
+      coef[2] = 2.f * c[3];
+      coef[3] = 4.f * c[4];
+      coef[4] = c[0] - c[4] - 1.f;
+      coef[5] = c[1] - c[3];
+      coef[6] = c[2];
+      ca = -1.f;                               // the matrix that the products of such a step start from is U = 2 M - I
+      cb = -2.f;
+    }
+    // the steps behind the early ones take T - I where they may be of the fourth degree
+    coef[0] = g.quartic != 0 && k > 0 && lane >= k ? ca - 1.f : ca;
+    coef[1] = cb;
   }
   if (lane == 0) {
     G.st.accel[z] = k;
@@ -575,7 +653,7 @@ static __global__ __launch_bounds__(256) void root_start_kernel(RootGroups G) {
   if (g.np != 0) return;
   const int n = g.n, ld = g.ld;
   const float zs = G.st.zscale[z], r0 = powf(zs, 1.0f / g.p);
-  const float a = G.st.coef[z * 2 * kRootSteps], b = G.st.coef[z * 2 * kRootSteps + 1];
+  const float a = G.st.coef[z * kCoefs * kRootSteps], b = G.st.coef[z * kCoefs * kRootSteps + 1];
   const int64_t mat = static_cast<int64_t>(n) * ld, buf = mat * g.batch;
   const float* __restrict__ S = g.S + (z - g.z0) * g.strideS;
   float* __restrict__ base = g.bufs + (z - g.z0) * mat;
@@ -611,7 +689,7 @@ static __global__ __launch_bounds__(256) void root_start_planes_kernel(RootState
   const float zs = st.zscale[z];
   const float r0 = NP == 2 ? g.scale_r : powf(zs, 1.0f / g.p);
   const float sm = NP == 2 ? kRootScaleM : 1.f;
-  const float a = st.coef[z * 2 * kRootSteps], b = st.coef[z * 2 * kRootSteps + 1];
+  const float a = st.coef[z * kCoefs * kRootSteps], b = st.coef[z * kCoefs * kRootSteps + 1];
   const int n = g.n, n_pad = g.n_pad;
   const int64_t plane = static_cast<int64_t>(n_pad) * n_pad, set = NP * plane, buf = set * g.batch;
   const float* __restrict__ S = g.S + zl * g.strideS;
@@ -773,13 +851,21 @@ static __global__ void root_stats_kernel(RootGroups G) {
 // ---- products on small tiles ----------------------------------------------------------------------------------------------
 
 enum RootKind { kFp32 = 0, kPlanes2 = 2, kPlanes3 = 3 };
+// A product of a step, C = A B (b_late: of the steps behind the early ones of a matrix with steps of the fourth degree).
+// next.index >= 0: it forms M', and writes the next step's polynomial, or the U that it starts from, and the error.
+struct RootOp {
+  PairedBuf a, b, c, next, b_late{-1, 0}, second{-1, 0}, u{-1, 0}, p{-1, 0};      // second, u, p: of the epilogue
+  int epi = kEpiPlain;
+  float shift_u = 0.f, shift_i = 0.f;
+};
 struct RootJob {
   float* bufs;                  // of its group
   int64_t buf_elems, mat_elems; // floats (planes: 16-bit elements) between buffers, between matrices
-  PairedBuf a, b, c, c2;        // C = A B; c2.index >= 0: the product that forms M', which also writes the next T and the error
+  RootOp op;
   int n, ld;                    // ld: padded size on planes
   int z0, tiles;                // first matrix; tiles of one matrix: on planes those on one side of the diagonal
   int kind;
+  int quartic;                  // steps of the fourth degree are among its group's products
   float scale_r;
 };
 // (What leads a work group to its matrix lies side by side: the matrix's step count is then requested beside the job, whose
@@ -796,8 +882,15 @@ struct RootJobs {
 // (q, w) sums chunk q of every four (two) of block w.  THREADS = 256 (launches without planes): 32 x 32, wave q sums chunk q of
 // every four, so that few columns still spread over the device.  Operands go from memory to registers as the matrix instruction wants them.
 // Bound by latency and, in the 64 x 64 form, by the fp32 matrix instruction (1.7 us per chunk and CU).
-template <int THREADS>
-__device__ __forceinline__ float root_tile_fp32(const GemmParams& p, int ti, int tj, AK_LDS floatx4* part) {
+// EPI other than plain: U, P, the second result and the coefficients in `further`.
+struct RootFurther {
+  const float* U;
+  const float* P;
+  float* second;
+  QuarticCoefs qc;
+};
+template <int THREADS, int EPI>
+__device__ __forceinline__ float root_tile_fp32(const GemmParams& p, const RootFurther& further, int ti, int tj, AK_LDS floatx4* part) {
   constexpr int BLOCKS = THREADS == 256 ? 1 : 4, GROUPS = THREADS / 64 / BLOCKS, TILE = BLOCKS == 4 ? 64 : 32;
   constexpr int U = BLOCKS == 4 ? 2 : 4;                      // steps of 16 k loaded at once
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
@@ -854,6 +947,13 @@ __device__ __forceinline__ float root_tile_fp32(const GemmParams& p, int ti, int
       const float v = tot[r >> 2][r & 3];
       const int gi = i0 + 8 * (q * (4 / GROUPS) + (r >> 2)) + 4 * g + (r & 3), gj = j0 + l32;
       if (gi >= p.M) continue;
+      if constexpr (EPI != kEpiPlain) {
+        const int64_t at = static_cast<int64_t>(gi) * ld + gj;
+        const float u = further.U[at];
+        p.C[at] = quartic_first<EPI>(further.qc, v, u, EPI == kEpiQuartic ? further.P[at] : 0.f, gi == gj);
+        if constexpr (EPI == kEpiSquare) further.second[at] = quartic_second(further.qc, v, u, gi == gj);
+        continue;
+      }
       p.C[static_cast<int64_t>(gi) * ld + gj] = v;
       vmax = gemm_fold_absmax(vmax, v, gi == gj, 1);
       if (p.C2 != nullptr) p.C2[static_cast<int64_t>(gi) * ld + gj] = p.c2_scale * v + (gi == gj ? p.c2_diag : 0.f);
@@ -864,48 +964,58 @@ __device__ __forceinline__ float root_tile_fp32(const GemmParams& p, int ti, int
 
 // A product on planes (fp16 planes: the two roots carry scale_r, every other matrix kRootScaleM).
 __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0, int np, int n, int n_pad, int tile, float scale_r,
-                                                     float* bufs, int64_t buf_elems, PairedBuf a, PairedBuf b, PairedBuf c,
-                                                     PairedBuf c2) {
+                                                     float* bufs, int64_t buf_elems, const RootOp& op, int quartic) {
   PlaneGemm pg;
   pg.bufs = reinterpret_cast<__bf16*>(bufs);
   pg.plane_elems = static_cast<int64_t>(n_pad) * n_pad;
   pg.set_elems = np * pg.plane_elems;
   pg.buf_elems = buf_elems;
-  pg.A = a; pg.B = b; pg.C = c; pg.C2 = c2;
+  pg.A = op.a; pg.B = op.b; pg.C = op.c; pg.C2 = op.epi == kEpiPlain ? op.next : op.second;
+  pg.B_late = op.b_late; pg.U = op.u; pg.P = op.p; pg.epi = op.epi;
+  pg.u_scale = op.u.index == 0 ? scale_r : kRootScaleM;
+  pg.shift_u = op.shift_u; pg.shift_i = op.shift_i;
   pg.count = st.count + z0;
-  pg.coef = st.coef + static_cast<int64_t>(z0) * 2 * kRootSteps;
-  pg.coef_stride = 2 * kRootSteps; pg.coef_last = kRootSteps - 1;
-  pg.errword = c2.index >= 0 ? st.errword + z0 * kErrSlots * kErrStride : nullptr;
+  pg.accel = st.accel + z0;
+  pg.early = quartic != 0 ? kRootEarly : 0;
+  pg.coef = st.coef + static_cast<int64_t>(z0) * kCoefs * kRootSteps;
+  pg.coef_stride = kCoefs * kRootSteps; pg.coef_last = kRootSteps - 1;
+  pg.errword = op.next.index >= 0 ? st.errword + z0 * kErrSlots * kErrStride : nullptr;
   pg.active = st.active + z0;
   pg.overflow = st.ovf + z0;
   pg.n = n; pg.n_pad = n_pad; pg.T = n_pad / tile;
-  const float sa = a.index == 0 ? scale_r : kRootScaleM, sb = b.index == 0 ? scale_r : kRootScaleM;
+  const float sa = op.a.index == 0 ? scale_r : kRootScaleM, sb = op.b.index == 0 ? scale_r : kRootScaleM;
   pg.in_unscale = 1.0f / (sa * sb);
-  pg.c_scale = c.index == 0 ? scale_r : kRootScaleM;
+  pg.c_scale = op.c.index == 0 ? scale_r : kRootScaleM;
   pg.c2_plane_scale = kRootScaleM;
   return pg;
 }
 
-__device__ __forceinline__ bool root_idle(const RootJob& job, int active, int steps) {
-  return active == 0 || (steps == 0 && job.c.index == 0);            // (the first X is written by the start)
+// (with `quartic`, the steps of the matrix's table in front of the classical ones; 0: every step is plain)
+__device__ __forceinline__ int root_step_kind(int steps, int quartic) {
+  return quartic == 0 || steps < kRootEarly ? kStepPlain : (steps < quartic ? kStepQuartic : kStepLate);
+}
+__device__ __forceinline__ bool root_idle(const RootJob& job, int active, int steps, int kind) {
+  return active == 0 || (steps == 0 && job.op.c.index == 0) ||       // (the first X is written by the start)
+         ((job.op.epi == kEpiSquare || job.op.epi == kEpiQuartic) && kind != kStepQuartic);
 }
 
 // The product of matrix zl of a group in fp32; c2_*: of the step `steps` is followed by.
-__device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, const RootJob& job, int zl, int z, int steps) {
+__device__ __forceinline__ GemmParams root_fp32_product(const RootState& st, const RootJob& job, int zl, int z, int steps, int kind) {
   const int parity = steps & 1;
+  const RootOp& op = job.op;
   float* base = job.bufs + zl * job.mat_elems;
   GemmParams p;
-  p.A = base + paired_buf(job.a, parity) * job.buf_elems;
-  p.B = base + paired_buf(job.b, parity) * job.buf_elems;
-  p.C = base + paired_buf(job.c, parity) * job.buf_elems;
+  p.A = base + paired_buf(op.a, parity, kind) * job.buf_elems;
+  p.B = base + paired_buf(op.b_late.index >= 0 && kind != kStepPlain ? op.b_late : op.b, parity, kind) * job.buf_elems;
+  p.C = base + paired_buf(op.c, parity, kind) * job.buf_elems;
   p.lda = p.ldb = p.ldc = job.ld;
   p.M = p.N = job.n;
   p.K = job.ld;
   p.transB = 1;                 // (a symmetric operand is its own transpose)
   p.tile_mode = TILE_ALL;
-  if (job.c2.index >= 0) {
-    const float* next = st.coef + z * 2 * kRootSteps + 2 * min(steps + 1, kRootSteps - 1);
-    p.C2 = base + paired_buf(job.c2, parity) * job.buf_elems;
+  if (op.next.index >= 0) {
+    const float* next = st.coef + (z * kRootSteps + min(steps + 1, kRootSteps - 1)) * kCoefs;
+    p.C2 = base + paired_buf(op.next, parity, kind) * job.buf_elems;
     p.ldc2 = job.ld;
     p.c2_diag = next[0];
     p.c2_scale = -next[1];
@@ -920,8 +1030,8 @@ static __global__ __launch_bounds__(256) void root_split_kernel(RootState st, Ro
   __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 2 * 3 * X3_PLANE];
   const int zl = static_cast<int>(blockIdx.x) / job.tiles, z = job.z0 + zl, local = static_cast<int>(blockIdx.x) - zl * job.tiles;
   const int steps = st.count[z], T = (job.n + X3_BT - 1) / X3_BT;
-  if (root_idle(job, st.active[z], steps)) return;
-  GemmParams p = root_fp32_product(st, job, zl, z, steps);
+  if (root_idle(job, st.active[z], steps, kStepPlain)) return;
+  GemmParams p = root_fp32_product(st, job, zl, z, steps, kStepPlain);
   p.K = job.n;
   p.transB = 0;
   gemm_x3_tile<3, true, 1, 0, false, true>(p, local / T, local % T, 0, (AK_LDS3 unsigned char*)x3_smem);
@@ -972,12 +1082,13 @@ static __global__ __launch_bounds__(THREADS, THREADS == 256 ? 1 : 4) void root_s
   const int zl = (wg - start) / tiles, z = z0 + zl, local = wg - start - zl * tiles;
   const int entry = half * st.total + z;
   const RootJob job = J.j[ji];
+  const int accel = st.accel[z];
   int steps, active;
   if (pending != 0) {
-    const RootProgress r = newton_decide(st, (1 - half) * st.total + z, st.accel[z], tol, max_iter);
+    const RootProgress r = newton_decide(st, (1 - half) * st.total + z, accel, tol, max_iter);
     steps = r.count;
     active = r.active;
-    if (local == 0 && job.c.index != 0 && threadIdx.x == 0) {
+    if (local == 0 && job.op.c.index != 0 && threadIdx.x == 0) {
       st.err[entry] = r.err;
       st.count[entry] = r.count;
       st.active[entry] = r.active;
@@ -987,22 +1098,41 @@ static __global__ __launch_bounds__(THREADS, THREADS == 256 ? 1 : 4) void root_s
     active = st.active[entry];
   }
   steps = __builtin_amdgcn_readfirstlane(steps);
-  if (root_idle(job, __builtin_amdgcn_readfirstlane(active), steps)) return;
+  const int kind = root_step_kind(steps, job.quartic != 0 ? __builtin_amdgcn_readfirstlane(accel) : 0);
+  if (root_idle(job, __builtin_amdgcn_readfirstlane(active), steps, kind)) return;
   float vmax = 0.f;
   bool fits = true;
   if (THREADS == 256 || job.kind == kFp32) {
     const int T = (job.n + (THREADS == 256 ? 31 : 63)) / (THREADS == 256 ? 32 : 64);
-    vmax = root_tile_fp32<THREADS>(root_fp32_product(st, job, zl, z, steps), local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+    const GemmParams p = root_fp32_product(st, job, zl, z, steps, kind);
+    RootFurther f = {};
+    if (job.op.epi == kEpiPlain || (job.op.epi == kEpiShifted && kind == kStepPlain)) {
+      vmax = root_tile_fp32<THREADS, kEpiPlain>(p, f, local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+    } else {
+      float* base = job.bufs + zl * job.mat_elems;
+      f.U = base + paired_buf(job.op.u, steps & 1, kind) * job.buf_elems;
+      f.qc = quartic_coefs(st.coef + (z * kRootSteps + min(steps, kRootSteps - 1)) * kCoefs);
+      if (job.op.epi == kEpiShifted) {
+        f.qc = QuarticCoefs{0.f, 0.f, job.op.shift_i, job.op.shift_u, 0.f};
+        root_tile_fp32<THREADS, kEpiShifted>(p, f, local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+      } else if (job.op.epi == kEpiSquare) {
+        f.second = base + paired_buf(job.op.second, steps & 1, kind) * job.buf_elems;
+        root_tile_fp32<THREADS, kEpiSquare>(p, f, local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+      } else {
+        f.P = base + paired_buf(job.op.p, steps & 1, kind) * job.buf_elems;
+        root_tile_fp32<THREADS, kEpiQuartic>(p, f, local / T, local % T, (AK_LDS floatx4*)dtl_smem);
+      }
+    }
   } else {
     int ti, tj;
     decode_lower_tile(local, ti, tj);
     const PlaneGemm pg = root_plane_gemm(st, job.z0, job.kind == kPlanes2 ? 2 : 3, job.n, job.ld, kPlaneSmallTile, job.scale_r,
-                                         job.bufs, job.buf_elems, job.a, job.b, job.c, job.c2);
+                                         job.bufs, job.buf_elems, job.op, job.quartic);
     constexpr int GROUPS = THREADS == 512 ? 2 : 4;
-    if (job.kind == kPlanes2) plane_tile_small<2, GROUPS>(pg, tj, ti, zl, steps, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
-    else plane_tile_small<3, GROUPS>(pg, tj, ti, zl, steps, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
+    if (job.kind == kPlanes2) plane_tile_small<2, GROUPS>(pg, tj, ti, zl, steps, kind, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
+    else plane_tile_small<3, GROUPS>(pg, tj, ti, zl, steps, kind, (AK_LDS unsigned char*)dtl_smem, vmax, fits);
   }
-  if (job.c2.index >= 0) {
+  if (job.op.next.index >= 0) {
     if (local == 0 && threadIdx.x == 0) root_clear_words(st, (1 - half) * st.total + z);
     root_fold(st, entry, local % kErrSlots, vmax, fits);
   } else if (__ballot(!fits) != 0 && (threadIdx.x & 63) == 0) {
@@ -1015,12 +1145,29 @@ static __global__ __launch_bounds__(THREADS, THREADS == 256 ? 1 : 4) void root_s
 enum RootBuf { R0 = 0, M0 = 2, T0 = 4, B0 = 6 };
 constexpr int kRootMaxSlots = 64;
 constexpr PairedBuf kRin{R0, 1}, kRout{R0, 2}, kMin{M0, 1}, kMout{M0, 2}, kTin{T0, 1}, kTout{T0, 2}, kNone{-1, 0};
-
-struct RootOp { PairedBuf a, b, c, c2; };
+constexpr int kQuarticSlots = 2;        // products in front of the classical ones
 
 // The products of one Newton step by slots: the products of a slot are independent of each other.  T^p by repeated
 // squaring, with the multiplication order of the reference's MatPower for other powers.
-static int root_ops(int p, RootOp (*slots)[2], int* counts, int max_slots) {
+// quartic (p = 4): two products in front that only steps of the fourth degree have, P = 2 U^2 - I with Y = y(U, P), then
+// T = t(U, P) + P Y, which lies where the step's polynomial for the next one will; and behind the early steps M' is not
+// (T^2)^2 M but (T^2 M) T^2.
+static int root_ops(int p, bool quartic, RootOp (*slots)[2], int* counts, int max_slots) {
+  if (quartic) {
+    const PairedBuf b0{B0, 0}, b1{B0 + 1, 0}, t{T0, 3};
+    const RootOp ops[5] = {{kTin, kTin, b0, kNone, kNone, b1, kTin, kNone, kEpiSquare},
+                           {b0, b1, kTout, kNone, kNone, kNone, kTin, b0, kEpiQuartic},
+                           {t, t, b0, kNone, kNone, kNone, t, kNone, kEpiShifted, 2.f, 1.f},
+                           {b0, b0, b1, kNone, kMin},
+                           {b1, kMin, kMout, kTout, b0}};
+    for (int k = 0; k < 5; ++k) {
+      slots[k][0] = ops[k];
+      counts[k] = 1;
+    }
+    slots[kQuarticSlots][1] = RootOp{kRin, t, kRout, kNone, kNone, kNone, kRin, kNone, kEpiShifted, 1.f, 0.f};
+    counts[kQuarticSlots] = 2;
+    return 5;
+  }
   int n = 0;
   auto put = [&](PairedBuf a, PairedBuf b, PairedBuf c, PairedBuf c2) {
     if (n < max_slots) { slots[n][0] = RootOp{a, b, c, c2}; counts[n] = 1; }
@@ -1062,7 +1209,7 @@ static int root_ops(int p, RootOp (*slots)[2], int* counts, int max_slots) {
 static int root_buffers(int p) {
   RootOp slots[kRootMaxSlots][2];
   int counts[kRootMaxSlots];
-  const int n = root_ops(p, slots, counts, kRootMaxSlots);
+  const int n = root_ops(p, false, slots, counts, kRootMaxSlots);       // (steps of the fourth degree take no buffer more)
   int most = kRootFixedBuffers;
   for (int k = 0; k < n; ++k)
     for (int o = 0; o < counts[k]; ++o)
@@ -1071,7 +1218,7 @@ static int root_buffers(int p) {
 }
 
 static size_t root_state_floats(int total) {
-  return (static_cast<size_t>(total) * (4 + RCHUNKS + 2 * kLanczosSteps + 2 * kRootSteps + 2 * kErrSlots * kErrStride + 9) + 63) / 64 * 64;
+  return (static_cast<size_t>(total) * (4 + RCHUNKS + 2 * kLanczosSteps + kCoefs * kRootSteps + 2 * kErrSlots * kErrStride + 9) + 63) / 64 * 64;
 }
 // matrix buffers and Lanczos vectors of a group
 static size_t root_group_matrix_floats(int64_t n, int64_t batch, int np, int buffers) {
@@ -1139,18 +1286,14 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
     RootOp slots[kRootMaxGroups][kRootMaxSlots][2];
     int counts[kRootMaxGroups][kRootMaxSlots], nslots[kRootMaxGroups], most = 0;
     for (int i = 0; i < G.count; ++i) {
-      nslots[i] = root_ops(G.g[i].p, slots[i], counts[i], kRootMaxSlots);
+      nslots[i] = root_ops(G.g[i].p, G.g[i].quartic != 0, slots[i], counts[i], kRootMaxSlots);
       if (nslots[i] < 0) return AK_ERR_ARG;
       most = std::max(most, nslots[i]);
     }
     bool planes = false, small = true;          // products on planes among the small tiles; nothing but small tiles
-    auto split = [&](const RootGroup& g) {      // fp32 groups with many wide matrices
-      const int t = (g.n + 127) / 128;
-      return t * t * static_cast<int64_t>(g.batch) >= 100 && g.n >= 256 && g.n % 4 == 0;
-    };
     for (int i = 0; i < G.count; ++i) {
       const RootGroup& g = G.g[i];
-      const bool on_small = g.np != 0 ? g.tile == kPlaneSmallTile : !split(g);
+      const bool on_small = g.np != 0 ? g.tile == kPlaneSmallTile : !root_split(g.n, g.batch);
       planes = planes || (g.np != 0 && on_small);
       // (with a single slot the first launch of a step is also its last)
       small = small && on_small && nslots[i] > 1;
@@ -1168,24 +1311,29 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
       attr_set = true;
     }
     for (int it = 0; it < iters; ++it) {
-      for (int k = 0; k < most; ++k) {
+      // (where the call's own first steps are known to be early, no products of the fourth degree are launched)
+      const int skip = (phases & 1) != 0 && it < kRootEarly ? kQuarticSlots : 0;
+      for (int slot = 0; slot < most; ++slot) {
         RootJobs J;
         int jobs = 0, blocks = 0, widest = 0;
         for (int i = 0; i < G.count; ++i) {
           const RootGroup& g = G.g[i];
+          const int k = slot + (g.quartic != 0 ? skip : 0);
           if (k >= nslots[i]) continue;
           const int64_t mat = g.np == 0 ? static_cast<int64_t>(g.n) * g.ld : static_cast<int64_t>(g.np) * g.n_pad * g.n_pad;
           for (int o = 0; o < counts[i][k]; ++o) {
-            const RootOp& op = slots[i][k][o];
+            RootOp op = slots[i][k][o];
+            if (skip != 0) op.epi = kEpiPlain;
             if (g.np != 0 && g.tile == kPlaneTile) {
               const int rc = launch_plane_gemm(root_plane_gemm(G.st, g.z0, g.np, g.n, g.n_pad, g.tile, g.scale_r, g.bufs,
-                                                               mat * g.batch, op.a, op.b, op.c, op.c2), g.np, g.batch, s);
+                                                               mat * g.batch, op, g.quartic), g.np, g.batch, s);
               if (rc != AK_OK) return rc;
               continue;
             }
             RootJob job;
             job.bufs = g.bufs; job.buf_elems = mat * g.batch; job.mat_elems = mat;
-            job.a = op.a; job.b = op.b; job.c = op.c; job.c2 = op.c2;
+            job.op = op;
+            job.quartic = g.quartic;
             job.n = g.n; job.ld = g.np == 0 ? g.ld : g.n_pad;
             job.z0 = g.z0;
             job.scale_r = g.scale_r;
@@ -1199,7 +1347,7 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
             if (g.np != 0) {
               const int t = g.n_pad / kPlaneSmallTile;
               put(g.np, t * (t + 1) / 2);
-            } else if (split(g)) {
+            } else if (root_split(g.n, g.batch)) {
               const int t = (g.n + 127) / 128;
               job.kind = kFp32; job.tiles = t * t;
               hipLaunchKernelGGL(root_split_kernel, dim3(job.tiles * g.batch), b256, 0, s, G.st, job);
@@ -1215,7 +1363,7 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
           J.tiles[i] = 1;
           J.z0[i] = 0;
         }
-        const int half = small ? it & 1 : 0, pending = small && it > 0 && k == 0 ? 1 : 0;
+        const int half = small ? it & 1 : 0, pending = small && it > 0 && slot == 0 ? 1 : 0;
         if (!planes)
           hipLaunchKernelGGL(root_small_kernel<256>, dim3(blocks), b256, 16384, s, G.st, J, half, pending, tol, max_iter);
         else if (blocks > 256)
@@ -1285,6 +1433,7 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
     // the same arguments, hence the same answer
     g.scale_r = root_fp16_scale(n[i], p[i], ridge_eps);
     g.np = root_planes(n[i], p[i], ridge_eps);
+    g.quartic = p[i] == 4 && (g.np == 2 || (g.np == 0 && !root_split(n[i], batch[i]))) ? 1 : 0;
     g.buffers = root_buffers(p[i]);
     g.bufs = w;
     g.vec = w + root_group_matrix_floats(n[i], batch[i], g.np, g.buffers);
@@ -1309,7 +1458,7 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
   st.partial = floats(static_cast<int64_t>(total) * RCHUNKS);
   st.alpha = floats(static_cast<int64_t>(total) * kLanczosSteps);
   st.beta = floats(static_cast<int64_t>(total) * kLanczosSteps);
-  st.coef = floats(static_cast<int64_t>(total) * 2 * kRootSteps);
+  st.coef = floats(static_cast<int64_t>(total) * kCoefs * kRootSteps);
   return root_run(phases, iters, G, ridge_eps, max_power_iter, power_tol, max_iter, tol,
                   static_cast<hipStream_t>(stream));
 }

@@ -1680,10 +1680,10 @@ def kron_precond_grouped(items, grad_scale=1.0):
 
 
 # ------------------------------------------------------------------------------ Shampoo inverse root
-ROOT_POLL_AFTER = (15, 2)   # Newton iterations enqueued before the first read of the convergence flags, and between the later
-                            # ones: p = 4 takes 8 to 15 at a ridge of 1e-6 (full-rank to rank-deficient statistics), seldom
-                            # 16 to 19 (a few tiny eigenvalues, more than 1000 columns).  An iteration that nothing needs
-                            # costs its launches, a read drains the device.
+ROOT_POLL_AFTER = (11, 2)   # Newton iterations enqueued before the first read of the convergence flags, and between the later
+                            # ones: p = 4 takes 7 to 11 at a ridge of 1e-6 (full-rank to rank-deficient statistics), seldom
+                            # 12 to 15 (a few tiny eigenvalues).  An iteration that nothing needs costs its launches, a
+                            # read drains the device.
 ROOT_MAX_GROUPS = 16
 
 

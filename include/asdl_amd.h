@@ -405,7 +405,7 @@ int ak_kron_precond_static(const float* Binv, const float* Ainv, float* G, int64
  * below tol, or grows by more than 1.2x (then its previous root is kept), the remaining launches return
  * immediately for it.  Where the ends of the spectrum, as the power iteration saw them, say that it is shorter (ridge_eps >= 1e-7,
  * 2 <= p <= 8, max_iter >= 32), the steps have other coefficients than the reference's, from a lower bound of the spectrum:
- * 15 steps instead of 20 for a rank-deficient statistic at p = 4 and a ridge of 1e-6.
+ * 10 or 11 steps instead of 20 for a rank-deficient statistic at p = 4 and a ridge of 1e-6 (there a step may be of the fourth degree).
  * stats: device float [batch, 4] = {lambda_max, power iterations, newton iterations,
  * final error}.  n >= 2 (the reference returns the identity for n == 1 without any arithmetic).
  * Statistics of 512 columns and more iterate on 16-bit planes written by the product that makes each matrix

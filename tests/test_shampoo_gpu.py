@@ -199,6 +199,33 @@ def test_inv_root_is_as_good_as_the_classical_one_where_the_gradient_lies(m, n, 
     assert here <= 1.3 * classical
 
 
+@pytest.mark.parametrize('n,batch', [(33, 3), (255, 2), (511, 1), (512, 3), (513, 45), (577, 3), (1000, 1)])
+def test_inv_root_steps_of_the_fourth_degree(n, batch):
+    """Rank-deficient statistics beside a well-conditioned one (whose steps stay classical) on fp32 matrices, small tiles and 192-wide tiles
+    (45 of 513 columns): far fewer steps than the first degree takes, each root the one that its matrix gets in a call of its own (on
+    planes bit for bit, whichever tile it takes), and the exact one: 1e-5 for the well-conditioned one, 5 % for the others, whose
+    smallest eigenvalues, 1e-6 of the largest, the rounding of fp32 moves by up to 2e-7 of the largest, a quarter of that in the root."""
+    g = torch.Generator('cuda').manual_seed(n)
+    S = torch.empty(batch + 1, n, n, device='cuda')
+    for b in range(batch):
+        X = torch.randn(max(2, n // (3 + b % 3)), n, generator=g, device='cuda')
+        S[b] = X.T @ X
+    S[batch] = _with_eigenvalues(torch.linspace(1, 2, n, device='cuda'), g)
+    v0 = torch.rand(batch + 1, n, generator=g, device='cuda') * 2 - 1
+    ridged = S.clone()
+    print(f'inv_root fourth degree n={n} batch={batch}', flush=True)
+    root, stats = K.inv_root_newton(ridged, 4, 1e-6, v0)
+    assert (stats[:, 3] <= 1e-6).all() and (stats[:batch, 2] <= 13).all(), stats
+    for b in {0, batch // 2, batch - 1, batch}:
+        alone, st = K.inv_root_newton(S[b:b + 1].clone(), 4, 1e-6, v0[b:b + 1])
+        assert torch.equal(st[0], stats[b]), (b, st, stats[b])
+        if n >= 512:
+            assert torch.equal(alone[0], root[b]) and torch.equal(root[b], root[b].T), b
+        else:
+            assert relerr(alone[0], root[b]) < 1e-6, b
+        assert relerr(root[b], _closed_form_root(ridged[b], 4)) < (1e-5 if b == batch else 5e-2), b
+
+
 @pytest.mark.parametrize('groups,ridge', [
     (((2, 1, 1), (65, 3, 2), (130, 4, 1), (33, 5, 3), (40, 7, 1), (64, 11, 1)), 1e-6),
     (((512, 4, 1), (600, 2, 2), (577, 7, 1), (300, 8, 2), (520, 10, 1)), 1e-6),
