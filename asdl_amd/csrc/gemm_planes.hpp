@@ -89,6 +89,7 @@ struct PlaneGemm {
   int coef_last;            // steps beyond the table take its last entry
   float* errword;           // optional, kErrSlots words per batch entry, kErrStride apart
   const int* active;        // entry z runs only if active[z] != 0
+  const float* settled;     // optional: entry z does not run where settled[z] > 0 (fp16 form)
   int* overflow;            // fp16 form: word z is set when a value of C or C2 does not fit the fp16 range
   int64_t plane_elems;      // n_pad * n_pad
   int n, n_pad, T;          // T = n_pad / tile
@@ -657,6 +658,7 @@ __device__ __forceinline__ void plane_tile_h2(const PlaneGemm& p, int ti, int tj
   const int steps = p.count[z], parity = steps & 1, kind = p.kind_of(steps, z);
   if (p.active[z] == 0 || (steps == 0 && p.C.index == 0)) return;      // (buffer 0 of the first step is given)
   if ((EPI == kEpiSquare || EPI == kEpiQuartic) && kind != kStepQuartic) return;
+  if (p.settled != nullptr && p.settled[z] > 0.f) return;
   const PairedBuf B = p.B_late.index >= 0 && kind != kStepPlain ? p.B_late : p.B;
 
   const int tid = threadIdx.x, lane = tid & 63;

@@ -18,7 +18,8 @@
 // For p = 4 T is a polynomial of the fourth degree there: two products more than a classical step's four, P = 2 U^2 - I with
 // U = 2 M - I and T = t(U, P) + P y(U, P), for a factor of 29 per step where the first degree, held to the same top of the
 // spectrum, has 4.6: 10 or 11 steps and 45 to 51 products where 15 or 16 steps of the first degree took 59 to 63 (98 statistics of
-// 768 to 3072 columns 140 -> 122 ms; the device's power limit holds the products of either near 1.15 PFLOP/s of fp16).
+// 768 to 3072 columns 140 -> 122 ms, 111 without the last step's M' (root_settled_kernel); the device's power limit holds the products of
+// all of them near 1.15 PFLOP/s of fp16).
 // Its rounding: T^4 reaches 29, and T^4 M inherits what rounding T^4 does, that much larger than the top of the spectrum it is
 // added to.  Behind the early steps M' is therefore (T^2 M) T^2, and T^2 and X T are formed from D = T - I as D^2 + 2 D + I
 // and X D + X: without either the root lost a factor of 3.5 where the gradient lies, with both it gains (root_schedule_kernel).
@@ -131,6 +132,7 @@ struct RootState {
   int* count;       // accepted steps
   int* accel;       // steps of the table that are not the classical one
   int* ovf;         // fp16 planes: a product of the step under way left the fp16 range
+  float* settled;   // > 0: the next step is the last one and needs no M' (root_settled_kernel); what bounds its error
   // err, active, count, ovf and errword have a second half, `total` entries further on: root_small_kernel
   int total;
 };
@@ -293,6 +295,7 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     if (part == 0 && tid == 0) {
       st.lz_dim[z] = 0;
       st.active[z] = st.count[z] = 0;
+      st.settled[z] = 0.f;
       root_clear_words(st, z);
       root_clear_words(st, st.total + z);
       st.beta[z * kLanczosSteps] = 0.f;
@@ -748,6 +751,11 @@ static __global__ void root_begin_kernel(RootState st, float tol, int max_iter) 
   st.active[z] = (e > tol && max_iter > 0) ? 1 : 0;
 }
 
+// (with `quartic`, the steps of the matrix's table in front of the classical ones; 0: every step is plain)
+__device__ __forceinline__ int root_step_kind(int steps, int quartic) {
+  return quartic == 0 || steps < kRootEarly ? kStepPlain : (steps < quartic ? kStepQuartic : kStepLate);
+}
+
 // A matrix's own state of the iteration.
 struct RootProgress {
   float err;
@@ -780,13 +788,58 @@ __device__ __forceinline__ RootProgress newton_decide(const RootState& st, int z
 // grid (total), one wave: the decision about the step in half `half`, into the first half; all words are cleared.
 static __global__ __launch_bounds__(64) void newton_decide_kernel(RootState st, int half, float tol, int max_iter) {
   const int z = blockIdx.x;
-  const RootProgress r = newton_decide(st, half * st.total + z, st.accel[z], tol, max_iter);
+  const float last = st.settled[z];
+  const int steps = st.count[half * st.total + z];
+  RootProgress r = newton_decide(st, half * st.total + z, st.accel[z], tol, max_iter);
   if (threadIdx.x != 0) return;
+  if (last > 0.f && r.count > steps) r.err = last;       // (that step had X' alone, which leaves no error behind)
+  st.settled[z] = 0.f;
   st.err[z] = r.err;
   st.count[z] = r.count;
   st.active[z] = r.active;
   root_clear_words(st, z);
   root_clear_words(st, st.total + z);
+}
+
+// The last step in sight: M' = I - (5/8) E^2 - O(E^3), E = M - I, for p = 4, and |(E^2)_ij| is at most the largest squared length of a row
+// of E.  Where that is tol or less the coming step ends the iteration by the very test of the reference, max |M' - I| <= tol (5/8 tol
+// and the rounding of M', 2.4e-7), and its products T^2, T^2 M and M' are left out: three of 45, 11 ms of 98 statistics'
+// 122, for one reading of M, 0.3 ms.
+// grid (blocks of 32 columns, batch), behind a decision, groups on 192-wide tiles.  Bound by the memory: a wave reads 512 consecutive bytes.
+static __global__ __launch_bounds__(256) void root_settled_kernel(RootState st, RootGroup g, float tol) {
+  __shared__ float part[4][32];
+  const int z = g.z0 + blockIdx.y, steps = st.count[z], accel = st.accel[z];
+  const float e = st.err[z];
+  if (st.active[z] == 0 || root_step_kind(steps, accel) != kStepLate || !(e * e <= tol)) return;
+  const int64_t plane = static_cast<int64_t>(g.n_pad) * g.n_pad, set = 2 * plane;
+  const unsigned short* __restrict__ M = reinterpret_cast<const unsigned short*>(g.bufs) + (2 + (steps & 1)) * set * g.batch +
+                                         blockIdx.y * set + static_cast<int64_t>(blockIdx.x) * g.n_pad * 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = 4 * (lane & 7), j = 32 * blockIdx.x + col;
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int i = 8 * wave + (lane >> 3); i < g.n; i += 32) {
+    const u16x4 hi = *reinterpret_cast<const u16x4*>(M + i * 32 + col), lo = *reinterpret_cast<const u16x4*>(M + plane + i * 32 + col);
+    const floatx4 m = plane_values(hi, lo, 1.f / kRootScaleM);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float d = m[k] - (i == j + k ? 1.f : 0.f);
+      sum[k] = __builtin_fmaf(d, d, sum[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    sum[k] += __shfl_xor(sum[k], 8);
+    sum[k] += __shfl_xor(sum[k], 16);
+    sum[k] += __shfl_xor(sum[k], 32);
+    if (lane < 8) part[wave][col + k] = sum[k];
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  const int c = lane & 31;
+  const float largest = wave_max((part[0][c] + part[1][c]) + (part[2][c] + part[3][c]));
+  // (a NaN stays out; too long a row makes the word negative for good: as an unsigned number it is above all others)
+  const bool fits = largest <= tol;
+  if (lane == 0) atomicMax(reinterpret_cast<uint32_t*>(st.settled + z), __builtin_bit_cast(uint32_t, fits ? fmaxf(0.625f * largest, 1e-30f) : -1.f));
 }
 
 // grid (RCHUNKS, total): the caller's fp32 result
@@ -981,6 +1034,7 @@ __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0
   pg.coef_stride = kCoefs * kRootSteps; pg.coef_last = kRootSteps - 1;
   pg.errword = op.next.index >= 0 ? st.errword + z0 * kErrSlots * kErrStride : nullptr;
   pg.active = st.active + z0;
+  pg.settled = quartic != 0 && op.c.index != 0 ? st.settled + z0 : nullptr;
   pg.overflow = st.ovf + z0;
   pg.n = n; pg.n_pad = n_pad; pg.T = n_pad / tile;
   const float sa = op.a.index == 0 ? scale_r : kRootScaleM, sb = op.b.index == 0 ? scale_r : kRootScaleM;
@@ -990,10 +1044,6 @@ __host__ __device__ inline PlaneGemm root_plane_gemm(const RootState& st, int z0
   return pg;
 }
 
-// (with `quartic`, the steps of the matrix's table in front of the classical ones; 0: every step is plain)
-__device__ __forceinline__ int root_step_kind(int steps, int quartic) {
-  return quartic == 0 || steps < kRootEarly ? kStepPlain : (steps < quartic ? kStepQuartic : kStepLate);
-}
 __device__ __forceinline__ bool root_idle(const RootJob& job, int active, int steps, int kind) {
   return active == 0 || (steps == 0 && job.op.c.index == 0) ||       // (the first X is written by the start)
          ((job.op.epi == kEpiSquare || job.op.epi == kEpiQuartic) && kind != kStepQuartic);
@@ -1218,7 +1268,7 @@ static int root_buffers(int p) {
 }
 
 static size_t root_state_floats(int total) {
-  return (static_cast<size_t>(total) * (4 + RCHUNKS + 2 * kLanczosSteps + kCoefs * kRootSteps + 2 * kErrSlots * kErrStride + 9) + 63) / 64 * 64;
+  return (static_cast<size_t>(total) * (4 + RCHUNKS + 2 * kLanczosSteps + kCoefs * kRootSteps + 2 * kErrSlots * kErrStride + 10) + 63) / 64 * 64;
 }
 // matrix buffers and Lanczos vectors of a group
 static size_t root_group_matrix_floats(int64_t n, int64_t batch, int np, int buffers) {
@@ -1371,7 +1421,14 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
         else
           hipLaunchKernelGGL(root_small_kernel<1024>, dim3(blocks), dim3(1024), kLds[0][widest], s, G.st, J, half, pending, tol, max_iter);
       }
-      if (!small) hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, 0, tol, max_iter);
+      if (small) continue;
+      hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, 0, tol, max_iter);
+      if ((phases & 1) != 0 && it < kRootEarly) continue;
+      for (int i = 0; i < G.count; ++i) {
+        const RootGroup& g = G.g[i];
+        if (g.quartic != 0 && g.np == 2 && g.tile == kPlaneTile)
+          hipLaunchKernelGGL(root_settled_kernel, dim3(g.n_pad / 32, g.batch), b256, 0, s, G.st, g, tol);
+      }
     }
     if (small && iters > 0) hipLaunchKernelGGL(newton_decide_kernel, gz, b64, 0, s, G.st, (iters - 1) & 1, tol, max_iter);
   }
@@ -1453,6 +1510,7 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
   st.pi_iters = ints(total);
   st.sv = floats(total);
   st.err = floats(2 * total);
+  st.settled = floats(total);
   st.zscale = floats(total);
   st.errword = floats(static_cast<int64_t>(2 * total) * kErrSlots * kErrStride);
   st.partial = floats(static_cast<int64_t>(total) * RCHUNKS);

