@@ -9,20 +9,19 @@
 // the chain at 1.4 to 1.7 times the error of LAPACK's fp32 potrf + potri; a recursion that multiplied by the inverse of a whole half
 // was at 3 to 8 times that).
 //
-// The steps of all matrices are merged: step k of the chain is one launch for all matrices that have a block k, the products
-// at the end of a group are one launch for all matrices (one work group per tile of any product, descriptor found through a
-// tile -> product map; 128 x 128 split-operand MFMA tiles of gemm_x3.hpp, or the smaller fp32 tiles of gemm_deep.hpp where
-// those would leave the device idle: cg_prefer_deep).
+// The steps of all matrices are merged: step k of the chain is one launch for all matrices that have a block k, and so are the products
+// that are due at the end of a group; products that are not due yet go along with the steps.
 //
 // The plan (descriptor tables, launch sequence) depends on the sizes only; every address in it is an offset into the
 // workspace.  The caller builds it once per size set on the host (ak_chol_group_plan), keeps a device copy, and
 // passes both to every call.
 //
 // Matrices are padded to a multiple of 4 columns with an identity block (the padded rows and columns drop out of the
-// result), which keeps every operand of the split kernel 16-byte aligned.  Only the lower triangle of the input is
+// result), which keeps every operand 16-byte aligned.  Only the lower triangle of the input is
 // read; the strictly upper 128-blocks of W are never touched.
 #include <algorithm>
 #include <cstring>
+#include <utility>
 #include <vector>
 #include "gemm_f32.hpp"
 #include "chol_sweep.hpp"
@@ -30,14 +29,9 @@
 
 namespace ak {
 
-constexpr int64_t CG_MAGIC = 0x3447524c4f4843ll;     // "CHOLGR4"
-constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_PROD = 2, CG_PROD_DEEP = 3, CG_SWEEP = 4, CG_OUT = 5;
+constexpr int64_t CG_MAGIC = 0x3547524c4f4843ll;     // "CHOLGR5"
+constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_PRODUCT = 2, CG_SWEEP = 3, CG_OUT = 4;
 
-// What an operand of a product holds, for the fp16-piece products (bits 4-5 of CgProd::flags: A, bits 6-7: B).  With
-// a = the largest diagonal element of A + lam I, every element is bounded in magnitude: of the Cholesky factor L by sqrt(a),
-// of M = L^-1 by 1 / sqrt(lam).
-constexpr int CG_KIND_L = 1, CG_KIND_M = 2;
-constexpr int CG_SCALE_FLOATS = 4;                    // per matrix: the fp16 switch, the scales of both kinds, padding
 #ifdef AK_TUNING_HOOKS
 static float CG_HALF_MAX_COND = 65536.f;              // tuning builds: ak_debug_set_chol_half_max_cond
 #else
@@ -50,7 +44,7 @@ struct CgHeader {
   int64_t total_bytes;
   int64_t ws_floats;
   int64_t scales_off;       // floats from the workspace base: CG_SCALE_FLOATS per matrix
-  int64_t mats_off, steps_off, tasks_off, prods_off, map_off;      // byte offsets of the tables inside the plan
+  int64_t mats_off, steps_off, tasks_off, tiles_off;      // byte offsets of the tables inside the plan (tiles: of the sweep)
   int32_t count, nsteps, copy_blocks, out_blocks;
   double us;                // estimated time of one call (cg_build)
 };
@@ -62,18 +56,7 @@ struct CgMat {
 };
 
 struct CgStep {
-  int32_t type, first, count, grid;    // chain: first task, step k, tasks; products: first product, products, tiles
-  int32_t first_tile, pad0;            // products: where the step's tile -> product map starts
-};
-
-struct CgProd {
-  int64_t a_off, b_off, c_off;
-  int32_t lda, ldb, ldc;
-  int32_t M, N, K;
-  int32_t flags, kmode, tile_mode;
-  float alpha, beta;
-  int32_t mat;
-  int32_t first_tile, tiles_m, tiles_n;
+  int32_t type, first, count, grid;    // chain: first task, step k, tasks
 };
 
 struct CgArgs {
@@ -213,164 +196,52 @@ static __global__ __launch_bounds__(256) void cg_out_kernel(CgArgs a, int count)
   }
 }
 
-// Tile (ti, tj) number `local` of a product, longest contraction first where the range depends on the tile.
-__device__ __forceinline__ void cg_decode_tile(const CgProd& d, int local, int& ti, int& tj) {
-  if (d.tile_mode != TILE_ALL) {     // tiles on and below the diagonal, row by row (K_GE_MAXIJ: longest first)
-    ti = static_cast<int>((__builtin_sqrtf(8.f * static_cast<float>(local) + 1.f) - 1.f) * 0.5f);
-    while ((ti + 1) * (ti + 2) / 2 <= local) ++ti;
-    while (ti * (ti + 1) / 2 > local) --ti;
-    tj = local - ti * (ti + 1) / 2;
-    return;
-  }
-  if (d.kmode == K_GE_J) {           // k >= column tile: first column first
-    tj = local / d.tiles_m;
-    ti = local % d.tiles_m;
-  } else {
-    ti = local / d.tiles_n;
-    tj = local % d.tiles_n;
-  }
-}
-
-// One work group per 128 x 128 tile of any product of the step; tile_map[w] = the product of work group w.
-static __global__ __launch_bounds__(256, 2) void cg_prod_kernel(CgArgs a, const CgProd* __restrict__ prods,
-                                                             const int32_t* __restrict__ tile_map) {
-  __shared__ __attribute__((aligned(16))) unsigned char x3_smem[2 * 3 * X3_PLANE];
-  const int w = blockIdx.x;
-  const CgProd d = prods[tile_map[w]];
-  // (a skipped matrix's work area holds whatever the last call left there; its steps still run and touch nothing else)
-  int ti, tj;
-  cg_decode_tile(d, w - d.first_tile, ti, tj);
-  GemmParams p;
-  p.A = a.ws + d.a_off;
-  p.B = a.ws + d.b_off;
-  p.C = a.ws + d.c_off;
-  p.C_list = nullptr;
-  p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
-  p.sA = p.sB = p.sC = 0;
-  p.M = d.M; p.N = d.N; p.K = d.K;
-  p.transA = 0; p.transB = 1;
-  p.alpha = d.alpha; p.beta = d.beta;
-  p.kmode = d.kmode; p.tile_mode = d.tile_mode;
-  p.active = nullptr; p.active_stride = 0;
-  p.split = 3;
-  p.scaleA = p.scaleB = 1.f;
-  const float* __restrict__ sc = a.scales + static_cast<int64_t>(d.mat) * CG_SCALE_FLOATS;
-  if (sc[0] != 0.f) {
-    // fp16 pieces: two per operand element, three matrix instructions per product instead of six
-    p.scaleA = sc[(d.flags >> 4) & 3];
-    p.scaleB = sc[(d.flags >> 6) & 3];
-    p.alpha = d.alpha / (p.scaleA * p.scaleB);      // powers of two: exact
-    if (d.beta != 0.f) gemm_x3_tile<2, false, 1, 1, true, false, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
-    else gemm_x3_tile<2, false, 1, 1, true>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
-  } else {
-    gemm_x3_tile<3, false, 1, 1>(p, ti, tj, 0, (AK_LDS3 unsigned char*)x3_smem);
-  }
-}
-
-// The same for the steps whose 128 x 128 tiles would leave most of the device idle: deep fp32 tiles of 64 x 64 (gemm_deep.hpp).
-static __global__ __launch_bounds__(256, 2) void cg_prod_deep_kernel(CgArgs a, const CgProd* __restrict__ prods,
-                                                                  const int32_t* __restrict__ tile_map) {
-  __shared__ __attribute__((aligned(16))) float lds[deep_lds_floats<64, 64, 128>()];
-  const int w = blockIdx.x;
-  const CgProd d = prods[tile_map[w]];
-  int ti, tj;
-  cg_decode_tile(d, w - d.first_tile, ti, tj);
-  GemmParams p;
-  p.A = a.ws + d.a_off;
-  p.B = a.ws + d.b_off;
-  p.C = a.ws + d.c_off;
-  p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
-  p.M = d.M; p.N = d.N; p.K = d.K;
-  p.transA = 0; p.transB = 1;
-  p.alpha = d.alpha; p.beta = d.beta;
-  p.kmode = d.kmode; p.tile_mode = d.tile_mode;
-  gemm_deep_tile<64, 64, 128>(p, ti, tj, 0, lds);
-}
-
 // ---- host: the plan ------------------------------------------------------------------------------------------
 
 static inline int64_t cg_align64(int64_t x) { return (x + 63) / 64 * 64; }
 
-static int64_t cg_tiles(const CgProd& p) {
-  return p.tile_mode == TILE_ALL ? static_cast<int64_t>(p.tiles_m) * p.tiles_n
-                                 : static_cast<int64_t>(p.tiles_m) * (p.tiles_m + 1) / 2;
+// Products in launches of their own, on 128 x 128 tiles of split operands or on deep fp32 tiles of 64 x 64: what the rule between sweep and
+// chain was measured with (cg_build).
+struct CgShape {
+  int64_t tiles, deep_tiles, K;
+};
+static void cg_add_shape(std::vector<CgShape>& ps, int64_t M, int64_t N, int64_t K, bool lower) {
+  if (M <= 0 || N <= 0) return;
+  const int64_t m = (M + 127) / 128, n = (N + 127) / 128, dm = (M + 63) / 64, dn = (N + 63) / 64;
+  ps.push_back(lower ? CgShape{m * (m + 1) / 2, dm * (dm + 1) / 2, K} : CgShape{m * n, dm * dn, K});
 }
-
-// Tiles of the deep kernel instead of 128 x 128.
-static void cg_make_deep(CgProd& p) {
-  p.tiles_m = (p.M + 63) / 64;
-  p.tiles_n = (p.N + 63) / 64;
-}
-
-// Microseconds of the products of one super-step (cg_prefer_deep), its launch not counted.
-static double cg_product_us(const std::vector<CgProd>& ps, bool deep) {
-  double longest = 0, sum = 0;
-  for (const CgProd& p : ps) {
-    CgProd q = p;
-    if (deep) cg_make_deep(q);
-    const double c = deep ? (p.K + 127) / 128 : (p.K + 31) / 32;
+// Microseconds of one launch: as long as its longest tile, or as its work spread over the CUs.
+static double cg_shapes_us(const std::vector<CgShape>& ps) {
+  if (ps.empty()) return 0.0;
+  double longest = 0, sum = 0, deep_longest = 0, deep_sum = 0;
+  for (const CgShape& p : ps) {
+    const double c = static_cast<double>((p.K + 31) / 32), d = static_cast<double>((p.K + 127) / 128);
     longest = std::max(longest, c);
-    sum += c * static_cast<double>(cg_tiles(q));
+    sum += c * static_cast<double>(p.tiles);
+    deep_longest = std::max(deep_longest, d);
+    deep_sum += d * static_cast<double>(p.deep_tiles);
   }
-  return deep ? 2.0 * std::max(longest, sum / 256) : std::max(1.6 * longest, 1.05 * sum / 256);
+  return 4 + std::min(2.0 * std::max(deep_longest, deep_sum / 256), std::max(1.6 * longest, 1.05 * sum / 256));
 }
-
-// Which kernel a super-step's products take.  The split kernel's 128 x 128 tiles have three times the rate once they
-// fill the device (about 1 us per k-tile of 32 and CU), but a tile takes 1.6 us per k-tile however few there are; the
-// deep tiles take 2 us per chunk of 128 k.  The step is as long as its longest tile or as its work spread over the CUs.
-static bool cg_prefer_deep(const std::vector<CgProd>& ps) { return cg_product_us(ps, true) < cg_product_us(ps, false); }
-
-// C = beta C + alpha A B^T
-static CgProd cg_prod(int mat, int kind_a, int kind_b, int M, int N, int K, float alpha, int64_t a, int lda,
-                      int64_t b, int ldb, float beta, int64_t c, int ldc, int kmode, int tile_mode) {
-  CgProd p;
-  std::memset(&p, 0, sizeof(p));
-  p.a_off = a; p.b_off = b; p.c_off = c;
-  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
-  p.M = M; p.N = N; p.K = K;
-  p.flags = (kind_a << 4) | (kind_b << 6); p.kmode = kmode; p.tile_mode = tile_mode;
-  p.alpha = alpha; p.beta = beta;
-  p.mat = mat;
-  p.tiles_m = (M + 127) / 128;
-  p.tiles_n = (N + 127) / 128;
-  return p;
+// Of the products at the end of the group of columns [c0, c1) of one matrix; of the tiles of step k.
+static void cg_group_shapes(std::vector<CgShape>& ps, int64_t dp, int64_t c0, int64_t c1) {
+  const int64_t width = c1 - c0, below = dp - c1;
+  cg_add_shape(ps, below, below, width, true);
+  cg_add_shape(ps, below, width, width, false);
+  cg_add_shape(ps, below, c0, width, false);
+  cg_add_shape(ps, width, c0, width, false);
+  cg_add_shape(ps, width, width, width, true);
+  cg_add_shape(ps, c0, c0, width, true);
 }
-
-// The products at the end of the group of columns [c0, c1) of one matrix: X -+ V V^T.  Rows and columns of the group, whose
-// old values have become V, are formed anew.
-static void cg_group_products(std::vector<CgProd>& ps, int mat, int64_t w, int64_t v, int dp, int c0, int c1) {
-  const int width = c1 - c0, below = dp - c1;
-  auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
-  auto put = [&](int kind_a, int kind_b, int r, int M, int c, int N, float alpha, float beta, int kmode, int tile_mode) {
-    if (M <= 0 || N <= 0) return;
-    ps.push_back(cg_prod(mat, kind_a, kind_b, M, N, width, alpha, v + static_cast<int64_t>(r) * CC_VLD, CC_VLD,
-                         v + static_cast<int64_t>(c) * CC_VLD, CC_VLD, beta, at(r, c), dp, kmode, tile_mode));
-  };
-  put(CG_KIND_L, CG_KIND_L, c1, below, c1, below, -1.f, 1.f, K_FULL, TILE_LOWER);
-  put(CG_KIND_L, CG_KIND_M, c1, below, c0, width, -1.f, 0.f, K_GE_J, TILE_ALL);
-  put(CG_KIND_L, CG_KIND_M, c1, below, 0, c0, -1.f, 1.f, K_FULL, TILE_ALL);
-  put(CG_KIND_M, CG_KIND_M, c0, width, 0, c0, 1.f, 0.f, K_GE_I, TILE_ALL);
-  put(CG_KIND_M, CG_KIND_M, c0, width, c0, width, 1.f, 0.f, K_GE_MAXIJ, TILE_LOWER);
-  put(CG_KIND_M, CG_KIND_M, 0, c0, 0, c0, 1.f, 1.f, K_FULL, TILE_LOWER);
-}
-
-// The tiles of step k of one matrix (chol_chain.hpp) as products of 128 columns of V, for launches of their own.
-static void cg_step_products(std::vector<CgProd>& ps, int mat, int64_t w, int64_t v, int64_t e, int dp, int k, int g0, int ge) {
-  const int c0 = g0 * LEAF, c1 = (k + 1) * LEAF, c2 = std::min(ge * LEAF, dp);
-  auto at = [&](int r, int c) { return w + static_cast<int64_t>(r) * dp + c; };
-  auto row = [&](int r) { return v + static_cast<int64_t>(r) * CC_VLD + (k - g0) * LEAF; };
-  auto put = [&](int kind_b, int r, int M, int c, int N, float beta, int64_t to, int ld, int tile_mode) {
-    if (M > 0 && N > 0)
-      ps.push_back(cg_prod(mat, CG_KIND_L, kind_b, M, N, LEAF, -1.f, row(r), CC_VLD, row(c), CC_VLD, beta, to, ld, K_FULL, tile_mode));
-  };
-  put(CG_KIND_L, c1, c2 - c1, c1, c2 - c1, 1.f, at(c1, c1), dp, TILE_LOWER);
-  put(CG_KIND_L, c2, dp - c2, c1, c2 - c1, 1.f, at(c2, c1), dp, TILE_ALL);
-  put(CG_KIND_L, c2, std::min(LEAF, dp - c2), c2, std::min(LEAF, dp - c2), 1.f, at(c2, c2), dp, TILE_LOWER);
-  put(CG_KIND_M, c1, c2 - c1, 0, c0, 1.f, at(c1, 0), dp, TILE_ALL);
+static void cg_step_shapes(std::vector<CgShape>& ps, int64_t dp, int k, int g0, int ge) {
+  const int64_t c0 = static_cast<int64_t>(g0) * LEAF, c1 = static_cast<int64_t>(k + 1) * LEAF, c2 = std::min<int64_t>(static_cast<int64_t>(ge) * LEAF, dp);
+  const int64_t next = std::min<int64_t>(LEAF, dp - c2);
+  cg_add_shape(ps, c2 - c1, c2 - c1, LEAF, true);
+  cg_add_shape(ps, dp - c2, c2 - c1, LEAF, false);
+  cg_add_shape(ps, next, next, LEAF, true);
+  cg_add_shape(ps, c2 - c1, c0, LEAF, false);
   for (int r = k + 1; r < ge; ++r)
-    for (int i = g0; i <= k; ++i)
-      put(CG_KIND_M, r * LEAF, std::min(LEAF, dp - r * LEAF), i * LEAF, LEAF, i < k ? 1.f : 0.f,
-          e + static_cast<int64_t>((r - g0) * (r - g0 - 1) / 2 + i - g0) * ST_TILE, LEAF, TILE_ALL);
+    for (int i = g0; i <= k; ++i) cg_add_shape(ps, std::min<int64_t>(LEAF, dp - static_cast<int64_t>(r) * LEAF), LEAF, LEAF, false);
 }
 
 struct CgPlan {
@@ -378,8 +249,6 @@ struct CgPlan {
   std::vector<CgMat> mats;
   std::vector<CgStep> steps;
   std::vector<CcTask> tasks;
-  std::vector<CgProd> prods;
-  std::vector<int32_t> tile_map;
   std::vector<SwTask> sweep_leaves, sweep_tiles;
 };
 
@@ -447,7 +316,7 @@ static void cg_build_sweep(const int64_t* dims, int count, CgPlan& plan) {
       if (blocks(m) > k + 1) ++leaves;
       if (k >= 0 && blocks(m) > k) tiles += blocks(m) * (blocks(m) + 1) / 2;
     }
-    plan.steps.push_back(CgStep{CG_SWEEP, k, leaves, leaves + tiles, 0, 0});
+    plan.steps.push_back(CgStep{CG_SWEEP, k, leaves, leaves + tiles});
   }
   CgHeader& h = plan.h;
   std::memset(&h, 0, sizeof(h));
@@ -458,8 +327,8 @@ static void cg_build_sweep(const int64_t* dims, int count, CgPlan& plan) {
   int64_t b = cg_align(sizeof(CgHeader), 64);
   h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
   h.tasks_off = b; b = cg_align(b + plan.sweep_leaves.size() * sizeof(SwTask), 64);
-  h.prods_off = b; b = cg_align(b + plan.sweep_tiles.size() * sizeof(SwTask), 64);
-  h.mats_off = h.map_off = b;
+  h.tiles_off = b; b = cg_align(b + plan.sweep_tiles.size() * sizeof(SwTask), 64);
+  h.mats_off = b;
   h.total_bytes = b;
 }
 
@@ -469,8 +338,43 @@ static int CG_FORCE = 0;               // tuning builds: 1 the sweep, 2 the chai
 constexpr int CG_FORCE = 0;
 #endif
 
-// The chain's tables.  Returns its estimated time: 26 us a step, or 9 and 18 per round of tiles (of panels alone: 9) where that is
-// more, the products by cg_product_us, the copies by their bytes.
+// The tiles of a lower triangle along a Z curve: neighbours in the list read the same rows of V.
+static std::vector<std::pair<int, int>> cg_blocked_tiles(int nb) {
+  std::vector<std::pair<int, int>> tiles;
+  int side = 1;
+  while (side < nb) side *= 2;
+  for (int64_t z = 0; z < static_cast<int64_t>(side) * side; ++z) {
+    int bi = 0, bj = 0;
+    for (int bit = 0; (1 << bit) < side; ++bit) {
+      bj |= static_cast<int>(z >> (2 * bit) & 1) << bit;
+      bi |= static_cast<int>(z >> (2 * bit + 1) & 1) << bit;
+    }
+    if (bi < nb && bj <= bi) tiles.emplace_back(bi, bj);
+  }
+  return tiles;
+}
+// Appends a list to the tasks of the launch that starts at task `first` so that every XCD (work group number modulo 8) gets a
+// contiguous eighth of it, whose rows of V its L2 then holds (the 42 factors of ResNet-18 3030 -> 2855 us).
+static void cg_append_by_xcd(std::vector<CcTask>& tasks, int first, const std::vector<CcTask>& list) {
+  const size_t n = list.size(), base = tasks.size() - static_cast<size_t>(first);
+  size_t next[8], at = 0;
+  for (size_t x = 0; x < 8; ++x) {
+    next[x] = at;
+    at += (n + 7 - (x + 8 - base % 8) % 8) / 8;          // places of the list on this XCD
+  }
+  for (size_t i = 0; i < n; ++i) {
+    const size_t x = (base + i) % 8;
+    tasks.push_back(list[next[x]++]);
+  }
+}
+
+constexpr size_t kProductChunk = 16;   // tiles that stay together
+// us of a CU: a tile of a group's products in a step's launch (18 measured), in one of its own (16 to 20), a tile of a step in one of its own;
+// what a step's launch takes along without being longer for it: its leaf takes 26.  (Tiles beyond that in the steps' launches, each of which
+// asks for a whole CU: 24 x 1100 605 -> 625 us, ResNet-18's step, beside the loss backward pass, 1 % more.)
+constexpr double kProductUs = 18.0, kOwnProductUs = 16.0, kStepUs = 5.0, kBesideUs = 26.0;
+// The chain's tables.  Returns the time that the rule goes by: 26 us a step, or 9 and 18 per round of tiles (of panels alone: 9) where that is
+// more, all products in launches of their own (cg_shapes_us), the copies by their bytes.
 static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
   struct Mat { int64_t w, v, e, m; int d, dp, nb; };
   std::vector<Mat> mats(count);
@@ -496,93 +400,124 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
     bytes += 2.5 * 4 * x.d * x.d;
   }
   double us = 24 + bytes / 3.5e6;
-  // one launch of products, if any: its estimated time; written to the plan or not
-  auto products = [&](std::vector<CgProd> ps, bool write) {
-    if (ps.empty()) return 0.0;
-    CgStep pr{CG_PROD, static_cast<int>(plan.prods.size()), static_cast<int>(ps.size()), 0, static_cast<int>(plan.tile_map.size()), 0};
-    const bool deep = cg_prefer_deep(ps);
-    if (deep) {
-      pr.type = CG_PROD_DEEP;
-      for (CgProd& p : ps) cg_make_deep(p);
-    }
-    const double time = 4 + cg_product_us(ps, deep);
-    if (!write) return time;
-    // longest contraction first: the long tiles start early, the short ones (those that start in the middle of it) fill the tail
-    auto depth = [](const CgProd& p) { return p.kmode == K_FULL ? 2 * p.K : p.K; };
-    std::stable_sort(ps.begin(), ps.end(), [&](const CgProd& x, const CgProd& y) { return depth(x) > depth(y); });
-    int64_t n = 0;
-    for (size_t i = 0; i < ps.size(); ++i) {
-      ps[i].first_tile = static_cast<int>(n);
-      const int64_t mine = cg_tiles(ps[i]);
-      n += mine;
-      plan.tile_map.insert(plan.tile_map.end(), static_cast<size_t>(mine), static_cast<int32_t>(i));
-    }
-    pr.grid = static_cast<int>(n);
-    plan.prods.insert(plan.prods.end(), ps.begin(), ps.end());
-    plan.steps.push_back(pr);
-    return time;
+  plan.steps.push_back(CgStep{CG_COPY, 0, count, copy_blocks});
+  auto each = [&](int k, auto&& f) {             // the matrices at work in step k
+    for (int i = 0; i < count; ++i)
+      if (mats[i].nb > std::max(k, 0)) f(i, mats[i]);
   };
-  plan.steps.push_back(CgStep{CG_COPY, 0, count, copy_blocks, 0, 0});
+  auto group_of = [](int k) { return std::max(k, 0) / CG_GROUP * CG_GROUP; };
+  std::vector<char> split(nb_max, 0);            // V alone in a step's launch, its tiles in another one
+  std::vector<double> load(nb_max, 0.0);         // us of one CU that the work groups of a step's launch take
+  std::vector<double> alone(nb_max, 26.0);       // the launch without products
+  std::vector<double> apart(nb_max, 0.0);        // the launch of the tiles
+  double rule_us = us + 18;
+  for (int k = 0; k < nb_max; ++k) {
+    int tiles = 0, rows = 0, leaves = 0;
+    std::vector<CgShape> ps;
+    const int g0 = group_of(k);
+    each(k, [&](int, const Mat& x) {
+      const int ge = std::min(g0 + CG_GROUP, x.nb), left = ge - k - 1;
+      rows += x.nb;
+      tiles += left * (x.nb - k - 1) - left * (left - 1) / 2 + left * (k + 1);
+      leaves += k + 1 < x.nb ? 1 : 0;
+      if (left > 0) cg_step_shapes(ps, x.dp, k, g0, ge);
+    });
+    const double panels = std::max(26.0, 9.0 + 9.0 * rows / 256), fused = std::max(26.0, 9.0 + 18.0 * tiles / 256);
+    apart[k] = 4.0 + kStepUs * std::max(1.0, tiles / 256.0);
+    split[k] = tiles > 0 && (panels + apart[k] < fused || CG_FORCE == 3) && CG_FORCE != 4;
+    alone[k] = split[k] || tiles == 0 ? panels : fused;
+    load[k] = 26.0 * leaves + (split[k] || tiles == 0 ? 9.0 * rows : 15.0 * tiles);
+    rule_us += tiles == 0 ? panels : std::min(fused, panels + cg_shapes_us(ps));
+    ps.clear();
+    each(k, [&](int, const Mat& x) {
+      const int ge = std::min(g0 + CG_GROUP, x.nb);
+      if (k + 1 == ge) cg_group_shapes(ps, x.dp, static_cast<int64_t>(g0) * LEAF, std::min<int64_t>(static_cast<int64_t>(ge) * LEAF, x.dp));
+    });
+    rule_us += cg_shapes_us(ps);
+  }
+  std::vector<std::vector<CcTask>> beside(nb_max);      // products that step k's launch takes along
   for (int k = -1; k < nb_max; ++k) {
-    CgStep st{CG_CHAIN, static_cast<int>(plan.tasks.size()), k, 0, 0, 0};
-    auto each = [&](auto&& f) {
-      for (int i = 0; i < count; ++i)
-        if (mats[i].nb > std::max(k, 0)) f(i, mats[i]);
-    };
-    auto put = [&](int i, int kind, int bi, int bj) {
+    CgStep st{CG_CHAIN, static_cast<int>(plan.tasks.size()), k, 0};
+    const int g0 = group_of(k);
+    auto task = [&](int i, int kind, int bi, int bj) {
       const Mat& x = mats[i];
-      const int g0 = std::max(k, 0) / CG_GROUP * CG_GROUP;
-      plan.tasks.push_back(CcTask{x.w, x.v, x.e, x.m, i, x.d, x.dp, x.nb, kind, bi, bj, g0});
+      return CcTask{x.w, x.v, x.e, x.m, i, x.d, x.dp, x.nb, kind, bi, bj, g0};
     };
-    each([&](int i, const Mat& x) {
+    auto put = [&](int i, int kind, int bi, int bj) { plan.tasks.push_back(task(i, kind, bi, bj)); };
+    each(k, [&](int i, const Mat& x) {
       if (k + 1 < x.nb) put(i, CC_LEAF, k + 1, k + 1);
     });
-    const int g0 = std::max(k, 0) / CG_GROUP * CG_GROUP;
-    std::vector<CgProd> ps;
-    bool split = false;
-    if (k >= 0) {
-      int tiles = 0, rows = 0;
-      each([&](int i, const Mat& x) {
-        const int ge = std::min(g0 + CG_GROUP, x.nb), left = ge - k - 1;
-        rows += x.nb;
-        tiles += left * (x.nb - k - 1) - left * (left - 1) / 2 + left * (k + 1);
-        if (left > 0) cg_step_products(ps, i, x.w, x.v + static_cast<int64_t>(g0 / CG_GROUP & 1) * x.dp * CC_VLD, x.e, x.dp, k, g0, ge);
-      });
-      const double fused = std::max(26.0, 9.0 + 18.0 * tiles / 256), apart = std::max(26.0, 9.0 + 9.0 * rows / 256) + products(ps, false);
-      split = !ps.empty() && (apart < fused || CG_FORCE == 3) && CG_FORCE != 4;
-      us += split || ps.empty() ? std::max(26.0, 9.0 + 9.0 * rows / 256) : fused;
-      each([&](int i, const Mat& x) {
+    auto tiles = [&](int kind) {
+      each(k, [&](int i, const Mat& x) {
         const int ge = std::min(g0 + CG_GROUP, x.nb);
-        if (k + 1 == ge || split) {                      // V only
-          for (int b = 0; b < x.nb; ++b)
-            if (b != k && b != k + 1) put(i, CC_PANEL, b, b);
-          return;
-        }
         for (int j = k + 1; j < ge; ++j)
           for (int b = j; b < x.nb; ++b)
-            if (b != k + 1 || j != k + 1) put(i, CC_TILE, b, j);
+            if (b != k + 1 || j != k + 1) put(i, kind, b, j);
         for (int r = k + 1; r < ge; ++r)
-          for (int b = 0; b <= k; ++b) put(i, CC_TILE, r, b);
-        if (ge < x.nb) put(i, CC_TILE, ge, ge);
+          for (int b = 0; b <= k; ++b) put(i, kind, r, b);
+        if (k + 1 < ge && ge < x.nb) put(i, kind, ge, ge);
       });
+    };
+    if (k >= 0) {
+      each(k, [&](int i, const Mat& x) {
+        if (k + 1 != std::min(g0 + CG_GROUP, x.nb) && !split[k]) return;
+        for (int b = 0; b < x.nb; ++b)                   // V only
+          if (b != k && b != k + 1) put(i, CC_PANEL, b, b);
+      });
+      if (!split[k]) tiles(CC_TILE);
+      each(k, [&](int i, const Mat&) { put(i, CC_OWN, k, k); });
+      cg_append_by_xcd(plan.tasks, st.first, beside[k]);
+      us += std::max(alone[k], 9.0 + load[k] / 256);
     } else {
       us += 18;
     }
     st.grid = static_cast<int>(plan.tasks.size()) - st.first;
     if (st.grid > 0) plan.steps.push_back(st);
-    if (split) us += products(ps, true);
-    ps.clear();
-    // the group's products, by the matrices whose group ends here
-    if (k >= 0) {
-      each([&](int i, const Mat& x) {
-        if (k + 1 != std::min(g0 + CG_GROUP, x.nb)) return;
-        const int64_t v = x.v + static_cast<int64_t>(g0 / CG_GROUP & 1) * x.dp * CC_VLD;
-        cg_group_products(ps, i, x.w, v, x.dp, g0 * LEAF, std::min((k + 1) * LEAF, x.dp));
-      });
+    if (k < 0) continue;
+    if (split[k]) {
+      CgStep own{CG_PRODUCT, static_cast<int>(plan.tasks.size()), k, 0};
+      tiles(CC_STEP);
+      own.grid = static_cast<int>(plan.tasks.size()) - own.first;
+      plan.steps.push_back(own);
+      us += apart[k];
     }
-    us += products(ps, true);
+    // The products of the matrices whose group ends here.  What the steps of the next group read, its columns, its rows and the
+    // diagonal block behind it, is due now; every other tile goes along with the launches of those steps, or, of a matrix that is
+    // done, of any step to come: that with the least work so far.  (V of this group is overwritten with the group after the next.)
+    std::vector<CcTask> now, later;
+    each(k, [&](int i, const Mat& x) {
+      const int ge = std::min(g0 + CG_GROUP, x.nb), after = std::min(ge + CG_GROUP, x.nb);
+      if (k + 1 != ge) return;
+      for (const auto& [bi, bj] : cg_blocked_tiles(x.nb)) {
+          if (ge < x.nb && bi == ge && bj == ge) continue;                 // that block is factored
+          const bool due = ge < x.nb && ((bi >= ge && bi < after) || (bj >= ge && bj < after) || (bi == after && bj == after));
+          (due ? now : later).push_back(task(i, CC_PRODUCT, bi, bj));
+      }
+      const int last = ge == x.nb ? nb_max - 1 : after - 1;
+      if (last <= k) now.insert(now.end(), later.begin(), later.end());
+      else
+        for (size_t from = 0; from < later.size(); from += kProductChunk) {
+          const size_t to = std::min(later.size(), from + kProductChunk);
+          int at = k + 1;
+          for (int step = k + 2; step <= last; ++step)
+            if (load[step] < load[at]) at = step;
+          const double more = kProductUs * static_cast<double>(to - from);
+          if (load[at] + more > kBesideUs * 256) {
+            now.insert(now.end(), later.begin() + from, later.begin() + to);
+            continue;
+          }
+          beside[at].insert(beside[at].end(), later.begin() + from, later.begin() + to);
+          load[at] += more;
+        }
+      later.clear();
+    });
+    if (!now.empty()) {
+      plan.steps.push_back(CgStep{CG_PRODUCT, static_cast<int>(plan.tasks.size()), k, static_cast<int>(now.size())});
+      cg_append_by_xcd(plan.tasks, static_cast<int>(plan.tasks.size()), now);
+      us += 4.0 + kOwnProductUs * std::max(1.0, static_cast<double>(now.size()) / 256);
+    }
   }
-  plan.steps.push_back(CgStep{CG_OUT, 0, count, out_blocks, 0, 0});
+  plan.steps.push_back(CgStep{CG_OUT, 0, count, out_blocks});
   CgHeader& h = plan.h;
   std::memset(&h, 0, sizeof(h));
   h.magic = CG_MAGIC;
@@ -598,18 +533,16 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
   h.mats_off = b; b = cg_align(b + plan.mats.size() * sizeof(CgMat), 64);
   h.steps_off = b; b = cg_align(b + plan.steps.size() * sizeof(CgStep), 64);
   h.tasks_off = b; b = cg_align(b + plan.tasks.size() * sizeof(CcTask), 64);
-  h.prods_off = b; b = cg_align(b + plan.prods.size() * sizeof(CgProd), 64);
-  h.map_off = b; b = cg_align(b + plan.tile_map.size() * sizeof(int32_t), 64);
   h.total_bytes = b;
-  return us;
+  return rule_us;
 }
 
 // The sweep holds more: its sums are 128 long and its operands have all their bits, the chain's products sum 512 and take two
 // fp16 pieces (22 bits).  Error against 64 bits of the inverses, sweep and chain: ReLU rows of rank d / 8, a / lam = 2^12, 3072 4.8e-3 and
-// 1.4e-2, 6 x 1700 2.7e-3 and 6.1e-3; full rank 3072 2.8e-7 and 3.8e-7.  (Three bf16 pieces in the chain's products: 1.7e-2, more
-// roundings.)  It takes half the memory, too (3072: 23 and 51 MB).  So the chain is for groups whose steps take three rounds of tiles
+// 5.2e-3, 1700 2.7e-3 and 3.2e-3; full rank 3072 2.8e-7 and 3.6e-7.  It takes half the memory, too (3072: 23 and 51 MB).  So the chain is for groups whose steps take three rounds of tiles
 // and more, and of matrices of 15 block columns and more whose third round is used (the 2.3) it has to save a quarter: up to there
-// the sweep served when it was as slow as fp32 products make it, so that no size has lost accuracy since.  Measured, sweep and
+// the sweep served when it was as slow as fp32 products make it, so that no size has lost accuracy since.  The rule goes by the chain with its
+// products in launches of their own, as it was when it was measured (it takes 5 to 20 % less now).  Measured then, sweep and
 // chain, us: two rounds 3072 868 and 846, 2600 with 2304, 2048, 1500, 700, 600 1030 and 930; three and more 4 x 2048 855 and 652,
 // 3 x 2304 886 and 704, 4 x 2400 with 8 x 512 1230 and 880, 60 x 513 373 and 346.  The bound of 4096 tiles keeps the tables of
 // hopeless cases from being built.
@@ -679,13 +612,10 @@ extern "C" int ak_chol_group_plan(const int64_t* dims, int count, void* plan_hos
   if (!plan.mats.empty()) std::memcpy(out + plan.h.mats_off, plan.mats.data(), plan.mats.size() * sizeof(CgMat));
   std::memcpy(out + plan.h.steps_off, plan.steps.data(), plan.steps.size() * sizeof(CgStep));
   if (!plan.tasks.empty()) std::memcpy(out + plan.h.tasks_off, plan.tasks.data(), plan.tasks.size() * sizeof(CcTask));
-  if (!plan.prods.empty()) std::memcpy(out + plan.h.prods_off, plan.prods.data(), plan.prods.size() * sizeof(CgProd));
   if (!plan.sweep_leaves.empty()) {
     std::memcpy(out + plan.h.tasks_off, plan.sweep_leaves.data(), plan.sweep_leaves.size() * sizeof(SwTask));
-    std::memcpy(out + plan.h.prods_off, plan.sweep_tiles.data(), plan.sweep_tiles.size() * sizeof(SwTask));
+    std::memcpy(out + plan.h.tiles_off, plan.sweep_tiles.data(), plan.sweep_tiles.size() * sizeof(SwTask));
   }
-  if (!plan.tile_map.empty())
-    std::memcpy(out + plan.h.map_off, plan.tile_map.data(), plan.tile_map.size() * sizeof(int32_t));
   cg_kept() = CgKept();
   return AK_OK;
 }
@@ -731,19 +661,18 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
       const SwArgs w{a.ws, A_list, out_list, lam, skip_flags, info, lam_stride, skip_stride};
       hipLaunchKernelGGL(cg_sweep_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, w,
                          reinterpret_cast<const SwTask*>(a.plan + h->tasks_off),
-                         reinterpret_cast<const SwTask*>(a.plan + h->prods_off), st.count, st.first);
+                         reinterpret_cast<const SwTask*>(a.plan + h->tiles_off), st.count, st.first);
     } else if (st.type == CG_COPY) {
       hipLaunchKernelGGL(cg_copy_in_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
       hipLaunchKernelGGL(cg_scale_kernel, dim3(h->count), dim3(256), 0, s, a, h->count, CG_HALF_MAX_COND);
     } else if (st.type == CG_OUT) {
       hipLaunchKernelGGL(cg_out_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
-    } else if (st.type == CG_CHAIN) {
-      hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, CcArgs{a.ws, skip_flags, info, skip_stride},
-                         reinterpret_cast<const CcTask*>(a.plan + h->tasks_off) + st.first, st.count);
-    } else
-      hipLaunchKernelGGL(st.type == CG_PROD ? cg_prod_kernel : cg_prod_deep_kernel, dim3(st.grid), dim3(256), 0, s, a,
-                         reinterpret_cast<const CgProd*>(a.plan + h->prods_off) + st.first,
-                         reinterpret_cast<const int32_t*>(a.plan + h->map_off) + st.first_tile);
+    } else {
+      const CcArgs c{a.ws, skip_flags, info, a.scales, skip_stride};
+      const CcTask* tasks = reinterpret_cast<const CcTask*>(a.plan + h->tasks_off) + st.first;
+      if (st.type == CG_CHAIN) hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, c, tasks, st.count);
+      else hipLaunchKernelGGL(cg_product_kernel, dim3(st.grid), dim3(512), 0, s, c, tasks, st.count);
+    }
   }
   return check_launch();
 }

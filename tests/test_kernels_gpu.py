@@ -682,6 +682,38 @@ def test_chol_inv_grouped_chain(K, dims):
                 assert relerr(o, inv) < 420 * 2.0 ** -22, (i, d)
 
 
+@pytest.mark.parametrize('lam_rel', [1e-2, 1e-6])
+@pytest.mark.parametrize('dims', [(4136,), (4136, 2084, 1060), (4700, 4136, 1060, 20), (1064,) * 24, (1092,) * 20 + (552,) * 10, (2100, 2068, 1044) * 4])
+def test_chol_inv_grouped_products_beside_the_steps(K, dims, lam_rel):
+    """Groups that end inside a block (40 ... 108 columns of 128), matrices that are done before others (their last products go along with
+    the others' steps), on fp16 pieces and (a / lam beyond 2^16) on three bf16 pieces: every inverse against 64 bits, to what 22 bits
+    and the condition a d / lam allow at most, and the same bits wherever in the group a matrix stands."""
+    plan = K.chol_group_plan(list(dims))
+    assert plan.launches != max((d + 127) // 128 for d in dims) + 1, 'the block sweep: one launch per block column'
+    print(f'chain products {len(dims)} x {dims[0]} {lam_rel}', flush=True)
+    g = torch.Generator('cuda').manual_seed(3)
+    made = {}
+    for d in dims:
+        if d not in made:
+            x = torch.randn(2 * d, d, device='cuda', generator=g)
+            made[d] = x.T @ x / (2 * d)
+    mats = [made[d] for d in dims]
+    lam = torch.tensor([lam_rel * float(m.diagonal().max()) for m in mats], device='cuda')
+    outs = [torch.full_like(m, float('nan')) for m in mats]
+    info = K.chol_inv_grouped(mats, outs, lam).cpu()
+    assert int(info.abs().max()) == 0
+    for d, A in made.items():
+        same = [i for i, m in enumerate(mats) if m is A]
+        for i in same[1:]:
+            assert torch.equal(outs[i], outs[same[0]]), (d, i)
+        o = outs[same[0]]
+        full = (torch.tril(A).double() + torch.tril(A, -1).double().T + float(lam[same[0]]) * torch.eye(d, device='cuda', dtype=torch.float64)).cpu()
+        exact = torch.cholesky_inverse(torch.linalg.cholesky(full))
+        assert torch.equal(o, o.T)
+        # eigenvalues within (0.29^2 ... 1.71^2) + lam: condition below 35
+        assert relerr(o, exact) < 35 * 2.0 ** -22, (d, relerr(o, exact))
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
