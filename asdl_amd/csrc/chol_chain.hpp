@@ -271,7 +271,17 @@ static __global__ __launch_bounds__(512, 4) void cg_product_kernel(CcArgs a, con
       if (!p.same) load_to_lds(d, at + CC_PANEL_BYTES, oj + block);
     };
     struct Operands { CcFragments a[2], b; };
-    auto step = [&](int s, Operands& now, const Operands& before, bool have) {
+    // (four addresses; a stage is a constant further, as the loop below takes a round of the ring at a time)
+    AK_LDS3 const unsigned char* pa[2];
+    AK_LDS3 const unsigned char* pb[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int chunk = 16 * ((2 * q + g) ^ ((l32 >> 2) & 3));
+      pa[q] = lds + (64 * wr + l32) * 64 + chunk;
+      pb[q] = lds + (p.same ? 0 : CC_PANEL_BYTES) + (32 * wc + l32) * 64 + chunk;
+    }
+    auto step = [&](int s, auto stage_tag, Operands& now, const Operands& before, bool have) {
+      constexpr int AT = decltype(stage_tag)::value * STAGE;
       // stage s has landed for this wave, then for all; and all have read stage s - 1, which the next loads overwrite
       const int ahead = min(s1 - 1 - s, STAGES - 2);
       if (ahead == 2) {
@@ -285,10 +295,12 @@ static __global__ __launch_bounds__(512, 4) void cg_product_kernel(CcArgs a, con
       }
       __syncthreads();
       if (s + STAGES - 1 < s1) issue(s + STAGES - 1);
-      AK_LDS3 const unsigned char* at = lds + (s & (STAGES - 1)) * STAGE;
-      now.b = cc_read(p.same ? at : at + CC_PANEL_BYTES, 32 * wc + l32, g);
 #pragma unroll
-      for (int x = 0; x < 2; ++x) now.a[x] = cc_read(at, 64 * wr + 32 * x + l32, g);
+      for (int q = 0; q < 2; ++q) {
+        now.b.x[q] = *reinterpret_cast<AK_LDS3 const bf16x8*>(pb[q] + AT);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) now.a[x].x[q] = *reinterpret_cast<AK_LDS3 const bf16x8*>(pa[q] + AT + 2048 * x);
+      }
       if (!have) return;
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
@@ -301,9 +313,11 @@ static __global__ __launch_bounds__(512, 4) void cg_product_kernel(CcArgs a, con
     for (int t = 0; t < STAGES - 1; ++t)
       if (s0 + t < s1) issue(s0 + t);
     Operands even, odd;
-    for (int s = s0; s < s1; s += 2) {             // (a multiple of four stages)
-      step(s, even, odd, s > s0);
-      step(s + 1, odd, even, true);
+    for (int s = s0; s < s1; s += STAGES) {        // (s0 and s1 are multiples of it)
+      step(s, std::integral_constant<int, 0>{}, even, odd, s > s0);
+      step(s + 1, std::integral_constant<int, 1>{}, odd, even, true);
+      step(s + 2, std::integral_constant<int, 2>{}, even, odd, true);
+      step(s + 3, std::integral_constant<int, 3>{}, odd, even, true);
     }
 #pragma unroll
     for (int x = 0; x < 2; ++x) {

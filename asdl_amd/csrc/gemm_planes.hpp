@@ -273,14 +273,16 @@ __device__ __forceinline__ void plane_epilogue_wide(const PlaneGemm& p, int ti, 
     if constexpr (AUX > 0) {
       if (number >= 9 || (EPI == kEpiShifted && kind == kStepPlain)) return;
       const int a = number / 3, b = number % 3;
-      const int gj = j0 + 32 * FR * wc + 32 * b + l32, gi = i0 + 32 * FR * wr + 32 * a + 4 * g;
+      // element (gj, gi): gi in block of columns (i0 + 96 wr) / 32 + a of 32, 4 g further
+      const uint32_t lane_at = (static_cast<uint32_t>((i0 >> 5) + FR * wr + a) * static_cast<uint32_t>(p.n_pad) + static_cast<uint32_t>(j0 + 32 * FR * wc + 32 * b + l32)) * 32u + 4u * g;
 #pragma unroll
       for (int x = 0; x < AUX; ++x) {
-        const unsigned short* from = sets + paired_buf(x == 0 ? p.U : p.P, parity, kind) * p.buf_elems + plane_index(gj, gi, p.n_pad);
+        // (a uniform base and a 32-bit offset of the lane, which both planes share)
+        const unsigned short* __restrict__ from = sets + paired_buf(x == 0 ? p.U : p.P, parity, kind) * p.buf_elems;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          aux[number & 1][x][q][0] = *reinterpret_cast<const u16x4*>(from + 8 * q);
-          aux[number & 1][x][q][1] = *reinterpret_cast<const u16x4*>(from + 8 * q + p.plane_elems);
+          aux[number & 1][x][q][0] = *reinterpret_cast<const u16x4*>(from + 8 * q + lane_at);
+          aux[number & 1][x][q][1] = *reinterpret_cast<const u16x4*>(from + p.plane_elems + 8 * q + lane_at);
         }
       }
     }
