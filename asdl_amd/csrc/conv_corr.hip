@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <initializer_list>
 #include <mutex>
 #include <unordered_map>
@@ -44,10 +45,8 @@ struct CorrProd {
   int32_t M;                           // positions
   int32_t Ho, Wo, kw, KK, pw;          // virtual convolution (stride 1, no padding above)
   uint32_t mWo, mHo, mKw, mBlk;
-  // Tiles: the row tap's C columns from tile ti0 on, `ntaps` column taps of C columns each from tile tj0 on.  With
-  // an input of three bf16 planes (C = 3 c channels, [hi | mid | lo]) whose planes are whole tiles, only the six plane
-  // pairs that matter are computed: npairs = 6, ppt = c / BT tiles per plane; else npairs = 1, ppt = C / BT.
-  int32_t ti0, tj0, ntaps, ppt, npairs, tpt;    // tpt: tiles per tap in the column direction (C / BT)
+  // Tiles: the row tap's C columns from tile ti0 on, `ntaps` column taps of C columns each from tile tj0 on.
+  int32_t ti0, tj0, ntaps, tpt;        // tpt: tiles per tap in either direction (C / BT)
   int32_t kt_split, nsplit;            // k-tiles per row split, splits
   int32_t first_item, first_tile;      // running counts over the products
   int64_t part_off;                    // float4 index of partial tile (split 0, tile 0)
@@ -73,19 +72,14 @@ __device__ __forceinline__ int corr_find(const CorrArgs& a, int w, bool by_tile)
 // Tile t of a product: (ti, tj) in the virtual Gram matrix, and (row, col) = where the tile starts in the product's
 // [C, ntaps C] block of the reduced matrix, in tiles.
 __device__ __forceinline__ void corr_tile_of(const CorrProd& cp, int t, int& ti, int& tj, int& row, int& col) {
-  const int per_pair = cp.ntaps * cp.ppt * cp.ppt;
-  const int pair = t / per_pair, rem = t - pair * per_pair;
-  const int tap = rem / (cp.ppt * cp.ppt), r2 = rem - tap * cp.ppt * cp.ppt;
-  const int ii = r2 / cp.ppt, jj = r2 - ii * cp.ppt;
-  // plane pairs in the order (0,0) (0,1) (0,2) (1,0) (1,1) (2,0): hi = 0, mid = 1, lo = 2, sum of the two <= 2
-  const int pi = pair < 3 ? 0 : (pair < 5 ? 1 : 2), pj = pair < 3 ? pair : (pair < 5 ? pair - 3 : 0);
-  row = pi * cp.ppt + ii;
-  col = tap * cp.tpt + pj * cp.ppt + jj;
+  const int tap = t / (cp.tpt * cp.tpt), rem = t - tap * cp.tpt * cp.tpt;
+  row = rem / cp.tpt;
+  col = tap * cp.tpt + rem - row * cp.tpt;
   ti = cp.ti0 + row;
   tj = cp.tj0 + col;
 }
 
-__device__ __forceinline__ int corr_ntiles(const CorrProd& cp) { return cp.npairs * cp.ntaps * cp.ppt * cp.ppt; }
+__device__ __forceinline__ int corr_ntiles(const CorrProd& cp) { return cp.ntaps * cp.tpt * cp.tpt; }
 
 // One work group per (product, row split, tile).
 template <int WR, int WC, int FR, int FC>
@@ -263,60 +257,6 @@ __global__ __launch_bounds__(kAsmThreads) void corr_assemble_kernel(CorrAsm a) {
   }
 }
 
-// ---- fp32 inputs: three bf16 planes ------------------------------------------------------------------------------
-// An fp32 NCHW input takes the same path on the bf16 matrix cores at the accuracy of fp32 products: every element
-// is split exactly into three bf16 pieces, x = hi + mid + lo (each the remainder rounded to the nearest bf16; the
-// third needs no rounding), written as a channels-last tensor with 3 C channels, [hi | mid | lo] per pixel.  The
-// products above then run on that tensor as they are (3 C channels), and before the assembly the 3 x 3 blocks of
-// every [3 C, 3 C] piece are folded into [C, C]:  x^T y ~= hi^T hi' + (hi^T mid' + mid^T hi') + (hi^T lo' + lo^T hi')
-// + mid^T mid'; the three dropped blocks are below 2^-24 of the product.  The pairs are added in this order so that
-// the fold of a symmetric piece is symmetric to the last bit.
-// Two fp16 planes of channels scaled by powers of two would need half the matrix work (128 x 64 x 32 x 32, 128 x 16 x 16,
-// 256 x 8 x 8, 512 x 4 x 4 channels and pixels: 142, 114, 118, 158 us instead of 203, 146, 164, 258), but hold 22 of the 24 bits:
-// single products are off by up to 3.6e-7 instead of 1.2e-7.
-
-// x: [N, C, HW] fp32 (HW contiguous) -> planes: [N, HW, 3 C] bf16.  One work group per (sample, 32 pixels, 32
-// channels): coalesced 128-byte reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
-__global__ __launch_bounds__(256) void corr_split_nchw_kernel(const float* __restrict__ x, uint16_t* __restrict__ planes,
-                                                              int C, int HW) {
-  __shared__ float tile[32][33];
-  const int n = blockIdx.z, p0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;          // 32 x 8
-  const float* src = x + (static_cast<int64_t>(n) * C + c0) * HW + p0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int c = ty + 8 * r;
-    tile[c][tx] = p0 + tx < HW ? src[static_cast<int64_t>(c) * HW + tx] : 0.f;
-  }
-  __syncthreads();
-  uint16_t* dst = planes + (static_cast<int64_t>(n) * HW + p0) * (3 * C) + c0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int px = ty + 8 * r;
-    if (p0 + px >= HW) continue;
-    const float v = tile[tx][px];
-    const __bf16 hi = static_cast<__bf16>(v);
-    const float r1 = v - static_cast<float>(hi);
-    const __bf16 mid = static_cast<__bf16>(r1);
-    const __bf16 lo = static_cast<__bf16>(r1 - static_cast<float>(mid));
-    uint16_t* q = dst + static_cast<int64_t>(px) * (3 * C) + tx;
-    q[0] = __builtin_bit_cast(uint16_t, hi);
-    q[C] = __builtin_bit_cast(uint16_t, mid);
-    q[2 * C] = __builtin_bit_cast(uint16_t, lo);
-  }
-}
-
-// red3: [3 C][29 * 3 C] (pieces of 3 C columns) -> red: [C][29 * C].  grid (29 C / 256, C).
-__global__ __launch_bounds__(256) void corr_fold_kernel(const float* __restrict__ red3, float* __restrict__ red, int C) {
-  const int col = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
-  if (col >= kCorrPieces * C) return;
-  const int pc = col / C, c2 = col - pc * C;
-  const int64_t ld3 = static_cast<int64_t>(kCorrPieces) * 3 * C;
-  auto at = [&](int p, int q) { return red3[static_cast<int64_t>(p * C + c) * ld3 + pc * 3 * C + q * C + c2]; };
-  const float hh = at(0, 0), hm = at(0, 1) + at(1, 0), hl = at(0, 2) + at(2, 0), mm = at(1, 1);
-  red[static_cast<int64_t>(c) * (kCorrPieces * C) + col] = ((hh + hm) + hl) + mm;
-}
-
 // ---- host side ------------------------------------------------------------------------------------------------
 
 struct CorrPlan {
@@ -353,14 +293,11 @@ static bool corr_eligible(int64_t N, int64_t C, int64_t H, int64_t W, int kh, in
   return true;
 }
 
-// planes: 1, or 3 when the C channels are the three bf16 planes of C / 3 channels
-static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int planes) {
+static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W) {
   CorrPlan pl{};
   const int bt = corr_tile_width(C);
   pl.bt = bt;
   const int cb = static_cast<int>(C / bt);
-  // the unneeded plane pairs can be left out when every plane is a whole number of tiles
-  const bool pairs = planes == 3 && (C / 3) % bt == 0;
   const int occ = bt == 64 ? 4 : (bt == 128 ? 2 : 1);      // work groups per CU
   const int64_t slots = 256 * occ;
   CorrArgs& a = pl.args;
@@ -378,8 +315,6 @@ static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int 
     p.mBlk = make_magic(static_cast<uint32_t>(C) * p.KK);
     p.ti0 = ti0; p.tj0 = tj0; p.ntaps = ntaps;
     p.tpt = cb;
-    p.npairs = pairs ? 6 : 1;
-    p.ppt = pairs ? cb / 3 : cb;
   };
   const int64_t px = C * 2;                      // bytes per pixel
   fill(0, 0, N * H * W, H, W, 3, 5, 2, 2 * cb, 2 * cb, kCorrShifts);
@@ -397,15 +332,11 @@ static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int 
   for (int i = 0; i < kCorrProds; ++i) {
     CorrProd& p = a.prod[i];
     const int64_t ktiles = (p.M + kDtlBK - 1) / kDtlBK,
-                  ntiles = static_cast<int64_t>(p.npairs) * p.ntaps * p.ppt * p.ppt;
+                  ntiles = static_cast<int64_t>(p.ntaps) * p.tpt * p.tpt;
     int64_t ns = 1;
     if (i == 0 && ntiles > 0) {
-      // the main product fills the device once (the corrections ride in its tail); at least 8 k-tiles per split.  Planes of an
-      // fp32 input: three times (256-wide tiles: twice), because a sum rounds at the magnitude of its split (error against 64 bits
-      // of 128 x 64 x 32 x 32, 128 x 16 x 16, 256 x 8 x 8, 512 x 4 x 4 channels and pixels after a ReLU, once and now: 1.2, 1.5, 1.5,
-      // 2.1e-7 and 0.9, 0.9, 0.9, 1.1e-7; 246, 167, 179, 241 and 203, 146, 164, 258 us).
-      const int64_t rounds = planes == 1 ? 1 : bt < 256 ? 3 : 2;
-      ns = (rounds * slots + ntiles / 2) / ntiles;
+      // the main product fills the device once (the corrections ride in its tail); at least 8 k-tiles per split
+      ns = (slots + ntiles / 2) / ntiles;
       const int64_t cap = ktiles / 8 < 1 ? 1 : ktiles / 8;
       if (ns > cap) ns = cap;
       if (ns < 1) ns = 1;
@@ -430,12 +361,13 @@ static CorrPlan corr_plan_build(int64_t N, int64_t C, int64_t H, int64_t W, int 
   return pl;
 }
 
-static CorrPlan corr_plan(int64_t N, int64_t C, int64_t H, int64_t W, int planes = 1) {
+// Plans by shape.
+template <class Plan>
+struct CorrPlanCache {
   struct Key {
     int64_t N, C, H, W;
     bool operator==(const Key& o) const { return N == o.N && C == o.C && H == o.H && W == o.W; }
   };
-  H = planes == 3 ? -H : H;      // the two kinds of plan for one shape are two cache entries
   struct Hash {
     size_t operator()(const Key& k) const {
       uint64_t h = 0x9e3779b97f4a7c15ull;
@@ -445,16 +377,24 @@ static CorrPlan corr_plan(int64_t N, int64_t C, int64_t H, int64_t W, int planes
       return static_cast<size_t>(h);
     }
   };
-  static std::unordered_map<Key, CorrPlan, Hash> cache;
-  static std::mutex lock;
-  const Key key{N, C, H, W};
-  std::lock_guard<std::mutex> guard(lock);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  if (cache.size() > 1024) cache.clear();
-  const CorrPlan plan = corr_plan_build(N, C, H < 0 ? -H : H, W, planes);
-  cache.emplace(key, plan);
-  return plan;
+  std::unordered_map<Key, Plan, Hash> plans;
+  std::mutex lock;
+  template <class Build>
+  Plan find(int64_t N, int64_t C, int64_t H, int64_t W, Build&& build) {
+    const Key key{N, C, H, W};
+    std::lock_guard<std::mutex> guard(lock);
+    auto it = plans.find(key);
+    if (it != plans.end()) return it->second;
+    if (plans.size() > 1024) plans.clear();
+    const Plan plan = build();
+    plans.emplace(key, plan);
+    return plan;
+  }
+};
+
+static CorrPlan corr_plan(int64_t N, int64_t C, int64_t H, int64_t W) {
+  static CorrPlanCache<CorrPlan> cache;
+  return cache.find(N, C, H, W, [&] { return corr_plan_build(N, C, H, W); });
 }
 
 static size_t corr_ws_layout(const CorrPlan& pl, size_t& red_at) {
@@ -536,42 +476,460 @@ int conv_corr_syrk(const void* x, int64_t N, int64_t C, int64_t H, int64_t W, in
   return corr_assemble(red, C, alpha, beta, A, lda, stream);
 }
 
-// fp32 NCHW input: [planes: N H W 3C bf16][workspace of the 3 C-channel products, its reduced matrix last][red: C x 29 C]
-static size_t corr_f32_layout(int64_t N, int64_t C, int64_t H, int64_t W, const CorrPlan& pl3, size_t& ws3_at,
-                              size_t& red3_in_ws3, size_t& red_at) {
-  const size_t planes = static_cast<size_t>(N) * H * W * 3 * C * 2;
-  ws3_at = (planes + 255) & ~static_cast<size_t>(255);
-  const size_t ws3 = corr_ws_layout(pl3, red3_in_ws3);
-  red_at = (ws3_at + ws3 + 255) & ~static_cast<size_t>(255);
+// ---- fp32 inputs: three bf16 planes ------------------------------------------------------------------------------
+// An fp32 NCHW input takes the same path on the bf16 matrix cores at the accuracy of fp32 products: every element
+// is split exactly into three bf16 pieces, x = hi + mid + lo (each the remainder rounded to the nearest bf16; the
+// third needs no rounding), written channels-last, [hi | mid | lo] per pixel.  Six of the nine piece products count (the others
+// are below 2^-24 of the product) and all of them belong to one element of the result: a work group brings the three planes of
+// both operands into the LDS and sums them there, hi hi' on one accumulator, the five small ones on another.
+// The planes lie in a frame of zeros, two columns in front of every image row and two rows behind every image: p + D of any
+// shift D is a pixel or a zero, so that a shift is a constant added to an address and no load tests a border.
+// Bound by the matrix instructions (24 per 16 pixels and wave, alone on its SIMD, with the LDS reads and the loads of the
+// stages ahead between them) and by the operands' way into the LDS.  With the planes as 3 C channels of the products above, each
+// piece product a tile of its own (all nine with 64 channels) and folded afterwards, all kernels of a layer took (128 samples)
+//   64 x 32 x 32  217 us, now 123;  128 x 16 x 16  157, now 98;  256 x 8 x 8  175, now 104;  512 x 4 x 4  267, now 142
+// (products alone 87, 71, 73 and 101), and the factor was twice as far from the one in 64 bits (9e-8 of its norm, now 4e-8).
+// Two fp16 planes of channels scaled by powers of two would need half the matrix work, but hold 22 of the 24 bits: single products
+// are off by up to 3.6e-7 instead of 1.2e-7.
+
+constexpr int kC3K = 16;               // pixels of a stage
+constexpr int kC3Chunk = 32;           // stages whose sums join a total: 512 pixels
+constexpr int kC3Stages = 4;
+
+struct Corr3Prod {
+  uint32_t base, sn, sy, sx;           // bytes: the first position's place in the planes, between images, rows, pixels of the positions
+  int32_t M, Ho, Wo;                   // positions
+  uint32_t mWo, mHo;
+  int32_t ntaps, tiles_n;              // column taps of C columns each; tiles of columns
+  int32_t k_split, nsplit;             // stages per split of the positions, splits
+  int32_t first_item, first_tile;      // running counts over the products
+  int64_t part_off;                    // float4 index of partial tile (split 0, tile 0)
+  int64_t out_off;                     // first column of the product in the reduced matrix red[C][29 C]
+  uint32_t toff[kCorrShifts];          // bytes from a position to its partner under each tap
+};
+
+struct Corr3Args {
+  Corr3Prod prod[kCorrProds];
+  const void* planes;
+  uint32_t bytes;                      // of the planes: what lies behind them reads as zero
+  int32_t C, tiles_m;
+  floatx4* part;
+  float* red;
+};
+
+// x: [N, C, H, W] fp32 -> planes: [N, H + 2, W + 2, 3 C] bf16.  One work group per (sample, 32 pixels of the frame, 32
+// channels): coalesced reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
+__global__ __launch_bounds__(256) void corr3_split_kernel(const float* __restrict__ x, uint16_t* __restrict__ planes, int C, int H, int W) {
+  __shared__ float tile[32][33];
+  const int n = blockIdx.z, p0 = blockIdx.x * 32, c0 = blockIdx.y * 32, Wp = W + 2, px_all = (H + 2) * Wp;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;          // 32 x 8
+  const int at = p0 + tx, row = at / Wp, col = at - row * Wp - 2;
+  const bool inside = row < H && col >= 0;
+  const float* src = x + (static_cast<int64_t>(n) * C + c0) * H * W + (inside ? row * W + col : 0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int c = ty + 8 * r;
+    tile[c][tx] = inside ? src[static_cast<int64_t>(c) * H * W] : 0.f;
+  }
+  __syncthreads();
+  uint16_t* dst = planes + (static_cast<int64_t>(n) * px_all + p0) * (3 * C) + c0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int px = ty + 8 * r;
+    if (p0 + px >= px_all) continue;
+    const float v = tile[tx][px];
+    const __bf16 hi = static_cast<__bf16>(v);
+    const float r1 = v - static_cast<float>(hi);
+    const __bf16 mid = static_cast<__bf16>(r1);
+    const __bf16 lo = static_cast<__bf16>(r1 - static_cast<float>(mid));
+    uint16_t* q = dst + static_cast<int64_t>(px) * (3 * C) + tx;
+    q[0] = __builtin_bit_cast(uint16_t, hi);
+    q[C] = __builtin_bit_cast(uint16_t, mid);
+    q[2 * C] = __builtin_bit_cast(uint16_t, lo);
+  }
+}
+
+// Element (row, col) of a product's block of the reduced matrix.  Its first tap is the pixel itself: that piece is symmetric, and
+// is made so exactly by its upper triangle.
+__device__ __forceinline__ void corr3_store(const Corr3Args& a, const Corr3Prod& cp, int row, int col, float v) {
+  if (col >= cp.ntaps * a.C) return;
+  const int64_t ld = static_cast<int64_t>(kCorrPieces) * a.C;
+  float* red = a.red + cp.out_off;
+  if (col >= a.C) {
+    red[row * ld + col] = v;
+  } else if (row <= col) {
+    red[row * ld + col] = v;
+    red[col * ld + row] = v;
+  }
+}
+
+// A tile wholly below the first tap's diagonal: its transpose writes it.
+__device__ __forceinline__ bool corr3_below(const Corr3Args& a, int row0, int col0, int cols) { return row0 >= col0 + cols && col0 + cols <= a.C; }
+
+__device__ __forceinline__ int corr3_find(const Corr3Args& a, int w, bool by_tile) {
+  int pi = 0;
+#pragma unroll
+  for (int i = 1; i < kCorrProds; ++i)
+    if (w >= (by_tile ? a.prod[i].first_tile : a.prod[i].first_item)) pi = i;
+  return pi;
+}
+
+// One work group per (product, split of the positions, tile of 64 WR channels x 64 WC columns), four waves of 64 x 64.
+template <int WR, int WC>
+__global__ __launch_bounds__(256, 1) void corr3_products_kernel(Corr3Args a) {
+  constexpr int BR = 64 * WR, BC = 64 * WC, CBR = BR / 32, CBC = BC / 32, BLOCKS = 3 * (CBR + CBC);
+  constexpr int LOADS = (BLOCKS + 3) / 4, STAGE = 4 * LOADS * 1024, S = kC3Stages;
+  static_assert(WR * WC == 4 && kC3Chunk % 2 == 0, "four waves; two stages at a time");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
+  AK_LDS unsigned char* lds = (AK_LDS unsigned char*)dtl_smem;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WC, wc = wave % WC;
+  // the main product's items, an XCD's in a row, then the corrections' in the tail (in one row, the last XCDs had all of those)
+  const int first = a.prod[1].first_item, blk0 = static_cast<int>(blockIdx.x);
+  const int w = blk0 < first ? static_cast<int>(xcd_contiguous_id(blk0, first)) : blk0;
+  const Corr3Prod& cp = a.prod[corr3_find(a, w, false)];
+  const int local = w - cp.first_item, ntiles = a.tiles_m * cp.tiles_n;
+  const int split = local / ntiles, t = local - split * ntiles, tn = t / a.tiles_m, tm = t - tn * a.tiles_m;
+  const int row0 = tm * BR, col0 = tn * BC;
+  if (corr3_below(a, row0, col0, BC)) return;
+  const int k0 = split * cp.k_split, k1 = min(k0 + cp.k_split, (cp.M + kC3K - 1) / kC3K);
+
+  u32x4 rsrc;
+  const uint64_t ba = reinterpret_cast<uint64_t>(a.planes);
+  rsrc[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba));
+  rsrc[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(ba >> 32) & 0xffffu);
+  rsrc[2] = a.bytes;
+  rsrc[3] = 0x00020000u;
+  // A stage: blocks of [16 pixels][32 channels] (1 KB), those of A by plane and 32 channels, then those of B; dealt to the waves round-robin.
+  // What a block adds to the address of its pixel:
+  uint32_t block_at[LOADS];
+#pragma unroll
+  for (int l = 0; l < LOADS; ++l) {
+    const int blk = wave + 4 * l;
+    uint32_t at = kDtlOob;
+    if (blk < 3 * CBR) {
+      at = static_cast<uint32_t>((blk / CBR) * a.C + row0 + 32 * (blk % CBR)) * 2u;
+    } else if (blk < BLOCKS) {
+      const int b = blk - 3 * CBR, col = col0 + 32 * (b % CBC), tap = col / a.C;
+      if (tap < cp.ntaps) at = cp.toff[tap] + static_cast<uint32_t>((b / CBC) * a.C + col - tap * a.C) * 2u;
+    }
+    block_at[l] = __builtin_amdgcn_readfirstlane(at);
+  }
+  const int prow = lane >> 2;
+  // byte offset of the lane's 16 bytes of its pixel of stage kt (kDtlOob: none), in parts without a branch (what they need is
+  // held in scalar registers: read from memory in the loop, its latency stood in every stage)
+  const auto held = [](uint32_t v) { return __builtin_amdgcn_readfirstlane(v); };
+  const uint32_t M = held(min(cp.M, k1 * kC3K)), Wo = held(cp.Wo), Ho = held(cp.Ho), mWo = held(Wo == 1 ? 0 : cp.mWo), mHo = held(Ho == 1 ? 0 : cp.mHo);
+  const uint32_t all_Wo = held(Wo == 1 ? ~0u : 0u), all_Ho = held(Ho == 1 ? ~0u : 0u), sn = held(cp.sn), sy = held(cp.sy), sx = held(cp.sx);
+  const uint32_t base_lane = cp.base + (lane & 3) * 16u;
+  struct Place { uint32_t pos, q1, n, at; };
+  constexpr int PARTS = 6;
+  auto place_part = [&](Place& p, int kt, int part) {
+    if (part == 0) p.pos = static_cast<uint32_t>(kt * kC3K + prow), p.q1 = __umulhi(p.pos, mWo) | (p.pos & all_Wo);
+    if (part == 1) p.n = __umulhi(p.q1, mHo) | (p.q1 & all_Ho);
+    if (part == 2) p.at = base_lane + (p.pos - p.q1 * Wo) * sx;
+    if (part == 3) p.at += p.n * sn;
+    if (part == 4) p.at += (p.q1 - p.n * Ho) * sy;
+    if (part == 5) p.at = p.pos < M ? p.at : kDtlOob;
+  };
+  auto load_one = [&](uint32_t pixel, int stage, int l) {
+    const uint32_t at = pixel == kDtlOob || block_at[l] == kDtlOob ? kDtlOob : pixel + block_at[l];
+    load_to_lds(rsrc, lds0 + stage * STAGE + (wave + 4 * l) * 1024, at);
+  };
+
+  floatx16 tot[2][2], big[2][2], small[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tot[x][y][r] = 0.f;
+
+  const int g = lane >> 5, hl = (lane >> 4) & 1, j16 = lane & 15;
+  const int frag_lane = (8 * g + (j16 >> 2)) * 64 + hl * 32 + (j16 & 3) * 8;
+  AK_LDS const unsigned char* frag_a = lds + frag_lane + 2 * wr * 1024;
+  AK_LDS const unsigned char* frag_b = lds + frag_lane + (3 * CBR + 2 * wc) * 1024;
+  auto tr = [](AK_LDS const unsigned char* q) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((AK_LDS short4v*)(q)); };
+  struct Fragments { bf16x8 a[3][2], b[3][2]; };       // [plane][32 channels]
+  // fragment u of twelve, in the order the matrix instructions want them: (lo, hi), (mid, hi), (mid, mid), (hi, mid), (hi, lo), (hi, hi)
+  auto read_one = [&](Fragments& f, int soff, int u) {
+    constexpr int PLANE[6] = {2, 0, 1, 1, 0, 2};
+    constexpr bool OF_A[6] = {true, false, true, false, true, false};
+    const int plane = PLANE[u >> 1], i = u & 1;
+    AK_LDS const unsigned char* q = (OF_A[u >> 1] ? frag_a + plane * CBR * 1024 : frag_b + plane * CBC * 1024) + soff + i * 1024;
+    (OF_A[u >> 1] ? f.a : f.b)[plane][i] = pack_bf16x8(tr(q), tr(q + 256));
+  };
+  // One stage: 24 matrix instructions on `now`; between them the fragments of the next stage, then the loads of the one S - 1 ahead.
+  auto step = [&](int kt, int soff_next, int fill, const Fragments& now, Fragments& next) {
+    wait_vmcnt<(S - 3) * LOADS>();             // stage kt + 1 has landed for this wave,
+    __syncthreads();                           // then for all; and all have read stage kt
+    Place p;
+    constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
+#pragma unroll
+    for (int m = 0; m < 24; ++m) {
+      const int pr = m >> 2, x = (m >> 1) & 1, y = m & 1;
+      if (pr == 5) big[x][y] = mfma_bf16(now.a[PA[pr]][x], now.b[PB[pr]][y], big[x][y]);
+      else small[x][y] = mfma_bf16(now.a[PA[pr]][x], now.b[PB[pr]][y], small[x][y]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (m < 12) {
+        read_one(next, soff_next, m);
+        if (m & 1) place_part(p, kt + S - 1, m >> 1);
+      } else if (m - 12 < LOADS) {
+        load_one(p.at, fill, m - 12);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s) {
+    Place p;
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) place_part(p, k0 + s, part);
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) load_one(p.at, s, l);
+  }
+  wait_vmcnt<(S - 2) * LOADS>();
+  __syncthreads();
+  Fragments even, odd;
+#pragma unroll
+  for (int u = 0; u < 12; ++u) read_one(even, 0, u);
+  int stage = 0;                               // of k-tile kt; (the stages behind the last one hold zeros)
+  for (int c = k0; c < k1; c += kC3Chunk) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) big[x][y][r] = small[x][y][r] = 0.f;
+    const int end = min(c + kC3Chunk, k1);
+    for (int kt = c; kt < end; kt += 2) {
+      step(kt, ((stage + 1) & (S - 1)) * STAGE, (stage + S - 1) & (S - 1), even, odd);
+      step(kt + 1, ((stage + 2) & (S - 1)) * STAGE, (stage + S) & (S - 1), odd, even);
+      stage = (stage + 2) & (S - 1);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[x][y][r] += big[x][y][r] + small[x][y][r];
+  }
+  wait_vmcnt<0>();                             // the loads behind the last stage, before the LDS is released
+  if (cp.nsplit == 1) {
+    const int l32 = lane & 31;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          corr3_store(a, cp, row0 + 64 * wr + 32 * x + 8 * (r >> 2) + 4 * g + (r & 3), col0 + 64 * wc + 32 * y + l32, tot[x][y][r]);
+    return;
+  }
+  floatx4* part = a.part + cp.part_off + static_cast<int64_t>(local) * (BR * BC / 4) + tid;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        part[((x * 2 + y) * 4 + q) * 256] = floatx4{tot[x][y][4 * q], tot[x][y][4 * q + 1], tot[x][y][4 * q + 2], tot[x][y][4 * q + 3]};
+}
+
+// Sums the partial tiles of the splits in a fixed order.  grid (tiles of all products, 16): one work group per float4 slot of every
+// thread's accumulators.
+template <int WR, int WC>
+__global__ __launch_bounds__(256) void corr3_reduce_kernel(Corr3Args a) {
+  constexpr int BR = 64 * WR, BC = 64 * WC;
+  constexpr int64_t tile_f4 = BR * BC / 4;
+  const Corr3Prod& cp = a.prod[corr3_find(a, blockIdx.x, true)];
+  if (cp.nsplit == 1) return;                          // written by the product itself
+  const int ntiles = a.tiles_m * cp.tiles_n, t = blockIdx.x - cp.first_tile, tn = t / a.tiles_m, tm = t - tn * a.tiles_m;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slot = blockIdx.y;
+  const int wr = wave / WC, wc = wave % WC, q = slot & 3, y = (slot >> 2) & 1, x = slot >> 3;
+  if (corr3_below(a, tm * BR, tn * BC, BC)) return;
+  const floatx4* src = a.part + cp.part_off + t * tile_f4 + slot * 256 + tid;
+  const int64_t stride = ntiles * tile_f4;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};                // (in floats, these sums were the larger part of the result's error)
+  int s = 0;
+  for (; s + 8 <= cp.nsplit; s += 8) {                 // eight loads in flight
+    floatx4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = src[(s + k) * stride];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += static_cast<double>(v[k][e]);
+  }
+  for (; s < cp.nsplit; ++s) {
+    const floatx4 v = src[s * stride];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += static_cast<double>(v[e]);
+  }
+  const int row = tm * BR + 64 * wr + 32 * x + 8 * q + 4 * (lane >> 5), col = tn * BC + 64 * wc + 32 * y + (lane & 31);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) corr3_store(a, cp, row + e, col, static_cast<float>(acc[e]));
+}
+
+struct Corr3Plan {
+  Corr3Args args;                      // planes, part and red are filled in per call
+  int items, tiles;
+  bool wide;                           // 128 x 128 tiles, else 64 x 256
+  size_t part_f4;
+};
+
+static int64_t corr3_pixel_bytes(int64_t C) { return 6 * C; }
+static int64_t corr3_plane_bytes(int64_t N, int64_t C, int64_t H, int64_t W) { return N * (H + 2) * (W + 2) * corr3_pixel_bytes(C); }
+
+// (the margin: what a shift of the last position adds)
+static bool corr3_eligible(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
+  return C % 64 == 0 && N <= 65535 && corr_eligible(N, 3 * C, H, W, kh, kw, sh, sw, ph, pw) &&
+         corr3_plane_bytes(N, C, H, W) + 3 * (W + 2) * corr3_pixel_bytes(C) <= static_cast<int64_t>(kDtlRange);
+}
+
+static Corr3Plan corr3_plan_build(int64_t N, int64_t C, int64_t H, int64_t W) {
+  Corr3Plan pl{};
+  pl.wide = C % 128 == 0;
+  const int64_t br = pl.wide ? 128 : 64, bc = pl.wide ? 128 : 256, px = corr3_pixel_bytes(C), Wp = W + 2, img = (H + 2) * Wp * px;
+  Corr3Args& a = pl.args;
+  a.bytes = static_cast<uint32_t>(corr3_plane_bytes(N, C, H, W));
+  a.C = static_cast<int32_t>(C);
+  a.tiles_m = static_cast<int32_t>(C / br);
+  // kind of the taps: 0 the 13 shifts, 1 along the row, 2 along the column, 3 the pixel alone
+  auto fill = [&](int i, int64_t first_px, int64_t M, int64_t Ho, int64_t Wo, int kind) {
+    Corr3Prod& p = a.prod[i];
+    p.base = static_cast<uint32_t>((first_px + 2) * px);
+    p.sn = static_cast<uint32_t>(img); p.sy = static_cast<uint32_t>(Wp * px); p.sx = static_cast<uint32_t>(px);
+    p.M = static_cast<int32_t>(M); p.Ho = static_cast<int32_t>(Ho); p.Wo = static_cast<int32_t>(Wo);
+    p.mWo = make_magic(p.Wo); p.mHo = make_magic(p.Ho);
+    p.ntaps = kind == 0 ? kCorrShifts : kind == 3 ? 1 : 3;
+    p.tiles_n = static_cast<int32_t>((p.ntaps * C + bc - 1) / bc);
+    for (int t = 0; t < p.ntaps; ++t) {
+      const int dy = kind == 0 ? (t + 2) / 5 : kind == 2 ? t : 0, dx = kind == 0 ? t - 5 * dy : kind == 1 ? t : 0;
+      p.toff[t] = static_cast<uint32_t>((dy * Wp + dx) * px);
+    }
+  };
+  fill(0, 0, N * H * W, H, W, 0);
+  for (int e = 0; e < 2; ++e) {
+    fill(1 + e, e * (H - 1) * Wp, N * W, 1, W, 1);
+    fill(3 + e, e * (W - 1), N * H, H, 1, 2);
+    for (int q = 0; q < 2; ++q) fill(5 + 2 * e + q, e * (H - 1) * Wp + q * (W - 1), N, 1, 1, 3);
+  }
+  auto stages = [&](const Corr3Prod& p) { return static_cast<int64_t>(p.M + kC3K - 1) / kC3K; };
+  // The main product in the number of splits (of at least 4 stages) and the corrections in chains of 32, 16 or 8 stages whose items end
+  // first on the shader engine (8 CUs) that has most of both.  Items are dealt to the 32 engines in turn, and one whose engine is full holds up those
+  // behind it: a 57th split of 128 x 64 x 32 x 32 leaves some engines no CU for their corrections.  In stages of the main product
+  // (0.45 us): an item has 13 besides its own, a correction's stage (pixels an image or a row apart) is 1.25, the reduction of partial
+  // tiles 10 and one per 20 tiles.  Splits and us, all kernels: 128 x 64 x 32 x 32: 48 124, 56 118, 57 130, 64 125;
+  // 128 x 128 x 16 x 16: 10 123, 16 97, 18 106, 20 130; 128 x 256 x 8 x 8: 3 115, 4 100, 5 131, 8 106; 128 x 512 x 4 x 4: 1 139, 3 152.
+  constexpr int64_t kEngines = 32, kCus = 8, kItem = 13;
+  const int64_t main_tiles = static_cast<int64_t>(a.tiles_m) * a.prod[0].tiles_n, all = stages(a.prod[0]);
+  auto chains = [&](const Corr3Prod& p, int64_t len) { return (stages(p) + len - 1) / len; };
+  int64_t best = 1, best_chain = kC3Chunk;
+  double best_time = 0;
+  for (int64_t chain : {32, 16, 8})
+    for (int64_t ns = 1; ns <= std::max<int64_t>(1, std::min<int64_t>(all / 4, 2 * kEngines * kCus / main_tiles + 1)); ++ns) {
+      const int64_t len = (all + ns - 1) / ns + kItem, n = main_tiles * ns, here = (n + kEngines - 1) / kEngines;
+      int64_t busy[kCus], before = 0;    // (a heap of the times at which the CUs are free)
+      for (int64_t c = 0; c < kCus; ++c) busy[c] = (here / kCus + (c < here % kCus)) * len;
+      std::make_heap(busy, busy + kCus, std::greater<>());
+      bool partial = ns > 1;
+      for (int i = 1; i < kCorrProds; ++i) {
+        const Corr3Prod& p = a.prod[i];
+        const int64_t cs = chains(p, chain), after = before + a.tiles_m * p.tiles_n * cs, each = (stages(p) + cs - 1) / cs * 5 / 4 + kItem;
+        int64_t count = (after + kEngines - 1) / kEngines - (before + kEngines - 1) / kEngines;
+        for (int64_t& t : busy) t += count / kCus * each;
+        for (count %= kCus; count > 0; --count) {
+          std::pop_heap(busy, busy + kCus, std::greater<>());
+          busy[kCus - 1] += each;
+          std::push_heap(busy, busy + kCus, std::greater<>());
+        }
+        before = after;
+        partial |= cs > 1;
+      }
+      const double time = static_cast<double>(*std::max_element(busy, busy + kCus)) + (partial ? 10.0 + 0.05 * static_cast<double>(n + before) : 0.0);
+      if ((ns == 1 && chain == 32) || time < best_time) {
+        best = ns;
+        best_chain = chain;
+        best_time = time;
+      }
+    }
+  int items = 0, tiles = 0;
+  size_t part = 0;
+  int64_t red_col = 0;
+  for (int i = 0; i < kCorrProds; ++i) {
+    Corr3Prod& p = a.prod[i];
+    const int64_t n = static_cast<int64_t>(a.tiles_m) * p.tiles_n, ns = i == 0 ? best : chains(p, best_chain);
+    p.k_split = static_cast<int32_t>(((stages(p) + ns - 1) / ns + 1) / 2 * 2);        // (an even number of stages)
+    p.nsplit = static_cast<int32_t>((stages(p) + p.k_split - 1) / p.k_split);
+    p.first_item = items;
+    p.first_tile = tiles;
+    p.part_off = static_cast<int64_t>(part);
+    p.out_off = red_col;
+    red_col += p.ntaps * C;            // C per piece: 13 C, 3 C or C
+    items += p.nsplit * static_cast<int>(n);
+    tiles += static_cast<int>(n);
+    if (p.nsplit > 1) part += static_cast<size_t>(p.nsplit * n * br * bc / 4);
+  }
+  pl.items = items;
+  pl.tiles = tiles;
+  pl.part_f4 = part;
+  return pl;
+}
+
+static Corr3Plan corr3_plan(int64_t N, int64_t C, int64_t H, int64_t W) {
+  static CorrPlanCache<Corr3Plan> cache;
+  return cache.find(N, C, H, W, [&] { return corr3_plan_build(N, C, H, W); });
+}
+
+// [planes][partial tiles][red: C x 29 C]
+static size_t corr3_layout(int64_t N, int64_t C, int64_t H, int64_t W, const Corr3Plan& pl, size_t& part_at, size_t& red_at) {
+  auto aligned = [](size_t b) { return (b + 255) & ~static_cast<size_t>(255); };
+  part_at = aligned(static_cast<size_t>(corr3_plane_bytes(N, C, H, W)));
+  red_at = aligned(part_at + pl.part_f4 * sizeof(floatx4));
   return red_at + static_cast<size_t>(C) * kCorrPieces * C * sizeof(float);
 }
 
 size_t conv_corr_f32_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
-  if (C % 64 != 0 || !corr_eligible(N, 3 * C, H, W, kh, kw, sh, sw, ph, pw)) return 0;
-  size_t a, b, c;
-  return corr_f32_layout(N, C, H, W, corr_plan(N, 3 * C, H, W, 3), a, b, c);
+  if (!corr3_eligible(N, C, H, W, kh, kw, sh, sw, ph, pw)) return 0;
+  size_t a, b;
+  return corr3_layout(N, C, H, W, corr3_plan(N, C, H, W), a, b);
+}
+
+template <int WR, int WC>
+static int corr3_launch(const Corr3Plan& pl, const Corr3Args& args, hipStream_t stream) {
+  constexpr int kLds = kC3Stages * 4 * ((6 * (WR + WC) + 3) / 4) * 1024;
+  static bool attr_set = false;     // idempotent; a race sets it twice at worst
+  if (!attr_set) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(corr3_products_kernel<WR, WC>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return AK_ERR_LAUNCH;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((corr3_products_kernel<WR, WC>), dim3(static_cast<unsigned>(pl.items)), dim3(256), kLds, stream, args);
+  if (pl.part_f4 > 0)
+    hipLaunchKernelGGL((corr3_reduce_kernel<WR, WC>), dim3(static_cast<unsigned>(pl.tiles), 16), dim3(256), 0, stream, args);
+  return AK_OK;
 }
 
 int conv_corr_syrk_f32(const float* x, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph,
                        int pw, float alpha, float beta, float* A, int64_t lda, void* ws, size_t ws_bytes,
                        hipStream_t stream) {
-  if (C % 64 != 0 || !corr_eligible(N, 3 * C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;
-  const CorrPlan pl3 = corr_plan(N, 3 * C, H, W, 3);
-  size_t ws3_at, red3_in_ws3, red_at;
-  const size_t need = corr_f32_layout(N, C, H, W, pl3, ws3_at, red3_in_ws3, red_at);
+  if (!corr3_eligible(N, C, H, W, kh, kw, sh, sw, ph, pw)) return AK_ERR_UNSUPPORTED;
+  const Corr3Plan pl = corr3_plan(N, C, H, W);
+  size_t part_at, red_at;
+  const size_t need = corr3_layout(N, C, H, W, pl, part_at, red_at);
   if (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255) != 0) return AK_ERR_WORKSPACE;
   unsigned char* base = static_cast<unsigned char*>(ws);
-  uint16_t* planes = reinterpret_cast<uint16_t*>(base);
-  const int HW = static_cast<int>(H * W);
-  hipLaunchKernelGGL(corr_split_nchw_kernel, dim3((HW + 31) / 32, static_cast<unsigned>(C / 32), static_cast<unsigned>(N)),
-                     dim3(256), 0, stream, x, planes, static_cast<int>(C), HW);
-  float* red3 = reinterpret_cast<float*>(base + ws3_at + red3_in_ws3);
-  const int rc = corr_products(pl3, planes, reinterpret_cast<floatx4*>(base + ws3_at), red3, stream);
+  Corr3Args args = pl.args;
+  args.planes = base;
+  args.part = reinterpret_cast<floatx4*>(base + part_at);
+  args.red = reinterpret_cast<float*>(base + red_at);
+  hipLaunchKernelGGL(corr3_split_kernel, dim3(static_cast<unsigned>(((H + 2) * (W + 2) + 31) / 32), static_cast<unsigned>(C / 32), static_cast<unsigned>(N)),
+                     dim3(256), 0, stream, x, reinterpret_cast<uint16_t*>(base), static_cast<int>(C), static_cast<int>(H), static_cast<int>(W));
+  const int rc = pl.wide ? corr3_launch<2, 2>(pl, args, stream) : corr3_launch<1, 4>(pl, args, stream);
   if (rc != AK_OK) return rc;
-  float* red = reinterpret_cast<float*>(base + red_at);
-  hipLaunchKernelGGL(corr_fold_kernel, dim3(static_cast<unsigned>((kCorrPieces * C + 255) / 256), static_cast<unsigned>(C)),
-                     dim3(256), 0, stream, red3, red, static_cast<int>(C));
-  return corr_assemble(red, C, alpha, beta, A, lda, stream);
+  return corr_assemble(args.red, C, alpha, beta, A, lda, stream);
 }
 
 }  // namespace ak

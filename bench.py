@@ -499,8 +499,8 @@ def main():
                          'batch': bs}
         if 'roofline' in out:
             out['roofline']['kernel'] = ('factor statistics of fp32 NCHW operands: the 3x3 stride-1 layers as shifted '
-                                         'correlations of three bf16 planes of the input (corr_split_nchw_kernel, '
-                                         'corr_products_kernel, corr_fold_kernel, corr_assemble_kernel: bf16 matrix '
+                                         'correlations of three bf16 planes of the input (corr3_split_kernel, '
+                                         'corr3_products_kernel, corr3_reduce_kernel, corr_assemble_kernel: bf16 matrix '
                                          'cores, fp32 accuracy), the others on syrk_window_kernel, syrk_wave_kernel, '
                                          'conv_patch_syrk_kernel<float> (v_mfma_f32_32x32x2_f32); '
                                          'SYRK FLOP M*d*(d+1) against the fp32 matrix peak, the rate the reference\'s '

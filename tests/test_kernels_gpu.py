@@ -1624,6 +1624,25 @@ def test_fp32_correlations_hold_all_24_bits(K, N, C, H, W):
     assert float((out.double().cpu() - rows.T @ rows).abs().max()) <= 2.0 ** -23
 
 
+@pytest.mark.parametrize("N,C,H,W", [(1, 64, 1, 1), (15, 128, 1, 1), (17, 64, 1, 3), (1, 128, 1, 33), (5, 192, 4, 1), (3, 320, 7, 2), (33, 384, 2, 3), (1, 64, 31, 64),
+                                     (129, 64, 2, 2), (2, 1024, 5, 5)])
+def test_fp32_correlations_of_small_and_odd_images(K, N, C, H, W):
+    """Images smaller than the window (every shift ends in the frame of zeros), pixels that fill no stage, column tiles that end behind
+    the last tap (64, 192 and 320 channels), tiles below the diagonal that are left out (1024); several splits and one."""
+    g = torch.Generator().manual_seed(N + C + H + W)
+    x = torch.randn(N, C, H, W, generator=g)
+    rows = nn.functional.unfold(x.double(), 3, 1, 1, 1).permute(0, 2, 1).reshape(-1, 9 * C)
+    ref = rows.T @ rows
+    guard = torch.full((9 * C + 2, 9 * C), 7.0, device='cuda')
+    out = K.conv_syrk(x.cuda(), (3, 3), (1, 1), (1, 1), out=guard[1:-1])
+    # sums of at most 2048 products, against the norms of their channels: a chain of 32 sums of 16 products and the joins after it
+    # round at most 2^-24 of a partial sum each, and so do the three corrections of an entry
+    scale = x.double().pow(2).sum(dim=(0, 2, 3)).sqrt().clamp_min(1e-30).repeat_interleave(9)
+    assert float(((out.double().cpu() - ref) / scale / scale[:, None]).abs().max()) < 64 * 2.0 ** -24
+    assert torch.equal(out, out.T)
+    assert bool((guard[0] == 7).all()) and bool((guard[-1] == 7).all())
+
+
 @pytest.mark.parametrize("N,C,H", [(128, 64, 32), (128, 128, 16), (128, 256, 8)])
 def test_fp32_correlations_are_as_close_as_one_rounding_of_the_result(K, N, C, H):
     """Sums over 8192 to 131072 pixels of ReLU outputs: their accumulators round at the magnitude of a split, and the factor ends
