@@ -487,13 +487,12 @@ int conv_corr_syrk(const void* x, int64_t N, int64_t C, int64_t H, int64_t W, in
 // Bound by the matrix instructions (24 per 16 pixels and wave, alone on its SIMD, with the LDS reads and the loads of the
 // stages ahead between them) and by the operands' way into the LDS.  With the planes as 3 C channels of the products above, each
 // piece product a tile of its own (all nine with 64 channels) and folded afterwards, all kernels of a layer took (128 samples)
-//   64 x 32 x 32  217 us, now 123;  128 x 16 x 16  157, now 98;  256 x 8 x 8  175, now 104;  512 x 4 x 4  267, now 142
-// (products alone 87, 71, 73 and 101), and the factor was twice as far from the one in 64 bits (9e-8 of its norm, now 4e-8).
+//   64 x 32 x 32  217 us, now 125;  128 x 16 x 16  157, now 102;  256 x 8 x 8  175, now 106;  512 x 4 x 4  267, now 148
+// (products alone 90, 74, 76 and 106), and the factor was twice as far from the one in 64 bits (9e-8 of its norm, now 4e-8).
 // Two fp16 planes of channels scaled by powers of two would need half the matrix work, but hold 22 of the 24 bits: single products
 // are off by up to 3.6e-7 instead of 1.2e-7.
 
 constexpr int kC3K = 16;               // pixels of a stage
-constexpr int kC3Chunk = 32;           // stages whose sums join a total: 512 pixels
 constexpr int kC3Stages = 4;
 
 struct Corr3Prod {
@@ -501,6 +500,8 @@ struct Corr3Prod {
   int32_t M, Ho, Wo;                   // positions
   uint32_t mWo, mHo;
   int32_t ntaps, tiles_n;              // column taps of C columns each; tiles of columns
+  int32_t kw;                          // of a window, whose taps are `pitch` bytes a row apart
+  uint32_t pitch;
   int32_t k_split, nsplit;             // stages per split of the positions, splits
   int32_t first_item, first_tile;      // running counts over the products
   int64_t part_off;                    // float4 index of partial tile (split 0, tile 0)
@@ -517,22 +518,24 @@ struct Corr3Args {
   float* red;
 };
 
-// x: [N, C, H, W] fp32 -> planes: [N, H + 2, W + 2, 3 C] bf16.  One work group per (sample, 32 pixels of the frame, 32
-// channels): coalesced reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
-__global__ __launch_bounds__(256) void corr3_split_kernel(const float* __restrict__ x, uint16_t* __restrict__ planes, int C, int H, int W) {
+// x: [N, C, H, W] fp32 -> planes: [N, Hp, Wp, 3 Cp] bf16, the image from (top, left) on in a frame of zeros (an image that does not fit
+// is cut off), channels padded with zeros to Cp, a multiple of 32.  One work group per (sample, 32 pixels of the frame, 32 channels):
+// coalesced reads along the pixels, 64-byte runs of channels per pixel and plane on the way out.
+__global__ __launch_bounds__(256) void corr3_split_kernel(const float* __restrict__ x, uint16_t* __restrict__ planes, int C, int Cp, int H, int W, int Hp, int Wp,
+                                                          int top, int left) {
   __shared__ float tile[32][33];
-  const int n = blockIdx.z, p0 = blockIdx.x * 32, c0 = blockIdx.y * 32, Wp = W + 2, px_all = (H + 2) * Wp;
+  const int n = blockIdx.z, p0 = blockIdx.x * 32, c0 = blockIdx.y * 32, px_all = Hp * Wp;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;          // 32 x 8
-  const int at = p0 + tx, row = at / Wp, col = at - row * Wp - 2;
-  const bool inside = row < H && col >= 0;
+  const int at = p0 + tx, fy = at / Wp, row = fy - top, col = at - fy * Wp - left;
+  const bool inside = at < px_all && row >= 0 && row < H && col >= 0 && col < W;
   const float* src = x + (static_cast<int64_t>(n) * C + c0) * H * W + (inside ? row * W + col : 0);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int c = ty + 8 * r;
-    tile[c][tx] = inside ? src[static_cast<int64_t>(c) * H * W] : 0.f;
+    tile[c][tx] = inside && c0 + c < C ? src[static_cast<int64_t>(c) * H * W] : 0.f;
   }
   __syncthreads();
-  uint16_t* dst = planes + (static_cast<int64_t>(n) * px_all + p0) * (3 * C) + c0;
+  uint16_t* dst = planes + (static_cast<int64_t>(n) * px_all + p0) * (3 * Cp) + c0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int px = ty + 8 * r;
@@ -542,10 +545,10 @@ __global__ __launch_bounds__(256) void corr3_split_kernel(const float* __restric
     const float r1 = v - static_cast<float>(hi);
     const __bf16 mid = static_cast<__bf16>(r1);
     const __bf16 lo = static_cast<__bf16>(r1 - static_cast<float>(mid));
-    uint16_t* q = dst + static_cast<int64_t>(px) * (3 * C) + tx;
+    uint16_t* q = dst + static_cast<int64_t>(px) * (3 * Cp) + tx;
     q[0] = __builtin_bit_cast(uint16_t, hi);
-    q[C] = __builtin_bit_cast(uint16_t, mid);
-    q[2 * C] = __builtin_bit_cast(uint16_t, lo);
+    q[Cp] = __builtin_bit_cast(uint16_t, mid);
+    q[2 * Cp] = __builtin_bit_cast(uint16_t, lo);
   }
 }
 
@@ -574,25 +577,39 @@ __device__ __forceinline__ int corr3_find(const Corr3Args& a, int w, bool by_til
   return pi;
 }
 
+// Tile t of an upper triangle, its columns' tiles one after the other: the column of tiles.
+__device__ __forceinline__ int corr3_column(int t) {
+  int n = static_cast<int>((sqrtf(8.f * static_cast<float>(t) + 1.f) - 1.f) * 0.5f);
+  n += (n + 1) * (n + 2) / 2 <= t;
+  n -= n * (n + 1) / 2 > t;
+  return n;
+}
+
 // One work group per (product, split of the positions, tile of 64 WR channels x 64 WC columns), four waves of 64 x 64.
-template <int WR, int WC>
+// WINDOW: one product, of all taps with all taps, by the tiles of its upper triangle.
+template <int WR, int WC, bool WINDOW>
 __global__ __launch_bounds__(256, 1) void corr3_products_kernel(Corr3Args a) {
   constexpr int BR = 64 * WR, BC = 64 * WC, CBR = BR / 32, CBC = BC / 32, BLOCKS = 3 * (CBR + CBC);
-  constexpr int LOADS = (BLOCKS + 3) / 4, STAGE = 4 * LOADS * 1024, S = kC3Stages;
-  static_assert(WR * WC == 4 && kC3Chunk % 2 == 0, "four waves; two stages at a time");
+  constexpr int LOADS = (BLOCKS + 3) / 4, STAGE = 4 * LOADS * 1024, S = kC3Stages, CHUNK = WINDOW ? 16 : 32;      // stages whose sums join a total
+  static_assert(WR * WC == 4 && (!WINDOW || WR == WC), "four waves; two stages at a time");
   extern __shared__ __attribute__((aligned(1024))) unsigned char dtl_smem[];
   AK_LDS unsigned char* lds = (AK_LDS unsigned char*)dtl_smem;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave / WC, wc = wave % WC;
   // the main product's items, an XCD's in a row, then the corrections' in the tail (in one row, the last XCDs had all of those)
-  const int first = a.prod[1].first_item, blk0 = static_cast<int>(blockIdx.x);
+  const int first = WINDOW ? static_cast<int>(gridDim.x) : a.prod[1].first_item, blk0 = static_cast<int>(blockIdx.x);
   const int w = blk0 < first ? static_cast<int>(xcd_contiguous_id(blk0, first)) : blk0;
-  const Corr3Prod& cp = a.prod[corr3_find(a, w, false)];
-  const int local = w - cp.first_item, ntiles = a.tiles_m * cp.tiles_n;
-  const int split = local / ntiles, t = local - split * ntiles, tn = t / a.tiles_m, tm = t - tn * a.tiles_m;
+  const Corr3Prod& cp = a.prod[WINDOW ? 0 : corr3_find(a, w, false)];
+  const int local = w - cp.first_item, ntiles = WINDOW ? a.tiles_m * (a.tiles_m + 1) / 2 : a.tiles_m * cp.tiles_n;
+  const int split = local / ntiles, t = local - split * ntiles;
+  int tn = t / a.tiles_m, tm = t - tn * a.tiles_m;
+  if constexpr (WINDOW) {
+    tn = corr3_column(t);
+    tm = t - tn * (tn + 1) / 2;
+  }
   const int row0 = tm * BR, col0 = tn * BC;
-  if (corr3_below(a, row0, col0, BC)) return;
+  if (!WINDOW && corr3_below(a, row0, col0, BC)) return;
   const int k0 = split * cp.k_split, k1 = min(k0 + cp.k_split, (cp.M + kC3K - 1) / kC3K);
 
   u32x4 rsrc;
@@ -608,11 +625,13 @@ __global__ __launch_bounds__(256, 1) void corr3_products_kernel(Corr3Args a) {
   for (int l = 0; l < LOADS; ++l) {
     const int blk = wave + 4 * l;
     uint32_t at = kDtlOob;
-    if (blk < 3 * CBR) {
-      at = static_cast<uint32_t>((blk / CBR) * a.C + row0 + 32 * (blk % CBR)) * 2u;
-    } else if (blk < BLOCKS) {
-      const int b = blk - 3 * CBR, col = col0 + 32 * (b % CBC), tap = col / a.C;
-      if (tap < cp.ntaps) at = cp.toff[tap] + static_cast<uint32_t>((b / CBC) * a.C + col - tap * a.C) * 2u;
+    const bool of_a = blk < 3 * CBR;
+    const int b = of_a ? blk : blk - 3 * CBR, blocks = of_a ? CBR : CBC, plane = b / blocks;
+    const int col = (of_a ? row0 : col0) + 32 * (b % blocks), tap = col / a.C;
+    if (blk < BLOCKS && tap < cp.ntaps) {
+      at = static_cast<uint32_t>(plane * a.C + col - tap * a.C) * 2u;
+      if constexpr (WINDOW) at += static_cast<uint32_t>(tap / cp.kw) * cp.pitch + static_cast<uint32_t>(tap % cp.kw) * static_cast<uint32_t>(6 * a.C);
+      else at += of_a ? 0u : cp.toff[tap];
     }
     block_at[l] = __builtin_amdgcn_readfirstlane(at);
   }
@@ -694,29 +713,47 @@ __global__ __launch_bounds__(256, 1) void corr3_products_kernel(Corr3Args a) {
   Fragments even, odd;
 #pragma unroll
   for (int u = 0; u < 12; ++u) read_one(even, 0, u);
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) small[x][y][r] = 0.f;
   int stage = 0;                               // of k-tile kt; (the stages behind the last one hold zeros)
-  for (int c = k0; c < k1; c += kC3Chunk) {
+  for (int c = k0; c < k1; c += CHUNK) {
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int y = 0; y < 2; ++y)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) big[x][y][r] = small[x][y][r] = 0.f;
-    const int end = min(c + kC3Chunk, k1);
+        for (int r = 0; r < 16; ++r) big[x][y][r] = 0.f;
+    const int end = min(c + CHUNK, k1);
     for (int kt = c; kt < end; kt += 2) {
       step(kt, ((stage + 1) & (S - 1)) * STAGE, (stage + S - 1) & (S - 1), even, odd);
       step(kt + 1, ((stage + 2) & (S - 1)) * STAGE, (stage + S) & (S - 1), odd, even);
       stage = (stage + 2) & (S - 1);
     }
+    // what a total rounds away goes to the small products' accumulator, which holds 2^-8 of the others and runs on to the end
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int y = 0; y < 2; ++y)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tot[x][y][r] += big[x][y][r] + small[x][y][r];
+        for (int r = 0; r < 16; ++r) {
+          const float t = tot[x][y][r], v = big[x][y][r], sum = t + v, more = sum - t;
+          small[x][y][r] += (t - (sum - more)) + (v - more);
+          tot[x][y][r] = sum;
+        }
   }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (!__builtin_isinf(tot[x][y][r])) tot[x][y][r] += small[x][y][r];
   wait_vmcnt<0>();                             // the loads behind the last stage, before the LDS is released
-  if (cp.nsplit == 1) {
+  if (!WINDOW && cp.nsplit == 1) {
     const int l32 = lane & 31;
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -826,7 +863,7 @@ static Corr3Plan corr3_plan_build(int64_t N, int64_t C, int64_t H, int64_t W) {
   constexpr int64_t kEngines = 32, kCus = 8, kItem = 13;
   const int64_t main_tiles = static_cast<int64_t>(a.tiles_m) * a.prod[0].tiles_n, all = stages(a.prod[0]);
   auto chains = [&](const Corr3Prod& p, int64_t len) { return (stages(p) + len - 1) / len; };
-  int64_t best = 1, best_chain = kC3Chunk;
+  int64_t best = 1, best_chain = 32;
   double best_time = 0;
   for (int64_t chain : {32, 16, 8})
     for (int64_t ns = 1; ns <= std::max<int64_t>(1, std::min<int64_t>(all / 4, 2 * kEngines * kCus / main_tiles + 1)); ++ns) {
@@ -902,11 +939,11 @@ static int corr3_launch(const Corr3Plan& pl, const Corr3Args& args, hipStream_t 
   constexpr int kLds = kC3Stages * 4 * ((6 * (WR + WC) + 3) / 4) * 1024;
   static bool attr_set = false;     // idempotent; a race sets it twice at worst
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(corr3_products_kernel<WR, WC>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(corr3_products_kernel<WR, WC, false>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
       return AK_ERR_LAUNCH;
     attr_set = true;
   }
-  hipLaunchKernelGGL((corr3_products_kernel<WR, WC>), dim3(static_cast<unsigned>(pl.items)), dim3(256), kLds, stream, args);
+  hipLaunchKernelGGL((corr3_products_kernel<WR, WC, false>), dim3(static_cast<unsigned>(pl.items)), dim3(256), kLds, stream, args);
   if (pl.part_f4 > 0)
     hipLaunchKernelGGL((corr3_reduce_kernel<WR, WC>), dim3(static_cast<unsigned>(pl.tiles), 16), dim3(256), 0, stream, args);
   return AK_OK;
@@ -926,10 +963,173 @@ int conv_corr_syrk_f32(const float* x, int64_t N, int64_t C, int64_t H, int64_t 
   args.part = reinterpret_cast<floatx4*>(base + part_at);
   args.red = reinterpret_cast<float*>(base + red_at);
   hipLaunchKernelGGL(corr3_split_kernel, dim3(static_cast<unsigned>(((H + 2) * (W + 2) + 31) / 32), static_cast<unsigned>(C / 32), static_cast<unsigned>(N)),
-                     dim3(256), 0, stream, x, reinterpret_cast<uint16_t*>(base), static_cast<int>(C), static_cast<int>(H), static_cast<int>(W));
+                     dim3(256), 0, stream, x, reinterpret_cast<uint16_t*>(base), static_cast<int>(C), static_cast<int>(C), static_cast<int>(H), static_cast<int>(W),
+                     static_cast<int>(H + 2), static_cast<int>(W + 2), 0, 2);
   const int rc = pl.wide ? corr3_launch<2, 2>(pl, args, stream) : corr3_launch<1, 4>(pl, args, stream);
   if (rc != AK_OK) return rc;
   return corr_assemble(args.red, C, alpha, beta, A, lda, stream);
+}
+
+// ---- other windows of fp32 inputs --------------------------------------------------------------------------------
+// A strided window has no shifts to share: its factor is the product of all taps with all taps over the output positions, on the same
+// planes and products, a tap another constant in the address of either operand.  The partial tiles lie in the order (tap, channel) of
+// the columns; their sum, in double, is put into the factor's order (channel, tap) by the last kernel, which reads them once.  Totals are
+// joined every 256 pixels, with what they round away: 3.0 to 4.9e-8 of the factor's norm from the one in 64 bits, the fp32 kernel's is
+// 4.1 to 6.7e-8 over the same 26 windows.
+
+// One work group per (32 channels of columns, 8 channels of rows, a tap of rows): 8 rows of 32 KK entries.  An entry is stored once, its
+// row before its column; the other way round it is read transposed.
+// (Many splits are few channels, and few work groups: a wave per tap of columns.)
+__global__ __launch_bounds__(1024) void corr3_window_kernel(Corr3Args a, int KK, int C, float alpha, float beta, float* __restrict__ A, int64_t lda) {
+  extern __shared__ float rows[];                      // [8][32 KK + 1]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x, t = blockIdx.z;
+  const int c0 = 8 * blockIdx.y, j0 = 32 * blockIdx.x, pitch = 32 * KK + 1, ntiles = a.tiles_m * (a.tiles_m + 1) / 2;
+  const int nsplit = a.prod[0].nsplit;
+  const int64_t stride = static_cast<int64_t>(ntiles) * 4096;
+  // float4 of rows 4 (r / 4) ... + 3 of column c, of a tile on or above the diagonal
+  auto place = [&](int r, int c) {
+    const int tm = r >> 7, tn = c >> 7, x = (r >> 5) & 1, q = (r >> 3) & 3, g = (r >> 2) & 1, y = (c >> 5) & 1;
+    return a.part + static_cast<int64_t>(tn * (tn + 1) / 2 + tm) * 4096 + ((x * 2 + y) * 4 + q) * 256 + (((r >> 6) & 1) * 2 + ((c >> 6) & 1)) * 64 + g * 32 + (c & 31);
+  };
+  for (int u = wave; u < KK; u += threads / 64) {
+    const int p0 = t * a.C + c0, q0 = u * a.C + j0;    // first row, first column
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](const floatx4* src) {
+      int s = 0;
+      for (; s + 8 <= nsplit; s += 8) {                // eight loads in flight
+        floatx4 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = src[(s + k) * stride];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[e] += static_cast<double>(v[k][e]);
+      }
+      for (; s < nsplit; ++s) {
+        const floatx4 v = src[s * stride];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += static_cast<double>(v[e]);
+      }
+    };
+    if ((p0 >> 5) < (q0 >> 5)) {
+      const int g = lane >> 5, l32 = lane & 31;
+      add(place(p0 + 4 * g, q0 + l32));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rows[(4 * g + e) * pitch + l32 * KK + u] = static_cast<float>(sum[e]);
+    } else if ((p0 >> 5) > (q0 >> 5)) {
+      const int r = 4 * (lane >> 3), c = lane & 7;
+      add(place(q0 + r, p0 + c));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rows[c * pitch + (r + e) * KK + u] = static_cast<float>(sum[e]);
+    } else {
+      const int g = lane >> 5, l32 = lane & 31;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = p0 + 4 * g + e, j = q0 + l32, r = min(i, j);
+        const float* src = reinterpret_cast<const float*>(place(r, max(i, j))) + (r & 3);
+        double one = 0.0;
+        for (int s = 0; s < nsplit; ++s) one += static_cast<double>(src[4 * s * stride]);
+        rows[(4 * g + e) * pitch + l32 * KK + u] = static_cast<float>(one);
+      }
+    }
+  }
+  __syncthreads();
+  const int width = min(32, C - j0) * KK;
+  for (int r = 0; r < 8; ++r) {
+    if (c0 + r >= C) return;
+    float* __restrict__ dst = A + (static_cast<int64_t>(c0 + r) * KK + t) * lda + static_cast<int64_t>(j0) * KK;
+    for (int j = tid; j < width; j += threads) {
+      const float v = alpha * rows[r * pitch + j];
+      dst[j] = beta != 0.f ? beta * dst[j] + v : v;
+    }
+  }
+}
+
+struct Corr3Window {
+  int64_t Cp, Hp, Wp, Ho, Wo, plane_bytes;
+  Corr3Args args;
+  int items;
+  size_t part_at, ws_bytes;
+};
+
+static bool corr3_window_plan(Corr3Window& v, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
+  v = Corr3Window{};
+  v.Ho = (H + 2 * ph - kh) / sh + 1;
+  v.Wo = (W + 2 * pw - kw) / sw + 1;
+  v.Cp = (C + 31) / 32 * 32;
+  v.Hp = (v.Ho - 1) * sh + kh;
+  v.Wp = (v.Wo - 1) * sw + kw;
+  const int64_t px = 6 * v.Cp, KK = static_cast<int64_t>(kh) * kw, d = KK * v.Cp, M = N * v.Ho * v.Wo;
+  if (!corr_enabled() || H + 2 * ph < kh || W + 2 * pw < kw || KK == 1 || KK > 32 || N > 65535 || v.Hp * v.Wp > (1 << 30) || d > 32768) return false;
+  v.plane_bytes = N * v.Hp * v.Wp * px;
+  if (v.plane_bytes + 64 * px > static_cast<int64_t>(kDtlRange) || (M + 1024) * std::max(v.Ho, v.Wo) >= (1ll << 32)) return false;
+  Corr3Args& a = v.args;
+  Corr3Prod& p = a.prod[0];
+  a.bytes = static_cast<uint32_t>(v.plane_bytes);
+  a.C = static_cast<int32_t>(v.Cp);
+  a.tiles_m = static_cast<int32_t>((d + 127) / 128);
+  p.sn = static_cast<uint32_t>(v.Hp * v.Wp * px); p.sy = static_cast<uint32_t>(sh * v.Wp * px); p.sx = static_cast<uint32_t>(sw * px);
+  p.M = static_cast<int32_t>(M); p.Ho = static_cast<int32_t>(v.Ho); p.Wo = static_cast<int32_t>(v.Wo);
+  p.mWo = make_magic(p.Wo); p.mHo = make_magic(p.Ho);
+  p.ntaps = static_cast<int32_t>(KK); p.kw = kw; p.pitch = static_cast<uint32_t>(v.Wp * px);
+  p.tiles_n = a.tiles_m;
+  // as few rounds of stages as the device takes, an item 13 of its own and the partial tiles one per 20 (corr3_plan_build)
+  const int64_t tiles = static_cast<int64_t>(a.tiles_m) * (a.tiles_m + 1) / 2, all = (M + kC3K - 1) / kC3K;
+  int64_t best = 1;
+  double best_time = 0;
+  for (int64_t ns = 1; ns <= std::max<int64_t>(1, std::min<int64_t>(all / 4, 512 / tiles + 1)); ++ns) {
+    const double time = static_cast<double>((tiles * ns + 255) / 256 * ((all + ns - 1) / ns + 13)) + 0.05 * static_cast<double>(tiles * ns);
+    if (ns == 1 || time < best_time) best = ns, best_time = time;
+  }
+  p.k_split = static_cast<int32_t>(((all + best - 1) / best + 1) / 2 * 2);
+  p.nsplit = static_cast<int32_t>((all + p.k_split - 1) / p.k_split);
+  v.items = static_cast<int>(tiles * p.nsplit);
+  v.part_at = (static_cast<size_t>(v.plane_bytes) + 255) & ~static_cast<size_t>(255);
+  v.ws_bytes = v.part_at + static_cast<size_t>(v.items) * 65536;
+  return true;
+}
+
+// Against the fp32 kernel of syrk_window.hpp, which multiplies 64 x 64 tiles at 46 to 82 TFLOP/s: here 20 us for three launches, 3 TB/s
+// into the planes, 110 TFLOP/s of 128 x 128 tiles of padded channels (a sixth of that is the matrix cores' bf16 rate) and the latency
+// of the splits' sum.  us there and here: samples x channels x image, 3 x 3 / 2: 128 x 64 x 32 x 32 231 and 115, 32 x 64 x 32 x 32 73 and 50,
+// 8 x 64 x 32 x 32 28 and 34, 128 x 96 x 8 x 8 39 and 38, 128 x 192 x 4 x 4 34 and 36, 32 x 300 x 14 x 14 188 and 125; 3 x 3 / 1:
+// 128 x 32 x 32 x 32 270 and 162, 128 x 32 x 16 x 16 75 and 76, 128 x 20 x 32 x 32 140 and 157, 128 x 24 x 32 x 32 183 and 157,
+// 128 x 96 x 16 x 16 391 and 163; 5 x 5 of 16 x 24 x 56 x 56 295 and 214; 2 x 2 / 2 of 128 x 64 x 16 x 16 34 and 60.
+static bool corr3_window_faster(const Corr3Window& v, int64_t C, int kh, int kw) {
+  const double M = v.args.prod[0].M, T = static_cast<double>((C * kh * kw + 63) / 64), tiles = static_cast<double>(v.items / v.args.prod[0].nsplit);
+  const double there = T * (T + 1) / 2 * 8192 * M / 55e6;
+  const double here = 20 + static_cast<double>(v.plane_bytes) / 3e6 + tiles * 16384 * M / 110e6 + 0.6 * v.args.prod[0].nsplit;
+  return here < there;
+}
+
+size_t conv_window_f32_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
+  Corr3Window v;
+  return corr3_window_plan(v, N, C, H, W, kh, kw, sh, sw, ph, pw) && corr3_window_faster(v, C, kh, kw) ? v.ws_bytes : 0;
+}
+
+int conv_window_syrk_f32(const float* x, int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw, float alpha,
+                         float beta, float* A, int64_t lda, void* ws, size_t ws_bytes, hipStream_t stream) {
+  Corr3Window v;
+  if (!corr3_window_plan(v, N, C, H, W, kh, kw, sh, sw, ph, pw) || !corr3_window_faster(v, C, kh, kw)) return AK_ERR_UNSUPPORTED;
+  if (ws == nullptr || ws_bytes < v.ws_bytes || (reinterpret_cast<uintptr_t>(ws) & 255) != 0) return AK_ERR_WORKSPACE;
+  constexpr int kLds = kC3Stages * 4 * 6 * 1024;
+  static bool attr_set = false;     // idempotent; a race sets it twice at worst
+  if (!attr_set) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(corr3_products_kernel<2, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return AK_ERR_LAUNCH;
+    attr_set = true;
+  }
+  unsigned char* base = static_cast<unsigned char*>(ws);
+  const int KK = kh * kw;
+  v.args.planes = base;
+  v.args.part = reinterpret_cast<floatx4*>(base + v.part_at);
+  hipLaunchKernelGGL(corr3_split_kernel, dim3(static_cast<unsigned>((v.Hp * v.Wp + 31) / 32), static_cast<unsigned>(v.Cp / 32), static_cast<unsigned>(N)),
+                     dim3(256), 0, stream, x, reinterpret_cast<uint16_t*>(base), static_cast<int>(C), static_cast<int>(v.Cp), static_cast<int>(H),
+                     static_cast<int>(W), static_cast<int>(v.Hp), static_cast<int>(v.Wp), ph, pw);
+  hipLaunchKernelGGL((corr3_products_kernel<2, 2, true>), dim3(static_cast<unsigned>(v.items)), dim3(256), kLds, stream, v.args);
+  hipLaunchKernelGGL(corr3_window_kernel, dim3(static_cast<unsigned>(v.Cp / 32), static_cast<unsigned>((C + 7) / 8), static_cast<unsigned>(KK)), dim3(v.args.prod[0].nsplit > 8 ? 64 * std::min(KK, 16) : 256),
+                     8 * (32 * KK + 1) * sizeof(float), stream, v.args, KK, static_cast<int>(C), alpha, beta, A, lda);
+  return check_launch();
 }
 
 }  // namespace ak

@@ -594,6 +594,7 @@ extern "C" size_t ak_conv_syrk_ws_bytes_of(int dtype, int64_t N, int64_t C, int6
   size_t need = 0;
   if (dtype != AK_BF16) need = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
   if (dtype == AK_F32) {
+    if (need == 0) need = ak::conv_window_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
     if (conv_wave_window(C, H, W, kh, kw, sh, sw, ph, pw)) need = std::max(need, ak::syrk_wave_ws_bytes(C, N * H * W));
     const int64_t Ho = (H + 2 * ph - kh) / sh + 1, Wo = (W + 2 * pw - kw) / sw + 1;
     if (H + 2 * ph >= kh && W + 2 * pw >= kw && ak::syrk_window_faster(N, C, H, W, kh, kw, sh, sw, Ho, Wo))
@@ -631,6 +632,11 @@ extern "C" int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int6
     const int rc = ak::conv_corr_syrk_f32(static_cast<const float*>(x), N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, A,
                                           lda, ws, ws_bytes, static_cast<hipStream_t>(stream));
     if (rc != AK_ERR_UNSUPPORTED) return rc;
+  }
+  if (dtype == AK_F32 && !in_order && lda >= C * kh * kw) {
+    const int rc = ak::conv_window_syrk_f32(static_cast<const float*>(x), N, C, H, W, kh, kw, sh, sw, ph, pw, alpha, beta, A, lda, ws, ws_bytes,
+                                            static_cast<hipStream_t>(stream));
+    if (rc != AK_ERR_UNSUPPORTED && rc != AK_ERR_WORKSPACE) return rc;
   }
   if (dtype == AK_F32 && !in_order && conv_wave_window(C, H, W, kh, kw, sh, sw, ph, pw) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && lda >= C) {
     const int rc = ak::launch_syrk_wave(static_cast<const float*>(x), C, N * H * W, H * W, C * H * W, static_cast<int>(H * W), alpha,

@@ -501,7 +501,8 @@ def main():
             out['roofline']['kernel'] = ('factor statistics of fp32 NCHW operands: the 3x3 stride-1 layers as shifted '
                                          'correlations of three bf16 planes of the input (corr3_split_kernel, '
                                          'corr3_products_kernel, corr3_reduce_kernel, corr_assemble_kernel: bf16 matrix '
-                                         'cores, fp32 accuracy), the others on syrk_window_kernel, syrk_wave_kernel, '
+                                         'cores, fp32 accuracy), the strided ones on the same planes (corr3_window_kernel), '
+                                         'the others on syrk_wave_kernel, '
                                          'conv_patch_syrk_kernel<float> (v_mfma_f32_32x32x2_f32); '
                                          'SYRK FLOP M*d*(d+1) against the fp32 matrix peak, the rate the reference\'s '
                                          'fp32 arithmetic is priced at')

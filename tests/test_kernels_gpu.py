@@ -1643,6 +1643,44 @@ def test_fp32_correlations_of_small_and_odd_images(K, N, C, H, W):
     assert bool((guard[0] == 7).all()) and bool((guard[-1] == 7).all())
 
 
+WINDOWS_ON_PLANES = [(128, 24, 32, 32, (3, 3), (1, 1), (1, 1)), (65, 64, 32, 31, (3, 3), (2, 2), (1, 1)), (130, 100, 14, 13, (3, 3), (2, 1), (1, 0)),
+                     (37, 70, 21, 20, (5, 3), (1, 2), (2, 0)), (128, 256, 8, 8, (3, 3), (2, 2), (1, 1)), (33, 200, 15, 15, (2, 3), (1, 2), (0, 1)),
+                     (90, 33, 17, 30, (5, 5), (3, 3), (4, 4)), (301, 96, 3, 5, (3, 3), (1, 1), (1, 1)), (2, 130, 40, 67, (1, 7), (1, 1), (0, 3))]
+
+
+@pytest.mark.parametrize("N,C,H,W,k,s,p", WINDOWS_ON_PLANES)
+def test_fp32_windows_on_bf16_planes(K, N, C, H, W, k, s, p):
+    """Strided and other windows of an fp32 input on its three bf16 planes: channels that fill no 32, frames that cut the image off or
+    reach beyond it, several splits and one."""
+    from asdl_amd import _lib
+    g = torch.Generator().manual_seed(N + C)
+    Ho, Wo, d = (H + 2 * p[0] - k[0]) // s[0] + 1, (W + 2 * p[1] - k[1]) // s[1] + 1, C * k[0] * k[1]
+    planes = N * ((Ho - 1) * s[0] + k[0]) * ((Wo - 1) * s[1] + k[1]) * 6 * ((C + 31) // 32 * 32)
+    assert _lib.load().ak_conv_syrk_ws_bytes_of(0, N, C, H, W, *k, *s, *p) >= planes
+    scale = torch.exp(torch.linspace(-20, 20, C)[torch.randperm(C, generator=g)])[None, :, None, None]
+    x = torch.randn(N, C, H, W, generator=g).relu().cuda() * scale.cuda()
+    rows = nn.functional.unfold(x.double(), k, 1, p, s).permute(0, 2, 1).reshape(-1, d)
+    ref = rows.T @ rows
+    guard = torch.full((d + 2, d + 3), 7.0, device='cuda')
+    out = K.conv_syrk(x, k, s, p, out=guard[1:-1, 1:-2])
+    # against the norms of the channels: 16 sums of 16 products round at most 2^-24 of their partial sum each, and so does the result; the
+    # pieces left out are below 2^-24 of a product
+    norm = x.double().pow(2).sum(dim=(0, 2, 3)).sqrt().clamp_min(1e-30).repeat_interleave(k[0] * k[1])
+    bound = 24 * 2.0 ** -24
+    assert float(((out.double() - ref) / norm / norm[:, None]).abs().max()) < bound
+    assert torch.equal(out, out.T)
+    before = out.clone()
+    K.conv_syrk(x, k, s, p, out=guard[1:-1, 1:-2], alpha=0.5, beta=2.0)
+    assert float(((out.double() - 2.5 * ref) / norm / norm[:, None]).abs().max()) < 3 * bound
+    assert bool((guard[0] == 7).all()) and bool((guard[-1] == 7).all()) and bool((guard[:, 0] == 7).all()) and bool((guard[:, -2:] == 7).all())
+    # a channel that is not finite spoils its own entries only
+    x[0, 3, H // 2, W // 2], x[1, 9, H // 2, W // 2] = float("inf"), float("nan")
+    spoiled = K.conv_syrk(x, k, s, p).view(C, -1, C, k[0] * k[1])
+    keep = [c for c in range(C) if c not in (3, 9)]
+    assert torch.equal(spoiled[keep][:, :, keep], before.view(C, -1, C, k[0] * k[1])[keep][:, :, keep])
+    assert not bool(torch.isfinite(spoiled[3, :, 3]).all()) and bool(torch.isnan(spoiled[9, :, 9]).any())
+
+
 @pytest.mark.parametrize("N,C,H", [(128, 64, 32), (128, 128, 16), (128, 256, 8)])
 def test_fp32_correlations_are_as_close_as_one_rounding_of_the_result(K, N, C, H):
     """Sums over 8192 to 131072 pixels of ReLU outputs: their accumulators round at the magnitude of a split, and the factor ends
