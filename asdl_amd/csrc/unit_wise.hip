@@ -162,6 +162,91 @@ static __global__ __launch_bounds__(256) void uw_cols_single_kernel(UwParams p) 
   dst[0] = ww; dst[1] = wb; dst[2] = bb;
 }
 
+// Four values of a row on their way.
+template <typename T> struct UwFour;
+template <> struct UwFour<float> {
+  floatx4 v;
+  __device__ __forceinline__ void load(const void* p, int64_t idx) { v = *reinterpret_cast<const floatx4*>(static_cast<const float*>(p) + idx); }
+  __device__ __forceinline__ float get(int e) const { return v[e]; }
+};
+template <> struct UwFour<uint16_t> {
+  uint2 v;
+  __device__ __forceinline__ void load(const void* p, int64_t idx) { v = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p) + idx); }
+  __device__ __forceinline__ float get(int e) const {
+    const uint32_t w = e < 2 ? v.x : v.y;
+    return __builtin_bit_cast(float, (e & 1) != 0 ? w & 0xffff0000u : w << 16);
+  }
+};
+
+// The same for whole fours of features (contiguous, aligned): 64 lanes of four features, the rows of a chunk dealt to eight waves, all
+// of a wave's loads in flight at once.  Bound by the memory.  With one element a load and one row at a time, every row was a memory
+// latency: 8192 x 768 in fp32 (50 MB) 40 us, on four waves here 20, on eight 14.
+constexpr int kUwWaves = 8;
+template <typename YT, typename GT>
+static __global__ __launch_bounds__(64 * kUwWaves) void uw_cols_single_vec_kernel(UwParams p) {
+  constexpr int AHEAD = 8;
+  __shared__ floatx4 red[kUwWaves - 1][3][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t f = static_cast<int64_t>(blockIdx.x) * 256 + 4 * lane, at = f < p.F ? f : 0;
+  const int64_t c = blockIdx.y, n0 = c * p.rows_per_chunk;
+  const int64_t n1 = n0 + p.rows_per_chunk < p.N ? n0 + p.rows_per_chunk : p.N;
+  float wf[4], bf[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    wf[e] = p.w[at + e];
+    bf[e] = p.b[at + e];
+  }
+  floatx4 ww = {0.f, 0.f, 0.f, 0.f}, wb = ww, bb = ww;
+  auto add = [&](const UwFour<YT>& y, const UwFour<GT>& g) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float gv = g.get(e), gw = (y.get(e) - bf[e]) / wf[e] * gv;
+      ww[e] += gw * gw;
+      wb[e] += gw * gv;
+      bb[e] += gv * gv;
+    }
+  };
+  int64_t n = n0 + wave;
+  for (; n + kUwWaves * (AHEAD - 1) < n1; n += kUwWaves * AHEAD) {
+    UwFour<YT> y[AHEAD];
+    UwFour<GT> g[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      y[u].load(p.y, (n + kUwWaves * u) * p.ysn + at);
+      g[u].load(p.g, (n + kUwWaves * u) * p.gsn + at);
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) add(y[u], g[u]);
+  }
+  for (; n < n1; n += kUwWaves) {
+    UwFour<YT> y;
+    UwFour<GT> g;
+    y.load(p.y, n * p.ysn + at);
+    g.load(p.g, n * p.gsn + at);
+    add(y, g);
+  }
+  if (wave > 0) {
+    red[wave - 1][0][lane] = ww;
+    red[wave - 1][1][lane] = wb;
+    red[wave - 1][2][lane] = bb;
+  }
+  __syncthreads();
+  if (wave > 0 || f >= p.F) return;
+#pragma unroll
+  for (int q = 0; q < kUwWaves - 1; ++q) {
+    ww += red[q][0][lane];
+    wb += red[q][1][lane];
+    bb += red[q][2][lane];
+  }
+  float* dst = p.part + (c * p.F + f) * 3;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    dst[3 * e] = ww[e];
+    dst[3 * e + 1] = wb[e];
+    dst[3 * e + 2] = bb[e];
+  }
+}
+
 // blocks[f] = beta*blocks[f] + alpha * sum over the partial rows; `width` 2: per-sample (gw, gb) in `chunks` pieces,
 // 3: product sums.  grid ceil(F/64), 1024 threads = 64 features x 16 row lanes; fixed summation order.
 static __global__ __launch_bounds__(1024) void uw_finalize_kernel(const float* __restrict__ part, int64_t rows, int64_t F,
@@ -361,8 +446,19 @@ extern "C" int ak_unit_wise_stats(const void* y, int y_dtype, int64_t ysn, int64
     rows = (N + kUwChunkRows - 1) / kUwChunkRows;
     width = 3;
     if (rows > 65535) return AK_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(uw_cols_single_kernel, dim3(static_cast<unsigned>((F + 255) / 256), static_cast<unsigned>(rows)),
-                       dim3(256), 0, s, p);
+    const dim3 grid(static_cast<unsigned>((F + 255) / 256), static_cast<unsigned>(rows));
+    auto fours = [](const void* x, int dtype, int64_t sn, int64_t sf) {
+      return sf == 1 && sn % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & (dtype == AK_BF16 ? 7 : 15)) == 0;
+    };
+    if (F % 4 != 0 || !fours(y, y_dtype, ysn, ysf) || !fours(g, g_dtype, gsn, gsf)) {
+      hipLaunchKernelGGL(uw_cols_single_kernel, grid, dim3(256), 0, s, p);
+    } else if (y_dtype == AK_BF16) {
+      if (g_dtype == AK_BF16) hipLaunchKernelGGL((uw_cols_single_vec_kernel<uint16_t, uint16_t>), grid, dim3(64 * kUwWaves), 0, s, p);
+      else hipLaunchKernelGGL((uw_cols_single_vec_kernel<uint16_t, float>), grid, dim3(64 * kUwWaves), 0, s, p);
+    } else {
+      if (g_dtype == AK_BF16) hipLaunchKernelGGL((uw_cols_single_vec_kernel<float, uint16_t>), grid, dim3(64 * kUwWaves), 0, s, p);
+      else hipLaunchKernelGGL((uw_cols_single_vec_kernel<float, float>), grid, dim3(64 * kUwWaves), 0, s, p);
+    }
   } else {
     rows = N;
     width = 2;

@@ -1239,6 +1239,28 @@ def test_unit_wise_stats_matches_oracle(K, dtype, kind, shape):
     assert relerr(out2, 1.0 * ref) < 1e-5
 
 
+@pytest.mark.parametrize('ydt,gdt', [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                     (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize('N,F', [(1, 4), (29, 12), (64, 256), (97, 260), (333, 768), (130, 770)])
+def test_unit_wise_stats_of_rows(K, ydt, gdt, N, F):
+    """Rows of features in fours and not, chunks of rows that end anywhere, rows with gaps between them and operands that no load of
+    four elements is aligned to."""
+    torch.manual_seed(N + F)
+    wide_y, wide_g = torch.randn(N, F + 8).to(ydt).cuda(), torch.randn(N, F + 9).to(gdt).cuda()
+    w, b = (torch.rand(F) + 0.5).cuda(), torch.randn(F).cuda()
+    for y, g in ((wide_y[:, :F].contiguous(), wide_g[:, :F].contiguous()), (wide_y[:, 4:F + 4], wide_g[:, :F]), (wide_y[:, 1:F + 1], wide_g[:, 4:F + 4]),
+                 (wide_y[:, :F].contiguous(), wide_g[:1, :F].contiguous().expand(N, F))):
+        gd = g.double()
+        gw = (y.double() - b.double()) / w.double() * gd
+        ref = torch.stack([(gw * gw).sum(0), (gw * gd).sum(0), (gw * gd).sum(0), (gd * gd).sum(0)], 1).view(F, 2, 2)
+        out = K.unit_wise_stats(y, g, w, b)
+        # a product's factors round three times, a chain is 8 rows, the joins 8 waves and the chunks: below 40 roundings of sums of N terms
+        size = ((gw * gw).sum(0) * (gd * gd).sum(0)).sqrt().clamp_min(1e-30)
+        err = (out.double() - ref).abs()
+        assert float((err[:, 0, 0] / ref[:, 0, 0]).max()) < 40 * 2.0 ** -24 and float((err[:, 1, 1] / ref[:, 1, 1]).max()) < 40 * 2.0 ** -24
+        assert float((err[:, 0, 1] / size).max()) < 40 * 2.0 ** -24 and torch.equal(out[:, 0, 1], out[:, 1, 0])
+
+
 def test_unit_wise_inv_and_mvp_match_oracle(K):
     torch.manual_seed(3)
     v = torch.randn(1000, 2, 3)
