@@ -193,6 +193,7 @@ struct LanczosGroup {
   const float* S;
   const float* v0;
   float* vec;
+  float* parts;
   int64_t strideS;
   int n, batch, z0, pad;
 };
@@ -204,7 +205,7 @@ struct LanczosGroups {
 // Lanczos step j: q_j from S q_{j-1}, then its work group's rows of S q_j.  Every work group of a matrix forms q_j for
 // itself in the LDS (three vectors from the L2, two reductions): one launch per step, no hand-over inside it.  The
 // rows of S are requested before that, their first 1024 columns kept in registers.
-// Bound by the launch and the chain of loads and reductions for small n, by reading S for a full batch.
+// Bound by the launch and the chain of loads and reductions; where it would be by reading S, root_lanczos_tiles_kernel reads half.
 // WIDE: vectors that the LDS does not hold (kLanczosLdsDim) are formed again, element by element, where they are used.
 // HELD: at most 1024 columns, and work groups that wait rather than fill the memory: the three vectors come into registers and are
 // requested first (loads return in order), then the rows of S, none under a lane's own condition, which would be waited for by
@@ -363,6 +364,153 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
     const float s = wave_sum(acc[r]);
     if (lane == 0 && row0 + r < n) wj[row0 + r] = s;
   }
+}
+
+// Lanczos steps of many large statistics, bound by reading S: its lower triangle alone, by tiles of 256 x 256 that serve both sides, and
+// the sum of their parts and the vectors in a launch between, a work group per matrix.  98 matrices of up to 3072 columns (1.3 GB):
+// a step 229 us, now 135 (8 rows' loads at a time instead of 16: 144) and 13.  From which sum of bytes on: the whole roots cut off after
+// one step, by whole rows and by halves, 3 x 3072 (113 MB) 2.24 and 2.32 ms, 5 x 3072 3.22 and 3.10, 11 x 3072 6.82 and 5.61;
+// 40 x 768 (94 MB) 1.32 and 1.35, 80 x 768 2.24 and 1.96.
+constexpr int kLanczosTile = 256;
+constexpr int64_t kLanczosHalfBytes = 128ll << 20;
+// parts: [batch][block of rows][block of columns][256], in the matrix buffers, which nothing else uses yet
+__device__ __forceinline__ float* lanczos_parts(float* bufs, int nb, int zl) { return bufs + static_cast<int64_t>(zl) * nb * nb * kLanczosTile; }
+
+// The parts of S q_j.
+static __global__ __launch_bounds__(256) void root_lanczos_tiles_kernel(RootState st, LanczosGroups L, int j) {
+  constexpr int ROWS = 16, LANES = 64 / ROWS;
+  __shared__ floatx4 sums[4][64];
+  const int wg = blockIdx.x;
+  int gi = 0;
+#pragma unroll
+  for (int k = 1; k < kRootMaxGroups; ++k) gi += wg >= L.first[k] ? 1 : 0;
+  const LanczosGroup g = L.g[gi];
+  const int n = g.n, nb = (n + kLanczosTile - 1) / kLanczosTile, per = nb * (nb + 1) / 2;
+  const int local = wg - L.first[gi], zl = local / per, t = local - zl * per;
+  if (j > 0 && st.lz_dim[g.z0 + zl] != 0) return;
+  int bi, bj;
+  decode_lower_tile(t, bi, bj);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row0 = kLanczosTile * bi + 64 * wave, col = kLanczosTile * bj + 4 * lane;
+  const float* __restrict__ S = g.S + zl * g.strideS;
+  const float* __restrict__ q = g.vec + (j % 3) * (static_cast<int64_t>(g.batch) * n) + static_cast<int64_t>(zl) * n;
+  float* __restrict__ parts = lanczos_parts(g.parts, nb, zl);
+  const bool whole = kLanczosTile * (bj + 1) <= n;         // (the last tile of the diagonal may reach beyond the matrix)
+  floatx4 x = {0.f, 0.f, 0.f, 0.f}, down = x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (col + e < n) x[e] = q[col + e];
+  const float mine = row0 + lane < n ? q[row0 + lane] : 0.f;
+  auto sweep = [&](auto whole_tag) {
+    for (int r0 = 0; r0 < 64; r0 += ROWS) {
+      floatx4 m[ROWS];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {                     // (rows beyond the end read the last one, times zero)
+        const float* __restrict__ src = S + static_cast<int64_t>(min(row0 + r0 + r, n - 1)) * n;
+        if constexpr (decltype(whole_tag)::value) m[r] = *reinterpret_cast<const floatx4u*>(src + col);
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e) m[r][e] = src[min(col + e, n - 1)];
+      }
+      float v[ROWS];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const float y = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), r0 + r));
+        v[r] = m[r][0] * x[0] + m[r][1] * x[1] + m[r][2] * x[2] + m[r][3] * x[3];
+        down += m[r] * y;
+      }
+      // the rows' sums over the lanes, half as many with every exchange: lanes LANES r ... end with row r's
+#pragma unroll
+      for (int o = 32, h = ROWS / 2; h >= 1; o >>= 1, h >>= 1)
+#pragma unroll
+        for (int r = 0; r < h; ++r) {
+          const bool up = (lane & o) != 0;
+          v[r] = (up ? v[r + h] : v[r]) + __shfl_xor(up ? v[r] : v[r + h], o);
+        }
+#pragma unroll
+      for (int o = LANES / 2; o >= 1; o >>= 1) v[0] += __shfl_xor(v[0], o);
+      if (lane % LANES == 0) parts[static_cast<int64_t>(bi * nb + bj) * kLanczosTile + 64 * wave + r0 + lane / LANES] = v[0];
+    }
+  };
+  if (whole) sweep(std::true_type{});
+  else sweep(std::false_type{});
+  if (bi == bj) return;
+  sums[wave][lane] = down;
+  __syncthreads();
+  const float* all = reinterpret_cast<const float*>(sums);
+  parts[static_cast<int64_t>(bj * nb + bi) * kLanczosTile + tid] = (all[tid] + all[256 + tid]) + (all[512 + tid] + all[768 + tid]);
+}
+
+// Sum over the 1024 threads of a work group; red: 16 floats of this sum's own.
+__device__ __forceinline__ float block_sum_1024(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) s += red[k];
+  return s;
+}
+
+// S q_{j-1} from its parts, T's entries and q_j (root_lanczos_kernel's); j = steps: S q_{j-1} alone, for T's last entry.  grid (total).
+static __global__ __launch_bounds__(1024) void root_lanczos_vector_kernel(RootState st, LanczosGroups L, int j, int steps) {
+  __shared__ float red[2][16];
+  const int z = blockIdx.x, tid = threadIdx.x;
+  int gi = 0;
+#pragma unroll
+  for (int k = 1; k < kRootMaxGroups; ++k) gi += L.first[k] != INT32_MAX && z >= L.g[k].z0 ? 1 : 0;
+  const LanczosGroup g = L.g[gi];
+  const int n = g.n, nb = (n + kLanczosTile - 1) / kLanczosTile, zl = z - g.z0;
+  const int64_t vec = static_cast<int64_t>(g.batch) * n, at = static_cast<int64_t>(zl) * n;
+  float* __restrict__ qj = g.vec + (j % 3) * vec + at;
+  if (j == 0) {
+    const float* __restrict__ v0 = g.v0 + at;
+    float s = 0.f;
+    for (int i = tid; i < n; i += 1024) s += v0[i] * v0[i];
+    const float inv = 1.f / sqrtf(block_sum_1024(s, red[0]));
+    for (int i = tid; i < n; i += 1024) qj[i] = v0[i] * inv;
+    if (tid == 0) {
+      st.lz_dim[z] = 0;
+      st.active[z] = st.count[z] = 0;
+      st.settled[z] = 0.f;
+      root_clear_words(st, z);
+      root_clear_words(st, st.total + z);
+      st.beta[z * kLanczosSteps] = 0.f;
+    }
+    return;
+  }
+  if (st.lz_dim[z] != 0) return;
+  const float* __restrict__ q1 = g.vec + ((j + 2) % 3) * vec + at;
+  const float* __restrict__ q2 = g.vec + ((j + 1) % 3) * vec + at;
+  float* __restrict__ w = g.vec + (3 + ((j + 1) & 1)) * vec + at;
+  const float* __restrict__ parts = lanczos_parts(g.parts, nb, zl);
+  const float b = st.beta[z * kLanczosSteps + j - 1];
+  float s = 0.f;
+  for (int i = tid; i < n; i += 1024) {
+    const float* __restrict__ src = parts + static_cast<int64_t>(i / kLanczosTile) * nb * kLanczosTile + i % kLanczosTile;
+    float x = 0.f;
+#pragma unroll 4
+    for (int c = 0; c < nb; ++c) x += src[c * kLanczosTile];
+    w[i] = x;
+    s += x * q1[i];
+  }
+  if (j == steps) return;
+  const float a = block_sum_1024(s, red[0]);
+  s = 0.f;
+  for (int i = tid; i < n; i += 1024) {                    // (a thread's own elements of w)
+    const float x = w[i] - a * q1[i] - (j > 1 ? b * q2[i] : 0.f);
+    w[i] = x;
+    s += x * x;
+  }
+  const float norm = sqrtf(block_sum_1024(s, red[1]));
+  const bool done = !(norm > 1e-7f * fabsf(a));
+  if (tid == 0) {
+    st.alpha[z * kLanczosSteps + j - 1] = a;
+    if (done) st.lz_dim[z] = j;
+    else st.beta[z * kLanczosSteps + j] = norm;
+  }
+  if (done) return;
+  const float inv = 1.f / norm;
+  for (int i = tid; i < n; i += 1024) qj[i] = w[i] * inv;
 }
 
 template <int CTRL>
@@ -1295,14 +1443,17 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
   if (phases & 1) {
     const int steps = std::min(kLanczosSteps, std::max(1, max_power_iter));
     LanczosGroups L;
-    int blocks = 0, widest = 0;
+    int blocks = 0, widest = 0, narrowest = INT32_MAX;
+    int64_t bytes = 0;
     for (int i = 0; i < kRootMaxGroups; ++i) {
       L.first[i] = i < G.count ? blocks : INT32_MAX;
       if (i >= G.count) continue;
       const RootGroup& g = G.g[i];
-      L.g[i] = LanczosGroup{g.S, g.v0, g.vec, g.strideS, g.n, g.batch, g.z0, 0};
+      L.g[i] = LanczosGroup{g.S, g.v0, g.vec, g.bufs, g.strideS, g.n, g.batch, g.z0, 0};
       blocks += g.batch * ((g.n + kLanczosRows - 1) / kLanczosRows);
       widest = std::max(widest, g.n);
+      narrowest = std::min(narrowest, g.n);
+      bytes += static_cast<int64_t>(4) * g.batch * g.n * g.n;
     }
     const bool wide = widest > kLanczosLdsDim, held = widest <= 1024 && blocks <= 512;       // (two work groups a CU)
     const size_t lds = static_cast<size_t>(widest) * sizeof(float);
@@ -1313,7 +1464,21 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
         return AK_ERR_LAUNCH;
       attr_set = true;
     }
-    for (int j = 0; j < steps; ++j) {
+    // (from 64 columns on a matrix's buffers hold its parts)
+    const bool half = !wide && narrowest >= 64 && bytes >= kLanczosHalfBytes;
+    if (half) {
+      blocks = 0;
+      for (int i = 0; i < G.count; ++i) {
+        const int nb = (G.g[i].n + kLanczosTile - 1) / kLanczosTile;
+        L.first[i] = blocks;
+        blocks += G.g[i].batch * (nb * (nb + 1) / 2);
+      }
+      for (int j = 0; j <= steps; ++j) {
+        hipLaunchKernelGGL(root_lanczos_vector_kernel, gz, dim3(1024), 0, s, G.st, L, j, steps);
+        if (j < steps) hipLaunchKernelGGL(root_lanczos_tiles_kernel, dim3(blocks), b256, 0, s, G.st, L, j);
+      }
+    }
+    for (int j = 0; j < steps && !half; ++j) {
       if (wide) hipLaunchKernelGGL((root_lanczos_kernel<true, false>), dim3(blocks), b256, 0, s, G.st, L, j);
       else if (held) hipLaunchKernelGGL((root_lanczos_kernel<false, true>), dim3(blocks), b256, lds, s, G.st, L, j);
       else hipLaunchKernelGGL((root_lanczos_kernel<false, false>), dim3(blocks), b256, lds, s, G.st, L, j);

@@ -817,3 +817,30 @@ def test_models_whose_products_go_to_the_grouped_path_are_not_asked_at_every_ste
         maker.precondition()                     # (the preconditioners are identities)
         assert not calls
         assert all(relerr(pc.param.grad, g) < 1e-5 for pc, g in zip(maker.preconditioners, expected))
+
+
+def test_inv_root_lanczos_on_half_the_statistics():
+    """The Lanczos steps of 128 MB of statistics read the lower triangles by tiles, here of ragged sizes, against the same statistics in
+    calls small enough for whole rows."""
+    gen = torch.Generator('cuda').manual_seed(7)
+    items = []
+    for n, batch in ((2817, 4), (1700, 2), (513, 40), (65, 3), (256, 2)):
+        x = torch.randn(batch, 2 * n, n, device='cuda', generator=gen) * torch.logspace(0, -2, n, device='cuda')
+        S = torch.stack([m.t() @ m for m in x])
+        S = torch.tril(S) + torch.tril(S, -1).transpose(1, 2)
+        items.append((S.contiguous(), 4, torch.rand(batch, n, device='cuda', generator=gen), None))
+    assert sum(S.numel() * 4 for S, *_ in items) >= 128 << 20
+    together = K.inv_root_group([(S.clone(), p, v, out) for S, p, v, out in items], 1e-6)
+    for (S, p, v, _), (out, stats) in zip(items, together):
+        for z in range(0, S.shape[0], 7):
+            one, alone = K.inv_root_group([(S[z:z + 1].clone(), p, v[z:z + 1], None)], 1e-6)[0]
+            # the largest eigenvalue: T's entries round in another order, by a few 2^-24 a step
+            assert float((stats[z, 0] - alone[0, 0]).abs() / alone[0, 0].abs()) < 32 * 4 * 2.0 ** -24
+            root = out[z].double()
+            for _ in range(2):
+                root = root @ root
+            exact = torch.linalg.inv(S[z].double() + 1e-6 * float(alone[0, 0]) * torch.eye(S.shape[1], device='cuda', dtype=torch.float64))
+            own = one[0].double()
+            for _ in range(2):
+                own = own @ own
+            assert float((root - exact).norm()) <= 1.5 * float((own - exact).norm()) + 1e-6 * float(exact.norm())
