@@ -673,8 +673,9 @@ def main_shampoo(args, dev, steps=None, warmup=None, emit=True):
                            'kernel': 'products of the coupled Newton iteration (plane_gemm_kernel: matrices kept as two '
                                      'fp16 planes where the ridge bounds the root, else three bf16 planes; gemm_x3_kernel / '
                                      'gemm_f32_kernel below 512 columns): 2 n^3 FLOP per product of the reference; '
-                                     'executed_bf16_tflops counts the 16-bit MFMA work actually run (3 fp16 or 6 bf16 piece '
-                                     'products per fp32 product, the tiles on and above the diagonal only)',
+                                     'executed_bf16_tflops counts the 16-bit MFMA work of the reference\'s products (3 fp16 or 6 '
+                                     'bf16 piece products per fp32 product, the tiles on and above the diagonal only): less than '
+                                     'what runs, for a step of the fourth degree has six products and counts as four',
                            'executed_bf16_tflops': executed_flops / secs / 1e12,
                            'executed_bf16_frac': executed_flops / secs / 1e12 / BF16_MFMA_PEAK_TFLOPS,
                            'fp32_peak_frac': algorithmic / FP32_MFMA_PEAK_TFLOPS,
