@@ -51,15 +51,20 @@ struct CcArgs {
   const int* skip;
   int* info;
   const float* scales;                       // CG_SCALE_FLOATS per matrix (cg_scale_kernel)
-  int skip_stride;
+  const float* const* A_list;                // the matrices themselves: what the first group's products update
+  const float* lam;
+  int skip_stride, lam_stride;
 };
+// W holds of A + lam I what the first group's steps read: CC_VLD columns and the diagonal block behind them.
+constexpr int CC_COPIED = CC_VLD + LEAF;     // rows that are copied beyond column CC_VLD
 
 // X <- old -+ V_i V_j^T, one 128 x 128 tile over columns 64 h0 ... 64 h1 - 1 of V; rows, cols: of the tile inside the matrix.
 struct CcProduct {
   const float* V;
   float* X;
-  int dp, bi, bj, ld, rows, cols, h0, h1;
-  float alpha;
+  const float* old;                          // of old_rows x old_cols, rows old_ld apart; beyond it zeros and `pad` on the diagonal
+  int dp, bi, bj, ld, rows, cols, h0, h1, old_ld, old_rows, old_cols;
+  float alpha, lam, pad;                     // lam is added to the old diagonal
   bool half, same, anew;                     // V on fp16 pieces; one operand; no old value
 };
 
@@ -97,14 +102,15 @@ __device__ __forceinline__ CcFragments cc_read(AK_LDS3 const unsigned char* pane
 __device__ __forceinline__ void cc_update(const CcProduct& p, const floatx16& sum, int r0, int c0, int lane) {
   const int i0 = r0 + 4 * (lane >> 5), j = c0 + (lane & 31);
   floatx16 old;
-  if (p.rows == LEAF && p.cols == LEAF) {
+  if (p.old_rows >= LEAF && p.old_cols >= LEAF && !(p.same && p.lam != 0.f)) {        // (the tile has no less)
     float* __restrict__ X = p.X;
-    const int ld = p.ld;
-    const uint32_t at = static_cast<uint32_t>(i0 * ld + j);
+    const float* __restrict__ Y = p.old;
+    const int ld = p.ld, old_ld = p.old_ld;
+    const uint32_t at = static_cast<uint32_t>(i0 * ld + j), from = static_cast<uint32_t>(i0 * old_ld + j);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       old[e] = 0.f;
-      if (!p.anew) old[e] = (X + (8 * (e >> 2) + (e & 3)) * ld)[at];
+      if (!p.anew) old[e] = (Y + (8 * (e >> 2) + (e & 3)) * old_ld)[from];
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) (X + (8 * (e >> 2) + (e & 3)) * ld)[at] = old[e] + p.alpha * sum[e];
@@ -114,12 +120,16 @@ __device__ __forceinline__ void cc_update(const CcProduct& p, const floatx16& su
   for (int e = 0; e < 16; ++e) {
     const int i = i0 + 8 * (e >> 2) + (e & 3);
     old[e] = 0.f;
-    if (!p.anew) old[e] = p.X[static_cast<int64_t>(min(i, p.rows - 1)) * p.ld + min(j, p.cols - 1)];
+    if (!p.anew) {
+      const float x = p.old[static_cast<uint32_t>(min(i, p.old_rows - 1) * p.old_ld + min(j, p.old_cols - 1))];
+      const bool diagonal = p.same && i == j;
+      old[e] = i < p.old_rows && j < p.old_cols ? x + (diagonal ? p.lam : 0.f) : diagonal ? p.pad : 0.f;
+    }
   }
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const int i = i0 + 8 * (e >> 2) + (e & 3);
-    if (i < p.rows && j < p.cols) p.X[static_cast<int64_t>(i) * p.ld + j] = old[e] + p.alpha * sum[e];
+    if (i < p.rows && j < p.cols) p.X[static_cast<uint32_t>(i * p.ld + j)] = old[e] + p.alpha * sum[e];
   }
 }
 
@@ -150,8 +160,8 @@ __device__ __forceinline__ floatx16 cc_sum_half(const CcProduct& p, AK_LDS3 unsi
   // The old tile, a word of every 64 bytes: on its way to the L2 while the last stages run (their registers leave no room for it; ahead of
   // the first stages it would hold those up).  The spare LDS takes what comes.
   auto touch = [&] {
-    const uint32_t i = min(tid >> 3, p.rows - 1), j = min(16 * (tid & 7), p.cols - 4);
-    load_to_lds(cc_descriptor(p.X), lds0 + STAGES * STAGE + wave * 1024, (i * p.ld + j) * 4);
+    const uint32_t i = min(tid >> 3, p.old_rows - 1), j = min(16 * (tid & 7), p.old_cols - 4);
+    load_to_lds(cc_descriptor(p.old), lds0 + STAGES * STAGE + wave * 1024, p.old_cols < 4 ? kDtlOob : (i * p.old_ld + j) * 4);
   };
   if (s1 - s0 < STAGES - 1) touch();
   struct Operands { CcFragments a, b; };
@@ -242,6 +252,17 @@ __device__ __forceinline__ CcProduct cc_task_product(const CcArgs& a, const CcTa
   p.half = scales[0] != 0.f;
   p.same = bi == bj;
   p.anew = step ? bj == k : own_row || own_col;
+  p.old = p.X; p.old_ld = p.ld; p.old_rows = p.rows; p.old_cols = p.cols;
+  p.lam = p.pad = 0.f;
+  if (!step && g0 == 0 && !p.anew) {         // never written before
+    const int d = t.d;
+    p.old = a.A_list[t.mat] + static_cast<int64_t>(LEAF) * bi * d + LEAF * bj;
+    p.old_ld = d;
+    p.old_rows = min(LEAF, d - LEAF * bi);
+    p.old_cols = min(LEAF, d - LEAF * bj);
+    p.lam = a.lam[static_cast<int64_t>(t.mat) * a.lam_stride];
+    p.pad = p.lam > 0.f ? p.lam : 1.f;
+  }
   p.alpha = bi > last ? -1.f : 1.f;
   if (p.half) p.alpha /= scales[bi > last ? CG_KIND_L : CG_KIND_M] * scales[bj > last ? CG_KIND_L : CG_KIND_M];        // (powers of two)
   return p;

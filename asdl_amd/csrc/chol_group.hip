@@ -75,8 +75,10 @@ __device__ __forceinline__ bool cg_skipped(const CgArgs& a, int mat) {
   return a.skip != nullptr && a.skip[static_cast<int64_t>(mat) * a.skip_stride] == 0;
 }
 
-// W_m <- lower(A_m) + lam_m I, padded rows carry the identity; info_m <- 0.  One work group per CG_COPY_ROWS rows of
-// one matrix (bisection on first_copy_block); a row is read and written up to its diagonal element only.
+// W_m <- what the chain's first group of lower(A_m) + lam_m I reads before its products, which take the rest from A_m itself
+// (cc_task_product); padded rows carry the identity; info_m <- 0.  One work group per CG_COPY_ROWS rows of one matrix (bisection on
+// first_copy_block); a row is read and written up to its diagonal element at most.  Bound by the memory: two matrices of 4096 columns 15 us,
+// where all of them took 40 (inverses of ResNet-18's 42 factors 2530 -> 2410 us, a decoder's 1450 -> 1385, 8192 3240 -> 3110).
 static __global__ __launch_bounds__(256) void cg_copy_in_kernel(CgArgs a, int count) {
   const CgHeader* __restrict__ h = reinterpret_cast<const CgHeader*>(a.plan);
   const CgMat* __restrict__ mats = reinterpret_cast<const CgMat*>(a.plan + h->mats_off);
@@ -100,22 +102,23 @@ static __global__ __launch_bounds__(256) void cg_copy_in_kernel(CgArgs a, int co
     const int r = r0 + e;
     if (r >= m.dp) break;
     float* __restrict__ dst = W + static_cast<int64_t>(r) * m.dp;
+    const int last = r < CC_COPIED ? r : CC_VLD - 1;
     if (r >= m.d) {
       // padding: a diagonal block that drops out of the result.  Its value lam (1 when lam <= 0) stays inside the
       // magnitude bounds the fp16-piece products scale their operands by (lam <= a, 1 / sqrt(lam) for the inverse).
       const float pad = l > 0.f ? l : 1.f;
-      for (int c = threadIdx.x; c <= r; c += 256) dst[c] = (c == r) ? pad : 0.f;
+      for (int c = threadIdx.x; c <= last; c += 256) dst[c] = (c == r) ? pad : 0.f;
       continue;
     }
     const float* __restrict__ src = A + static_cast<int64_t>(r) * m.d;
     if (vec) {
-      for (int c = 4 * threadIdx.x; c <= r; c += 1024) {
+      for (int c = 4 * threadIdx.x; c <= last; c += 1024) {
         floatx4 v = *reinterpret_cast<const floatx4*>(src + c);
         if (r >= c && r < c + 4) v[r - c] += l;
         *reinterpret_cast<floatx4*>(dst + c) = v;       // the elements right of the diagonal are never read
       }
     } else {
-      for (int c = threadIdx.x; c <= r; c += 256) dst[c] = src[c] + ((c == r) ? l : 0.f);
+      for (int c = threadIdx.x; c <= last; c += 256) dst[c] = src[c] + ((c == r) ? l : 0.f);
     }
   }
 }
@@ -668,7 +671,7 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
     } else if (st.type == CG_OUT) {
       hipLaunchKernelGGL(cg_out_kernel, dim3(st.grid), dim3(256), 0, s, a, h->count);
     } else {
-      const CcArgs c{a.ws, skip_flags, info, a.scales, skip_stride};
+      const CcArgs c{a.ws, skip_flags, info, a.scales, A_list, lam, skip_stride, lam_stride};
       const CcTask* tasks = reinterpret_cast<const CcTask*>(a.plan + h->tasks_off) + st.first;
       if (st.type == CG_CHAIN) hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, c, tasks, st.count);
       else hipLaunchKernelGGL(cg_product_kernel, dim3(st.grid), dim3(512), 0, s, c, tasks, st.count);

@@ -714,6 +714,38 @@ def test_chol_inv_grouped_products_beside_the_steps(K, dims, lam_rel):
         assert relerr(o, exact) < 35 * 2.0 ** -22, (d, relerr(o, exact))
 
 
+@pytest.mark.parametrize('dims', [(4133,), (2051, 2049, 2046, 1409, 1405, 641, 639) * 2, (641,) * 40 + (1023, 1281) * 6])
+def test_chol_inv_grouped_takes_the_first_updates_from_the_matrices(K, dims):
+    """Groups on the chain, whose first products read the matrices themselves (rows of any length, a last block of one to three columns,
+    behind which zeros and a diagonal stand): the same bits from matrices with anything above their diagonals, in memory that ends with
+    them, next to one that is left out."""
+    plan = K.chol_group_plan(list(dims))
+    assert plan.launches != max((d + 127) // 128 for d in dims) + 1, 'the block sweep: one launch per block column'
+    g = torch.Generator('cuda').manual_seed(5)
+    mats = []
+    for d in dims:
+        x = torch.randn(2 * d, d, device='cuda', generator=g)
+        mats.append(x.T @ x / (2 * d))
+    lam = torch.full((len(dims),), 0.03, device='cuda')
+    outs, junk = [torch.empty_like(m) for m in mats], [torch.empty_like(m) for m in mats]
+    assert int(K.chol_inv_grouped(mats, outs, lam).abs().max()) == 0
+    dirty = [torch.tril(m) + torch.triu(torch.full_like(m, float('nan')), 1) for m in mats]
+    active = torch.ones(len(dims), dtype=torch.int32, device='cuda')
+    if len(dims) > 1:
+        active[1] = 0
+        junk[1].fill_(7.0)
+    K.chol_inv_grouped(dirty, junk, lam, active=active)
+    for i, (d, A) in enumerate(zip(dims, mats)):
+        if active[i] == 0:
+            assert bool((junk[i] == 7).all())
+            continue
+        assert torch.equal(junk[i], outs[i]), (i, d)
+        if i < 8:
+            full = torch.tril(A).double() + torch.tril(A, -1).double().T + 0.03 * torch.eye(d, device='cuda', dtype=torch.float64)
+            # (A + lam I) X = I up to the condition, below 35, of what 22 bits hold
+            assert float((full @ outs[i].double() - torch.eye(d, device='cuda', dtype=torch.float64)).norm()) < 35 * 2.0 ** -22 * d ** 0.5
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
