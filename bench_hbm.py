@@ -139,18 +139,18 @@ def main(argv=None):
           sum(a + b for a, b in dims) * 4, lambda: K.kron_damping(A_list, B_list, 1e-3),
           note='latency bound: 0.4 MB in one launch')
 
-    # copy-in of the grouped inverse: lower triangles of all 108 factors + damping into the work matrices; timed
-    # with the rest of the inverse here, its own duration (ak::cg_copy_in_kernel) is in the kernel trace
+    # the grouped inverse of all 108 factors; the durations of its ways in and out (ak::cg_copy_in_kernel, ak::cg_out_kernel) are in
+    # the kernel trace
     mats = A_list + B_list
     for m in mats:
         m.copy_(torch.eye(m.shape[0], device=dev))
     outs = [torch.empty_like(m) for m in mats]
     lam = torch.full((len(mats),), 1e-3, device=dev)
     tri_bytes = sum(m.shape[0] * (m.shape[0] + 1) // 2 for m in mats) * 4
-    timed('grouped inverse of 108 factors (whole call; copy-in = ak::cg_copy_in_kernel in the trace)',
+    timed('grouped inverse of 108 factors (whole call)',
           ['ak::cg_copy_in_kernel', 'ak::cg_chain_kernel', 'ak::cg_product_kernel'], 2 * tri_bytes,
           lambda: K.chol_inv_grouped(mats, outs, lam),
-          note=f'copy-in alone moves {2 * tri_bytes} bytes (lower triangles read and written); the call is MFMA bound')
+          note='bytes: the lower triangles read and written once; the call is MFMA bound')
     del mats, outs, A_list, B_list
 
     # packed lower triangle of a saved factor and back
