@@ -157,11 +157,11 @@ __device__ __forceinline__ floatx16 cc_sum_half(const CcProduct& p, AK_LDS3 unsi
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t)
     if (s0 + t < s1) issue(s0 + t);
-  // The old tile, a word of every 64 bytes: on its way to the L2 while the last stages run (their registers leave no room for it; ahead of
-  // the first stages it would hold those up).  The spare LDS takes what comes.
+  // The old tile, if there is one, a word of every 64 bytes: on its way to the L2 while the last stages run (their registers leave no room
+  // for it; ahead of the first stages it would hold those up).  The spare LDS takes what comes.  (Its descriptor is formed here, in the loop.)
   auto touch = [&] {
     const uint32_t i = min(tid >> 3, p.old_rows - 1), j = min(16 * (tid & 7), p.old_cols - 4);
-    load_to_lds(cc_descriptor(p.old), lds0 + STAGES * STAGE + wave * 1024, p.old_cols < 4 ? kDtlOob : (i * p.old_ld + j) * 4);
+    load_to_lds<true>(cc_descriptor(p.old), lds0 + STAGES * STAGE + wave * 1024, p.anew || p.old_cols < 4 ? kDtlOob : (i * p.old_ld + j) * 4);
   };
   if (s1 - s0 < STAGES - 1) touch();
   struct Operands { CcFragments a, b; };

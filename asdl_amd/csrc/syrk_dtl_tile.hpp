@@ -56,9 +56,12 @@ struct DtlParams {
 
 // 16 bytes per lane, global -> LDS at m0 + 16*lane.  The compiler does not see the LDS write: callers
 // order it against LDS reads with s_waitcnt vmcnt + a barrier.
+// FRESH: the descriptor may come straight from a vector instruction (v_readfirstlane), which the load may read five wait states later;
+// the compiler does not look into the assembly and keeps no distance.
+template <bool FRESH = false>
 __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds_addr, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_addr), "v"(voff), "s"(rsrc), "n"(FRESH ? 4 : 0) : "memory");
 }
 
 template <int N> __device__ __forceinline__ void wait_vmcnt() {

@@ -66,6 +66,48 @@ def test_no_hot_kernel_spills_registers():
     assert not spilled, spilled
 
 
+def test_loads_to_the_lds_wait_for_descriptors_from_vector_instructions(tmp_path):
+    """A vector memory instruction may read a scalar register five wait states after a vector instruction (v_readfirstlane) wrote it.
+    The compiler keeps that distance for its own loads, not for the inline assembly of load_to_lds(): in the assembly of the library
+    as it is built no descriptor of such a load is younger, along the instructions in front of it."""
+    import re
+    import shutil
+    import subprocess
+    from asdl_amd import _lib
+    objdump = '/opt/rocm/llvm/bin/llvm-objdump'
+    if not os.path.exists(objdump):
+        pytest.skip('no llvm-objdump')
+    copy = shutil.copy(_lib.LIB_PATH, tmp_path / 'lib.so')
+    subprocess.run([objdump, '--offloading', str(copy)], cwd=tmp_path, check=True, capture_output=True)
+    loads, young = 0, []
+    for obj in sorted(tmp_path.glob('lib.so.*gfx950')):
+        kernel, before = '', []
+        text = subprocess.run([objdump, '-d', '--no-show-raw-insn', '--no-leading-addr', str(obj)], check=True, capture_output=True, text=True).stdout
+        for line in text.splitlines():
+            line = line.split('//')[0].strip()
+            if line.endswith('>:'):
+                kernel, before = line, []
+            elif line.startswith('buffer_load') and line.endswith(' lds'):
+                loads += 1
+                low, high = map(int, re.search(r' s\[(\d+):(\d+)\]', line).groups())
+                states = 0
+                for op, dest in reversed(before[-8:]):
+                    if op == 's_nop':
+                        states += int(dest, 0)
+                    elif op.startswith('v_') and states < 5:
+                        m = re.fullmatch(r's(\d+)|s\[(\d+):(\d+)\]', dest)
+                        if m:
+                            first = int(m.group(1) or m.group(2))
+                            if first <= high and int(m.group(3) or first) >= low:
+                                young.append((kernel[:60], line, op, dest, states))
+                    states += 1
+            if line and not line.endswith(':'):
+                words = line.replace(',', ' ').split()
+                before = before[-15:] + [(words[0], words[1] if len(words) > 1 else '')]
+    assert loads > 100
+    assert not young, young
+
+
 def test_root_workspace_of_a_call_over_all_sizes_is_below_that_of_its_largest_group():
     """A call takes the roots of all sizes at once, so its workspace is a sum.  For a twelve-layer decoder of 768 columns it has to stay
     below the bound for the largest group alone, which holds for any power."""
