@@ -268,136 +268,11 @@ __device__ __forceinline__ CcProduct cc_task_product(const CcArgs& a, const CcTa
   return p;
 }
 
-// The products of a launch of their own, two work groups a CU: 8 waves of 64 x 32 each, a stage of 16 k ahead of three others; one
-// work group's way from and to the memory runs beside the other's sums.  The same instructions in the same order as in a step's
-// launch: the same bits whichever a tile is in.
-static __global__ __launch_bounds__(512, 4) void cg_product_kernel(CcArgs a, const CcTask* __restrict__ tasks, int k) {
-  constexpr int STAGE = 2 * CC_PANEL_BYTES, STAGES = 4;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[STAGES * STAGE];
-  AK_LDS3 unsigned char* lds = (AK_LDS3 unsigned char*)smem;
-  const CcProduct p = cc_task_product(a, tasks[blockIdx.x], k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 5, l32 = lane & 31, wr = wave >> 2, wc = wave & 3;
-  const int s0 = 4 * p.h0, s1 = 4 * p.h1;
-  StSum sum[2];
-  sum[0].clear();
-  sum[1].clear();
-  if (p.half) {
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-    const u32x4 d = cc_descriptor(p.V);
-    const uint32_t oi = cc_lane_at(p.dp, p.bi, p.rows, wave, lane), oj = cc_lane_at(p.dp, p.bj, p.cols, wave, lane);
-    auto issue = [&](int s) {
-      const uint32_t at = lds0 + (s & (STAGES - 1)) * STAGE + wave * 1024, block = cc_v_at(p.dp, 0, s);
-      load_to_lds(d, at, oi + block);
-      if (!p.same) load_to_lds(d, at + CC_PANEL_BYTES, oj + block);
-    };
-    struct Operands { CcFragments a[2], b; };
-    // (four addresses; a stage is a constant further, as the loop below takes a round of the ring at a time)
-    AK_LDS3 const unsigned char* pa[2];
-    AK_LDS3 const unsigned char* pb[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int chunk = 16 * ((2 * q + g) ^ ((l32 >> 2) & 3));
-      pa[q] = lds + (64 * wr + l32) * 64 + chunk;
-      pb[q] = lds + (p.same ? 0 : CC_PANEL_BYTES) + (32 * wc + l32) * 64 + chunk;
-    }
-    auto step = [&](int s, auto stage_tag, Operands& now, const Operands& before, bool have) {
-      constexpr int AT = decltype(stage_tag)::value * STAGE;
-      // stage s has landed for this wave, then for all; and all have read stage s - 1, which the next loads overwrite
-      const int ahead = min(s1 - 1 - s, STAGES - 2);
-      if (ahead == 2) {
-        if (p.same) wait_vmcnt<2>();
-        else wait_vmcnt<4>();
-      } else if (ahead == 1) {
-        if (p.same) wait_vmcnt<1>();
-        else wait_vmcnt<2>();
-      } else {
-        wait_vmcnt<0>();
-      }
-      __syncthreads();
-      if (s + STAGES - 1 < s1) issue(s + STAGES - 1);
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        now.b.x[q] = *reinterpret_cast<AK_LDS3 const bf16x8*>(pb[q] + AT);
-#pragma unroll
-        for (int x = 0; x < 2; ++x) now.a[x].x[q] = *reinterpret_cast<AK_LDS3 const bf16x8*>(pa[q] + AT + 2048 * x);
-      }
-      if (!have) return;
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        sum[x].small = x3_mfma<true>(before.a[x].x[1], before.b.x[0], sum[x].small);
-        sum[x].big = x3_mfma<true>(before.a[x].x[0], before.b.x[0], sum[x].big);
-        sum[x].small = x3_mfma<true>(before.a[x].x[0], before.b.x[1], sum[x].small);
-      }
-    };
-#pragma unroll
-    for (int t = 0; t < STAGES - 1; ++t)
-      if (s0 + t < s1) issue(s0 + t);
-    Operands even, odd;
-    for (int s = s0; s < s1; s += STAGES) {        // (s0 and s1 are multiples of it)
-      step(s, std::integral_constant<int, 0>{}, even, odd, s > s0);
-      step(s + 1, std::integral_constant<int, 1>{}, odd, even, true);
-      step(s + 2, std::integral_constant<int, 2>{}, even, odd, true);
-      step(s + 3, std::integral_constant<int, 3>{}, odd, even, true);
-    }
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      sum[x].small = x3_mfma<true>(odd.a[x].x[1], odd.b.x[0], sum[x].small);
-      sum[x].big = x3_mfma<true>(odd.a[x].x[0], odd.b.x[0], sum[x].big);
-      sum[x].small = x3_mfma<true>(odd.a[x].x[0], odd.b.x[1], sum[x].small);
-    }
-  } else {
-    // three bf16 pieces of fp32, 32 k at a time
-    static_assert(6 * LEAF * 64 <= STAGES * STAGE, "planes of both operands");
-    const int row = tid >> 2, chunk = tid & 3, to = row * 64 + 16 * (chunk ^ ((row >> 2) & 3));
-    for (int s = s0; s < s1; s += 2) {
-      auto bring = [&](int blk, int rows, AK_LDS3 unsigned char* panel) {
-        const float* __restrict__ src = p.V + static_cast<int64_t>(LEAF * blk + min(row, rows - 1)) * CC_VLD + CC_BLOCK * s + 8 * chunk;
-        st_floatx8 x;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const floatx4 q = *reinterpret_cast<const floatx4*>(src + 4 * u);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[4 * u + e] = q[e];
-        }
-        bf16x8 o[3];
-        st_split(x, o);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) *reinterpret_cast<AK_LDS3 bf16x8*>(panel + q * CC_PANEL_BYTES + to) = o[q];
-      };
-      __syncthreads();
-      bring(p.bi, p.rows, lds);
-      if (!p.same) bring(p.bj, p.cols, lds + 3 * CC_PANEL_BYTES);
-      __syncthreads();
-      AK_LDS3 const unsigned char* pb = p.same ? lds : lds + 3 * CC_PANEL_BYTES;
-      auto read = [&](bf16x8 (&f)[3], AK_LDS3 const unsigned char* panel, int r, int t) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-          f[q] = *reinterpret_cast<AK_LDS3 const bf16x8*>(panel + q * CC_PANEL_BYTES + r * 64 + 16 * ((2 * t + g) ^ ((r >> 2) & 3)));
-      };
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        bf16x8 x[3], y[3];
-        read(y, pb, 32 * wc + l32, t);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          read(x, lds, 64 * wr + 32 * u + l32, t);
-          sum[u].small = mfma_bf16(x[1], y[1], sum[u].small);
-          sum[u].big = mfma_bf16(x[0], y[0], sum[u].big);
-          sum[u].small = mfma_bf16(x[0], y[2], sum[u].small);
-          sum[u].small = mfma_bf16(x[2], y[0], sum[u].small);
-          sum[u].small = mfma_bf16(x[0], y[1], sum[u].small);
-          sum[u].small = mfma_bf16(x[1], y[0], sum[u].small);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int x = 0; x < 2; ++x) cc_update(p, sum[x].value(), 64 * wr + 32 * x, 32 * wc, lane);
-}
-
-// Step k (-1: the first diagonal blocks are factored), one work group per task.
+// Step k (-1: the first diagonal blocks are factored), or products in a launch of their own; one work group per task.
+// (Products of 8 waves, two work groups a CU, 1056 tiles in 66 us: 2 x 4096 1250 us as here, ResNet-18's factors 2520, here 2660, ResNet-50's
+// 3350, here 3570.  They left half a CU to other kernels' waves: hold_cu.)
 static __global__ __launch_bounds__(LEAF_THREADS) void cg_chain_kernel(CcArgs a, const CcTask* __restrict__ tasks, int k) {
+  hold_cu();
   __shared__ __attribute__((aligned(16))) unsigned char st_smem[ST_LDS];
   __shared__ __attribute__((aligned(16))) LeafShared sh;
   AK_LDS3 unsigned char* lds = (AK_LDS3 unsigned char*)st_smem;

@@ -29,8 +29,8 @@
 
 namespace ak {
 
-constexpr int64_t CG_MAGIC = 0x3547524c4f4843ll;     // "CHOLGR5"
-constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_PRODUCT = 2, CG_SWEEP = 3, CG_OUT = 4;
+constexpr int64_t CG_MAGIC = 0x3647524c4f4843ll;     // "CHOLGR6"
+constexpr int CG_COPY = 0, CG_CHAIN = 1, CG_SWEEP = 2, CG_OUT = 3;
 
 #ifdef AK_TUNING_HOOKS
 static float CG_HALF_MAX_COND = 65536.f;              // tuning builds: ak_debug_set_chol_half_max_cond
@@ -372,10 +372,10 @@ static void cg_append_by_xcd(std::vector<CcTask>& tasks, int first, const std::v
 }
 
 constexpr size_t kProductChunk = 16;   // tiles that stay together
-// us of a CU: a tile of a group's products in a step's launch (18 measured), in one of its own (16 to 20), a tile of a step in one of its own;
+// us of a CU: a tile of a group's products, a tile of a step in a launch of its own;
 // what a step's launch takes along without being longer for it: its leaf takes 26.  (Tiles beyond that in the steps' launches, each of which
 // asks for a whole CU: 24 x 1100 605 -> 625 us, ResNet-18's step, beside the loss backward pass, 1 % more.)
-constexpr double kProductUs = 18.0, kOwnProductUs = 16.0, kStepUs = 5.0, kBesideUs = 26.0;
+constexpr double kProductUs = 18.0, kStepUs = 5.0, kBesideUs = 26.0;
 // The chain's tables.  Returns the time that the rule goes by: 26 us a step, or 9 and 18 per round of tiles (of panels alone: 9) where that is
 // more, all products in launches of their own (cg_shapes_us), the copies by their bytes.
 static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
@@ -478,7 +478,7 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
     if (st.grid > 0) plan.steps.push_back(st);
     if (k < 0) continue;
     if (split[k]) {
-      CgStep own{CG_PRODUCT, static_cast<int>(plan.tasks.size()), k, 0};
+      CgStep own{CG_CHAIN, static_cast<int>(plan.tasks.size()), k, 0};
       tiles(CC_STEP);
       own.grid = static_cast<int>(plan.tasks.size()) - own.first;
       plan.steps.push_back(own);
@@ -515,9 +515,9 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
       later.clear();
     });
     if (!now.empty()) {
-      plan.steps.push_back(CgStep{CG_PRODUCT, static_cast<int>(plan.tasks.size()), k, static_cast<int>(now.size())});
+      plan.steps.push_back(CgStep{CG_CHAIN, static_cast<int>(plan.tasks.size()), k, static_cast<int>(now.size())});
       cg_append_by_xcd(plan.tasks, static_cast<int>(plan.tasks.size()), now);
-      us += 4.0 + kOwnProductUs * std::max(1.0, static_cast<double>(now.size()) / 256);
+      us += 4.0 + kProductUs * std::max(1.0, static_cast<double>(now.size()) / 256);
     }
   }
   plan.steps.push_back(CgStep{CG_OUT, 0, count, out_blocks});
@@ -673,8 +673,7 @@ extern "C" int ak_chol_inv_grouped(const void* plan_host, const void* plan_dev, 
     } else {
       const CcArgs c{a.ws, skip_flags, info, a.scales, A_list, lam, skip_stride, lam_stride};
       const CcTask* tasks = reinterpret_cast<const CcTask*>(a.plan + h->tasks_off) + st.first;
-      if (st.type == CG_CHAIN) hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, c, tasks, st.count);
-      else hipLaunchKernelGGL(cg_product_kernel, dim3(st.grid), dim3(512), 0, s, c, tasks, st.count);
+      hipLaunchKernelGGL(cg_chain_kernel, dim3(st.grid), dim3(LEAF_THREADS), 0, s, c, tasks, st.count);
     }
   }
   return check_launch();

@@ -47,6 +47,7 @@ struct SwArgs {
 // diagonal block of a matrix, updated and factored; the others: one tile each.
 static __global__ __launch_bounds__(LEAF_THREADS) void cg_sweep_kernel(SwArgs a, const SwTask* __restrict__ leaves,
                                                                        const SwTask* __restrict__ tiles, int nleaf, int k) {
+  hold_cu();
   __shared__ __attribute__((aligned(16))) unsigned char st_smem[ST_LDS];
   __shared__ __attribute__((aligned(16))) LeafShared sh;
   AK_LDS3 unsigned char* lds = (AK_LDS3 unsigned char*)st_smem;

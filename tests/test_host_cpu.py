@@ -108,6 +108,21 @@ def test_loads_to_the_lds_wait_for_descriptors_from_vector_instructions(tmp_path
     assert not young, young
 
 
+def test_kernels_that_run_beside_the_framework_hold_their_cus():
+    """The kernels of the grouped inverses with 16-bit matrix instructions run on side streams.  A work group of theirs has all 512 vector
+    registers of its CU's lanes, by blocks of 8 a wave, so that no wave of another kernel runs there."""
+    report = os.path.join(os.path.dirname(asdl_amd.__file__), 'lib', 'kernel_resources.txt')
+    if not os.path.exists(report):
+        pytest.skip('no kernel_resources.txt: the library was not built by asdl_amd.build in this tree')
+    rows = [l.split() for l in open(report) if l.startswith('chol_group.hip')]
+    beside = {'cg_sweep_kernel': 1024, 'cg_chain_kernel': 1024, 'cg_copy_in_kernel': 0, 'cg_scale_kernel': 0, 'cg_out_kernel': 0}      # 0: no matrix instruction
+    found = {k: r for k in beside for r in rows if k in r[1]}
+    assert sorted(found) == sorted(beside) and sum('cg_' in r[1] for r in rows) == len(beside)
+    for name, threads in beside.items():
+        registers = (int(found[name][2]) + int(found[name][3]) + 7) // 8 * 8
+        assert threads == 0 or threads // 64 // 4 * registers == 512, found[name]
+
+
 def test_root_workspace_of_a_call_over_all_sizes_is_below_that_of_its_largest_group():
     """A call takes the roots of all sizes at once, so its workspace is a sum.  For a twelve-layer decoder of 768 columns it has to stay
     below the bound for the largest group alone, which holds for any power."""
