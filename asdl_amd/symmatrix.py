@@ -382,9 +382,13 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
                 kernels.chol_inv_batched([e[1] for e in entries], outs, lam_g, 1, active=act_g, active_stride=1,
                                          info=info)
 
+    # Beside the framework's kernels only what does not disturb them: 16-bit matrix instructions on their CUs take values from its
+    # sums over the rows of bf16 matrices (csrc/chol_step.hpp, hold_cu).  The grouped inverses hold their CUs, the grouped
+    # low-rank ones have fp32 products; the others' products do neither, so that what follows waits for them.
+    undisturbing = mats_on_gpu and GROUPED_INVERSE and len(together) == len(low_rank)
     side = []
     inline = not (beside and defer)
-    if mats_on_gpu and GROUPED_INVERSE and len(together) == len(low_rank) and not inline:
+    if undisturbing and not inline:
         # A few launches that leave most of the device idle: the changes of stream cost the host more than running beside
         # them saves the device.  (Low-rank factors: the Gram matrices' chain, then d^2 floats each at 3 TB/s.)
         us = kernels.chol_group_plan([e[1].shape[0] for e in square]).microseconds if square else 0
@@ -397,6 +401,8 @@ def batched_update_inv(krons, damping=_default_damping, calc_A_inv=True, calc_B_
             run_group(group)
     pending = PendingInverses(records, flags, nz_flat, side, replace,
                               keep_alive=(prepared, lam, A_list, B_list, scratch), fresh=fresh)
+    if not undisturbing:
+        pending.join()
     if defer:
         return pending
     pending.finish()

@@ -746,7 +746,7 @@ def test_chol_inv_grouped_takes_the_first_updates_from_the_matrices(K, dims):
             assert float((full @ outs[i].double() - torch.eye(d, device='cuda', dtype=torch.float64)).norm()) < 35 * 2.0 ** -22 * d ** 0.5
 
 
-@pytest.mark.parametrize('case', ['chain', 'chain of many', 'sweep', 'low rank'])
+@pytest.mark.parametrize('case', ['chain', 'chain of many', 'sweep', 'by size', 'low rank', 'low rank one by one'])
 def test_sums_of_the_framework_beside_inverses_on_a_side_stream(K, monkeypatch, case):
     """Deferred inverses run on side streams beside whatever the caller enqueues next, the loss backward pass in a step.  Its sums over
     the rows of bf16 matrices, the bias gradients, give the bits that they give alone: 16-bit matrix instructions of another
@@ -754,16 +754,17 @@ def test_sums_of_the_framework_beside_inverses_on_a_side_stream(K, monkeypatch, 
     from asdl_amd import symmatrix
     from asdl_amd.symmatrix import Kron, batched_update_inv
     monkeypatch.setattr(symmatrix, 'INLINE_MICROSECONDS', 0)      # (beside the current stream at all sizes)
+    monkeypatch.setattr(symmatrix, 'GROUPED_INVERSE', case != 'by size')
     g = torch.Generator('cuda').manual_seed(1)
 
     def factor(d, rows):
         x = torch.randn(rows, d, device='cuda', generator=g)
         return x if rows < d else x.t() @ x / rows
-    sizes = {'chain': [(4096, 5000)] * 2, 'chain of many': [(1100, 1500)] * 24, 'sweep': [(2000, 2500)] * 2,
-             'low rank': [(2304, 128)] * 8}[case]
+    sizes = {'chain': [(4096, 5000)] * 2, 'chain of many': [(1100, 1500)] * 24, 'sweep': [(2000, 2500)] * 2, 'by size': [(4096, 5000)] * 2,
+             'low rank': [(2304, 128)] * 8, 'low rank one by one': [(4608, 600)] * 4}[case]
     mats = [factor(d, rows) for d, rows in sizes]
     krons = [Kron(mats[i], mats[i + 1]) for i in range(0, len(mats), 2)]
-    if case != 'low rank':
+    if case in ('chain', 'chain of many', 'sweep'):
         assert (K.chol_group_plan([d for d, _ in sizes]).launches == max((d + 127) // 128 for d, _ in sizes) + 1) == (case == 'sweep')
     wide = torch.randn(8192, 4096, device='cuda', generator=g).bfloat16()
     low = torch.randn(1024, 3072, device='cuda', generator=g).bfloat16()
