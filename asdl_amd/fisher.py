@@ -31,7 +31,8 @@ GROUP_FLUSH_EVERY = (-2, 0)  # (forward, backward): launch the group after that 
                              # time of their single launches; the backward pass is bound by the device (ResNet-50 batch
                              # 64 in one process: 26.9 ms per step with single launches, 27.4 with (0, 0), 26.3 with
                              # (-1, 0), 26.0 with (-2, 0))
-FACTOR_SIDE_STREAM = False  # statistics kernels of the hooks on a side stream (ordering the two streams costs ~30 us of host time per hook: more than the overlap gains)
+FACTOR_SIDE_STREAM = False  # statistics kernels of the hooks on a side stream (ordering the two streams costs ~30 us of host time per hook); the current
+                            # stream waits for every batch of them: 16-bit products take values from the framework's sums beside them
 PRUNED_FISHER_BACKWARD = True   # sampled / exact Fisher passes skip the weight-gradient kernels (their results are never used)
 LATE_INVERSE_FLAGS = False  # Read the zero / not-positive-definite flags of an update with calc_loss_grad only when the next
                             # update reaches the same point (FisherMaker.late_inverse_flags; check_late_flags() after

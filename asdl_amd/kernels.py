@@ -373,6 +373,9 @@ class FactorStream:
             _override.handle, _override.stream = self.handle, self.stream
             for fn in fns:
                 fn()
+            # (16-bit products that do not hold their CUs: the framework's sums do not run beside them, symmatrix.batched_update_inv)
+            _lib.check(_lib.load().ak_stream_order(ctypes.c_void_p(self.handle), ctypes.c_void_p(main), self._event()),
+                       'ak_stream_order')
         finally:
             _override.handle, _override.stream = saved
             self._flushing = False

@@ -778,6 +778,22 @@ def test_sums_of_the_framework_beside_inverses_on_a_side_stream(K, monkeypatch, 
                 assert torch.equal(x, y), f'{int((x != y).sum())} of {x.numel()} sums differ'
 
 
+def test_sums_of_the_framework_beside_statistics_on_a_side_stream(K):
+    """The same of the factors' products, where they are queued on a side stream."""
+    g = torch.Generator('cuda').manual_seed(2)
+    rows, wide = torch.randn(8192, 1024, device='cuda', generator=g).bfloat16(), torch.randn(8192, 4096, device='cuda', generator=g).bfloat16()
+    alone, factor, out = wide.sum(0), K.syrk_tn(rows), torch.empty(1024, 1024, device='cuda')
+    stream = K.FactorStream('cuda')
+    for _ in range(10):
+        for _ in range(2 * K.FACTOR_STREAM_BATCH):
+            stream.run(lambda: K.syrk_tn(rows, out=out), rows, out)
+        beside = [wide.sum(0) for _ in range(20)]
+        stream.join()
+        for got in beside:
+            assert torch.equal(got, alone), f'{int((got != alone).sum())} of {got.numel()} sums differ'
+        assert torch.equal(out, factor)
+
+
 def test_chol_inv_grouped_reads_the_lower_triangle_only(K):
     d = 300
     A = _spd(d, 7)
