@@ -58,11 +58,14 @@ struct CcArgs {
 // W holds of A + lam I what the first group's steps read: CC_VLD columns and the diagonal block behind them.
 constexpr int CC_COPIED = CC_VLD + LEAF;     // rows that are copied beyond column CC_VLD
 
+// (said of pointers that are chosen between or read from memory: else their accesses are flat ones)
+#define CC_GLOBAL __attribute__((address_space(1)))
+
 // X <- old -+ V_i V_j^T, one 128 x 128 tile over columns 64 h0 ... 64 h1 - 1 of V; rows, cols: of the tile inside the matrix.
 struct CcProduct {
   const float* V;
-  float* X;
-  const float* old;                          // of old_rows x old_cols, rows old_ld apart; beyond it zeros and `pad` on the diagonal
+  CC_GLOBAL float* X;
+  CC_GLOBAL const float* old;                // of old_rows x old_cols, rows old_ld apart; beyond it zeros and `pad` on the diagonal
   int dp, bi, bj, ld, rows, cols, h0, h1, old_ld, old_rows, old_cols;
   float alpha, lam, pad;                     // lam is added to the old diagonal
   bool half, same, anew;                     // V on fp16 pieces; one operand; no old value
@@ -74,7 +77,7 @@ constexpr int CC_PANEL_BYTES = LEAF * 64;    // a block's 128 rows of one operan
 __host__ __device__ __forceinline__ uint32_t cc_v_at(int dp, int row, int b) {
   return (static_cast<uint32_t>(b) * static_cast<uint32_t>(dp) + static_cast<uint32_t>(row)) * 64u;
 }
-__device__ __forceinline__ u32x4 cc_descriptor(const void* at) {
+__device__ __forceinline__ u32x4 cc_descriptor(CC_GLOBAL const void* at) {
   const uint64_t b = reinterpret_cast<uint64_t>(at);
   u32x4 d;
   d[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b));
@@ -103,8 +106,8 @@ __device__ __forceinline__ void cc_update(const CcProduct& p, const floatx16& su
   const int i0 = r0 + 4 * (lane >> 5), j = c0 + (lane & 31);
   floatx16 old;
   if (p.old_rows >= LEAF && p.old_cols >= LEAF && !(p.same && p.lam != 0.f)) {        // (the tile has no less)
-    float* __restrict__ X = p.X;
-    const float* __restrict__ Y = p.old;
+    CC_GLOBAL float* X = p.X;                // (behind the first group the old values lie in X itself)
+    CC_GLOBAL const float* Y = p.old;
     const int ld = p.ld, old_ld = p.old_ld;
     const uint32_t at = static_cast<uint32_t>(i0 * ld + j), from = static_cast<uint32_t>(i0 * old_ld + j);
 #pragma unroll
@@ -141,7 +144,7 @@ __device__ __forceinline__ floatx16 cc_sum_half(const CcProduct& p, AK_LDS3 unsi
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31, wr = wave & 3, wc = wave >> 2;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
-  const u32x4 d = cc_descriptor(p.V);
+  const u32x4 d = cc_descriptor((CC_GLOBAL const void*)p.V);
   // a wave brings 16 rows of one block of 16 k of either operand
   const int blk = wave >> 3, part = wave & 7;
   const uint32_t oi = cc_lane_at(p.dp, p.bi, p.rows, part, lane), oj = cc_lane_at(p.dp, p.bj, p.cols, part, lane);
@@ -241,7 +244,7 @@ __device__ __forceinline__ CcProduct cc_task_product(const CcArgs& a, const CcTa
   const float* __restrict__ scales = a.scales + static_cast<int64_t>(t.mat) * CG_SCALE_FLOATS;
   CcProduct p;
   p.V = a.ws + t.v_off + static_cast<int64_t>(g0 / CG_GROUP & 1) * dp * CC_VLD;
-  p.X = inside ? a.ws + t.e_off + (rr * (rr - 1) / 2 + bj - g0) * ST_TILE : a.ws + t.w_off + static_cast<int64_t>(LEAF) * bi * dp + LEAF * bj;
+  p.X = (CC_GLOBAL float*)(inside ? a.ws + t.e_off + (rr * (rr - 1) / 2 + bj - g0) * ST_TILE : a.ws + t.w_off + static_cast<int64_t>(LEAF) * bi * dp + LEAF * bj);
   p.dp = dp; p.bi = bi; p.bj = bj;
   p.ld = inside ? LEAF : dp;
   p.rows = min(LEAF, dp - LEAF * bi);
@@ -256,7 +259,7 @@ __device__ __forceinline__ CcProduct cc_task_product(const CcArgs& a, const CcTa
   p.lam = p.pad = 0.f;
   if (!step && g0 == 0 && !p.anew) {         // never written before
     const int d = t.d;
-    p.old = a.A_list[t.mat] + static_cast<int64_t>(LEAF) * bi * d + LEAF * bj;
+    p.old = (CC_GLOBAL const float*)a.A_list[t.mat] + static_cast<int64_t>(LEAF) * bi * d + LEAF * bj;
     p.old_ld = d;
     p.old_rows = min(LEAF, d - LEAF * bi);
     p.old_cols = min(LEAF, d - LEAF * bj);

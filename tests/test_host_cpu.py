@@ -66,46 +66,63 @@ def test_no_hot_kernel_spills_registers():
     assert not spilled, spilled
 
 
-def test_loads_to_the_lds_wait_for_descriptors_from_vector_instructions(tmp_path):
-    """A vector memory instruction may read a scalar register five wait states after a vector instruction (v_readfirstlane) wrote it.
-    The compiler keeps that distance for its own loads, not for the inline assembly of load_to_lds(): in the assembly of the library
-    as it is built no descriptor of such a load is younger, along the instructions in front of it."""
-    import re
+@pytest.fixture(scope='module')
+def assembly(tmp_path_factory):
+    """The instructions of every kernel of the built library, {name: [text]}."""
     import shutil
     import subprocess
     from asdl_amd import _lib
     objdump = '/opt/rocm/llvm/bin/llvm-objdump'
     if not os.path.exists(objdump):
         pytest.skip('no llvm-objdump')
-    copy = shutil.copy(_lib.LIB_PATH, tmp_path / 'lib.so')
-    subprocess.run([objdump, '--offloading', str(copy)], cwd=tmp_path, check=True, capture_output=True)
-    loads, young = 0, []
-    for obj in sorted(tmp_path.glob('lib.so.*gfx950')):
-        kernel, before = '', []
+    where = tmp_path_factory.mktemp('assembly')
+    copy = shutil.copy(_lib.LIB_PATH, where / 'lib.so')
+    subprocess.run([objdump, '--offloading', str(copy)], cwd=where, check=True, capture_output=True)
+    kernels = {}
+    for i, obj in enumerate(sorted(where.glob('lib.so.*gfx950'))):
         text = subprocess.run([objdump, '-d', '--no-show-raw-insn', '--no-leading-addr', str(obj)], check=True, capture_output=True, text=True).stdout
         for line in text.splitlines():
             line = line.split('//')[0].strip()
             if line.endswith('>:'):
-                kernel, before = line, []
-            elif line.startswith('buffer_load') and line.endswith(' lds'):
-                loads += 1
-                low, high = map(int, re.search(r' s\[(\d+):(\d+)\]', line).groups())
-                states = 0
-                for op, dest in reversed(before[-8:]):
-                    if op == 's_nop':
-                        states += int(dest, 0)
-                    elif op.startswith('v_') and states < 5:
-                        m = re.fullmatch(r's(\d+)|s\[(\d+):(\d+)\]', dest)
-                        if m:
-                            first = int(m.group(1) or m.group(2))
-                            if first <= high and int(m.group(3) or first) >= low:
-                                young.append((kernel[:60], line, op, dest, states))
-                    states += 1
-            if line and not line.endswith(':'):
-                words = line.replace(',', ' ').split()
-                before = before[-15:] + [(words[0], words[1] if len(words) > 1 else '')]
+                lines = kernels.setdefault(f'{line[1:-2]} {i}', [])
+            elif line and not line.endswith(':') and 'file format' not in line:
+                lines.append(line)
+    return kernels
+
+
+def test_loads_to_the_lds_wait_for_descriptors_from_vector_instructions(assembly):
+    """A vector memory instruction may read a scalar register five wait states after a vector instruction (v_readfirstlane) wrote it.
+    The compiler keeps that distance for its own loads, not for the inline assembly of load_to_lds(): in the assembly of the library
+    as it is built no descriptor of such a load is younger, along the instructions in front of it."""
+    import re
+    loads, young = 0, []
+    for kernel, lines in assembly.items():
+        for at, line in enumerate(lines):
+            if not (line.startswith('buffer_load') and line.endswith(' lds')):
+                continue
+            loads += 1
+            low, high = map(int, re.search(r' s\[(\d+):(\d+)\]', line).groups())
+            states = 0
+            for earlier in reversed(lines[max(0, at - 5):at]):
+                op, *operands = earlier.replace(',', ' ').split()
+                if op == 's_nop':
+                    states += int(operands[0], 0)
+                elif op.startswith('v_') and states < 5:
+                    m = re.fullmatch(r's(\d+)|s\[(\d+):(\d+)\]', operands[0])
+                    if m:
+                        first = int(m.group(1) or m.group(2))
+                        if first <= high and int(m.group(3) or first) >= low:
+                            young.append((kernel[:60], line, earlier, states))
+                states += 1
     assert loads > 100
     assert not young, young
+
+
+def test_chain_of_the_grouped_inverses_has_no_flat_accesses(assembly):
+    """Its tiles come from the matrices or from the work matrix: both are global memory, and the kernel says so."""
+    chain = [lines for name, lines in assembly.items() if 'cg_chain_kernel' in name]
+    assert len(chain) == 1 and any(l.startswith('global_store') for l in chain[0])
+    assert not [l for l in chain[0] if l.startswith('flat_')]
 
 
 def test_kernels_that_run_beside_the_framework_hold_their_cus():
