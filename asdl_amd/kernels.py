@@ -1694,7 +1694,8 @@ def inv_root_newton(S, p, ridge_eps, v0, out=None, max_power_iter=100, power_tol
                     poll_every=None):
     """out[b] <- (S[b] + ridge_eps * lambda_max I)^(-1/p) for S = [batch, n, n] (or [n, n]); S keeps the
     ridge.  v0 = [batch, n] start vectors of the power iteration.  Returns (out, stats) with
-    stats = [batch, 4] = (lambda_max, power iterations, newton iterations, final error) on the device.
+    stats = [batch, 4] = (lambda_max, power iterations, newton iterations, final error) on the device; in groups of many large
+    statistics the final error may be an estimate from above (include/asdl_amd.h).
     ``poll_every`` (default ROOT_POLL_AFTER): the Newton iterations are enqueued that many at a time and the host reads
     the convergence flags in between (one small device-to-host copy), so that nothing is launched for a batch that has
     converged; 0 enqueues all ``max_iter`` iterations without ever waiting (the kernels of converged matrices exit at

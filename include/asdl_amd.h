@@ -407,7 +407,10 @@ int ak_kron_precond_static(const float* Binv, const float* Ainv, float* G, int64
  * 2 <= p <= 8, max_iter >= 32), the steps have other coefficients than the reference's, from a lower bound of the spectrum:
  * 10 or 11 steps instead of 20 for a rank-deficient statistic at p = 4 and a ridge of 1e-6 (there a step may be of the fourth degree).
  * stats: device float [batch, 4] = {lambda_max, power iterations, newton iterations,
- * final error}.  n >= 2 (the reference returns the identity for n == 1 without any arithmetic).
+ * final error}.  n >= 2 (the reference returns the identity for n == 1 without any arithmetic).  The final error is max |M - I| behind the
+ * last step.  Where M is known to be within tol of I without being formed (p = 4, two fp16 planes, 192-wide tiles: many large
+ * statistics in one group) the last step leaves it out, and the final error is 5/8 of the largest squared length of a row of M - I
+ * in front of it: to second order not below max |M - I|, and at most 5/8 tol.  The same statistic in a smaller group may report another one.
  * Statistics of 512 columns and more iterate on 16-bit planes written by the product that makes each matrix
  * (192- or 64-wide tiles, n padded to a multiple of that in the workspace): two fp16 planes (22 bits of the power-of-two
  * scaled value, three matrix instructions per fp32-grade product) where ridge_eps, p and n bound the root's largest

@@ -219,6 +219,9 @@ def test_inv_root_steps_of_the_fourth_degree(n, batch):
     for b in {0, batch // 2, batch - 1, batch}:
         alone, st = K.inv_root_newton(S[b:b + 1].clone(), 4, 1e-6, v0[b:b + 1])
         assert torch.equal(st[0, :3], stats[b, :3]), (b, st, stats[b])
+        # the final error is the same too, or (wide tiles, M not formed in the last step) an estimate from above, but for the rounding of M,
+        # four products of 22 bits
+        assert st[0, 3] == stats[b, 3] or (batch > 40 and st[0, 3] <= stats[b, 3] + 4 * 2.0 ** -22 and stats[b, 3] <= 0.625e-6), (b, st, stats[b])
         if n >= 512:
             assert torch.equal(alone[0], root[b]) and torch.equal(root[b], root[b].T), b
         else:
