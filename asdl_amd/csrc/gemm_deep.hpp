@@ -127,7 +127,6 @@ __device__ __forceinline__ void gemm_deep_tile(const GemmParams& p, int ti, int 
     case K_GE_J: kbeg = j0; break;
     case K_LE_I: kend = min(p.K, i0 + BM); break;
     case K_GE_MAXIJ: kbeg = max(i0, j0); break;
-    case K_GE_I: kbeg = i0; break;
     default: break;
   }
   const float* __restrict__ A = p.A + static_cast<int64_t>(z) * p.sA;

@@ -16,8 +16,7 @@ enum KMode {
   K_LE_J = 1,     // contraction limited to k <= column tile (B^T lower triangular)
   K_GE_J = 2,     // k >= column tile start (B lower triangular)
   K_LE_I = 3,     // k <= row tile (A lower triangular)
-  K_GE_MAXIJ = 4, // k >= max(row tile, column tile) start (A^T A with A lower triangular)
-  K_GE_I = 5      // k >= row tile start (A upper triangular)
+  K_GE_MAXIJ = 4  // k >= max(row tile, column tile) start (A^T A with A lower triangular)
 };
 enum TileMode {
   TILE_ALL = 0,
@@ -152,7 +151,6 @@ __device__ __forceinline__ void gemm_f32_tile(const GemmParams& p, int ti, int t
     case K_GE_J: kbeg = tj * BT; break;
     case K_LE_I: kend = min(p.K, (ti + 1) * BT); break;
     case K_GE_MAXIJ: kbeg = max(ti, tj) * BT; break;
-    case K_GE_I: kbeg = ti * BT; break;
     default: break;
   }
   const float* __restrict__ A = p.A + static_cast<int64_t>(z) * p.sA;

@@ -213,7 +213,6 @@ __device__ __forceinline__ void gemm_wave_tile(const GemmParams& p, int ti, int 
     case K_GE_J: kbeg = j0; break;
     case K_LE_I: kend = min(p.K, i0 + 64); break;
     case K_GE_MAXIJ: kbeg = max(i0, j0); break;
-    case K_GE_I: kbeg = i0; break;
     default: break;
   }
   const bool a_kc = (p.transA == 0), b_kc = (p.transB != 0);

@@ -170,12 +170,10 @@ __device__ __forceinline__ bf16x8 x3_frag(AK_LDS3 const unsigned char* plane, bo
 // second one (with two pieces the two cross products stay with the leading one: a third set of accumulators would
 // halve the work groups per CU).
 // The sum then carries about one rounding error instead of one that grows with 6 K / 16 accumulator roundings.
-// OLD_C: beta != 0, and the old result is requested behind the last panel, two k-tiles before it is needed (64 registers more).
-template <int NSPLIT, bool DB, int AKC = -1, int BKC = -1, bool HALF = false, bool CHUNKED = false, bool OLD_C = false>
+template <int NSPLIT, bool DB, int AKC = -1, int BKC = -1, bool HALF = false, bool CHUNKED = false>
 __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj, int z, AK_LDS3 unsigned char* lds) {
   static_assert(!HALF || (NSPLIT == 2 && !DB), "fp16 pieces: two of them, single-buffered loop");
   static_assert(!CHUNKED || NSPLIT >= 2, "chunked sums: split operands");
-  static_assert(!OLD_C || (!DB && !CHUNKED), "old result ahead: the plain single-buffered loop");
   constexpr int BT = X3_BT, BK = X3_BK;
   constexpr int BUF = 2 * NSPLIT * X3_PLANE;        // both operands' planes of one k-tile
   AK_LDS3 unsigned char* panelA = lds;
@@ -191,7 +189,6 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
     case K_GE_J: kbeg = tj * BT; break;
     case K_LE_I: kend = min(p.K, (ti + 1) * BT); break;
     case K_GE_MAXIJ: kbeg = max(ti, tj) * BT; break;
-    case K_GE_I: kbeg = ti * BT; break;
     default: break;
   }
   const float* __restrict__ A = p.A + static_cast<int64_t>(z) * p.sA;
@@ -233,21 +230,6 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
             for (int r = 0; r < 16; ++r) { tot[a][b][r] += acc[a][b][r]; acc[a][b][r] = 0.f; }
       }
     }
-  };
-
-  float old[OLD_C ? 64 : 1];
-  auto fetch_old = [&] {
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int gj = min(j0 + 64 * wc + 32 * b + l32, p.N - 1);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gi = min(i0 + 64 * wr + 32 * a + 8 * (r >> 2) + 4 * g + (r & 3), p.M - 1);
-          old[OLD_C ? 32 * a + 16 * b + r : 0] = C[static_cast<int64_t>(gi) * p.ldc + gj];
-        }
-      }
   };
 
   const int nk = kbeg < kend ? (kend - kbeg + BK - 1) / BK : 0;
@@ -410,20 +392,6 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
           for (int kt = kt0; kt < kt1; ++kt) one_ktile(kt);
           end_of_ktile(7);
         }
-      } else if constexpr (OLD_C) {
-        for (int kt = 0; kt + 2 < nk; ++kt) one_ktile(kt);
-        if (nk >= 2) {
-          fetch(nk - 1);
-          fetch_old();
-          __builtin_amdgcn_sched_barrier(0);
-          multiply(lds);
-          __syncthreads();
-          stash(lds);
-          __syncthreads();
-        } else {
-          fetch_old();
-        }
-        if (nk >= 1) multiply(lds);
       } else {
         for (int kt = 0; kt < nk; ++kt) one_ktile(kt);
       }
@@ -448,14 +416,7 @@ __device__ __forceinline__ void gemm_x3_tile(const GemmParams& p, int ti, int tj
   // triangles of a diagonal tile from the lower one
   const bool mirror = (p.tile_mode == TILE_LOWER_MIRROR);
   const bool lower_only = (p.tile_mode == TILE_LOWER) || (mirror && ti == tj);
-  if constexpr (OLD_C) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] = p.alpha * acc[a][b][r] + p.beta * old[32 * a + 16 * b + r];
-  } else if (p.beta != 0.f) {
+  if (p.beta != 0.f) {
     // all loads of C first: interleaved with the stores they would wait for one another (the compiler cannot tell
     // that the rows differ), one memory latency per element; and none under a lane's own condition, which is waited for by
     // itself.  Elements beyond the matrix, or above the diagonal where only the lower ones are written, are not stored.
