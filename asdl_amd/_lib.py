@@ -27,6 +27,7 @@ _SIGNATURES = {
     'ak_syrk_tn': (c_int, [c_ptr, c_int, c_i64, c_i64, c_i64, c_f32, c_f32, c_ptr, c_i64, c_ptr, c_size, c_ptr]),
     'ak_conv_syrk_ws_bytes': (c_size, [c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int]),
     'ak_conv_syrk_ws_bytes_of': (c_size, [c_int, c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int]),
+    'ak_conv_syrk_planes_ws_bytes': (c_size, [c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int]),
     'ak_conv_syrk': (c_int, [c_ptr, c_int, c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int,
                              c_f32, c_f32, c_ptr, c_i64, c_ptr, c_size, c_ptr]),
     'ak_conv_syrk_nhwc_ws_bytes': (c_size, [c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int]),

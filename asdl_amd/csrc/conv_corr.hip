@@ -1089,16 +1089,22 @@ static bool corr3_window_plan(Corr3Window& v, int64_t N, int64_t C, int64_t H, i
   return true;
 }
 
-// Against the fp32 kernel of syrk_window.hpp, which multiplies 64 x 64 tiles at 46 to 82 TFLOP/s: here 20 us for three launches, 3 TB/s
-// into the planes, 110 TFLOP/s of 128 x 128 tiles of padded channels (a sixth of that is the matrix cores' bf16 rate) and the latency
-// of the splits' sum.  us there and here: samples x channels x image, 3 x 3 / 2: 128 x 64 x 32 x 32 231 and 115, 32 x 64 x 32 x 32 73 and 50,
-// 8 x 64 x 32 x 32 28 and 34, 128 x 96 x 8 x 8 39 and 38, 128 x 192 x 4 x 4 34 and 36, 32 x 300 x 14 x 14 188 and 125; 3 x 3 / 1:
-// 128 x 32 x 32 x 32 270 and 162, 128 x 32 x 16 x 16 75 and 76, 128 x 20 x 32 x 32 140 and 157, 128 x 24 x 32 x 32 183 and 157,
-// 128 x 96 x 16 x 16 391 and 163; 5 x 5 of 16 x 24 x 56 x 56 295 and 214; 2 x 2 / 2 of 128 x 64 x 16 x 16 34 and 60.
+// Against the fp32 kernel of syrk_window.hpp, which multiplies 64 x 64 tiles at 46 to 82 TFLOP/s: here 18 us for three launches, 3.5 TB/s
+// into the planes, 0.45 us per stage of a round of 128 x 128 tiles (13 of a tile's own; a sixth of the matrix cores' bf16 rate), the
+// latency of the splits' sum, and the partial tiles, 64 KB that are written and read again at 5 TB/s, also of a single split.  The last is what
+// factors of many columns and few positions spend their time on (2 x 1600 x 9 x 9, 3 x 3 / 2, 50 positions: 434 us there, 555 here).
+// us there and here: samples x channels x image, 3 x 3 / 2: 128 x 64 x 32 x 32 231 and 115, 32 x 64 x 32 x 32 72 and 48,
+// 8 x 64 x 32 x 32 28 and 34, 128 x 96 x 8 x 8 38 and 37, 128 x 192 x 4 x 4 34 and 36, 32 x 300 x 14 x 14 188 and 125, 64 x 1024 x 4 x 4 354 and 301,
+// 16 x 1024 x 4 x 4 173 and 243, 16 x 2048 x 4 x 4 778 and 891, 64 x 2048 x 4 x 4 1410 and 1137; 3 x 3 / 1: 128 x 32 x 32 x 32 270 and 162,
+// 128 x 32 x 16 x 16 72 and 74, 128 x 20 x 32 x 32 140 and 157, 128 x 24 x 32 x 32 183 and 157, 128 x 96 x 16 x 16 391 and 163,
+// 8 x 300 x 7 x 7 60 and 64; 5 x 5 of 16 x 24 x 56 x 56 295 and 214; 2 x 2 / 2 of 128 x 64 x 16 x 16 34 and 60.  Over 90 windows of 24 to 2048 channels the
+// choice is 0.6 % from the faster one on average, at worst 53 us for 41 (5 x 189 x 14 x 14, 3 x 3 / 1 without padding).  The partial tiles take
+// half the factor's own bytes and 34 MB at most (more than one split only below 512 tiles).
 static bool corr3_window_faster(const Corr3Window& v, int64_t C, int kh, int kw) {
-  const double M = v.args.prod[0].M, T = static_cast<double>((C * kh * kw + 63) / 64), tiles = static_cast<double>(v.items / v.args.prod[0].nsplit);
-  const double there = T * (T + 1) / 2 * 8192 * M / 55e6;
-  const double here = 20 + static_cast<double>(v.plane_bytes) / 3e6 + tiles * 16384 * M / 110e6 + 0.6 * v.args.prod[0].nsplit;
+  const Corr3Prod& p = v.args.prod[0];
+  const double T = static_cast<double>((C * kh * kw + 63) / 64), rounds = (v.items + 255) / 256;
+  const double there = T * (T + 1) / 2 * 8192 * p.M / 55e6;
+  const double here = 18 + static_cast<double>(v.plane_bytes) / 3.5e6 + 0.45 * rounds * (p.k_split + 13) + 0.3 * p.nsplit + v.items * 131072.0 / 5e6;
   return here < there;
 }
 

@@ -605,6 +605,13 @@ extern "C" size_t ak_conv_syrk_ws_bytes_of(int dtype, int64_t N, int64_t C, int6
   return need;
 }
 
+extern "C" size_t ak_conv_syrk_planes_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw, int ph, int pw) {
+  if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || kh <= 0 || kw <= 0 || sh <= 0 || sw <= 0 || ph < 0 || pw < 0) return 0;
+  if (ak::conv_patch_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw) > 0) return 0;
+  const size_t corr = ak::conv_corr_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
+  return corr > 0 ? corr : ak::conv_window_f32_ws_bytes(N, C, H, W, kh, kw, sh, sw, ph, pw);
+}
+
 extern "C" size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int kh, int kw, int sh, int sw,
                                         int ph, int pw) {
   return std::max(ak_conv_syrk_ws_bytes_of(AK_F32, N, C, H, W, kh, kw, sh, sw, ph, pw),

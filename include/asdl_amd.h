@@ -82,6 +82,9 @@ size_t ak_conv_syrk_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W,
                              int kh, int kw, int sh, int sw, int ph, int pw);
 size_t ak_conv_syrk_ws_bytes_of(int dtype, int64_t N, int64_t C, int64_t H, int64_t W,
                                 int kh, int kw, int sh, int sw, int ph, int pw);
+/* What an fp32 call with these sizes needs to run on bf16 planes of its input; 0: it runs on an fp32 kernel. */
+size_t ak_conv_syrk_planes_ws_bytes(int64_t N, int64_t C, int64_t H, int64_t W,
+                                    int kh, int kw, int sh, int sw, int ph, int pw);
 int ak_conv_syrk(const void* x, int dtype, int64_t N, int64_t C, int64_t H, int64_t W,
                  int kh, int kw, int sh, int sw, int ph, int pw,
                  float alpha, float beta, float* A, int64_t lda,

@@ -224,6 +224,36 @@ def test_factor_workspaces_are_for_kernels_that_may_run():
         assert lib.ak_conv_syrk_ws_bytes(*conv) >= max(each) > 0
 
 
+@pytest.mark.parametrize('N,C,H,k,s,p,planes', [
+    # many columns and few positions, where the planes' partial tiles alone take longer: us measured on the fp32 kernel and on planes
+    (16, 1024, 4, 3, 2, 1, False),       # 173, 243
+    (2, 1600, 9, 3, 2, 1, False),        # 434, 555
+    (4, 1696, 7, 3, 2, 1, False),        # 503, 636
+    (4, 2048, 4, 3, 2, 1, False),        # 719, 840
+    (16, 2048, 4, 3, 2, 1, False),       # 778, 891
+    (8, 300, 7, 3, 1, 1, False),         # 60, 64
+    # and where the products do
+    (64, 1024, 4, 3, 2, 1, True),        # 354, 301
+    (64, 2048, 4, 3, 2, 1, True),        # 1410, 1137
+    (128, 2048, 8, 3, 2, 1, True),       # 7931, 3891
+    (64, 512, 4, 3, 2, 1, True),         # 99, 80
+    (128, 256, 8, 3, 2, 1, True),        # 163, 97
+    (128, 128, 8, 3, 2, 1, True),        # 61, 44
+    (32, 64, 32, 3, 2, 1, True),         # 72, 48
+    (8, 600, 7, 5, 1, 2, True),          # 1296, 942
+])
+def test_windows_of_fp32_inputs_go_to_the_faster_kernel(N, C, H, k, s, p, planes):
+    from asdl_amd import _lib
+    lib = _lib.load()
+    need = lib.ak_conv_syrk_planes_ws_bytes(N, C, H, H, k, k, s, s, p, p)
+    assert (need > 0) == planes
+    # the query for a call holds it, and the partial tiles stay below half the padded factor and a round of splits
+    assert lib.ak_conv_syrk_ws_bytes_of(0, N, C, H, H, k, k, s, s, p, p) >= need
+    frame, padded = ((H + 2 * p - k) // s * s + k) ** 2, (C + 31) // 32 * 32
+    tiles = -(-padded * k * k // 128)
+    assert need <= N * frame * 6 * padded + 256 + (512 + tiles * (tiles + 1) // 2) * 65536
+
+
 def test_small_module_preconditioning_leaves_sizes_beyond_its_own_to_the_other_paths():
     """The row matrices of the swift variant have inverses of more than 32768 columns.  The two-launch form declines them, before it
     launches anything, instead of refusing the call."""
