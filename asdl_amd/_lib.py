@@ -99,6 +99,7 @@ _SIGNATURES = {
     'ak_inv_root_group': (c_int, [c_int, c_int, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_f32, c_ptr, c_int, c_f32,
                                   c_int, c_f32, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr]),
     'ak_inv_root_plane_format': (c_int, [c_i64, c_int, c_f32]),
+    'ak_inv_root_lanczos_halves': (c_int, [c_ptr, c_ptr, c_int]),
     'ak_inv_root_newton_part': (c_int, [c_int, c_int, c_ptr, c_i64, c_int, c_i64, c_int, c_f32, c_ptr, c_int, c_f32,
                                         c_int, c_f32, c_ptr, c_i64, c_ptr, c_ptr, c_size, c_ptr]),
 }

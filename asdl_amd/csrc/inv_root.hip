@@ -373,6 +373,10 @@ static __global__ __launch_bounds__(256) void root_lanczos_kernel(RootState st, 
 // 40 x 768 (94 MB) 1.32 and 1.35, 80 x 768 2.24 and 1.96.
 constexpr int kLanczosTile = 256;
 constexpr int64_t kLanczosHalfBytes = 128ll << 20;
+// (from 64 columns on a matrix's buffers hold its parts)
+static bool lanczos_halves(int64_t widest, int64_t narrowest, int64_t bytes) {
+  return widest <= kLanczosLdsDim && narrowest >= 64 && bytes >= kLanczosHalfBytes;
+}
 // parts: [batch][block of rows][block of columns][256], in the matrix buffers, which nothing else uses yet
 __device__ __forceinline__ float* lanczos_parts(float* bufs, int nb, int zl) { return bufs + static_cast<int64_t>(zl) * nb * nb * kLanczosTile; }
 
@@ -1464,8 +1468,7 @@ static int root_run(int phases, int iters, RootGroups& G, float ridge_eps, int m
         return AK_ERR_LAUNCH;
       attr_set = true;
     }
-    // (from 64 columns on a matrix's buffers hold its parts)
-    const bool half = !wide && narrowest >= 64 && bytes >= kLanczosHalfBytes;
+    const bool half = lanczos_halves(widest, narrowest, bytes);
     if (half) {
       blocks = 0;
       for (int i = 0; i < G.count; ++i) {
@@ -1689,6 +1692,13 @@ extern "C" int ak_inv_root_group(int phases, int iters, int groups, float* const
 extern "C" int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps) {
   if (n <= 0 || !ak::root_plane_dim(n)) return 0;
   return ak::root_fp16_scale(n, p, ridge_eps) > 0.f ? 2 : 3;
+}
+
+extern "C" int ak_inv_root_lanczos_halves(const int64_t* n, const int* batch, int groups) {
+  if (!ak::root_args_ok(n, batch, groups)) return 0;
+  int64_t bytes = 0;
+  for (int i = 0; i < groups; ++i) bytes += 4 * batch[i] * n[i] * n[i];
+  return ak::lanczos_halves(*std::max_element(n, n + groups), *std::min_element(n, n + groups), bytes) ? 1 : 0;
 }
 
 // (for any power and ridge: three planes, four product buffers)

@@ -425,6 +425,8 @@ int ak_kron_precond_static(const float* Binv, const float* Ainv, float* G, int64
  * Replaces ComputePower / PowerIter / MatPower (asdl/precondition/shampoo.py:465-586). */
 size_t ak_inv_root_ws_bytes(int64_t n, int batch);
 int ak_inv_root_plane_format(int64_t n, int p, float ridge_eps);
+/* 1: the Lanczos steps of a call with these groups read the lower triangles alone (many large statistics). */
+int ak_inv_root_lanczos_halves(const int64_t* n, const int* batch, int groups);
 int ak_inv_root_newton(float* S, int64_t n, int batch, int64_t strideS, int p, float ridge_eps,
                        const float* v0, int max_power_iter, float power_tol, int max_iter, float tol,
                        float* out, int64_t strideOut, float* stats, void* ws, size_t ws_bytes,

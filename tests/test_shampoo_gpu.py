@@ -3,6 +3,7 @@ fp64 closed form, and ShampooGradientMaker against the reference's golden multi-
 oracle.  Tolerances: roots and preconditioned gradients 1e-3 relative Frobenius error (the iteration
 stops at max|M - I| <= 1e-6, so two fp32 implementations agree to ~1e-5 on well-conditioned input)."""
 import copy
+import ctypes
 import os
 
 import numpy as np
@@ -832,7 +833,10 @@ def test_inv_root_lanczos_on_half_the_statistics():
         S = torch.stack([m.t() @ m for m in x])
         S = torch.tril(S) + torch.tril(S, -1).transpose(1, 2)
         items.append((S.contiguous(), 4, torch.rand(batch, n, device='cuda', generator=gen), None))
-    assert sum(S.numel() * 4 for S, *_ in items) >= 128 << 20
+    def halves(batches):
+        n, b = [S.shape[1] for S, *_ in items], batches
+        return _lib.load().ak_inv_root_lanczos_halves((ctypes.c_int64 * len(n))(*n), (ctypes.c_int * len(b))(*b), len(n))
+    assert halves([S.shape[0] for S, *_ in items]) == 1 and halves([1] * len(items)) == 0
     together = K.inv_root_group([(S.clone(), p, v, out) for S, p, v, out in items], 1e-6)
     for (S, p, v, _), (out, stats) in zip(items, together):
         for z in range(0, S.shape[0], 7):
