@@ -57,8 +57,9 @@ constexpr int kRootSteps = 32;          // entries of a matrix's step table; the
 constexpr int kRootFixedBuffers = 6;    // R0 R1 M0 M1 T0 T1; product buffers behind them (root_buffers)
 constexpr int kRootMinPlaneDim = 512;
 
-// Scales of the two-plane fp16 form (gemm_planes.hpp).  M, the polynomials T and their powers are bounded by the
-// normalisation of the iteration: M <= (1 + p) / 2, T^k <= 12 (root_schedule_kernel), so 2^12 keeps them (and a fair excess of an
+// Scales of the two-plane fp16 form (gemm_planes.hpp).  M and the polynomials are bounded by the normalisation of the iteration:
+// M <= (1 + p) / 2; T^p of a step of the first degree is at most 12 (root_schedule_kernel); of a step of the fourth degree T^2 is at
+// most 5.5 and T^4 29, which is never stored: M' is (T^2 M) T^2 there (root_ops).  So 2^12 keeps them (and a fair excess of an
 // indefinite input) below the fp16 maximum.  The root is kept without its factor z^(1/p): it grows from I to
 // (z A)^(-1/p) <= lambda_min(M_0)^(-1/p), and the ridge bounds lambda_min(M_0) >= ridge_eps (1 + p) / (2 sqrt(n)) from
 // below (lambda_max from the power iteration; a value that is low by a factor f moves the bound by f^(1/p), which the four
@@ -687,7 +688,7 @@ __device__ __forceinline__ int classical_steps(float m, int p, float a0, float b
 // steps, for the classical iteration and kTopMin = 0.17, 0.5, 0.6, 0.7: G 512 x 784 of rank 128 5.6e-5 (20), 1.9e-4 (14), 8.3e-5 (15),
 // 6.5e-5 (15), 5.1e-5 (15); 256 x 300, rank 64 6.6e-5 (20), 2.0e-4 (14), 7.8e-5 (14), 6.4e-5 (15), 5.8e-5 (15); 300 x 600, rank 16
 // 1.2e-4 (20), 2.8e-4 (13), 1.5e-4 (14), 1.3e-4 (14), 1.3e-4 (15); 768 x 3072, rank 400 4.9e-5 (21), 1.3e-4 (14), 6.1e-5 (15),
-// 5.4e-5 (15), 4.6e-5 (16).  0.7 is the first that loses nothing.  T^p stays below 12 for the fp16 planes.
+// 5.4e-5 (15), 4.6e-5 (16).  0.7 is the first that loses nothing.  T^p of these steps stays below 12 for the fp16 planes.
 // Steps of the fourth degree with the top at 0.7, 0.8, 0.85, 0.9 and, last, the first degree, on matrices of the first, second and fourth
 // shape and 300 x 600 of rank 16: 5.7e-5 (10), 5.2e-5 (10), 4.9e-5 (10), 4.4e-5 (11), 5.2e-5 (15); 4.1e-5, 3.9e-5, 3.9e-5, 3.7e-5 (10 each), 5.9e-5 (15);
 // 5.2e-5 (10), 4.8e-5 (10), 4.5e-5 (11), 4.2e-5 (11), 4.6e-5 (16); 6.5e-5, 6.2e-5, 6.0e-5, 6.0e-5 (10 each), 1.3e-4 (15).  0.85 is the lowest that
@@ -1353,7 +1354,8 @@ constexpr int kQuarticSlots = 2;        // products in front of the classical on
 // squaring, with the multiplication order of the reference's MatPower for other powers.
 // quartic (p = 4): two products in front that only steps of the fourth degree have, P = 2 U^2 - I with Y = y(U, P), then
 // T = t(U, P) + P Y, which lies where the step's polynomial for the next one will; and behind the early steps M' is not
-// (T^2)^2 M but (T^2 M) T^2.
+// (T^2)^2 M but (T^2 M) T^2: its rounding (at the top of the file), and T^4 of up to 29 would leave the range of the fp16 planes, whose
+// scale of 2^12 ends at 16.
 static int root_ops(int p, bool quartic, RootOp (*slots)[2], int* counts, int max_slots) {
   if (quartic) {
     const PairedBuf b0{B0, 0}, b1{B0 + 1, 0}, t{T0, 3};
