@@ -17,10 +17,10 @@
 // between two buffers by k, V by the group (the steps of a group write one while the products of the group before read the other).
 // V is kept as the two fp16 pieces of its scaled values, which every tile of the products would form again, where 22 bits do.
 // Bound by the chain (25 to 30 us a step: the leaf 12, its v and update 9, its operands from a row-major matrix 3): with the products
-// beside it, 2 x 4096 takes 33 steps of 25 to 33 us, 7 launches of 244 urgent tiles of 20 us each, and 66 us for the last 1056 (1.2 PFLOP/s of
-// fp16 products would take 43).  All products in launches of their own, 80 us per 512 columns, pieces formed by every tile: 2 x 4096
-// 1720 -> 1400 us, 4096 1265 -> 1070, the 42 factors of ResNet-18 2975 -> 2655, 16 decoder factors of 768 ... 3073 1725 -> 1520,
-// 12 x 1537 825 -> 740, 24 x 1100 665 -> 625, 8192 4080 -> 3440.
+// beside it, 2 x 4096 takes 33 steps of 25 to 33 us, 7 launches of 244 urgent tiles of 19 us each, and 77 us for the last 1056 (1.2 PFLOP/s of
+// fp16 products would take 43).  All products in launches of their own, 80 us per 512 columns, pieces formed by every tile, and now: 2 x 4096
+// 1720 -> 1250 us, 4096 1265 -> 1020, the 42 factors of ResNet-18 2975 -> 2640, 16 decoder factors of 768 ... 3073 1725 -> 1480,
+// 12 x 1537 825 -> 745, 24 x 1100 665 -> 625, 8192 4080 -> 3410.
 // Cross products on an accumulator of their own, and three bf16 pieces in the tiles of the steps, round less than one accumulator for all:
 // error against 64 bits, full rank 5.5e-7 -> 4.5e-7, ReLU rows of rank d / 8 at a / lam = 2^12 4096 1.9e-2 -> 7e-3, 2048 8.8e-3 -> 4e-3.
 #pragma once

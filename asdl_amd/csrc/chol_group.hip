@@ -78,7 +78,7 @@ __device__ __forceinline__ bool cg_skipped(const CgArgs& a, int mat) {
 // W_m <- what the chain's first group of lower(A_m) + lam_m I reads before its products, which take the rest from A_m itself
 // (cc_task_product); padded rows carry the identity; info_m <- 0.  One work group per CG_COPY_ROWS rows of one matrix (bisection on
 // first_copy_block); a row is read and written up to its diagonal element at most.  Bound by the memory: two matrices of 4096 columns 15 us,
-// where all of them took 40 (inverses of ResNet-18's 42 factors 2530 -> 2410 us, a decoder's 1450 -> 1385, 8192 3240 -> 3110).
+// where all of them took 40 (the whole of ResNet-18's 42 factors took 120 us less, a decoder's 65, 8192 130).
 static __global__ __launch_bounds__(256) void cg_copy_in_kernel(CgArgs a, int count) {
   const CgHeader* __restrict__ h = reinterpret_cast<const CgHeader*>(a.plan);
   const CgMat* __restrict__ mats = reinterpret_cast<const CgMat*>(a.plan + h->mats_off);
@@ -357,7 +357,7 @@ static std::vector<std::pair<int, int>> cg_blocked_tiles(int nb) {
   return tiles;
 }
 // Appends a list to the tasks of the launch that starts at task `first` so that every XCD (work group number modulo 8) gets a
-// contiguous eighth of it, whose rows of V its L2 then holds (the 42 factors of ResNet-18 3030 -> 2855 us).
+// contiguous eighth of it, whose rows of V its L2 then holds (the 42 factors of ResNet-18 took 175 us less).
 static void cg_append_by_xcd(std::vector<CcTask>& tasks, int first, const std::vector<CcTask>& list) {
   const size_t n = list.size(), base = tasks.size() - static_cast<size_t>(first);
   size_t next[8], at = 0;
@@ -545,7 +545,7 @@ static double cg_build_chain(const int64_t* dims, int count, CgPlan& plan) {
 // 5.2e-3, 1700 2.7e-3 and 3.2e-3; full rank 3072 2.8e-7 and 3.6e-7.  It takes half the memory, too (3072: 23 and 51 MB).  So the chain is for groups whose steps take three rounds of tiles
 // and more, and of matrices of 15 block columns and more whose third round is used (the 2.3) it has to save a quarter: up to there
 // the sweep served when it was as slow as fp32 products make it, so that no size has lost accuracy since.  The rule goes by the chain with its
-// products in launches of their own, as it was when it was measured (it takes 5 to 20 % less now).  Measured then, sweep and
+// products in launches of their own, as it was when it was measured (it takes up to a tenth less now).  Measured then, sweep and
 // chain, us: two rounds 3072 868 and 846, 2600 with 2304, 2048, 1500, 700, 600 1030 and 930; three and more 4 x 2048 855 and 652,
 // 3 x 2304 886 and 704, 4 x 2400 with 8 x 512 1230 and 880, 60 x 513 373 and 346.  The bound of 4096 tiles keeps the tables of
 // hopeless cases from being built.

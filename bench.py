@@ -386,7 +386,7 @@ def inverse_roofline(w, damping, reps=5):
     return {'bound': 'mfma', 'achieved': achieved, 'peak': FP32_MFMA_PEAK_TFLOPS, 'unit': 'TFLOP/s',
             'frac': achieved / FP32_MFMA_PEAK_TFLOPS, 'executed_fp16_frac': 3 * achieved / BF16_MFMA_PEAK_TFLOPS,
             'flop_per_step': flop, 'matrices': 2 * len(krons), 'standalone_ms': ms,
-            'kernel': 'damped Cholesky inverses of all Kronecker factors of a step (cg_chain_kernel, cg_product_kernel, '
+            'kernel': 'damped Cholesky inverses of all Kronecker factors of a step (cg_chain_kernel, cg_scale_kernel, '
                       'cg_copy_in_kernel, damping kernels), one grouped call with its flag read, nothing beside it; in '
                       'the step the same call runs on a side stream beside the loss backward pass'}
 

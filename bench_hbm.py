@@ -148,7 +148,7 @@ def main(argv=None):
     lam = torch.full((len(mats),), 1e-3, device=dev)
     tri_bytes = sum(m.shape[0] * (m.shape[0] + 1) // 2 for m in mats) * 4
     timed('grouped inverse of 108 factors (whole call)',
-          ['ak::cg_copy_in_kernel', 'ak::cg_chain_kernel', 'ak::cg_product_kernel'], 2 * tri_bytes,
+          ['ak::cg_copy_in_kernel', 'ak::cg_chain_kernel', 'ak::cg_out_kernel'], 2 * tri_bytes,
           lambda: K.chol_inv_grouped(mats, outs, lam),
           note='bytes: the lower triangles read and written once; the call is MFMA bound')
     del mats, outs, A_list, B_list
