@@ -778,6 +778,34 @@ def test_sums_of_the_framework_beside_inverses_on_a_side_stream(K, monkeypatch, 
                 assert torch.equal(x, y), f'{int((x != y).sum())} of {x.numel()} sums differ'
 
 
+@pytest.mark.parametrize('sizes', [[4096] * 2, [4608, 4608, 2304, 2304, 1152, 1152, 576, 512, 256, 128, 64, 27]])
+def test_inverses_on_a_side_stream_beside_products_of_the_framework(K, monkeypatch, sizes):
+    """The same the other way round: the inverses have the bits that they have alone, whatever runs beside them."""
+    from asdl_amd import symmatrix
+    from asdl_amd.symmatrix import Kron, batched_update_inv
+    monkeypatch.setattr(symmatrix, 'INLINE_MICROSECONDS', 0)
+    g = torch.Generator('cuda').manual_seed(3)
+    mats = []
+    for d in sizes:
+        x = torch.randn(d + 100, d, device='cuda', generator=g).relu()
+        mats.append(x.t() @ x / d)
+    krons = [Kron(mats[i], mats[i + 1]) for i in range(0, len(mats), 2)]
+    batched_update_inv(krons, 1e-3)
+    alone = [m.clone() for k in krons for m in (k.A_inv, k.B_inv)]
+    wide = torch.randn(4096, 4096, device='cuda', generator=g).bfloat16()
+    for i in range(24):
+        for k in krons:
+            k.A_inv.fill_(float('nan'))
+            k.B_inv.fill_(float('nan'))
+        pending = batched_update_inv(krons, 1e-3, defer=True)
+        for _ in range(8):
+            wide @ wide
+            wide.float().softmax(1)
+        pending.finish()
+        for m, (x, y) in enumerate(zip((m for k in krons for m in (k.A_inv, k.B_inv)), alone)):
+            assert torch.equal(x, y), f'round {i}, matrix {m}: {int((x != y).sum())} elements differ'
+
+
 def test_sums_of_the_framework_beside_statistics_on_a_side_stream(K):
     """The same of the factors' products, where they are queued on a side stream."""
     g = torch.Generator('cuda').manual_seed(2)
